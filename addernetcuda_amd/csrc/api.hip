@@ -269,7 +269,7 @@ int adder_conv2d_fwd_bf16(const adder_bf16 *x, const float *w, adder_bf16 *y, in
     const size_t nx = sizeof(adder_bf16) * (size_t)N * Ci * H * W, nw = sizeof(float) * (size_t)Co * d.K(),
                  ny = sizeof(adder_bf16) * (size_t)N * Co * d.Ho * d.Wo;
     if (overlaps(y, ny, x, nx) || overlaps(y, ny, w, nw)) return ADDER_ERR_ALIAS;
-    return launch_fwd_bf16(x, w, y, d, static_cast<hipStream_t>(stream));
+    return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream));
 }
 
 int adder_conv2d_bwd_bf16(const adder_bf16 *gy, const adder_bf16 *x, const float *w, adder_bf16 *gx, float *gw,
@@ -294,9 +294,9 @@ int adder_conv2d_bwd_bf16(const adder_bf16 *gy, const adder_bf16 *x, const float
             return ADDER_ERR_ALIAS;
     }
     if (gx)
-        if (int rc = launch_grad_x_bf16(gy, x, w, gx, d, s)) return rc;
+        if (int rc = launch_grad_x(gy, x, w, gx, d, s)) return rc;
     if (gw)
-        if (int rc = launch_grad_w_bf16(gy, x, w, gw, eta, ws, ws_bytes, d, s)) return rc;
+        if (int rc = launch_grad_w(gy, x, w, gw, eta, ws, ws_bytes, d, s)) return rc;
     return ADDER_OK;
 }
 

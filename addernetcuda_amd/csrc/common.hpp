@@ -67,6 +67,10 @@ __device__ __forceinline__ void stf2(bf16_t *p, float2 v) {
     *reinterpret_cast<uint32_t *>(p) = (uint32_t)f32_to_bf16(v.x) | ((uint32_t)f32_to_bf16(v.y) << 16);
 }
 
+// Whether a tensor's base lets four consecutive elements be moved as one group (NULL: no tensor).
+template <class T>
+inline bool aligned_groups(const T *p) { return (reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0; }
+
 // Clamp to [0, 1]: the compiler folds it into the clamp output modifier of the instruction that
 // produces v, so it costs no instruction of its own.
 __device__ __forceinline__ float sat01(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, 1.f); }
@@ -231,14 +235,16 @@ int record_hip_error(hipError_t e);  // stores the message, returns ADDER_ERR_HI
 int check_launch();                  // hipGetLastError -> status
 
 // Launchers implemented in the kernel translation units.
-int launch_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
+// T: storage type of the activations and their gradients, float or bf16_t (the optional reduced-storage mode).
+template <class T>
+int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s);
 int fwd_stats_slots(const ConvDims &d);
 bool fwd_pair_supported(const ConvDims &d);
 int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats,
                     double *stats_side, const ConvDims &d, hipStream_t s);
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);   // 0: no statistics epilogue for these dimensions
-int launch_grad_x(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d,
-                  hipStream_t s, const float *gadd = nullptr);
+template <class T>
+int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
 size_t grad_w_workspace_bytes(const ConvDims &d);
 // The sums of the backward of the BatchNorm behind a layer, as the consumer's input-gradient kernel left them
 // ((C, slots, 2) floats -- a wave's fp32 totals: sum dz, sum dz * xhat), with what turns them into the four coefficients per channel.
@@ -252,7 +258,8 @@ struct BnSums {
     float *dgamma, *dbeta;
 };
 static constexpr BnSums kNoBnSums{nullptr, 0, 0.0, nullptr, nullptr, nullptr, nullptr, nullptr};
-int launch_grad_w(const float *gy, const float *x, const float *w, float *gw, float eta,
+template <class T>
+int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                   void *ws, size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y = nullptr,
                   const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums);
 // the BatchNorm backward passes of a layer's neighbours inside the layer's backward kernels (adder_bn_links)
@@ -266,8 +273,9 @@ int launch_bn_bwd_coef(const float *part, int slots, const float *gamma, const f
 // matrix-core weight gradient of the 3x3 / pad-1 layers (grad_w_mfma.hip); variant 0 = not applicable
 struct GradWMfmaPlan { int variant, slots, gy, gz, tilesH, tilesW, ntiles; };
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d);
-int launch_grad_w_mfma(const float *gy, const float *x, double *part, double *sgpart, const ConvDims &d,
-                       const GradWMfmaPlan &p, hipStream_t s);
+template <class T>
+int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p,
+                       hipStream_t s);
 int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double *sgpart, const ConvDims &d,
                           const GradWMfmaPlan &p, const float *bn_y, const float *bn_coef, float *gy_out, hipStream_t s,
                           const BnSums &sums = kNoBnSums);
@@ -275,12 +283,13 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
 // 1x1 / pad 0 / stride 1-2 kernels (conv1x1.hip)
 bool conv1x1_supported(const ConvDims &d, const void *a, const void *b);
 int fwd_1x1_stats_slots(const ConvDims &d);
-int launch_fwd_1x1(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
-int launch_grad_x_1x1(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d,
-                      hipStream_t s);
+template <class T>
+int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s);
+template <class T>
+int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s);
 int grad_w_1x1_slots(const ConvDims &d);
-int launch_grad_w_1x1(const float *gy, const float *x, float *part, float *sgpart, int slots,
-                      const ConvDims &d, hipStream_t s);
+template <class T>
+int launch_grad_w_1x1(const T *gy, const T *x, float *part, float *sgpart, int slots, const ConvDims &d, hipStream_t s);
 
 // fused BatchNorm + residual + ReLU (bn_act.hip)
 size_t bn_workspace_bytes(int N, int C, int HW);
@@ -325,14 +334,6 @@ int launch_norm_scale_batched(int count, float *const *g, const long *n, const f
 
 int launch_grad_w_slab_finalize(const double *part, const double *sgpart, const float *w, float *gw, int slots, int Co,
                                 int K, bool accumulate, hipStream_t s);
-// bfloat16 storage of x / y / gy / gx (weights and weight gradients stay fp32): the tiled 3x3 / pad-1 kernels and
-// the generic ones
-int launch_fwd_bf16(const bf16_t *x, const float *w, bf16_t *y, const ConvDims &d, hipStream_t s);
-int launch_grad_x_bf16(const bf16_t *gy, const bf16_t *x, const float *w, bf16_t *gx, const ConvDims &d, hipStream_t s);
-int launch_grad_w_bf16(const bf16_t *gy, const bf16_t *x, const float *w, float *gw, float eta, void *ws, size_t ws_bytes,
-                       const ConvDims &d, hipStream_t s);
-int launch_grad_w_mfma_bf16(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d,
-                            const GradWMfmaPlan &p, hipStream_t s);
 int launch_col_fwd(const float *X, const float *W, float *out, int K, long NL, int Co, hipStream_t s);
 size_t col_grad_w_workspace_bytes(int K, long NL, int Co);
 int launch_col_grad_w(const float *gy, const float *X, const float *W, float *gW, int K, long NL,

@@ -29,51 +29,52 @@ struct Lane1x1 {
     }
 };
 
-// Four consecutive floats of a row.  VEC: one aligned float4.  Otherwise (stride 1 on planes whose size is
-// not a multiple of 4, walked as one long row) element by element, `valid` of them inside the row.
-template <bool VEC>
-__device__ __forceinline__ float4 ld4(const float *p, int valid) {
-    if constexpr (VEC) return *reinterpret_cast<const float4 *>(p);
+// Four consecutive elements of a row as floats.  VEC: one aligned group of four.  Otherwise (stride 1 on planes whose
+// size is not a multiple of 4, walked as one long row) element by element, `valid` of them inside the row.
+// T: storage type of the activations (float or bf16_t); arithmetic is fp32 either way.
+template <bool VEC, class T>
+__device__ __forceinline__ float4 ld4(const T *p, int valid) {
+    if constexpr (VEC) return ldf4(p);
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (valid > 0) v.x = p[0];
-    if (valid > 1) v.y = p[1];
-    if (valid > 2) v.z = p[2];
-    if (valid > 3) v.w = p[3];
+    if (valid > 0) v.x = ldf(p);
+    if (valid > 1) v.y = ldf(p + 1);
+    if (valid > 2) v.z = ldf(p + 2);
+    if (valid > 3) v.w = ldf(p + 3);
     return v;
 }
-template <bool VEC>
-__device__ __forceinline__ void st4(float *p, const float4 v, int valid) {
+template <bool VEC, class T>
+__device__ __forceinline__ void st4(T *p, const float4 v, int valid) {
     if constexpr (VEC) {
-        *reinterpret_cast<float4 *>(p) = v;
+        stf4(p, v);
     } else {
-        if (valid > 0) p[0] = v.x;
-        if (valid > 1) p[1] = v.y;
-        if (valid > 2) p[2] = v.z;
-        if (valid > 3) p[3] = v.w;
+        if (valid > 0) stf(p, v.x);
+        if (valid > 1) stf(p + 1, v.y);
+        if (valid > 2) stf(p + 2, v.z);
+        if (valid > 3) stf(p + 3, v.w);
     }
 }
 
-template <bool VEC>
-__device__ __forceinline__ float2 ld2(const float *p, int valid) {
-    if constexpr (VEC) return *reinterpret_cast<const float2 *>(p);
+template <bool VEC, class T>
+__device__ __forceinline__ float2 ld2(const T *p, int valid) {
+    if constexpr (VEC) return ldf2(p);
     float2 v = make_float2(0.f, 0.f);
-    if (valid > 0) v.x = p[0];
-    if (valid > 1) v.y = p[1];
+    if (valid > 0) v.x = ldf(p);
+    if (valid > 1) v.y = ldf(p + 1);
     return v;
 }
-template <bool VEC>
-__device__ __forceinline__ void st2(float *p, const float2 v, int valid) {
+template <bool VEC, class T>
+__device__ __forceinline__ void st2(T *p, const float2 v, int valid) {
     if constexpr (VEC) {
-        *reinterpret_cast<float2 *>(p) = v;
+        stf2(p, v);
     } else {
-        if (valid > 0) p[0] = v.x;
-        if (valid > 1) p[1] = v.y;
+        if (valid > 0) stf(p, v.x);
+        if (valid > 1) stf(p + 1, v.y);
     }
 }
 
-template <int S, int TM, bool VEC = true>
-__global__ __launch_bounds__(256) void fwd_1x1_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                      float *__restrict__ y, double *__restrict__ stats, int N, int Ci,
+template <int S, int TM, bool VEC = true, class T = float>
+__global__ __launch_bounds__(256) void fwd_1x1_kernel(const T *__restrict__ x, const float *__restrict__ w,
+                                                      T *__restrict__ y, double *__restrict__ stats, int N, int Ci,
                                                       int H, int W, int Co, int Ho, int Wo, int gpr, int groups) {
     constexpr int TN = 4 / S;
     const Lane1x1<S> L(blockIdx.x * 256 + threadIdx.x, groups, gpr, Ho);
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256) void fwd_1x1_kernel(const float *__restrict__ 
     l2_warm(w + (size_t)co0 * Ci, 1, 0, min(TM, Co - co0) * Ci);   // the scalar weight loads below run one step ahead
 
     const size_t plane = (size_t)H * W;
-    const float *xp = x + (size_t)L.n * Ci * plane + (size_t)(L.ho * S) * W + L.wo0 * S;
+    const T *xp = x + (size_t)L.n * Ci * plane + (size_t)(L.ho * S) * W + L.wo0 * S;
     const int valid = L.ok ? W - L.wo0 * S : 0;   // only read when !VEC
     int ci = 0;
     for (; ci + 4 <= Ci; ci += 4) {
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(256) void fwd_1x1_kernel(const float *__restrict__ 
 #pragma unroll
         for (int m = 0; m < TM; ++m) {
             if (co0 + m >= Co) continue;
-            float *dst = y + (((size_t)L.n * Co + co0 + m) * Ho + L.ho) * Wo + L.wo0;
+            T *dst = y + (((size_t)L.n * Co + co0 + m) * Ho + L.ho) * Wo + L.wo0;
             if constexpr (TN == 4)
                 st4<VEC>(dst, make_float4(tot[m][0], tot[m][1], tot[m][2], tot[m][3]), valid);
             else
@@ -167,10 +168,10 @@ __global__ __launch_bounds__(256) void fwd_1x1_kernel(const float *__restrict__ 
     }
 }
 
-template <int S, int TM, bool VEC = true>
-__global__ __launch_bounds__(256) void grad_x_1x1_kernel(const float *__restrict__ gy,
-                                                         const float *__restrict__ x,
-                                                         const float *__restrict__ w, float *__restrict__ gx,
+template <int S, int TM, bool VEC = true, class T = float>
+__global__ __launch_bounds__(256) void grad_x_1x1_kernel(const T *__restrict__ gy,
+                                                         const T *__restrict__ x,
+                                                         const float *__restrict__ w, T *__restrict__ gx,
                                                          int N, int Ci, int H, int W, int Co, int Ho, int Wo,
                                                          int gpr, int groups) {
     constexpr int TN = 4 / S;
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(256) void grad_x_1x1_kernel(const float *__restrict
     }
     l2_warm(w + min(ci0, Ci - 1), Co, Ci, min(TM, Ci - ci0));   // one run of TM weights per output channel
     const size_t gplane = (size_t)Ho * Wo;
-    const float *gp = gy + (size_t)L.n * Co * gplane + (size_t)L.ho * Wo + L.wo0;
+    const T *gp = gy + (size_t)L.n * Co * gplane + (size_t)L.ho * Wo + L.wo0;
     // eight output channels per round: their gy loads are issued together (little arithmetic per load, so
     // the loop is bound by how many loads are in flight); channels past Co load nothing and count as gy = 0
     constexpr int UN = 8;
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void grad_x_1x1_kernel(const float *__restrict
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const bool live = co0 + u < Co;
-            const float *src = gp + (size_t)min(co0 + u, Co - 1) * gplane;
+            const T *src = gp + (size_t)min(co0 + u, Co - 1) * gplane;
             if constexpr (TN == 4) {
                 const float4 v = ld4<VEC>(src, live ? valid : 0);
                 g[u][0] = v.x; g[u][1] = v.y; g[u][2] = v.z; g[u][3] = v.w;
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(256) void grad_x_1x1_kernel(const float *__restrict
 #pragma unroll
         for (int m = 0; m < TM; ++m) {
             if (ci0 + m >= Ci) continue;
-            float *dst = gx + xoff + (size_t)(ci0 + m) * plane;
+            T *dst = gx + xoff + (size_t)(ci0 + m) * plane;
             if constexpr (S == 1) {
                 st4<VEC>(dst, make_float4(tot[m][0], tot[m][1], tot[m][2], tot[m][3]), valid);
             } else {
@@ -260,9 +261,9 @@ __global__ __launch_bounds__(256) void grad_x_1x1_kernel(const float *__restrict
 
 // grad_w: a wave owns TM output channels x TC input channels; its lanes walk over position
 // groups, then the 64 lanes are folded through LDS (16 sums per round).
-template <int S, int TM, int TC, bool VEC = true>
-__global__ __launch_bounds__(256) void grad_w_1x1_kernel(const float *__restrict__ gy,
-                                                         const float *__restrict__ x, float *__restrict__ part,
+template <int S, int TM, int TC, bool VEC = true, class T = float>
+__global__ __launch_bounds__(256) void grad_w_1x1_kernel(const T *__restrict__ gy,
+                                                         const T *__restrict__ x, float *__restrict__ part,
                                                          float *__restrict__ sgpart, int N, int Ci, int H,
                                                          int W, int Co, int Ho, int Wo, int gpr, int groups) {
     constexpr int TN = 4 / S, A = TM * TC;
@@ -277,8 +278,8 @@ __global__ __launch_bounds__(256) void grad_w_1x1_kernel(const float *__restrict
     }
     for (int g0 = blockIdx.x * 256 + threadIdx.x; g0 < groups; g0 += gridDim.x * 256) {
         const Lane1x1<S> L(g0, groups, gpr, Ho);
-        const float *xp = x + (size_t)L.n * Ci * plane + (size_t)(L.ho * S) * W + L.wo0 * S;
-        const float *gp = gy + (size_t)L.n * Co * gplane + (size_t)L.ho * Wo + L.wo0;
+        const T *xp = x + (size_t)L.n * Ci * plane + (size_t)(L.ho * S) * W + L.wo0 * S;
+        const T *gp = gy + (size_t)L.n * Co * gplane + (size_t)L.ho * Wo + L.wo0;
         const int valid = W - L.wo0 * S;   // only read when !VEC
         float xs[TC][TN], gs[TM][TN];
 #pragma unroll
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(256) void grad_w_1x1_kernel(const float *__restrict
         }
 #pragma unroll
         for (int m = 0; m < TM; ++m) {
-            const float *p = gp + (size_t)min(co0 + m, Co - 1) * gplane;
+            const T *p = gp + (size_t)min(co0 + m, Co - 1) * gplane;
             if constexpr (TN == 4) {
                 const float4 v = ld4<VEC>(p, valid);
                 gs[m][0] = v.x; gs[m][1] = v.y; gs[m][2] = v.z; gs[m][3] = v.w;
@@ -352,6 +353,7 @@ __global__ __launch_bounds__(256) void grad_w_1x1_kernel(const float *__restrict
 // whose size is not a multiple of 4 (7x7) or whose base is not 16-byte aligned take the element-wise loads.
 // Stride 2: one float4 of the source row per lane (two of its elements are sampled) and a float2 of the
 // output row; rows that are not whole aligned groups (W % 4, Wo % 2, base pointers) are read element-wise.
+// (For bfloat16 storage the groups of four are 8 bytes.)
 bool conv1x1_supported(const ConvDims &d, const void *, const void *) {
     return d.kh == 1 && d.kw == 1 && d.pad == 0 && (d.stride == 1 || d.stride == 2);
 }
@@ -363,10 +365,11 @@ static ConvDims lane_dims(const ConvDims &d) {
     return f;
 }
 
-static bool vec_ok(const ConvDims &f, const void *a, const void *b, const void *c) {
-    const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c);
-    if (f.stride == 2) return f.W % 4 == 0 && f.Wo % 2 == 0 && (bits & 15) == 0;
-    return f.W % 4 == 0 && (bits & 15) == 0;
+template <class T>
+static bool vec_ok(const ConvDims &f, const T *a, const T *b, const T *c) {
+    const bool aligned = aligned_groups(a) && aligned_groups(b) && aligned_groups(c);
+    if (f.stride == 2) return f.W % 4 == 0 && f.Wo % 2 == 0 && aligned;
+    return f.W % 4 == 0 && aligned;
 }
 
 static void lane_space(const ConvDims &f, int &gpr, int &groups) {
@@ -383,48 +386,41 @@ int fwd_1x1_stats_slots(const ConvDims &d) {
 }
 
 // stats (nullable): per-channel partial sums of y and y*y, fwd_1x1_stats_slots(d) slots per channel
-int launch_fwd_1x1(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s) {
+template <class T>
+int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s) {
     constexpr int TM = 8;
     const ConvDims f = lane_dims(d);
     int gpr, groups;
     lane_space(f, gpr, groups);
-    const dim3 grid(ceil_div(groups, 256), ceil_div(f.Co, TM));
-    if (f.stride == 2 && vec_ok(f, x, y, nullptr))
-        hipLaunchKernelGGL((fwd_1x1_kernel<2, TM, true>), grid, dim3(256), 0, s, x, w, y, stats, f.N, f.Ci, f.H, f.W, f.Co,
-                           f.Ho, f.Wo, gpr, groups);
-    else if (f.stride == 2)
-        hipLaunchKernelGGL((fwd_1x1_kernel<2, TM, false>), grid, dim3(256), 0, s, x, w, y, stats, f.N, f.Ci, f.H, f.W, f.Co,
-                           f.Ho, f.Wo, gpr, groups);
-    else if (vec_ok(f, x, y, nullptr))
-        hipLaunchKernelGGL((fwd_1x1_kernel<1, TM, true>), grid, dim3(256), 0, s, x, w, y, stats, f.N, f.Ci, f.H, f.W, f.Co,
-                           f.Ho, f.Wo, gpr, groups);
-    else
-        hipLaunchKernelGGL((fwd_1x1_kernel<1, TM, false>), grid, dim3(256), 0, s, x, w, y, stats, f.N, f.Ci, f.H, f.W, f.Co,
-                           f.Ho, f.Wo, gpr, groups);
-    return check_launch();
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(ceil_div(groups, 256), ceil_div(f.Co, TM)), dim3(256), 0, s, x, w, y, stats, f.N, f.Ci,
+                           f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
+        return check_launch();
+    };
+    const bool vec = vec_ok<T>(f, x, y, nullptr);
+    if (f.stride == 2) return vec ? launch(fwd_1x1_kernel<2, TM, true, T>) : launch(fwd_1x1_kernel<2, TM, false, T>);
+    return vec ? launch(fwd_1x1_kernel<1, TM, true, T>) : launch(fwd_1x1_kernel<1, TM, false, T>);
 }
+template int launch_fwd_1x1<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t);
+template int launch_fwd_1x1<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t);
 
-int launch_grad_x_1x1(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d,
-                      hipStream_t s) {
+template <class T>
+int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s) {
     constexpr int TM = 4;   // latency-bound at ResNet sizes: more workgroups beat more reuse per lane
     const ConvDims f = lane_dims(d);
     int gpr, groups;
     lane_space(f, gpr, groups);
-    const dim3 grid(ceil_div(groups, 256), ceil_div(f.Ci, TM));
-    if (f.stride == 2 && vec_ok(f, gy, x, gx))
-        hipLaunchKernelGGL((grad_x_1x1_kernel<2, TM, true>), grid, dim3(256), 0, s, gy, x, w, gx, f.N, f.Ci, f.H, f.W,
-                           f.Co, f.Ho, f.Wo, gpr, groups);
-    else if (f.stride == 2)
-        hipLaunchKernelGGL((grad_x_1x1_kernel<2, TM, false>), grid, dim3(256), 0, s, gy, x, w, gx, f.N, f.Ci, f.H,
-                           f.W, f.Co, f.Ho, f.Wo, gpr, groups);
-    else if (vec_ok(f, gy, x, gx))
-        hipLaunchKernelGGL((grad_x_1x1_kernel<1, TM, true>), grid, dim3(256), 0, s, gy, x, w, gx, f.N, f.Ci, f.H, f.W,
-                           f.Co, f.Ho, f.Wo, gpr, groups);
-    else
-        hipLaunchKernelGGL((grad_x_1x1_kernel<1, TM, false>), grid, dim3(256), 0, s, gy, x, w, gx, f.N, f.Ci, f.H,
-                           f.W, f.Co, f.Ho, f.Wo, gpr, groups);
-    return check_launch();
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(ceil_div(groups, 256), ceil_div(f.Ci, TM)), dim3(256), 0, s, gy, x, w, gx, f.N, f.Ci,
+                           f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
+        return check_launch();
+    };
+    const bool vec = vec_ok<T>(f, gy, x, gx);
+    if (f.stride == 2) return vec ? launch(grad_x_1x1_kernel<2, TM, true, T>) : launch(grad_x_1x1_kernel<2, TM, false, T>);
+    return vec ? launch(grad_x_1x1_kernel<1, TM, true, T>) : launch(grad_x_1x1_kernel<1, TM, false, T>);
 }
+template int launch_grad_x_1x1<float>(const float *, const float *, const float *, float *, const ConvDims &, hipStream_t);
+template int launch_grad_x_1x1<bf16_t>(const bf16_t *, const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t);
 
 static constexpr int kGw1x1TM = 8, kGw1x1TC = 8;
 
@@ -439,25 +435,23 @@ int grad_w_1x1_slots(const ConvDims &d) {
     return want < 1 ? 1 : want;
 }
 
-int launch_grad_w_1x1(const float *gy, const float *x, float *part, float *sgpart, int slots,
-                      const ConvDims &d, hipStream_t s) {
+template <class T>
+int launch_grad_w_1x1(const T *gy, const T *x, float *part, float *sgpart, int slots, const ConvDims &d, hipStream_t s) {
+    constexpr int TM = kGw1x1TM, TC = kGw1x1TC;
     const ConvDims f = lane_dims(d);
     int gpr, groups;
     lane_space(f, gpr, groups);
-    const dim3 grid(slots, ceil_div(f.Co, kGw1x1TM), ceil_div(f.Ci, kGw1x1TC));
-    if (f.stride == 2 && vec_ok(f, gy, x, nullptr))
-        hipLaunchKernelGGL((grad_w_1x1_kernel<2, kGw1x1TM, kGw1x1TC, true>), grid, dim3(256), 0, s, gy, x, part,
-                           sgpart, f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
-    else if (f.stride == 2)
-        hipLaunchKernelGGL((grad_w_1x1_kernel<2, kGw1x1TM, kGw1x1TC, false>), grid, dim3(256), 0, s, gy, x, part,
-                           sgpart, f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
-    else if (vec_ok(f, gy, x, nullptr))
-        hipLaunchKernelGGL((grad_w_1x1_kernel<1, kGw1x1TM, kGw1x1TC, true>), grid, dim3(256), 0, s, gy, x, part,
-                           sgpart, f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
-    else
-        hipLaunchKernelGGL((grad_w_1x1_kernel<1, kGw1x1TM, kGw1x1TC, false>), grid, dim3(256), 0, s, gy, x, part,
-                           sgpart, f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
-    return check_launch();
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(slots, ceil_div(f.Co, TM), ceil_div(f.Ci, TC)), dim3(256), 0, s, gy, x, part, sgpart,
+                           f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
+        return check_launch();
+    };
+    const bool vec = vec_ok<T>(f, gy, x, nullptr);
+    if (f.stride == 2)
+        return vec ? launch(grad_w_1x1_kernel<2, TM, TC, true, T>) : launch(grad_w_1x1_kernel<2, TM, TC, false, T>);
+    return vec ? launch(grad_w_1x1_kernel<1, TM, TC, true, T>) : launch(grad_w_1x1_kernel<1, TM, TC, false, T>);
 }
+template int launch_grad_w_1x1<float>(const float *, const float *, float *, float *, int, const ConvDims &, hipStream_t);
+template int launch_grad_w_1x1<bf16_t>(const bf16_t *, const bf16_t *, float *, float *, int, const ConvDims &, hipStream_t);
 
 }  // namespace adder

@@ -501,24 +501,26 @@ int fwd_stats_slots(const ConvDims &d) {
     }
 }
 
-// stats (nullable): per-channel partial sums of y and y*y, fwd_stats_slots(d) > 0 slots per channel
-int launch_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s) {
-    // rows that are whole float4 groups are moved as float4 and need 16-byte aligned bases
-    const bool k3p1 = d.kh == 3 && d.kw == 3 && d.pad == 1 &&
-                      (d.W % 4 != 0 || (reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
-                      (d.Wo % 4 != 0 || (reinterpret_cast<uintptr_t>(y) & 15) == 0);
+// stats (nullable): per-channel partial sums of y and y*y, fwd_stats_slots(d) > 0 slots per channel.
+// Both storage types take the same kernels and tile shapes: the arithmetic, which bounds them, is the same fp32.
+// (bfloat16 layers other than 3x3 once went to the generic kernel: 128 -> 512 1x1 @28x28, 32 images, 561 us.)
+template <class T>
+int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s) {
+    // rows that are whole groups of four are moved as such and need bases aligned to a group
+    const bool k3p1 = d.kh == 3 && d.kw == 3 && d.pad == 1 && (d.W % 4 != 0 || aligned_groups(x)) &&
+                      (d.Wo % 4 != 0 || aligned_groups(y));
     const int variant = fwd_tiled_variant(d);
     const bool strided = variant == 8 || variant == 9 || variant == 12 || variant == 13;
     if (strided) {   // x is read element by element; y is a dense row per plane
         const ConvDims f = as_one_row(d);
-        if (f.Wo % 4 != 0 || (reinterpret_cast<uintptr_t>(y) & 15) == 0) switch (variant) {
-            case 8: case 9: return launch_fwd_3x3_v<Fwd1x1sub, false, true>(x, w, y, stats, f, s, sampling_of(d));
-            case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true>(x, w, y, stats, f, s, sampling_of(d));
-            default: return launch_fwd_3x3_v<Fwd1x1sq, false, true>(x, w, y, stats, f, s, sampling_of(d));
+        if (f.Wo % 4 != 0 || aligned_groups(y)) switch (variant) {
+            case 8: case 9: return launch_fwd_3x3_v<Fwd1x1sub, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d));
+            case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d));
+            default: return launch_fwd_3x3_v<Fwd1x1sq, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d));
         }
     } else if (variant >= 6) {
         const ConvDims f = as_one_row(d);
-        if (f.W % 4 != 0 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0) switch (variant) {
+        if (f.W % 4 != 0 || (aligned_groups(x) && aligned_groups(y))) switch (variant) {
             case 6: return launch_fwd_3x3<Fwd1x1>(x, w, y, stats, f, s);
             case 7: return launch_fwd_3x3<Fwd1x1s>(x, w, y, stats, f, s);
             case 10: return launch_fwd_3x3<Fwd1x1q>(x, w, y, stats, f, s);
@@ -548,34 +550,12 @@ int launch_fwd(const float *x, const float *w, float *y, double *stats, const Co
     if (stats) return ADDER_ERR_UNSUPPORTED;   // the generic kernel has no statistics epilogue
     constexpr int TM = 8;
     const long total = (long)d.N * d.Ho * d.Wo;
-    hipLaunchKernelGGL(fwd_generic_kernel<TM>, dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Co, TM)),
+    hipLaunchKernelGGL((fwd_generic_kernel<TM, T>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Co, TM)),
                        dim3(256), 0, s, x, w, y, d);
     return check_launch();
 }
-
-// bfloat16 storage: the tiled 3x3 / pad-1 kernels (stride 1 or 2), the generic kernel for everything else
-int launch_fwd_bf16(const bf16_t *x, const float *w, bf16_t *y, const ConvDims &d, hipStream_t s) {
-    const bool k3p1 = d.kh == 3 && d.kw == 3 && d.pad == 1 &&
-                      (d.W % 4 != 0 || (reinterpret_cast<uintptr_t>(x) & 7) == 0) &&
-                      (d.Wo % 4 != 0 || (reinterpret_cast<uintptr_t>(y) & 7) == 0);
-    if (k3p1) {
-        const int variant = d.stride == 1 ? (d.Wo > 16 ? 1 : (d.Wo > 8 ? 2 : 3)) : (d.stride == 2 ? (d.Wo > 8 ? 4 : 5) : 0);
-        switch (variant) {
-            case 1: return launch_fwd_3x3<FwdW32, bf16_t>(x, w, y, nullptr, d, s);
-            case 2: return launch_fwd_3x3<FwdW16, bf16_t>(x, w, y, nullptr, d, s);
-            case 3: return launch_fwd_3x3<FwdW8, bf16_t>(x, w, y, nullptr, d, s);
-            case 4: return launch_fwd_3x3<FwdW16S2, bf16_t>(x, w, y, nullptr, d, s);
-            case 5: return d.Ci >= 128 ? launch_fwd_3x3<FwdW8S2L, bf16_t>(x, w, y, nullptr, d, s)
-                                       : launch_fwd_3x3<FwdW8S2, bf16_t>(x, w, y, nullptr, d, s);
-            default: break;
-        }
-    }
-    constexpr int TM = 8;
-    const long total = (long)d.N * d.Ho * d.Wo;
-    hipLaunchKernelGGL((fwd_generic_kernel<TM, bf16_t>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Co, TM)),
-                       dim3(256), 0, s, x, w, y, d);
-    return check_launch();
-}
+template int launch_fwd<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t);
+template int launch_fwd<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t);
 
 // An ordinary convolution y = sum w * x through the tiled forward kernels: 3x3 / stride 1 / pad 1 only
 // (ADDER_ERR_UNSUPPORTED elsewhere).  stats as in launch_fwd; the slot count is fwd_stats_slots(d).

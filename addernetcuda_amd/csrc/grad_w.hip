@@ -376,23 +376,24 @@ size_t grad_w_workspace_bytes(const ConvDims &d) {
 
 // bn_y with either bn_coef or sums.part: gy is the gradient dz of the output of the BatchNorm behind the layer and
 // the kernel forms the layer's own output gradient from it, leaving it in gy_out (nullable) on the way (matrix-core
-// kernels only: ADDER_ERR_UNSUPPORTED, nothing launched, elsewhere)
-int launch_grad_w(const float *gy, const float *x, const float *w, float *gw, float eta, void *ws,
+// kernels only: ADDER_ERR_UNSUPPORTED, nothing launched, elsewhere).  Both storage types take the same kernels (gw and w
+// are fp32 either way); bfloat16 1x1 layers once went to the generic one: 128 -> 512 @28x28, 32 images, 2826 us.
+template <class T>
+int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws,
                   size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y, const float *bn_coef,
                   float *gy_out, const BnSums &sums) {
     if (ws_bytes < grad_w_workspace_bytes(d)) return ADDER_ERR_WORKSPACE;
     GradWPlan p = plan_grad_w(d);
-    if (bn_y && !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part))
+    if (bn_y && (sizeof(T) != 4 ||
+                 !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part)))
         return ADDER_ERR_UNSUPPORTED;
-    // float4 loads need 16-byte aligned bases; tensors whose rows are read element by element do not
+    // loads of four elements need bases aligned to a group; tensors whose rows are read element by element do not
     // (1x1 layers on the matrix cores walk whole planes as rows: their row length is H*W)
     const bool rows_1x1 = p.variant == 2 && d.kh == 1;
     const bool need_x16 = p.variant == 2 && !(rows_1x1 && d.stride > 1) &&   // (a strided 1x1 layer samples x element-wise)
                           (rows_1x1 ? d.H * d.W : d.W) % 4 == 0;
     const bool need_g16 = p.variant == 2 && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
-    if (p.variant && ((need_x16 && (reinterpret_cast<uintptr_t>(x) & 15)) ||
-                      (need_g16 && (reinterpret_cast<uintptr_t>(gy) & 15))))
-        p.variant = 0;
+    if (p.variant && ((need_x16 && !aligned_groups(x)) || (need_g16 && !aligned_groups(gy)))) p.variant = 0;
     double *ss = reinterpret_cast<double *>(ws);
     const int K = d.K();
     const long n = (long)d.Co * K;
@@ -403,8 +404,11 @@ int launch_grad_w(const float *gy, const float *x, const float *w, float *gw, fl
         if (p.variant == 2) {
             double *part = reinterpret_cast<double *>(ss + kNormBlocksMax);
             double *sgpart = part + (size_t)p.slots * d.Co * K;
-            rc = bn_y ? launch_grad_w_mfma_bn(gy, x, part, sgpart, d, p.mfma, bn_y, bn_coef, gy_out, s, sums)
-                      : launch_grad_w_mfma(gy, x, part, sgpart, d, p.mfma, s);
+            if constexpr (sizeof(T) == 4)
+                rc = bn_y ? launch_grad_w_mfma_bn(gy, x, part, sgpart, d, p.mfma, bn_y, bn_coef, gy_out, s, sums)
+                          : launch_grad_w_mfma(gy, x, part, sgpart, d, p.mfma, s);
+            else
+                rc = launch_grad_w_mfma(gy, x, part, sgpart, d, p.mfma, s);
             if (rc) return rc;
             hipLaunchKernelGGL(grad_w_finalize_kernel<double>, dim3(nb), dim3(kFinOut * kFinLanes), 0, s, part,
                                sgpart, w, gw, fused_norm ? ss : nullptr, p.slots, d.Co, K);
@@ -426,51 +430,21 @@ int launch_grad_w(const float *gy, const float *x, const float *w, float *gw, fl
     const int KK = d.kh * d.kw;
     const long wgs = (long)d.Co * d.Ci;
     if (d.kh == 3 && d.kw == 3)
-        hipLaunchKernelGGL((grad_w_generic_kernel<3, 3>), dim3((unsigned)wgs), dim3(256), 0, s, gy, x, w, gw, d);
+        hipLaunchKernelGGL((grad_w_generic_kernel<3, 3, T>), dim3((unsigned)wgs), dim3(256), 0, s, gy, x, w, gw, d);
     else if (d.kh == 1 && d.kw == 1)
-        hipLaunchKernelGGL((grad_w_generic_kernel<1, 1>), dim3((unsigned)wgs), dim3(256), 0, s, gy, x, w, gw, d);
+        hipLaunchKernelGGL((grad_w_generic_kernel<1, 1, T>), dim3((unsigned)wgs), dim3(256), 0, s, gy, x, w, gw, d);
     else
-        hipLaunchKernelGGL((grad_w_generic_kernel<0, 0>), dim3((unsigned)(wgs * KK)), dim3(256), 0, s, gy, x, w,
+        hipLaunchKernelGGL((grad_w_generic_kernel<0, 0, T>), dim3((unsigned)(wgs * KK)), dim3(256), 0, s, gy, x, w,
                            gw, d);
     int rc = check_launch();
     if (rc) return rc;
     if (eta > 0.f) return launch_norm_scale(gw, n, eta, 1e-12f, ws, s);
     return ADDER_OK;
 }
-
-// bfloat16 storage of gy and x (gw and w stay fp32): the matrix-core kernel for 3x3 / pad-1 layers, the generic
-// kernel for everything else; the same finalize and scaling as the fp32 path
-int launch_grad_w_bf16(const bf16_t *gy, const bf16_t *x, const float *w, float *gw, float eta, void *ws,
-                       size_t ws_bytes, const ConvDims &d, hipStream_t s) {
-    if (ws_bytes < grad_w_workspace_bytes(d)) return ADDER_ERR_WORKSPACE;
-    GradWPlan p = plan_grad_w(d);
-    const bool tiled = p.variant == 2 && d.kh == 3 && (d.W % 4 != 0 || (reinterpret_cast<uintptr_t>(x) & 7) == 0) &&
-                       (d.Wo % 4 != 0 || (reinterpret_cast<uintptr_t>(gy) & 7) == 0);
-    double *ss = reinterpret_cast<double *>(ws);
-    const int K = d.K();
-    const long n = (long)d.Co * K;
-    if (tiled) {
-        double *part = reinterpret_cast<double *>(ss + kNormBlocksMax);
-        double *sgpart = part + (size_t)p.slots * d.Co * K;
-        if (int rc = launch_grad_w_mfma_bf16(gy, x, part, sgpart, d, p.mfma, s)) return rc;
-        const int nb = (int)ceil_div_l(n, fin_out_for(p.slots));
-        hipLaunchKernelGGL(grad_w_finalize_kernel<double>, dim3(nb), dim3(kFinOut * kFinLanes), 0, s, part, sgpart, w, gw,
-                           nullptr, p.slots, d.Co, K);
-    } else {
-        const int KK = d.kh * d.kw;
-        const long wgs = (long)d.Co * d.Ci;
-        if (d.kh == 3 && d.kw == 3)
-            hipLaunchKernelGGL((grad_w_generic_kernel<3, 3, bf16_t>), dim3((unsigned)wgs), dim3(256), 0, s, gy, x, w, gw, d);
-        else if (d.kh == 1 && d.kw == 1)
-            hipLaunchKernelGGL((grad_w_generic_kernel<1, 1, bf16_t>), dim3((unsigned)wgs), dim3(256), 0, s, gy, x, w, gw, d);
-        else
-            hipLaunchKernelGGL((grad_w_generic_kernel<0, 0, bf16_t>), dim3((unsigned)(wgs * KK)), dim3(256), 0, s, gy, x, w,
-                               gw, d);
-    }
-    if (int rc = check_launch()) return rc;
-    if (eta > 0.f) return launch_norm_scale(gw, n, eta, 1e-12f, ws, s);
-    return ADDER_OK;
-}
+template int launch_grad_w<float>(const float *, const float *, const float *, float *, float, void *, size_t, const ConvDims &,
+                                  hipStream_t, const float *, const float *, float *, const BnSums &);
+template int launch_grad_w<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *, size_t,
+                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &);
 
 // ---- staged weight gradient: partial slabs now, finalize + scaling for many layers later --------------
 int launch_grad_w_staged(const float *gy, const float *x, const float *w, float *gw, float eta, void *ws,

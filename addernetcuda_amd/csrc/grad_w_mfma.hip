@@ -471,20 +471,6 @@ static int launch_one(const T *gy, const T *x, double *part, double *sgpart, con
     return launch_one_v<G, false, false, T>(gy, x, part, sgpart, d, p, s);
 }
 
-// bfloat16 storage of gy and x: the 3x3 / pad-1 variants (1..5 of the plan)
-int launch_grad_w_mfma_bf16(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d,
-                            const GradWMfmaPlan &p, hipStream_t s) {
-    switch (p.variant) {
-        case 1: return launch_one<GmW32, bf16_t>(gy, x, part, sgpart, d, p, s);
-        case 2: return launch_one<GmW16, bf16_t>(gy, x, part, sgpart, d, p, s);
-        case 3: return launch_one<GmW8, bf16_t>(gy, x, part, sgpart, d, p, s);
-        case 4: return launch_one<GmW16S2, bf16_t>(gy, x, part, sgpart, d, p, s);
-        case 5: return launch_one<GmW8S2, bf16_t>(gy, x, part, sgpart, d, p, s);
-        case 14: return launch_one<GmW32K32, bf16_t>(gy, x, part, sgpart, d, p, s);
-        default: return ADDER_ERR_UNSUPPORTED;
-    }
-}
-
 // The 3x3 / pad-1 and the stride-1 1x1 variants with gy formed from (dz = gy, bn_y, bn_coef) while it is staged and
 // left in gy_out (nullable) on the way (see gy_commit_m_bn); ADDER_ERR_UNSUPPORTED for other variants and for rows
 // (planes, for 1x1 layers) that are not whole float4 groups.
@@ -516,8 +502,9 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
     }
 }
 
-int launch_grad_w_mfma(const float *gy, const float *x, double *part, double *sgpart, const ConvDims &d,
-                       const GradWMfmaPlan &p, hipStream_t s) {
+template <class T>
+int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p,
+                       hipStream_t s) {
     switch (p.variant) {
         case 1: return launch_one<GmW32>(gy, x, part, sgpart, d, p, s);
         case 2: return launch_one<GmW16>(gy, x, part, sgpart, d, p, s);
@@ -531,15 +518,15 @@ int launch_grad_w_mfma(const float *gy, const float *x, double *part, double *sg
         case 11: {
             const ConvDims f = mfma_one_row(d);
             const Subsample sub{d.stride, d.Wo, d.W, d.H * d.W};
-            return f.Wo % 4 == 0 ? launch_one_v<Gm1x1b, true, true>(gy, x, part, sgpart, f, p, s, sub)
-                                 : launch_one_v<Gm1x1b, false, true>(gy, x, part, sgpart, f, p, s, sub);
+            return f.Wo % 4 == 0 ? launch_one_v<Gm1x1b, true, true, T>(gy, x, part, sgpart, f, p, s, sub)
+                                 : launch_one_v<Gm1x1b, false, true, T>(gy, x, part, sgpart, f, p, s, sub);
         }
         case 12: return launch_one<Gm1x1c>(gy, x, part, sgpart, mfma_one_row(d), p, s);
         case 13: {
             const ConvDims f = mfma_one_row(d);
             const Subsample sub{d.stride, d.Wo, d.W, d.H * d.W};
-            return f.Wo % 4 == 0 ? launch_one_v<Gm1x1c, true, true>(gy, x, part, sgpart, f, p, s, sub)
-                                 : launch_one_v<Gm1x1c, false, true>(gy, x, part, sgpart, f, p, s, sub);
+            return f.Wo % 4 == 0 ? launch_one_v<Gm1x1c, true, true, T>(gy, x, part, sgpart, f, p, s, sub)
+                                 : launch_one_v<Gm1x1c, false, true, T>(gy, x, part, sgpart, f, p, s, sub);
         }
         case 8:
         case 9: {
@@ -547,13 +534,17 @@ int launch_grad_w_mfma(const float *gy, const float *x, double *part, double *sg
             const Subsample sub{d.stride, d.Wo, d.W, d.H * d.W};
             const bool vec = f.Wo % 4 == 0;
             if (p.variant == 8)
-                return vec ? launch_one_v<Gm1x1, true, true>(gy, x, part, sgpart, f, p, s, sub)
-                           : launch_one_v<Gm1x1, false, true>(gy, x, part, sgpart, f, p, s, sub);
-            return vec ? launch_one_v<Gm1x1s, true, true>(gy, x, part, sgpart, f, p, s, sub)
-                       : launch_one_v<Gm1x1s, false, true>(gy, x, part, sgpart, f, p, s, sub);
+                return vec ? launch_one_v<Gm1x1, true, true, T>(gy, x, part, sgpart, f, p, s, sub)
+                           : launch_one_v<Gm1x1, false, true, T>(gy, x, part, sgpart, f, p, s, sub);
+            return vec ? launch_one_v<Gm1x1s, true, true, T>(gy, x, part, sgpart, f, p, s, sub)
+                       : launch_one_v<Gm1x1s, false, true, T>(gy, x, part, sgpart, f, p, s, sub);
         }
         default: return ADDER_ERR_BAD_SHAPE;
     }
 }
+template int launch_grad_w_mfma<float>(const float *, const float *, double *, double *, const ConvDims &, const GradWMfmaPlan &,
+                                       hipStream_t);
+template int launch_grad_w_mfma<bf16_t>(const bf16_t *, const bf16_t *, double *, double *, const ConvDims &,
+                                        const GradWMfmaPlan &, hipStream_t);
 
 }  // namespace adder

@@ -1061,36 +1061,36 @@ static_assert(GxW32::TM == GxW16::TM && GxW16::TM == GxW8::TM && GxS2W32::TM == 
 
 // gadd (nullable): a tensor shaped like gx that is added to the result (tiled 3x3 / pad 1 kernels and the tiled
 // 1x1 stride-1 kernels only; ADDER_ERR_UNSUPPORTED elsewhere)
-int launch_grad_x(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d,
-                  hipStream_t s, const float *gadd) {
+// Both storage types take the same kernels and tile shapes.  (bfloat16 layers other than 3x3 once went to the generic
+// kernel: 128 -> 512 1x1 @28x28, 32 images, 845 us.)
+template <class T>
+int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
     const bool k3s1p1 = d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1;
-    if (k3s1p1 && d.Ci >= GxW32::TM &&
-        (d.W % 4 != 0 || ((reinterpret_cast<uintptr_t>(gy) | reinterpret_cast<uintptr_t>(gx) |
-                           reinterpret_cast<uintptr_t>(gadd)) & 15) == 0)) {
+    const bool aligned = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
+    if (k3s1p1 && d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned)) {
         if (d.W > 16) switch (rows_per_tile_w32(d.H)) {
-            case 16: return launch_grad_x_3x3s1<GxW32>(gy, x, w, gx, d, s, gadd);
-            case 8: return launch_grad_x_3x3s1<GxW32H8>(gy, x, w, gx, d, s, gadd);
-            default: return launch_grad_x_3x3s1<GxW32H4>(gy, x, w, gx, d, s, gadd);
+            case 16: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
+            case 8: return launch_grad_x_3x3s1<GxW32H8, false, T>(gy, x, w, gx, d, s, gadd);
+            default: return launch_grad_x_3x3s1<GxW32H4, false, T>(gy, x, w, gx, d, s, gadd);
         }
-        if (d.W > 8) return launch_grad_x_3x3s1<GxW16>(gy, x, w, gx, d, s, gadd);
-        return launch_grad_x_3x3s1<GxW8>(gy, x, w, gx, d, s, gadd);
+        if (d.W > 8) return launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
+        return launch_grad_x_3x3s1<GxW8, false, T>(gy, x, w, gx, d, s, gadd);
     }
     if (d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM &&
-        (d.Wo % 4 != 0 || (reinterpret_cast<uintptr_t>(gy) & 15) == 0) &&
-        ((reinterpret_cast<uintptr_t>(gx) | reinterpret_cast<uintptr_t>(gadd)) & 7) == 0) {
-        if (d.W > 16) return launch_grad_x_3x3s2<GxS2W32>(gy, x, w, gx, d, s, gadd);
-        return launch_grad_x_3x3s2<GxS2W16>(gy, x, w, gx, d, s, gadd);
+        (d.Wo % 4 != 0 || aligned_groups(gy)) &&
+        ((reinterpret_cast<uintptr_t>(gx) | reinterpret_cast<uintptr_t>(gadd)) & (2 * sizeof(T) - 1)) == 0) {
+        if (d.W > 16) return launch_grad_x_3x3s2<GxS2W32, T>(gy, x, w, gx, d, s, gadd);
+        return launch_grad_x_3x3s2<GxS2W16, T>(gy, x, w, gx, d, s, gadd);
     }
     // (from 48 output channels on the tiled kernel is ahead of the plain one: DenseNet's 48-channel bottlenecks)
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride == 1 && d.Ci >= 64 && d.Co >= 48) {
         ConvDims f = d;   // every (H, W) plane as one row of H*W positions
         f.H = f.Ho = 1;
         f.W = f.Wo = d.H * d.W;
-        if (f.W % 4 != 0 || ((reinterpret_cast<uintptr_t>(gy) | reinterpret_cast<uintptr_t>(gx) |
-                              reinterpret_cast<uintptr_t>(gadd)) & 15) == 0) {
-            if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1>(gy, x, w, gx, f, s, gadd);
-            return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t>(gy, x, w, gx, f, s, gadd)
-                                       : launch_grad_x_3x3s1<Gx1x1s>(gy, x, w, gx, f, s, gadd);
+        if (f.W % 4 != 0 || aligned) {
+            if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, false, T>(gy, x, w, gx, f, s, gadd);
+            return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, false, T>(gy, x, w, gx, f, s, gadd)
+                                       : launch_grad_x_3x3s1<Gx1x1s, false, T>(gy, x, w, gx, f, s, gadd);
         }
     }
     if (gadd) return ADDER_ERR_UNSUPPORTED;
@@ -1100,20 +1100,25 @@ int launch_grad_x(const float *gy, const float *x, const float *w, float *gx, co
         f.W = f.Wo = d.Ho * d.Wo;
         f.stride = 1;
         const Subsample sub{d.stride, d.Wo, d.W, d.H * d.W};
-        if (f.W % 4 != 0 || (reinterpret_cast<uintptr_t>(gy) & 15) == 0) {
-            if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, true>(gy, x, w, gx, f, s, (const float *)nullptr, sub);
-            return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, true>(gy, x, w, gx, f, s, (const float *)nullptr, sub)
-                                       : launch_grad_x_3x3s1<Gx1x1s, true>(gy, x, w, gx, f, s, (const float *)nullptr, sub);
+        const T *none = nullptr;
+        if (f.W % 4 != 0 || aligned_groups(gy)) {
+            if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, true, T>(gy, x, w, gx, f, s, none, sub);
+            return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, true, T>(gy, x, w, gx, f, s, none, sub)
+                                       : launch_grad_x_3x3s1<Gx1x1s, true, T>(gy, x, w, gx, f, s, none, sub);
         }
     }
     if (conv1x1_supported(d, gy, gx))
         return launch_grad_x_1x1(gy, x, w, gx, d, s);
     constexpr int TM = 8;
     const long total = (long)d.N * d.H * d.W;
-    hipLaunchKernelGGL(grad_x_generic_kernel<TM>, dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Ci, TM)),
+    hipLaunchKernelGGL((grad_x_generic_kernel<TM, T>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Ci, TM)),
                        dim3(256), 0, s, gy, x, w, gx, d);
     return check_launch();
 }
+template int launch_grad_x<float>(const float *, const float *, const float *, float *, const ConvDims &, hipStream_t,
+                                  const float *);
+template int launch_grad_x<bf16_t>(const bf16_t *, const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t,
+                                   const bf16_t *);
 
 // a 1x1 stride-1 layer seen as images of one row of H * W positions
 static ConvDims one_row(const ConvDims &d) {
@@ -1185,28 +1190,6 @@ int launch_grad_x_bn(const float *gy, const float *x, const float *w, float *gx,
         case 8: return launch_grad_x_3x3s1_bn<Gx1x1s>(gy, x, w, gx, one_row(d), s, gadd, bn);
         default: return ADDER_ERR_UNSUPPORTED;
     }
-}
-
-// bfloat16 storage: the tiled 3x3 / pad-1 kernels (stride 1 or 2), the generic kernel for everything else
-int launch_grad_x_bf16(const bf16_t *gy, const bf16_t *x, const float *w, bf16_t *gx, const ConvDims &d,
-                       hipStream_t s) {
-    const bf16_t *none = nullptr;
-    if (d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1 && d.Ci >= GxW32::TM &&
-        (d.W % 4 != 0 || ((reinterpret_cast<uintptr_t>(gy) | reinterpret_cast<uintptr_t>(gx)) & 7) == 0)) {
-        if (d.W > 16) return launch_grad_x_3x3s1<GxW32, false, bf16_t>(gy, x, w, gx, d, s, none);
-        if (d.W > 8) return launch_grad_x_3x3s1<GxW16, false, bf16_t>(gy, x, w, gx, d, s, none);
-        return launch_grad_x_3x3s1<GxW8, false, bf16_t>(gy, x, w, gx, d, s, none);
-    }
-    if (d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM &&
-        (d.Wo % 4 != 0 || (reinterpret_cast<uintptr_t>(gy) & 7) == 0) && (reinterpret_cast<uintptr_t>(gx) & 3) == 0) {
-        if (d.W > 16) return launch_grad_x_3x3s2<GxS2W32, bf16_t>(gy, x, w, gx, d, s, none);
-        return launch_grad_x_3x3s2<GxS2W16, bf16_t>(gy, x, w, gx, d, s, none);
-    }
-    constexpr int TM = 8;
-    const long total = (long)d.N * d.H * d.W;
-    hipLaunchKernelGGL((grad_x_generic_kernel<TM, bf16_t>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Ci, TM)),
-                       dim3(256), 0, s, gy, x, w, gx, d);
-    return check_launch();
 }
 
 }  // namespace adder

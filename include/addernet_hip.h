@@ -149,8 +149,8 @@ ADDER_API int adder_conv2d_bwd_add_f32(const float *gy, const float *x, const fl
  * activation memory; weights and weight gradients stay fp32, every sum is accumulated as in the fp32 entry points
  * (fp32 for y and gx, fp64 for gw).  The reference computes in fp32 only (adder.cu:310-318 hard-codes
  * data<float>()), so these have no counterpart there and are never the default.  Same dimensions, semantics, eta
- * and workspace (adder_conv2d_bwd_workspace_bytes) as adder_conv2d_fwd_f32 / adder_conv2d_bwd_f32.  3x3 / pad 1
- * layers (stride 1 or 2) run on the tiled kernels, everything else on the generic ones. */
+ * and workspace (adder_conv2d_bwd_workspace_bytes) as adder_conv2d_fwd_f32 / adder_conv2d_bwd_f32, and the same
+ * kernels and tile shapes. */
 typedef unsigned short adder_bf16;
 ADDER_API int adder_conv2d_fwd_bf16(const adder_bf16 *x, const float *w, adder_bf16 *y,
                          int N, int Ci, int H, int W, int Co, int kh, int kw,
