@@ -217,7 +217,7 @@ int adder_conv2d_bwd_workspace_bytes(int N, int Ci, int H, int W, int Co, int kh
 
 static int conv2d_bwd(const float *gy, const float *x, const float *w, const float *gx_add, float *gx, float *gw,
                       float eta, void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
-                      int stride, int pad, void *stream);
+                      int stride, int pad, void *stream, bool general = false);
 
 int adder_conv2d_bwd_f32(const float *gy, const float *x, const float *w, float *gx, float *gw, float eta,
                          void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
@@ -234,7 +234,7 @@ int adder_conv2d_bwd_add_f32(const float *gy, const float *x, const float *w, co
 
 static int conv2d_bwd(const float *gy, const float *x, const float *w, const float *gx_add, float *gx, float *gw,
                       float eta, void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
-                      int stride, int pad, void *stream) {
+                      int stride, int pad, void *stream, bool general) {
     if (!gy || !x || !w) return ADDER_ERR_NULL_POINTER;
     if (!gx && !gw) return ADDER_ERR_NULL_POINTER;
     if (!(eta >= 0.f)) return ADDER_ERR_BAD_SHAPE;
@@ -248,7 +248,7 @@ static int conv2d_bwd(const float *gy, const float *x, const float *w, const flo
         return ADDER_ERR_ALIAS;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (gw) {
-        const size_t need = grad_w_workspace_bytes(d);
+        const size_t need = general ? kGradWGeneralWs : grad_w_workspace_bytes(d);
         if (!ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255)) return ADDER_ERR_WORKSPACE;
         if (overlaps(ws, need, x, nx) || overlaps(ws, need, w, nw) || overlaps(ws, need, gy, ny) ||
             overlaps(ws, need, gx, nx) || overlaps(ws, need, gw, nw) || overlaps(ws, need, gx_add, nx))
@@ -257,7 +257,9 @@ static int conv2d_bwd(const float *gy, const float *x, const float *w, const flo
     if (gx)
         if (int rc = launch_grad_x(gy, x, w, gx, d, s, gx_add)) return rc;
     if (gw)
-        if (int rc = launch_grad_w(gy, x, w, gw, eta, ws, ws_bytes, d, s)) return rc;
+        if (int rc = general ? launch_grad_w_general(gy, x, w, gw, eta, ws, d, s)
+                             : launch_grad_w(gy, x, w, gw, eta, ws, ws_bytes, d, s))
+            return rc;
     return ADDER_OK;
 }
 
@@ -309,13 +311,16 @@ int adder_conv2d_bwd_noalloc_f32(const float *gy, const float *x, const float *w
     if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
     void *ws = nullptr;
     size_t need = 0;
+    bool general = false;
     if (gw) {   // only the weight gradient uses scratch
         need = grad_w_workspace_bytes(d);
-        if (need > ADDER_NOALLOC_SCRATCH_BYTES) return ADDER_ERR_WORKSPACE;   // before any HIP call
+        // 5x5 layers whose slabs do not fit have the general kernel, which needs none; other layers are refused
+        general = need > ADDER_NOALLOC_SCRATCH_BYTES && kh == 5 && kw == 5;
+        if (need > ADDER_NOALLOC_SCRATCH_BYTES && !general) return ADDER_ERR_WORKSPACE;   // before any HIP call
         if (int rc = scratch_of_current_device(&ws)) return rc;
     }
     // every kernel writes the part of the scratch it later reads (slabs, norm partials): nothing to clear
-    return conv2d_bwd(gy, x, w, nullptr, gx, gw, eta, ws, need, N, Ci, H, W, Co, kh, kw, stride, pad, stream);
+    return conv2d_bwd(gy, x, w, nullptr, gx, gw, eta, ws, need, N, Ci, H, W, Co, kh, kw, stride, pad, stream, general);
 }
 
 static int check_col(int K, long NL, int Co) {

@@ -262,6 +262,11 @@ template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                   void *ws, size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y = nullptr,
                   const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums);
+// launch_grad_w without slabs (any layer): `ws` holds the norm partials only, kGradWGeneralWs bytes
+static constexpr size_t kGradWGeneralWs = 128 * 1024;
+template <class T>
+int launch_grad_w_general(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws, const ConvDims &d,
+                          hipStream_t s);
 // the BatchNorm backward passes of a layer's neighbours inside the layer's backward kernels (adder_bn_links)
 int grad_x_bn_slots(const ConvDims &d);
 int launch_grad_x_bn(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d, hipStream_t s,
@@ -270,7 +275,7 @@ bool grad_w_bn_supported(const ConvDims &d, const void *gy, const void *x, const
 int launch_bn_bwd_coef(const float *part, int slots, const float *gamma, const float *mean, const float *rstd,
                        double count, float *coef, float *dgamma, float *dbeta, int C, hipStream_t s);
 
-// matrix-core weight gradient of the 3x3 / pad-1 layers (grad_w_mfma.hip); variant 0 = not applicable
+// matrix-core weight gradient of the 3x3 / pad-1, 5x5 / pad-2 and wide 1x1 layers (grad_w_mfma.hip); variant 0 = not applicable
 struct GradWMfmaPlan { int variant, slots, gy, gz, tilesH, tilesW, ntiles; };
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d);
 template <class T>

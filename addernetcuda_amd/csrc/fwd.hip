@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void fwd_generic_kernel(const T *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Tiled kernel for 3x3, pad 1, stride S = 1 or 2.
+// Tiled kernel for 3x3 / pad 1 and 5x5 / pad 2, stride S = 1 or 2 (the figures are the 3x3 ones).
 //
 // A workgroup owns NIMG images x a TH x TW patch of output positions and
 // TM*COW output channels.  TW = TN*SPR: each lane owns a strip of TN adjacent
@@ -414,6 +414,15 @@ using Fwd1x1sq = Tile3x3Cfg<4, 16, 1, 4, 4, 8, 16, 4, 1, 1>;
 // 128 -> 128 @28x28 330 -> 298 us); on 32 rows they are no faster than FwdW32
 using FwdW32H8 = Tile3x3Cfg<4, 8, 8, 1, 4, 4, 8, 1, 1>;    // 8 rows of one image x 16 channels
 using FwdW32H4 = Tile3x3Cfg<4, 8, 4, 2, 4, 4, 8, 1, 1>;    // 4 rows of two images x 16 channels
+// 5x5 taps: a unit is one output channel x one input channel as well (25 weights, 50*TN vector instructions); five
+// strips of eight values per buffer leave room for two output channels per lane.  Two vector instructions per term
+// bound it: 32 -> 64 @16x16, 64 images (0.84e9 terms, 27 us at the issue ceiling): generic kernel 247 us, this 40 us.
+using Fwd5W32   = Tile3x3Cfg<4, 8, 8, 1, 2, 8, 8, 1, 1, 5>;     // 8 rows of one image x 16 channels
+using Fwd5W16   = Tile3x3Cfg<4, 4, 16, 1, 2, 8, 8, 1, 1, 5>;    // outputs 9..16 wide: one image x 16 channels
+using Fwd5W8    = Tile3x3Cfg<4, 2, 8, 4, 2, 8, 8, 1, 1, 5>;     // outputs up to 8 wide: four images x 16 channels
+using Fwd5W16S2 = Tile3x3Cfg<2, 8, 8, 1, 2, 8, 8, 1, 2, 5>;     // stride 2: 8 rows x 16 outputs of one image
+using Fwd5W8S2  = Tile3x3Cfg<2, 4, 8, 2, 2, 8, 8, 1, 2, 5>;     // stride 2, outputs up to 8 wide: two images
+
 // rows per tile (16, 8 or 4) that pad a map of H rows least; the larger tile on a tie
 static int rows_per_tile_w32(int H) {
     const int p16 = round_up(H, 16), p8 = round_up(H, 8), p4 = round_up(H, 4);
@@ -422,7 +431,7 @@ static int rows_per_tile_w32(int H) {
 
 // which tiled kernel serves these dimensions (0 = none): 1..3 3x3 stride 1 by output width, 4..5 3x3 stride 2,
 // 6..7 1x1 stride 1 by plane size, 8..9 1x1 with a stride (the sampled positions walked like a stride-1 plane),
-// 10..13 = 6..9 with units of four input channels
+// 10..13 = 6..9 with units of four input channels, 14..18 5x5 (stride 1 by output width, then stride 2)
 static int fwd_tiled_variant(const ConvDims &d) {
     // (below 64 input channels the plain 1x1 kernel of conv1x1.hip is as fast or faster)
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci % Fwd1x1q::CQ == 0 && d.Ci >= 64) {
@@ -433,6 +442,11 @@ static int fwd_tiled_variant(const ConvDims &d) {
         const bool wide = ceil_div(plane, Fwd1x1::TW) * Fwd1x1::TW <= ceil_div(plane, Fwd1x1s::TW) * Fwd1x1s::TW;
         if (d.stride == 1) return (wide ? 6 : 7) + quad;
         return (wide ? 8 : 9) + quad;
+    }
+    if (d.kh == 5 && d.kw == 5 && d.pad == 2) {
+        if (d.stride == 1) return d.Wo > 16 ? 14 : (d.Wo > 8 ? 15 : 16);
+        if (d.stride == 2) return d.Wo > 8 ? 17 : 18;
+        return 0;
     }
     if (d.kh != 3 || d.kw != 3 || d.pad != 1) return 0;
     if (d.stride == 1) return d.Wo > 16 ? 1 : (d.Wo > 8 ? 2 : 3);
@@ -507,8 +521,7 @@ int fwd_stats_slots(const ConvDims &d) {
 template <class T>
 int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s) {
     // rows that are whole groups of four are moved as such and need bases aligned to a group
-    const bool k3p1 = d.kh == 3 && d.kw == 3 && d.pad == 1 && (d.W % 4 != 0 || aligned_groups(x)) &&
-                      (d.Wo % 4 != 0 || aligned_groups(y));
+    const bool rows_ok = (d.W % 4 != 0 || aligned_groups(x)) && (d.Wo % 4 != 0 || aligned_groups(y));
     const int variant = fwd_tiled_variant(d);
     const bool strided = variant == 8 || variant == 9 || variant == 12 || variant == 13;
     if (strided) {   // x is read element by element; y is a dense row per plane
@@ -518,7 +531,7 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
             case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d));
             default: return launch_fwd_3x3_v<Fwd1x1sq, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d));
         }
-    } else if (variant >= 6) {
+    } else if (variant >= 6 && variant <= 11) {
         const ConvDims f = as_one_row(d);
         if (f.W % 4 != 0 || (aligned_groups(x) && aligned_groups(y))) switch (variant) {
             case 6: return launch_fwd_3x3<Fwd1x1>(x, w, y, stats, f, s);
@@ -527,7 +540,7 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
             default: return launch_fwd_3x3<Fwd1x1sq>(x, w, y, stats, f, s);
         }
     }
-    if (k3p1) {
+    if (rows_ok && !(stats && variant >= 14)) {   // 3x3 and 5x5 taps; statistics are offered for 3x3 and 1x1 layers
         switch (variant) {
             case 1: switch (rows_per_tile_w32(d.Ho)) {
                 case 16: return launch_fwd_3x3<FwdW32>(x, w, y, stats, d, s);
@@ -539,6 +552,11 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
             case 4: return launch_fwd_3x3<FwdW16S2>(x, w, y, stats, d, s);
             case 5: return d.Ci >= 128 ? launch_fwd_3x3<FwdW8S2L>(x, w, y, stats, d, s)
                                        : launch_fwd_3x3<FwdW8S2>(x, w, y, stats, d, s);
+            case 14: return launch_fwd_3x3<Fwd5W32>(x, w, y, stats, d, s);
+            case 15: return launch_fwd_3x3<Fwd5W16>(x, w, y, stats, d, s);
+            case 16: return launch_fwd_3x3<Fwd5W8>(x, w, y, stats, d, s);
+            case 17: return launch_fwd_3x3<Fwd5W16S2>(x, w, y, stats, d, s);
+            case 18: return launch_fwd_3x3<Fwd5W8S2>(x, w, y, stats, d, s);
             default: break;
         }
     }

@@ -15,6 +15,7 @@
 namespace adder {
 
 static constexpr int kNormBlocksMax = 16384;  // sum-of-squares partials kept at the head of the workspace
+static_assert(kGradWGeneralWs == sizeof(double) * kNormBlocksMax, "the general path needs these partials and nothing else");
 
 // ---------------------------------------------------------------------------
 // Generic kernel: one workgroup per (co, ci) [KH x KW taps in registers] or,
@@ -427,6 +428,12 @@ int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
         if (rc || fused_norm || !(eta > 0.f)) return rc;
         return launch_norm_scale(gw, n, eta, 1e-12f, ws, s);
     }
+    return launch_grad_w_general(gy, x, w, gw, eta, ws, d, s);
+}
+
+template <class T>
+int launch_grad_w_general(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws, const ConvDims &d,
+                          hipStream_t s) {
     const int KK = d.kh * d.kw;
     const long wgs = (long)d.Co * d.Ci;
     if (d.kh == 3 && d.kw == 3)
@@ -438,9 +445,13 @@ int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                            gw, d);
     int rc = check_launch();
     if (rc) return rc;
-    if (eta > 0.f) return launch_norm_scale(gw, n, eta, 1e-12f, ws, s);
+    if (eta > 0.f) return launch_norm_scale(gw, wgs * KK, eta, 1e-12f, ws, s);
     return ADDER_OK;
 }
+template int launch_grad_w_general<float>(const float *, const float *, const float *, float *, float, void *, const ConvDims &,
+                                          hipStream_t);
+template int launch_grad_w_general<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *,
+                                           const ConvDims &, hipStream_t);
 template int launch_grad_w<float>(const float *, const float *, const float *, float *, float, void *, size_t, const ConvDims &,
                                   hipStream_t, const float *, const float *, float *, const BnSums &);
 template int launch_grad_w<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *, size_t,

@@ -1,4 +1,4 @@
-// Weight gradient of the AdderNet convolution (3x3 / pad 1, or 1x1 / stride 1) on the matrix cores, in full precision.
+// Weight gradient of the AdderNet convolution (3x3 / pad 1, 5x5 / pad 2, or 1x1) on the matrix cores, in full precision.
 //
 //   gw[co,k] = sum_pos xcol[k,pos] * gy[co,pos]  -  w[co,k] * sum_pos gy[co,pos]      (k = (ci, i, j))
 //
@@ -30,7 +30,7 @@ typedef double double4v __attribute__((ext_vector_type(4)));
 template <int S_, int TH_, int TW_, int NIMG_, int MT_, int NT_, int MW_, int NW_, int PW_, int KS_ = 3>
 struct GwMfmaCfg {
     static constexpr int S = S_, TH = TH_, TW = TW_, NIMG = NIMG_, MT = MT_, NT = NT_, MW = MW_, NW = NW_, PW = PW_;
-    static constexpr int KS = KS_, KK = KS_ * KS_, PAD = KS_ / 2;   // 3x3 taps with pad 1, or a single tap
+    static constexpr int KS = KS_, KK = KS_ * KS_, PAD = KS_ / 2;   // 3x3 / pad 1, 5x5 / pad 2, or a single tap
     static constexpr int COB = 16 * MT * MW;          // output channels per workgroup
     static constexpr int KB = 16 * NT * NW;           // k columns per workgroup
     static constexpr int CIB = ceil_div(KB, KK);      // input channels per workgroup (staged)
@@ -39,8 +39,8 @@ struct GwMfmaCfg {
     static constexpr bool WHOLE = KB % KK == 0;
     static constexpr int NWAVES = MW * NW * PW;
     static constexpr int NTHREADS = 64 * NWAVES;
-    // LPAD puts the interior columns on a 16-byte boundary (3 + one halo column, or no halo at all)
-    using XP = PatchCfg<NIMG, CIB, (TH - 1) * S + KS, TW * S, PAD, (S == 1) ? PAD : 0, NTHREADS, PAD ? 3 : 0>;
+    // LPAD puts the interior columns on a 16-byte boundary (3 + one halo column, 2 + two, or no halo at all)
+    using XP = PatchCfg<NIMG, CIB, (TH - 1) * S + KS, TW * S, PAD, S == 1 || PAD == 0 ? PAD : PAD - 1, NTHREADS, (4 - PAD) % 4>;
     static constexpr int GPLANE = TH * TW + 4;        // +4: channel planes start 4 banks apart
     static constexpr int GBUF = NIMG * COB * GPLANE;
     static constexpr int GUNITS = NIMG * COB * TH * TW / 4;
@@ -383,6 +383,13 @@ using GmW8S2  = GwMfmaCfg<2, 8, 8, 2, 1, 3, 1, 3, 4>;    // stride 2, outputs 8 
 // all of K, eight position waves.  Through the 144-column block above, four fifths of the matrix instructions of
 // such a layer multiply staged zeros: 28 us for 0.23 GFLOP.
 using GmW32K32 = GwMfmaCfg<1, 8, 32, 1, 1, 2, 1, 1, 8>;
+// 5x5: 16 output x 16 input channels again, K = 400 columns as five k waves of five tiles, two position waves.
+// (32 -> 64 @16x16, 64 images, 1.7 GFLOP fp64 = 21 us at the matrix peak: generic kernel 1475 us, this 45 us.)
+using Gm5W32   = GwMfmaCfg<1, 8, 32, 1, 1, 5, 1, 5, 2, 5>;
+using Gm5W16   = GwMfmaCfg<1, 16, 16, 1, 1, 5, 1, 5, 2, 5>;
+using Gm5W8    = GwMfmaCfg<1, 8, 8, 2, 1, 5, 1, 5, 2, 5>;
+using Gm5W16S2 = GwMfmaCfg<2, 8, 16, 1, 1, 5, 1, 5, 2, 5>;
+using Gm5W8S2  = GwMfmaCfg<2, 8, 8, 1, 1, 5, 1, 5, 2, 5>;
 // 1x1, stride 1: a plain (Co x positions) x (positions x Ci) product; (H, W) planes walked as one row.
 // 64 output channels x 64 input channels per workgroup (two k waves with eight accumulator tiles each, times four
 // position waves), 128 positions per staged tile; every wave does eight steps of 8 MFMAs on 4 + 2 LDS reads per tile.
@@ -432,6 +439,17 @@ GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d) {
         p.variant = (f.W > 64 ? 6 : 7) + (d.stride > 1 ? 2 : 0);   // 8, 9: x sampled likewise
         if (f.W > 64) plan_one<Gm1x1>(f, p);
         else plan_one<Gm1x1s>(f, p);
+        return p;
+    }
+    if (d.kh == 5 && d.kw == 5 && d.pad == 2 && d.stride <= 2) {
+        p.variant = d.stride == 1 ? (d.Wo > 16 ? 15 : (d.Wo > 8 ? 16 : 17)) : (d.Wo > 8 ? 18 : 19);
+        switch (p.variant) {
+            case 15: plan_one<Gm5W32>(d, p); break;
+            case 16: plan_one<Gm5W16>(d, p); break;
+            case 17: plan_one<Gm5W8>(d, p); break;
+            case 18: plan_one<Gm5W16S2>(d, p); break;
+            default: plan_one<Gm5W8S2>(d, p); break;
+        }
         return p;
     }
     const bool ok = d.kh == 3 && d.kw == 3 && d.pad == 1;
@@ -512,6 +530,11 @@ int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, co
         case 4: return launch_one<GmW16S2>(gy, x, part, sgpart, d, p, s);
         case 5: return launch_one<GmW8S2>(gy, x, part, sgpart, d, p, s);
         case 14: return launch_one<GmW32K32>(gy, x, part, sgpart, d, p, s);
+        case 15: return launch_one<Gm5W32>(gy, x, part, sgpart, d, p, s);
+        case 16: return launch_one<Gm5W16>(gy, x, part, sgpart, d, p, s);
+        case 17: return launch_one<Gm5W8>(gy, x, part, sgpart, d, p, s);
+        case 18: return launch_one<Gm5W16S2>(gy, x, part, sgpart, d, p, s);
+        case 19: return launch_one<Gm5W8S2>(gy, x, part, sgpart, d, p, s);
         case 6: return launch_one<Gm1x1>(gy, x, part, sgpart, mfma_one_row(d), p, s);
         case 7: return launch_one<Gm1x1s>(gy, x, part, sgpart, mfma_one_row(d), p, s);
         case 10: return launch_one<Gm1x1b>(gy, x, part, sgpart, mfma_one_row(d), p, s);

@@ -91,12 +91,12 @@ __global__ __launch_bounds__(256) void grad_x_generic_kernel(const T *__restrict
 }
 
 // ---------------------------------------------------------------------------
-// Tiled kernel for 3x3, stride 1, pad 1.  Same tile geometry as the forward
+// Tiled kernel for 3x3 / pad 1 and 5x5 / pad 2, stride 1 (and single taps).  Same tile geometry as the forward
 // kernel with the roles swapped: the LDS tile holds gy (chunks of CC output
 // channels, reduction axis), a lane owns TN input positions x TM input
 // channels, COW wave groups take different input channels.
-//   gx[hi,wi] += hardtanh(w[co,ci,i,j] - x[hi,wi]) * gy[hi+1-i, wi+1-j]
-// In tile coordinates (row 0 = h0-1, column 0 = w0-1) that is row+2-i, t+2-j.
+//   gx[hi,wi] += hardtanh(w[co,ci,i,j] - x[hi,wi]) * gy[hi+p-i, wi+p-j]
+// In tile coordinates (row 0 = h0-p, column 0 = w0-p) that is row+2p-i, t+2p-j.
 // ---------------------------------------------------------------------------
 // SUB (single tap only): x and gx are sampled tensors (see Subsample); the kernel walks the sampled
 // positions as one row per plane, reads x there, and stores each result together with the zeros of the
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
             static_assert(CQ == 1, "this pipeline takes one output channel per step");
             // input channels per unit: keeps ~100 vector instructions per unit and both weight
             // buffers (2 * 9 * HM SGPRs) well inside the scalar register file
-            constexpr int HM = KS == 1 ? TM : (TN >= 4 ? 1 : 2), NU = TM / HM, HW = HM * KK;
+            constexpr int HM = KS == 1 ? TM : (KS == 5 || TN >= 4 ? 1 : 2), NU = TM / HM, HW = HM * KK;
             static_assert(TM % HM == 0 && (NU % 2 == 0 || NU == 1), "one unit or an even number of units per output channel");
             float gr[2][KS][TN + KS - 1];
             float wv[2][HW];
@@ -308,8 +308,8 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
                 if (cc + 1 < ccnt) one_channel(cc + 1, 1);
                 // the two-instruction form folds its first-level sums every eight output channels (72 terms): with
                 // 144-term first levels its worst element sat at 0.71 of the parity tolerance for 1152 terms per
-                // output, with 72-term ones at 0.51
-                if (SAT && KS == 3 && ((cc + 2) & 7) == 0 && cc + 2 < ccnt) {
+                // output, with 72-term ones at 0.51.  25 taps: both forms, every four channels (100 terms)
+                if ((KS == 5 ? ((cc + 2) & 3) == 0 : SAT && KS == 3 && ((cc + 2) & 7) == 0) && cc + 2 < ccnt) {
 #pragma unroll
                     for (int m = 0; m < TM; ++m)
 #pragma unroll
@@ -549,7 +549,10 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
 // the three-instruction form sits at 0.45, and at 0.54 for 4608.  Layers with more than 1152 terms per output
 // therefore keep the three-instruction form.  Single-tap layers stop at 1024: their chunks are CC terms long, not 9 * CC, so the second level of the
 // sum is long and carries the full magnitude (0.46 at 1024 with the first level folded every fourth chunk).
-static constexpr int kSatMaxTerms = 1152, kSatMaxTerms1x1 = 1024;
+// 5x5 layers (100-term first levels): relative error 2.7e-7 at 1150 terms, 2.9e-7 at 2500, where the kernel without tiles has 3.4e-7.
+static constexpr int kSatMaxTerms = 1152, kSatMaxTerms1x1 = 1024, kSatMaxTerms5x5 = 2500;
+template <class C>
+constexpr int sat_max_terms() { return C::KS == 1 ? kSatMaxTerms1x1 : (C::KS == 5 ? kSatMaxTerms5x5 : kSatMaxTerms); }
 
 static const adder_bn_links kNoLinks{};
 
@@ -573,7 +576,7 @@ static int launch_grad_x_3x3s1_v(const T *gy, const T *x, const float *w, T *gx,
 template <class C>
 static int launch_grad_x_3x3s1_bn(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d,
                                   hipStream_t s, const float *gadd, const adder_bn_links &bn) {
-    if (d.Co * C::KK > (C::KS == 1 ? kSatMaxTerms1x1 : kSatMaxTerms))
+    if (d.Co * C::KK > sat_max_terms<C>())
         return launch_grad_x_3x3s1_v<C, true, false, false, float, true>(gy, x, w, gx, d, s, Subsample{1, 0, 0, 0}, gadd, bn);
     return launch_grad_x_3x3s1_v<C, true, true, false, float, true>(gy, x, w, gx, d, s, Subsample{1, 0, 0, 0}, gadd, bn);
 }
@@ -585,7 +588,7 @@ static int launch_grad_x_3x3s1(const T *gy, const T *x, const float *w, T *gx,
                                const ConvDims &d, hipStream_t s, const T *gadd = nullptr,
                                const Subsample sub = Subsample{1, 0, 0, 0}) {
     const bool vec = d.W % 4 == 0;
-    if (d.Co * C::KK > (C::KS == 1 ? kSatMaxTerms1x1 : kSatMaxTerms))
+    if (d.Co * C::KK > sat_max_terms<C>())
         return vec ? launch_grad_x_3x3s1_v<C, true, false, SUB, T>(gy, x, w, gx, d, s, sub, gadd)
                    : launch_grad_x_3x3s1_v<C, false, false, SUB, T>(gy, x, w, gx, d, s, sub, gadd);
     return vec ? launch_grad_x_3x3s1_v<C, true, true, SUB, T>(gy, x, w, gx, d, s, sub, gadd)
@@ -1037,6 +1040,12 @@ using GxW32 = Tile3x3Cfg<4, 8, 16, 1, 4, 4, 8, 1>;    // inputs 32 wide: half an
 using GxW16 = Tile3x3Cfg<4, 4, 16, 1, 4, 8, 16, 1>;   // inputs 16 wide: one image x 32 channels
 using GxW8  = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 16, 1>;    // inputs 8 wide: two images x 32 channels
 // 1x1, stride 1: (H, W) planes walked as one row; a unit is one output channel x the lane's 8 input channels
+// 5x5 taps, two input channels x two positions per lane, so that a layer of a few dozen channels still has two waves per
+// SIMD: 32 -> 64 @16x16, 64 images (0.84e9 terms) generic kernel 529 us, this 62 us; four positions per lane 94 us (but
+// 128 -> 64 167 against 184 us: a chip with enough waves would rather have fewer LDS reads per term)
+using Gx5W32 = Tile3x3Cfg<2, 16, 8, 1, 2, 4, 8, 1, 1, 5>;   // 8 rows of one image x 8 channels
+using Gx5W16 = Tile3x3Cfg<2, 8, 16, 1, 2, 4, 8, 1, 1, 5>;   // inputs 9..16 wide: one image x 8 channels
+using Gx5W8  = Tile3x3Cfg<2, 4, 8, 4, 2, 4, 8, 1, 1, 5>;    // inputs up to 8 wide: four images x 8 channels
 using Gx1x1  = Tile3x3Cfg<2, 64, 1, 1, 8, 8, 16, 2, 1, 1>;    // 128 positions of one image x 64 channels
 using Gx1x1s = Tile3x3Cfg<4, 16, 1, 4, 8, 8, 16, 1, 1, 1>;    // planes of <= 64 positions: four images
 using Gx1x1t = Tile3x3Cfg<2, 32, 1, 2, 4, 8, 16, 8, 1, 1>;    // ... two images x 32 channels, where Gx1x1s would leave CUs idle
@@ -1059,7 +1068,7 @@ static int rows_per_tile_w32(int H) {
 static_assert(GxW32::TM == GxW16::TM && GxW16::TM == GxW8::TM && GxS2W32::TM == GxS2W16::TM,
               "the launcher checks Ci against one TM per stride");
 
-// gadd (nullable): a tensor shaped like gx that is added to the result (tiled 3x3 / pad 1 kernels and the tiled
+// gadd (nullable): a tensor shaped like gx that is added to the result (tiled 3x3 / pad 1, 5x5 / pad 2 / stride 1 and tiled
 // 1x1 stride-1 kernels only; ADDER_ERR_UNSUPPORTED elsewhere)
 // Both storage types take the same kernels and tile shapes.  (bfloat16 layers other than 3x3 once went to the generic
 // kernel: 128 -> 512 1x1 @28x28, 32 images, 845 us.)
@@ -1075,6 +1084,11 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         }
         if (d.W > 8) return launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
         return launch_grad_x_3x3s1<GxW8, false, T>(gy, x, w, gx, d, s, gadd);
+    }
+    if (d.kh == 5 && d.kw == 5 && d.stride == 1 && d.pad == 2 && d.Ci >= Gx5W32::TM && (d.W % 4 != 0 || aligned)) {
+        if (d.W > 16) return launch_grad_x_3x3s1<Gx5W32, false, T>(gy, x, w, gx, d, s, gadd);
+        if (d.W > 8) return launch_grad_x_3x3s1<Gx5W16, false, T>(gy, x, w, gx, d, s, gadd);
+        return launch_grad_x_3x3s1<Gx5W8, false, T>(gy, x, w, gx, d, s, gadd);
     }
     if (d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM &&
         (d.Wo % 4 != 0 || aligned_groups(gy)) &&

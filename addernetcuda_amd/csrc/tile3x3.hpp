@@ -1,5 +1,5 @@
-// Tile geometry and global->LDS staging shared by the tiled 3x3 / pad-1 kernels
-// (stride 1 or 2).  A workgroup covers NIMG images x TH x TW positions of the
+// Tile geometry and global->LDS staging shared by the tiled 3x3 / pad-1 and 5x5 / pad-2
+// kernels (stride 1 or 2; the figures below are the 3x3 ones).  A workgroup covers NIMG images x TH x TW positions of the
 // "lane space" (output positions for the forward and weight-gradient kernels,
 // input positions for the stride-1 input gradient) and stages, per channel, the
 // haloed patch of the source tensor those positions touch:
@@ -14,7 +14,7 @@ namespace adder {
 
 // A rectangular patch of an NCHW tensor staged per channel into LDS as
 // [img][cc][ROWS][PITCH]: ICOLS float4-aligned interior columns starting at LDS
-// column LPAD + LHALO, plus an optional single halo column on either side.  LPAD = 3 puts the
+// column LPAD + LHALO, plus up to two halo columns on either side.  LPAD = 3 puts the
 // interior on a 16-byte boundary (one ds_write_b128 per staged float4) for kernels whose reads
 // do not care about alignment; LPAD = 0 keeps a lane's strips aligned instead.
 template <int NIMG_, int CC_, int ROWS_, int ICOLS_, int LHALO_, int RHALO_, int NTHREADS_, int LPAD_ = 0>
@@ -32,8 +32,9 @@ struct PatchCfg {
     static constexpr int NUH = NIMG * CC * ROWS * NSIDES;
     static constexpr int HITER = NSIDES ? ceil_div(NUH, NTHREADS) : 0;
     static_assert(ICOLS % 4 == 0, "interior must cover whole float4 groups of the source");
-    static_assert(LHALO == 0 || LHALO == 1, "at most one halo column per side");
-    static_assert(RHALO == 0 || RHALO == 1, "at most one halo column per side");
+    static_assert(LHALO >= 0 && LHALO <= 2 && RHALO >= 0 && RHALO <= 2, "at most two halo columns per side");
+    // halo column `side` (the left ones first): its place relative to the first interior column
+    static __host__ __device__ constexpr int halo_col(int side) { return side < LHALO ? side - LHALO : ICOLS + side - LHALO; }
 };
 
 // A tensor that is read at every s-th row and column only (a strided single-tap layer): the kernels walk
@@ -102,12 +103,11 @@ __device__ __forceinline__ void tile_fetch(TileStage<P> &st, const T *__restrict
 #pragma unroll
     for (int it = 0; it < P::HITER; ++it) {
         const int u = tid + it * P::NTHREADS;
-        const int side = P::LHALO ? u % P::SIDE_DIV : 1;  // 0 = left, 1 = right
         const int rest = u / P::SIDE_DIV;
         const int r = rest % P::ROWS;
         const int cc = rest / P::ROWS % P::CC;
         const int img = rest / P::ROWS / P::CC;
-        const int n = n0 + img, ch = chan0 + cc, hi = hb + r, wi = side ? wb + P::ICOLS : wb - 1;
+        const int n = n0 + img, ch = chan0 + cc, hi = hb + r, wi = wb + P::halo_col(u % P::SIDE_DIV);
         const bool ok = (P::NUH % P::NTHREADS == 0 || u < P::NUH) && n < nimg_total && ch < nchan &&
                         hi >= 0 && hi < H && wi >= 0 && wi < W;
         st.h[it] = ok ? ldf(src + (((n * nchan + ch) * H + hi) * W + wi)) : 0.f;
@@ -136,14 +136,13 @@ __device__ __forceinline__ void tile_commit(const TileStage<P> &st, float *buf) 
     for (int it = 0; it < P::HITER; ++it) {
         const int u = tid + it * P::NTHREADS;
         if (P::NUH % P::NTHREADS == 0 || u < P::NUH) {
-            const int side = P::LHALO ? u % P::SIDE_DIV : 1;
             const int rest = u / P::SIDE_DIV;
-            buf[rest * P::PITCH + (side ? P::ICOL0 + P::ICOLS : P::LPAD)] = st.h[it];
+            buf[rest * P::PITCH + P::ICOL0 + P::halo_col(u % P::SIDE_DIV)] = st.h[it];
         }
     }
 }
 
-// Geometry of the tiled kernels (see the header comment).  KS = 3: 3x3 taps, pad 1.  KS = 1: a single tap,
+// Geometry of the tiled kernels (see the header comment).  KS = 3: 3x3 taps, pad 1.  KS = 5: 5x5 taps, pad 2.  KS = 1: a single tap,
 // pad 0 -- no halo; the forward uses it for 1x1 layers, whose (H, W) planes it walks as one long row.
 template <int TN_, int SPR_, int TH_, int NIMG_, int TM_, int COW_, int CC_, int CQ_, int S_ = 1, int KS_ = 3>
 struct Tile3x3Cfg {
@@ -153,14 +152,15 @@ struct Tile3x3Cfg {
     static constexpr int LANES = NIMG * TH * SPR;
     static constexpr int POSW = ceil_div(LANES, 64);
     static constexpr int NTHREADS = 64 * POSW * COW;
-    // stride 2 never reads past the interior on the right; a single tap has no halo at all
-    using Patch = PatchCfg<NIMG, CC, (TH - 1) * S + KS, TW * S, PAD, (S == 1) ? PAD : 0, NTHREADS>;
+    // stride 2 reads one column less past the interior on the right; a single tap has no halo at all
+    static constexpr int RHALO = S == 1 || PAD == 0 ? PAD : PAD - 1;
+    using Patch = PatchCfg<NIMG, CC, (TH - 1) * S + KS, TW * S, PAD, RHALO, NTHREADS>;
     static constexpr int PITCH = Patch::PITCH, PLANE = Patch::PLANE, BUF = Patch::BUF;
     static constexpr int LDS_BYTES = 2 * BUF * 4;
     static constexpr int STRIP = (TN - 1) * S + KS;  // floats a lane reads per tile row
     static constexpr int STRIP_ALIGN = ((TN * S) % 4 == 0) ? 4 : ((TN * S) % 2 == 0 ? 2 : 1);
     static_assert(S == 1 || S == 2, "stride 1 or 2");
-    static_assert(KS == 1 || KS == 3, "one tap or 3x3 taps");
+    static_assert(KS == 1 || KS == 3 || KS == 5, "one tap, 3x3 or 5x5 taps");
     static_assert(CC % CQ == 0, "CC must be a multiple of CQ");
 };
 
