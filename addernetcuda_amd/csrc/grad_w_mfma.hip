@@ -403,6 +403,29 @@ using Gm1x1b  = GwMfmaCfg<1, 1, 64, 1, 4, 4, 2, 2, 2, 1>;
 // (196 = 3 x 52 + 40 and 49 positions) fill tiles of 52 to 94 %, tiles of 64 to 77 %
 using Gm1x1c  = GwMfmaCfg<1, 1, 52, 1, 4, 2, 2, 4, 1, 1>;
 
+// Position splits ("slots") for `blocks` (co, k) blocks and `ntiles` tiles.  One workgroup per CU at a time (its two staged
+// tiles fill half of a CU's LDS and more), so slots * blocks workgroups run in rounds of 256, and a round takes the tiles
+// of one workgroup plus about one more for its start, fold and slab; writing and reading the slabs costs about a tile time
+// per 400 workgroups.  The least of that wins, then the fewest slabs.  (Aiming at 256 workgroups with the quotient
+// rounded up leaves e.g. 22 x 12 = 264 workgroups, a second round for eight of them: 192 -> 192 3x3 @14x14, 32 images,
+// 205 -> 147 us without that round; 300 -> 300 1x1 @14x14, 64 images, 147 -> 94 us.)
+// More slabs than that quotient are taken only up to the scratch of the entry point without a workspace.
+static int plan_slots(int blocks, int ntiles, size_t slab_bytes) {
+    const int quotient = ceil_div(256, blocks);
+    int best = 1;
+    long best_cost = -1;
+    for (int rounds = 1; rounds <= 8; ++rounds) {   // as many slots as fill so many rounds, and no more than the tiles need
+        int s = 256 * rounds / blocks;
+        if (s < 1) continue;
+        const int each = ceil_div(ntiles, s);
+        s = ceil_div(ntiles, each);
+        if (s > quotient && s * slab_bytes + kGradWGeneralWs + 256 > ADDER_NOALLOC_SCRATCH_BYTES) break;
+        const long cost = 400L * ceil_div(s * blocks, 256) * (each + 1) + (long)s * blocks;
+        if (best_cost < 0 || cost < best_cost) { best = s; best_cost = cost; }
+    }
+    return best;
+}
+
 template <class G>
 static void plan_one(const ConvDims &d, GradWMfmaPlan &p) {
     p.tilesH = ceil_div(d.Ho, G::TH);
@@ -410,10 +433,7 @@ static void plan_one(const ConvDims &d, GradWMfmaPlan &p) {
     p.ntiles = ceil_div(d.N, G::NIMG) * p.tilesH * p.tilesW;
     p.gy = ceil_div(d.Co, G::COB);
     p.gz = ceil_div(d.Ci * G::KK, G::KB);
-    // one workgroup per CU (a workgroup's two staged tiles fill half of a CU's LDS and more)
-    int want = ceil_div(256, p.gy * p.gz);
-    p.slots = want < p.ntiles ? want : p.ntiles;
-    if (p.slots < 1) p.slots = 1;
+    p.slots = plan_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)d.Co * d.Ci * G::KK + d.Co));
 }
 
 // a 1x1 layer seen as images of one row of Ho*Wo positions (the whole plane when the stride is 1)

@@ -168,7 +168,8 @@ ADDER_API int adder_conv2d_bwd_bf16(const adder_bf16 *gy, const adder_bf16 *x, c
  * (every GPU the library runs on holds one copy until the process ends); the call allocates and frees nothing.
  * Same arguments and results as adder_conv2d_bwd_f32 without ws / ws_bytes.  Layers whose
  * adder_conv2d_bwd_workspace_bytes exceeds ADDER_NOALLOC_SCRATCH_BYTES are refused with ADDER_ERR_WORKSPACE
- * before anything is launched (every ResNet-20 layer at batch 256 fits).  All calls on one GPU share that
+ * before anything is launched (every ResNet-20 layer at batch 256 fits) -- except 5x5 layers, which then take the general
+ * kernel, whose sums have another order.  All calls on one GPU share that
  * GPU's buffer: calls that overlap in time on one GPU (different streams, or threads) race; serialise them.
  * The first call on a device looks the buffer's address up (hipGetSymbolAddress); make that call outside
  * stream capture. */
