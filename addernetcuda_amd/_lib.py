@@ -29,6 +29,8 @@ _SIGNATURES = {
     "adder_abi_version": (_i, []),
     "adder_out_dim": (_i, [_i, _i, _i, _i]),
     "adder_conv2d_fwd_f32": (_i, [_p, _p, _p] + [_i] * 9 + [_p]),
+    "adder_conv2d_fwd_bn_eval_f32": (_i, [_p] * 7 + [_f, _p] + [_i] * 10 + [_p]),
+    "adder_bn_eval_f32": (_i, [_p] * 6 + [_f, _p] + [_i] * 4 + [_p]),
     "adder_conv2d_fwd_stats_slots": (_i, [_i] * 9 + [ctypes.POINTER(ctypes.c_int)]),
     "adder_conv2d_fwd_pair_stats_f32": (_i, [_p] * 7 + [_i] * 10 + [_p]),
     "adder_conv2d_fwd_stats_f32": (_i, [_p, _p, _p, _p, _i] + [_i] * 9 + [_p]),
@@ -147,6 +149,14 @@ def stream_ptr(device):
 def ptr(t):
     """Device address of a tensor (None -> NULL) for a ``void *`` / ``float *`` argument."""
     return t.data_ptr() if t is not None else None
+
+
+def plain_call(x):
+    """Whether ``x`` is an ordinary tensor in an ordinary call without gradients: nothing that records, transforms or
+    differentiates the operators in between would miss those that one kernel does together."""
+    return (type(x) is torch.Tensor and not torch.is_grad_enabled() and not torch._C._functorch.peek_interpreter_stack()
+            and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling())
 
 
 class on_device:

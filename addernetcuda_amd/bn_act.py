@@ -4,7 +4,8 @@
 training-mode forward on the GPU runs as two HIP passes, statistics then
 ``relu(gamma * (x - mean) * rstd + beta [+ residual])``, and whose backward is two more; see
 csrc/bn_act.hip.  It replaces the separate bn / += residual / relu ops of resnet20.py:28-39.
-Anything the fused kernels do not cover (eval mode, CPU tensors, non-fp32) goes through the
+In evaluation mode, without gradients, the same is one launch on the running statistics.
+Anything the fused kernels do not cover (evaluation with gradients, CPU tensors, non-fp32) goes through the
 ordinary torch ops with identical semantics.
 """
 import torch
@@ -12,7 +13,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd import Function
 
-from ._lib import lib, check, ptr, stream_ptr, on_device, bn_act_sizes
+from ._lib import lib, check, ptr, stream_ptr, on_device, bn_act_sizes, plain_call
 
 
 def _workspace(N, C, HW, device):
@@ -104,10 +105,29 @@ class BatchNormAct2d(nn.BatchNorm2d):
         return (self.training and x.is_cuda and x.dtype == torch.float32 and self.affine and x.dim() == 4
                 and self.weight.dtype == torch.float32 and self.momentum is not None)
 
+    def _eval_fusable(self, x, C, residual):
+        """Whether the inference kernels can apply this module to C channels of values made from ``x``."""
+        if (self.training or self.running_mean is None or self.running_var is None or not self.affine or not x.is_cuda
+                or x.dtype != torch.float32 or x.dim() != 4 or C != self.num_features or not plain_call(x)):
+            return False
+        if residual is not None and not (plain_call(residual) and residual.dtype == torch.float32
+                                         and residual.device == x.device and residual.is_contiguous()):
+            return False
+        return all(t.dtype == torch.float32 and t.device == x.device and t.is_contiguous() and t.numel() == C
+                   for t in (self.weight, self.bias, self.running_mean, self.running_var))
+
     def forward(self, x, residual=None, stats=None):
         """``stats``: optional per-channel partial sums of x and x*x from the layer that produced x
         (``adder2d.forward_with_stats``); they replace this module's own statistics pass."""
         if not self._fusable(x):
+            if (x.dim() == 4 and x.is_contiguous() and x.numel() and (residual is None or residual.shape == x.shape)
+                    and self._eval_fusable(x, x.shape[1], residual)):
+                y = torch.empty_like(x)
+                with on_device(x.device):
+                    check(lib.adder_bn_eval_f32(ptr(x), ptr(y), ptr(self.weight), ptr(self.bias), ptr(self.running_mean),
+                                                ptr(self.running_var), self.eps, ptr(residual), int(self.relu), x.shape[0],
+                                                x.shape[1], x.shape[2] * x.shape[3], stream_ptr(x.device)), "adder_bn_eval_f32")
+                return y
             out = super().forward(x)
             if residual is not None:
                 out = out + residual

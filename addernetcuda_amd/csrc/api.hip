@@ -133,6 +133,33 @@ int adder_conv2d_fwd_f32(const float *x, const float *w, float *y, int N, int Ci
     return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream));
 }
 
+int adder_conv2d_fwd_bn_eval_f32(const float *x, const float *w, float *y, const float *gamma, const float *beta,
+                                 const float *mean, const float *var, float eps, const float *residual, int relu, int N,
+                                 int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, void *stream) {
+    if (!x || !w || !y || !gamma || !beta || !mean || !var) return ADDER_ERR_NULL_POINTER;
+    ConvDims d;
+    if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
+    const size_t nco = sizeof(float) * (size_t)Co, ny = sizeof(float) * (size_t)N * Co * d.Ho * d.Wo;
+    const Span outs[] = {{y, ny}};
+    const Span ins[] = {{x, sizeof(float) * (size_t)N * Ci * H * W}, {w, sizeof(float) * (size_t)Co * d.K()}, {gamma, nco},
+                        {beta, nco}, {mean, nco}, {var, nco}, {residual, ny}};
+    if (any_alias(outs, ins)) return ADDER_ERR_ALIAS;
+    const BnEval bn{gamma, beta, mean, var, residual, eps, relu, aligned_groups(residual)};
+    return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream), bn);
+}
+
+int adder_bn_eval_f32(const float *x, float *y, const float *gamma, const float *beta, const float *mean, const float *var,
+                      float eps, const float *residual, int relu, int N, int C, int HW, void *stream) {
+    if (!x || !y || !gamma || !beta || !mean || !var) return ADDER_ERR_NULL_POINTER;
+    if (N <= 0 || C <= 0 || HW <= 0) return ADDER_ERR_BAD_SHAPE;
+    if ((double)N * C * HW > (double)kMaxElems) return ADDER_ERR_TOO_LARGE;
+    const size_t nc = sizeof(float) * (size_t)C, nx = sizeof(float) * (size_t)N * C * HW;
+    const Span outs[] = {{y, nx}};
+    const Span ins[] = {{x, nx}, {gamma, nc}, {beta, nc}, {mean, nc}, {var, nc}, {residual, nx}};
+    if (any_alias(outs, ins)) return ADDER_ERR_ALIAS;
+    return launch_bn_eval(x, y, BnEval{gamma, beta, mean, var, residual, eps, relu, 0}, N, C, HW, static_cast<hipStream_t>(stream));
+}
+
 int adder_conv2d_fwd_stats_slots(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad,
                                  int *slots) {
     if (!slots) return ADDER_ERR_NULL_POINTER;

@@ -119,6 +119,28 @@ __device__ __forceinline__ void bn_reduce_partials(const T *__restrict__ part, i
     s2 = (rb[0] + rb[1]) + (rb[2] + rb[3]);
 }
 
+// BatchNorm with fixed statistics, shortcut and ReLU in one pass over groups of V elements.  One read and one write of the
+// tensor bound it (plus the shortcut's read); torch runs it as two or three launches, which is what a small map pays for.
+template <int V>
+__global__ __launch_bounds__(kBnThreads) void bn_eval_kernel(const float *__restrict__ x, float *__restrict__ y, const BnEval bn,
+                                                             int C, int HWV, int total) {
+    for (int i = blockIdx.x * kBnThreads + threadIdx.x; i < total; i += gridDim.x * kBnThreads) {
+        const BnEvalChannel ch(bn, i / HWV % C);
+        const Pack<V> v = ld<V>(x, i);
+        Pack<V> r;
+#pragma unroll
+        for (int e = 0; e < V; ++e) r.v[e] = 0.f;
+        if (bn.res) r = ld<V>(bn.res, i);
+        Pack<V> o;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            o.v[e] = ch(v.v[e]) + r.v[e];
+            if (bn.relu) o.v[e] = relu_keep_nan(o.v[e]);
+        }
+        st<V>(y, i, o);
+    }
+}
+
 // Forward pass 2.  grid = (A, C); block (a, c) finishes the statistics of channel c and normalises the
 // float4 groups a*256 + tid, a*256 + tid + A*256, ... of that channel.  Block (0, c) also stores
 // mean / rstd for the backward pass and updates the running statistics; block (0, 0) advances
@@ -368,6 +390,15 @@ static int bn_bwd_v(const float *dy, const float *y, const unsigned *mask, const
 }
 
 // mask (nullable): the sign bits the forward left; replaces y
+int launch_bn_eval(const float *x, float *y, const BnEval &bn, int N, int C, int HW, hipStream_t s) {
+    const bool vec = HW % 4 == 0 && aligned_groups(x) && aligned_groups(y) && aligned_groups(bn.res);
+    const int total = (int)((long)N * C * HW / (vec ? 4 : 1));
+    const int blocks = (int)(ceil_div_l(total, kBnThreads) < 4096 ? ceil_div_l(total, kBnThreads) : 4096);
+    if (vec) hipLaunchKernelGGL(bn_eval_kernel<4>, dim3(blocks), dim3(kBnThreads), 0, s, x, y, bn, C, HW / 4, total);
+    else hipLaunchKernelGGL(bn_eval_kernel<1>, dim3(blocks), dim3(kBnThreads), 0, s, x, y, bn, C, HW, total);
+    return check_launch();
+}
+
 int launch_bn_act_bwd(const float *dy, const float *y, const unsigned *mask, const float *x, const float *gamma,
                       const float *mean, const float *rstd, float *dx, float *dres, float *dgamma, float *dbeta,
                       int relu, int N, int C, int HW, void *ws, hipStream_t s) {

@@ -225,6 +225,24 @@ __device__ __forceinline__ float wave_sum_scatter(float (&v)[K], int lane) {
     return r;
 }
 
+// BatchNorm with fixed statistics (inference), applied to a finished value of channel c:
+// act((v - mean) / sqrt(var + eps) * gamma + beta [+ residual]).  gamma == null: not used.  The roundings -- reciprocal square
+// root in one instruction, normalised value, multiply-add, shortcut -- are those of the BatchNorm that torch runs, so that a
+// network gives the same bits whichever of the two it goes through (deep untrained ones amplify the last bit to 1e-3).
+struct BnEval {
+    const float *gamma, *beta, *mean, *var, *res;   // res (nullable): shaped like the output
+    float eps;
+    int relu, res_vec;                              // res_vec: res is aligned to groups of four
+};
+static constexpr BnEval kNoBnEval{nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0, 0};
+struct BnEvalChannel {
+    float mean, rstd, gamma, beta;
+    __device__ __forceinline__ BnEvalChannel(const BnEval &b, int c)
+        : mean(b.mean[c]), rstd(rsqrtf(b.var[c] + b.eps)), gamma(b.gamma[c]), beta(b.beta[c]) {}
+    __device__ __forceinline__ float operator()(float v) const { return fmaf(gamma, (v - mean) * rstd, beta); }
+};
+__device__ __forceinline__ float relu_keep_nan(float v) { return v < 0.f ? 0.f : v; }
+
 struct ConvDims {
     int N, Ci, H, W, Co, kh, kw, stride, pad, Ho, Wo;
     __host__ __device__ int K() const { return Ci * kh * kw; }
@@ -237,7 +255,7 @@ int check_launch();                  // hipGetLastError -> status
 // Launchers implemented in the kernel translation units.
 // T: storage type of the activations and their gradients, float or bf16_t (the optional reduced-storage mode).
 template <class T>
-int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s);
+int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
 int fwd_stats_slots(const ConvDims &d);
 bool fwd_pair_supported(const ConvDims &d);
 int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats,
@@ -289,7 +307,7 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
 bool conv1x1_supported(const ConvDims &d, const void *a, const void *b);
 int fwd_1x1_stats_slots(const ConvDims &d);
 template <class T>
-int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s);
+int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
 template <class T>
 int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s);
 int grad_w_1x1_slots(const ConvDims &d);
@@ -303,6 +321,7 @@ int launch_bn_act_fwd(const float *x, const float *res, const float *gamma, cons
                       unsigned *mask, float *mean, float *rstd, float *running_mean, float *running_var,
                       long long *num_batches, float momentum, float eps, int relu, int N, int C, int HW, void *ws,
                       const double *stats, int stats_slots, hipStream_t s);
+int launch_bn_eval(const float *x, float *y, const BnEval &bn, int N, int C, int HW, hipStream_t s);
 int launch_bn_act_bwd(const float *dy, const float *y, const unsigned *mask, const float *x, const float *gamma,
                       const float *mean, const float *rstd, float *dx, float *dres, float *dgamma, float *dbeta,
                       int relu, int N, int C, int HW, void *ws, hipStream_t s);

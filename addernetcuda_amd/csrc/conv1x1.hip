@@ -75,7 +75,8 @@ __device__ __forceinline__ void st2(T *p, const float2 v, int valid) {
 template <int S, int TM, bool VEC = true, class T = float>
 __global__ __launch_bounds__(256) void fwd_1x1_kernel(const T *__restrict__ x, const float *__restrict__ w,
                                                       T *__restrict__ y, double *__restrict__ stats, int N, int Ci,
-                                                      int H, int W, int Co, int Ho, int Wo, int gpr, int groups) {
+                                                      int H, int W, int Co, int Ho, int Wo, int gpr, int groups,
+                                                      const BnEval bn) {
     constexpr int TN = 4 / S;
     const Lane1x1<S> L(blockIdx.x * 256 + threadIdx.x, groups, gpr, Ho);
     const int co0 = blockIdx.y * TM;
@@ -156,6 +157,22 @@ __global__ __launch_bounds__(256) void fwd_1x1_kernel(const T *__restrict__ x, c
         }
     }
     if (L.ok) {
+        if constexpr (sizeof(T) == 4) {
+            if (bn.gamma) {   // inference: the BatchNorm behind the layer, the shortcut and the ReLU on the way out
+#pragma unroll
+                for (int m = 0; m < TM; ++m) {
+                    const int co = min(co0 + m, Co - 1);
+                    const BnEvalChannel ch(bn, co);
+                    const float *res = bn.res + (((size_t)L.n * Co + co) * Ho + L.ho) * Wo + L.wo0;
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) {
+                        tot[m][t] = ch(tot[m][t]);
+                        if (bn.res && L.wo0 + t < Wo) tot[m][t] += res[t];
+                        if (bn.relu) tot[m][t] = relu_keep_nan(tot[m][t]);
+                    }
+                }
+            }
+        }
 #pragma unroll
         for (int m = 0; m < TM; ++m) {
             if (co0 + m >= Co) continue;
@@ -387,22 +404,23 @@ int fwd_1x1_stats_slots(const ConvDims &d) {
 
 // stats (nullable): per-channel partial sums of y and y*y, fwd_1x1_stats_slots(d) slots per channel
 template <class T>
-int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s) {
+int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn) {
     constexpr int TM = 8;
     const ConvDims f = lane_dims(d);
     int gpr, groups;
     lane_space(f, gpr, groups);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(ceil_div(groups, 256), ceil_div(f.Co, TM)), dim3(256), 0, s, x, w, y, stats, f.N, f.Ci,
-                           f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
+                           f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups, bn);
         return check_launch();
     };
     const bool vec = vec_ok<T>(f, x, y, nullptr);
     if (f.stride == 2) return vec ? launch(fwd_1x1_kernel<2, TM, true, T>) : launch(fwd_1x1_kernel<2, TM, false, T>);
     return vec ? launch(fwd_1x1_kernel<1, TM, true, T>) : launch(fwd_1x1_kernel<1, TM, false, T>);
 }
-template int launch_fwd_1x1<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t);
-template int launch_fwd_1x1<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t);
+template int launch_fwd_1x1<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t, const BnEval &);
+template int launch_fwd_1x1<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t,
+                                    const BnEval &);
 
 template <class T>
 int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s) {

@@ -27,7 +27,7 @@ import torch
 from torch.autograd import Function
 
 from . import adder as _adder
-from ._lib import require_gpu_f32, bwd_bn_slots, conv_dims
+from ._lib import lib, check, ptr, stream_ptr, on_device, require_gpu_f32, bwd_bn_slots, conv_dims
 from .bn_act import BatchNormAct2d, bn_forward, bn_backward
 
 
@@ -147,6 +147,9 @@ def adder_bn_act(conv, bn, x, residual=None, with_shortcut=False, side_conv=None
                                     and residual.shape[0] == x.shape[0] and residual.dtype == torch.float32
                                     and residual.device == x.device)))
     if not ok:
+        out = _eval_unit(conv, bn, x, residual)
+        if out is not None:
+            return (out, x) if with_shortcut else out
         if (not with_shortcut and residual is None and hasattr(conv, "forward_bn_act") and bn.training and x.is_cuda
                 and torch.is_grad_enabled()):
             return conv.forward_bn_act(x, bn)   # an ordinary convolution with the same kernels (the stem of a network)
@@ -183,6 +186,34 @@ def adder_bn_act(conv, bn, x, residual=None, with_shortcut=False, side_conv=None
             side.w_ptr, side.w_version = side_conv.adder.data_ptr(), side_conv.adder._version
             res[1]._adder_side_output = side
     return res
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks")
+
+
+def _eval_unit(conv, bn, x, residual):
+    """``bn(conv(x)) [+ residual]`` and the ReLU in one launch, for inference (evaluation mode, no gradients); None where
+    the modules have to run one by one (hooks on either, another forward of a subclass, ...)."""
+    if (bn.training or torch.is_grad_enabled() or not isinstance(conv, _adder.adder2d) or not isinstance(bn, BatchNormAct2d)
+            or conv.bias or type(conv).forward is not _adder.adder2d.forward
+            or type(bn).forward is not BatchNormAct2d.forward or any(getattr(m, h) for m in (conv, bn) for h in _HOOKS)
+            or torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks):
+        return None
+    W = conv.adder
+    if (x.dim() != 4 or W.dtype != torch.float32 or W.device != x.device or W.shape[2] != W.shape[3]
+            or not bn._eval_fusable(x, W.shape[0], residual)):
+        return None
+    dims, Ho, Wo = conv_dims(x.shape, W.shape, int(conv.stride), int(conv.padding))
+    shape = (x.shape[0], W.shape[0], Ho, Wo)
+    if residual is not None and residual.shape != shape:
+        return None
+    X, W = x.contiguous(), W.contiguous()
+    out = torch.empty(shape, device=x.device, dtype=torch.float32)
+    with on_device(x.device):
+        check(lib.adder_conv2d_fwd_bn_eval_f32(ptr(X), ptr(W), ptr(out), ptr(bn.weight), ptr(bn.bias), ptr(bn.running_mean),
+                                               ptr(bn.running_var), bn.eps, ptr(residual), int(bn.relu), *dims,
+                                               stream_ptr(x.device)), "adder_conv2d_fwd_bn_eval_f32")
+    return out
 
 
 def _out_hw(conv, x):

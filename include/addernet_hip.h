@@ -82,6 +82,14 @@ ADDER_API int adder_conv2d_fwd_f32(const float *x, const float *w, float *y,
                          int N, int Ci, int H, int W, int Co, int kh, int kw,
                          int stride, int pad, void *stream);
 
+/* The same forward with the BatchNorm that follows it (fixed statistics: inference), the shortcut and the ReLU applied on
+ * the way out: y = act((conv - mean) / sqrt(var + eps) * gamma + beta [+ residual]), act = ReLU when relu is set;
+ * gamma, beta, mean, var (Co), residual (nullable) shaped like y.  resnet20.py:28-39 in evaluation mode. */
+ADDER_API int adder_conv2d_fwd_bn_eval_f32(const float *x, const float *w, float *y, const float *gamma, const float *beta,
+                         const float *mean, const float *var, float eps, const float *residual, int relu,
+                         int N, int Ci, int H, int W, int Co, int kh, int kw,
+                         int stride, int pad, void *stream);
+
 /* The same forward with the statistics of the BatchNorm that follows it (resnet20.py:28-39: every adder
  * layer feeds a BatchNorm2d) collected on the way out: stats[(co * slots + s) * 2 + {0, 1}] receive partial
  * sums of y and y*y over disjoint sets of positions, in fp64; adder_bn_act_fwd_stats_f32 consumes them and
@@ -291,6 +299,11 @@ ADDER_API int adder_bn_act_fwd_stats_f32(const float *x, const float *residual, 
                                          float *running_mean, float *running_var, long long *num_batches_tracked,
                                          float momentum, float eps, int relu,
                                          int N, int C, int HW, const double *stats, int stats_slots, void *stream);
+/* The BatchNorm with fixed statistics (inference), shortcut and ReLU on their own, in one launch; arguments as in
+ * adder_conv2d_fwd_bn_eval_f32 with C channels of HW elements. */
+ADDER_API int adder_bn_eval_f32(const float *x, float *y, const float *gamma, const float *beta, const float *mean,
+                                const float *var, float eps, const float *residual, int relu, int N, int C, int HW,
+                                void *stream);
 ADDER_API int adder_bn_act_bwd_f32(const float *dy, const float *y, const unsigned int *relu_mask,
                                    const float *x, const float *gamma,
                                    const float *save_mean, const float *save_rstd,
