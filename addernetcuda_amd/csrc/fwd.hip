@@ -387,6 +387,131 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
     if constexpr (PAIR) finish(tots, y_side, stats_side);
 }
 
+// ---------------------------------------------------------------------------
+// Few positions: one output position x TM output channels per lane, the waves of a workgroup share the reduction.
+//
+// The tiled kernels give a lane 8-16 results and walk all input channels in one wave; one image leaves them with a handful
+// of workgroups, and the launch lasts as long as that serial chain (64 -> 64 3x3 @8x8, one image: 4 workgroups, 25 us).
+// Here wave v of a workgroup takes the channel chunks v, v + waves, ...; after each round the chunk sums go through LDS and
+// are added in channel order, so every result has the bits of the tiled kernel whose chunk length is given (`chunk`
+// channels per first-level sum).  x is read from global memory (a map this small sits in L1 / L2) one channel ahead
+// of the arithmetic, as are the weights.  Whole networks: ResNet-50, one image, 4.6 -> 1.7 ms; VGG-small, two, 720 -> 184 us.
+// ---------------------------------------------------------------------------
+template <int KS, int TM, int G, class T>
+__global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
+                                                      double *__restrict__ stats, ConvDims d, int chunk, const BnEval bn) {
+    constexpr int KK = KS * KS;
+    __shared__ float part[8][TM][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int plane = d.H * d.W, L = d.Ho * d.Wo, total = d.N * L, K = d.Ci * KK, co0 = blockIdx.y * TM;
+    const int pos = min((int)blockIdx.x * 64 + lane, total - 1);
+    const int n = pos / L, ho = pos % L / d.Wo, wo = pos % L % d.Wo;
+    int off[KK];
+    bool ok[KK];
+#pragma unroll
+    for (int e = 0; e < KK; ++e) {
+        const int hi = ho * d.stride + e / KS - d.pad, wi = wo * d.stride + e % KS - d.pad;
+        ok[e] = hi >= 0 && hi < d.H && wi >= 0 && wi < d.W;
+        off[e] = n * d.Ci * plane + (ok[e] ? hi * d.W + wi : 0);
+    }
+    uniform_f32_ptr wc = as_uniform(w);
+    int wrow[TM];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) wrow[m] = min(co0 + m, d.Co - 1) * K;
+    const int nchunks = ceil_div(d.Ci, chunk);
+    float tot[TM];   // of result threadIdx.x + k * blockDim.x of the workgroup's TM x 64
+#pragma unroll
+    for (int k = 0; k < TM; ++k) tot[k] = 0.f;
+
+    for (int c0 = 0; c0 < nchunks; c0 += waves) {
+        const int c = c0 + wave;
+        if (c < nchunks) {
+            const int first = c * chunk, end = min(first + chunk, d.Ci);
+            float acc[TM], xv[2][G * KK], wv[2][TM * G * KK];
+#pragma unroll
+            for (int m = 0; m < TM; ++m) acc[m] = 0.f;
+            auto load = [&](const int b, const int ci) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const int cc = min(ci + g, end - 1);
+#pragma unroll
+                    for (int m = 0; m < TM; ++m)
+#pragma unroll
+                        for (int e = 0; e < KK; ++e) wv[b][(m * G + g) * KK + e] = wc[wrow[m] + cc * KK + e];
+                    const T *xc = x + (size_t)cc * plane;
+#pragma unroll
+                    for (int e = 0; e < KK; ++e) xv[b][g * KK + e] = ldf(xc + off[e]);
+                }
+            };
+            auto add = [&](const int b, const int ci) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    if (ci + g >= end) break;
+#pragma unroll
+                    for (int e = 0; e < KK; ++e) {
+                        const float v = ok[e] ? xv[b][g * KK + e] : 0.f;
+#pragma unroll
+                        for (int m = 0; m < TM; ++m) acc[m] -= fabsf(wv[b][(m * G + g) * KK + e] - v);
+                    }
+                }
+            };
+            load(0, first);
+#pragma unroll 1
+            for (int ci = first; ci < end; ci += 2 * G) {
+                load(1, ci + G);
+                __builtin_amdgcn_sched_barrier(0);
+                add(0, ci);
+                load(0, ci + 2 * G);
+                __builtin_amdgcn_sched_barrier(0);
+                add(1, ci + G);
+            }
+#pragma unroll
+            for (int m = 0; m < TM; ++m) part[wave][m][lane] = acc[m];
+        }
+        __syncthreads();
+        const int here = min(waves, nchunks - c0);
+#pragma unroll
+        for (int k = 0; k < TM; ++k) {
+            const int e = threadIdx.x + k * blockDim.x;
+            if (e < TM * 64)
+                for (int v = 0; v < here; ++v) tot[k] += part[v][e >> 6][e & 63];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < TM; ++k) {
+        const int e = threadIdx.x + k * blockDim.x, p = blockIdx.x * 64 + (e & 63), co = co0 + (e >> 6);
+        if (stats && e < TM * 64 && co < d.Co) {   // (wave-uniform: a wave holds 64 positions of one channel)
+            const double v = p < total ? (double)tot[k] : 0.0, s1 = wave_sum(v), s2 = wave_sum(v * v);
+            if (lane == 0) {
+                double *dst = stats + ((size_t)co * gridDim.x + blockIdx.x) * 2;
+                dst[0] = s1;
+                dst[1] = s2;
+            }
+        }
+        if (e < TM * 64 && p < total && co < d.Co) {
+            const size_t o = ((size_t)(p / L) * d.Co + co) * L + p % L;
+            float v = tot[k];
+            if (sizeof(T) == 4 && bn.gamma) {
+                v = BnEvalChannel(bn, co)(v);
+                if (bn.res) v += bn.res[o];
+                if (bn.relu) v = relu_keep_nan(v);
+            }
+            stf(y + o, v);
+        }
+    }
+}
+
+template <int KS, class T>
+static int launch_fwd_few(const T *x, const float *w, T *y, double *stats, const ConvDims &d, int chunk, hipStream_t s,
+                          const BnEval &bn) {
+    constexpr int TM = 4, G = KS == 1 ? 8 : 1;
+    const int waves = ceil_div(d.Ci, chunk) < 8 ? ceil_div(d.Ci, chunk) : 8;
+    hipLaunchKernelGGL((fwd_few_kernel<KS, TM, G, T>), dim3(ceil_div(d.N * d.Ho * d.Wo, 64), ceil_div(d.Co, TM)),
+                       dim3(64 * waves), 0, s, x, w, y, stats, d, chunk, bn);
+    return check_launch();
+}
+
 template <class C, bool VEC, bool SUB = false, bool MUL = false, class T = float>
 static int launch_fwd_3x3_v(const T *x, const float *w, T *y, double *stats, const ConvDims &d,
                             hipStream_t s, const Subsample sub = Subsample{1, 0, 0, 0}, const BnEval &bn = kNoBnEval) {
@@ -506,6 +631,40 @@ static int fwd_tiled_variant(const ConvDims &d) {
     return 0;
 }
 
+// input channels per first-level sum of the kernel that serves these dimensions
+static int fwd_chunk(const ConvDims &d, int variant) {
+    switch (variant) {
+        case 1: return FwdW32::CC;
+        case 2: return FwdW16::CC;
+        case 3: return FwdW8::CC;
+        case 4: return FwdW16S2::CC;
+        case 5: return d.Ci >= 128 ? FwdW8S2L::CC : FwdW8S2::CC;
+        case 8: case 9: return Fwd1x1sub::CC;
+        default: return Fwd1x1::CC;
+    }
+}
+static_assert(FwdW32::CC == FwdW32H8::CC && FwdW32::CC == FwdW32H4::CC && Fwd1x1::CC == Fwd1x1s::CC &&
+              Fwd1x1::CC == Fwd1x1q::CC && Fwd1x1::CC == Fwd1x1sq::CC, "one chunk length per variant");
+
+// Whether the kernel for few positions takes a 3x3 or 1x1 layer.  The tiled kernels last as long as one wave's chain of
+// channels x taps x results per lane, 6 ns a term, until the chip is full; this one has a chain of its share of the
+// channels (0.4 us each with nine taps, 0.25 with one) and then works at 10.9 (nine taps) or 3.2 (one tap) terms per ps.
+// Fitted to 48 layers; us, tiled -> this: 64 -> 64 3x3 @8x8, 1 / 16 / 64 images, 27 -> 8, 28 -> 8, 28 -> 17; 512 -> 512 3x3
+// @7x7, 1 / 4 images, 205 -> 30, 213 -> 69; 1024 -> 256 1x1 @14x14, 1 / 4 images, 105 -> 34, 105 -> 94.  Beyond the line
+// the tiled kernels win: 16 -> 16 3x3 @32x32, 64 images, 15 against 18; 1024 -> 256 1x1 @14x14, 16 images, 106 against 281.
+// (The plain 1x1 kernel has short chains; 5x5 layers are not built here.)
+static bool few_positions(const ConvDims &d, int variant) {
+    if (variant == 0 || variant >= 14) return false;
+    const int per_lane = variant == 3 ? FwdW8::TM * FwdW8::TN : variant == 4 || variant == 5 ? FwdW16S2::TM * FwdW16S2::TN
+                       : variant == 8 || variant == 9 ? Fwd1x1sub::TM * Fwd1x1sub::TN : FwdW32::TM * FwdW32::TN;
+    const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;
+    const int chunk = fwd_chunk(d, variant);
+    const float tiled = 0.006f * d.K() * per_lane;
+    const float share = (float)(ceil_div(ceil_div(d.Ci, chunk), 8) * chunk);
+    const float few = 2.f + (d.kh == 3 ? 0.4f * share + terms / 10.9e6f : 0.25f * share + terms / 3.2e6f);
+    return few < 0.9f * tiled;
+}
+
 // a 1x1 layer seen as N x Ci "images" of one row of Ho*Wo positions (the whole plane when the stride is 1)
 static ConvDims as_one_row(const ConvDims &d) {
     ConvDims f = d;
@@ -546,6 +705,7 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 }
 
 int fwd_stats_slots(const ConvDims &d) {
+    if (d.kh == 1 && few_positions(d, fwd_tiled_variant(d))) return ceil_div(d.N * d.Ho * d.Wo, 64);
     switch (fwd_tiled_variant(d)) {
         case 1: switch (rows_per_tile_w32(d.Ho)) {
             case 16: return stats_slots_3x3<FwdW32>(d);
@@ -575,6 +735,10 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
     // rows that are whole groups of four are moved as such and need bases aligned to a group
     const bool rows_ok = (d.W % 4 != 0 || aligned_groups(x)) && (d.Wo % 4 != 0 || aligned_groups(y));
     const int variant = fwd_tiled_variant(d);
+    if ((!stats || d.kh == 1) && few_positions(d, variant)) {   // (its statistics are offered for 1x1 layers: fwd_stats_slots)
+        const int chunk = fwd_chunk(d, variant);
+        return d.kh == 3 ? launch_fwd_few<3>(x, w, y, stats, d, chunk, s, bn) : launch_fwd_few<1>(x, w, y, stats, d, chunk, s, bn);
+    }
     const bool strided = variant == 8 || variant == 9 || variant == 12 || variant == 13;
     if (strided) {   // x is read element by element; y is a dense row per plane
         const ConvDims f = as_one_row(d);
