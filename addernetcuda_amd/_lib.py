@@ -154,9 +154,12 @@ def ptr(t):
 def plain_call(x):
     """Whether ``x`` is an ordinary tensor in an ordinary call without gradients: nothing that records, transforms or
     differentiates the operators in between would miss those that one kernel does together."""
-    return (type(x) is torch.Tensor and not torch.is_grad_enabled() and not torch._C._functorch.peek_interpreter_stack()
-            and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing()
-            and not torch.compiler.is_compiling())
+    return (type(x) is torch.Tensor and not torch.is_grad_enabled() and not _functorch_stack()
+            and _forward_ad._current_level < 0 and not _is_tracing() and not _is_compiling())
+
+
+_functorch_stack, _forward_ad = torch._C._functorch.peek_interpreter_stack, torch.autograd.forward_ad
+_is_tracing, _is_compiling = torch._C._is_tracing, torch.compiler.is_compiling
 
 
 class on_device:

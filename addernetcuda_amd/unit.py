@@ -27,7 +27,7 @@ import torch
 from torch.autograd import Function
 
 from . import adder as _adder
-from ._lib import lib, check, ptr, stream_ptr, on_device, require_gpu_f32, bwd_bn_slots, conv_dims
+from ._lib import lib, check, ptr, stream_ptr, on_device, plain_call, require_gpu_f32, bwd_bn_slots, conv_dims
 from .bn_act import BatchNormAct2d, bn_forward, bn_backward
 
 
@@ -141,15 +141,16 @@ def adder_bn_act(conv, bn, x, residual=None, with_shortcut=False, side_conv=None
     layer's node then leaves its input gradient to this node (``adder.SideOutput``), whose strided input-gradient
     kernel adds it on the positions the 1x1 layer read -- so ``shortcut`` is for ``side_conv`` and nothing else:
     a gradient taken with respect to ``shortcut`` itself would miss that part."""
+    if not bn.training:
+        out = _eval_unit(conv, bn, x, residual)
+        if out is not None:
+            return (out, x) if with_shortcut else out
     ok = (isinstance(conv, _adder.adder2d) and isinstance(bn, BatchNormAct2d) and not conv.bias and bn._fusable(x)
           and torch.is_grad_enabled() and conv.adder.dtype == torch.float32
           and (residual is None or (residual.shape[1:] == (conv.output_channel,) + _out_hw(conv, x)
                                     and residual.shape[0] == x.shape[0] and residual.dtype == torch.float32
                                     and residual.device == x.device)))
     if not ok:
-        out = _eval_unit(conv, bn, x, residual)
-        if out is not None:
-            return (out, x) if with_shortcut else out
         if (not with_shortcut and residual is None and hasattr(conv, "forward_bn_act") and bn.training and x.is_cuda
                 and torch.is_grad_enabled()):
             return conv.forward_bn_act(x, bn)   # an ordinary convolution with the same kernels (the stem of a network)
@@ -188,31 +189,40 @@ def adder_bn_act(conv, bn, x, residual=None, with_shortcut=False, side_conv=None
     return res
 
 
-_HOOKS = ("_forward_hooks", "_forward_pre_hooks")
+_module = torch.nn.modules.module
 
 
 def _eval_unit(conv, bn, x, residual):
     """``bn(conv(x)) [+ residual]`` and the ReLU in one launch, for inference (evaluation mode, no gradients); None where
-    the modules have to run one by one (hooks on either, another forward of a subclass, ...)."""
-    if (bn.training or torch.is_grad_enabled() or not isinstance(conv, _adder.adder2d) or not isinstance(bn, BatchNormAct2d)
-            or conv.bias or type(conv).forward is not _adder.adder2d.forward
-            or type(bn).forward is not BatchNormAct2d.forward or any(getattr(m, h) for m in (conv, bn) for h in _HOOKS)
-            or torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks):
+    the modules have to run one by one (hooks on either, another forward of a subclass, ...).
+
+    A network of small maps spends its time here, on the host: the modules' tables are read directly (a parametrised or
+    missing tensor is not in them and ends the attempt), 24 -> 19 us a call."""
+    if (bn.training or torch.is_grad_enabled() or type(bn) is not BatchNormAct2d or type(conv) is not _adder.adder2d
+            or conv.bias or conv._forward_hooks or conv._forward_pre_hooks or bn._forward_hooks or bn._forward_pre_hooks
+            or _module._global_forward_hooks or _module._global_forward_pre_hooks or not plain_call(x)):
         return None
-    W = conv.adder
-    if (x.dim() != 4 or W.dtype != torch.float32 or W.device != x.device or W.shape[2] != W.shape[3]
-            or not bn._eval_fusable(x, W.shape[0], residual)):
+    params, buffers = bn._parameters, bn._buffers
+    W, tensors = conv._parameters.get("adder"), (params.get("weight"), params.get("bias"), buffers.get("running_mean"),
+                                                 buffers.get("running_var"))
+    dev = x.device
+    if (W is None or W.dtype != torch.float32 or W.device != dev or dev.type != "cuda" or x.dtype != torch.float32
+            or x.dim() != 4 or W.dim() != 4 or W.shape[2] != W.shape[3] or bn.num_features != W.shape[0]):
         return None
+    for t in tensors:
+        if t is None or t.dtype != torch.float32 or t.device != dev or not t.is_contiguous() or t.numel() != bn.num_features:
+            return None
     dims, Ho, Wo = conv_dims(x.shape, W.shape, int(conv.stride), int(conv.padding))
-    shape = (x.shape[0], W.shape[0], Ho, Wo)
-    if residual is not None and residual.shape != shape:
+    shape = (dims[0], dims[4], Ho, Wo)
+    if residual is not None and not (residual.shape == shape and residual.dtype == torch.float32 and residual.device == dev
+                                     and residual.is_contiguous() and plain_call(residual)):
         return None
     X, W = x.contiguous(), W.contiguous()
-    out = torch.empty(shape, device=x.device, dtype=torch.float32)
-    with on_device(x.device):
-        check(lib.adder_conv2d_fwd_bn_eval_f32(ptr(X), ptr(W), ptr(out), ptr(bn.weight), ptr(bn.bias), ptr(bn.running_mean),
-                                               ptr(bn.running_var), bn.eps, ptr(residual), int(bn.relu), *dims,
-                                               stream_ptr(x.device)), "adder_conv2d_fwd_bn_eval_f32")
+    out = torch.empty(shape, device=dev, dtype=torch.float32)
+    with on_device(dev):
+        check(lib.adder_conv2d_fwd_bn_eval_f32(X.data_ptr(), W.data_ptr(), out.data_ptr(), *[t.data_ptr() for t in tensors],
+                                               bn.eps, ptr(residual), 1 if bn.relu else 0, *dims, stream_ptr(dev)),
+              "adder_conv2d_fwd_bn_eval_f32")
     return out
 
 

@@ -93,6 +93,7 @@ def test_what_stays_with_the_separate_modules(gpu):
         plain = copy.deepcopy(bn)
         plain.track_running_stats, plain.running_mean, plain.running_var = False, None, None
         assert _eval_unit(layer, plain, x, None) is None             # batch statistics
+        assert _eval_unit(layer, bn, torch.nn.Parameter(x), None) is None
         with torch.autograd.forward_ad.dual_level():
             dual = torch.autograd.forward_ad.make_dual(torch.randn(2, 6, 9, 9, device=gpu), torch.ones(2, 6, 9, 9, device=gpu))
             assert torch.autograd.forward_ad.unpack_dual(bn(dual)).tangent is not None
