@@ -47,6 +47,26 @@ __device__ __forceinline__ ColVec<COLS> col_load(const float *__restrict__ row, 
 // KW = 4 (matrices with few columns): the four waves of a workgroup share their 64 * COLS columns and split the
 // rows of every block of X between them, so that the chain of dependent row batches is a quarter as long; their
 // partial sums are added through LDS at the end.
+//
+// Staging them: 256 / TM lanes per row of W, eight loads in flight per thread.  (One element at a time, with the row
+// found by a division, was a chain of 18 trips to L2 before the first row of X: a quarter of the kernel's time.)
+template <int TM, bool ZERO_PAST_CO>
+__device__ __forceinline__ void stage_weights(float *__restrict__ wt, const float *__restrict__ Wm, int K, int co0, int Co,
+                                              int k0, int kcnt) {
+    constexpr int LPR = 256 / TM, U = 8;
+    const int m = threadIdx.x / LPR, l = threadIdx.x % LPR;
+    const float *row = Wm + (size_t)min(co0 + m, Co - 1) * K + k0;
+    const bool zero = ZERO_PAST_CO && co0 + m >= Co;
+    for (int kk = l; kk < kcnt; kk += LPR * U) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = row[min(kk + u * LPR, kcnt - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (kk + u * LPR < kcnt) wt[(kk + u * LPR) * TM + m] = zero ? 0.f : v[u];
+    }
+}
+
 template <int TM, int COLS, bool VEC, int PF, int KW>
 __global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restrict__ X,
                                                           const float *__restrict__ Wm,
@@ -79,10 +99,6 @@ __global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restric
     for (int k0 = 0; k0 < K; k0 += KB) {
         const int kcnt = min(KB, K - k0);
         if (k0) __syncthreads();
-        for (int i = threadIdx.x; i < kcnt * TM; i += 256) {
-            const int m = i / kcnt, kk = i - m * kcnt;   // consecutive threads read consecutive k of one row of W
-            wt[kk * TM + m] = Wm[(size_t)min(co0 + m, Co - 1) * K + k0 + kk];
-        }
         // this wave's rows of the block
         const int share = KW == 1 ? kcnt : ceil_div(kcnt, KW);
         const int kb = KW == 1 ? 0 : min(wave * share, kcnt), ke = KW == 1 ? kcnt : min(kb + share, kcnt);
@@ -92,6 +108,7 @@ __global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restric
 #pragma unroll
             for (int r = 0; r < PF; ++r) nxt[r] = col_load<COLS, VEC>(X + (size_t)(k0 + kb + r) * NL, c0, NL);
         }
+        stage_weights<TM, false>(wt, Wm, K, co0, Co, k0, kcnt);
         __syncthreads();
         for (int kk = kb; kk < kfull; kk += PF) {
             ColVec<COLS> cur[PF];
@@ -167,10 +184,7 @@ __global__ __launch_bounds__(256) void col_grad_x_reg_kernel(const float *__rest
     constexpr int PF = 4;
     extern __shared__ __align__(16) float wt[];   // [KB][COB]
     const int k0 = blockIdx.y * KB, kcnt = min(KB, K - k0);
-    for (int i = threadIdx.x; i < kcnt * COB; i += 256) {
-        const int co = i / kcnt, kk = i - co * kcnt;       // consecutive threads read consecutive k of one row of W
-        wt[kk * COB + co] = co < Co ? Wm[(size_t)co * K + k0 + kk] : 0.f;
-    }
+    stage_weights<COB, true>(wt, Wm, K, 0, Co, k0, kcnt);
     long c0 = ((long)blockIdx.x * 256 + threadIdx.x) * COLS;
     const bool active = c0 < NL;
     if (!active) c0 = VEC ? NL - COLS : NL - 1;
@@ -271,10 +285,7 @@ __global__ __launch_bounds__(256) void col_bwd_fused_kernel(const float *__restr
     double *cred = reinterpret_cast<double *>(stage + 4 * 16 * kFusedPitch);   // [4 waves][256] blocks to fold
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
     const int k0 = blockIdx.y * KB, kcnt = min(KB, K - k0);
-    for (int i = threadIdx.x; i < kcnt * COB; i += 256) {
-        const int co = i / kcnt, kk = i - co * kcnt;
-        wt[kk * COB + co] = co < Co ? Wm[(size_t)co * K + k0 + kk] : 0.f;
-    }
+    stage_weights<COB, true>(wt, Wm, K, 0, Co, k0, kcnt);
     long c0 = ((long)blockIdx.x * 256 + threadIdx.x) * 2;
     const bool active = c0 < NL;
     if (!active) c0 = NL - 2;
@@ -371,33 +382,69 @@ __global__ __launch_bounds__(256) void col_bwd_fused_kernel(const float *__restr
     }
 }
 
-// gX[k, nl] += sum_co hardtanh(W[co,k] - X[k,nl]) * gy[co,nl], any number of output channels: lane = column,
-// TK rows of X per lane in registers, gy streamed per output channel.
-template <int TK>
+// gX[k, nl] += sum_co hardtanh(W[co,k] - X[k,nl]) * gy[co,nl], any number of output channels: a lane owns one column and
+// TK rows of X in registers; gy streams past PF output channels at a time with the next PF in flight, and the weights of
+// CB output channels sit in LDS as [co][TK] (two broadcast ds_read_b128 per 24 instructions).  Vector-issue-bound:
+// Co = 64, K = 576, NL = 16384 in 51 us, 12 T terms/s; 200, 300, 30000 in 156 us.  (Eight scalar weight loads and one load of
+// gy per output channel, each waited for: 139 and 381 us.  Two columns per lane: the same within 5 %, and slower
+// where it halves too few workgroups: 256, 128, 4096, 33 -> 47 us.)
+static constexpr int kColGradXRows = 8;
 __global__ __launch_bounds__(256) void col_grad_x_kernel(const float *__restrict__ gy,
                                                          const float *__restrict__ X,
                                                          const float *__restrict__ Wm,
-                                                         float *__restrict__ gX, int K, long NL, int Co) {
+                                                         float *__restrict__ gX, int K, long NL, int Co, int CB) {
+    constexpr int PF = 8, TK = kColGradXRows;
+    static_assert(TK == 8 && 64 % PF == 0, "eight weights per output channel in LDS, 64 output channels between two folds of acc");
+    extern __shared__ __align__(16) float wl[];   // [CB][TK]
     long nl = (long)blockIdx.x * 256 + threadIdx.x;
     const bool active = nl < NL;
     if (!active) nl = NL - 1;
     const int k0 = blockIdx.y * TK;
-    uniform_f32_ptr wc = as_uniform(Wm);
     float xv[TK], acc[TK], tot[TK];   // two-level sum: acc holds at most 64 rows of W
-    int kk[TK];
 #pragma unroll
     for (int t = 0; t < TK; ++t) {
-        kk[t] = min(k0 + t, K - 1);
-        xv[t] = X[(size_t)kk[t] * NL + nl];
+        xv[t] = X[(size_t)min(k0 + t, K - 1) * NL + nl];
         acc[t] = tot[t] = 0.f;
     }
-    for (int co = 0; co < Co; ++co) {
-        const float g = gy[(size_t)co * NL + nl];
+    float nxt[PF];
+    auto fetch = [&](const int co) {
 #pragma unroll
-        for (int t = 0; t < TK; ++t) acc[t] = fmaf(hardtanh(wc[co * K + kk[t]] - xv[t]), g, acc[t]);
-        if ((co & 63) == 63) {
+        for (int u = 0; u < PF; ++u) nxt[u] = gy[(size_t)min(co + u, Co - 1) * NL + nl];
+    };
+    fetch(0);
+    for (int cb = 0; cb < Co; cb += CB) {   // (CB: all output channels, or a multiple of 64)
+        const int cnt = min(CB, Co - cb);
+        if (cb) __syncthreads();
+        for (int i = threadIdx.x; i < cnt * TK; i += 256 * 4) {
+            float v[4];
 #pragma unroll
-            for (int t = 0; t < TK; ++t) { tot[t] += acc[t]; acc[t] = 0.f; }
+            for (int u = 0; u < 4; ++u) {
+                const int e = min(i + u * 256, cnt * TK - 1);
+                v[u] = Wm[(size_t)(cb + e / TK) * K + min(k0 + e % TK, K - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (i + u * 256 < cnt * TK) wl[i + u * 256] = v[u];
+        }
+        __syncthreads();
+        for (int cc = 0; cc < cnt; cc += PF) {
+            float g[PF];
+#pragma unroll
+            for (int u = 0; u < PF; ++u) g[u] = nxt[u];
+            if (cb + cc + PF < Co) fetch(cb + cc + PF);
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                if (cc + u >= cnt) break;
+                const float4 wa = *reinterpret_cast<const float4 *>(wl + (cc + u) * TK);
+                const float4 wb = *reinterpret_cast<const float4 *>(wl + (cc + u) * TK + 4);
+                const float wv[TK] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
+#pragma unroll
+                for (int t = 0; t < TK; ++t) acc[t] = fmaf(hardtanh(wv[t] - xv[t]), g[u], acc[t]);
+            }
+            if ((cc & 63) == 64 - PF) {
+#pragma unroll
+                for (int t = 0; t < TK; ++t) { tot[t] += acc[t]; acc[t] = 0.f; }
+            }
         }
     }
     if (active) {
@@ -742,20 +789,33 @@ int launch_col_bwd_small(const float *gy, const float *X, const float *Wm, float
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 static bool aligned8(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; }
 
+template <int TM, int COLS, bool VEC, int PF, int KW>
+static void launch_col_fwd_t(const float *X, const float *Wm, float *out, int K, long NL, int Co, hipStream_t s) {
+    // rows of X per LDS block of weights: 32 KB, 16 KB beside the split kernels' partial sums; blocks of one length
+    const int KB = ceil_div(K, ceil_div(K, KW == 1 ? 512 : 256));
+    hipLaunchKernelGGL((col_fwd_lds_kernel<TM, COLS, VEC, PF, KW>),
+                       dim3((unsigned)ceil_div_l(NL, (KW == 1 ? 256 : 64) * COLS), ceil_div(Co, TM)), dim3(256), KB * TM * 4, s,
+                       X, Wm, out, K, NL, Co, KB);
+}
+
+// One wave for all rows of X only where that leaves two workgroups of 512 columns x 16 rows of W per CU; below, the four
+// waves of a workgroup split the rows (us, unsplit -> split: Co = 32, K = 288, NL = 65536, 59 -> 39; 16, 144, 65536,
+// 29 -> 12; 64, 576, 32768, 79 -> 68; above the line 16, 144, 262144, 33 -> 37; 200, 300, 30000, 94 -> 99).  The split
+// kernels' tile shrinks with the number of workgroups: 16 x 128 while there are two per CU (256, 128, 4096: 10.7, with 8 x 128 10.8,
+// 8 x 64 14.3), 8 x 128 down to a quarter of that (32, 288, 16384: 18.1 -> 13.3), then 8 x 64 (32, 288, 4096: 17.9, 12.3, 9.9).
 int launch_col_fwd(const float *X, const float *Wm, float *out, int K, long NL, int Co, hipStream_t s) {
-    const int KB = K < 512 ? K : 512;   // rows of X per LDS block of weights (32 KB at 16 rows of W)
-    if (NL >= 65536 && NL % 2 == 0 && aligned8(X) && aligned8(out)) {
-        // many columns: two per lane (twice the arithmetic per row load), 16 rows of W per lane
-        hipLaunchKernelGGL((col_fwd_lds_kernel<16, 2, true, 8, 1>), dim3((unsigned)ceil_div_l(NL, 512), ceil_div(Co, 16)),
-                           dim3(256), KB * 16 * 4, s, X, Wm, out, K, NL, Co, KB);
-    } else if (NL >= 16384) {
-        hipLaunchKernelGGL((col_fwd_lds_kernel<16, 1, false, 8, 1>), dim3((unsigned)ceil_div_l(NL, 256), ceil_div(Co, 16)),
-                           dim3(256), KB * 16 * 4, s, X, Wm, out, K, NL, Co, KB);
+    const bool vec2 = NL % 2 == 0 && aligned8(X) && aligned8(out);
+    const long tiles = ceil_div_l(NL, 128) * ceil_div(Co, 16);
+    if (ceil_div_l(NL, 512) * ceil_div(Co, 16) >= 512) {
+        if (vec2 && NL >= 65536) launch_col_fwd_t<16, 2, true, 8, 1>(X, Wm, out, K, NL, Co, s);
+        else launch_col_fwd_t<16, 1, false, 8, 1>(X, Wm, out, K, NL, Co, s);
+    } else if (tiles >= 512) {
+        if (vec2) launch_col_fwd_t<16, 2, true, 4, 4>(X, Wm, out, K, NL, Co, s);
+        else launch_col_fwd_t<16, 1, false, 8, 4>(X, Wm, out, K, NL, Co, s);
+    } else if (tiles >= 128 && vec2) {
+        launch_col_fwd_t<8, 2, true, 8, 4>(X, Wm, out, K, NL, Co, s);
     } else {
-        // few columns: the work is a chain of row batches per wave -- 8 rows of W per lane (more workgroups) and the
-        // rows of X split over the four waves of a workgroup
-        hipLaunchKernelGGL((col_fwd_lds_kernel<8, 1, false, 8, 4>), dim3((unsigned)ceil_div_l(NL, 64), ceil_div(Co, 8)),
-                           dim3(256), KB * 8 * 4, s, X, Wm, out, K, NL, Co, KB);
+        launch_col_fwd_t<8, 1, false, 8, 4>(X, Wm, out, K, NL, Co, s);
     }
     return check_launch();
 }
@@ -775,9 +835,10 @@ static ColGwPlan plan_col_grad_w(int K, long NL, int Co) {
     else { p.ct = 2; p.kt = ktn < 2 ? 1 : 2; }
     p.gz = ceil_div(Co, 16 * p.ct);
     p.gy = ceil_div(K, 16 * p.kt);
-    // two workgroups per CU (two waves per SIMD: the accumulator tiles are chosen to leave room for that), at least
-    // one 16-column group per wave
-    long want = ceil_div_l(512, (long)p.gy * p.gz);
+    // at most two workgroups per CU (two waves per SIMD: the accumulator tiles are chosen to leave room for that; a few
+    // more than 512 would be a second round for them alone: Co = 32, K = 288, NL = 65536, 513 workgroups 42 us, 504 33 us;
+    // 64, 576, 32768, 71 -> 56; 200, 300, 30000, 112 -> 93), at least one 16-column group per wave
+    long want = 512 / ((long)p.gy * p.gz);
     const long most = ceil_div_l(NL / 16, 4);
     if (want > most) want = most;
     p.slots = (int)(want < 1 ? 1 : want);
@@ -873,9 +934,10 @@ int launch_col_grad_x(const float *gy, const float *X, const float *Wm, float *g
                                dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB);
         return check_launch();
     }
-    constexpr int TK = 8;
-    hipLaunchKernelGGL(col_grad_x_kernel<TK>, dim3((unsigned)ceil_div_l(NL, 256), ceil_div(K, TK)), dim3(256), 0, s,
-                       gy, X, Wm, gX, K, NL, Co);
+    constexpr int TK = kColGradXRows;
+    const int CB = Co < 512 ? Co : 512;   // output channels per LDS block of weights (16 KB), a multiple of 64 or all
+    hipLaunchKernelGGL(col_grad_x_kernel, dim3((unsigned)ceil_div_l(NL, 256), ceil_div(K, TK)), dim3(256), CB * TK * 4, s, gy,
+                       X, Wm, gX, K, NL, Co, CB);
     return check_launch();
 }
 

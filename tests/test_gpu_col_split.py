@@ -1,0 +1,56 @@
+"""Column-matrix kernels at the lines of their dispatch: forward tiles whose waves split the rows of X, input gradients of
+more than 32 output channels, weight-gradient slabs that fill whole rounds of workgroups."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (Co, K, NL).  Forward: 512 workgroups of 512 columns and one fewer, even and odd NL; 512 and 128 tiles of 128 columns, and
+# one fewer; rows of X that do not divide by four waves or by a block of 256; fewer rows than waves.
+FORWARD = [(16, 37, 512 * 512), (16, 37, 511 * 512), (16, 20, 511 * 512 + 1), (16, 20, 511 * 512 - 1), (17, 259, 256 * 128),
+           (17, 259, 255 * 128), (33, 513, 255 * 64 + 1), (16, 130, 128 * 128), (16, 130, 127 * 128), (20, 257, 16 * 1024),
+           (16, 3, 65536), (15, 1, 65538), (100, 2, 16386)]
+# Input gradient: one output channel above 32, around the folds at 64 and the blocks of 512, rows of X around groups of
+# eight, columns around 256; grad_W: 9 blocks (504 workgroups), more than 512 blocks (one slab)
+BACKWARD = [(33, 8, 2049), (63, 9, 2303), (64, 7, 2304), (65, 17, 2305), (511, 8, 2052), (512, 11, 2053), (513, 8, 2052),
+            (521, 3, 2049), (1030, 9, 2051), (32, 288, 4096), (64, 576, 4100), (260, 2304, 2064)]
+
+
+def _data(Co, K, NL, gpu, seed):
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    return (torch.randn(K, NL, device=gpu, generator=g), torch.randn(Co, K, device=gpu, generator=g),
+            torch.randn(Co, NL, device=gpu, generator=g))
+
+
+@pytest.mark.parametrize("case", FORWARD, ids=str)
+def test_forward(case, gpu):
+    from addernetcuda_amd import adder_cuda
+    X, W, _ = _data(*case, gpu, 3)
+    X[:, -1] = float("inf")                              # a column of its own: no other sees it
+    out = torch.full((case[0], case[2]), 7.0, device=gpu)
+    adder_cuda.ADDER_CONV(X, W, out)
+    want = torch.stack([-(w.double()[:, None] - X.double()).abs().sum(0) for w in W])
+    assert torch.isinf(out[:, -1]).all() and (out[:, -1] < 0).all()
+    # first-level sums of at most 64 terms of mean 1.1, then K / 64 of those: 2^-24 * (64 + K / 64 + 4) of the result
+    bound = 2.0 ** -24 * (64 + case[1] / 64 + 4) * want[:, :-1].abs() + 1e-6
+    assert ((out[:, :-1].double() - want[:, :-1]).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("case", BACKWARD, ids=str)
+def test_backward(case, gpu):
+    from addernetcuda_amd import adder_cuda
+    Co, K, NL = case
+    X, W, G = _data(*case, gpu, 4)
+    gw, gx = torch.ones_like(W), torch.ones_like(X)      # accumulated into
+    adder_cuda.ADDER_BACKWARD(G, X, W, gw, gx)
+    Xd, Wd, Gd = X.double(), W.double(), G.double()
+    want = torch.stack([((Wd[:, k, None] - Xd[k]).clamp(-1, 1) * Gd).sum(0) for k in range(K)])
+    size = torch.stack([((Wd[:, k, None] - Xd[k]).clamp(-1, 1) * Gd).abs().sum(0) for k in range(K)])
+    # the difference w - x and the products round once each; sums of at most 64 terms, then Co / 64 of those.  Up to 32
+    # output channels the clamp is 2 sat(..) - 1: the sum of |gy| stands in for that of the products
+    size = torch.maximum(size, Gd.abs().sum(0)) if Co <= 32 else size
+    assert ((gx.double() - 1 - want).abs() <= 2.0 ** -24 * (64 + Co / 64 + 8) * (size + 1) * (2 if Co <= 32 else 1)).all()
+    want_w = Gd @ Xd.t() - Wd * Gd.sum(1, keepdim=True)
+    # fp64 products and sums, one rounding of each of the two terms and of the result
+    size_w = Gd.abs() @ Xd.abs().t() + Wd.abs() * Gd.abs().sum(1, keepdim=True)
+    assert ((gw.double() - 1 - want_w).abs() <= 2.0 ** -24 * 4 * (size_w + 1)).all()
