@@ -1068,6 +1068,137 @@ static int rows_per_tile_w32(int H) {
 static_assert(GxW32::TM == GxW16::TM && GxW16::TM == GxW8::TM && GxS2W32::TM == GxS2W16::TM,
               "the launcher checks Ci against one TM per stride");
 
+// ---------------------------------------------------------------------------
+// Few positions: one input position x TM input channels per lane, the waves of a workgroup share the output channels
+// (the forward's counterpart of this kernel is fwd_few_kernel).  Wave v takes the chunks v, v + waves, ... of `chunk` output
+// channels, with gy (read from global memory: a map this small sits in L1 / L2) and the weights G output channels ahead
+// of the arithmetic; the chunk sums go through LDS and are added in channel order.
+// ---------------------------------------------------------------------------
+template <int KS, int TM, int G, class T>
+__global__ __launch_bounds__(512) void grad_x_few_kernel(const T *__restrict__ gy, const T *__restrict__ x,
+                                                         const float *__restrict__ w, T *__restrict__ gx,
+                                                         const T *__restrict__ gadd, ConvDims d, int chunk) {
+    constexpr int KK = KS * KS;
+    __shared__ float part[8][TM][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int plane = d.H * d.W, total = d.N * plane, K = d.Ci * KK;   // (stride 1, pad KS / 2: gy has the planes of x)
+    // the last group of channels is shifted down to end at Ci; channels below ci_first are not stored by it
+    const int ci_first = blockIdx.y * TM, ci0 = min(ci_first, d.Ci - TM);
+    const int pos = min((int)blockIdx.x * 64 + lane, total - 1);
+    const int n = pos / plane, hi = pos % plane / d.W, wi = pos % plane % d.W;
+    int off[KK];
+    bool ok[KK];
+#pragma unroll
+    for (int e = 0; e < KK; ++e) {
+        const int ho = hi + KS / 2 - e / KS, wo = wi + KS / 2 - e % KS;
+        ok[e] = ho >= 0 && ho < d.H && wo >= 0 && wo < d.W;
+        off[e] = n * d.Co * plane + (ok[e] ? ho * d.W + wo : 0);
+    }
+    uniform_f32_ptr wc = as_uniform(w) + ci0 * KK;
+    float xv[TM];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) xv[m] = ldf(x + ((size_t)n * d.Ci + ci0 + m) * plane + pos % plane);
+    const int nchunks = ceil_div(d.Co, chunk);
+    float tot[TM];   // of result threadIdx.x + k * blockDim.x of the workgroup's TM x 64
+#pragma unroll
+    for (int k = 0; k < TM; ++k) tot[k] = 0.f;
+
+    for (int c0 = 0; c0 < nchunks; c0 += waves) {
+        const int c = c0 + wave;
+        if (c < nchunks) {
+            const int first = c * chunk, end = min(first + chunk, d.Co);
+            float acc[TM], gv[2][G * KK], wv[2][G * TM * KK];
+#pragma unroll
+            for (int m = 0; m < TM; ++m) acc[m] = 0.f;
+            auto load = [&](const int b, const int co) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const int cc = min(co + g, end - 1);
+#pragma unroll
+                    for (int e = 0; e < TM * KK; ++e) wv[b][g * TM * KK + e] = wc[cc * K + e];
+                    const T *gc = gy + (size_t)cc * plane;
+#pragma unroll
+                    for (int e = 0; e < KK; ++e) gv[b][g * KK + e] = ldf(gc + off[e]);
+                }
+            };
+            auto add = [&](const int b, const int co) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    if (co + g >= end) break;
+#pragma unroll
+                    for (int e = 0; e < KK; ++e) {
+                        const float v = ok[e] ? gv[b][g * KK + e] : 0.f;
+#pragma unroll
+                        for (int m = 0; m < TM; ++m)
+                            acc[m] = fmaf(hardtanh(wv[b][(g * TM + m) * KK + e] - xv[m]), v, acc[m]);
+                    }
+                }
+            };
+            load(0, first);
+#pragma unroll 1
+            for (int co = first; co < end; co += 2 * G) {
+                load(1, co + G);
+                __builtin_amdgcn_sched_barrier(0);
+                add(0, co);
+                load(0, co + 2 * G);
+                __builtin_amdgcn_sched_barrier(0);
+                add(1, co + G);
+            }
+#pragma unroll
+            for (int m = 0; m < TM; ++m) part[wave][m][lane] = acc[m];
+        }
+        __syncthreads();
+        const int here = min(waves, nchunks - c0);
+#pragma unroll
+        for (int k = 0; k < TM; ++k) {
+            const int e = threadIdx.x + k * blockDim.x;
+            if (e < TM * 64)
+                for (int v = 0; v < here; ++v) tot[k] += part[v][e >> 6][e & 63];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < TM; ++k) {
+        const int e = threadIdx.x + k * blockDim.x, p = blockIdx.x * 64 + (e & 63), ci = ci0 + (e >> 6);
+        if (e < TM * 64 && p < total && ci >= ci_first) {
+            const size_t o = ((size_t)(p / plane) * d.Ci + ci) * plane + p % plane;
+            stf(gx + o, gadd ? tot[k] + ldf(gadd + o) : tot[k]);
+        }
+    }
+}
+
+// output channels per first-level sum: 72 terms with nine taps, 16 to 64 with one
+static int few_chunk(const ConvDims &d) {
+    const int eighth = round_up(ceil_div(d.Co, 8), 8);
+    return d.kh == 3 ? 8 : eighth < 16 ? 16 : eighth > 64 ? 64 : eighth;
+}
+
+// Whether it takes a 3x3 / pad 1 or 1x1 layer of stride 1.  The tiled kernels last as long as one wave's chain of output
+// channels x taps x results per lane, 5.5 ns a term with nine taps and 9.5 with one, until the chip is full; this one has a
+// chain of its share of the output channels (0.45 / 0.15 us each) and then works at 9 / 6.5 terms per ps.  Fitted to 60
+// layers; us, tiled -> this: 37 -> 51 3x3 @27x19, 7 images, 43 -> 13; 64 -> 64 @8x8, 1 / 64 images, 29 -> 6, 30 -> 19; 512 -> 512
+// @7x7, 1 / 7 images, 267 -> 38, 323 -> 111; 128 -> 128 @16x16, 1 / 7, 90 -> 11, 92 -> 36; 64 -> 512 1x1 @8x8, 16, 44 -> 10; 512 -> 2048
+// 1x1 @7x7, 4, 202 -> 76.  Beyond the line: 16 -> 16 @32x32, 64 images, 17 against 19; 1024 -> 256 1x1 @14x14, 7, 43 against 59.
+static bool few_positions(const ConvDims &d, int per_lane) {
+    const bool nine = d.kh == 3;
+    const int chunk = few_chunk(d);
+    const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
+    const float tiled = nine ? 2.f + 0.0055f * 9 * per_lane * d.Co : 3.f + 0.0095f * per_lane * d.Co;
+    const float share = (float)(ceil_div(ceil_div(d.Co, chunk), 8) * chunk);
+    const float few = nine ? 2.f + 0.45f * share + terms / 9e6f : 3.f + 0.15f * share + terms / 6.5e6f;
+    return few < 0.9f * tiled;
+}
+
+template <int KS, class T>
+static int launch_grad_x_few(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
+    constexpr int TM = 4, G = KS == 1 ? 8 : 1;
+    const int chunk = few_chunk(d);
+    const int chunks = ceil_div(d.Co, chunk), waves = chunks < 8 ? chunks : 8;
+    hipLaunchKernelGGL((grad_x_few_kernel<KS, TM, G, T>), dim3(ceil_div(d.N * d.H * d.W, 64), ceil_div(d.Ci, TM)),
+                       dim3(64 * waves), 0, s, gy, x, w, gx, gadd, d, chunk);
+    return check_launch();
+}
+
 // gadd (nullable): a tensor shaped like gx that is added to the result (tiled 3x3 / pad 1, 5x5 / pad 2 / stride 1 and tiled
 // 1x1 stride-1 kernels only; ADDER_ERR_UNSUPPORTED elsewhere)
 // Both storage types take the same kernels and tile shapes.  (bfloat16 layers other than 3x3 once went to the generic
@@ -1077,6 +1208,8 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
     const bool k3s1p1 = d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1;
     const bool aligned = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
     if (k3s1p1 && d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned)) {
+        if (few_positions(d, d.W > 16 ? GxW32::TM * GxW32::TN : d.W > 8 ? GxW16::TM * GxW16::TN : GxW8::TM * GxW8::TN))
+            return launch_grad_x_few<3>(gy, x, w, gx, d, s, gadd);
         if (d.W > 16) switch (rows_per_tile_w32(d.H)) {
             case 16: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
             case 8: return launch_grad_x_3x3s1<GxW32H8, false, T>(gy, x, w, gx, d, s, gadd);
@@ -1102,6 +1235,8 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         f.H = f.Ho = 1;
         f.W = f.Wo = d.H * d.W;
         if (f.W % 4 != 0 || aligned) {
+            if ((f.W > 64 || small_plane_tile(f)) && few_positions(d, f.W > 64 ? Gx1x1::TM * Gx1x1::TN : Gx1x1t::TM * Gx1x1t::TN))
+                return launch_grad_x_few<1>(gy, x, w, gx, d, s, gadd);
             if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, false, T>(gy, x, w, gx, f, s, gadd);
             return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, false, T>(gy, x, w, gx, f, s, gadd)
                                        : launch_grad_x_3x3s1<Gx1x1s, false, T>(gy, x, w, gx, f, s, gadd);
