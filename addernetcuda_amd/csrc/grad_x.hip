@@ -1179,7 +1179,12 @@ static int few_chunk(const ConvDims &d) {
 // layers; us, tiled -> this: 37 -> 51 3x3 @27x19, 7 images, 43 -> 13; 64 -> 64 @8x8, 1 / 64 images, 29 -> 6, 30 -> 19; 512 -> 512
 // @7x7, 1 / 7 images, 267 -> 38, 323 -> 111; 128 -> 128 @16x16, 1 / 7, 90 -> 11, 92 -> 36; 64 -> 512 1x1 @8x8, 16, 44 -> 10; 512 -> 2048
 // 1x1 @7x7, 4, 202 -> 76.  Beyond the line: 16 -> 16 @32x32, 64 images, 17 against 19; 1024 -> 256 1x1 @14x14, 7, 43 against 59.
+// Not for float32 layers that have a BatchNorm-linked kernel (whole groups of four): linked and plain backward of a layer
+// give the same bits, and the linked kernels sum in the tiled order.
+static int grad_x_bn_variant(const ConvDims &d);
+template <class T>
 static bool few_positions(const ConvDims &d, int per_lane) {
+    if (sizeof(T) == 4 && grad_x_bn_variant(d)) return false;
     const bool nine = d.kh == 3;
     const int chunk = few_chunk(d);
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
@@ -1208,7 +1213,7 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
     const bool k3s1p1 = d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1;
     const bool aligned = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
     if (k3s1p1 && d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned)) {
-        if (few_positions(d, d.W > 16 ? GxW32::TM * GxW32::TN : d.W > 8 ? GxW16::TM * GxW16::TN : GxW8::TM * GxW8::TN))
+        if (few_positions<T>(d, d.W > 16 ? GxW32::TM * GxW32::TN : d.W > 8 ? GxW16::TM * GxW16::TN : GxW8::TM * GxW8::TN))
             return launch_grad_x_few<3>(gy, x, w, gx, d, s, gadd);
         if (d.W > 16) switch (rows_per_tile_w32(d.H)) {
             case 16: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
@@ -1235,7 +1240,7 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         f.H = f.Ho = 1;
         f.W = f.Wo = d.H * d.W;
         if (f.W % 4 != 0 || aligned) {
-            if ((f.W > 64 || small_plane_tile(f)) && few_positions(d, f.W > 64 ? Gx1x1::TM * Gx1x1::TN : Gx1x1t::TM * Gx1x1t::TN))
+            if ((f.W > 64 || small_plane_tile(f)) && few_positions<T>(d, f.W > 64 ? Gx1x1::TM * Gx1x1::TN : Gx1x1t::TM * Gx1x1t::TN))
                 return launch_grad_x_few<1>(gy, x, w, gx, d, s, gadd);
             if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, false, T>(gy, x, w, gx, f, s, gadd);
             return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, false, T>(gy, x, w, gx, f, s, gadd)

@@ -10,9 +10,9 @@ from tests.test_gpu_bf16 import _close_bf16
 pytestmark = pytest.mark.gpu
 
 # (N, Ci, H, W, Co, k, stride, pad)
-SHAPES = [(1, 4, 32, 32, 16, 3, 1, 1), (1, 64, 8, 8, 64, 3, 1, 1), (2, 33, 14, 14, 37, 3, 1, 1), (1, 6, 7, 7, 200, 3, 1, 1),
-          (3, 5, 1, 1, 17, 3, 1, 1), (1, 7, 9, 33, 40, 3, 1, 1), (7, 37, 27, 19, 51, 3, 1, 1), (1, 65, 8, 8, 48, 1, 1, 0),
-          (2, 66, 7, 7, 300, 1, 1, 0), (1, 127, 3, 3, 521, 1, 1, 0), (1, 64, 14, 14, 130, 1, 1, 0), (1, 256, 28, 28, 64, 1, 1, 0)]
+SHAPES = [(1, 4, 32, 31, 16, 3, 1, 1), (1, 64, 8, 8, 64, 3, 1, 1), (1, 64, 9, 7, 64, 3, 1, 1), (2, 33, 14, 14, 37, 3, 1, 1), (1, 6, 7, 7, 200, 3, 1, 1),
+          (3, 5, 1, 1, 17, 3, 1, 1), (1, 7, 9, 33, 40, 3, 1, 1), (7, 37, 27, 19, 51, 3, 1, 1), (1, 65, 9, 7, 48, 1, 1, 0),
+          (2, 66, 7, 7, 300, 1, 1, 0), (1, 127, 3, 3, 521, 1, 1, 0), (1, 64, 13, 15, 130, 1, 1, 0), (1, 256, 27, 27, 64, 1, 1, 0)]
 
 
 def _grad_x(x, w, gy, case):
@@ -44,7 +44,7 @@ def test_agrees_with_a_large_batch(case, gpu):
     assert torch.equal(_grad_x(x, w, gy, case), few)     # no race: the same bits again
 
 
-@pytest.mark.parametrize("case", [SHAPES[2], SHAPES[8]], ids=str)
+@pytest.mark.parametrize("case", [SHAPES[3], SHAPES[9]], ids=str)
 def test_second_gradient_is_added_once(case, gpu):
     import ctypes
     from addernetcuda_amd._lib import lib, ptr, stream_ptr
