@@ -44,6 +44,7 @@ _SIGNATURES = {
     "adder_col_fwd_f32": (_i, [_p, _p, _p, _i, _l, _i, _p]),
     "adder_col_bwd_workspace_bytes": (_i, [_i, _l, _i, _szp]),
     "adder_col_bwd_f32": (_i, [_p, _p, _p, _p, _p, _i, _l, _i, _p, _sz, _p]),
+    "adder_col_bwd_set_f32": (_i, [_p, _p, _p, _p, _p, _i, _l, _i, _p, _sz, _p]),
     "adder_col_gradw_f32": (_i, [_p, _p, _p, _p, _i, _l, _i, _p, _sz, _p]),
     "adder_col_gradx_f32": (_i, [_p, _p, _p, _p, _i, _l, _i, _p]),
     "adder_norm_scale_workspace_bytes": (_i, [_l, _szp]),

@@ -41,9 +41,9 @@ class adder(Function):
     def backward(ctx, grad_output):
         W_col, X_col = ctx.saved_tensors
         grad_output = grad_output.contiguous()
-        grad_W_col = torch.zeros_like(W_col)
-        grad_X_col = torch.zeros_like(X_col)
-        adder_cuda.ADDER_BACKWARD(grad_output, X_col, W_col, grad_W_col, grad_X_col)
+        grad_W_col = torch.empty_like(W_col)
+        grad_X_col = torch.empty_like(X_col)
+        adder_cuda.backward_set(grad_output, X_col, W_col, grad_W_col, grad_X_col)
         if ctx.eta:
             dev = grad_W_col.device
             n = grad_W_col.numel()

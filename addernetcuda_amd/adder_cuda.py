@@ -73,14 +73,23 @@ def ADDER_CONV_INPUT(grad_y, x, w, grad_i):
 
 def ADDER_BACKWARD(grad_y, x, w, grad_w, grad_i):
     """Both gradients in one call   (adder_cuda.cpp:74-86)."""
+    _backward(lib.adder_col_bwd_f32, grad_y, x, w, grad_w, grad_i)
+
+
+def backward_set(grad_y, x, w, grad_w, grad_i):
+    """ADDER_BACKWARD that overwrites ``grad_w`` and ``grad_i`` instead of adding to them."""
+    _backward(lib.adder_col_bwd_set_f32, grad_y, x, w, grad_w, grad_i)
+
+
+def _backward(entry, grad_y, x, w, grad_w, grad_i):
     for t, n in ((grad_y, "grad_y"), (x, "x"), (w, "w"), (grad_w, "grad_w"), (grad_i, "grad_i")):
         require_gpu_f32(t, n)
     dev = same_device(grad_y, x, w, grad_w, grad_i)
     K, NL, Co = _col_shapes(x, w, grad_y=grad_y, grad_w=grad_w, grad_i=grad_i)
     with on_device(dev):
         ws, nbytes = _ws(K, NL, Co, dev)
-        check(lib.adder_col_bwd_f32(ptr(grad_y), ptr(x), ptr(w), ptr(grad_w), ptr(grad_i), K, NL, Co, ptr(ws),
-                                    nbytes, stream_ptr(dev)), "ADDER_BACKWARD")
+        check(entry(ptr(grad_y), ptr(x), ptr(w), ptr(grad_w), ptr(grad_i), K, NL, Co, ptr(ws), nbytes, stream_ptr(dev)),
+              "ADDER_BACKWARD")
 
 
 __all__ = ["ADDER_CONV", "ADDER_CONV_WEIGHT", "ADDER_CONV_INPUT", "ADDER_BACKWARD"]

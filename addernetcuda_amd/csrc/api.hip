@@ -409,19 +409,29 @@ int adder_col_gradx_f32(const float *gy, const float *Xcol, const float *Wcol, f
     return launch_col_grad_x(gy, Xcol, Wcol, gX, K, NL, Co, static_cast<hipStream_t>(stream));
 }
 
-int adder_col_bwd_f32(const float *gy, const float *Xcol, const float *Wcol, float *gW, float *gX, int K,
-                      long NL, int Co, void *ws, size_t ws_bytes, void *stream) {
+static int col_bwd(const float *gy, const float *Xcol, const float *Wcol, float *gW, float *gX, int K, long NL, int Co,
+                   void *ws, size_t ws_bytes, void *stream, bool add) {
     if (!gy || !Xcol || !Wcol || !gW || !gX) return ADDER_ERR_NULL_POINTER;
     if (int rc = check_col(K, NL, Co)) return rc;
     if (int rc = col_alias(gy, Xcol, Wcol, gW, gX, K, NL, Co)) return rc;
     if (int rc = check_col_ws(ws, ws_bytes, K, NL, Co)) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int small = launch_col_bwd_small(gy, Xcol, Wcol, gW, gX, K, NL, Co, s);   // few columns: one launch
+    const int small = launch_col_bwd_small(gy, Xcol, Wcol, gW, gX, K, NL, Co, s, add);   // few columns: one launch
     if (small != ADDER_ERR_UNSUPPORTED) return small;
-    const int fused = launch_col_bwd_fused(gy, Xcol, Wcol, gW, gX, K, NL, Co, ws, s);   // one pass over Xcol where it applies
+    const int fused = launch_col_bwd_fused(gy, Xcol, Wcol, gW, gX, K, NL, Co, ws, s, add);   // one pass over Xcol where it applies
     if (fused != ADDER_ERR_UNSUPPORTED) return fused;
-    if (int rc = launch_col_grad_x(gy, Xcol, Wcol, gX, K, NL, Co, s)) return rc;
-    return launch_col_grad_w(gy, Xcol, Wcol, gW, K, NL, Co, ws, s);
+    if (int rc = launch_col_grad_x(gy, Xcol, Wcol, gX, K, NL, Co, s, add)) return rc;
+    return launch_col_grad_w(gy, Xcol, Wcol, gW, K, NL, Co, ws, s, add);
+}
+
+int adder_col_bwd_f32(const float *gy, const float *Xcol, const float *Wcol, float *gW, float *gX, int K,
+                      long NL, int Co, void *ws, size_t ws_bytes, void *stream) {
+    return col_bwd(gy, Xcol, Wcol, gW, gX, K, NL, Co, ws, ws_bytes, stream, true);
+}
+
+int adder_col_bwd_set_f32(const float *gy, const float *Xcol, const float *Wcol, float *gW, float *gX, int K,
+                          long NL, int Co, void *ws, size_t ws_bytes, void *stream) {
+    return col_bwd(gy, Xcol, Wcol, gW, gX, K, NL, Co, ws, ws_bytes, stream, false);
 }
 
 int adder_norm_scale_workspace_bytes(long n, size_t *bytes) {

@@ -5,8 +5,9 @@
 // Replaces adder_cuda/adder.cu:19-70 (CONV), 72-131 (CONV_WEIGHT), 133-192
 // (CONV_INPUT) and 194-272 (CONV_BACKWARD) for callers that already hold an
 // unfolded X_col.  Gradients ACCUMULATE into their outputs, as the reference's
-// atomicAdd kernels do into caller-zeroed buffers; the sums themselves are
-// deterministic (fixed order, no atomics).
+// atomicAdd kernels do into caller-zeroed buffers (add = false writes them: the
+// autograd function would only fill zeros for that, and gX is as large as X); the
+// sums themselves are deterministic (fixed order, no atomics).
 #include "common.hpp"
 
 namespace adder {
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(256) void col_grad_x_reg_kernel(const float *__rest
                                                              const float *__restrict__ X,
                                                              const float *__restrict__ Wm,
                                                              float *__restrict__ gX, int K, long NL, int Co,
-                                                             int KB) {
+                                                             int KB, bool add) {
     constexpr int PF = 4;
     extern __shared__ __align__(16) float wt[];   // [KB][COB]
     const int k0 = blockIdx.y * KB, kcnt = min(KB, K - k0);
@@ -231,13 +232,16 @@ __global__ __launch_bounds__(256) void col_grad_x_reg_kernel(const float *__rest
         }
     };
 
+    auto before = [&](const int k) {   // what the result is added to
+        return add ? col_load<COLS, VEC>(gX + (size_t)k * NL, c0, NL) : ColVec<COLS>{};
+    };
     ColVec<COLS> nx[PF], no[PF];
     const int kfull = kcnt / PF * PF;
     if (kfull > 0) {
 #pragma unroll
         for (int r = 0; r < PF; ++r) {
             nx[r] = col_load<COLS, VEC>(X + (size_t)(k0 + r) * NL, c0, NL);
-            no[r] = col_load<COLS, VEC>(gX + (size_t)(k0 + r) * NL, c0, NL);
+            no[r] = before(k0 + r);
         }
     }
     for (int kk = 0; kk < kfull; kk += PF) {
@@ -248,15 +252,14 @@ __global__ __launch_bounds__(256) void col_grad_x_reg_kernel(const float *__rest
 #pragma unroll
             for (int r = 0; r < PF; ++r) {
                 nx[r] = col_load<COLS, VEC>(X + (size_t)(k0 + kk + PF + r) * NL, c0, NL);
-                no[r] = col_load<COLS, VEC>(gX + (size_t)(k0 + kk + PF + r) * NL, c0, NL);
+                no[r] = before(k0 + kk + PF + r);
             }
         }
 #pragma unroll
         for (int r = 0; r < PF; ++r) one_row(kk + r, cx[r], co_[r]);
     }
     for (int kk = kfull; kk < kcnt; ++kk)
-        one_row(kk, col_load<COLS, VEC>(X + (size_t)(k0 + kk) * NL, c0, NL),
-                col_load<COLS, VEC>(gX + (size_t)(k0 + kk) * NL, c0, NL));
+        one_row(kk, col_load<COLS, VEC>(X + (size_t)(k0 + kk) * NL, c0, NL), before(k0 + kk));
 }
 
 // ---------------------------------------------------------------------------
@@ -277,7 +280,7 @@ static constexpr int kFusedPitch = 132;   // floats per staged row of 128 column
 __global__ __launch_bounds__(256) void col_bwd_fused_kernel(const float *__restrict__ gy, const float *__restrict__ X,
                                                             const float *__restrict__ Wm, float *__restrict__ gX,
                                                             double *__restrict__ part, double *__restrict__ sgpart,
-                                                            int K, long NL, int Co, int KB) {
+                                                            int K, long NL, int Co, int KB, bool add) {
     constexpr int COB = 16, PF = 8;
     extern __shared__ __align__(16) float smem[];
     float *wt = smem;                                          // [KB][16] transposed weights of this row block
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(256) void col_bwd_fused_kernel(const float *__restr
 
     float2 nx[PF], no[PF];
 #pragma unroll
-    for (int r = 0; r < PF; ++r) { nx[r] = ld2(X, r); no[r] = ld2(gX, r); }
+    for (int r = 0; r < PF; ++r) { nx[r] = ld2(X, r); no[r] = add ? ld2(gX, r) : make_float2(0.f, 0.f); }
     const int nbatches = ceil_div(kcnt, 16);
     for (int b = 0; b < nbatches; ++b) {
 #pragma unroll
@@ -346,7 +349,10 @@ __global__ __launch_bounds__(256) void col_bwd_fused_kernel(const float *__restr
             for (int r = 0; r < PF; ++r) { cx[r] = nx[r]; co_[r] = no[r]; }
             const int kb = b * 16 + h * PF;
 #pragma unroll
-            for (int r = 0; r < PF; ++r) { nx[r] = ld2(X, kb + PF + r); no[r] = ld2(gX, kb + PF + r); }
+            for (int r = 0; r < PF; ++r) {
+                nx[r] = ld2(X, kb + PF + r);
+                no[r] = add ? ld2(gX, kb + PF + r) : make_float2(0.f, 0.f);
+            }
 #pragma unroll
             for (int r = 0; r < PF; ++r) {
                 if (kb + r < kcnt) one_row(kb + r, cx[r], co_[r]);
@@ -392,7 +398,7 @@ static constexpr int kColGradXRows = 8;
 __global__ __launch_bounds__(256) void col_grad_x_kernel(const float *__restrict__ gy,
                                                          const float *__restrict__ X,
                                                          const float *__restrict__ Wm,
-                                                         float *__restrict__ gX, int K, long NL, int Co, int CB) {
+                                                         float *__restrict__ gX, int K, long NL, int Co, int CB, bool add) {
     constexpr int PF = 8, TK = kColGradXRows;
     static_assert(TK == 8 && 64 % PF == 0, "eight weights per output channel in LDS, 64 output channels between two folds of acc");
     extern __shared__ __align__(16) float wl[];   // [CB][TK]
@@ -450,7 +456,10 @@ __global__ __launch_bounds__(256) void col_grad_x_kernel(const float *__restrict
     if (active) {
 #pragma unroll
         for (int t = 0; t < TK; ++t)
-            if (k0 + t < K) gX[(size_t)(k0 + t) * NL + nl] += tot[t] + acc[t];
+            if (k0 + t < K) {
+                float *dst = gX + (size_t)(k0 + t) * NL + nl;
+                *dst = (add ? *dst : 0.f) + (tot[t] + acc[t]);
+            }
     }
 }
 
@@ -607,7 +616,7 @@ template <int TM, int TK>
 __global__ __launch_bounds__(256) void col_grad_w_kernel(const float *__restrict__ gy,
                                                          const float *__restrict__ X,
                                                          const float *__restrict__ Wm,
-                                                         float *__restrict__ gW, int K, long NL, int Co) {
+                                                         float *__restrict__ gW, int K, long NL, int Co, bool add) {
     const int k0 = blockIdx.x * TK, co0 = blockIdx.y * TM;
     int kk[TK], cc[TM];
 #pragma unroll
@@ -647,7 +656,8 @@ __global__ __launch_bounds__(256) void col_grad_w_kernel(const float *__restrict
         const int m = threadIdx.x / TK, t = threadIdx.x % TK;
         if (co0 + m < Co && k0 + t < K) {
             const int e = threadIdx.x;
-            gW[(size_t)(co0 + m) * K + k0 + t] += (float)((red[0][e] + red[1][e]) + (red[2][e] + red[3][e]));
+            float *dst = gW + (size_t)(co0 + m) * K + k0 + t;
+            *dst = (add ? *dst : 0.f) + (float)((red[0][e] + red[1][e]) + (red[2][e] + red[3][e]));
         }
     }
 }
@@ -668,7 +678,7 @@ __global__ __launch_bounds__(256) void col_grad_w_kernel(const float *__restrict
 template <int KB, int CPT, int GB>
 __global__ __launch_bounds__(256) void col_bwd_small_kernel(const float *__restrict__ gy, const float *__restrict__ X,
                                                             const float *__restrict__ Wm, float *__restrict__ gW,
-                                                            float *__restrict__ gX, int K, int NL, int Co) {
+                                                            float *__restrict__ gX, int K, int NL, int Co, bool add) {
     extern __shared__ __align__(16) float smem[];
     float *wl = smem;                      // [Co][KB] weights of this workgroup's rows
     float *red = smem + Co * KB;           // [4 waves][Co][KB + 1] wave sums
@@ -748,7 +758,10 @@ __global__ __launch_bounds__(256) void col_bwd_small_kernel(const float *__restr
 #pragma unroll
             for (int j = 0; j < CPT; ++j) {
                 const int c = threadIdx.x + j * 256;
-                if (k0 + kk < K && c < NL) gX[(size_t)(k0 + kk) * NL + c] += acc[kk][j];
+                if (k0 + kk < K && c < NL) {
+                    float *dst = gX + (size_t)(k0 + kk) * NL + c;
+                    *dst = (add ? *dst : 0.f) + acc[kk][j];
+                }
             }
     }
     if (gW) {
@@ -760,7 +773,8 @@ __global__ __launch_bounds__(256) void col_bwd_small_kernel(const float *__restr
             const float *r = red + co * (KB + 1);
             const float sxg = (r[kk] + r[stride + kk]) + (r[2 * stride + kk] + r[3 * stride + kk]);
             const float sg = (r[KB] + r[stride + KB]) + (r[2 * stride + KB] + r[3 * stride + KB]);
-            gW[(size_t)co * K + k0 + kk] += sxg - wl[e] * sg;
+            float *dst = gW + (size_t)co * K + k0 + kk;
+            *dst = (add ? *dst : 0.f) + (sxg - wl[e] * sg);
         }
     }
 }
@@ -770,12 +784,12 @@ static bool col_bwd_small_applies(int K, long NL, int Co) { return NL <= 2048 &&
 
 // gW / gX: either may be null
 int launch_col_bwd_small(const float *gy, const float *X, const float *Wm, float *gW, float *gX, int K, long NL, int Co,
-                         hipStream_t s) {
+                         hipStream_t s, bool add) {
     if (!col_bwd_small_applies(K, NL, Co)) return ADDER_ERR_UNSUPPORTED;
     const int cpt = (int)ceil_div_l(NL, 256);
 #define ADDER_COL_SMALL(KB, CPT, GB)                                                                                 \
     hipLaunchKernelGGL((col_bwd_small_kernel<KB, CPT, GB>), dim3(ceil_div(K, KB)), dim3(256),                            \
-                       (Co * KB + 4 * Co * (KB + 1)) * 4, s, gy, X, Wm, gW, gX, K, (int)NL, Co)
+                       (Co * KB + 4 * Co * (KB + 1)) * 4, s, gy, X, Wm, gW, gX, K, (int)NL, Co, add)
     // one row of X per workgroup while that fills the chip, two on taller matrices
     const bool tall = K >= 1024;
     if (cpt <= 1) { if (tall) ADDER_COL_SMALL(2, 1, 8); else ADDER_COL_SMALL(1, 1, 8); }
@@ -861,7 +875,7 @@ size_t col_grad_w_workspace_bytes(int K, long NL, int Co) {
 // Both gradients in one pass over X (col_bwd_fused_kernel); ADDER_ERR_UNSUPPORTED (nothing launched) where it does
 // not apply, and the caller runs the two separate kernels.
 int launch_col_bwd_fused(const float *gy, const float *X, const float *Wm, float *gW, float *gX, int K, long NL, int Co,
-                         void *ws, hipStream_t s) {
+                         void *ws, hipStream_t s, bool add) {
     if (!col_bwd_fused_applies(K, NL, Co) || !ws || !aligned8(X) || !aligned8(gy) || !aligned8(gX) ||
         (reinterpret_cast<uintptr_t>(ws) & 255))
         return ADDER_ERR_UNSUPPORTED;
@@ -873,9 +887,9 @@ int launch_col_bwd_fused(const float *gy, const float *X, const float *Wm, float
     double *part = reinterpret_cast<double *>(ws);
     double *sgpart = part + (size_t)slots * Co * K;
     hipLaunchKernelGGL(col_bwd_fused_kernel, dim3(slots, ceil_div(K, KB)), dim3(256), lds, s, gy, X, Wm, gX, part, sgpart,
-                       K, NL, Co, KB);
+                       K, NL, Co, KB, add);
     if (int rc = check_launch()) return rc;
-    return launch_grad_w_slab_finalize(part, sgpart, Wm, gW, slots, Co, K, /*accumulate=*/true, s);
+    return launch_grad_w_slab_finalize(part, sgpart, Wm, gW, slots, Co, K, /*accumulate=*/add, s);
 }
 
 template <int CT, int KT>
@@ -886,8 +900,8 @@ static void launch_col_gw(const float *gy, const float *X, double *part, double 
 }
 
 int launch_col_grad_w(const float *gy, const float *X, const float *Wm, float *gW, int K, long NL, int Co,
-                      void *ws, hipStream_t s) {
-    if (col_bwd_small_applies(K, NL, Co)) return launch_col_bwd_small(gy, X, Wm, gW, nullptr, K, NL, Co, s);
+                      void *ws, hipStream_t s, bool add) {
+    if (col_bwd_small_applies(K, NL, Co)) return launch_col_bwd_small(gy, X, Wm, gW, nullptr, K, NL, Co, s, add);
     const ColGwPlan p = plan_col_grad_w(K, NL, Co);
     if (p.mfma && ws && aligned16(X) && aligned16(gy) && (reinterpret_cast<uintptr_t>(ws) & 255) == 0) {
         double *part = reinterpret_cast<double *>(ws);
@@ -902,17 +916,17 @@ int launch_col_grad_w(const float *gy, const float *X, const float *Wm, float *g
             default: launch_col_gw<2, 2>(gy, X, part, sgpart, K, NL, Co, p, s); break;
         }
         if (int rc = check_launch()) return rc;
-        return launch_grad_w_slab_finalize(part, sgpart, Wm, gW, p.slots, Co, K, /*accumulate=*/true, s);
+        return launch_grad_w_slab_finalize(part, sgpart, Wm, gW, p.slots, Co, K, /*accumulate=*/add, s);
     }
     constexpr int TM = 4, TK = 4;
     hipLaunchKernelGGL((col_grad_w_kernel<TM, TK>), dim3(ceil_div(K, TK), ceil_div(Co, TM)), dim3(256), 0, s, gy, X,
-                       Wm, gW, K, NL, Co);
+                       Wm, gW, K, NL, Co, add);
     return check_launch();
 }
 
 int launch_col_grad_x(const float *gy, const float *X, const float *Wm, float *gX, int K, long NL, int Co,
-                      hipStream_t s) {
-    if (col_bwd_small_applies(K, NL, Co)) return launch_col_bwd_small(gy, X, Wm, nullptr, gX, K, NL, Co, s);
+                      hipStream_t s, bool add) {
+    if (col_bwd_small_applies(K, NL, Co)) return launch_col_bwd_small(gy, X, Wm, nullptr, gX, K, NL, Co, s, add);
     if (Co <= 32) {
         // gy in registers, X streamed once; rows in blocks of KB whose weights fit a 32 KB LDS tile
         const int COB = Co <= 16 ? 16 : 32;
@@ -925,19 +939,19 @@ int launch_col_grad_x(const float *gy, const float *X, const float *Wm, float *g
         const bool vec2 = NL % 2 == 0 && aligned8(X) && aligned8(gy) && aligned8(gX) && NL >= 65536;
         if (COB == 16 && vec2)
             hipLaunchKernelGGL((col_grad_x_reg_kernel<16, 2, true>), dim3((unsigned)ceil_div_l(NL, 512), ceil_div(K, KB)),
-                               dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB);
+                               dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB, add);
         else if (COB == 16)
             hipLaunchKernelGGL((col_grad_x_reg_kernel<16, 1, false>), dim3((unsigned)colblocks, ceil_div(K, KB)),
-                               dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB);
+                               dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB, add);
         else
             hipLaunchKernelGGL((col_grad_x_reg_kernel<32, 1, false>), dim3((unsigned)colblocks, ceil_div(K, KB)),
-                               dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB);
+                               dim3(256), lds, s, gy, X, Wm, gX, K, NL, Co, KB, add);
         return check_launch();
     }
     constexpr int TK = kColGradXRows;
     const int CB = Co < 512 ? Co : 512;   // output channels per LDS block of weights (16 KB), a multiple of 64 or all
     hipLaunchKernelGGL(col_grad_x_kernel, dim3((unsigned)ceil_div_l(NL, 256), ceil_div(K, TK)), dim3(256), CB * TK * 4, s, gy,
-                       X, Wm, gX, K, NL, Co, CB);
+                       X, Wm, gX, K, NL, Co, CB, add);
     return check_launch();
 }
 

@@ -361,12 +361,12 @@ int launch_grad_w_slab_finalize(const double *part, const double *sgpart, const 
 int launch_col_fwd(const float *X, const float *W, float *out, int K, long NL, int Co, hipStream_t s);
 size_t col_grad_w_workspace_bytes(int K, long NL, int Co);
 int launch_col_grad_w(const float *gy, const float *X, const float *W, float *gW, int K, long NL,
-                      int Co, void *ws, hipStream_t s);
+                      int Co, void *ws, hipStream_t s, bool add = true);
 int launch_col_grad_x(const float *gy, const float *X, const float *W, float *gX, int K, long NL,
-                      int Co, hipStream_t s);
+                      int Co, hipStream_t s, bool add = true);
 int launch_col_bwd_small(const float *gy, const float *X, const float *W, float *gW, float *gX, int K, long NL, int Co,
-                         hipStream_t s);
+                         hipStream_t s, bool add = true);
 int launch_col_bwd_fused(const float *gy, const float *X, const float *W, float *gW, float *gX, int K, long NL, int Co,
-                         void *ws, hipStream_t s);
+                         void *ws, hipStream_t s, bool add = true);
 
 }  // namespace adder

@@ -206,6 +206,11 @@ ADDER_API int adder_col_bwd_f32(const float *gy, const float *Xcol, const float 
                       float *gW, float *gX, int K, long NL, int Co,
                       void *ws, size_t ws_bytes, void *stream);
 
+/* The same with gW = ..., gX = ...: the outputs need not be cleared first. */
+ADDER_API int adder_col_bwd_set_f32(const float *gy, const float *Xcol, const float *Wcol,
+                      float *gW, float *gX, int K, long NL, int Co,
+                      void *ws, size_t ws_bytes, void *stream);
+
 /* ADDER_CONV_WEIGHT (adder_cuda.cpp:48-59; adder.cu:72-131, 322-355): gW += sum_nl (X - W) * gy */
 ADDER_API int adder_col_gradw_f32(const float *gy, const float *Xcol, const float *Wcol,
                         float *gW, int K, long NL, int Co,

@@ -54,3 +54,15 @@ def test_backward(case, gpu):
     # fp64 products and sums, one rounding of each of the two terms and of the result
     size_w = Gd.abs() @ Xd.abs().t() + Wd.abs() * Gd.abs().sum(1, keepdim=True)
     assert ((gw.double() - 1 - want_w).abs() <= 2.0 ** -24 * 4 * (size_w + 1)).all()
+
+
+@pytest.mark.parametrize("case", [(32, 288, 1024), (3, 2050, 513), (16, 144, 65544), (9, 20, 70004), (24, 50, 66000), (33, 17, 2305),
+                                  (20, 100, 2051), (32, 288, 4096)], ids=str)
+def test_gradients_written_instead_of_added(case, gpu):
+    from addernetcuda_amd import adder_cuda
+    X, W, G = _data(*case, gpu, 5)
+    gw, gx = torch.zeros_like(W), torch.zeros_like(X)
+    adder_cuda.ADDER_BACKWARD(G, X, W, gw, gx)
+    gw2, gx2 = torch.full_like(W, float("nan")), torch.full_like(X, float("nan"))
+    adder_cuda.backward_set(G, X, W, gw2, gx2)
+    assert torch.equal(gw, gw2) and torch.equal(gx, gx2)
