@@ -129,11 +129,13 @@ __global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restric
             }
         }
         for (int kk = kfull; kk < ke; ++kk) one_row(kk, col_load<COLS, VEC>(X + (size_t)(k0 + kk) * NL, c0, NL));
+        // ... nor does it carry the rest of a block into the next one: a wave's share may be below 64 rows (carried on,
+        // 2016 rows on 16 x 8192 were off by 1.6e-7 of the result, 4e-8 like this)
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int e = 0; e < COLS; ++e) { tot[m][e] += acc[m][e]; acc[m][e] = 0.f; }
     }
-#pragma unroll
-    for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int e = 0; e < COLS; ++e) tot[m][e] += acc[m][e];
     if constexpr (KW > 1) {
         __shared__ float red[(KW - 1) * TM * COLS * 64];
         if (wave > 0) {

@@ -31,9 +31,24 @@ def test_forward(case, gpu):
     adder_cuda.ADDER_CONV(X, W, out)
     want = torch.stack([-(w.double()[:, None] - X.double()).abs().sum(0) for w in W])
     assert torch.isinf(out[:, -1]).all() and (out[:, -1] < 0).all()
-    # first-level sums of at most 64 terms of mean 1.1, then K / 64 of those: 2^-24 * (64 + K / 64 + 4) of the result
+    # first-level sums of at most 64 terms, at most K / 64 + 4 of those: 2^-24 * (64 + K / 64 + 4) of the result
     bound = 2.0 ** -24 * (64 + case[1] / 64 + 4) * want[:, :-1].abs() + 1e-6
     assert ((out[:, :-1].double() - want[:, :-1]).abs() <= bound).all()
+
+
+# one matrix per forward tile: unsplit by pairs and by single columns, split 16 x 128, 16 x 64, 8 x 128 and 8 x 64
+@pytest.mark.parametrize("K", [1000, 1025, 2016, 2049, 2200])
+@pytest.mark.parametrize("Co,NL", [(64, 65536), (128, 32767), (16, 65536), (33, 22001), (16, 16384), (16, 8191)], ids=str)
+def test_forward_of_many_rows_sums_in_two_levels(Co, NL, K, gpu):
+    from addernetcuda_amd import adder_cuda
+    X, W, _ = _data(Co, K, NL, gpu, 6)
+    out = torch.empty(Co, NL, device=gpu)
+    adder_cuda.ADDER_CONV(X, W, out)
+    want = torch.stack([-(w.double()[:, None] - X.double()).abs().sum(0) for w in W])
+    # The terms have one sign: a sum of n rounds to about 0.4 * 2^-24 * sqrt(n / 3) of itself.  First-level sums of
+    # n1 <= 64 of which n2 are added up: sqrt((n1 / n2 + n2) / 3), at most 3.5 for 2200 rows in one wave (n2 = 35), 8.3e-8;
+    # four waves that share the rows do better.  Sums of 250 terms and more, carried from block to block: from 1.1e-7.
+    assert (out.double() - want).norm() <= 1e-7 * want.norm()
 
 
 @pytest.mark.parametrize("case", BACKWARD, ids=str)
