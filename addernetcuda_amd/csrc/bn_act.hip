@@ -121,10 +121,13 @@ __device__ __forceinline__ void bn_reduce_partials(const T *__restrict__ part, i
 
 // BatchNorm with fixed statistics, shortcut and ReLU in one pass over groups of V elements.  One read and one write of the
 // tensor bound it (plus the shortcut's read); torch runs it as two or three launches, which is what a small map pays for.
+static constexpr unsigned kBnEvalBlocks = 4096;
 template <int V>
 __global__ __launch_bounds__(kBnThreads) void bn_eval_kernel(const float *__restrict__ x, float *__restrict__ y, const BnEval bn,
-                                                             int C, int HWV, int total) {
-    for (int i = blockIdx.x * kBnThreads + threadIdx.x; i < total; i += gridDim.x * kBnThreads) {
+                                                             unsigned C, unsigned HWV, unsigned total) {
+    // unsigned: total goes up to 2^31 - 1, and the last step past it must not wrap around
+    static_assert(0x7fffffffu < 0x7fffffffu + kBnEvalBlocks * kBnThreads, "the index ends past the largest tensor");
+    for (unsigned i = blockIdx.x * kBnThreads + threadIdx.x; i < total; i += gridDim.x * kBnThreads) {
         const BnEvalChannel ch(bn, i / HWV % C);
         const Pack<V> v = ld<V>(x, i);
         Pack<V> r;
@@ -389,16 +392,17 @@ static int bn_bwd_v(const float *dy, const float *y, const unsigned *mask, const
     return check_launch();
 }
 
-// mask (nullable): the sign bits the forward left; replaces y
 int launch_bn_eval(const float *x, float *y, const BnEval &bn, int N, int C, int HW, hipStream_t s) {
     const bool vec = HW % 4 == 0 && aligned_groups(x) && aligned_groups(y) && aligned_groups(bn.res);
-    const int total = (int)((long)N * C * HW / (vec ? 4 : 1));
-    const int blocks = (int)(ceil_div_l(total, kBnThreads) < 4096 ? ceil_div_l(total, kBnThreads) : 4096);
+    const unsigned total = (unsigned)((long)N * C * HW / (vec ? 4 : 1));
+    const long all = ceil_div_l(total, kBnThreads);
+    const unsigned blocks = all < kBnEvalBlocks ? (unsigned)all : kBnEvalBlocks;
     if (vec) hipLaunchKernelGGL(bn_eval_kernel<4>, dim3(blocks), dim3(kBnThreads), 0, s, x, y, bn, C, HW / 4, total);
     else hipLaunchKernelGGL(bn_eval_kernel<1>, dim3(blocks), dim3(kBnThreads), 0, s, x, y, bn, C, HW, total);
     return check_launch();
 }
 
+// mask (nullable): the sign bits the forward left; replaces y
 int launch_bn_act_bwd(const float *dy, const float *y, const unsigned *mask, const float *x, const float *gamma,
                       const float *mean, const float *rstd, float *dx, float *dres, float *dgamma, float *dbeta,
                       int relu, int N, int C, int HW, void *ws, hipStream_t s) {

@@ -118,3 +118,21 @@ def test_networks_in_evaluation_mode(name, gpu):
         got = net(images)
     # the BatchNorm keeps torch's roundings; the ordinary layers may be summed in another order
     assert (got - want).norm() <= 1e-4 * want.norm()
+
+
+def test_batch_norm_on_its_own_near_the_largest_tensor(gpu):
+    # 2^31 - 2^20 elements and more, moved one at a time: the last step of the index goes past 2^31
+    from addernetcuda_amd.bn_act import BatchNormAct2d
+    N, C, side = 21395, 2048, 7
+    assert (1 << 31) - (1 << 20) < N * C * side * side < 1 << 31 and side * side % 4
+    bn = BatchNormAct2d(C, relu=True).to(gpu).eval()
+    gen = torch.Generator(device=gpu).manual_seed(9)
+    with torch.no_grad():
+        for t in (bn.weight, bn.bias, bn.running_mean):
+            t.copy_(torch.randn(C, device=gpu, generator=gen))
+        bn.running_var.copy_(torch.rand(C, device=gpu, generator=gen) + 0.5)
+        x = torch.randn(N, C, side, side, device=gpu, generator=gen)
+        y = bn(x)
+        for n in range(0, N, 2048):
+            want = torch.relu(torch.nn.BatchNorm2d.forward(bn, x[n:n + 2048]))
+            assert torch.allclose(y[n:n + 2048], want, rtol=1e-5, atol=1e-5), f"images {n}.."
