@@ -20,6 +20,8 @@ lib = ctypes.CDLL(LIB_PATH)
 ADDER_OK, ADDER_ERR_NULL_POINTER, ADDER_ERR_BAD_SHAPE, ADDER_ERR_TOO_LARGE = 0, -1, -2, -3
 ADDER_ERR_WORKSPACE, ADDER_ERR_HIP, ADDER_ERR_ALIAS, ADDER_ERR_UNSUPPORTED = -4, -5, -6, -7
 
+MAX_ELEMENTS = 0x7fffffff   # of one tensor; entry points answer ADDER_ERR_TOO_LARGE above it
+
 _i, _l, _f, _p, _sz = ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t
 _szp = ctypes.POINTER(ctypes.c_size_t)
 

@@ -13,7 +13,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd import Function
 
-from ._lib import lib, check, ptr, stream_ptr, on_device, bn_act_sizes, plain_call
+from ._lib import lib, check, ptr, stream_ptr, on_device, bn_act_sizes, plain_call, MAX_ELEMENTS
 
 
 def _workspace(N, C, HW, device):
@@ -108,7 +108,8 @@ class BatchNormAct2d(nn.BatchNorm2d):
     def _eval_fusable(self, x, C, residual):
         """Whether the inference kernels can apply this module to C channels of values made from ``x``."""
         if (self.training or self.running_mean is None or self.running_var is None or not self.affine or not x.is_cuda
-                or x.dtype != torch.float32 or x.dim() != 4 or C != self.num_features or not plain_call(x)):
+                or x.dtype != torch.float32 or x.dim() != 4 or C != self.num_features or x.numel() > MAX_ELEMENTS
+                or not plain_call(x)):
             return False
         if residual is not None and not (plain_call(residual) and residual.dtype == torch.float32
                                          and residual.device == x.device and residual.is_contiguous()):

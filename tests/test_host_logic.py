@@ -155,3 +155,14 @@ def test_batched_eta_scaling_drops_unfinished_gradients_on_an_exceptional_exit()
             adder._eta_batch.append((w1, 0.2, None, None))
             adder._eta_batch.append((w2, 0.2, None, None))    # its .grad never arrived
     assert w1.grad is None and w2.grad is None and adder._eta_batch is None
+
+
+def test_evaluation_of_tensors_beyond_the_kernels_stays_with_torch(monkeypatch):
+    """The inference kernel takes 2^31 - 1 elements; torch's BatchNorm takes more, and gets them as before."""
+    from types import SimpleNamespace
+    from addernetcuda_amd import bn_act
+    bn = bn_act.BatchNormAct2d(4).eval()
+    monkeypatch.setattr(bn_act, "plain_call", lambda x: True)
+    like_gpu = lambda n: SimpleNamespace(is_cuda=True, dtype=torch.float32, device=bn.weight.device, dim=lambda: 4, numel=lambda: n)
+    assert bn._eval_fusable(like_gpu(2 ** 31 - 1), 4, None)
+    assert not bn._eval_fusable(like_gpu(2 ** 31), 4, None)
