@@ -4,6 +4,7 @@ import functools
 import os
 
 import torch
+from torch.utils._device import DeviceContext as _DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # ADDERNET_HIP_LIB: another build of the same library (a debug build, a tuning variant) instead of the in-tree one
@@ -158,10 +159,17 @@ def plain_call(x):
     """Whether ``x`` is an ordinary tensor in an ordinary call without gradients: nothing that records, transforms or
     differentiates the operators in between would miss those that one kernel does together."""
     return (type(x) is torch.Tensor and not torch.is_grad_enabled() and not _functorch_stack()
-            and _forward_ad._current_level < 0 and not _is_tracing() and not _is_compiling())
+            and _forward_ad._current_level < 0 and not _dispatch_modes() and (not _function_modes() or _only_default_device())
+            and not _is_tracing() and not _is_compiling())
+
+
+def _only_default_device():
+    # torch.set_default_device is a function mode too, which looks at the calls that make tensors and at nothing else
+    return all(type(torch._C._get_function_stack_at(i)) is _DeviceContext for i in range(_function_modes()))
 
 
 _functorch_stack, _forward_ad = torch._C._functorch.peek_interpreter_stack, torch.autograd.forward_ad
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 _is_tracing, _is_compiling = torch._C._is_tracing, torch.compiler.is_compiling
 
 

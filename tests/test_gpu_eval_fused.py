@@ -87,6 +87,11 @@ def test_what_stays_with_the_separate_modules(gpu):
         handle = layer.register_forward_hook(lambda m, a, out: seen.append(out))
         assert torch.allclose(adder_bn_act(layer, bn, x), want, rtol=1e-5, atol=1e-5) and len(seen) == 1
         handle.remove()
+        for module in (layer, bn):                                   # a forward of the instance (offloading, instrumentation)
+            calls, inner = [], module.forward
+            module.forward = lambda *a, **k: calls.append(1) or inner(*a, **k)
+            assert torch.allclose(adder_bn_act(layer, bn, x), want, rtol=1e-5, atol=1e-5) and calls == [1]
+            del module.forward
         res = torch.randn(1, 6, 1, 1, device=gpu)                    # a residual that broadcasts
         ref = torch.relu(torch.nn.BatchNorm2d.forward(bn, layer(x)) + res)
         assert torch.allclose(adder_bn_act(layer, bn, x, residual=res), ref, rtol=1e-5, atol=1e-5)

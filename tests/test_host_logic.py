@@ -166,3 +166,29 @@ def test_evaluation_of_tensors_beyond_the_kernels_stays_with_torch(monkeypatch):
     like_gpu = lambda n: SimpleNamespace(is_cuda=True, dtype=torch.float32, device=bn.weight.device, dim=lambda: 4, numel=lambda: n)
     assert bn._eval_fusable(like_gpu(2 ** 31 - 1), 4, None)
     assert not bn._eval_fusable(like_gpu(2 ** 31), 4, None)
+
+
+def test_one_launch_units_give_way_to_whoever_watches_the_operators():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from addernetcuda_amd._lib import plain_call
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class WatchCalls(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(2, 3)
+    assert not plain_call(x)
+    with torch.no_grad():
+        assert plain_call(x)
+        for mode in (Watch, WatchCalls):
+            with mode():
+                assert not plain_call(x)
+        with torch.device("cpu"):                 # a default device looks at the calls that make tensors only
+            assert plain_call(x)
+            with WatchCalls():
+                assert not plain_call(x)
