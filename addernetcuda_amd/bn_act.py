@@ -111,8 +111,9 @@ class BatchNormAct2d(nn.BatchNorm2d):
                 or x.dtype != torch.float32 or x.dim() != 4 or C != self.num_features or x.numel() > MAX_ELEMENTS
                 or not plain_call(x)):
             return False
-        if residual is not None and not (plain_call(residual) and residual.dtype == torch.float32
-                                         and residual.device == x.device and residual.is_contiguous()):
+        if residual is not None and not (type(residual) is torch.Tensor and residual.shape == x.shape
+                                         and residual.dtype == torch.float32 and residual.device == x.device
+                                         and residual.is_contiguous()):
             return False
         return all(t.dtype == torch.float32 and t.device == x.device and t.is_contiguous() and t.numel() == C
                    for t in (self.weight, self.bias, self.running_mean, self.running_var))
@@ -121,8 +122,7 @@ class BatchNormAct2d(nn.BatchNorm2d):
         """``stats``: optional per-channel partial sums of x and x*x from the layer that produced x
         (``adder2d.forward_with_stats``); they replace this module's own statistics pass."""
         if not self._fusable(x):
-            if (x.dim() == 4 and x.is_contiguous() and x.numel() and (residual is None or residual.shape == x.shape)
-                    and self._eval_fusable(x, x.shape[1], residual)):
+            if x.dim() == 4 and x.is_contiguous() and x.numel() and self._eval_fusable(x, x.shape[1], residual):
                 y = torch.empty_like(x)
                 with on_device(x.device):
                     check(lib.adder_bn_eval_f32(ptr(x), ptr(y), ptr(self.weight), ptr(self.bias), ptr(self.running_mean),

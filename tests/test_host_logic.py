@@ -192,3 +192,13 @@ def test_one_launch_units_give_way_to_whoever_watches_the_operators():
             assert plain_call(x)
             with WatchCalls():
                 assert not plain_call(x)
+
+
+def test_evaluation_adds_a_residual_that_is_a_number():
+    from addernetcuda_amd.bn_act import BatchNormAct2d
+    bn = BatchNormAct2d(3).eval()
+    x = torch.randn(2, 3, 4, 4)
+    want = torch.relu(torch.nn.BatchNorm2d.forward(bn, x) + 0.5)
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            assert torch.equal(bn(x, residual=0.5), want)
