@@ -45,6 +45,20 @@ def test_5x5_tensors_at_odd_addresses(case, gpu):
     _check(case, gpu, torch.float32, offset=1)
 
 
+@pytest.mark.parametrize("Ci", [272, 280, 813, 1024])
+@pytest.mark.parametrize("H,stride", [(20, 1), (12, 1), (7, 1), (20, 2), (13, 2)])
+def test_5x5_forward_of_many_channels_keeps_its_precision(H, stride, Ci, gpu):
+    from addernetcuda_amd import adder
+    from oracle import c_oracle
+    x, w, _ = make_case(1, Ci, H, H, 16, 5, stride, 2, w_init="normal")
+    want = c_oracle.conv2d_fwd(x, w, stride, 2)
+    got = adder.adder2d_function(x.to(gpu), w.to(gpu), stride, 2).double().cpu()
+    # One-signed terms: sums of 400 of which n2 = Ci / 16 are added up round to 0.4 * 2^-24 * sqrt((400 / n2 + n2) / 3) of the result --
+    # what the layer had as 16-channel sums without tiles (of 200, Ci / 8: 1.6e-7 at 813 channels against 1.1e-7)
+    n2 = Ci / 16
+    assert (got - want).norm() <= 1.2 * 0.4 * 2.0 ** -24 * ((400 / n2 + n2) / 3) ** 0.5 * want.norm()
+
+
 def test_without_a_workspace_where_the_slabs_do_not_fit(gpu):
     from addernetcuda_amd._lib import lib, ptr, stream_ptr, conv_dims, check, conv2d_bwd_workspace
     from oracle import c_oracle
