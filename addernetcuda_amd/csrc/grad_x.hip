@@ -308,8 +308,9 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
                 if (cc + 1 < ccnt) one_channel(cc + 1, 1);
                 // the two-instruction form folds its first-level sums every eight output channels (72 terms): with
                 // 144-term first levels its worst element sat at 0.71 of the parity tolerance for 1152 terms per
-                // output, with 72-term ones at 0.51.  25 taps: both forms, every four channels (100 terms)
-                if ((KS == 5 ? ((cc + 2) & 3) == 0 : SAT && KS == 3 && ((cc + 2) & 7) == 0) && cc + 2 < ccnt) {
+                // output, with 72-term ones at 0.51.  25 taps: both forms, every two channels (50 terms; at 2500 terms per
+                // output the worst element sits at 0.56, with 100-term sums at 0.88, and the time is the same)
+                if ((KS == 5 || (SAT && KS == 3 && ((cc + 2) & 7) == 0)) && cc + 2 < ccnt) {
 #pragma unroll
                     for (int m = 0; m < TM; ++m)
 #pragma unroll
@@ -549,7 +550,8 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
 // the three-instruction form sits at 0.45, and at 0.54 for 4608.  Layers with more than 1152 terms per output
 // therefore keep the three-instruction form.  Single-tap layers stop at 1024: their chunks are CC terms long, not 9 * CC, so the second level of the
 // sum is long and carries the full magnitude (0.46 at 1024 with the first level folded every fourth chunk).
-// 5x5 layers (100-term first levels): relative error 2.7e-7 at 1150 terms, 2.9e-7 at 2500, where the kernel without tiles has 3.4e-7.
+// 5x5 layers (50-term first levels): worst element 0.40 at 1150 terms, 0.56 at 2500; relative error 2.7e-7 and 3.1e-7, where the kernel
+// without tiles has 3.4e-7 and 3.5e-7.
 static constexpr int kSatMaxTerms = 1152, kSatMaxTerms1x1 = 1024, kSatMaxTerms5x5 = 2500;
 template <class C>
 constexpr int sat_max_terms() { return C::KS == 1 ? kSatMaxTerms1x1 : (C::KS == 5 ? kSatMaxTerms5x5 : kSatMaxTerms); }

@@ -2,13 +2,13 @@
 a second sum taken off) on the layers with the most terms per output that still use it.
 
 The form costs accuracy against the three-instruction one, so layers above a term count keep the latter
-(grad_x.hip: 1152 terms for 3x3 layers, 1024 for single-tap ones).  This test runs the layers that sit at those
-switch points -- 128 -> 128 3x3 and ResNet-50's 256 -> 1024 @14x14 -- two below them (128 -> 512 @28x28, ResNet-20's
-64 -> 64 @8x8) and two above, which run the three-instruction form (VGG-small's 256 -> 256 @16x16 and
-512 -> 512 @8x8), over 8 seeds x {Kaiming, N(0,1)} weights x input scale {1, 5} and holds the worst
-element of every case to 0.7 of the parity tolerance 1e-4 + 1e-5 |gx| against the float64 C oracle
-(test_cuda.py:57-60; adder.cu:17,246).  The input gradient of an image depends on that image alone, so four
-images per case stand for any batch size.
+(grad_x.hip: 1152 terms for 3x3 layers, 1024 for single-tap ones, 2500 for 5x5 ones).  This test runs the layers that
+sit at those switch points -- 128 -> 128 3x3, ResNet-50's 256 -> 1024 @14x14, 5x5 layers of 100 output channels --,
+some below them (128 -> 512 @28x28, ResNet-20's 64 -> 64 @8x8, 5x5 with 90 output channels) and some above, which run the
+three-instruction form (VGG-small's 256 -> 256 @16x16 and 512 -> 512 @8x8, 5x5 with 101), over 8 seeds x {Kaiming,
+N(0,1)} weights x input scale {1, 5} and holds the worst element of every case to 0.7 of the parity tolerance
+1e-4 + 1e-5 |gx| against the float64 C oracle (test_cuda.py:57-60; adder.cu:17,246).  The input gradient of an image
+depends on that image alone, so four images per case stand for any batch size.
 """
 import ctypes
 import math
@@ -20,7 +20,8 @@ pytestmark = pytest.mark.gpu
 
 # (Ci, H, W, Co, k, stride, pad), terms per input position = Co * k * k
 LAYERS = [(128, 16, 16, 128, 3, 1, 1), (256, 14, 14, 1024, 1, 1, 0), (128, 28, 28, 512, 1, 1, 0), (64, 8, 8, 64, 3, 1, 1),
-          (256, 16, 16, 256, 3, 1, 1), (512, 8, 8, 512, 3, 1, 1)]
+          (256, 16, 16, 256, 3, 1, 1), (512, 8, 8, 512, 3, 1, 1),
+          (16, 16, 16, 100, 5, 1, 2), (16, 8, 8, 100, 5, 1, 2), (16, 24, 24, 90, 5, 1, 2), (16, 16, 16, 101, 5, 1, 2)]
 IMAGES = 4
 MARGIN = 0.7
 
