@@ -311,8 +311,10 @@ int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDi
 template <class T>
 int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s);
 int grad_w_1x1_slots(const ConvDims &d);
-template <class T>
-int launch_grad_w_1x1(const T *gy, const T *x, float *part, float *sgpart, int slots, const ConvDims &d, hipStream_t s);
+// P: float slabs for float storage, double ones for bfloat16; with gw (bfloat16 only, slots = 1) the finished gradient and no slabs
+template <class T, class P>
+int launch_grad_w_1x1(const T *gy, const T *x, P *part, P *sgpart, const float *w, float *gw, int slots, const ConvDims &d,
+                      hipStream_t s);
 
 // fused BatchNorm + residual + ReLU (bn_act.hip)
 size_t bn_workspace_bytes(int N, int C, int HW);

@@ -11,6 +11,8 @@
 // unfold/fold copies of adder.py:32-33,38-39.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace adder {
 
 // A lane owns 4/S adjacent outputs of one output row: one float4 of the source row.
@@ -278,14 +280,24 @@ __global__ __launch_bounds__(256) void grad_x_1x1_kernel(const T *__restrict__ g
 
 // grad_w: a wave owns TM output channels x TC input channels; its lanes walk over position
 // groups, then the 64 lanes are folded through LDS (16 sums per round).
+// float storage: fp32 sums and slabs, as many slabs as keep a lane's sums short.  bfloat16 storage (fp64 accumulation is what
+// its entry point promises): the lanes are folded into fp64 every 64 positions per lane, and the slabs are fp64.  gw
+// (bfloat16 storage, one slab): the finished gradient sum x g - w sum g goes there, and there are no slabs.
+template <class T> using GwSum1x1 = std::conditional_t<sizeof(T) == 4, float, double>;
+
 template <int S, int TM, int TC, bool VEC = true, class T = float>
-__global__ __launch_bounds__(256) void grad_w_1x1_kernel(const T *__restrict__ gy,
-                                                         const T *__restrict__ x, float *__restrict__ part,
-                                                         float *__restrict__ sgpart, int N, int Ci, int H,
-                                                         int W, int Co, int Ho, int Wo, int gpr, int groups) {
-    constexpr int TN = 4 / S, A = TM * TC;
+__global__ __launch_bounds__(256) void grad_w_1x1_kernel(const T *__restrict__ gy, const T *__restrict__ x,
+                                                         GwSum1x1<T> *__restrict__ part, GwSum1x1<T> *__restrict__ sgpart,
+                                                         const float *__restrict__ w, float *__restrict__ gw, int N, int Ci,
+                                                         int H, int W, int Co, int Ho, int Wo, int gpr, int groups) {
+    using P = GwSum1x1<T>;
+    constexpr bool WIDE = sizeof(P) == 8;
+    constexpr int TN = 4 / S, A = TM * TC, TOT = A + TM, RUN = 64 / TN;   // RUN: position groups between two folds (WIDE)
     const int co0 = blockIdx.y * TM, ci0 = blockIdx.z * TC;
     const size_t plane = (size_t)H * W, gplane = (size_t)Ho * Wo;
+    __shared__ float red[4][64 * 17];
+    __shared__ P wsum[4][TOT];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     float acc[TM][TC], sg[TM];
 #pragma unroll
     for (int m = 0; m < TM; ++m) {
@@ -293,7 +305,29 @@ __global__ __launch_bounds__(256) void grad_w_1x1_kernel(const T *__restrict__ g
 #pragma unroll
         for (int c = 0; c < TC; ++c) acc[m][c] = 0.f;
     }
-    for (int g0 = blockIdx.x * 256 + threadIdx.x; g0 < groups; g0 += gridDim.x * 256) {
+    auto fold = [&](const bool first) {   // the sums of the wave's lanes into (first) or onto wsum; acc and sg restart
+        float all[TOT];
+#pragma unroll
+        for (int a = 0; a < A; ++a) { all[a] = acc[a / TC][a % TC]; acc[a / TC][a % TC] = 0.f; }
+#pragma unroll
+        for (int m = 0; m < TM; ++m) { all[A + m] = sg[m]; sg[m] = 0.f; }
+        constexpr int ROUNDS = ceil_div(TOT, 16);
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) red[wave][lane * 17 + e] = (r * 16 + e < TOT) ? all[(r * 16 + e) % TOT] : 0.f;
+            __syncthreads();
+            const int e = lane & 15, rg = lane >> 4;
+            P s = P(0);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) s += (P)red[wave][(rg * 16 + k) * 17 + e];
+            s += __shfl_xor(s, 16, 64);
+            s += __shfl_xor(s, 32, 64);
+            if (rg == 0 && r * 16 + e < TOT) wsum[wave][r * 16 + e] = first ? s : wsum[wave][r * 16 + e] + s;
+            __syncthreads();
+        }
+    };
+    auto step = [&](const int g0) {
         const Lane1x1<S> L(g0, groups, gpr, Ho);
         const T *xp = x + (size_t)L.n * Ci * plane + (size_t)(L.ho * S) * W + L.wo0 * S;
         const T *gp = gy + (size_t)L.n * Co * gplane + (size_t)L.ho * Wo + L.wo0;
@@ -326,40 +360,32 @@ __global__ __launch_bounds__(256) void grad_w_1x1_kernel(const T *__restrict__ g
                 for (int c = 0; c < TC; ++c) acc[m][c] = fmaf(gs[m][t], xs[c][t], acc[m][c]);
             }
         }
+    };
+    bool first = true;
+    if constexpr (WIDE) {
+        int run = 0;
+        for (int base = blockIdx.x * 256; base < groups; base += gridDim.x * 256) {   // (uniform: fold has barriers)
+            if (base + (int)threadIdx.x < groups) step(base + threadIdx.x);
+            if (++run == RUN) { fold(first); first = false; run = 0; }
+        }
+    } else {
+        for (int g0 = blockIdx.x * 256 + threadIdx.x; g0 < groups; g0 += gridDim.x * 256) step(g0);
     }
-    // fold lanes, then the 4 waves of the workgroup
-    __shared__ float red[4][64 * 17];
-    __shared__ float wsum[4][A + TM];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    constexpr int TOT = A + TM;
-    float all[TOT];
-#pragma unroll
-    for (int a = 0; a < A; ++a) all[a] = acc[a / TC][a % TC];
-#pragma unroll
-    for (int m = 0; m < TM; ++m) all[A + m] = sg[m];
-    constexpr int ROUNDS = ceil_div(TOT, 16);
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) red[wave][lane * 17 + e] = (r * 16 + e < TOT) ? all[(r * 16 + e) % TOT] : 0.f;
-        __syncthreads();
-        const int e = lane & 15, rg = lane >> 4;
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) s += red[wave][(rg * 16 + k) * 17 + e];
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
-        if (rg == 0 && r * 16 + e < TOT) wsum[wave][r * 16 + e] = s;
-        __syncthreads();
-    }
+    // the last positions, then the 4 waves of the workgroup
+    fold(first);
     if (threadIdx.x < TOT) {
         const int a = threadIdx.x;
-        const float s = (wsum[0][a] + wsum[1][a]) + (wsum[2][a] + wsum[3][a]);
-        if (a < A) {
-            const int co = co0 + a / TC, ci = ci0 + a % TC;
+        const P s = (wsum[0][a] + wsum[1][a]) + (wsum[2][a] + wsum[3][a]);
+        const int co = co0 + (a < A ? a / TC : a - A), ci = ci0 + a % TC;
+        if (WIDE && gw) {
+            if (a < A && co < Co && ci < Ci) {
+                const int b = A + a / TC;
+                const P sum_g = (wsum[0][b] + wsum[1][b]) + (wsum[2][b] + wsum[3][b]);
+                gw[(size_t)co * Ci + ci] = (float)(s - (P)w[(size_t)co * Ci + ci] * sum_g);
+            }
+        } else if (a < A) {
             if (co < Co && ci < Ci) part[(size_t)blockIdx.x * Co * Ci + (size_t)co * Ci + ci] = s;
         } else if (blockIdx.z == 0) {
-            const int co = co0 + a - A;
             if (co < Co) sgpart[(size_t)blockIdx.x * Co + co] = s;
         }
     }
@@ -453,15 +479,19 @@ int grad_w_1x1_slots(const ConvDims &d) {
     return want < 1 ? 1 : want;
 }
 
-template <class T>
-int launch_grad_w_1x1(const T *gy, const T *x, float *part, float *sgpart, int slots, const ConvDims &d, hipStream_t s) {
+// bfloat16 storage, 48 -> 48 @64x64, 64 images: generic kernel 1219 us, fp32 sums and slabs 52, fp64 ones 52.5; 32 -> 1024 @28x28, 256
+// images: 11 125, 354 and 376.
+template <class T, class P>
+int launch_grad_w_1x1(const T *gy, const T *x, P *part, P *sgpart, const float *w, float *gw, int slots, const ConvDims &d,
+                      hipStream_t s) {
+    static_assert(std::is_same<P, GwSum1x1<T>>::value, "fp32 slabs for float storage, fp64 for bfloat16");
     constexpr int TM = kGw1x1TM, TC = kGw1x1TC;
     const ConvDims f = lane_dims(d);
     int gpr, groups;
     lane_space(f, gpr, groups);
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(slots, ceil_div(f.Co, TM), ceil_div(f.Ci, TC)), dim3(256), 0, s, gy, x, part, sgpart,
-                           f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
+        hipLaunchKernelGGL(kernel, dim3(slots, ceil_div(f.Co, TM), ceil_div(f.Ci, TC)), dim3(256), 0, s, gy, x, part, sgpart, w,
+                           gw, f.N, f.Ci, f.H, f.W, f.Co, f.Ho, f.Wo, gpr, groups);
         return check_launch();
     };
     const bool vec = vec_ok<T>(f, gy, x, nullptr);
@@ -469,7 +499,9 @@ int launch_grad_w_1x1(const T *gy, const T *x, float *part, float *sgpart, int s
         return vec ? launch(grad_w_1x1_kernel<2, TM, TC, true, T>) : launch(grad_w_1x1_kernel<2, TM, TC, false, T>);
     return vec ? launch(grad_w_1x1_kernel<1, TM, TC, true, T>) : launch(grad_w_1x1_kernel<1, TM, TC, false, T>);
 }
-template int launch_grad_w_1x1<float>(const float *, const float *, float *, float *, int, const ConvDims &, hipStream_t);
-template int launch_grad_w_1x1<bf16_t>(const bf16_t *, const bf16_t *, float *, float *, int, const ConvDims &, hipStream_t);
+template int launch_grad_w_1x1<float, float>(const float *, const float *, float *, float *, const float *, float *, int,
+                                             const ConvDims &, hipStream_t);
+template int launch_grad_w_1x1<bf16_t, double>(const bf16_t *, const bf16_t *, double *, double *, const float *, float *, int,
+                                               const ConvDims &, hipStream_t);
 
 }  // namespace adder

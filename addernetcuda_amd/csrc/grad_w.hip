@@ -12,6 +12,8 @@
 // conv1x1.hip); the finalize kernel in this file adds the slabs in fp64 and applies -w*sum_g.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace adder {
 
 static constexpr int kNormBlocksMax = 16384;  // sum-of-squares partials kept at the head of the workspace
@@ -370,8 +372,9 @@ bool grad_w_bn_supported(const ConvDims &d, const void *gy, const void *x, const
 size_t grad_w_workspace_bytes(const ConvDims &d) {
     const GradWPlan p = plan_grad_w(d);
     size_t bytes = sizeof(double) * kNormBlocksMax;
+    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
     if (p.variant)
-        bytes += (p.variant == 2 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
+        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
     return (bytes + 255) & ~(size_t)255;
 }
 
@@ -398,6 +401,13 @@ int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
     double *ss = reinterpret_cast<double *>(ws);
     const int K = d.K();
     const long n = (long)d.Co * K;
+    if constexpr (sizeof(T) != 4) {   // (a plain 1x1 layer whose positions make one slab: the kernel finishes the gradient itself)
+        if (p.variant == 1 && p.slots == 1) {
+            double *none = nullptr;
+            if (int rc = launch_grad_w_1x1(gy, x, none, none, w, gw, 1, d, s)) return rc;
+            return eta > 0.f ? launch_norm_scale(gw, n, eta, 1e-12f, ws, s) : ADDER_OK;
+        }
+    }
     if (p.variant) {
         const int nb = (int)ceil_div_l(n, fin_out_for(p.slots));
         const bool fused_norm = eta > 0.f && nb <= kNormBlocksMax;
@@ -414,11 +424,12 @@ int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
             hipLaunchKernelGGL(grad_w_finalize_kernel<double>, dim3(nb), dim3(kFinOut * kFinLanes), 0, s, part,
                                sgpart, w, gw, fused_norm ? ss : nullptr, p.slots, d.Co, K);
         } else {
-            float *part = reinterpret_cast<float *>(ss + kNormBlocksMax);
-            float *sgpart = part + (size_t)p.slots * d.Co * K;
-            rc = launch_grad_w_1x1(gy, x, part, sgpart, p.slots, d, s);
+            using P = std::conditional_t<sizeof(T) == 4, float, double>;
+            P *part = reinterpret_cast<P *>(ss + kNormBlocksMax);
+            P *sgpart = part + (size_t)p.slots * d.Co * K;
+            rc = launch_grad_w_1x1(gy, x, part, sgpart, w, (float *)nullptr, p.slots, d, s);
             if (rc) return rc;
-            hipLaunchKernelGGL(grad_w_finalize_kernel<float>, dim3(nb), dim3(kFinOut * kFinLanes), 0, s, part,
+            hipLaunchKernelGGL(grad_w_finalize_kernel<P>, dim3(nb), dim3(kFinOut * kFinLanes), 0, s, part,
                                sgpart, w, gw, fused_norm ? ss : nullptr, p.slots, d.Co, K);
         }
         if (fused_norm)
@@ -484,7 +495,7 @@ int launch_grad_w_staged(const float *gy, const float *x, const float *w, float 
     } else {
         float *part = reinterpret_cast<float *>(ss + kNormBlocksMax);
         float *sgpart = part + (size_t)p.slots * d.Co * K;
-        rc = launch_grad_w_1x1(gy, x, part, sgpart, p.slots, d, s);
+        rc = launch_grad_w_1x1(gy, x, part, sgpart, w, (float *)nullptr, p.slots, d, s);
         stage->part = part;
         stage->sgpart = sgpart;
     }

@@ -42,3 +42,29 @@ def test_bfloat16_kernels_match_the_oracle(case, gpu):
 @pytest.mark.parametrize("case", [SHAPES[0], SHAPES[5], SHAPES[8], SHAPES[12]], ids=str)
 def test_bfloat16_tensors_at_odd_addresses(case, gpu):
     _check(case, gpu, 1)
+
+
+# plain 1x1 layers (fewer than 64 channels on a side): one slab and long sums, one slab of few positions, several slabs,
+# rows that are not whole groups of four, stride 2
+@pytest.mark.parametrize("case", [(256, 63, 28, 28, 1024, 1, 1, 0), (1, 9, 8, 8, 5, 1, 1, 0), (8, 63, 56, 56, 40, 1, 1, 0),
+                                  (40, 24, 57, 55, 20, 1, 1, 0), (40, 24, 64, 64, 20, 1, 2, 0), (90, 17, 57, 55, 70, 1, 2, 0)], ids=str)
+def test_plain_1x1_weight_gradient_is_summed_in_float64(case, gpu):
+    from addernetcuda_amd import adder
+    N, Ci, H, W, Co, k, s, p = case
+    g = torch.Generator(device=gpu).manual_seed(8)
+    x = torch.relu(torch.randn(N, Ci, H, W, device=gpu, generator=g)).bfloat16()
+    w = torch.randn(Co, Ci, 1, 1, device=gpu, generator=g).requires_grad_(True)
+    y = adder.adder2d_function(x, w, s, p, eta=0.0)
+    gy = torch.randn(y.shape, device=gpu, generator=g).bfloat16()
+    y.backward(gy)
+    xs = x[:, :, ::s, ::s].double().transpose(0, 1).reshape(Ci, -1)
+    gs = gy.double().transpose(0, 1).reshape(Co, -1)
+    want = gs @ xs.t().contiguous() - w.detach().double().view(Co, Ci) * gs.sum(1, keepdim=True)
+    # The product of two bfloat16 values has 16 bits, so fp32 sums of 64 of them hardly round; with fp64 from there on the
+    # result's own rounding is left, 0.4 * 2^-24 = 2.4e-8 (fp32 to the end: 5.6e-8 to 1.2e-7, and more the longer the sums)
+    assert (w.grad.double().view(Co, Ci) - want).norm() <= 5e-8 * want.norm()
+    # and the finished gradient is scaled in place (adder.py:78): three more roundings
+    raw, w.grad = w.grad, None
+    adder.adder2d_function(x, w, s, p, eta=0.2).backward(gy)
+    scaled = raw.double() / raw.double().norm() * 0.2 * raw.numel() ** 0.5
+    assert (w.grad.double() - scaled).norm() <= 1e-7 * scaled.norm()
