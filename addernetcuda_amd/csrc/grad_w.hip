@@ -369,14 +369,14 @@ bool grad_w_bn_supported(const ConvDims &d, const void *gy, const void *x, const
     return p.variant == 2 && (k3 || k1) && (align & 15) == 0;
 }
 
-size_t grad_w_workspace_bytes(const ConvDims &d) {
-    const GradWPlan p = plan_grad_w(d);
+static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
     size_t bytes = sizeof(double) * kNormBlocksMax;
     // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
     if (p.variant)
         bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
     return (bytes + 255) & ~(size_t)255;
 }
+size_t grad_w_workspace_bytes(const ConvDims &d) { return workspace_bytes_of(plan_grad_w(d), d); }
 
 // bn_y with either bn_coef or sums.part: gy is the gradient dz of the output of the BatchNorm behind the layer and
 // the kernel forms the layer's own output gradient from it, leaving it in gy_out (nullable) on the way (matrix-core
@@ -386,8 +386,8 @@ template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws,
                   size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y, const float *bn_coef,
                   float *gy_out, const BnSums &sums) {
-    if (ws_bytes < grad_w_workspace_bytes(d)) return ADDER_ERR_WORKSPACE;
-    GradWPlan p = plan_grad_w(d);
+    GradWPlan p = plan_grad_w(d);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
+    if (ws_bytes < workspace_bytes_of(p, d)) return ADDER_ERR_WORKSPACE;
     if (bn_y && (sizeof(T) != 4 ||
                  !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part)))
         return ADDER_ERR_UNSUPPORTED;
@@ -472,8 +472,8 @@ template int launch_grad_w<bf16_t>(const bf16_t *, const bf16_t *, const float *
 int launch_grad_w_staged(const float *gy, const float *x, const float *w, float *gw, float eta, void *ws,
                          size_t ws_bytes, const ConvDims &d, adder_grad_w_stage *stage, hipStream_t s,
                          const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
-    if (ws_bytes < grad_w_workspace_bytes(d)) return ADDER_ERR_WORKSPACE;
-    GradWPlan p = plan_grad_w(d);
+    GradWPlan p = plan_grad_w(d);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
+    if (ws_bytes < workspace_bytes_of(p, d)) return ADDER_ERR_WORKSPACE;
     if (bn_y && !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part))
         return ADDER_ERR_UNSUPPORTED;
     const bool rows_1x1 = p.variant == 2 && d.kh == 1;
