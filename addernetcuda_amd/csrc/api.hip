@@ -160,6 +160,14 @@ int adder_bn_eval_f32(const float *x, float *y, const float *gamma, const float 
     return launch_bn_eval(x, y, BnEval{gamma, beta, mean, var, residual, eps, relu, 0}, N, C, HW, static_cast<hipStream_t>(stream));
 }
 
+int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel) {
+    if (!kernel) return ADDER_ERR_NULL_POINTER;
+    ConvDims d;
+    if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
+    *kernel = fwd_kernel(d);
+    return ADDER_OK;
+}
+
 int adder_conv2d_fwd_stats_slots(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad,
                                  int *slots) {
     if (!slots) return ADDER_ERR_NULL_POINTER;

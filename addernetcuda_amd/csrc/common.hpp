@@ -256,6 +256,7 @@ int check_launch();                  // hipGetLastError -> status
 // T: storage type of the activations and their gradients, float or bf16_t (the optional reduced-storage mode).
 template <class T>
 int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
+int fwd_kernel(const ConvDims &d);
 int fwd_stats_slots(const ConvDims &d);
 bool fwd_pair_supported(const ConvDims &d);
 int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats,

@@ -708,6 +708,16 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
                        : launch_fwd_pair_3x3<FwdW8S2>(x, w, w_side, y, y_side, stats, stats_side, d, s);
 }
 
+// Which kernel launch_fwd runs without statistics and for bases aligned to groups of four: 0 general, 1 plain 1x1, 2 few
+// positions, else 10 * variant + which of its tiles (rows 16 / 8 / 4: 0 / 1 / 2; channels from 128 on: 1).
+int fwd_kernel(const ConvDims &d) {
+    const int variant = fwd_tiled_variant(d);
+    if (few_positions(d, variant)) return 2;
+    if (variant == 0) return conv1x1_supported(d, nullptr, nullptr) ? 1 : 0;
+    const int rows = rows_per_tile_w32(d.Ho);
+    return 10 * variant + (variant == 1 ? (rows == 16 ? 0 : rows == 8 ? 1 : 2) : variant == 5 && d.Ci >= 128 ? 1 : 0);
+}
+
 int fwd_stats_slots(const ConvDims &d) {
     if (d.kh == 1 && few_positions(d, fwd_tiled_variant(d))) return ceil_div(d.N * d.Ho * d.Wo, 64);
     switch (fwd_tiled_variant(d)) {

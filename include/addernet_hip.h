@@ -82,6 +82,11 @@ ADDER_API int adder_conv2d_fwd_f32(const float *x, const float *w, float *y,
                          int N, int Ci, int H, int W, int Co, int kh, int kw,
                          int stride, int pad, void *stream);
 
+/* Which kernel the forward calls above and below (without statistics) take for the dimensions and aligned tensors, in the
+ * dispatch's own numbers: 0 the general one, 1 the plain 1x1 one, 2 the one for few positions, from 10 on the tiled ones.
+ * Host code only; for tests that have to reach a certain kernel, and no promise that the numbers stay. */
+ADDER_API int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel);
+
 /* The same forward with the BatchNorm that follows it (fixed statistics: inference), the shortcut and the ReLU applied on
  * the way out: y = act((conv - mean) / sqrt(var + eps) * gamma + beta [+ residual]), act = ReLU when relu is set;
  * gamma, beta, mean, var (Co), residual (nullable) shaped like y.  resnet20.py:28-39 in evaluation mode. */

@@ -1,18 +1,18 @@
 """The forward kernel for few positions (small batches and maps): against the float64 oracle at its edges -- maps of 1 to 32, tails
 in positions, channels and channel chunks, strides, more chunks than waves -- with its statistics, its inference epilogue
-and both storage types; and the same bits as the tiled kernel, which computes the same images in a batch large enough for it."""
+and both storage types; and the same bits as each tiled kernel, which computes the same image in a batch large enough for it."""
 import pytest
 import torch
 
-from tests.util import make_case, assert_close
+from tests.util import make_case, assert_close, fwd_kernel, FEW_AND_TILED, FEW_POSITIONS
 from tests.test_gpu_bf16 import _close_bf16
 
 pytestmark = pytest.mark.gpu
 
 # (N, Ci, H, W, Co, k, stride, pad)
 SHAPES = [(1, 16, 32, 32, 16, 3, 1, 1), (1, 64, 8, 8, 64, 3, 1, 1), (2, 33, 14, 14, 37, 3, 1, 1), (1, 200, 7, 7, 31, 3, 1, 1),
-          (3, 17, 1, 1, 5, 3, 1, 1), (1, 40, 9, 33, 6, 3, 1, 1), (1, 32, 17, 32, 33, 3, 2, 1), (2, 130, 15, 7, 18, 3, 2, 1),
-          (1, 64, 8, 8, 48, 1, 1, 0), (2, 300, 7, 7, 21, 1, 1, 0), (1, 68, 14, 14, 64, 1, 2, 0), (1, 512, 4, 4, 40, 1, 3, 0)]
+          (3, 33, 1, 1, 5, 3, 1, 1), (1, 40, 9, 33, 6, 3, 1, 1), (1, 32, 17, 32, 33, 3, 2, 1), (2, 130, 15, 7, 18, 3, 2, 1),
+          (1, 200, 8, 8, 48, 1, 1, 0), (2, 300, 7, 7, 21, 1, 1, 0), (1, 132, 14, 14, 64, 1, 2, 0), (1, 512, 4, 4, 40, 1, 3, 0)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
@@ -20,6 +20,7 @@ SHAPES = [(1, 16, 32, 32, 16, 3, 1, 1), (1, 64, 8, 8, 64, 3, 1, 1), (2, 33, 14, 
 def test_few_positions_match_the_oracle(case, dtype, gpu):
     from addernetcuda_amd import adder
     from oracle import c_oracle
+    assert fwd_kernel(case) == FEW_POSITIONS
     s, p = case[6], case[7]
     x, w, _ = make_case(*case)
     x = x.to(dtype)
@@ -34,12 +35,13 @@ def test_few_positions_match_the_oracle(case, dtype, gpu):
         assert torch.allclose(tot[:, 1], (want * want).sum(dim=(0, 2, 3)), rtol=1e-5, atol=1e-2)
 
 
-@pytest.mark.parametrize("case", SHAPES, ids=str)
-def test_same_bits_in_a_large_batch(case, gpu):
+@pytest.mark.parametrize("kernel", FEW_AND_TILED)
+def test_same_bits_as_the_tiled_kernel_of_a_large_batch(kernel, gpu):
     from addernetcuda_amd import adder
-    N, Ci, H, W, Co, k, s, p = case
+    case, batch = FEW_AND_TILED[kernel]
+    assert fwd_kernel(case) == FEW_POSITIONS and fwd_kernel((batch,) + case[1:]) == kernel
     x, w, _ = make_case(*case)
     xg, wg = x.to(gpu), w.to(gpu)
-    few = adder.adder2d_function(xg, wg, s, p)
-    big = adder.adder2d_function(xg.repeat(2048 // N if H * W < 200 else 256 // N, 1, 1, 1), wg, s, p)
-    assert torch.equal(big[:N], few) and torch.equal(big[-N:], few)
+    few = adder.adder2d_function(xg, wg, case[6], case[7])
+    big = adder.adder2d_function(xg.repeat(batch, 1, 1, 1), wg, case[6], case[7])
+    assert torch.equal(big, few.expand_as(big))

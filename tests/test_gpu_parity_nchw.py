@@ -12,7 +12,9 @@ from tests.util import make_case, assert_close
 
 pytestmark = pytest.mark.gpu
 
-# (N, Ci, H, W, Co, k, stride, pad)
+# (N, Ci, H, W, Co, k, stride, pad).  The comments name the tiled kernels; in the forward about half of these small layers run the
+# few-positions kernel instead, and so do the float32 input gradients of the odd widths (test_gpu_eval_fused.py runs every
+# tiled forward, test_gpu_bn_act.py the 3x3 ones with statistics).
 TILED = [
     (3, 16, 32, 32, 16, 3, 1, 1),   # 32-wide tiled path
     (2, 32, 16, 16, 32, 3, 1, 1),   # 16-wide tiled path

@@ -1,4 +1,5 @@
-"""Seeded synthetic tensors shared by the tests (CPU float32)."""
+"""Seeded synthetic tensors shared by the tests (CPU float32), and layers that reach each forward kernel."""
+import ctypes
 import math
 
 import torch
@@ -36,3 +37,48 @@ def assert_close(actual, expected, what, rtol=RTOL, atol=ATOL):
             f"{what}: {int(bad.sum())}/{bad.numel()} elements outside rtol={rtol} atol={atol}; "
             f"max abs err {err.max().item():.3e} (|ref| max {e.abs().max().item():.3e}); first at {idx}: "
             f"{a[tuple(idx)].item()} vs {e[tuple(idx)].item()}")
+
+
+def fwd_kernel(case):
+    """The number of the forward kernel that the library takes for (N, Ci, H, W, Co, k, stride, pad)."""
+    from addernetcuda_amd._lib import lib, check
+    N, Ci, H, W, Co, k, stride, pad = case
+    kernel = ctypes.c_int(-1)
+    check(lib.adder_conv2d_fwd_kernel(N, Ci, H, W, Co, k, k, stride, pad, ctypes.byref(kernel)), "adder_conv2d_fwd_kernel")
+    return kernel.value
+
+
+FEW_POSITIONS = 2
+# every tiled forward kernel, by its number, on a layer whose rows (1x1: planes) are whole groups of four and on one whose are not
+TILED_FORWARD = {
+    10: [(2, 3, 32, 32, 18, 3, 1, 1), (1, 5, 32, 30, 18, 3, 1, 1)],
+    11: [(2, 3, 24, 24, 18, 3, 1, 1), (3, 5, 24, 27, 7, 3, 1, 1)],
+    12: [(3, 3, 20, 20, 18, 3, 1, 1), (1, 3, 18, 18, 18, 3, 1, 1)],
+    20: [(33, 17, 13, 16, 70, 3, 1, 1), (2, 5, 9, 9, 18, 3, 1, 1)],
+    30: [(1, 17, 8, 8, 18, 3, 1, 1), (5, 16, 7, 7, 17, 3, 1, 1)],
+    40: [(1, 3, 20, 24, 18, 3, 2, 1), (1, 3, 20, 20, 18, 3, 2, 1), (2, 3, 18, 18, 18, 3, 2, 1)],
+    50: [(1, 17, 8, 8, 18, 3, 2, 1), (1, 17, 9, 9, 18, 3, 2, 1)],
+    51: [(65, 128, 16, 16, 130, 3, 2, 1), (130, 128, 9, 9, 130, 3, 2, 1)],
+    60: [(1, 64, 14, 14, 18, 1, 1, 0), (1, 64, 15, 15, 18, 1, 1, 0)],
+    70: [(1, 64, 8, 8, 18, 1, 1, 0), (1, 64, 7, 7, 18, 1, 1, 0)],
+    80: [(16, 72, 32, 32, 70, 1, 2, 0), (33, 64, 32, 30, 70, 1, 2, 0)],
+    90: [(33, 72, 24, 24, 70, 1, 2, 0), (33, 64, 17, 33, 70, 1, 2, 0)],
+    100: [(1, 68, 14, 14, 18, 1, 1, 0), (1, 68, 15, 15, 18, 1, 1, 0)],
+    110: [(1, 68, 8, 8, 18, 1, 1, 0), (1, 68, 7, 7, 18, 1, 1, 0)],
+    120: [(1, 68, 28, 28, 18, 1, 2, 0), (1, 68, 32, 30, 18, 1, 2, 0)],
+    130: [(1, 68, 8, 8, 18, 1, 2, 0), (1, 68, 7, 7, 18, 1, 3, 0)],
+    140: [(1, 3, 20, 20, 18, 5, 1, 2), (2, 9, 17, 30, 18, 5, 1, 2)],
+    150: [(1, 3, 12, 12, 18, 5, 1, 2), (2, 9, 14, 14, 18, 5, 1, 2)],
+    160: [(5, 3, 8, 8, 18, 5, 1, 2), (1, 9, 7, 7, 18, 5, 1, 2)],
+    170: [(1, 9, 20, 24, 18, 5, 2, 2), (2, 3, 18, 18, 18, 5, 2, 2)],
+    180: [(3, 3, 16, 16, 18, 5, 2, 2), (1, 9, 13, 7, 18, 5, 2, 2)],
+}
+# layers of one image for the few-positions kernel, with a batch that is large enough for the tiled kernel of that number
+FEW_AND_TILED = {
+    10: ((1, 16, 32, 32, 40, 3, 1, 1), 16), 11: ((1, 16, 24, 24, 16, 3, 1, 1), 64), 12: ((1, 16, 17, 32, 16, 3, 1, 1), 64),
+    20: ((1, 33, 14, 14, 37, 3, 1, 1), 128), 30: ((1, 200, 7, 7, 31, 3, 1, 1), 2048), 40: ((1, 32, 17, 32, 33, 3, 2, 1), 256),
+    50: ((1, 33, 7, 7, 40, 3, 2, 1), 256), 51: ((1, 130, 9, 9, 16, 3, 2, 1), 1024), 60: ((1, 128, 32, 32, 16, 1, 1, 0), 8),
+    70: ((1, 128, 20, 20, 40, 1, 1, 0), 8), 80: ((1, 64, 28, 28, 16, 1, 2, 0), 128), 90: ((1, 64, 9, 9, 16, 1, 2, 0), 1024),
+    100: ((1, 300, 32, 32, 16, 1, 1, 0), 8), 110: ((1, 300, 7, 7, 21, 1, 1, 0), 1024), 120: ((1, 300, 32, 32, 16, 1, 2, 0), 32),
+    130: ((1, 300, 7, 7, 16, 1, 2, 0), 512),
+}
