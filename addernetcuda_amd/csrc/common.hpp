@@ -67,6 +67,10 @@ __device__ __forceinline__ void stf2(bf16_t *p, float2 v) {
     *reinterpret_cast<uint32_t *>(p) = (uint32_t)f32_to_bf16(v.x) | ((uint32_t)f32_to_bf16(v.y) << 16);
 }
 
+// Most workgroups along a grid's y (hipDeviceProp_t::maxGridSize: 65536).  Kernels with few channels per workgroup leave layers
+// with more channels than that to those with many.
+static constexpr int kMaxGridY = 65535;
+
 // Whether a tensor's base lets four consecutive elements be moved as one group (NULL: no tensor).
 template <class T>
 inline bool aligned_groups(const T *p) { return (reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0; }
@@ -309,6 +313,7 @@ bool conv1x1_supported(const ConvDims &d, const void *a, const void *b);
 int fwd_1x1_stats_slots(const ConvDims &d);
 template <class T>
 int launch_fwd_1x1(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
+static constexpr int kGx1x1TM = 4;   // input channels per workgroup; latency-bound at ResNet sizes: more workgroups beat more reuse per lane
 template <class T>
 int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s);
 int grad_w_1x1_slots(const ConvDims &d);

@@ -450,7 +450,7 @@ template int launch_fwd_1x1<bf16_t>(const bf16_t *, const float *, bf16_t *, dou
 
 template <class T>
 int launch_grad_x_1x1(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s) {
-    constexpr int TM = 4;   // latency-bound at ResNet sizes: more workgroups beat more reuse per lane
+    constexpr int TM = kGx1x1TM;
     const ConvDims f = lane_dims(d);
     int gpr, groups;
     lane_space(f, gpr, groups);

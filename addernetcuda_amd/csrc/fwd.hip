@@ -401,6 +401,7 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
 // channels per first-level sum).  x is read from global memory (a map this small sits in L1 / L2) one channel ahead
 // of the arithmetic, as are the weights.  Whole networks: ResNet-50, one image, 4.6 -> 1.7 ms; VGG-small, two, 720 -> 184 us.
 // ---------------------------------------------------------------------------
+static constexpr int kFewTM = 4;
 template <int KS, int TM, int G, class T>
 __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
                                                       double *__restrict__ stats, ConvDims d, int chunk, const BnEval bn) {
@@ -509,7 +510,7 @@ __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, c
 template <int KS, class T>
 static int launch_fwd_few(const T *x, const float *w, T *y, double *stats, const ConvDims &d, int chunk, hipStream_t s,
                           const BnEval &bn) {
-    constexpr int TM = 4, G = KS == 1 ? 8 : 1;
+    constexpr int TM = kFewTM, G = KS == 1 ? 8 : 1;
     const int waves = ceil_div(d.Ci, chunk) < 8 ? ceil_div(d.Ci, chunk) : 8;
     hipLaunchKernelGGL((fwd_few_kernel<KS, TM, G, T>), dim3(ceil_div(d.N * d.Ho * d.Wo, 64), ceil_div(d.Co, TM)),
                        dim3(64 * waves), 0, s, x, w, y, stats, d, chunk, bn);
@@ -658,7 +659,7 @@ static_assert(FwdW32::CC == FwdW32H8::CC && FwdW32::CC == FwdW32H4::CC && Fwd1x1
 // the tiled kernels win: 16 -> 16 3x3 @32x32, 64 images, 15 against 18; 1024 -> 256 1x1 @14x14, 16 images, 106 against 281.
 // (The plain 1x1 kernel has short chains; 5x5 layers are not built here.)
 static bool few_positions(const ConvDims &d, int variant) {
-    if (variant == 0 || variant >= 14) return false;
+    if (variant == 0 || variant >= 14 || ceil_div(d.Co, kFewTM) > kMaxGridY) return false;
     const int per_lane = variant == 3 ? FwdW8::TM * FwdW8::TN : variant == 4 || variant == 5 ? FwdW16S2::TM * FwdW16S2::TN
                        : variant == 8 || variant == 9 ? Fwd1x1sub::TM * Fwd1x1sub::TN : FwdW32::TM * FwdW32::TN;
     const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;

@@ -1076,6 +1076,7 @@ static_assert(GxW32::TM == GxW16::TM && GxW16::TM == GxW8::TM && GxS2W32::TM == 
 // channels, with gy (read from global memory: a map this small sits in L1 / L2) and the weights G output channels ahead
 // of the arithmetic; the chunk sums go through LDS and are added in channel order.
 // ---------------------------------------------------------------------------
+static constexpr int kFewTM = 4;
 template <int KS, int TM, int G, class T>
 __global__ __launch_bounds__(512) void grad_x_few_kernel(const T *__restrict__ gy, const T *__restrict__ x,
                                                          const float *__restrict__ w, T *__restrict__ gx,
@@ -1186,7 +1187,7 @@ static int few_chunk(const ConvDims &d) {
 static int grad_x_bn_variant(const ConvDims &d);
 template <class T>
 static bool few_positions(const ConvDims &d, int per_lane) {
-    if (sizeof(T) == 4 && grad_x_bn_variant(d)) return false;
+    if ((sizeof(T) == 4 && grad_x_bn_variant(d)) || ceil_div(d.Ci, kFewTM) > kMaxGridY) return false;
     const bool nine = d.kh == 3;
     const int chunk = few_chunk(d);
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
@@ -1198,7 +1199,7 @@ static bool few_positions(const ConvDims &d, int per_lane) {
 
 template <int KS, class T>
 static int launch_grad_x_few(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
-    constexpr int TM = 4, G = KS == 1 ? 8 : 1;
+    constexpr int TM = kFewTM, G = KS == 1 ? 8 : 1;
     const int chunk = few_chunk(d);
     const int chunks = ceil_div(d.Co, chunk), waves = chunks < 8 ? chunks : 8;
     hipLaunchKernelGGL((grad_x_few_kernel<KS, TM, G, T>), dim3(ceil_div(d.N * d.H * d.W, 64), ceil_div(d.Ci, TM)),
@@ -1263,7 +1264,7 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
                                        : launch_grad_x_3x3s1<Gx1x1s, true, T>(gy, x, w, gx, f, s, none, sub);
         }
     }
-    if (conv1x1_supported(d, gy, gx))
+    if (conv1x1_supported(d, gy, gx) && ceil_div(d.Ci, kGx1x1TM) <= kMaxGridY)
         return launch_grad_x_1x1(gy, x, w, gx, d, s);
     constexpr int TM = 8;
     const long total = (long)d.N * d.H * d.W;

@@ -18,6 +18,12 @@ def test_layers_change_from_the_few_positions_to_the_tiled_kernel_with_the_batch
         assert fwd_kernel(case) == FEW_POSITIONS and fwd_kernel((batch,) + case[1:]) == kernel, case
 
 
+def test_layers_beyond_the_grid_of_the_few_positions_kernel_stay_tiled():
+    # four output channels per workgroup, at most 65535 workgroups
+    assert fwd_kernel((1, 256, 1, 1, 4 * 65535, 3, 1, 1)) == FEW_POSITIONS
+    assert fwd_kernel((1, 256, 1, 1, 4 * 65535 + 1, 3, 1, 1)) == 30
+
+
 def test_the_query_refuses_what_the_forward_refuses():
     from addernetcuda_amd._lib import lib
     kernel = ctypes.c_int()
