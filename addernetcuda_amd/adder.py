@@ -435,9 +435,8 @@ class _adder_nchw(Function):
 
 class _adder_nchw_bf16(Function):
     """The optional reduced-storage mode: X, the output and their gradients are bfloat16 tensors (half the HBM
-    traffic and activation memory), W and its gradient stay float32, and every sum is accumulated exactly as in the
-    float32 path (fp32 for the output and grad_X, fp64 for grad_W); results are rounded to bfloat16 once, on the
-    way out.  The reference has no such mode (adder.cu:310-318 is float only); it is chosen by passing a bfloat16
+    traffic and activation memory), W and its gradient stay float32, and so do the sums of the output and grad_X;
+    those of grad_W are carried in fp64; results are rounded to bfloat16 once, on the way out.  The reference has no such mode (adder.cu:310-318 is float only); it is chosen by passing a bfloat16
     input and is never a default."""
 
     @staticmethod

@@ -40,16 +40,7 @@ __device__ __forceinline__ ColVec<COLS> col_load(const float *__restrict__ row, 
     return r;
 }
 
-// The weights live in LDS, not in scalar registers: the block's TM rows of W sit transposed ([k][TM], blocks of
-// KB rows of X at a time) and every lane reads the same four at a time (broadcast ds_read_b128).  LDS reads return
-// in order, so the waits for them are counted ones and several rows' weights stay in flight; scalar loads return
-// out of order and every wait for them is a wait for all of them (measured on K = 144, NL = 262 144, 16 rows of W:
-// 50 us with scalar weights in any blocking, 39 us like this).
-// KW = 4 (matrices with few columns): the four waves of a workgroup share their 64 * COLS columns and split the
-// rows of every block of X between them, so that the chain of dependent row batches is a quarter as long; their
-// partial sums are added through LDS at the end.
-//
-// Staging them: 256 / TM lanes per row of W, eight loads in flight per thread.  (One element at a time, with the row
+// Rows of W, transposed, into LDS: 256 / TM lanes per row, eight loads in flight per thread.  (One element at a time, with the row
 // found by a division, was a chain of 18 trips to L2 before the first row of X: a quarter of the kernel's time.)
 template <int TM, bool ZERO_PAST_CO>
 __device__ __forceinline__ void stage_weights(float *__restrict__ wt, const float *__restrict__ Wm, int K, int co0, int Co,
@@ -68,6 +59,14 @@ __device__ __forceinline__ void stage_weights(float *__restrict__ wt, const floa
     }
 }
 
+// The weights live in LDS, not in scalar registers: the block's TM rows of W sit transposed ([k][TM], blocks of
+// KB rows of X at a time) and every lane reads the same four at a time (broadcast ds_read_b128).  LDS reads return
+// in order, so the waits for them are counted ones and several rows' weights stay in flight; scalar loads return
+// out of order and every wait for them is a wait for all of them (measured on K = 144, NL = 262 144, 16 rows of W:
+// 50 us with scalar weights in any blocking, 39 us like this).
+// KW = 4 (matrices with few columns): the four waves of a workgroup share their 64 * COLS columns and split the
+// rows of every block of X between them, so that the chain of dependent row batches is a quarter as long; their
+// partial sums are added through LDS at the end.
 template <int TM, int COLS, bool VEC, int PF, int KW>
 __global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restrict__ X,
                                                           const float *__restrict__ Wm,

@@ -6,7 +6,7 @@
 //   forward  y[n,co,ho,wo]  = -sum_ci |w[co,ci] - x[n,ci,ho*S,wo*S]|
 //   grad_x   gx[n,ci,hi,wi] =  sum_co hardtanh(w[co,ci] - x) * gy[n,co,hi/S,wi/S]  on the sampled
 //                              grid, exactly 0 on the positions stride 2 skips
-//   grad_w   gw[co,ci]      =  sum x*gy - w * sum gy   (partials folded per wave, summed in fp64)
+//   grad_w   gw[co,ci]      =  sum x*gy - w * sum gy   (see the kernel for the precision of its partial sums)
 // Replaces adder.cu:19-70 / 194-272 for these shapes together with the
 // unfold/fold copies of adder.py:32-33,38-39.
 #include "common.hpp"

@@ -342,7 +342,7 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
             static_assert(sizeof(T) == 4 && !MUL && !PAIR, "inference epilogue: float adder layers");
             // Inference: the BatchNorm behind the layer, the shortcut and the ReLU on the way out instead of three more passes
             // over the map (two launches and a fill for the BatchNorm, one each for add and ReLU): ResNet-50, 32 images,
-            // 9.53 -> 8.31 ms, of which 1.65 ms were those passes; ResNet-20, one image, 90 -> 28 launches, 870 -> 470 us.
+            // 9.53 -> 8.31 ms, of which 1.65 ms were those passes; ResNet-20, one image, 90 -> 25 launches, 870 -> 470 us.
             {
                 float r[TM][TN];
 #pragma unroll

@@ -338,7 +338,7 @@ int launch_norm_scale(float *g, long n, float eta, float eps, void *ws, hipStrea
 
 // ---- dispatch -----------------------------------------------------------------
 struct GradWPlan {
-    int variant;  // 0 generic, 1 1x1 kernel (fp32 partial slabs), 2 3x3 matrix-core kernel (fp64 partial slabs)
+    int variant;  // 0 generic, 1 plain 1x1 kernel (slabs fp32, for bfloat16 storage fp64), 2 matrix-core kernel (fp64 slabs)
     GradWMfmaPlan mfma;
     int slots;
 };

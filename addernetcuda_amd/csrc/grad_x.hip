@@ -1041,13 +1041,13 @@ using GxS2W16 = GradX3x3S2Cfg<2, 8, 16, 1, 4, 8, 16>;    // inputs 16 wide: one 
 using GxW32 = Tile3x3Cfg<4, 8, 16, 1, 4, 4, 8, 1>;    // inputs 32 wide: half an image x 16 channels
 using GxW16 = Tile3x3Cfg<4, 4, 16, 1, 4, 8, 16, 1>;   // inputs 16 wide: one image x 32 channels
 using GxW8  = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 16, 1>;    // inputs 8 wide: two images x 32 channels
-// 1x1, stride 1: (H, W) planes walked as one row; a unit is one output channel x the lane's 8 input channels
 // 5x5 taps, two input channels x two positions per lane, so that a layer of a few dozen channels still has two waves per
-// SIMD: 32 -> 64 @16x16, 64 images (0.84e9 terms) generic kernel 529 us, this 62 us; four positions per lane 94 us (but
+// SIMD: 32 -> 64 @16x16, 64 images (0.84e9 terms) generic kernel 529 us, this 49 us (62 when the shape was picked, four positions per lane 94; but
 // 128 -> 64 167 against 184 us: a chip with enough waves would rather have fewer LDS reads per term)
 using Gx5W32 = Tile3x3Cfg<2, 16, 8, 1, 2, 4, 8, 1, 1, 5>;   // 8 rows of one image x 8 channels
 using Gx5W16 = Tile3x3Cfg<2, 8, 16, 1, 2, 4, 8, 1, 1, 5>;   // inputs 9..16 wide: one image x 8 channels
 using Gx5W8  = Tile3x3Cfg<2, 4, 8, 4, 2, 4, 8, 1, 1, 5>;    // inputs up to 8 wide: four images x 8 channels
+// 1x1, stride 1: (H, W) planes walked as one row; a unit is one output channel x the lane's 8 input channels
 using Gx1x1  = Tile3x3Cfg<2, 64, 1, 1, 8, 8, 16, 2, 1, 1>;    // 128 positions of one image x 64 channels
 using Gx1x1s = Tile3x3Cfg<4, 16, 1, 4, 8, 8, 16, 1, 1, 1>;    // planes of <= 64 positions: four images
 using Gx1x1t = Tile3x3Cfg<2, 32, 1, 2, 4, 8, 16, 8, 1, 1>;    // ... two images x 32 channels, where Gx1x1s would leave CUs idle

@@ -159,8 +159,8 @@ ADDER_API int adder_conv2d_bwd_add_f32(const float *gy, const float *x, const fl
 
 /* Optional reduced-storage mode: the activations and their gradients (x, y, gy, gx) are stored as bfloat16 (the
  * upper half of an fp32, rounded to nearest even on the way out) and take half the HBM traffic and half the
- * activation memory; weights and weight gradients stay fp32, every sum is accumulated as in the fp32 entry points
- * (fp32 for y and gx, fp64 for gw).  The reference computes in fp32 only (adder.cu:310-318 hard-codes
+ * activation memory; weights and weight gradients stay fp32, and so do the sums of y and gx; those of gw are carried in
+ * fp64 (fp32 runs of at most 64 terms in the kernels for narrow 1x1 layers and for the shapes without a tiled kernel).  The reference computes in fp32 only (adder.cu:310-318 hard-codes
  * data<float>()), so these have no counterpart there and are never the default.  Same dimensions, semantics, eta
  * and workspace (adder_conv2d_bwd_workspace_bytes) as adder_conv2d_fwd_f32 / adder_conv2d_bwd_f32, and the same
  * kernels and tile shapes. */
