@@ -552,9 +552,15 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
 // sum is long and carries the full magnitude (0.46 at 1024 with the first level folded every fourth chunk).
 // 5x5 layers (50-term first levels): worst element 0.40 at 1150 terms, 0.56 at 2500; relative error 2.7e-7 and 3.1e-7, where the kernel
 // without tiles has 3.4e-7 and 3.5e-7.
-static constexpr int kSatMaxTerms = 1152, kSatMaxTerms1x1 = 1024, kSatMaxTerms5x5 = 2500;
+// Below ten output channels the doubled and the subtracted sum are what rounds, not the length of the sums: 5x5 layers of 1 / 4 / 8
+// channels 1.8e-7 / 2.4e-7 / 2.5e-7 with two instructions, 0.9e-7 / 1.25e-7 / 1.3e-7 with three (kernel without tiles 0.9e-7 / 1.7e-7 / 2.4e-7);
+// 64 -> 8 @32x32, 64 images, 52 -> 63 us.
+static constexpr int kSatMaxTerms = 1152, kSatMaxTerms1x1 = 1024, kSatMaxTerms5x5 = 2500, kSatMinChannels5x5 = 10;
 template <class C>
-constexpr int sat_max_terms() { return C::KS == 1 ? kSatMaxTerms1x1 : (C::KS == 5 ? kSatMaxTerms5x5 : kSatMaxTerms); }
+static bool two_instructions(int Co) {
+    if (C::KS == 5 && Co < kSatMinChannels5x5) return false;
+    return Co * C::KK <= (C::KS == 1 ? kSatMaxTerms1x1 : (C::KS == 5 ? kSatMaxTerms5x5 : kSatMaxTerms));
+}
 
 static const adder_bn_links kNoLinks{};
 
@@ -578,19 +584,19 @@ static int launch_grad_x_3x3s1_v(const T *gy, const T *x, const float *w, T *gx,
 template <class C>
 static int launch_grad_x_3x3s1_bn(const float *gy, const float *x, const float *w, float *gx, const ConvDims &d,
                                   hipStream_t s, const float *gadd, const adder_bn_links &bn) {
-    if (d.Co * C::KK > sat_max_terms<C>())
+    if (!two_instructions<C>(d.Co))
         return launch_grad_x_3x3s1_v<C, true, false, false, float, true>(gy, x, w, gx, d, s, Subsample{1, 0, 0, 0}, gadd, bn);
     return launch_grad_x_3x3s1_v<C, true, true, false, float, true>(gy, x, w, gx, d, s, Subsample{1, 0, 0, 0}, gadd, bn);
 }
 
 // picks the element-wise tile loads (rows of the staged tensor that are not whole float4 groups) and the
-// three-instruction form (more terms per output than kSatMaxTerms)
+// three-instruction form (two_instructions)
 template <class C, bool SUB = false, class T = float>
 static int launch_grad_x_3x3s1(const T *gy, const T *x, const float *w, T *gx,
                                const ConvDims &d, hipStream_t s, const T *gadd = nullptr,
                                const Subsample sub = Subsample{1, 0, 0, 0}) {
     const bool vec = d.W % 4 == 0;
-    if (d.Co * C::KK > sat_max_terms<C>())
+    if (!two_instructions<C>(d.Co))
         return vec ? launch_grad_x_3x3s1_v<C, true, false, SUB, T>(gy, x, w, gx, d, s, sub, gadd)
                    : launch_grad_x_3x3s1_v<C, false, false, SUB, T>(gy, x, w, gx, d, s, sub, gadd);
     return vec ? launch_grad_x_3x3s1_v<C, true, true, SUB, T>(gy, x, w, gx, d, s, sub, gadd)

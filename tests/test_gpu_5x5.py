@@ -59,6 +59,21 @@ def test_5x5_forward_of_many_channels_keeps_its_precision(H, stride, Ci, gpu):
     assert (got - want).norm() <= 1.2 * 0.4 * 2.0 ** -24 * ((400 / n2 + n2) / 3) ** 0.5 * want.norm()
 
 
+@pytest.mark.parametrize("Co", [1, 2, 4, 9])
+@pytest.mark.parametrize("H", [24, 16, 7])
+def test_5x5_grad_x_of_few_output_channels_keeps_its_precision(H, Co, gpu):
+    from addernetcuda_amd import adder
+    from oracle import c_oracle
+    x, w, gy = make_case(4, 16, H, H, Co, 5, 1, 2)
+    want = c_oracle.conv2d_grad_x(gy, x, w, 1, 2)
+    xg = x.to(gpu).requires_grad_(True)
+    adder.adder2d_function(xg, w.to(gpu), 1, 2).backward(gy.to(gpu))
+    # Terms of either sign: adding n of them rounds to 0.4 * 2^-24 * sqrt(n / 2) of the result, here sums of at most 50 and Co / 2 of
+    # those, and a term's difference to about one addition.  (Two-instruction form, 2 sum d g - sum g: 1.8e-7 to 2.4e-7.)
+    bound = 0.4 * 2.0 ** -24 * (min(25 * Co, 50) / 2 + Co / 4 + 1) ** 0.5
+    assert (xg.grad.double().cpu() - want).norm() <= 1.2 * bound * want.norm()
+
+
 def test_without_a_workspace_where_the_slabs_do_not_fit(gpu):
     from addernetcuda_amd._lib import lib, ptr, stream_ptr, conv_dims, check, conv2d_bwd_workspace
     from oracle import c_oracle
