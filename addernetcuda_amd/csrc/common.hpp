@@ -307,6 +307,13 @@ int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, co
 int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double *sgpart, const ConvDims &d,
                           const GradWMfmaPlan &p, const float *bn_y, const float *bn_coef, float *gy_out, hipStream_t s,
                           const BnSums &sums = kNoBnSums);
+int plan_grad_w_slots(int blocks, int ntiles, size_t slab_bytes);
+// the same on the 8-bit matrix cores (grad_w_i8.hip): variants from 20 on; bn_y and the rest as in launch_grad_w
+bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p);
+template <class T>
+int launch_grad_w_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
+                     const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,
+                     const BnSums &sums = kNoBnSums);
 
 // 1x1 / pad 0 / stride 1-2 kernels (conv1x1.hip)
 bool conv1x1_supported(const ConvDims &d, const void *a, const void *b);

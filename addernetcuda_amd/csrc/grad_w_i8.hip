@@ -1,0 +1,629 @@
+// Weight gradient of 3x3 / pad 1 and 5x5 / pad 2 layers of stride 1 on the 8-bit matrix cores, as exact as the fp64 ones.
+//
+//   gw[co,ci,i,j] = sum_pos x[ci, pos + (i,j)] * gy[co,pos]  -  w[co,ci,i,j] * sum_pos gy[co,pos]
+//
+// The sum over positions needs more than fp32 (see grad_w_mfma.hip), and v_mfma_f64_16x16x4_f64 gives it at 16 multiply-adds a
+// cycle and SIMD.  v_mfma_i32_16x16x64_i8 does 1000, exactly, so the operands are written in fixed point, four signed 8-bit digits
+// each, and thirteen digit products (of the sixteen: the three left out lie below the last digit) stand for one fp64 product:
+//   x = 2^ex * sum_d X_d 2^-8d,   gy = 2^eg * sum_d G_d 2^-8d,   x * gy = 2^(ex+eg) * sum_{s<5} 2^-8s sum_{d+e=s} X_d G_e.
+// The scales 2^ex, 2^eg belong to one channel of one staged tile (256 positions), so the fixed point is relative to the
+// largest of 256 values: 32 bits, every value down to 1/64 of the largest keeps all its 24 bits, and as the largest of 256 is at
+// most 16 times their root mean square, whatever the data, a tile's sums are off by at most 2^-25 of |x| |gy|, in practice by
+// 2^-30 of the result (relative error of the raw gradient, 2-norm: 2.549e-8 where the fp64 kernel has 2.549e-8, 128 -> 128 @32x32, 128
+// images; ten products: 2.56e-8).  The digit sums of a tile are exact in 32 bits (at most four products of 2^14, 256 positions) and go
+// into fp64 sums with their scales.  A tile with a value that is infinite or not a number is worked out in fp64 from the same LDS cells.
+//
+// Layout: a tile is four images x 64 positions.  Its LDS cells are dwords of one digit of four images, so that a
+// lane's sixteen 8-bit operands -- four adjacent columns x four images -- are four cells of a row, and a tap's shift moves whole
+// cells: j shifts by register, i by row.  MFMA rows are output channels, columns are input channels; a wave owns one tap
+// row of a 16 x 16 channel block, i.e. KS accumulator tiles x five digit weights.
+//
+// Half of a workgroup's waves multiply, the other half load, find the largest values and write digits, a tile ahead: the conversion is
+// 6.5 vector instructions a value, nearly as much time as the matrix instructions it feeds, and on other waves it runs beside them.
+// What bounds it (128 -> 128 @32x32, 128 images, 1.9e10 multiply-adds: 690 -> 272 us): the multiplying waves -- 78 matrix
+// instructions of 16 cycles per step with the operand moves between them; without the loading waves' work it takes 252 us, without the
+// multiplying waves' 175.  (All waves doing both in turn: 605; loads that branch, so that every wait is for all of them: 300.)
+#include "common.hpp"
+#include "grad_w_bn.hpp"
+
+#include <type_traits>
+
+namespace adder {
+
+typedef int int4v __attribute__((ext_vector_type(4)));
+
+template <int KS_, int TH_, int TW_, int MB_, int NB_, int PW_, int LWAVES_, int MINWAVES_>
+struct GwI8Cfg {
+    static constexpr int KS = KS_, KK = KS_ * KS_, PAD = KS_ / 2, TH = TH_, TW = TW_, MB = MB_, NB = NB_, MINWAVES = MINWAVES_;
+    static constexpr int COB = 16 * MB, CIB = 16 * NB;
+    // A tile's rows fall into strips of eight columns; a step of the multiplying waves takes four strips, one per 16 lanes.
+    static constexpr int STRIPS = TW / 8, PW = PW_, STEPS = TH * STRIPS / 4 / PW;   // PW waves share a tile's steps
+    static constexpr int MWAVES = KS * MB * NB * PW, LWAVES = LWAVES_;      // multiplying and loading waves
+    static constexpr int NTHREADS = 64 * (MWAVES + LWAVES), LTHREADS = 64 * LWAVES;
+    static constexpr int QW = TW / 4;                          // groups of four columns per row
+    // x cells: [channel][digit][row][column] with the halo columns of the rows behind them, [row][2 PAD]; gy cells alike.  Channels start
+    // four banks apart (16-byte reads of eight channels meet 32 banks).
+    static constexpr int XR = TH + KS - 1, HC = 2 * PAD, XH = XR * TW, XDIG = XH + XR * HC, XPLANE = round_up(4 * XDIG, 32) + 4;
+    static constexpr int GDIG = TH * TW, GPLANE = 4 * GDIG + 4;
+    static constexpr int XUNITS = CIB * XR * QW, HUNITS = CIB * XR * HC, GUNITS = COB * TH * QW;
+    static constexpr int XITER = ceil_div(XUNITS, LTHREADS), HITER = ceil_div(HUNITS, LTHREADS), GITER = ceil_div(GUNITS, LTHREADS);
+    static constexpr int G0 = CIB * XPLANE;                    // a tile's x cells, then its gy cells
+    static constexpr int TILE_WORDS = G0 + COB * GPLANE;
+    static constexpr int OUT = COB * CIB * KK;                 // results, folded and reordered through LDS at the end (fp64)
+    static constexpr int CH = COB + CIB;                       // largest-value slots: gy channels, then x channels
+    static constexpr int MX0 = 2 * TILE_WORDS, COEF0 = MX0 + 4 * CH + 4;
+    static constexpr int LDS_BYTES = COEF0 * 4;
+    static_assert(TW % 8 == 0 && 4 % STRIPS == 0 && TH * STRIPS % (4 * PW) == 0 && KS % 2 == 1, "whole steps of four strips");
+    static_assert((XR * QW) % 4 == 0 && (XR * HC) % 4 == 0 && (TH * QW) % 4 == 0, "four units in a row share a channel");
+    static_assert(LDS_BYTES + COB * 16 <= 160 * 1024 && NTHREADS <= 1024, "workgroup limits");
+    static_assert(2 * (OUT + COB) <= 2 * TILE_WORDS, "the results fit the cells' place");
+    static_assert(XDIG % 4 == 0 && XH % 4 == 0 && GPLANE % 4 == 0 && COEF0 % 4 == 0, "16-byte alignment of the cells");
+};
+
+// Four images of a tensor as a buffer: loads from beyond its end (images that do not exist) or at kNowhere give zeros, so they need no
+// branch -- with loads under way in two register sets, a wait has to know how many are newer.
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+static constexpr unsigned kNowhere = 0x80000000u;
+static constexpr int kBufferImage = 1 << 27;   // elements per image: four of float fill 2^31 bytes, and kNowhere + three does not wrap
+template <class T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t i8_images(const T *base, int image, int n0, int N) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(base + (size_t)n0 * image), 0, min(4, N - n0) * image * (int)sizeof(T), 0x00020000);
+}
+template <class T>
+__device__ __forceinline__ float i8_load1(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    if constexpr (sizeof(T) == 4) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    else return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+}
+// four consecutive elements of a row, `left` elements before its end (VEC: rows are whole groups of four)
+template <bool VEC, class T>
+__device__ __forceinline__ float4 i8_load4(__amdgpu_buffer_rsrc_t r, unsigned off, int left) {
+    if constexpr (!VEC) {
+        constexpr unsigned E = sizeof(T);
+        return make_float4(i8_load1<T>(r, off), i8_load1<T>(r, left > 1 ? off + E : kNowhere), i8_load1<T>(r, left > 2 ? off + 2 * E : kNowhere),
+                           i8_load1<T>(r, left > 3 ? off + 3 * E : kNowhere));
+    } else if constexpr (sizeof(T) == 4) {
+        const uint4v u = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+        return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
+    } else {
+        const uint2v u = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+        return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                           __uint_as_float(u.y & 0xffff0000u));
+    }
+}
+
+// the larger magnitude, as bits (NaN and infinity come out above every number)
+__device__ __forceinline__ float i8_absmax(float m, float a, float b) {
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(a), fabsf(b)), m);
+}
+__device__ __forceinline__ float i8_absmax4(float m, const float4 &v) { return i8_absmax(i8_absmax(m, v.x, v.y), v.z, v.w); }
+
+// A channel's exponent from the bits of its largest magnitude: magnitudes from 1.96875 up count as the next power of two,
+// so that |v| 2^(30-e) < 2^31 - 2^24 and the first digit stays within +-127 (the last three carry into it).  255: not finite (or within
+// 1.6 % of the largest float), the tile takes the fp64 path.  Below 2^-97 the last digit stays at 2^-127, which 2^127 still reaches.
+__device__ __forceinline__ int i8_exponent(unsigned m) { return max((int)((m + 0x40000u) >> 23), 30); }
+__device__ __forceinline__ double i8_unit(int e) { return __hiloint2double((e - 127 - 30 + 1023) << 20, 0); }   // 2^(e - 127 - 30): the last digit's
+__device__ __forceinline__ float i8_scale(int e) { return __uint_as_float((unsigned)(30 + 127 + 127 - e) << 23); }   // its reciprocal, 2^(30 - (e - 127))
+
+// largest magnitude of the four lanes of a quad into its channel's slot
+__device__ __forceinline__ void i8_note_max(float m, unsigned *slot, unsigned *flag, bool ok) {
+    unsigned u = __float_as_uint(m) & 0x7fffffffu;
+    u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+    u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+    if (ok && (threadIdx.x & 3) == 0) {
+        atomicMax(slot, u);
+        if (i8_exponent(u) >= 255) *flag = 1;
+    }
+}
+
+// v times a power of two, to the nearest integer.  (v_cvt_rpi_i32_f32 would do both steps, but rounds odd results above 2^23 away.)
+__device__ __forceinline__ unsigned i8_round(float v, float scale) { return (unsigned)(int)rintf(v * scale); }
+// four values (one column of four images) as four cells, one per digit.  Adding 0x808080 turns the lower three digits into unsigned
+// ones with carries, the exclusive-or makes them signed again.
+__device__ __forceinline__ void i8_digits(float a, float b, float c, float d, float scale, int (&cell)[4]) {
+    const unsigned u0 = i8_round(a, scale) + 0x808080u, u1 = i8_round(b, scale) + 0x808080u,
+                   u2 = i8_round(c, scale) + 0x808080u, u3 = i8_round(d, scale) + 0x808080u;
+    const unsigned lo01 = __builtin_amdgcn_perm(u1, u0, 0x05010400u), hi01 = __builtin_amdgcn_perm(u1, u0, 0x07030602u);
+    const unsigned lo23 = __builtin_amdgcn_perm(u3, u2, 0x05010400u), hi23 = __builtin_amdgcn_perm(u3, u2, 0x07030602u);
+    cell[0] = (int)__builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+    cell[1] = (int)(__builtin_amdgcn_perm(hi23, hi01, 0x05040100u) ^ 0x80808080u);
+    cell[2] = (int)(__builtin_amdgcn_perm(lo23, lo01, 0x07060302u) ^ 0x80808080u);
+    cell[3] = (int)(__builtin_amdgcn_perm(lo23, lo01, 0x05040100u) ^ 0x80808080u);
+}
+
+// a unit of four columns x four images into the cells at p (p + digit * pitch); raw: the values themselves, image k in the
+// place of digit k
+__device__ __forceinline__ void i8_put4(const float4 (&v)[4], float scale, bool raw, int *p, int pitch) {
+    if (!raw) {
+        int c0[4], c1[4], c2[4], c3[4];
+        i8_digits(v[0].x, v[1].x, v[2].x, v[3].x, scale, c0);
+        i8_digits(v[0].y, v[1].y, v[2].y, v[3].y, scale, c1);
+        i8_digits(v[0].z, v[1].z, v[2].z, v[3].z, scale, c2);
+        i8_digits(v[0].w, v[1].w, v[2].w, v[3].w, scale, c3);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) *reinterpret_cast<int4v *>(p + k * pitch) = int4v{c0[k], c1[k], c2[k], c3[k]};
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) *reinterpret_cast<float4 *>(p + k * pitch) = v[k];
+    }
+}
+
+// The digit sums of one result (a[s]: digit weights 2^-8s) in units of the third: first digits lie within +-127, the others within
+// +-128, a tile has 256 positions, so the sums stay below 2^26 and the first two fit one 32-bit number.  (The fifth and fourth are
+// rounded to the unit of the third, 2^-29 of the result: the fourth starts at half of that.)
+__device__ __forceinline__ double i8_product(int a0, int a1, int a2, int a3, int a4) {
+    return fma((double)((a0 << 8) + a1), 256.0, (double)(a2 + ((a3 + (a4 >> 8)) >> 8)));
+}
+// the digit sums of at most 256 values as their sum, exactly
+__device__ __forceinline__ double i8_sum(int a0, int a1, int a2, int a3) {
+    return fma((double)((a0 << 8) + a1), 65536.0, (double)((a2 << 8) + a3));
+}
+
+template <class G, bool VEC = true, class T = float, bool FUSE = false>
+__global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(const T *__restrict__ gy, const T *__restrict__ x,
+                                                                double *__restrict__ part, double *__restrict__ sgpart, int N,
+                                                                int Ci, int H, int W, int Co, int tilesH, int tilesW, int ntiles,
+                                                                const float *__restrict__ bn_y, const float *__restrict__ bn_coef,
+                                                                float *__restrict__ gy_out, const BnSums sums) {
+    static_assert(!FUSE || (VEC && sizeof(T) == 4), "the BatchNorm link belongs to the float kernels");
+    constexpr int KS = G::KS, PAD = G::PAD, QW = G::QW, SQ = 2;   // SQ: groups of four columns in a strip
+    extern __shared__ __align__(16) int cells[];   // two tiles: x cells, gy cells
+    unsigned *const mx = reinterpret_cast<unsigned *>(cells + G::MX0);   // largest magnitudes of four tiles, then four flags
+    unsigned *const flags = mx + 4 * G::CH;
+    float4 *const coef = reinterpret_cast<float4 *>(cells + G::COEF0);
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+    const bool loader = wave >= G::MWAVES;
+    const int lt = tid - 64 * G::MWAVES;   // loader thread
+    // a multiplying wave's accumulators (tap row, block of 16 output channels, of 16 input channels) and its share of a tile's steps
+    const int ti = wave % KS, pw = wave / KS % G::PW, mb = wave / KS / G::PW % G::MB, nb = wave / KS / G::PW / G::MB;
+    const int co_blk = blockIdx.y * G::COB, ci_blk = blockIdx.z * G::CIB;
+    float *const gy_dst = blockIdx.z == 0 ? gy_out : nullptr;   // every gy tile is staged once per block of input channels
+    // the workgroup's tiles lie side by side: the lines that neighbouring tiles share stay in one L2
+    const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, tile0 = blockIdx.x * each, mine = min(each, ntiles - tile0);
+
+    if constexpr (FUSE) {   // the block's BatchNorm coefficients
+        if (sums.part) {
+            bn_coef_from_sums<G>(sums, co_blk, Co, coef, blockIdx.x == 0 && blockIdx.z == 0);
+        } else {
+            for (int e = tid; e < G::COB; e += G::NTHREADS) coef[e] = reinterpret_cast<const float4 *>(bn_coef)[min(co_blk + e, Co - 1)];
+        }
+    }
+    for (int e = tid; e < 4 * G::CH + 4; e += G::NTHREADS) mx[e] = 0;
+    __syncthreads();
+
+    // ---- the loading waves ----
+    // A thread's units: channel, row and column within the tile, offset from the tile's first position, place among the cells.
+    const int ximg = Ci * H * W, gimg = Co * H * W;
+    int gch[G::GITER], grow[G::GITER], gcol[G::GITER], xch[G::XITER], xrow[G::XITER], xcol[G::XITER], hch[G::HITER], hrow[G::HITER], hcol[G::HITER];
+#pragma unroll
+    for (int it = 0; it < G::GITER; ++it) {
+        const int u = lt + it * G::LTHREADS;
+        gcol[it] = u % QW * 4; grow[it] = u / QW % G::TH; gch[it] = u / QW / G::TH;
+    }
+#pragma unroll
+    for (int it = 0; it < G::XITER; ++it) {
+        const int u = lt + it * G::LTHREADS;
+        xcol[it] = u % QW * 4; xrow[it] = u / QW % G::XR; xch[it] = u / QW / G::XR;
+    }
+#pragma unroll
+    for (int it = 0; it < G::HITER; ++it) {
+        const int u = lt + it * G::LTHREADS;
+        hcol[it] = u % G::HC; hrow[it] = u / G::HC % G::XR; hch[it] = u / G::HC / G::XR;
+    }
+    // Two tiles under way in registers; one, where a thread has two gy units: the multiplying waves last longer than a load there, and
+    // a second set would spill (128 -> 128 @32x32, 128 images, 275 us with two, 272 with one).
+    constexpr int SETS = KS == 3 && G::GITER > 1 ? 1 : 2;
+    float4 xv[SETS][G::XITER][4], gv[SETS][G::GITER][4], yv[SETS][FUSE ? G::GITER : 1][4];
+    float hv[SETS][G::HITER][4];
+    auto place = [&](const int i, int &n0, int &h0, int &w0) {
+        int t = tile0 + i;
+        const int tw = t % tilesW; t /= tilesW;
+        const int th = t % tilesH; t /= tilesH;
+        n0 = t * 4; h0 = th * G::TH; w0 = tw * G::TW;
+    };
+    // (Always inlined: a call would put the registers it captures into memory.)
+    // tile i of the workgroup (nothing, if it has none) into register set b
+    auto fetch = [&](const int i, auto set) __attribute__((always_inline)) {
+        constexpr int b = decltype(set)::value;
+        constexpr unsigned E = sizeof(T);
+        int n0, h0, w0;
+        place(min(i, mine - 1), n0, h0, w0);
+        const auto gbuf = i8_images(gy, gimg, n0, N), xbuf = i8_images(x, ximg, n0, N);
+#pragma unroll
+        for (int it = 0; it < G::GITER; ++it) {
+            const int ch = co_blk + gch[it], ho = h0 + grow[it], wo = w0 + gcol[it];
+            const bool ok = i < mine && (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB) && ch < Co && ho < H && wo < W;
+            const unsigned off = ok ? ((ch * H + ho) * W + wo) * E : kNowhere;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) gv[b][it][k] = i8_load4<VEC, T>(gbuf, off + k * gimg * E, W - wo);
+            if constexpr (FUSE) {
+                const auto ybuf = i8_images(bn_y, gimg, n0, N);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) yv[b][it][k] = i8_load4<true, float>(ybuf, off + k * gimg * E, W - wo);
+            }
+        }
+#pragma unroll
+        for (int it = 0; it < G::XITER; ++it) {
+            const int ch = ci_blk + xch[it], hi = h0 - PAD + xrow[it], wi = w0 + xcol[it];
+            const bool ok = i < mine && (G::XUNITS % G::LTHREADS == 0 || xch[it] < G::CIB) && ch < Ci && hi >= 0 && hi < H && wi < W;
+            const unsigned off = ok ? ((ch * H + hi) * W + wi) * E : kNowhere;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xv[b][it][k] = i8_load4<VEC, T>(xbuf, off + k * ximg * E, W - wi);
+        }
+#pragma unroll
+        for (int it = 0; it < G::HITER; ++it) {
+            const int ch = ci_blk + hch[it], hi = h0 - PAD + hrow[it], wi = w0 + (hcol[it] < PAD ? hcol[it] - PAD : G::TW + hcol[it] - PAD);
+            const bool ok = i < mine && (G::HUNITS % G::LTHREADS == 0 || hch[it] < G::CIB) && ch < Ci && hi >= 0 && hi < H && wi >= 0 && wi < W;
+            const unsigned off = ok ? ((ch * H + hi) * W + wi) * E : kNowhere;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) hv[b][it][k] = i8_load1<T>(xbuf, off + k * ximg * E);
+        }
+    };
+    // the largest magnitudes of the channels of tile i, which is in set b (FUSE: its gy is formed first)
+    auto note = [&](const int i, auto set) __attribute__((always_inline)) {
+        constexpr int b = decltype(set)::value;
+        unsigned *const mxs = mx + (i & 3) * G::CH, *const flag = flags + (i & 3);
+        if constexpr (FUSE) {
+            int n0, h0, w0;
+            place(i, n0, h0, w0);
+#pragma unroll
+            for (int it = 0; it < G::GITER; ++it) {
+                const int ch = co_blk + gch[it], ho = h0 + grow[it], wo = w0 + gcol[it];
+                const bool ok = i < mine && (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB) && ch < Co && ho < H && wo < W;
+                const float4 cf = coef[min(gch[it], G::COB - 1)];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const bool in = ok && n0 + k < N;   // (rows are whole groups of four)
+                    const float4 g = gv[b][it][k], y = yv[b][it][k];
+                    float4 v;
+                    v.x = in ? fmaf(cf.x, g.x, fmaf(cf.y, y.x - cf.z, -cf.w)) : 0.f;
+                    v.y = in ? fmaf(cf.x, g.y, fmaf(cf.y, y.y - cf.z, -cf.w)) : 0.f;
+                    v.z = in ? fmaf(cf.x, g.z, fmaf(cf.y, y.z - cf.z, -cf.w)) : 0.f;
+                    v.w = in ? fmaf(cf.x, g.w, fmaf(cf.y, y.w - cf.z, -cf.w)) : 0.f;
+                    gv[b][it][k] = v;
+                    if (gy_dst && in) *reinterpret_cast<float4 *>(gy_dst + ((n0 + k) * gimg + (ch * H + ho) * W + wo)) = v;
+                }
+            }
+        }
+#pragma unroll
+        for (int it = 0; it < G::GITER; ++it) {
+            const bool ok = G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB;
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) m = i8_absmax4(m, gv[b][it][k]);
+            i8_note_max(m, mxs + (ok ? gch[it] : 0), flag, ok);
+        }
+#pragma unroll
+        for (int it = 0; it < G::XITER; ++it) {
+            const bool ok = G::XUNITS % G::LTHREADS == 0 || xch[it] < G::CIB;
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) m = i8_absmax4(m, xv[b][it][k]);
+            i8_note_max(m, mxs + G::COB + (ok ? xch[it] : 0), flag, ok);
+        }
+#pragma unroll
+        for (int it = 0; it < G::HITER; ++it) {
+            const bool ok = G::HUNITS % G::LTHREADS == 0 || hch[it] < G::CIB;
+            const float m = i8_absmax(i8_absmax(0.f, hv[b][it][0], hv[b][it][1]), hv[b][it][2], hv[b][it][3]);
+            i8_note_max(m, mxs + G::COB + (ok ? hch[it] : 0), flag, ok);
+        }
+    };
+    // set b into the cells of tile i
+    auto commit = [&](const int i, auto set) __attribute__((always_inline)) {
+        constexpr int b = decltype(set)::value;
+        int *const tile = cells + (i & 1) * G::TILE_WORDS;
+        const unsigned *const mxs = mx + (i & 3) * G::CH;
+        const bool raw = __builtin_amdgcn_readfirstlane((int)flags[i & 3]) != 0;
+#pragma unroll
+        for (int it = 0; it < G::GITER; ++it)
+            if (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB)
+                i8_put4(gv[b][it], i8_scale(i8_exponent(mxs[gch[it]])), raw,
+                        tile + G::G0 + gch[it] * G::GPLANE + grow[it] * G::TW + gcol[it], G::GDIG);
+#pragma unroll
+        for (int it = 0; it < G::XITER; ++it)
+            if (G::XUNITS % G::LTHREADS == 0 || xch[it] < G::CIB)
+                i8_put4(xv[b][it], i8_scale(i8_exponent(mxs[G::COB + xch[it]])), raw,
+                        tile + xch[it] * G::XPLANE + xrow[it] * G::TW + xcol[it], G::XDIG);
+#pragma unroll
+        for (int it = 0; it < G::HITER; ++it)
+            if (G::HUNITS % G::LTHREADS == 0 || hch[it] < G::CIB) {
+                int cell[4];
+                if (!raw) {
+                    i8_digits(hv[b][it][0], hv[b][it][1], hv[b][it][2], hv[b][it][3], i8_scale(i8_exponent(mxs[G::COB + hch[it]])), cell);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) cell[k] = __float_as_int(hv[b][it][k]);
+                }
+                int *p = tile + hch[it] * G::XPLANE + G::XH + hrow[it] * G::HC + hcol[it];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) p[k * G::XDIG] = cell[k];
+            }
+    };
+
+    // ---- the multiplying waves ----
+    const bool sg_wave = ti == 0 && nb == 0 && blockIdx.z == 0;   // also adds gy up
+    double tot[KS][4], sgt = 0.0;   // tot[j][e]: row 4 * lk + e (output channel), column l16 (input channel), tap (ti, j)
+#pragma unroll
+    for (int j = 0; j < KS; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tot[j][e] = 0.0;
+    // The wave's operands: lane group lk takes strip lk of a step's four.  The cells before and after a strip are its neighbours' or,
+    // at the ends of a row, the halo's.  (Steps are whole rows apart, 4 / STRIPS of them.)
+    constexpr int ROWS = 4 / G::STRIPS;
+    const int strip = lk % G::STRIPS, lrow = pw * G::STEPS * ROWS + lk / G::STRIPS;
+    const int goff = G::G0 + (mb * 16 + l16) * G::GPLANE + lrow * G::TW + 8 * strip;
+    const int xch0 = (nb * 16 + l16) * G::XPLANE, xoff = xch0 + (lrow + ti) * G::TW + 8 * strip, xhalo = xch0 + G::XH + (lrow + ti) * G::HC;
+    const bool first = strip == 0, last = strip == G::STRIPS - 1;
+    const int loff = first ? xhalo : xoff - PAD, roff = last ? xhalo + PAD : xoff + 8;
+    const int lstep = ROWS * (first ? G::HC : G::TW), rstep = ROWS * (last ? G::HC : G::TW);
+    auto multiply = [&](const int i) {
+        const int *const tile = cells + (i & 1) * G::TILE_WORDS;
+        const unsigned *const mxs = mx + (i & 3) * G::CH;
+        int4v acc[KS][5];
+#pragma unroll
+        for (int j = 0; j < KS; ++j)
+#pragma unroll
+            for (int s = 0; s < 5; ++s) acc[j][s] = s != 3 ? int4v{0, 0, 0, 0} : int4v{128, 128, 128, 128};
+        // The x cells of one digit and step are a phase: KS matrix instructions per digit of gy that goes with it.  The next phase's cells
+        // are asked for before a phase's instructions, a step's last gy digits (which the last phase does not need) with them.
+        int4v a[SQ][4], mid[2][SQ];
+        int edge[2][2 * PAD];
+        auto ask_a = [&](const int rs, const int d) {
+#pragma unroll
+            for (int q = 0; q < SQ; ++q) a[q][d] = *reinterpret_cast<const int4v *>(tile + goff + rs * ROWS * G::TW + d * G::GDIG + 4 * q);
+        };
+        auto ask_x = [&](const int p) {
+            const int rs = p / 4, dx = p % 4;
+#pragma unroll
+            for (int q = 0; q < SQ; ++q) mid[p & 1][q] = *reinterpret_cast<const int4v *>(tile + xoff + rs * ROWS * G::TW + dx * G::XDIG + 4 * q);
+#pragma unroll
+            for (int e = 0; e < PAD; ++e) {
+                edge[p & 1][e] = tile[loff + rs * lstep + dx * G::XDIG + e];
+                edge[p & 1][PAD + e] = tile[roff + rs * rstep + dx * G::XDIG + e];
+            }
+        };
+        ask_x(0);
+        ask_a(0, 3);
+        ask_a(0, 2);
+#pragma unroll
+        for (int p = 0; p < 4 * G::STEPS; ++p) {
+            const int dx = p % 4;
+            if (dx == 0) { ask_a(p / 4, 1); ask_a(p / 4, 0); }
+            int win[8 + 2 * PAD];   // tap j of column c of the strip meets cell c + j
+#pragma unroll
+            for (int e = 0; e < PAD; ++e) { win[e] = edge[p & 1][e]; win[PAD + 8 + e] = edge[p & 1][PAD + e]; }
+#pragma unroll
+            for (int q = 0; q < SQ; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) win[PAD + 4 * q + e] = mid[p & 1][q][e];
+            if (p + 1 < 4 * G::STEPS) ask_x(p + 1);
+            if (dx == 3 && p + 1 < 4 * G::STEPS) { ask_a(p / 4 + 1, 3); ask_a(p / 4 + 1, 2); }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < SQ; ++q) {
+                int4v b[KS];
+#pragma unroll
+                for (int j = 0; j < KS; ++j) b[j] = int4v{win[4 * q + j], win[4 * q + j + 1], win[4 * q + j + 2], win[4 * q + j + 3]};
+#pragma unroll
+                for (int dg = dx == 0 ? 3 : 4 - dx; dg >= 0; --dg)
+#pragma unroll
+                    for (int j = 0; j < KS; ++j)
+                        acc[j][dx + dg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[q][dg], b[j], acc[j][dx + dg], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const double sx = i8_unit(i8_exponent(mxs[G::COB + nb * 16 + l16])) * 4294967296.0;   // (i8_product counts in 2^32)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const double sc = sx * i8_unit(i8_exponent(mxs[mb * 16 + 4 * lk + e]));
+#pragma unroll
+            for (int j = 0; j < KS; ++j)
+                tot[j][e] = fma(i8_product(acc[j][0][e], acc[j][1][e], acc[j][2][e], acc[j][3][e], acc[j][4][e]), sc, tot[j][e]);
+        }
+        if (sg_wave) {   // (read again: the digits that the matrix instructions had are gone)
+            int sd[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int rs = 0; rs < G::STEPS; ++rs)
+#pragma unroll
+                for (int q = 0; q < SQ; ++q)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const int4v g = *reinterpret_cast<const int4v *>(tile + goff + rs * ROWS * G::TW + d * G::GDIG + 4 * q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sd[d] = __builtin_amdgcn_sdot4(g[e], 0x01010101, sd[d], false);
+                    }
+            sgt = fma(i8_sum(sd[0], sd[1], sd[2], sd[3]), i8_unit(i8_exponent(mxs[mb * 16 + l16])), sgt);
+        }
+    };
+    // a tile with an infinity or a NaN: fp64 from the values; positions outside the tensor do not count (zero times infinity)
+    auto multiply_raw = [&](const int i) {
+        int n0, h0, w0;
+        place(i, n0, h0, w0);
+        const int *const tile = cells + (i & 1) * G::TILE_WORDS;
+        constexpr int SHARE = 4 * G::TH * G::TW / G::PW;
+        for (int pos = pw * SHARE; pos < (pw + 1) * SHARE; ++pos) {
+            const int k = pos % 4, c = pos / 4 % G::TW, r = pos / 4 / G::TW;
+            if (n0 + k >= N || h0 + r >= H || w0 + c >= W) continue;
+            const int *gp = tile + G::G0 + mb * 16 * G::GPLANE + k * G::GDIG + r * G::TW + c;
+            float xr[KS];
+#pragma unroll
+            for (int j = 0; j < KS; ++j) {
+                const int cc = c + j - PAD, hc = cc < 0 ? cc + PAD : cc - G::TW + PAD;
+                xr[j] = __int_as_float(tile[xch0 + k * G::XDIG + (cc >= 0 && cc < G::TW ? (r + ti) * G::TW + cc : G::XH + (r + ti) * G::HC + hc)]);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double gval = (double)__int_as_float(gp[(4 * lk + e) * G::GPLANE]);
+#pragma unroll
+                for (int j = 0; j < KS; ++j) tot[j][e] = fma((double)xr[j], gval, tot[j][e]);
+            }
+            if (sg_wave && lk == 0) sgt += (double)__int_as_float(gp[l16 * G::GPLANE]);
+        }
+    };
+
+    // While the multiplying waves work on tile i, the loading ones write the cells of tile i + 1, ask for tile i + 3 and note the
+    // largest values of tile i + 2, which has arrived meanwhile: one barrier a tile.  (Each kind of wave runs a loop of its own,
+    // with the same barriers, so that neither kind's registers are kept for the other's.)
+    if (loader) {
+        constexpr std::integral_constant<int, 0> even{};
+        constexpr std::integral_constant<int, SETS - 1> odd{};
+        fetch(0, even);
+        if (SETS == 2) fetch(1, odd);
+        note(0, even);
+        __syncthreads();
+        commit(0, even);
+        fetch(SETS, even);
+        note(1, odd);
+        __syncthreads();
+        auto turn = [&](const int i, auto next, auto after) __attribute__((always_inline)) {   // the sets that hold tiles i + 1 and i + 2
+            if (i + 1 < mine) commit(i + 1, next);
+            for (int e = lt; e < G::CH; e += G::LTHREADS) mx[((i + 3) & 3) * G::CH + e] = 0;
+            if (lt == 0) flags[(i + 3) & 3] = 0;
+            fetch(i + 1 + SETS, next);
+            if (i + 2 < mine) note(i + 2, after);
+            __syncthreads();
+        };
+        for (int i = 0; i < mine; i += 2) {   // (always both: a wait for one set must not have to allow for the turn left out)
+            turn(i, odd, even);
+            turn(i + 1, even, odd);
+        }
+    } else {
+        __syncthreads();
+        __syncthreads();
+        for (int i = 0; i < mine; ++i) {
+            if (__builtin_amdgcn_readfirstlane((int)flags[i & 3]) == 0) multiply(i);
+            else multiply_raw(i);
+            __syncthreads();
+        }
+        if (mine & 1) __syncthreads();
+    }
+
+    // ---- fold the waves that shared a tile's steps and put the block in the order of the slab, through LDS ----
+    double *const out = reinterpret_cast<double *>(cells), *const sgs = out + G::OUT;
+    sgt += __shfl_xor(sgt, 16, 64);   // the four lanes that held the channel's strips
+    sgt += __shfl_xor(sgt, 32, 64);
+    for (int p = 0; p < G::PW; ++p) {
+        if (!loader && pw == p) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                double *o = out + ((mb * 16 + 4 * lk + e) * G::CIB + nb * 16 + l16) * G::KK + ti * KS;
+#pragma unroll
+                for (int j = 0; j < KS; ++j) o[j] = p == 0 ? tot[j][e] : o[j] + tot[j][e];
+            }
+            if (ti == 0 && nb == 0 && lane < 16) sgs[mb * 16 + lane] = p == 0 ? sgt : sgs[mb * 16 + lane] + sgt;
+        }
+        __syncthreads();
+    }
+    const int K = Ci * G::KK, kcols = min(G::CIB, Ci - ci_blk) * G::KK;
+    double *dst = part + ((size_t)blockIdx.x * Co + co_blk) * K + (size_t)ci_blk * G::KK;
+    for (int c = 0; c < min(G::COB, Co - co_blk); ++c)
+        for (int k = tid; k < kcols; k += G::NTHREADS) dst[(size_t)c * K + k] = out[c * (G::CIB * G::KK) + k];
+    if (blockIdx.z == 0 && tid < min(G::COB, Co - co_blk)) sgpart[(size_t)blockIdx.x * Co + co_blk + tid] = sgs[tid];
+}
+
+// ---- host side ------------------------------------------------------------------
+// Channel blocks of 16 x 16 (two waves per tap row) and 32 x 16, tiles of 2 x 32, 4 x 16 and 8 x 8 positions of four images.
+//                       KS TH TW MB NB PW loading waves, waves per SIMD
+using Gi3a32 = GwI8Cfg<3, 2, 32, 1, 1, 2, 6, 3>;
+using Gi3a16 = GwI8Cfg<3, 4, 16, 1, 1, 2, 6, 3>;
+using Gi3a8  = GwI8Cfg<3, 8, 8, 1, 1, 2, 6, 3>;
+using Gi3b16 = GwI8Cfg<3, 4, 16, 2, 1, 1, 6, 3>;
+using Gi3b8  = GwI8Cfg<3, 8, 8, 2, 1, 1, 6, 3>;
+using Gi5w32 = GwI8Cfg<5, 2, 32, 1, 1, 1, 3, 2>;
+using Gi5w16 = GwI8Cfg<5, 4, 16, 1, 1, 1, 3, 2>;
+using Gi5w8  = GwI8Cfg<5, 8, 8, 1, 1, 1, 3, 2>;
+
+template <class G, bool VEC, class T, bool FUSE = false>
+static int launch_i8_v(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
+                       const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,
+                       const BnSums &sums = kNoBnSums) {
+    constexpr int LDS_BYTES = G::LDS_BYTES + (FUSE ? G::COB * 16 : 0);
+    if (int rc = allow_dynamic_lds<&grad_w_i8_kernel<G, VEC, T, FUSE>>(LDS_BYTES)) return rc;
+    hipLaunchKernelGGL((grad_w_i8_kernel<G, VEC, T, FUSE>), dim3(p.slots, p.gy, p.gz), dim3(G::NTHREADS), LDS_BYTES, s, gy, x, part, sgpart,
+                       d.N, d.Ci, d.H, d.W, d.Co, p.tilesH, p.tilesW, p.ntiles, bn_y, bn_coef, gy_out, sums);
+    return check_launch();
+}
+
+template <class G, class T>
+static int launch_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
+                     const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
+    if (bn_y) {
+        if constexpr (sizeof(T) == 4 && G::KS == 3) {
+            if (d.W % 4) return ADDER_ERR_UNSUPPORTED;
+            return launch_i8_v<G, true, T, true>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        }
+        return ADDER_ERR_UNSUPPORTED;
+    }
+    return d.W % 4 == 0 ? launch_i8_v<G, true, T>(gy, x, part, sgpart, d, p, s) : launch_i8_v<G, false, T>(gy, x, part, sgpart, d, p, s);
+}
+
+template <class G>
+static void plan_i8(const ConvDims &d, GradWMfmaPlan &p) {
+    p.tilesH = ceil_div(d.H, G::TH);
+    p.tilesW = ceil_div(d.W, G::TW);
+    p.ntiles = ceil_div(d.N, 4) * p.tilesH * p.tilesW;
+    p.gy = ceil_div(d.Co, G::COB);
+    p.gz = ceil_div(d.Ci, G::CIB);
+    p.slots = plan_grad_w_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)d.Co * d.Ci * G::KK + d.Co));
+}
+
+// Whether it takes a layer.  Against the fp64 matrix kernel it has some more to set up (half a workgroup's waves load, digits, four
+// images at a time), 1-2 us, and a fifth to a half of the matrix time; us, fp64 -> this, layers of 4..64 images:
+//   3x3, multiply-adds with the channels filled up to 16: 1.5e8 14.5 -> 16.1, 2.3e8 19.9 -> 19.6 and 18.6 -> 16.7, 3e8 29.1 -> 18.8,
+//   6e8 30.4 -> 21.6, 1.9e9 92.7 -> 42.4, 1.9e10 (128 -> 128 @32x32, 128 images) 690 -> 272;
+//   5x5: maps wider than 8, 7e6 24.1 -> 17.7 to 2.6e9 147 -> 59 (the fp64 kernel's 25-tap blocks start late); 8x8, 1e8 19.1 -> 19.2,
+//   2e8 22.4 -> 20.8, 4e8 30.8 -> 24.3.
+// Three channels on wide maps have a block of 32 columns there (stem, 256 images @32x32: 17 against 28).  Fewer than four images
+// would leave digits empty.
+bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
+    if (d.stride != 1 || d.kh != d.kw || d.pad != d.kh / 2 || d.N < 4 || (d.kh != 3 && d.kh != 5)) return false;
+    if ((long)d.Ci * d.H * d.W > kBufferImage || (long)d.Co * d.H * d.W > kBufferImage) return false;
+    if (d.kh == 3 && d.Ci * 9 <= 32 && d.W > 16) return false;
+    const double macs = (double)round_up(d.Ci, 16) * round_up(d.Co, 16) * d.kh * d.kw * d.N * d.H * d.W;
+    if (macs < (d.kh == 3 ? 2.2e8 : d.W > 8 ? 0.0 : 1.5e8)) return false;
+    // the tile that needs fewest; rows in one piece load whole lines and no halo columns, which is worth a seventh
+    const int n32 = ceil_div(d.H, 2) * ceil_div(d.W, 32), n16 = ceil_div(d.H, 4) * ceil_div(d.W, 16), n8 = ceil_div(d.H, 8) * ceil_div(d.W, 8);
+    const int shape = 7 * n32 <= 7 * n16 && 7 * n32 <= 8 * n8 ? 0 : 7 * n16 <= 8 * n8 ? 1 : 2;
+    if (d.kh == 3) {
+        p.variant = (d.Co > 16 ? 24 : 20) + shape;
+        switch (p.variant) {
+            case 20: plan_i8<Gi3a32>(d, p); break;
+            case 21: plan_i8<Gi3a16>(d, p); break;
+            case 22: plan_i8<Gi3a8>(d, p); break;
+            case 24: case 25: plan_i8<Gi3b16>(d, p); break;
+            default: plan_i8<Gi3b8>(d, p); break;
+        }
+        return true;
+    }
+    if (d.kh == 5) {
+        p.variant = 28 + shape;
+        if (shape == 0) plan_i8<Gi5w32>(d, p);
+        else if (shape == 1) plan_i8<Gi5w16>(d, p);
+        else plan_i8<Gi5w8>(d, p);
+        return true;
+    }
+    return false;
+}
+
+template <class T>
+int launch_grad_w_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
+                     const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
+    switch (p.variant) {
+        case 20: return launch_i8<Gi3a32>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 21: return launch_i8<Gi3a16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 22: return launch_i8<Gi3a8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 24: case 25: return launch_i8<Gi3b16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 26: return launch_i8<Gi3b8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 28: return launch_i8<Gi5w32>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 29: return launch_i8<Gi5w16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 30: return launch_i8<Gi5w8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        default: return ADDER_ERR_BAD_SHAPE;
+    }
+}
+template int launch_grad_w_i8<float>(const float *, const float *, double *, double *, const ConvDims &, const GradWMfmaPlan &, hipStream_t,
+                                     const float *, const float *, float *, const BnSums &);
+template int launch_grad_w_i8<bf16_t>(const bf16_t *, const bf16_t *, double *, double *, const ConvDims &, const GradWMfmaPlan &,
+                                      hipStream_t, const float *, const float *, float *, const BnSums &);
+
+}  // namespace adder

@@ -21,6 +21,7 @@
 // the (co, k) block of the workgroup; the waves are folded in fp64 through LDS at the end.
 // sum_pos gy is collected on the A fragments.  Partials: one fp64 (Co, K) slab per grid.x slot.
 #include "common.hpp"
+#include "grad_w_bn.hpp"
 #include "tile3x3.hpp"
 
 namespace adder {
@@ -132,51 +133,6 @@ __device__ __forceinline__ void gy_commit_m_bn(const GyStageM<G> &sg, const GySt
             *reinterpret_cast<float4 *>(buf + pc * G::GPLANE + r * G::TW + 4 * q) = v;
             if (gy_out && ok)
                 *reinterpret_cast<float4 *>(gy_out + ((((n0 + img) * Co + co0 + c) * Ho + h0 + r) * Wo + w0 + 4 * q)) = v;
-        }
-    }
-}
-
-// The four coefficients of gy_commit_m_bn for the workgroup's COB channels, from the sums the consumer's
-// input-gradient kernel left (BnSums): 32 lanes add the slots of one channel, always in the same order, so every
-// workgroup that needs a channel arrives at the same bits.  `write`: also store dgamma / dbeta of these channels
-// (one workgroup per channel block does).  Stands in for a launch of its own between the two kernels.
-template <class G>
-__device__ __forceinline__ void bn_coef_from_sums(const BnSums &b, int co0, int Co, float4 *coef, bool write) {
-    constexpr int GROUPS = G::NTHREADS / 32;
-    constexpr int CHUNK = 16;
-    const int sub = threadIdx.x & 31, grp = threadIdx.x >> 5;
-    for (int cb = 0; cb < G::COB; cb += GROUPS) {
-        const int c = cb + grp;
-        if (G::COB % GROUPS == 0 || c < G::COB) {
-            const int co = min(co0 + c, Co - 1);
-            const float rs = b.rstd[co], gm = b.gamma[co], mu = b.mean[co];
-            const float2 *p = reinterpret_cast<const float2 *>(b.part) + (size_t)co * b.slots;
-            double s1 = 0.0, s2 = 0.0;
-            for (int s0 = sub; s0 < b.slots; s0 += 32 * CHUNK) {   // CHUNK loads in flight, then added in slot order
-                float2 v[CHUNK];
-#pragma unroll
-                for (int j = 0; j < CHUNK; ++j) v[j] = p[min(s0 + 32 * j, b.slots - 1)];   // (unconditional: no waits between them)
-#pragma unroll
-                for (int j = 0; j < CHUNK; ++j) {
-                    const bool in = s0 + 32 * j < b.slots;
-                    s1 += in ? (double)v[j].x : 0.0;
-                    s2 += in ? (double)v[j].y : 0.0;
-                }
-            }
-#pragma unroll
-            for (int m = 16; m >= 1; m >>= 1) {   // (stays inside the 32-lane half)
-                s1 += __shfl_xor(s1, m, 64);
-                s2 += __shfl_xor(s2, m, 64);
-            }
-            if (sub == 0) {
-                const float m1 = (float)(s1 / b.count), m2 = (float)(s2 / b.count);
-                const float k = gm * rs;
-                coef[c] = make_float4(k, -k * rs * m2, mu, k * m1);
-                if (write && co0 + c < Co) {
-                    b.dbeta[co] = (float)s1;
-                    b.dgamma[co] = (float)s2;
-                }
-            }
         }
     }
 }
@@ -410,7 +366,7 @@ using Gm1x1c  = GwMfmaCfg<1, 1, 52, 1, 4, 2, 2, 4, 1, 1>;
 // rounded up leaves e.g. 22 x 12 = 264 workgroups, a second round for eight of them: 192 -> 192 3x3 @14x14, 32 images,
 // 205 -> 147 us without that round; 300 -> 300 1x1 @14x14, 64 images, 147 -> 94 us.)
 // More slabs than that quotient are taken only up to the scratch of the entry point without a workspace.
-static int plan_slots(int blocks, int ntiles, size_t slab_bytes) {
+int plan_grad_w_slots(int blocks, int ntiles, size_t slab_bytes) {
     const int quotient = ceil_div(256, blocks);
     int best = 1;
     long best_cost = -1;
@@ -433,7 +389,7 @@ static void plan_one(const ConvDims &d, GradWMfmaPlan &p) {
     p.ntiles = ceil_div(d.N, G::NIMG) * p.tilesH * p.tilesW;
     p.gy = ceil_div(d.Co, G::COB);
     p.gz = ceil_div(d.Ci * G::KK, G::KB);
-    p.slots = plan_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)d.Co * d.Ci * G::KK + d.Co));
+    p.slots = plan_grad_w_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)d.Co * d.Ci * G::KK + d.Co));
 }
 
 // a 1x1 layer seen as images of one row of Ho*Wo positions (the whole plane when the stride is 1)
@@ -447,6 +403,7 @@ static ConvDims mfma_one_row(const ConvDims &d) {
 
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d) {
     GradWMfmaPlan p{};
+    if (plan_grad_w_i8(d, p)) return p;
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci >= 64 && d.Co >= 64) {
         const ConvDims f = mfma_one_row(d);
         if (d.Ci >= 128 && d.Co >= 128) {
@@ -515,6 +472,7 @@ static int launch_one(const T *gy, const T *x, double *part, double *sgpart, con
 int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double *sgpart, const ConvDims &d,
                           const GradWMfmaPlan &p, const float *bn_y, const float *bn_coef, float *gy_out, hipStream_t s,
                           const BnSums &sums) {
+    if (p.variant >= 20) return launch_grad_w_i8(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
     const Subsample none{1, 0, 0, 0};
     if (((p.variant >= 1 && p.variant <= 5) || p.variant == 14) && (d.W % 4 != 0 || d.Wo % 4 != 0))
         return ADDER_ERR_UNSUPPORTED;
@@ -543,6 +501,7 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
 template <class T>
 int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p,
                        hipStream_t s) {
+    if (p.variant >= 20) return launch_grad_w_i8(gy, x, part, sgpart, d, p, s);
     switch (p.variant) {
         case 1: return launch_one<GmW32>(gy, x, part, sgpart, d, p, s);
         case 2: return launch_one<GmW16>(gy, x, part, sgpart, d, p, s);

@@ -1,0 +1,118 @@
+"""The weight gradient on the 8-bit matrix cores (csrc/grad_w_i8.hip): layers large enough for it, at the edges of its tiles.
+
+Bound: with e the unit of a channel's fixed point in a tile (2^-30 of its largest magnitude, within a factor of two) and 256 positions,
+the rounding of x costs at most 2^-31 max|x| * 16 ||gy||, i.e. 2^-27 ||x|| ||gy|| over the tile, that of gy the same, the digit products left
+out 2^-29 and the two roundings of digit sums 2^-28 each: below 2^-25 ||x_ci|| ||gy_co|| together, and over the tiles of a channel pair
+(Cauchy-Schwarz) against the norms of whole channels.  Plus the float32 rounding of the result."""
+import pytest
+import torch
+
+from oracle import c_oracle
+from tests import test_gpu_bn_links
+
+pytestmark = pytest.mark.gpu
+
+# (N, Ci, H, W, Co, k): every tile shape and block, images not a multiple of four, channels around multiples of 16 and 32, maps that end
+# inside a tile, rows that are whole groups of four and rows that are not
+CASES = [(4, 16, 128, 64, 33, 3), (5, 17, 100, 33, 47, 3), (11, 30, 160, 31, 15, 3), (6, 64, 65, 29, 40, 3), (15, 33, 67, 17, 40, 3), (17, 48, 15, 16, 144, 3),
+         (50, 80, 14, 14, 32, 3), (70, 130, 16, 12, 16, 3), (45, 79, 8, 8, 110, 3), (170, 90, 7, 7, 31, 3), (200, 60, 6, 5, 68, 3), (5, 16, 500, 40, 8, 3),
+         (4, 3, 9, 17, 5, 5), (5, 18, 12, 33, 20, 5), (6, 16, 21, 13, 40, 5), (9, 5, 10, 16, 16, 5), (46, 40, 8, 8, 40, 5), (101, 33, 7, 6, 31, 5)]
+
+
+def _on_the_digit_kernels(case):
+    """Its rule, so that a change of it does not leave this file testing another kernel."""
+    N, Ci, H, W, Co, k = case
+    macs = -(-Ci // 16) * -(-Co // 16) * 256 * k * k * N * H * W
+    return N >= 4 and macs >= (2.2e8 if k == 3 else 0 if W > 8 else 1.5e8)
+
+
+def _grad_w(gpu, x, w, gy, eta=0.0):
+    from addernetcuda_amd._lib import lib, check, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace
+    dims, _, _ = conv_dims(x.shape, w.shape, 1, w.shape[2] // 2)
+    ws, nbytes = conv2d_bwd_workspace(dims, gpu)
+    gw = torch.full(w.shape, float("nan"), device=gpu)
+    name = "adder_conv2d_bwd_f32" if x.dtype == torch.float32 else "adder_conv2d_bwd_bf16"
+    check(getattr(lib, name)(ptr(gy), ptr(x), ptr(w), None, ptr(gw), eta, ptr(ws), nbytes, *dims, stream_ptr(gpu)), name)
+    torch.cuda.synchronize()
+    return gw.cpu()
+
+
+def _data(case, seed):
+    N, Ci, H, W, Co, k = case
+    g = torch.Generator().manual_seed(seed)
+    return (torch.relu(torch.randn(N, Ci, H, W, generator=g)), torch.randn(Co, Ci, k, k, generator=g),
+            torch.randn(N, Co, H, W, generator=g) * 0.1)
+
+
+def _check(got, x, w, gy):
+    pad = w.shape[2] // 2
+    want = c_oracle.conv2d_grad_w(gy, x, w, 1, pad)
+    nx, ng = x.double().pow(2).sum((0, 2, 3)).sqrt(), gy.double().pow(2).sum((0, 2, 3)).sqrt()
+    total = (gy.double().sum((0, 2, 3))[:, None, None, None] * w.double()).abs()   # the term of w is rounded with the sum
+    bound = 2.0 ** -23 * want.abs() + 2.0 ** -25 * (ng[:, None] * nx[None, :])[:, :, None, None] + 2.0 ** -50 * total
+    err = (got.double() - want).abs()
+    assert bool((err <= bound).all()), f"worst element at {(err / bound).max().item():.2f} of the bound"
+
+
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_parity(gpu, case):
+    assert _on_the_digit_kernels(case)
+    x, w, gy = _data(case, 1)
+    got = _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu))
+    _check(got, x, w, gy)
+    assert torch.equal(got, _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)))
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[8], CASES[13]], ids=str)
+def test_bfloat16_storage(gpu, case):
+    x, w, gy = _data(case, 2)
+    x, gy = x.bfloat16(), gy.bfloat16()
+    _check(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), x.float(), w, gy.float())
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[9], CASES[15]], ids=str)
+def test_channels_of_very_different_size_and_long_tails(gpu, case):
+    x, w, gy = _data(case, 3)
+    g = torch.Generator().manual_seed(4)
+    x = x * torch.exp(2.0 * torch.randn(x.shape, generator=g)) * 10.0 ** (torch.rand(1, x.shape[1], 1, 1, generator=g) * 20 - 10)
+    gy = gy * torch.exp(2.0 * torch.randn(gy.shape, generator=g)) * 10.0 ** (torch.rand(1, gy.shape[1], 1, 1, generator=g) * 20 - 15)
+    x[:, 1] = 0.0
+    gy[:, 0] = 0.0
+    w = torch.zeros_like(w)   # (a sum of gy that is large against the products would hide them)
+    _check(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), x, w, gy)
+
+
+@pytest.mark.parametrize("case", [CASES[2], CASES[10], CASES[17]], ids=str)
+def test_whole_numbers_are_exact(gpu, case):
+    N, Ci, H, W, Co, k = case
+    g = torch.Generator().manual_seed(5)
+    x, w, gy = (torch.randint(-7, 8, s, generator=g).float() for s in ((N, Ci, H, W), (Co, Ci, k, k), (N, Co, H, W)))
+    assert torch.equal(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)).double(), c_oracle.conv2d_grad_w(gy, x, w, 1, k // 2).double())
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[6], CASES[14]], ids=str)
+def test_infinities_and_nan(gpu, case):
+    """One infinite x and one gy that is not a number: the same elements are infinite and not a number, the others within the bound."""
+    x, w, gy = _data(case, 6)
+    N, Ci, H, W, Co, k = case
+    x[N - 1, Ci - 1, H // 2, W - 2] = float("inf")
+    gy[0, 3, 1, 2] = float("nan")
+    got, want = _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)).double(), c_oracle.conv2d_grad_w(gy, x, w, 1, k // 2).double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+    x[N - 1, Ci - 1] = 0.0
+    gy[0, 3] = 0.0
+    keep = torch.ones_like(got, dtype=torch.bool)
+    keep[3], keep[:, Ci - 1] = False, False
+    clean = _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)).double()
+    fine = got[keep]
+    assert bool(fine.isfinite().all()) and bool(torch.isclose(fine, clean[keep], rtol=1e-6, atol=1e-5).all())
+
+
+# layers whose backward takes the BatchNorm links, large enough; the last: one tile for a workgroup, beside others'
+@pytest.mark.parametrize("case", [(26, 20, 32, 32, 30, 1), (64, 32, 16, 16, 48, 1), (104, 64, 8, 8, 64, 1)],
+                         ids=str)
+def test_linked_batchnorm(gpu, case):
+    N, Ci, H, W, Co, _ = case
+    assert _on_the_digit_kernels((N, Ci, H, W, Co, 3))
+    test_gpu_bn_links.test_fused_backward_matches_the_unfused_chain_in_float64(case, True, False, gpu)
