@@ -268,7 +268,7 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);   // 0: no statistics epilogue for these dimensions
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
-size_t grad_w_workspace_bytes(const ConvDims &d);
+size_t grad_w_workspace_bytes(const ConvDims &d, size_t limit = SIZE_MAX);
 // The sums of the backward of the BatchNorm behind a layer, as the consumer's input-gradient kernel left them
 // ((C, slots, 2) floats -- a wave's fp32 totals: sum dz, sum dz * xhat), with what turns them into the four coefficients per channel.
 // A weight-gradient kernel that is given these instead of ready coefficients adds the slots itself (every
@@ -284,7 +284,8 @@ static constexpr BnSums kNoBnSums{nullptr, 0, 0.0, nullptr, nullptr, nullptr, nu
 template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                   void *ws, size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y = nullptr,
-                  const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums);
+                  const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums,
+                  size_t limit = SIZE_MAX);   // limit, as given to grad_w_workspace_bytes: fewer slabs where they are too many for it
 // launch_grad_w without slabs (any layer): `ws` holds the norm partials only, kGradWGeneralWs bytes
 static constexpr size_t kGradWGeneralWs = 128 * 1024;
 template <class T>
@@ -301,6 +302,7 @@ int launch_bn_bwd_coef(const float *part, int slots, const float *gamma, const f
 // matrix-core weight gradient of the 3x3 / pad-1, 5x5 / pad-2 and wide 1x1 layers (grad_w_mfma.hip); variant 0 = not applicable
 struct GradWMfmaPlan { int variant, slots, gy, gz, tilesH, tilesW, ntiles; };
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d);
+GradWMfmaPlan plan_grad_w_fp64(const ConvDims &d);   // the same without the 8-bit kernels
 template <class T>
 int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p,
                        hipStream_t s);

@@ -343,10 +343,18 @@ struct GradWPlan {
     int slots;
 };
 
-static GradWPlan plan_grad_w(const ConvDims &d) {
+static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
+    size_t bytes = sizeof(double) * kNormBlocksMax;
+    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
+    if (p.variant)
+        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
+    return (bytes + 255) & ~(size_t)255;
+}
+
+static GradWPlan plan_of(const ConvDims &d, const GradWMfmaPlan &mfma) {
     GradWPlan p{};
     const long partial_cap = 1L << 28;  // partial slab elements
-    p.mfma = plan_grad_w_mfma(d);
+    p.mfma = mfma;
     if (p.mfma.variant) {
         p.variant = 2;
         p.slots = p.mfma.slots;
@@ -355,6 +363,22 @@ static GradWPlan plan_grad_w(const ConvDims &d) {
         p.slots = grad_w_1x1_slots(d);
     }
     if (p.variant && (long)p.slots * d.Co * d.K() > partial_cap) p.variant = 0;
+    return p;
+}
+
+// `limit`: the scratch of the entry point without a workspace.  The 8-bit kernels' larger blocks are fewer, so they take up to
+// twice the slabs to fill the chip; a layer whose slabs fit that scratch with the blocks of the other kernels runs here with as many
+// as fit (32 -> 32 3x3 @16x16, 256 images: 128 slabs, 9.6 MB, become 86).
+static GradWPlan plan_grad_w(const ConvDims &d, size_t limit = SIZE_MAX) {
+    GradWPlan p = plan_of(d, plan_grad_w_mfma(d));
+    if (p.variant == 2 && p.mfma.variant >= 20 && workspace_bytes_of(p, d) > limit) {
+        const GradWPlan other = plan_of(d, plan_grad_w_fp64(d));
+        if (workspace_bytes_of(other, d) > limit) return p;
+        const size_t slab = sizeof(double) * ((size_t)d.Co * d.K() + d.Co);
+        const int fit = (int)((limit - kGradWGeneralWs - 256) / slab);
+        if (fit < 1) return other;
+        p.slots = p.mfma.slots = ceil_div(p.mfma.ntiles, ceil_div(p.mfma.ntiles, fit));
+    }
     return p;
 }
 
@@ -369,14 +393,7 @@ bool grad_w_bn_supported(const ConvDims &d, const void *gy, const void *x, const
     return p.variant == 2 && (k3 || k1) && (align & 15) == 0;
 }
 
-static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
-    size_t bytes = sizeof(double) * kNormBlocksMax;
-    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
-    if (p.variant)
-        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
-    return (bytes + 255) & ~(size_t)255;
-}
-size_t grad_w_workspace_bytes(const ConvDims &d) { return workspace_bytes_of(plan_grad_w(d), d); }
+size_t grad_w_workspace_bytes(const ConvDims &d, size_t limit) { return workspace_bytes_of(plan_grad_w(d, limit), d); }
 
 // bn_y with either bn_coef or sums.part: gy is the gradient dz of the output of the BatchNorm behind the layer and
 // the kernel forms the layer's own output gradient from it, leaving it in gy_out (nullable) on the way (matrix-core
@@ -385,8 +402,8 @@ size_t grad_w_workspace_bytes(const ConvDims &d) { return workspace_bytes_of(pla
 template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws,
                   size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y, const float *bn_coef,
-                  float *gy_out, const BnSums &sums) {
-    GradWPlan p = plan_grad_w(d);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
+                  float *gy_out, const BnSums &sums, size_t limit) {
+    GradWPlan p = plan_grad_w(d, limit);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
     if (ws_bytes < workspace_bytes_of(p, d)) return ADDER_ERR_WORKSPACE;
     if (bn_y && (sizeof(T) != 4 ||
                  !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part)))
@@ -464,9 +481,9 @@ template int launch_grad_w_general<float>(const float *, const float *, const fl
 template int launch_grad_w_general<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *,
                                            const ConvDims &, hipStream_t);
 template int launch_grad_w<float>(const float *, const float *, const float *, float *, float, void *, size_t, const ConvDims &,
-                                  hipStream_t, const float *, const float *, float *, const BnSums &);
+                                  hipStream_t, const float *, const float *, float *, const BnSums &, size_t);
 template int launch_grad_w<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *, size_t,
-                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &);
+                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &, size_t);
 
 // ---- staged weight gradient: partial slabs now, finalize + scaling for many layers later --------------
 int launch_grad_w_staged(const float *gy, const float *x, const float *w, float *gw, float eta, void *ws,

@@ -403,7 +403,11 @@ static ConvDims mfma_one_row(const ConvDims &d) {
 
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d) {
     GradWMfmaPlan p{};
-    if (plan_grad_w_i8(d, p)) return p;
+    return plan_grad_w_i8(d, p) ? p : plan_grad_w_fp64(d);
+}
+
+GradWMfmaPlan plan_grad_w_fp64(const ConvDims &d) {
+    GradWMfmaPlan p{};
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci >= 64 && d.Co >= 64) {
         const ConvDims f = mfma_one_row(d);
         if (d.Ci >= 128 && d.Co >= 128) {

@@ -116,3 +116,17 @@ def test_linked_batchnorm(gpu, case):
     N, Ci, H, W, Co, _ = case
     assert _on_the_digit_kernels((N, Ci, H, W, Co, 3))
     test_gpu_bn_links.test_fused_backward_matches_the_unfused_chain_in_float64(case, True, False, gpu)
+
+
+# more slabs than the scratch of the entry point without a workspace holds: it takes as many as fit
+@pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5)], ids=str)
+def test_without_a_workspace(gpu, case):
+    from addernetcuda_amd._lib import lib, check, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace
+    assert _on_the_digit_kernels(case)
+    x, w, gy = _data(case, 7)
+    dims, _, _ = conv_dims(x.shape, w.shape, 1, case[5] // 2)
+    assert conv2d_bwd_workspace(dims, gpu)[1] > 8 << 20
+    xg, wg, gyg, gw = x.to(gpu), w.to(gpu), gy.to(gpu), torch.full(w.shape, float("nan"), device=gpu)
+    check(lib.adder_conv2d_bwd_noalloc_f32(ptr(gyg), ptr(xg), ptr(wg), None, ptr(gw), 0.0, *dims, stream_ptr(gpu)), "noalloc")
+    torch.cuda.synchronize()
+    _check(gw.cpu(), x, w, gy)
