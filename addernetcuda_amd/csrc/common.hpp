@@ -312,6 +312,9 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
 int plan_grad_w_slots(int blocks, int ntiles, size_t slab_bytes);
 // the same on the 8-bit matrix cores (grad_w_i8.hip): variants from 20 on; bn_y and the rest as in launch_grad_w
 bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p);
+bool plan_grad_w_i8_rows(int N, int Ci, int Co, long L, GradWMfmaPlan &p);   // single taps: N images of L positions
+int launch_grad_w_i8_rows(const float *gy, const float *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p,
+                          hipStream_t s);
 template <class T>
 int launch_grad_w_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
                      const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,

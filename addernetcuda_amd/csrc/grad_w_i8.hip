@@ -522,6 +522,323 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     if (blockIdx.z == 0 && tid < min(G::COB, Co - co_blk)) sgpart[(size_t)blockIdx.x * Co + co_blk + tid] = sgs[tid];
 }
 
+// ---------------------------------------------------------------------------
+// Single taps: gw[co,ci] = sum_pos x[ci,pos] gy[co,pos] over the positions of all planes in a row (so planes of any size fill the
+// tiles), and the column matrices' gW, whose rows are such planes.  The same fixed point and digits.  A tile is 128 positions; the four
+// digits that share a cell are 32 positions apart, so that a thread's four loads are each part of a 128-byte line that eight threads
+// read, and those eight threads hold a channel's tile: its largest value needs no exchange with other waves, and a thread converts a unit
+// as soon as it has arrived and asks for the same unit of the next tile.  Each multiplying wave owns 16 MT x 16 NT results.  A tile
+// with a value that is not finite is worked out in fp64 from memory.
+// ---------------------------------------------------------------------------
+template <int MT_, int NT_, int MB_, int NB_, int LWAVES_, int MINWAVES_>
+struct GwI8RowCfg {
+    static constexpr int MT = MT_, NT = NT_, MB = MB_, NB = NB_, LWAVES = LWAVES_, MINWAVES = MINWAVES_, TP = 128;
+    static constexpr int COB = 16 * MT * MB, CIB = 16 * NT * NB, ROWS = COB + CIB;
+    static constexpr int MWAVES = MB * NB, NTHREADS = 64 * (MWAVES + LWAVES), LTHREADS = 64 * LWAVES;
+    static constexpr int CELLS = TP / 4, PLANE = 4 * CELLS + 4;      // cells per digit, per channel (channels start four banks apart)
+    static constexpr int UNITS = ROWS * 8, ITER = ceil_div(UNITS, LTHREADS), STEPS = TP / 64;
+    static constexpr int TILE_WORDS = ROWS * PLANE, EX0 = 2 * TILE_WORDS, COEF0 = round_up(EX0 + 2 * ROWS + 4, 4), LDS_BYTES = COEF0 * 4;
+    static_assert(LDS_BYTES + COB * 16 <= 160 * 1024 && NTHREADS <= 1024 && LTHREADS % 8 == 0, "workgroup limits");
+};
+
+// P = N * L positions of N images with planes of L; VEC: planes are whole groups of four.  x and gy: (N, Ci, L) and (N, Co, L).
+template <class G, bool VEC = true, class T = float, bool FUSE = false>
+__global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel(const T *__restrict__ gy, const T *__restrict__ x,
+                                                                    double *__restrict__ part, double *__restrict__ sgpart, int N,
+                                                                    int Ci, int Co, int L, int ntiles, const float *__restrict__ bn_y,
+                                                                    const float *__restrict__ bn_coef, float *__restrict__ gy_out,
+                                                                    const BnSums sums) {
+    static_assert(!FUSE || (VEC && sizeof(T) == 4), "the BatchNorm link belongs to the float kernels");
+    constexpr int MT = G::MT, NT = G::NT;
+    constexpr unsigned E = sizeof(T);
+    extern __shared__ __align__(16) int cells[];
+    int *const ex = cells + G::EX0, *const flags = ex + 2 * G::ROWS;   // the channels' exponents of two tiles; a flag for each of four
+    float4 *const coef = reinterpret_cast<float4 *>(cells + G::COEF0);
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+    const int co_blk = blockIdx.y * G::COB, ci_blk = blockIdx.z * G::CIB;
+    float *const gy_dst = blockIdx.z == 0 ? gy_out : nullptr;
+    const long P = (long)N * L;
+    const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, tile0 = blockIdx.x * each, mine = min(each, ntiles - tile0);
+    const double rL = 1.0 / L;
+    // image and place in its plane of position p
+    auto place = [&](const long p, int &n, int &l) __attribute__((always_inline)) {
+        n = (int)((double)p * rL);
+        l = (int)(p - (long)n * L);
+        if (l < 0) { l += L; --n; }
+        if (l >= L) { l -= L; ++n; }
+    };
+    if constexpr (FUSE) {
+        if (sums.part) {
+            bn_coef_from_sums<G>(sums, co_blk, Co, coef, blockIdx.x == 0 && blockIdx.z == 0);
+        } else {
+            for (int e = tid; e < G::COB; e += G::NTHREADS) coef[e] = reinterpret_cast<const float4 *>(bn_coef)[min(co_blk + e, Co - 1)];
+        }
+    }
+    if (tid < 4) flags[tid] = 0;
+    __syncthreads();
+
+    double tot[MT][NT][4], sgt[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        sgt[m] = 0.0;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tot[m][n][e] = 0.0;
+    }
+    const int mb = wave % G::MB, nb = wave / G::MB % G::NB;
+    const bool sg_wave = nb == 0 && blockIdx.z == 0;
+
+    if (wave >= G::MWAVES) {
+        // ---- the loading waves: unit u = thread's channel row0 + it * (LTHREADS / 8), columns 4 * (u % 8) .. + 3 of each 32 ----
+        const int lt = tid - 64 * G::MWAVES, col = 4 * (lt & 7), row0 = lt >> 3;
+        float4 v[G::ITER][4], yv[FUSE ? G::ITER : 1][4];
+        // Offsets (bytes) of the thread's four groups from the first image of the tile that is being asked for, and of its channels; those
+        // that do not exist push the sum beyond every buffer, which ends below 2^31.
+        constexpr unsigned NO_GROUP = 0x80000000u, NO_ROW = 0x7fffffffu;
+        unsigned xoff[4], goff[4], rowoff[G::ITER];
+        int l[4], left[4], nlo = 0;
+        const int wrow0 = __builtin_amdgcn_readfirstlane(row0 & ~7);   // (a wave's eight rows are of one tensor)
+#pragma unroll
+        for (int it = 0; it < G::ITER; ++it) {
+            const int row = row0 + it * (G::LTHREADS / 8);
+            const bool is_x = row >= G::COB, ok = row < G::ROWS && (is_x ? ci_blk + row - G::COB < Ci : co_blk + row < Co);
+            rowoff[it] = ok ? (unsigned)((is_x ? ci_blk + row - G::COB : co_blk + row) * L) * E : NO_ROW;
+        }
+        auto aim = [&](const int i) __attribute__((always_inline)) {
+            const long base = (long)(tile0 + i) * G::TP;
+            int n, l0;
+            place(min(base, P - 1), nlo, l0);
+            nlo = __builtin_amdgcn_readfirstlane(nlo);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const long p = base + col + 32 * k;
+                place(p, n, l[k]);
+                left[k] = i < mine ? (int)max(min(P - p, 4L), 0L) : 0;
+                xoff[k] = left[k] ? (unsigned)((n - nlo) * Ci * L + l[k]) * E : NO_GROUP;
+                goff[k] = left[k] ? (unsigned)((n - nlo) * Co * L + l[k]) * E : NO_GROUP;
+            }
+        };
+        auto ask = [&](const int it) __attribute__((always_inline)) {
+            const bool is_x = wrow0 + it * (G::LTHREADS / 8) >= G::COB;
+            const int C = is_x ? Ci : Co;
+            auto one = [&](const T *t, float4 (&dst)[4]) __attribute__((always_inline)) {
+                const long rest = ((long)N - nlo) * C * L * (long)E;
+                const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(t + (size_t)nlo * C * L), 0,
+                                                                   (int)(rest < 0x7fffffffL ? rest : 0x7fffffffL), 0x00020000);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const unsigned off = (is_x ? xoff[k] : goff[k]) + rowoff[it];
+                    if constexpr (VEC) {
+                        dst[k] = i8_load4<true, T>(buf, off, 4);
+                    } else {   // a group may run on into the next image's plane
+                        float q[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            q[e] = i8_load1<T>(buf, e < left[k] ? off + e * E + (l[k] + e >= L ? (unsigned)(C - 1) * L * E : 0u) : kNowhere);
+                        dst[k] = make_float4(q[0], q[1], q[2], q[3]);
+                    }
+                }
+            };
+            one(is_x ? x : gy, v[it]);
+            if constexpr (FUSE) {
+                if (!is_x) one(bn_y, yv[it]);
+            }
+        };
+        static_assert(G::COB % 8 == 0, "eight rows of a wave are of one tensor");
+        auto turn = [&](const int i) __attribute__((always_inline)) {   // writes tile i, asks for tile i + 1
+            int *const tile = cells + (i & 1) * G::TILE_WORDS;
+            unsigned out_off[4];   // FUSE: where the tile's gy goes
+            const int out_n = nlo;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) out_off[k] = goff[k];
+            aim(i + 1);
+            if (tid == 64 * G::MWAVES) flags[(i + 2) & 3] = 0;
+#pragma unroll
+            for (int it = 0; it < G::ITER; ++it) {
+                const int row = row0 + it * (G::LTHREADS / 8);
+                const bool ok = G::UNITS % G::LTHREADS == 0 || row < G::ROWS;
+                if constexpr (FUSE) {
+                    if (row < G::COB) {
+                        const float4 cf = coef[row];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const bool in = rowoff[it] != NO_ROW && out_off[k] != NO_GROUP;
+                            const float4 g = v[it][k], y = yv[it][k];
+                            float4 r;
+                            r.x = in ? fmaf(cf.x, g.x, fmaf(cf.y, y.x - cf.z, -cf.w)) : 0.f;
+                            r.y = in ? fmaf(cf.x, g.y, fmaf(cf.y, y.y - cf.z, -cf.w)) : 0.f;
+                            r.z = in ? fmaf(cf.x, g.z, fmaf(cf.y, y.z - cf.z, -cf.w)) : 0.f;
+                            r.w = in ? fmaf(cf.x, g.w, fmaf(cf.y, y.w - cf.z, -cf.w)) : 0.f;
+                            v[it][k] = r;
+                            if (gy_dst && in)
+                                *reinterpret_cast<float4 *>(gy_dst + (size_t)out_n * Co * L + (out_off[k] + rowoff[it]) / E) = r;
+                        }
+                    }
+                }
+                float m = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) m = i8_absmax4(m, v[it][k]);
+                unsigned u = __float_as_uint(m) & 0x7fffffffu;   // over the eight lanes of the channel
+                u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
+                u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
+                u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x141, 0xF, 0xF, true));   // row_half_mirror
+                const int e = i8_exponent(u);
+                if (ok) {
+                    if ((lt & 7) == 0) {
+                        ex[(i & 1) * G::ROWS + row] = e;
+                        if (e >= 255) flags[i & 3] = 1;
+                    }
+                    i8_put4(v[it], i8_scale(min(e, 254)), false, tile + row * G::PLANE + col, G::CELLS);
+                }
+                ask(it);
+            }
+        };
+        aim(0);
+#pragma unroll
+        for (int it = 0; it < G::ITER; ++it) ask(it);
+        turn(0);
+        __syncthreads();
+        for (int i = 0; i < mine; ++i) {
+            if (i + 1 < mine) turn(i + 1);
+            __syncthreads();
+        }
+    } else {
+        // ---- the multiplying waves ----
+        const int goff = (mb * MT * 16 + l16) * G::PLANE + 4 * lk, xoff = (G::COB + nb * NT * 16 + l16) * G::PLANE + 4 * lk;
+        auto multiply = [&](const int i) __attribute__((always_inline)) {
+            const int *const tile = cells + (i & 1) * G::TILE_WORDS, *const exs = ex + (i & 1) * G::ROWS;
+            int4v acc[MT][NT][5], a[MT][4], b[2][NT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int s = 0; s < 5; ++s) acc[m][n][s] = s != 3 ? int4v{0, 0, 0, 0} : int4v{128, 128, 128, 128};
+            auto ask_a = [&](const int st, const int d) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    a[m][d] = *reinterpret_cast<const int4v *>(tile + goff + m * 16 * G::PLANE + d * G::CELLS + 16 * st);
+            };
+            auto ask_b = [&](const int p) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    b[p & 1][n] = *reinterpret_cast<const int4v *>(tile + xoff + n * 16 * G::PLANE + p % 4 * G::CELLS + 16 * (p / 4));
+            };
+            ask_b(0);
+            ask_a(0, 3);
+            ask_a(0, 2);
+#pragma unroll
+            for (int p = 0; p < 4 * G::STEPS; ++p) {   // (phases as in the kernel above)
+                const int dx = p % 4;
+                if (dx == 0) { ask_a(p / 4, 1); ask_a(p / 4, 0); }
+                if (p + 1 < 4 * G::STEPS) ask_b(p + 1);
+                if (dx == 3 && p + 1 < 4 * G::STEPS) { ask_a(p / 4 + 1, 3); ask_a(p / 4 + 1, 2); }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int dg = dx == 0 ? 3 : 4 - dx; dg >= 0; --dg)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+#pragma unroll
+                        for (int n = 0; n < NT; ++n)
+                            acc[m][n][dx + dg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m][dg], b[p & 1][n], acc[m][n][dx + dg], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            double sx[NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) sx[n] = i8_unit(exs[G::COB + (nb * NT + n) * 16 + l16]) * 4294967296.0;
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double sg = i8_unit(exs[(mb * MT + m) * 16 + 4 * lk + e]);
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        tot[m][n][e] = fma(i8_product(acc[m][n][0][e], acc[m][n][1][e], acc[m][n][2][e], acc[m][n][3][e], acc[m][n][4][e]),
+                                           sx[n] * sg, tot[m][n][e]);
+                }
+            if (sg_wave) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    int sd[4] = {0, 0, 0, 0};
+#pragma unroll
+                    for (int st = 0; st < G::STEPS; ++st)
+#pragma unroll
+                        for (int d = 0; d < 4; ++d) {
+                            const int4v g = *reinterpret_cast<const int4v *>(tile + goff + m * 16 * G::PLANE + d * G::CELLS + 16 * st);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) sd[d] = __builtin_amdgcn_sdot4(g[e], 0x01010101, sd[d], false);
+                        }
+                    sgt[m] = fma(i8_sum(sd[0], sd[1], sd[2], sd[3]), i8_unit(exs[(mb * MT + m) * 16 + l16]), sgt[m]);
+                }
+            }
+        };
+        auto multiply_from_memory = [&](const int i) {
+            for (int q = 0; q < G::TP; ++q) {
+                const long p = (long)(tile0 + i) * G::TP + q;
+                if (p >= P) break;
+                int n, l;
+                place(p, n, l);
+                auto value = [&](const T *t, const int C, const int ch) { return ch < C ? (double)ldf(t + ((size_t)n * C + ch) * L + l) : 0.0; };
+                auto grad = [&](const int r) {
+                    const double g = value(gy, Co, co_blk + r);
+                    if constexpr (FUSE) {
+                        const float4 cf = coef[r];
+                        if (co_blk + r < Co)
+                            return (double)fmaf(cf.x, (float)g, fmaf(cf.y, bn_y[((size_t)n * Co + co_blk + r) * L + l] - cf.z, -cf.w));
+                    }
+                    return g;
+                };
+#pragma unroll 1
+                for (int m = 0; m < MT; ++m) {
+#pragma unroll 1
+                    for (int e = 0; e < 4; ++e) {
+                        const double g = grad((mb * MT + m) * 16 + 4 * lk + e);
+#pragma unroll
+                        for (int mm = 0; mm < MT; ++mm)
+#pragma unroll
+                            for (int ee = 0; ee < 4; ++ee)
+#pragma unroll
+                                for (int c = 0; c < NT; ++c)
+                                    if (mm == m && ee == e) tot[mm][c][ee] = fma(value(x, Ci, ci_blk + (nb * NT + c) * 16 + l16), g, tot[mm][c][ee]);
+                    }
+                    if (sg_wave && lk == 0) {
+                        const double g = grad((mb * MT + m) * 16 + l16);
+#pragma unroll
+                        for (int mm = 0; mm < MT; ++mm)
+                            if (mm == m) sgt[mm] += g;
+                    }
+                }
+            }
+        };
+        __syncthreads();
+        for (int i = 0; i < mine; ++i) {
+            if (__builtin_amdgcn_readfirstlane(flags[i & 3]) == 0) multiply(i);
+            else multiply_from_memory(i);
+            __syncthreads();
+        }
+        // ---- straight to the slab: sixteen lanes hold sixteen columns in a row ----
+        double *dst = part + (size_t)blockIdx.x * Co * Ci;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int co = co_blk + (mb * MT + m) * 16 + 4 * lk + e;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    const int ci = ci_blk + (nb * NT + n) * 16 + l16;
+                    if (co < Co && ci < Ci) dst[(size_t)co * Ci + ci] = tot[m][n][e];
+                }
+            }
+            sgt[m] += __shfl_xor(sgt[m], 16, 64);   // the four lanes that held the channel's cells
+            sgt[m] += __shfl_xor(sgt[m], 32, 64);
+            const int co = co_blk + (mb * MT + m) * 16 + lane;
+            if (sg_wave && lane < 16 && co < Co) sgpart[(size_t)blockIdx.x * Co + co] = sgt[m];
+        }
+    }
+}
+
 // ---- host side ------------------------------------------------------------------
 // Channel blocks of 16 x 16 (two waves per tap row) and 32 x 16, tiles of 2 x 32, 4 x 16 and 8 x 8 positions of four images.
 //                       KS TH TW MB NB PW loading waves, waves per SIMD
@@ -533,6 +850,49 @@ using Gi3b8  = GwI8Cfg<3, 8, 8, 2, 1, 1, 6, 3>;
 using Gi5w32 = GwI8Cfg<5, 2, 32, 1, 1, 1, 3, 2>;
 using Gi5w16 = GwI8Cfg<5, 4, 16, 1, 1, 1, 3, 2>;
 using Gi5w8  = GwI8Cfg<5, 8, 8, 1, 1, 1, 3, 2>;
+
+// Single taps: 64 x 64 and, for few output channels, 32 x 96, each of 16 (14) waves on a CU of its own.  Whole calls with their
+// finalizing and scaling kernels, fp64 matrix cores -> this: 1024 -> 256 @14x14, 64 images 146 -> 82 us (bfloat16 storage 168 -> 88),
+// 128 -> 512 @28x28, 32 images 90 -> 48, 256 -> 64 @56x56, 64 images 148 -> 82, 512 -> 2048 @7x7, 64 images 177 -> 148; against the
+// plain kernel's fp32 runs 100 -> 48 @32x32 37 -> 23, 48 -> 200 72 -> 33.  Bound by the issue of both kinds of waves together: of the
+// first layer's 82 us the multiplying waves alone take 59, the loading waves alone 60, and without their loads both 80.
+//                           MT NT MB NB loading waves, waves per SIMD
+using GiRow  = GwI8RowCfg<2, 1, 2, 4, 8, 4>;
+using GiRowN = GwI8RowCfg<2, 1, 1, 6, 8, 4>;
+
+template <class G, bool VEC, class T, bool FUSE = false>
+static int launch_i8_row_v(const T *gy, const T *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p, hipStream_t s,
+                           const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,
+                           const BnSums &sums = kNoBnSums) {
+    constexpr int LDS_BYTES = G::LDS_BYTES + (FUSE ? G::COB * 16 : 0);
+    if (int rc = allow_dynamic_lds<&grad_w_i8_row_kernel<G, VEC, T, FUSE>>(LDS_BYTES)) return rc;
+    hipLaunchKernelGGL((grad_w_i8_row_kernel<G, VEC, T, FUSE>), dim3(p.slots, p.gy, p.gz), dim3(G::NTHREADS), LDS_BYTES, s, gy, x, part, sgpart,
+                       N, Ci, Co, L, p.ntiles, bn_y, bn_coef, gy_out, sums);
+    return check_launch();
+}
+
+template <class G, class T>
+static int launch_i8_row(const T *gy, const T *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p, hipStream_t s,
+                         const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
+    if (bn_y) {
+        if constexpr (sizeof(T) == 4 && G::COB == 64) {   // (linked layers have 64 channels and more)
+            if (L % 4) return ADDER_ERR_UNSUPPORTED;
+            return launch_i8_row_v<G, true, T, true>(gy, x, part, sgpart, N, Ci, Co, L, p, s, bn_y, bn_coef, gy_out, sums);
+        }
+        return ADDER_ERR_UNSUPPORTED;
+    }
+    return L % 4 == 0 && aligned_groups(x) && aligned_groups(gy)
+                      ? launch_i8_row_v<G, true, T>(gy, x, part, sgpart, N, Ci, Co, L, p, s)
+                      : launch_i8_row_v<G, false, T>(gy, x, part, sgpart, N, Ci, Co, L, p, s);
+}
+
+template <class G>
+static void plan_i8_row(int N, int Ci, int Co, int L, GradWMfmaPlan &p) {
+    p.ntiles = (int)ceil_div_l((long)N * L, G::TP);
+    p.gy = ceil_div(Co, G::COB);
+    p.gz = ceil_div(Ci, G::CIB);
+    p.slots = plan_grad_w_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)Co * Ci + Co));
+}
 
 template <class G, bool VEC, class T, bool FUSE = false>
 static int launch_i8_v(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
@@ -568,16 +928,43 @@ static void plan_i8(const ConvDims &d, GradWMfmaPlan &p) {
     p.slots = plan_grad_w_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)d.Co * d.Ci * G::KK + d.Co));
 }
 
+bool plan_grad_w_i8_rows(int N, int Ci, int Co, long L, GradWMfmaPlan &p) {
+    if (L < 4 || (128 + 2 * L) * (Ci > Co ? Ci : Co) > 2L * kBufferImage || N * L > 1L << 30) return false;   // 32-bit offsets from a tile's first image
+    p.variant = Co > 32 ? 32 : 33;
+    if (p.variant == 32) plan_i8_row<GiRow>(N, Ci, Co, (int)L, p);
+    else plan_i8_row<GiRowN>(N, Ci, Co, (int)L, p);
+    return true;
+}
+
+int launch_grad_w_i8_rows(const float *gy, const float *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p,
+                          hipStream_t s) {
+    return p.variant == 32 ? launch_i8_row<GiRow>(gy, x, part, sgpart, N, Ci, Co, L, p, s, nullptr, nullptr, nullptr, kNoBnSums)
+                           : launch_i8_row<GiRowN>(gy, x, part, sgpart, N, Ci, Co, L, p, s, nullptr, nullptr, nullptr, kNoBnSums);
+}
+
 // Whether it takes a layer.  Against the fp64 matrix kernel it has some more to set up (half a workgroup's waves load, digits, four
 // images at a time), 1-2 us, and a fifth to a half of the matrix time; us, fp64 -> this, layers of 4..64 images:
 //   3x3, multiply-adds with the channels filled up to 16: 1.5e8 14.5 -> 16.1, 2.3e8 19.9 -> 19.6 and 18.6 -> 16.7, 3e8 29.1 -> 18.8,
 //   6e8 30.4 -> 21.6, 1.9e9 92.7 -> 42.4, 1.9e10 (128 -> 128 @32x32, 128 images) 690 -> 272;
 //   5x5: maps wider than 8, 7e6 24.1 -> 17.7 to 2.6e9 147 -> 59 (the fp64 kernel's 25-tap blocks start late); 8x8, 1e8 19.1 -> 19.2,
 //   2e8 22.4 -> 20.8, 4e8 30.8 -> 24.3.
+//   1x1, from 64 channels on both sides: 64 -> 64 @8x8, 16 images 13.4 -> 11.6, 128 -> 128 @28x28, 16 images 31 -> 15, 256 -> 512 90 -> 44;
+//   fewer channels, planes of whole groups of four: 160 -> 48 @28x28, 16 images (9.6e7) 12.5 -> 14.0, 64 images (3.9e8) 48 -> 23,
+//   512 -> 32, 16 images (2.1e8) 23.3 -> 16.8, 1024 -> 16 (bfloat16) 48 -> 58; other planes (15x15): 48 -> 12, 2 images 11.6 -> 12.2,
+//   16 images 21.0 -> 13.2.
 // Three channels on wide maps have a block of 32 columns there (stem, 256 images @32x32: 17 against 28).  Fewer than four images
 // would leave digits empty.
 bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
-    if (d.stride != 1 || d.kh != d.kw || d.pad != d.kh / 2 || d.N < 4 || (d.kh != 3 && d.kh != 5)) return false;
+    if (d.stride != 1 || d.kh != d.kw || d.pad != d.kh / 2) return false;
+    if (d.kh == 1) {
+        // (the layers below 64 channels have a plain kernel beside this one, which reads planes that are not whole groups of four
+        // element by element; a block of fewer than 32 channels wastes more than the digits give)
+        const long L = (long)d.H * d.W;
+        const double macs = (double)round_up(d.Ci, 16) * round_up(d.Co, 16) * d.N * L;
+        if (!(d.Ci >= 64 && d.Co >= 64) && !(L % 4 && d.N * L >= 3000) && !(d.Ci >= 32 && d.Co >= 32 && macs >= 2.2e8)) return false;
+        return plan_grad_w_i8_rows(d.N, d.Ci, d.Co, L, p);
+    }
+    if (d.N < 4 || (d.kh != 3 && d.kh != 5)) return false;
     if ((long)d.Ci * d.H * d.W > kBufferImage || (long)d.Co * d.H * d.W > kBufferImage) return false;
     if (d.kh == 3 && d.Ci * 9 <= 32 && d.W > 16) return false;
     const double macs = (double)round_up(d.Ci, 16) * round_up(d.Co, 16) * d.kh * d.kw * d.N * d.H * d.W;
@@ -618,6 +1005,8 @@ int launch_grad_w_i8(const T *gy, const T *x, double *part, double *sgpart, cons
         case 28: return launch_i8<Gi5w32>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
         case 29: return launch_i8<Gi5w16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
         case 30: return launch_i8<Gi5w8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
+        case 32: return launch_i8_row<GiRow>(gy, x, part, sgpart, d.N, d.Ci, d.Co, d.H * d.W, p, s, bn_y, bn_coef, gy_out, sums);
+        case 33: return launch_i8_row<GiRowN>(gy, x, part, sgpart, d.N, d.Ci, d.Co, d.H * d.W, p, s, bn_y, bn_coef, gy_out, sums);
         default: return ADDER_ERR_BAD_SHAPE;
     }
 }

@@ -16,12 +16,17 @@ pytestmark = pytest.mark.gpu
 # inside a tile, rows that are whole groups of four and rows that are not
 CASES = [(4, 16, 128, 64, 33, 3), (5, 17, 100, 33, 47, 3), (11, 30, 160, 31, 15, 3), (6, 64, 65, 29, 40, 3), (15, 33, 67, 17, 40, 3), (17, 48, 15, 16, 144, 3),
          (50, 80, 14, 14, 32, 3), (70, 130, 16, 12, 16, 3), (45, 79, 8, 8, 110, 3), (170, 90, 7, 7, 31, 3), (200, 60, 6, 5, 68, 3), (5, 16, 500, 40, 8, 3),
-         (4, 3, 9, 17, 5, 5), (5, 18, 12, 33, 20, 5), (6, 16, 21, 13, 40, 5), (9, 5, 10, 16, 16, 5), (46, 40, 8, 8, 40, 5), (101, 33, 7, 6, 31, 5)]
+         (4, 3, 9, 17, 5, 5), (5, 18, 12, 33, 20, 5), (6, 16, 21, 13, 40, 5), (9, 5, 10, 16, 16, 5), (46, 40, 8, 8, 40, 5), (101, 33, 7, 6, 31, 5),
+         # single taps: tiles that end inside a plane and inside a group of four, planes smaller than a group of rows, both blocks
+         (1, 64, 2, 3, 64, 1), (3, 130, 7, 7, 70, 1), (2, 65, 14, 14, 129, 1), (14, 5, 15, 15, 7, 1), (11, 100, 17, 19, 33, 1), (30000, 33, 2, 2, 40, 1),
+         (120, 97, 15, 15, 31, 1), (90, 40, 40, 32, 47, 1), (130, 200, 32, 20, 32, 1), (5, 70, 1, 4, 300, 1)]
 
 
 def _on_the_digit_kernels(case):
     """Its rule, so that a change of it does not leave this file testing another kernel."""
     N, Ci, H, W, Co, k = case
+    if k == 1:
+        return min(Ci, Co) >= 64 or (H * W % 4 and N * H * W >= 3000) or (min(Ci, Co) >= 32 and -(-Ci // 16) * -(-Co // 16) * 256 * N * H * W >= 2.2e8)
     macs = -(-Ci // 16) * -(-Co // 16) * 256 * k * k * N * H * W
     return N >= 4 and macs >= (2.2e8 if k == 3 else 0 if W > 8 else 1.5e8)
 
@@ -63,14 +68,14 @@ def test_parity(gpu, case):
     assert torch.equal(got, _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)))
 
 
-@pytest.mark.parametrize("case", [CASES[1], CASES[8], CASES[13]], ids=str)
+@pytest.mark.parametrize("case", [CASES[1], CASES[8], CASES[13], CASES[19], CASES[22], CASES[26]], ids=str)
 def test_bfloat16_storage(gpu, case):
     x, w, gy = _data(case, 2)
     x, gy = x.bfloat16(), gy.bfloat16()
     _check(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), x.float(), w, gy.float())
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[9], CASES[15]], ids=str)
+@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[9], CASES[15], CASES[19], CASES[24]], ids=str)
 def test_channels_of_very_different_size_and_long_tails(gpu, case):
     x, w, gy = _data(case, 3)
     g = torch.Generator().manual_seed(4)
@@ -82,7 +87,7 @@ def test_channels_of_very_different_size_and_long_tails(gpu, case):
     _check(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), x, w, gy)
 
 
-@pytest.mark.parametrize("case", [CASES[2], CASES[10], CASES[17]], ids=str)
+@pytest.mark.parametrize("case", [CASES[2], CASES[10], CASES[17], CASES[20], CASES[25]], ids=str)
 def test_whole_numbers_are_exact(gpu, case):
     N, Ci, H, W, Co, k = case
     g = torch.Generator().manual_seed(5)
@@ -90,7 +95,7 @@ def test_whole_numbers_are_exact(gpu, case):
     assert torch.equal(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)).double(), c_oracle.conv2d_grad_w(gy, x, w, 1, k // 2).double())
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[6], CASES[14]], ids=str)
+@pytest.mark.parametrize("case", [CASES[0], CASES[6], CASES[14], CASES[19], CASES[25]], ids=str)
 def test_infinities_and_nan(gpu, case):
     """One infinite x and one gy that is not a number: the same elements are infinite and not a number, the others within the bound."""
     x, w, gy = _data(case, 6)
@@ -110,16 +115,15 @@ def test_infinities_and_nan(gpu, case):
 
 
 # layers whose backward takes the BatchNorm links, large enough; the last: one tile for a workgroup, beside others'
-@pytest.mark.parametrize("case", [(26, 20, 32, 32, 30, 1), (64, 32, 16, 16, 48, 1), (104, 64, 8, 8, 64, 1)],
+@pytest.mark.parametrize("case", [(26, 20, 32, 32, 30, 1), (64, 32, 16, 16, 48, 1), (104, 64, 8, 8, 64, 1), (30, 70, 14, 14, 136, 1, 1)],
                          ids=str)
 def test_linked_batchnorm(gpu, case):
-    N, Ci, H, W, Co, _ = case
-    assert _on_the_digit_kernels((N, Ci, H, W, Co, 3))
+    assert _on_the_digit_kernels((*case[:5], 1 if len(case) > 6 else 3))
     test_gpu_bn_links.test_fused_backward_matches_the_unfused_chain_in_float64(case, True, False, gpu)
 
 
 # more slabs than the scratch of the entry point without a workspace holds: it takes as many as fit
-@pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5)], ids=str)
+@pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5), (200, 63, 16, 16, 4096, 1)], ids=str)
 def test_without_a_workspace(gpu, case):
     from addernetcuda_amd._lib import lib, check, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace
     assert _on_the_digit_kernels(case)
@@ -130,3 +134,28 @@ def test_without_a_workspace(gpu, case):
     check(lib.adder_conv2d_bwd_noalloc_f32(ptr(gyg), ptr(xg), ptr(wg), None, ptr(gw), 0.0, *dims, stream_ptr(gpu)), "noalloc")
     torch.cuda.synchronize()
     _check(gw.cpu(), x, w, gy)
+
+
+@pytest.mark.parametrize("case", [CASES[20], CASES[25]], ids=str)
+def test_bases_between_the_groups(gpu, case):
+    """Tensors that begin one element into an allocation: the same results, element by element."""
+    x, w, gy = _data(case, 8)
+    off = lambda t: torch.cat([torch.zeros(1), t.flatten()]).to(gpu)[1:].view(t.shape)
+    assert torch.equal(_grad_w(gpu, off(x), w.to(gpu), off(gy)), _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)))
+
+
+# column matrices with long sums (Co, K, NL)
+@pytest.mark.parametrize("case", [(17, 33, 300004), (64, 576, 12100), (130, 100, 30000)], ids=str)
+def test_column_matrices(gpu, case):
+    from addernetcuda_amd import adder_cuda
+    Co, K, NL = case
+    assert -(-Co // 16) * -(-K // 16) * 256 * NL >= 2.2e8
+    x, w, gy = _data((1, K, 1, NL, Co, 1), 9)
+    X, G, Wm = x.view(K, NL).to(gpu), gy.view(Co, NL).to(gpu), w.view(Co, K).to(gpu)
+    gw = torch.full_like(Wm, 2.0)
+    adder_cuda.ADDER_CONV_WEIGHT(G, X, Wm, gw)
+    torch.cuda.synchronize()
+    want = c_oracle.col_grad_w(gy.view(Co, NL), x.view(K, NL), w.view(Co, K))
+    bound = 2.0 ** -23 * (want.abs() + 2.0) + 2.0 ** -25 * gy.view(Co, NL).double().norm(dim=1)[:, None] * x.view(K, NL).double().norm(dim=1)[None]
+    bound += 2.0 ** -50 * (gy.double().sum((0, 2, 3))[:, None] * w.view(Co, K).double()).abs()
+    assert bool(((gw.cpu().double() - 2.0 - want).abs() <= bound).all())
