@@ -1,4 +1,5 @@
-// Weight gradient of 3x3 / pad 1 and 5x5 / pad 2 layers of stride 1 on the 8-bit matrix cores, as exact as the fp64 ones.
+// Weight gradient of 3x3 / pad 1, 5x5 / pad 2 and 1x1 layers of stride 1, and of column matrices, on the 8-bit matrix cores, as exact
+// as the fp64 ones.  (First the kernel of the 3x3 and 5x5 layers, then that of the single taps.)
 //
 //   gw[co,ci,i,j] = sum_pos x[ci, pos + (i,j)] * gy[co,pos]  -  w[co,ci,i,j] * sum_pos gy[co,pos]
 //

@@ -1,4 +1,5 @@
-// Weight gradient of the AdderNet convolution (3x3 / pad 1, 5x5 / pad 2, or 1x1) on the matrix cores, in full precision.
+// Weight gradient of the AdderNet convolution (3x3 / pad 1, 5x5 / pad 2, or 1x1) on the matrix cores, in full precision: the layers
+// with a stride, the small ones and those of fewer than four images (the others: grad_w_i8.hip).
 //
 //   gw[co,k] = sum_pos xcol[k,pos] * gy[co,pos]  -  w[co,k] * sum_pos gy[co,pos]      (k = (ci, i, j))
 //
