@@ -392,9 +392,11 @@ __global__ __launch_bounds__(256) void col_bwd_fused_kernel(const float *__restr
 // gX[k, nl] += sum_co hardtanh(W[co,k] - X[k,nl]) * gy[co,nl], any number of output channels: a lane owns one column and
 // TK rows of X in registers; gy streams past PF output channels at a time with the next PF in flight, and the weights of
 // CB output channels sit in LDS as [co][TK] (two broadcast ds_read_b128 per 24 instructions).  Vector-issue-bound:
-// Co = 64, K = 576, NL = 16384 in 51 us, 12 T terms/s; 200, 300, 30000 in 156 us.  (Eight scalar weight loads and one load of
+// Co = 64, K = 576, NL = 16384 in 51 us, 12 T terms/s; 200, 300, 30000 in 152 us.  Full batches of gy run without a test between the
+// channels, so that their weight reads are under way together: 256, 128, 4096 32.2 -> 28.3 us, 250, 150, 8000 38.2 -> 36.2, 40, 70, 3000
+// 8.9 -> 8.2.  (Eight scalar weight loads and one load of
 // gy per output channel, each waited for: 139 and 381 us.  Two columns per lane: the same within 5 %, and slower
-// where it halves too few workgroups: 256, 128, 4096, 33 -> 47 us.)
+// where it halves too few workgroups.)
 static constexpr int kColGradXRows = 8;
 __global__ __launch_bounds__(256) void col_grad_x_kernel(const float *__restrict__ gy,
                                                          const float *__restrict__ X,
@@ -439,14 +441,20 @@ __global__ __launch_bounds__(256) void col_grad_x_kernel(const float *__restrict
 #pragma unroll
             for (int u = 0; u < PF; ++u) g[u] = nxt[u];
             if (cb + cc + PF < Co) fetch(cb + cc + PF);
-#pragma unroll
-            for (int u = 0; u < PF; ++u) {
-                if (cc + u >= cnt) break;
+            auto one_channel = [&](const int u) {
                 const float4 wa = *reinterpret_cast<const float4 *>(wl + (cc + u) * TK);
                 const float4 wb = *reinterpret_cast<const float4 *>(wl + (cc + u) * TK + 4);
                 const float wv[TK] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
 #pragma unroll
                 for (int t = 0; t < TK; ++t) acc[t] = fmaf(hardtanh(wv[t] - xv[t]), g[u], acc[t]);
+            };
+            if (cc + PF <= cnt) {
+#pragma unroll
+                for (int u = 0; u < PF; ++u) one_channel(u);
+            } else {
+#pragma unroll
+                for (int u = 0; u < PF; ++u)
+                    if (cc + u < cnt) one_channel(u);
             }
             if ((cc & 63) == 64 - PF) {
 #pragma unroll
