@@ -68,7 +68,7 @@ __device__ __forceinline__ void stage_weights(float *__restrict__ wt, const floa
 // rows of every block of X between them, so that the chain of dependent row batches is a quarter as long; their
 // partial sums are added through LDS at the end.
 template <int TM, int COLS, bool VEC, int PF, int KW>
-__global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restrict__ X,
+__global__ __launch_bounds__(256, COLS == 4 ? 2 : 1) void col_fwd_lds_kernel(const float *__restrict__ X,
                                                           const float *__restrict__ Wm,
                                                           float *__restrict__ out, int K, long NL, int Co, int KB) {
     static_assert(KW == 1 || KW == 4, "all waves on their own columns, or all four on the same");
@@ -158,6 +158,8 @@ __global__ __launch_bounds__(256) void col_fwd_lds_kernel(const float *__restric
                 float *dst = out + (size_t)(co0 + m) * NL + c0;
                 if constexpr (VEC && COLS == 2) {
                     *reinterpret_cast<float2 *>(dst) = make_float2(tot[m][0], tot[m][1]);
+                } else if constexpr (VEC && COLS == 4) {
+                    *reinterpret_cast<float4 *>(dst) = make_float4(tot[m][0], tot[m][1], tot[m][2], tot[m][3]);
                 } else {
 #pragma unroll
                     for (int e = 0; e < COLS; ++e)
@@ -826,6 +828,11 @@ static void launch_col_fwd_t(const float *X, const float *Wm, float *out, int K,
 // 29 -> 12; 64, 576, 32768, 79 -> 68; above the line 16, 144, 262144, 33 -> 37; 200, 300, 30000, 94 -> 99).  The split
 // kernels' tile shrinks with the number of workgroups: 16 x 128 while there are two per CU (256, 128, 4096: 10.7, with 8 x 128 10.8,
 // 8 x 64 14.3), 8 x 128 down to a quarter of that (32, 288, 16384: 18.1 -> 13.3), then 8 x 64 (32, 288, 4096: 17.9, 12.3, 9.9).
+// 16 x 256 where that is one round of workgroups, two per CU (its 256 registers a lane leave two waves per SIMD): a read of four weights
+// feeds 32 instructions instead of 16, and LDS reads, eight cycles each for four SIMDs, bounded the pairs of columns.  Those hold three
+// workgroups per CU, so up to 384 of the wide tiles they are one round, above they need two; us, 16 x 128 -> 16 x 256: 32, 288, 65536
+// (512 tiles) 40 -> 34, 64, 576, 32768 68 -> 56, 32, 288, 49664 (388) 38.5 -> 31.4, 128, 200, 12800 (400) 27 -> 23.5; with a few more
+// than 512 the wide tiles start a second round: 24, 600, 66000 (516) 81 -> 111, 48, 288, 65536 (768) 50 -> 58.
 int launch_col_fwd(const float *X, const float *Wm, float *out, int K, long NL, int Co, hipStream_t s) {
     const bool vec2 = NL % 2 == 0 && aligned8(X) && aligned8(out);
     const long tiles = ceil_div_l(NL, 128) * ceil_div(Co, 16);
@@ -833,7 +840,10 @@ int launch_col_fwd(const float *X, const float *Wm, float *out, int K, long NL, 
         if (vec2 && NL >= 65536) launch_col_fwd_t<16, 2, true, 8, 1>(X, Wm, out, K, NL, Co, s);
         else launch_col_fwd_t<16, 1, false, 8, 1>(X, Wm, out, K, NL, Co, s);
     } else if (tiles >= 512) {
-        if (vec2) launch_col_fwd_t<16, 2, true, 4, 4>(X, Wm, out, K, NL, Co, s);
+        const long wide = ceil_div_l(NL, 256) * ceil_div(Co, 16);
+        if (NL % 4 == 0 && wide > 384 && wide <= 512 && aligned16(X) && aligned16(out))
+            launch_col_fwd_t<16, 4, true, 2, 4>(X, Wm, out, K, NL, Co, s);
+        else if (vec2) launch_col_fwd_t<16, 2, true, 4, 4>(X, Wm, out, K, NL, Co, s);
         else launch_col_fwd_t<16, 1, false, 8, 4>(X, Wm, out, K, NL, Co, s);
     } else if (tiles >= 128 && vec2) {
         launch_col_fwd_t<8, 2, true, 8, 4>(X, Wm, out, K, NL, Co, s);

@@ -6,14 +6,16 @@ import torch
 pytestmark = pytest.mark.gpu
 
 # (Co, K, NL).  Forward: 512 workgroups of 512 columns and one fewer, even and odd NL; 512 and 128 tiles of 128 columns, and
-# one fewer; rows of X that do not divide by four waves or by a block of 256; fewer rows than waves.
+# one fewer; rows of X that do not divide by four waves or by a block of 256; fewer rows than waves; tiles of 256 columns: 512 and 386
+# of them, one row and two more, an NL that is no multiple of four.
 FORWARD = [(16, 37, 512 * 512), (16, 37, 511 * 512), (16, 20, 511 * 512 + 1), (16, 20, 511 * 512 - 1), (17, 259, 256 * 128),
            (17, 259, 255 * 128), (33, 513, 255 * 64 + 1), (16, 130, 128 * 128), (16, 130, 127 * 128), (20, 257, 16 * 1024),
-           (16, 3, 65536), (15, 1, 65538), (100, 2, 16386)]
+           (16, 3, 65536), (15, 1, 65538), (100, 2, 16386),
+           (32, 37, 65540), (20, 259, 65284), (17, 3, 65282), (32, 66, 49408), (32, 66, 49152), (33, 257, 43520), (32, 512, 49664)]
 # Input gradient: one output channel above 32, around the folds at 64 and the blocks of 512, rows of X around groups of
 # eight, columns around 256; grad_W: 9 blocks (504 workgroups), more than 512 blocks (one slab)
 BACKWARD = [(33, 8, 2049), (63, 9, 2303), (64, 7, 2304), (65, 17, 2305), (511, 8, 2052), (512, 11, 2053), (513, 8, 2052),
-            (521, 3, 2049), (1030, 9, 2051), (32, 288, 4096), (64, 576, 4100), (260, 2304, 2064)]
+            (521, 3, 2049), (1030, 9, 2051), (32, 37, 65540), (17, 9, 65537), (31, 66, 65538), (32, 288, 4096), (64, 576, 4100), (260, 2304, 2064)]
 
 
 def _data(Co, K, NL, gpu, seed):
@@ -34,6 +36,16 @@ def test_forward(case, gpu):
     # first-level sums of at most 64 terms, at most K / 64 + 4 of those: 2^-24 * (64 + K / 64 + 4) of the result
     bound = 2.0 ** -24 * (64 + case[1] / 64 + 4) * want[:, :-1].abs() + 1e-6
     assert ((out[:, :-1].double() - want[:, :-1]).abs() <= bound).all()
+
+
+def test_forward_of_bases_between_the_groups(gpu):
+    """Tensors that begin two elements into an allocation take tiles of pairs: the same sums in the same order."""
+    from addernetcuda_amd import adder_cuda
+    X, W, _ = _data(32, 66, 49664, gpu, 6)
+    out, off = torch.empty(32, 49664, device=gpu), torch.empty(32 * 49664 + 2, device=gpu)[2:].view(32, 49664)
+    adder_cuda.ADDER_CONV(X, W, out)
+    adder_cuda.ADDER_CONV(torch.cat([X.new_zeros(2), X.flatten()])[2:].view(66, 49664), W, off)
+    assert torch.equal(out, off)
 
 
 # one matrix per forward tile: unsplit by pairs and by single columns, split 16 x 128, 16 x 64, 8 x 128 and 8 x 64
