@@ -491,7 +491,7 @@ def plain_conv2d_forward(X, W, stride, padding):
 
 def conv2d_weight_grad(grad_out, X, W, stride, padding, out_link=None):
     """Weight gradient of an *ordinary* convolution ``F.conv2d(X, W, None, stride, padding)``, i.e. the
-    ``sum x * gy`` half of the adder layer's weight gradient, from the same matrix-core kernels (the slab
+    ``sum x * gy`` half of the adder layer's weight gradient, from the same fp64 matrix-core kernel (the slab
     finalize leaves the ``- w * sum gy`` term out).  Inside a ``batched_eta_scaling()`` block it is finished
     together with the adder layers' gradients.  Returns None where the geometry has no such kernel.
     ``out_link``: a BnLink that ``claims`` grad_out -- ``grad_out`` is then dz of the BatchNorm behind the

@@ -854,20 +854,12 @@ int launch_col_fwd(const float *X, const float *Wm, float *out, int K, long NL, 
 }
 
 // ---- weight gradient: slab plan -------------------------------------------------------------------------
-struct ColGwPlan { int ct, kt, slots, gy, gz; bool mfma, digits; GradWMfmaPlan rows; };
+struct ColGwPlan { int ct, kt, slots, gy, gz; bool mfma; };
 
 static ColGwPlan plan_col_grad_w(int K, long NL, int Co) {
     ColGwPlan p{};
     p.mfma = NL % 4 == 0 && NL >= 16;
     if (!p.mfma) return p;
-    // long sums on the 8-bit matrix cores, as those of a 1x1 layer with one image of NL positions (fp64 -> digits, us: Co 64, K 576,
-    // NL 8192 21.1 -> 17.6, 64, 576, 32768 56 -> 36, 128, 1152, 4096 36 -> 24; 32, 288, 8192 12.4 -> 12.0; 8, 100, 100000 20 -> 27)
-    const double macs = (double)round_up(K, 16) * round_up(Co, 16) * NL;
-    p.digits = macs >= 2.2e8 && K >= 32 && Co > 16 && plan_grad_w_i8_rows(1, K, Co, NL, p.rows);
-    if (p.digits) {
-        p.slots = p.rows.slots;
-        return p;
-    }
     // accumulator tiles per wave: one row of up to five for layers with up to 16 output channels (X is read once,
     // gy once per block of 80 rows of X), else 2 x 4 or 2 x 2 / 3 x 1: enough to amortise the operand loads, few
     // enough for two waves per SIMD (nine tiles were slower: one wave per SIMD, or spills)
@@ -933,10 +925,6 @@ int launch_col_grad_w(const float *gy, const float *X, const float *Wm, float *g
     if (p.mfma && ws && aligned16(X) && aligned16(gy) && (reinterpret_cast<uintptr_t>(ws) & 255) == 0) {
         double *part = reinterpret_cast<double *>(ws);
         double *sgpart = part + (size_t)p.slots * Co * K;
-        if (p.digits) {
-            if (int rc = launch_grad_w_i8_rows(gy, X, part, sgpart, 1, K, Co, (int)NL, p.rows, s)) return rc;
-            return launch_grad_w_slab_finalize(part, sgpart, Wm, gW, p.slots, Co, K, /*accumulate=*/add, s);
-        }
         const int tag = p.ct * 16 + p.kt;
         switch (tag) {
             case 1 * 16 + 1: launch_col_gw<1, 1>(gy, X, part, sgpart, K, NL, Co, p, s); break;

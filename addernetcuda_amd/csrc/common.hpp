@@ -268,7 +268,7 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);   // 0: no statistics epilogue for these dimensions
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
-size_t grad_w_workspace_bytes(const ConvDims &d, size_t limit = SIZE_MAX);
+size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false);   // of the storage type's kernels
 // The sums of the backward of the BatchNorm behind a layer, as the consumer's input-gradient kernel left them
 // ((C, slots, 2) floats -- a wave's fp32 totals: sum dz, sum dz * xhat), with what turns them into the four coefficients per channel.
 // A weight-gradient kernel that is given these instead of ready coefficients adds the slots itself (every
@@ -284,8 +284,7 @@ static constexpr BnSums kNoBnSums{nullptr, 0, 0.0, nullptr, nullptr, nullptr, nu
 template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                   void *ws, size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y = nullptr,
-                  const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums,
-                  size_t limit = SIZE_MAX);   // limit, as given to grad_w_workspace_bytes: fewer slabs where they are too many for it
+                  const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums);
 // launch_grad_w without slabs (any layer): `ws` holds the norm partials only, kGradWGeneralWs bytes
 static constexpr size_t kGradWGeneralWs = 128 * 1024;
 template <class T>
@@ -302,7 +301,6 @@ int launch_bn_bwd_coef(const float *part, int slots, const float *gamma, const f
 // matrix-core weight gradient of the 3x3 / pad-1, 5x5 / pad-2 and wide 1x1 layers (grad_w_mfma.hip); variant 0 = not applicable
 struct GradWMfmaPlan { int variant, slots, gy, gz, tilesH, tilesW, ntiles; };
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d);
-GradWMfmaPlan plan_grad_w_fp64(const ConvDims &d);   // the same without the 8-bit kernels
 template <class T>
 int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p,
                        hipStream_t s);
@@ -310,15 +308,9 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
                           const GradWMfmaPlan &p, const float *bn_y, const float *bn_coef, float *gy_out, hipStream_t s,
                           const BnSums &sums = kNoBnSums);
 int plan_grad_w_slots(int blocks, int ntiles, size_t slab_bytes);
-// the same on the 8-bit matrix cores (grad_w_i8.hip): variants from 20 on; bn_y and the rest as in launch_grad_w
+// large layers in bfloat16 storage, on the 8-bit matrix cores (grad_w_i8.hip): variants from 20 on
 bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p);
-bool plan_grad_w_i8_rows(int N, int Ci, int Co, long L, GradWMfmaPlan &p);   // single taps: N images of L positions
-int launch_grad_w_i8_rows(const float *gy, const float *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p,
-                          hipStream_t s);
-template <class T>
-int launch_grad_w_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
-                     const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,
-                     const BnSums &sums = kNoBnSums);
+int launch_grad_w_i8(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s);
 
 // 1x1 / pad 0 / stride 1-2 kernels (conv1x1.hip)
 bool conv1x1_supported(const ConvDims &d, const void *a, const void *b);

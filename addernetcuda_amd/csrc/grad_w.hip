@@ -343,18 +343,11 @@ struct GradWPlan {
     int slots;
 };
 
-static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
-    size_t bytes = sizeof(double) * kNormBlocksMax;
-    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
-    if (p.variant)
-        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
-    return (bytes + 255) & ~(size_t)255;
-}
-
-static GradWPlan plan_of(const ConvDims &d, const GradWMfmaPlan &mfma) {
+// `bf16`: large layers in bfloat16 storage have kernels of their own (grad_w_i8.hip)
+static GradWPlan plan_grad_w(const ConvDims &d, bool bf16 = false) {
     GradWPlan p{};
     const long partial_cap = 1L << 28;  // partial slab elements
-    p.mfma = mfma;
+    if (!(bf16 && plan_grad_w_i8(d, p.mfma))) p.mfma = plan_grad_w_mfma(d);
     if (p.mfma.variant) {
         p.variant = 2;
         p.slots = p.mfma.slots;
@@ -366,34 +359,25 @@ static GradWPlan plan_of(const ConvDims &d, const GradWMfmaPlan &mfma) {
     return p;
 }
 
-// `limit`: the scratch of the entry point without a workspace.  The 8-bit kernels' larger blocks are fewer, so they take up to
-// twice the slabs to fill the chip; a layer whose slabs fit that scratch with the blocks of the other kernels runs here with as many
-// as fit (32 -> 32 3x3 @16x16, 256 images: 128 slabs, 9.6 MB, become 86).
-static GradWPlan plan_grad_w(const ConvDims &d, size_t limit = SIZE_MAX) {
-    GradWPlan p = plan_of(d, plan_grad_w_mfma(d));
-    if (p.variant == 2 && p.mfma.variant >= 20 && workspace_bytes_of(p, d) > limit) {
-        const GradWPlan other = plan_of(d, plan_grad_w_fp64(d));
-        if (workspace_bytes_of(other, d) > limit) return p;
-        const size_t slab = sizeof(double) * ((size_t)d.Co * d.K() + d.Co);
-        const int fit = (int)((limit - kGradWGeneralWs - 256) / slab);
-        if (fit < 1) return other;
-        p.slots = p.mfma.slots = ceil_div(p.mfma.ntiles, ceil_div(p.mfma.ntiles, fit));
-    }
-    return p;
-}
-
 // whether launch_grad_w / launch_grad_w_staged take the BatchNorm link for this layer and these tensors
 bool grad_w_bn_supported(const ConvDims &d, const void *gy, const void *x, const void *bn_y, const void *bn_coef) {
     const GradWPlan p = plan_grad_w(d);
     const uintptr_t align = reinterpret_cast<uintptr_t>(gy) | reinterpret_cast<uintptr_t>(x) |
                             reinterpret_cast<uintptr_t>(bn_y) | reinterpret_cast<uintptr_t>(bn_coef);
     const int v = p.mfma.variant;
-    const bool k3 = ((v >= 1 && v <= 5) || v == 14 || (v >= 20 && v < 28)) && d.W % 4 == 0 && d.Wo % 4 == 0;
-    const bool k1 = (v == 6 || v == 7 || v == 10 || v == 12 || v == 32) && d.Ci >= 64 && d.Co >= 64 && d.stride == 1 && (d.H * d.W) % 4 == 0;
+    const bool k3 = ((v >= 1 && v <= 5) || v == 14) && d.W % 4 == 0 && d.Wo % 4 == 0;
+    const bool k1 = (v == 6 || v == 7 || v == 10 || v == 12) && d.stride == 1 && (d.H * d.W) % 4 == 0;
     return p.variant == 2 && (k3 || k1) && (align & 15) == 0;
 }
 
-size_t grad_w_workspace_bytes(const ConvDims &d, size_t limit) { return workspace_bytes_of(plan_grad_w(d, limit), d); }
+static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
+    size_t bytes = sizeof(double) * kNormBlocksMax;
+    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
+    if (p.variant)
+        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
+    return (bytes + 255) & ~(size_t)255;
+}
+size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16) { return workspace_bytes_of(plan_grad_w(d, bf16), d); }
 
 // bn_y with either bn_coef or sums.part: gy is the gradient dz of the output of the BatchNorm behind the layer and
 // the kernel forms the layer's own output gradient from it, leaving it in gy_out (nullable) on the way (matrix-core
@@ -402,8 +386,8 @@ size_t grad_w_workspace_bytes(const ConvDims &d, size_t limit) { return workspac
 template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws,
                   size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y, const float *bn_coef,
-                  float *gy_out, const BnSums &sums, size_t limit) {
-    GradWPlan p = plan_grad_w(d, limit);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
+                  float *gy_out, const BnSums &sums) {
+    GradWPlan p = plan_grad_w(d, sizeof(T) != 4);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
     if (ws_bytes < workspace_bytes_of(p, d)) return ADDER_ERR_WORKSPACE;
     if (bn_y && (sizeof(T) != 4 ||
                  !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part)))
@@ -437,7 +421,8 @@ int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                 rc = bn_y ? launch_grad_w_mfma_bn(gy, x, part, sgpart, d, p.mfma, bn_y, bn_coef, gy_out, s, sums)
                           : launch_grad_w_mfma(gy, x, part, sgpart, d, p.mfma, s);
             else
-                rc = launch_grad_w_mfma(gy, x, part, sgpart, d, p.mfma, s);
+                rc = p.mfma.variant >= 20 ? launch_grad_w_i8(gy, x, part, sgpart, d, p.mfma, s)
+                                          : launch_grad_w_mfma(gy, x, part, sgpart, d, p.mfma, s);
             if (rc) return rc;
             hipLaunchKernelGGL(grad_w_finalize_kernel<double>, dim3(nb), dim3(kFinOut * kFinLanes), 0, s, part,
                                sgpart, w, gw, fused_norm ? ss : nullptr, p.slots, d.Co, K);
@@ -482,9 +467,9 @@ template int launch_grad_w_general<float>(const float *, const float *, const fl
 template int launch_grad_w_general<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *,
                                            const ConvDims &, hipStream_t);
 template int launch_grad_w<float>(const float *, const float *, const float *, float *, float, void *, size_t, const ConvDims &,
-                                  hipStream_t, const float *, const float *, float *, const BnSums &, size_t);
+                                  hipStream_t, const float *, const float *, float *, const BnSums &);
 template int launch_grad_w<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *, size_t,
-                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &, size_t);
+                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &);
 
 // ---- staged weight gradient: partial slabs now, finalize + scaling for many layers later --------------
 int launch_grad_w_staged(const float *gy, const float *x, const float *w, float *gw, float eta, void *ws,
@@ -495,9 +480,8 @@ int launch_grad_w_staged(const float *gy, const float *x, const float *w, float 
     if (bn_y && !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part))
         return ADDER_ERR_UNSUPPORTED;
     const bool rows_1x1 = p.variant == 2 && d.kh == 1;
-    const bool any_base = p.variant == 2 && p.mfma.variant >= 32;
-    const bool need_x16 = p.variant == 2 && !any_base && !(rows_1x1 && d.stride > 1) && (rows_1x1 ? d.H * d.W : d.W) % 4 == 0;
-    const bool need_g16 = p.variant == 2 && !any_base && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
+    const bool need_x16 = p.variant == 2 && !(rows_1x1 && d.stride > 1) && (rows_1x1 ? d.H * d.W : d.W) % 4 == 0;
+    const bool need_g16 = p.variant == 2 && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
     if (!p.variant || (need_x16 && (reinterpret_cast<uintptr_t>(x) & 15)) ||
         (need_g16 && (reinterpret_cast<uintptr_t>(gy) & 15)))
         return ADDER_ERR_UNSUPPORTED;   // no slab-based kernel for this layer: nothing to stage

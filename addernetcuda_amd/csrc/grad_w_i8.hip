@@ -25,7 +25,6 @@
 // instructions of 16 cycles per step with the operand moves between them; without the loading waves' work it takes 252 us, without the
 // multiplying waves' 175.  (All waves doing both in turn: 605; loads that branch, so that every wait is for all of them: 300.)
 #include "common.hpp"
-#include "grad_w_bn.hpp"
 
 #include <type_traits>
 
@@ -56,36 +55,27 @@ struct GwI8Cfg {
     static constexpr int LDS_BYTES = COEF0 * 4;
     static_assert(TW % 8 == 0 && 4 % STRIPS == 0 && TH * STRIPS % (4 * PW) == 0 && KS % 2 == 1, "whole steps of four strips");
     static_assert((XR * QW) % 4 == 0 && (XR * HC) % 4 == 0 && (TH * QW) % 4 == 0, "four units in a row share a channel");
-    static_assert(LDS_BYTES + COB * 16 <= 160 * 1024 && NTHREADS <= 1024, "workgroup limits");
+    static_assert(LDS_BYTES <= 160 * 1024 && NTHREADS <= 1024, "workgroup limits");
     static_assert(2 * (OUT + COB) <= 2 * TILE_WORDS, "the results fit the cells' place");
     static_assert(XDIG % 4 == 0 && XH % 4 == 0 && GPLANE % 4 == 0 && COEF0 % 4 == 0, "16-byte alignment of the cells");
 };
 
 // Four images of a tensor as a buffer: loads from beyond its end (images that do not exist) or at kNowhere give zeros, so they need no
 // branch -- with loads under way in two register sets, a wait has to know how many are newer.
-typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 static constexpr unsigned kNowhere = 0x80000000u;
 static constexpr int kBufferImage = 1 << 27;   // elements per image: four of float fill 2^31 bytes, and kNowhere + three does not wrap
-template <class T>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t i8_images(const T *base, int image, int n0, int N) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(base + (size_t)n0 * image), 0, min(4, N - n0) * image * (int)sizeof(T), 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t i8_images(const bf16_t *base, int image, int n0, int N) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(base + (size_t)n0 * image), 0, min(4, N - n0) * image * (int)sizeof(bf16_t), 0x00020000);
 }
-template <class T>
-__device__ __forceinline__ float i8_load1(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    if constexpr (sizeof(T) == 4) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-    else return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
-}
+__device__ __forceinline__ float i8_load1(__amdgpu_buffer_rsrc_t r, unsigned off) { return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0)); }
 // four consecutive elements of a row, `left` elements before its end (VEC: rows are whole groups of four)
-template <bool VEC, class T>
+template <bool VEC>
 __device__ __forceinline__ float4 i8_load4(__amdgpu_buffer_rsrc_t r, unsigned off, int left) {
     if constexpr (!VEC) {
-        constexpr unsigned E = sizeof(T);
-        return make_float4(i8_load1<T>(r, off), i8_load1<T>(r, left > 1 ? off + E : kNowhere), i8_load1<T>(r, left > 2 ? off + 2 * E : kNowhere),
-                           i8_load1<T>(r, left > 3 ? off + 3 * E : kNowhere));
-    } else if constexpr (sizeof(T) == 4) {
-        const uint4v u = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-        return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
+        constexpr unsigned E = sizeof(bf16_t);
+        return make_float4(i8_load1(r, off), i8_load1(r, left > 1 ? off + E : kNowhere), i8_load1(r, left > 2 ? off + 2 * E : kNowhere),
+                           i8_load1(r, left > 3 ? off + 3 * E : kNowhere));
     } else {
         const uint2v u = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
         return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
@@ -160,18 +150,14 @@ __device__ __forceinline__ double i8_sum(int a0, int a1, int a2, int a3) {
     return fma((double)((a0 << 8) + a1), 65536.0, (double)((a2 << 8) + a3));
 }
 
-template <class G, bool VEC = true, class T = float, bool FUSE = false>
-__global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(const T *__restrict__ gy, const T *__restrict__ x,
+template <class G, bool VEC>
+__global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(const bf16_t *__restrict__ gy, const bf16_t *__restrict__ x,
                                                                 double *__restrict__ part, double *__restrict__ sgpart, int N,
-                                                                int Ci, int H, int W, int Co, int tilesH, int tilesW, int ntiles,
-                                                                const float *__restrict__ bn_y, const float *__restrict__ bn_coef,
-                                                                float *__restrict__ gy_out, const BnSums sums) {
-    static_assert(!FUSE || (VEC && sizeof(T) == 4), "the BatchNorm link belongs to the float kernels");
+                                                                int Ci, int H, int W, int Co, int tilesH, int tilesW, int ntiles) {
     constexpr int KS = G::KS, PAD = G::PAD, QW = G::QW, SQ = 2;   // SQ: groups of four columns in a strip
     extern __shared__ __align__(16) int cells[];   // two tiles: x cells, gy cells
     unsigned *const mx = reinterpret_cast<unsigned *>(cells + G::MX0);   // largest magnitudes of four tiles, then four flags
     unsigned *const flags = mx + 4 * G::CH;
-    float4 *const coef = reinterpret_cast<float4 *>(cells + G::COEF0);
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
     const bool loader = wave >= G::MWAVES;
@@ -179,17 +165,9 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     // a multiplying wave's accumulators (tap row, block of 16 output channels, of 16 input channels) and its share of a tile's steps
     const int ti = wave % KS, pw = wave / KS % G::PW, mb = wave / KS / G::PW % G::MB, nb = wave / KS / G::PW / G::MB;
     const int co_blk = blockIdx.y * G::COB, ci_blk = blockIdx.z * G::CIB;
-    float *const gy_dst = blockIdx.z == 0 ? gy_out : nullptr;   // every gy tile is staged once per block of input channels
     // the workgroup's tiles lie side by side: the lines that neighbouring tiles share stay in one L2
     const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, tile0 = blockIdx.x * each, mine = min(each, ntiles - tile0);
 
-    if constexpr (FUSE) {   // the block's BatchNorm coefficients
-        if (sums.part) {
-            bn_coef_from_sums<G>(sums, co_blk, Co, coef, blockIdx.x == 0 && blockIdx.z == 0);
-        } else {
-            for (int e = tid; e < G::COB; e += G::NTHREADS) coef[e] = reinterpret_cast<const float4 *>(bn_coef)[min(co_blk + e, Co - 1)];
-        }
-    }
     for (int e = tid; e < 4 * G::CH + 4; e += G::NTHREADS) mx[e] = 0;
     __syncthreads();
 
@@ -215,7 +193,7 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     // Two tiles under way in registers; one, where a thread has two gy units: the multiplying waves last longer than a load there, and
     // a second set would spill (128 -> 128 @32x32, 128 images, 275 us with two, 272 with one).
     constexpr int SETS = KS == 3 && G::GITER > 1 ? 1 : 2;
-    float4 xv[SETS][G::XITER][4], gv[SETS][G::GITER][4], yv[SETS][FUSE ? G::GITER : 1][4];
+    float4 xv[SETS][G::XITER][4], gv[SETS][G::GITER][4];
     float hv[SETS][G::HITER][4];
     auto place = [&](const int i, int &n0, int &h0, int &w0) {
         int t = tile0 + i;
@@ -227,7 +205,7 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     // tile i of the workgroup (nothing, if it has none) into register set b
     auto fetch = [&](const int i, auto set) __attribute__((always_inline)) {
         constexpr int b = decltype(set)::value;
-        constexpr unsigned E = sizeof(T);
+        constexpr unsigned E = sizeof(bf16_t);
         int n0, h0, w0;
         place(min(i, mine - 1), n0, h0, w0);
         const auto gbuf = i8_images(gy, gimg, n0, N), xbuf = i8_images(x, ximg, n0, N);
@@ -237,12 +215,7 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
             const bool ok = i < mine && (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB) && ch < Co && ho < H && wo < W;
             const unsigned off = ok ? ((ch * H + ho) * W + wo) * E : kNowhere;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) gv[b][it][k] = i8_load4<VEC, T>(gbuf, off + k * gimg * E, W - wo);
-            if constexpr (FUSE) {
-                const auto ybuf = i8_images(bn_y, gimg, n0, N);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) yv[b][it][k] = i8_load4<true, float>(ybuf, off + k * gimg * E, W - wo);
-            }
+            for (int k = 0; k < 4; ++k) gv[b][it][k] = i8_load4<VEC>(gbuf, off + k * gimg * E, W - wo);
         }
 #pragma unroll
         for (int it = 0; it < G::XITER; ++it) {
@@ -250,7 +223,7 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
             const bool ok = i < mine && (G::XUNITS % G::LTHREADS == 0 || xch[it] < G::CIB) && ch < Ci && hi >= 0 && hi < H && wi < W;
             const unsigned off = ok ? ((ch * H + hi) * W + wi) * E : kNowhere;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) xv[b][it][k] = i8_load4<VEC, T>(xbuf, off + k * ximg * E, W - wi);
+            for (int k = 0; k < 4; ++k) xv[b][it][k] = i8_load4<VEC>(xbuf, off + k * ximg * E, W - wi);
         }
 #pragma unroll
         for (int it = 0; it < G::HITER; ++it) {
@@ -258,35 +231,13 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
             const bool ok = i < mine && (G::HUNITS % G::LTHREADS == 0 || hch[it] < G::CIB) && ch < Ci && hi >= 0 && hi < H && wi >= 0 && wi < W;
             const unsigned off = ok ? ((ch * H + hi) * W + wi) * E : kNowhere;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) hv[b][it][k] = i8_load1<T>(xbuf, off + k * ximg * E);
+            for (int k = 0; k < 4; ++k) hv[b][it][k] = i8_load1(xbuf, off + k * ximg * E);
         }
     };
-    // the largest magnitudes of the channels of tile i, which is in set b (FUSE: its gy is formed first)
+    // the largest magnitudes of the channels of tile i, which is in set b
     auto note = [&](const int i, auto set) __attribute__((always_inline)) {
         constexpr int b = decltype(set)::value;
         unsigned *const mxs = mx + (i & 3) * G::CH, *const flag = flags + (i & 3);
-        if constexpr (FUSE) {
-            int n0, h0, w0;
-            place(i, n0, h0, w0);
-#pragma unroll
-            for (int it = 0; it < G::GITER; ++it) {
-                const int ch = co_blk + gch[it], ho = h0 + grow[it], wo = w0 + gcol[it];
-                const bool ok = i < mine && (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB) && ch < Co && ho < H && wo < W;
-                const float4 cf = coef[min(gch[it], G::COB - 1)];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const bool in = ok && n0 + k < N;   // (rows are whole groups of four)
-                    const float4 g = gv[b][it][k], y = yv[b][it][k];
-                    float4 v;
-                    v.x = in ? fmaf(cf.x, g.x, fmaf(cf.y, y.x - cf.z, -cf.w)) : 0.f;
-                    v.y = in ? fmaf(cf.x, g.y, fmaf(cf.y, y.y - cf.z, -cf.w)) : 0.f;
-                    v.z = in ? fmaf(cf.x, g.z, fmaf(cf.y, y.z - cf.z, -cf.w)) : 0.f;
-                    v.w = in ? fmaf(cf.x, g.w, fmaf(cf.y, y.w - cf.z, -cf.w)) : 0.f;
-                    gv[b][it][k] = v;
-                    if (gy_dst && in) *reinterpret_cast<float4 *>(gy_dst + ((n0 + k) * gimg + (ch * H + ho) * W + wo)) = v;
-                }
-            }
-        }
 #pragma unroll
         for (int it = 0; it < G::GITER; ++it) {
             const bool ok = G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB;
@@ -539,26 +490,21 @@ struct GwI8RowCfg {
     static constexpr int CELLS = TP / 4, PLANE = 4 * CELLS + 4;      // cells per digit, per channel (channels start four banks apart)
     static constexpr int UNITS = ROWS * 8, ITER = ceil_div(UNITS, LTHREADS), STEPS = TP / 64;
     static constexpr int TILE_WORDS = ROWS * PLANE, EX0 = 2 * TILE_WORDS, COEF0 = round_up(EX0 + 2 * ROWS + 4, 4), LDS_BYTES = COEF0 * 4;
-    static_assert(LDS_BYTES + COB * 16 <= 160 * 1024 && NTHREADS <= 1024 && LTHREADS % 8 == 0, "workgroup limits");
+    static_assert(LDS_BYTES <= 160 * 1024 && NTHREADS <= 1024 && LTHREADS % 8 == 0, "workgroup limits");
 };
 
 // P = N * L positions of N images with planes of L; VEC: planes are whole groups of four.  x and gy: (N, Ci, L) and (N, Co, L).
-template <class G, bool VEC = true, class T = float, bool FUSE = false>
-__global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel(const T *__restrict__ gy, const T *__restrict__ x,
+template <class G, bool VEC>
+__global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel(const bf16_t *__restrict__ gy, const bf16_t *__restrict__ x,
                                                                     double *__restrict__ part, double *__restrict__ sgpart, int N,
-                                                                    int Ci, int Co, int L, int ntiles, const float *__restrict__ bn_y,
-                                                                    const float *__restrict__ bn_coef, float *__restrict__ gy_out,
-                                                                    const BnSums sums) {
-    static_assert(!FUSE || (VEC && sizeof(T) == 4), "the BatchNorm link belongs to the float kernels");
+                                                                    int Ci, int Co, int L, int ntiles) {
     constexpr int MT = G::MT, NT = G::NT;
-    constexpr unsigned E = sizeof(T);
+    constexpr unsigned E = sizeof(bf16_t);
     extern __shared__ __align__(16) int cells[];
     int *const ex = cells + G::EX0, *const flags = ex + 2 * G::ROWS;   // the channels' exponents of two tiles; a flag for each of four
-    float4 *const coef = reinterpret_cast<float4 *>(cells + G::COEF0);
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
     const int co_blk = blockIdx.y * G::COB, ci_blk = blockIdx.z * G::CIB;
-    float *const gy_dst = blockIdx.z == 0 ? gy_out : nullptr;
     const long P = (long)N * L;
     const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, tile0 = blockIdx.x * each, mine = min(each, ntiles - tile0);
     const double rL = 1.0 / L;
@@ -569,13 +515,6 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
         if (l < 0) { l += L; --n; }
         if (l >= L) { l -= L; ++n; }
     };
-    if constexpr (FUSE) {
-        if (sums.part) {
-            bn_coef_from_sums<G>(sums, co_blk, Co, coef, blockIdx.x == 0 && blockIdx.z == 0);
-        } else {
-            for (int e = tid; e < G::COB; e += G::NTHREADS) coef[e] = reinterpret_cast<const float4 *>(bn_coef)[min(co_blk + e, Co - 1)];
-        }
-    }
     if (tid < 4) flags[tid] = 0;
     __syncthreads();
 
@@ -594,7 +533,7 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
     if (wave >= G::MWAVES) {
         // ---- the loading waves: unit u = thread's channel row0 + it * (LTHREADS / 8), columns 4 * (u % 8) .. + 3 of each 32 ----
         const int lt = tid - 64 * G::MWAVES, col = 4 * (lt & 7), row0 = lt >> 3;
-        float4 v[G::ITER][4], yv[FUSE ? G::ITER : 1][4];
+        float4 v[G::ITER][4];
         // Offsets (bytes) of the thread's four groups from the first image of the tile that is being asked for, and of its channels; those
         // that do not exist push the sum beyond every buffer, which ends below 2^31.
         constexpr unsigned NO_GROUP = 0x80000000u, NO_ROW = 0x7fffffffu;
@@ -624,60 +563,35 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
         auto ask = [&](const int it) __attribute__((always_inline)) {
             const bool is_x = wrow0 + it * (G::LTHREADS / 8) >= G::COB;
             const int C = is_x ? Ci : Co;
-            auto one = [&](const T *t, float4 (&dst)[4]) __attribute__((always_inline)) {
+            auto one = [&](const bf16_t *t, float4 (&dst)[4]) __attribute__((always_inline)) {
                 const long rest = ((long)N - nlo) * C * L * (long)E;
-                const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(t + (size_t)nlo * C * L), 0,
+                const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(t + (size_t)nlo * C * L), 0,
                                                                    (int)(rest < 0x7fffffffL ? rest : 0x7fffffffL), 0x00020000);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const unsigned off = (is_x ? xoff[k] : goff[k]) + rowoff[it];
                     if constexpr (VEC) {
-                        dst[k] = i8_load4<true, T>(buf, off, 4);
+                        dst[k] = i8_load4<true>(buf, off, 4);
                     } else {   // a group may run on into the next image's plane
                         float q[4];
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            q[e] = i8_load1<T>(buf, e < left[k] ? off + e * E + (l[k] + e >= L ? (unsigned)(C - 1) * L * E : 0u) : kNowhere);
+                            q[e] = i8_load1(buf, e < left[k] ? off + e * E + (l[k] + e >= L ? (unsigned)(C - 1) * L * E : 0u) : kNowhere);
                         dst[k] = make_float4(q[0], q[1], q[2], q[3]);
                     }
                 }
             };
             one(is_x ? x : gy, v[it]);
-            if constexpr (FUSE) {
-                if (!is_x) one(bn_y, yv[it]);
-            }
         };
         static_assert(G::COB % 8 == 0, "eight rows of a wave are of one tensor");
         auto turn = [&](const int i) __attribute__((always_inline)) {   // writes tile i, asks for tile i + 1
             int *const tile = cells + (i & 1) * G::TILE_WORDS;
-            unsigned out_off[4];   // FUSE: where the tile's gy goes
-            const int out_n = nlo;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) out_off[k] = goff[k];
             aim(i + 1);
             if (tid == 64 * G::MWAVES) flags[(i + 2) & 3] = 0;
 #pragma unroll
             for (int it = 0; it < G::ITER; ++it) {
                 const int row = row0 + it * (G::LTHREADS / 8);
                 const bool ok = G::UNITS % G::LTHREADS == 0 || row < G::ROWS;
-                if constexpr (FUSE) {
-                    if (row < G::COB) {
-                        const float4 cf = coef[row];
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            const bool in = rowoff[it] != NO_ROW && out_off[k] != NO_GROUP;
-                            const float4 g = v[it][k], y = yv[it][k];
-                            float4 r;
-                            r.x = in ? fmaf(cf.x, g.x, fmaf(cf.y, y.x - cf.z, -cf.w)) : 0.f;
-                            r.y = in ? fmaf(cf.x, g.y, fmaf(cf.y, y.y - cf.z, -cf.w)) : 0.f;
-                            r.z = in ? fmaf(cf.x, g.z, fmaf(cf.y, y.z - cf.z, -cf.w)) : 0.f;
-                            r.w = in ? fmaf(cf.x, g.w, fmaf(cf.y, y.w - cf.z, -cf.w)) : 0.f;
-                            v[it][k] = r;
-                            if (gy_dst && in)
-                                *reinterpret_cast<float4 *>(gy_dst + (size_t)out_n * Co * L + (out_off[k] + rowoff[it]) / E) = r;
-                        }
-                    }
-                }
                 float m = 0.f;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) m = i8_absmax4(m, v[it][k]);
@@ -781,14 +695,9 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
                 if (p >= P) break;
                 int n, l;
                 place(p, n, l);
-                auto value = [&](const T *t, const int C, const int ch) { return ch < C ? (double)ldf(t + ((size_t)n * C + ch) * L + l) : 0.0; };
+                auto value = [&](const bf16_t *t, const int C, const int ch) { return ch < C ? (double)ldf(t + ((size_t)n * C + ch) * L + l) : 0.0; };
                 auto grad = [&](const int r) {
                     const double g = value(gy, Co, co_blk + r);
-                    if constexpr (FUSE) {
-                        const float4 cf = coef[r];
-                        if (co_blk + r < Co)
-                            return (double)fmaf(cf.x, (float)g, fmaf(cf.y, bn_y[((size_t)n * Co + co_blk + r) * L + l] - cf.z, -cf.w));
-                    }
                     return g;
                 };
 #pragma unroll 1
@@ -861,30 +770,18 @@ using Gi5w8  = GwI8Cfg<5, 8, 8, 1, 1, 1, 3, 2>;
 using GiRow  = GwI8RowCfg<2, 1, 2, 4, 8, 4>;
 using GiRowN = GwI8RowCfg<2, 1, 1, 6, 8, 4>;
 
-template <class G, bool VEC, class T, bool FUSE = false>
-static int launch_i8_row_v(const T *gy, const T *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p, hipStream_t s,
-                           const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,
-                           const BnSums &sums = kNoBnSums) {
-    constexpr int LDS_BYTES = G::LDS_BYTES + (FUSE ? G::COB * 16 : 0);
-    if (int rc = allow_dynamic_lds<&grad_w_i8_row_kernel<G, VEC, T, FUSE>>(LDS_BYTES)) return rc;
-    hipLaunchKernelGGL((grad_w_i8_row_kernel<G, VEC, T, FUSE>), dim3(p.slots, p.gy, p.gz), dim3(G::NTHREADS), LDS_BYTES, s, gy, x, part, sgpart,
-                       N, Ci, Co, L, p.ntiles, bn_y, bn_coef, gy_out, sums);
+template <class G, bool VEC>
+static int launch_i8_row_v(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s) {
+    if (int rc = allow_dynamic_lds<&grad_w_i8_row_kernel<G, VEC>>(G::LDS_BYTES)) return rc;
+    hipLaunchKernelGGL((grad_w_i8_row_kernel<G, VEC>), dim3(p.slots, p.gy, p.gz), dim3(G::NTHREADS), G::LDS_BYTES, s, gy, x, part, sgpart, d.N, d.Ci, d.Co,
+                       d.H * d.W, p.ntiles);
     return check_launch();
 }
 
-template <class G, class T>
-static int launch_i8_row(const T *gy, const T *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p, hipStream_t s,
-                         const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
-    if (bn_y) {
-        if constexpr (sizeof(T) == 4 && G::COB == 64) {   // (linked layers have 64 channels and more)
-            if (L % 4) return ADDER_ERR_UNSUPPORTED;
-            return launch_i8_row_v<G, true, T, true>(gy, x, part, sgpart, N, Ci, Co, L, p, s, bn_y, bn_coef, gy_out, sums);
-        }
-        return ADDER_ERR_UNSUPPORTED;
-    }
-    return L % 4 == 0 && aligned_groups(x) && aligned_groups(gy)
-                      ? launch_i8_row_v<G, true, T>(gy, x, part, sgpart, N, Ci, Co, L, p, s)
-                      : launch_i8_row_v<G, false, T>(gy, x, part, sgpart, N, Ci, Co, L, p, s);
+template <class G>
+static int launch_i8_row(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s) {
+    return d.H * d.W % 4 == 0 && aligned_groups(x) && aligned_groups(gy) ? launch_i8_row_v<G, true>(gy, x, part, sgpart, d, p, s)
+                                                                        : launch_i8_row_v<G, false>(gy, x, part, sgpart, d, p, s);
 }
 
 template <class G>
@@ -895,28 +792,17 @@ static void plan_i8_row(int N, int Ci, int Co, int L, GradWMfmaPlan &p) {
     p.slots = plan_grad_w_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)Co * Ci + Co));
 }
 
-template <class G, bool VEC, class T, bool FUSE = false>
-static int launch_i8_v(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
-                       const float *bn_y = nullptr, const float *bn_coef = nullptr, float *gy_out = nullptr,
-                       const BnSums &sums = kNoBnSums) {
-    constexpr int LDS_BYTES = G::LDS_BYTES + (FUSE ? G::COB * 16 : 0);
-    if (int rc = allow_dynamic_lds<&grad_w_i8_kernel<G, VEC, T, FUSE>>(LDS_BYTES)) return rc;
-    hipLaunchKernelGGL((grad_w_i8_kernel<G, VEC, T, FUSE>), dim3(p.slots, p.gy, p.gz), dim3(G::NTHREADS), LDS_BYTES, s, gy, x, part, sgpart,
-                       d.N, d.Ci, d.H, d.W, d.Co, p.tilesH, p.tilesW, p.ntiles, bn_y, bn_coef, gy_out, sums);
+template <class G, bool VEC>
+static int launch_i8_v(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s) {
+    if (int rc = allow_dynamic_lds<&grad_w_i8_kernel<G, VEC>>(G::LDS_BYTES)) return rc;
+    hipLaunchKernelGGL((grad_w_i8_kernel<G, VEC>), dim3(p.slots, p.gy, p.gz), dim3(G::NTHREADS), G::LDS_BYTES, s, gy, x, part, sgpart, d.N, d.Ci, d.H, d.W,
+                       d.Co, p.tilesH, p.tilesW, p.ntiles);
     return check_launch();
 }
 
-template <class G, class T>
-static int launch_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
-                     const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
-    if (bn_y) {
-        if constexpr (sizeof(T) == 4 && G::KS == 3) {
-            if (d.W % 4) return ADDER_ERR_UNSUPPORTED;
-            return launch_i8_v<G, true, T, true>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        }
-        return ADDER_ERR_UNSUPPORTED;
-    }
-    return d.W % 4 == 0 ? launch_i8_v<G, true, T>(gy, x, part, sgpart, d, p, s) : launch_i8_v<G, false, T>(gy, x, part, sgpart, d, p, s);
+template <class G>
+static int launch_i8(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s) {
+    return d.W % 4 == 0 ? launch_i8_v<G, true>(gy, x, part, sgpart, d, p, s) : launch_i8_v<G, false>(gy, x, part, sgpart, d, p, s);
 }
 
 template <class G>
@@ -929,18 +815,13 @@ static void plan_i8(const ConvDims &d, GradWMfmaPlan &p) {
     p.slots = plan_grad_w_slots(p.gy * p.gz, p.ntiles, sizeof(double) * ((size_t)d.Co * d.Ci * G::KK + d.Co));
 }
 
-bool plan_grad_w_i8_rows(int N, int Ci, int Co, long L, GradWMfmaPlan &p) {
-    if (L < 4 || (128 + 2 * L) * (Ci > Co ? Ci : Co) > 2L * kBufferImage || N * L > 1L << 30) return false;   // 32-bit offsets from a tile's first image
-    p.variant = Co > 32 ? 32 : 33;
-    if (p.variant == 32) plan_i8_row<GiRow>(N, Ci, Co, (int)L, p);
-    else plan_i8_row<GiRowN>(N, Ci, Co, (int)L, p);
+static bool plan_i8_rows(const ConvDims &d, GradWMfmaPlan &p) {
+    const long L = (long)d.H * d.W;
+    if (L < 4 || (128 + 2 * L) * (d.Ci > d.Co ? d.Ci : d.Co) > 2L * kBufferImage || d.N * L > 1L << 30) return false;   // 32-bit offsets from a tile's first image
+    p.variant = d.Co > 32 ? 32 : 33;
+    if (p.variant == 32) plan_i8_row<GiRow>(d.N, d.Ci, d.Co, (int)L, p);
+    else plan_i8_row<GiRowN>(d.N, d.Ci, d.Co, (int)L, p);
     return true;
-}
-
-int launch_grad_w_i8_rows(const float *gy, const float *x, double *part, double *sgpart, int N, int Ci, int Co, int L, const GradWMfmaPlan &p,
-                          hipStream_t s) {
-    return p.variant == 32 ? launch_i8_row<GiRow>(gy, x, part, sgpart, N, Ci, Co, L, p, s, nullptr, nullptr, nullptr, kNoBnSums)
-                           : launch_i8_row<GiRowN>(gy, x, part, sgpart, N, Ci, Co, L, p, s, nullptr, nullptr, nullptr, kNoBnSums);
 }
 
 // Whether it takes a layer.  Against the fp64 matrix kernel it has some more to set up (half a workgroup's waves load, digits, four
@@ -963,7 +844,7 @@ bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
         const long L = (long)d.H * d.W;
         const double macs = (double)round_up(d.Ci, 16) * round_up(d.Co, 16) * d.N * L;
         if (!(d.Ci >= 64 && d.Co >= 64) && !(L % 4 && d.N * L >= 3000) && !(d.Ci >= 32 && d.Co >= 32 && macs >= 2.2e8)) return false;
-        return plan_grad_w_i8_rows(d.N, d.Ci, d.Co, L, p);
+        return plan_i8_rows(d, p);
     }
     if (d.N < 4 || (d.kh != 3 && d.kh != 5)) return false;
     if ((long)d.Ci * d.H * d.W > kBufferImage || (long)d.Co * d.H * d.W > kBufferImage) return false;
@@ -994,26 +875,20 @@ bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
     return false;
 }
 
-template <class T>
-int launch_grad_w_i8(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s,
-                     const float *bn_y, const float *bn_coef, float *gy_out, const BnSums &sums) {
+int launch_grad_w_i8(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s) {
     switch (p.variant) {
-        case 20: return launch_i8<Gi3a32>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 21: return launch_i8<Gi3a16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 22: return launch_i8<Gi3a8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 24: case 25: return launch_i8<Gi3b16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 26: return launch_i8<Gi3b8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 28: return launch_i8<Gi5w32>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 29: return launch_i8<Gi5w16>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 30: return launch_i8<Gi5w8>(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
-        case 32: return launch_i8_row<GiRow>(gy, x, part, sgpart, d.N, d.Ci, d.Co, d.H * d.W, p, s, bn_y, bn_coef, gy_out, sums);
-        case 33: return launch_i8_row<GiRowN>(gy, x, part, sgpart, d.N, d.Ci, d.Co, d.H * d.W, p, s, bn_y, bn_coef, gy_out, sums);
+        case 20: return launch_i8<Gi3a32>(gy, x, part, sgpart, d, p, s);
+        case 21: return launch_i8<Gi3a16>(gy, x, part, sgpart, d, p, s);
+        case 22: return launch_i8<Gi3a8>(gy, x, part, sgpart, d, p, s);
+        case 24: case 25: return launch_i8<Gi3b16>(gy, x, part, sgpart, d, p, s);
+        case 26: return launch_i8<Gi3b8>(gy, x, part, sgpart, d, p, s);
+        case 28: return launch_i8<Gi5w32>(gy, x, part, sgpart, d, p, s);
+        case 29: return launch_i8<Gi5w16>(gy, x, part, sgpart, d, p, s);
+        case 30: return launch_i8<Gi5w8>(gy, x, part, sgpart, d, p, s);
+        case 32: return launch_i8_row<GiRow>(gy, x, part, sgpart, d, p, s);
+        case 33: return launch_i8_row<GiRowN>(gy, x, part, sgpart, d, p, s);
         default: return ADDER_ERR_BAD_SHAPE;
     }
 }
-template int launch_grad_w_i8<float>(const float *, const float *, double *, double *, const ConvDims &, const GradWMfmaPlan &, hipStream_t,
-                                     const float *, const float *, float *, const BnSums &);
-template int launch_grad_w_i8<bf16_t>(const bf16_t *, const bf16_t *, double *, double *, const ConvDims &, const GradWMfmaPlan &,
-                                      hipStream_t, const float *, const float *, float *, const BnSums &);
 
 }  // namespace adder

@@ -1,5 +1,4 @@
-// Weight gradient of the AdderNet convolution (3x3 / pad 1, 5x5 / pad 2, or 1x1) on the matrix cores, in full precision: the layers
-// with a stride, the small ones and those of fewer than four images (the others: grad_w_i8.hip).
+// Weight gradient of the AdderNet convolution (3x3 / pad 1, 5x5 / pad 2, or 1x1) on the matrix cores, in full precision.
 //
 //   gw[co,k] = sum_pos xcol[k,pos] * gy[co,pos]  -  w[co,k] * sum_pos gy[co,pos]      (k = (ci, i, j))
 //
@@ -22,7 +21,6 @@
 // the (co, k) block of the workgroup; the waves are folded in fp64 through LDS at the end.
 // sum_pos gy is collected on the A fragments.  Partials: one fp64 (Co, K) slab per grid.x slot.
 #include "common.hpp"
-#include "grad_w_bn.hpp"
 #include "tile3x3.hpp"
 
 namespace adder {
@@ -134,6 +132,51 @@ __device__ __forceinline__ void gy_commit_m_bn(const GyStageM<G> &sg, const GySt
             *reinterpret_cast<float4 *>(buf + pc * G::GPLANE + r * G::TW + 4 * q) = v;
             if (gy_out && ok)
                 *reinterpret_cast<float4 *>(gy_out + ((((n0 + img) * Co + co0 + c) * Ho + h0 + r) * Wo + w0 + 4 * q)) = v;
+        }
+    }
+}
+
+// The four coefficients of gy_commit_m_bn for the workgroup's COB channels, from the sums the consumer's
+// input-gradient kernel left (BnSums): 32 lanes add the slots of one channel, always in the same order, so every
+// workgroup that needs a channel arrives at the same bits.  `write`: also store dgamma / dbeta of these channels
+// (one workgroup per channel block does).  Stands in for a launch of its own between the two kernels.
+template <class G>
+__device__ __forceinline__ void bn_coef_from_sums(const BnSums &b, int co0, int Co, float4 *coef, bool write) {
+    constexpr int GROUPS = G::NTHREADS / 32;
+    constexpr int CHUNK = 16;
+    const int sub = threadIdx.x & 31, grp = threadIdx.x >> 5;
+    for (int cb = 0; cb < G::COB; cb += GROUPS) {
+        const int c = cb + grp;
+        if (G::COB % GROUPS == 0 || c < G::COB) {
+            const int co = min(co0 + c, Co - 1);
+            const float rs = b.rstd[co], gm = b.gamma[co], mu = b.mean[co];
+            const float2 *p = reinterpret_cast<const float2 *>(b.part) + (size_t)co * b.slots;
+            double s1 = 0.0, s2 = 0.0;
+            for (int s0 = sub; s0 < b.slots; s0 += 32 * CHUNK) {   // CHUNK loads in flight, then added in slot order
+                float2 v[CHUNK];
+#pragma unroll
+                for (int j = 0; j < CHUNK; ++j) v[j] = p[min(s0 + 32 * j, b.slots - 1)];   // (unconditional: no waits between them)
+#pragma unroll
+                for (int j = 0; j < CHUNK; ++j) {
+                    const bool in = s0 + 32 * j < b.slots;
+                    s1 += in ? (double)v[j].x : 0.0;
+                    s2 += in ? (double)v[j].y : 0.0;
+                }
+            }
+#pragma unroll
+            for (int m = 16; m >= 1; m >>= 1) {   // (stays inside the 32-lane half)
+                s1 += __shfl_xor(s1, m, 64);
+                s2 += __shfl_xor(s2, m, 64);
+            }
+            if (sub == 0) {
+                const float m1 = (float)(s1 / b.count), m2 = (float)(s2 / b.count);
+                const float k = gm * rs;
+                coef[c] = make_float4(k, -k * rs * m2, mu, k * m1);
+                if (write && co0 + c < Co) {
+                    b.dbeta[co] = (float)s1;
+                    b.dgamma[co] = (float)s2;
+                }
+            }
         }
     }
 }
@@ -404,11 +447,6 @@ static ConvDims mfma_one_row(const ConvDims &d) {
 
 GradWMfmaPlan plan_grad_w_mfma(const ConvDims &d) {
     GradWMfmaPlan p{};
-    return plan_grad_w_i8(d, p) ? p : plan_grad_w_fp64(d);
-}
-
-GradWMfmaPlan plan_grad_w_fp64(const ConvDims &d) {
-    GradWMfmaPlan p{};
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci >= 64 && d.Co >= 64) {
         const ConvDims f = mfma_one_row(d);
         if (d.Ci >= 128 && d.Co >= 128) {
@@ -477,7 +515,6 @@ static int launch_one(const T *gy, const T *x, double *part, double *sgpart, con
 int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double *sgpart, const ConvDims &d,
                           const GradWMfmaPlan &p, const float *bn_y, const float *bn_coef, float *gy_out, hipStream_t s,
                           const BnSums &sums) {
-    if (p.variant >= 20) return launch_grad_w_i8(gy, x, part, sgpart, d, p, s, bn_y, bn_coef, gy_out, sums);
     const Subsample none{1, 0, 0, 0};
     if (((p.variant >= 1 && p.variant <= 5) || p.variant == 14) && (d.W % 4 != 0 || d.Wo % 4 != 0))
         return ADDER_ERR_UNSUPPORTED;
@@ -506,7 +543,6 @@ int launch_grad_w_mfma_bn(const float *gy, const float *x, double *part, double 
 template <class T>
 int launch_grad_w_mfma(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p,
                        hipStream_t s) {
-    if (p.variant >= 20) return launch_grad_w_i8(gy, x, part, sgpart, d, p, s);
     switch (p.variant) {
         case 1: return launch_one<GmW32>(gy, x, part, sgpart, d, p, s);
         case 2: return launch_one<GmW16>(gy, x, part, sgpart, d, p, s);

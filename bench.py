@@ -25,9 +25,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
-# MI355X fp64 matrix peak: the strided and small 3x3 weight gradients run on v_mfma_f64_16x16x4_f64.  (The large stride-1
-# ones multiply fixed-point digits on the 8-bit matrix cores instead, so their share of it can pass 1.)
-PEAK_FP64_MFMA_TFLOPS = 78.6
+PEAK_FP64_MFMA_TFLOPS = 78.6       # MI355X fp64 matrix peak: the 3x3 weight gradient runs on v_mfma_f64_16x16x4_f64
 PEAK_FP32_TFLOPS = 157.3           # MI355X vendor fp32 vector peak (256 CU x 64 lanes x 2 (packed) x 2 (FMA) x 2.4 GHz)
 # lane-instructions per second: a SIMD starts two vector instructions per 4-cycle slot when two of its
 # waves are ready (one per wave), so 256 CU x 4 SIMD x 2 x 64 lanes / 4 cycles x 2.4 GHz; with an FMA in
@@ -173,7 +171,7 @@ def bench_layers(dev, warmup=5, iters=20, which="resnet20"):
                 "algorithmic_bytes": nbytes[name], "hbm_gbs": round(nbytes[name] / t / 1e9, 1),
                 "frac_hbm_peak": round(nbytes[name] / t / 1e9 / PEAK_HBM_GBS, 4),
             }
-            if name in ("grad_w", "grad_w_bn") and k == 3:   # matrix-core kernel (+ finalize and scaling launches)
+            if name in ("grad_w", "grad_w_bn") and k == 3:   # fp64 matrix-core kernel (+ finalize and scaling launches)
                 row["frac_fp64_mfma_peak"] = round(2 * E / t / 1e12 / PEAK_FP64_MFMA_TFLOPS, 4)
             else:
                 row["valu_issue_util"] = round(slots * E / t / PEAK_VALU_ISSUE, 4)
