@@ -1,5 +1,5 @@
-// Weight gradient of 3x3 / pad 1, 5x5 / pad 2 and 1x1 layers of stride 1, and of column matrices, on the 8-bit matrix cores, as exact
-// as the fp64 ones.  (First the kernel of the 3x3 and 5x5 layers, then that of the single taps.)
+// Weight gradient of large 3x3 / pad 1, 5x5 / pad 2 and 1x1 layers of stride 1 in bfloat16 storage, on the 8-bit matrix cores.  (First the kernel
+// of the 3x3 and 5x5 layers, then that of the single taps.)
 //
 //   gw[co,ci,i,j] = sum_pos x[ci, pos + (i,j)] * gy[co,pos]  -  w[co,ci,i,j] * sum_pos gy[co,pos]
 //
@@ -7,12 +7,15 @@
 // cycle and SIMD.  v_mfma_i32_16x16x64_i8 does 1000, exactly, so the operands are written in fixed point, four signed 8-bit digits
 // each, and thirteen digit products (of the sixteen: the three left out lie below the last digit) stand for one fp64 product:
 //   x = 2^ex * sum_d X_d 2^-8d,   gy = 2^eg * sum_d G_d 2^-8d,   x * gy = 2^(ex+eg) * sum_{s<5} 2^-8s sum_{d+e=s} X_d G_e.
-// The scales 2^ex, 2^eg belong to one channel of one staged tile (256 positions), so the fixed point is relative to the
-// largest of 256 values: 32 bits, every value down to 1/64 of the largest keeps all its 24 bits, and as the largest of 256 is at
-// most 16 times their root mean square, whatever the data, a tile's sums are off by at most 2^-25 of |x| |gy|, in practice by
-// 2^-30 of the result (relative error of the raw gradient, 2-norm: 2.549e-8 where the fp64 kernel has 2.549e-8, 128 -> 128 @32x32, 128
-// images; ten products: 2.56e-8).  The digit sums of a tile are exact in 32 bits (at most four products of 2^14, 256 positions) and go
-// into fp64 sums with their scales.  A tile with a value that is infinite or not a number is worked out in fp64 from the same LDS cells.
+// The scales 2^ex, 2^eg belong to one channel of one staged tile (256 positions of gy, those and the halo of x), so the fixed point is
+// relative to the largest of these values: 32 bits, which hold the eight bits of every value down to 2^-22 of it.  The digit sums of a tile are
+// exact in 32 bits (at most four products of 2^14, 256 positions) and go into fp64 sums with their scales; gy is added up in fp64 as it is.  Where values
+// were rounded that matter, and where one is infinite or not a number, the workgroup goes through its tiles again with the values
+// and fp64 products ("whether the digits will do", below).  Error of the raw gradient against float64 on the tensors of a ResNet-20 training
+// step, 2-norm, worst layer: 2.591e-8, all of it the rounding to float, where the fp64 kernels have 2.591e-8; no layer is gone through again.
+// (Not for float storage: its 24 bits are exact down to 2^-6 of the largest only, and half of a training step's gradients lie below 2^-10.  Without
+// a rule the same layers' error was 2.89e-8 for 2.59e-8, and wrong altogether where large values met zeros; with a rule that holds it, ordinary
+// steps were gone through again: VGG-small 8.0 -> 11 ms, with the fp64 kernels 9.8.)
 //
 // Layout: a tile is four images x 64 positions.  Its LDS cells are dwords of one digit of four images, so that a
 // lane's sixteen 8-bit operands -- four adjacent columns x four images -- are four cells of a row, and a tap's shift moves whole
@@ -20,10 +23,10 @@
 // row of a 16 x 16 channel block, i.e. KS accumulator tiles x five digit weights.
 //
 // Half of a workgroup's waves multiply, the other half load, find the largest values and write digits, a tile ahead: the conversion is
-// 6.5 vector instructions a value, nearly as much time as the matrix instructions it feeds, and on other waves it runs beside them.
-// What bounds it (128 -> 128 @32x32, 128 images, 1.9e10 multiply-adds: 690 -> 272 us): the multiplying waves -- 78 matrix
-// instructions of 16 cycles per step with the operand moves between them; without the loading waves' work it takes 252 us, without the
-// multiplying waves' 175.  (All waves doing both in turn: 605; loads that branch, so that every wait is for all of them: 300.)
+// eight vector instructions a value, as much time as the matrix instructions it feeds, and on other waves it runs beside them.
+// What bounds it: the issue of both kinds' instructions, which hardly overlap (per tile and SIMD, 128 -> 128 @32x32: 3700 cycles of matrix
+// instructions and 6600 of vector ones, 10 200 measured).  128 -> 128 @32x32, 128 images: fp64 737 us, this 253 (the passes again with values: 1110 in all);
+// 64 -> 64 @56x56, 32 images 170 -> 70; 512 -> 512 @8x8, 128 images 830 -> 283.
 #include "common.hpp"
 
 #include <type_traits>
@@ -51,20 +54,23 @@ struct GwI8Cfg {
     static constexpr int TILE_WORDS = G0 + COB * GPLANE;
     static constexpr int OUT = COB * CIB * KK;                 // results, folded and reordered through LDS at the end (fp64)
     static constexpr int CH = COB + CIB;                       // largest-value slots: gy channels, then x channels
-    static constexpr int MX0 = 2 * TILE_WORDS, COEF0 = MX0 + 4 * CH + 4;
+    static constexpr int MX0 = 2 * TILE_WORDS, SM0 = MX0 + 4 * CH, FLAG0 = SM0 + 4 * CH;
+    // the error sums of the multiplying waves' results lie in LDS: beside the accumulators they would not stay in registers
+    static constexpr int ERR0 = FLAG0 + 4, COEF0 = ERR0 + 64 * MWAVES * 8;
     static constexpr int LDS_BYTES = COEF0 * 4;
     static_assert(TW % 8 == 0 && 4 % STRIPS == 0 && TH * STRIPS % (4 * PW) == 0 && KS % 2 == 1, "whole steps of four strips");
     static_assert((XR * QW) % 4 == 0 && (XR * HC) % 4 == 0 && (TH * QW) % 4 == 0, "four units in a row share a channel");
     static_assert(LDS_BYTES <= 160 * 1024 && NTHREADS <= 1024, "workgroup limits");
-    static_assert(2 * (OUT + COB) <= 2 * TILE_WORDS, "the results fit the cells' place");
+    static_assert(2 * (OUT + GUNITS) <= 2 * TILE_WORDS, "the results fit the cells' place");
     static_assert(XDIG % 4 == 0 && XH % 4 == 0 && GPLANE % 4 == 0 && COEF0 % 4 == 0, "16-byte alignment of the cells");
 };
 
 // Four images of a tensor as a buffer: loads from beyond its end (images that do not exist) or at kNowhere give zeros, so they need no
 // branch -- with loads under way in two register sets, a wait has to know how many are newer.
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 static constexpr unsigned kNowhere = 0x80000000u;
-static constexpr int kBufferImage = 1 << 27;   // elements per image: four of float fill 2^31 bytes, and kNowhere + three does not wrap
+static constexpr int kBufferImage = 1 << 27;   // elements per image: four fill 2^30 bytes, and kNowhere + three does not wrap
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t i8_images(const bf16_t *base, int image, int n0, int N) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(base + (size_t)n0 * image), 0, min(4, N - n0) * image * (int)sizeof(bf16_t), 0x00020000);
 }
@@ -91,13 +97,13 @@ __device__ __forceinline__ float i8_absmax4(float m, const float4 &v) { return i
 
 // A channel's exponent from the bits of its largest magnitude: magnitudes from 1.96875 up count as the next power of two,
 // so that |v| 2^(30-e) < 2^31 - 2^24 and the first digit stays within +-127 (the last three carry into it).  255: not finite (or within
-// 1.6 % of the largest float), the tile takes the fp64 path.  Below 2^-97 the last digit stays at 2^-127, which 2^127 still reaches.
+// 1.6 % of the largest float).  Below 2^-97 the last digit stays at 2^-127, which 2^127 still reaches.
 __device__ __forceinline__ int i8_exponent(unsigned m) { return max((int)((m + 0x40000u) >> 23), 30); }
 __device__ __forceinline__ double i8_unit(int e) { return __hiloint2double((e - 127 - 30 + 1023) << 20, 0); }   // 2^(e - 127 - 30): the last digit's
 __device__ __forceinline__ float i8_scale(int e) { return __uint_as_float((unsigned)(30 + 127 + 127 - e) << 23); }   // its reciprocal, 2^(30 - (e - 127))
 
 // largest magnitude of the four lanes of a quad into its channel's slot
-__device__ __forceinline__ void i8_note_max(float m, unsigned *slot, unsigned *flag, bool ok) {
+__device__ __forceinline__ void i8_note_max(float m, unsigned *slot, int *flag, bool ok) {
     unsigned u = __float_as_uint(m) & 0x7fffffffu;
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
@@ -106,14 +112,31 @@ __device__ __forceinline__ void i8_note_max(float m, unsigned *slot, unsigned *f
         if (i8_exponent(u) >= 255) *flag = 1;
     }
 }
+// sum over the four lanes of a quad into its channel's slot
+__device__ __forceinline__ void i8_note_sum(int u, int *slot) {
+    if (__builtin_amdgcn_ballot_w64(u) == 0) return;
+    u += __builtin_amdgcn_update_dpp(0, u, 0xB1, 0xF, 0xF, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x4E, 0xF, 0xF, true);
+    if ((threadIdx.x & 3) == 0 && u) atomicAdd(slot, u);
+}
 
-// v times a power of two, to the nearest integer.  (v_cvt_rpi_i32_f32 would do both steps, but rounds odd results above 2^23 away.)
-__device__ __forceinline__ unsigned i8_round(float v, float scale) { return (unsigned)(int)rintf(v * scale); }
+// v times a power of two, to the nearest integer; off: the largest distance from it so far.  (v_cvt_rpi_i32_f32 would do both steps, but rounds odd
+// results above 2^23 away.)
+__device__ __forceinline__ unsigned i8_round(float v, float scale, float &off) {
+    const float t = v * scale, r = rintf(t);
+    off = fmaxf(off, fabsf(t - r));
+    return (unsigned)(int)r;
+}
+// how many of four values were rounded
+__device__ __forceinline__ int i8_count(float a, float b, float c, float d, float scale) {
+    auto one = [&](const float v) { return v * scale != rintf(v * scale) ? 1 : 0; };
+    return (one(a) + one(b)) + (one(c) + one(d));
+}
 // four values (one column of four images) as four cells, one per digit.  Adding 0x808080 turns the lower three digits into unsigned
 // ones with carries, the exclusive-or makes them signed again.
-__device__ __forceinline__ void i8_digits(float a, float b, float c, float d, float scale, int (&cell)[4]) {
-    const unsigned u0 = i8_round(a, scale) + 0x808080u, u1 = i8_round(b, scale) + 0x808080u,
-                   u2 = i8_round(c, scale) + 0x808080u, u3 = i8_round(d, scale) + 0x808080u;
+__device__ __forceinline__ void i8_digits(float a, float b, float c, float d, float scale, int (&cell)[4], float &off) {
+    const unsigned u0 = i8_round(a, scale, off) + 0x808080u, u1 = i8_round(b, scale, off) + 0x808080u,
+                   u2 = i8_round(c, scale, off) + 0x808080u, u3 = i8_round(d, scale, off) + 0x808080u;
     const unsigned lo01 = __builtin_amdgcn_perm(u1, u0, 0x05010400u), hi01 = __builtin_amdgcn_perm(u1, u0, 0x07030602u);
     const unsigned lo23 = __builtin_amdgcn_perm(u3, u2, 0x05010400u), hi23 = __builtin_amdgcn_perm(u3, u2, 0x07030602u);
     cell[0] = (int)__builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
@@ -122,33 +145,64 @@ __device__ __forceinline__ void i8_digits(float a, float b, float c, float d, fl
     cell[3] = (int)(__builtin_amdgcn_perm(lo23, lo01, 0x05040100u) ^ 0x80808080u);
 }
 
-// a unit of four columns x four images into the cells at p (p + digit * pitch); raw: the values themselves, image k in the
-// place of digit k
-__device__ __forceinline__ void i8_put4(const float4 (&v)[4], float scale, bool raw, int *p, int pitch) {
-    if (!raw) {
+// a unit of four columns x four images into the cells at p (p + digit * pitch); RAW: the values themselves, image k in the
+// place of digit k.  Gives how many were rounded.
+template <bool RAW>
+__device__ __forceinline__ int i8_put4(const float4 (&v)[4], float scale, int *p, int pitch) {
+    int rounded = 0;
+    if constexpr (!RAW) {
+        float off = 0.f;
         int c0[4], c1[4], c2[4], c3[4];
-        i8_digits(v[0].x, v[1].x, v[2].x, v[3].x, scale, c0);
-        i8_digits(v[0].y, v[1].y, v[2].y, v[3].y, scale, c1);
-        i8_digits(v[0].z, v[1].z, v[2].z, v[3].z, scale, c2);
-        i8_digits(v[0].w, v[1].w, v[2].w, v[3].w, scale, c3);
+        i8_digits(v[0].x, v[1].x, v[2].x, v[3].x, scale, c0, off);
+        i8_digits(v[0].y, v[1].y, v[2].y, v[3].y, scale, c1, off);
+        i8_digits(v[0].z, v[1].z, v[2].z, v[3].z, scale, c2, off);
+        i8_digits(v[0].w, v[1].w, v[2].w, v[3].w, scale, c3, off);
 #pragma unroll
         for (int k = 0; k < 4; ++k) *reinterpret_cast<int4v *>(p + k * pitch) = int4v{c0[k], c1[k], c2[k], c3[k]};
+        if (__builtin_amdgcn_ballot_w64(off > 0.f))   // (seldom)
+            rounded = (i8_count(v[0].x, v[1].x, v[2].x, v[3].x, scale) + i8_count(v[0].y, v[1].y, v[2].y, v[3].y, scale)) +
+                      (i8_count(v[0].z, v[1].z, v[2].z, v[3].z, scale) + i8_count(v[0].w, v[1].w, v[2].w, v[3].w, scale));
     } else {
 #pragma unroll
         for (int k = 0; k < 4; ++k) *reinterpret_cast<float4 *>(p + k * pitch) = v[k];
     }
+    return rounded;
 }
 
-// The digit sums of one result (a[s]: digit weights 2^-8s) in units of the third: first digits lie within +-127, the others within
-// +-128, a tile has 256 positions, so the sums stay below 2^26 and the first two fit one 32-bit number.  (The fifth and fourth are
-// rounded to the unit of the third, 2^-29 of the result: the fourth starts at half of that.)
+// The digit sums of one result (a[s]: digit weights 2^-8s) in units of the third, in fp64: first digits lie within +-127, the others
+// within +-128, a tile has at most 256 positions, so the sums stay within 2^24 and the first two fit one 32-bit number.
 __device__ __forceinline__ double i8_product(int a0, int a1, int a2, int a3, int a4) {
-    return fma((double)((a0 << 8) + a1), 256.0, (double)(a2 + ((a3 + (a4 >> 8)) >> 8)));
+    return fma((double)(((a3 & 255) << 8) + a4), 0x1p-16, fma((double)((a0 << 8) + a1), 256.0, (double)(a2 + (a3 >> 8))));
 }
-// the digit sums of at most 256 values as their sum, exactly
-__device__ __forceinline__ double i8_sum(int a0, int a1, int a2, int a3) {
-    return fma((double)((a0 << 8) + a1), 65536.0, (double)((a2 << 8) + a3));
+
+// ---- whether the digits will do ----
+// A bfloat16 value has eight significant bits, so the fixed point holds it exactly down to 2^-22 of its channel's largest in the tile; the products left
+// out are those of two digits below 2^-16.  What can go wrong is a tile whose largest values meet nothing but zeros, so that the sum consists of
+// values far below them.  In units of the two channels' first digits (X = |x| / 2^(ex-6) < 126, G alike) the square of a tile's error is, on the average
+// over roundings, at most 2^-50 / 3 of  126^2 * the number of values that were rounded  (+ kLeftOut for the products left out).  A lane adds that up over all
+// tiles for its results, and at the end the block's rows and columns are looked at one by one: where the errors' sum of squares is above 2^-48 of the
+// results', the workgroup works its block out again in fp64.  (126 is the most a partner can have; it has a quarter of that on the average.)
+static constexpr int kRounded = 126 * 126, kLeftOut = 42;
+static constexpr double kFine = 3 * 0x1p-30;   // 3 * 2^50 * 2^-48, and scales count in the third digit, 2^16 a product less
+__device__ __forceinline__ bool i8_fine(double errors, double results) { return errors <= kFine * results; }
+
+// sum over the sixteen lanes of a row of a wave (in registers: forty sums through LDS would be 3 us of a small layer's 16)
+__device__ __forceinline__ double i8_row_sum(double v) {
+    auto from = [&](auto ctrl) __attribute__((always_inline)) {
+        return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), decltype(ctrl)::value, 0xF, 0xF, true),
+                                __builtin_amdgcn_update_dpp(0, __double2loint(v), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    v += from(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
+    v += from(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
+    v += from(std::integral_constant<int, 0x141>{});   // row_half_mirror
+    v += from(std::integral_constant<int, 0x140>{});   // row_mirror
+    return v;
 }
+
+typedef double double4v __attribute__((ext_vector_type(4)));
+// The row of 16 that lane l of a wave gives v_mfma_f64_16x16x4_f64, so that the results, rows 4 e + l / 16 there, lie like those of the 8-bit
+// ones, rows 4 (l / 16) + e.
+__device__ __forceinline__ int i8_fp64_row(int l16) { return 4 * (l16 & 3) + (l16 >> 2); }
 
 template <class G, bool VEC>
 __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(const bf16_t *__restrict__ gy, const bf16_t *__restrict__ x,
@@ -156,8 +210,9 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
                                                                 int Ci, int H, int W, int Co, int tilesH, int tilesW, int ntiles) {
     constexpr int KS = G::KS, PAD = G::PAD, QW = G::QW, SQ = 2;   // SQ: groups of four columns in a strip
     extern __shared__ __align__(16) int cells[];   // two tiles: x cells, gy cells
-    unsigned *const mx = reinterpret_cast<unsigned *>(cells + G::MX0);   // largest magnitudes of four tiles, then four flags
-    unsigned *const flags = mx + 4 * G::CH;
+    unsigned *const mx = reinterpret_cast<unsigned *>(cells + G::MX0);   // the channels' largest magnitudes in four tiles,
+    int *const sm = cells + G::SM0;   // how many of their values were rounded
+    int *const flag = cells + G::FLAG0;   // the digits will not do
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
     const bool loader = wave >= G::MWAVES;
@@ -166,9 +221,10 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     const int ti = wave % KS, pw = wave / KS % G::PW, mb = wave / KS / G::PW % G::MB, nb = wave / KS / G::PW / G::MB;
     const int co_blk = blockIdx.y * G::COB, ci_blk = blockIdx.z * G::CIB;
     // the workgroup's tiles lie side by side: the lines that neighbouring tiles share stay in one L2
-    const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, tile0 = blockIdx.x * each, mine = min(each, ntiles - tile0);
+    const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, mine = min(each, ntiles - (int)blockIdx.x * each);
+    int tile0 = blockIdx.x * each;
 
-    for (int e = tid; e < 4 * G::CH + 4; e += G::NTHREADS) mx[e] = 0;
+    for (int e = tid; e < G::FLAG0 + 1 - G::MX0; e += G::NTHREADS) mx[e] = 0;
     __syncthreads();
 
     // ---- the loading waves ----
@@ -191,10 +247,11 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
         hcol[it] = u % G::HC; hrow[it] = u / G::HC % G::XR; hch[it] = u / G::HC / G::XR;
     }
     // Two tiles under way in registers; one, where a thread has two gy units: the multiplying waves last longer than a load there, and
-    // a second set would spill (128 -> 128 @32x32, 128 images, 275 us with two, 272 with one).
-    constexpr int SETS = KS == 3 && G::GITER > 1 ? 1 : 2;
+    // a second set would spill (and a wait for a spilled address is a wait for all loads: 48 -> 48 5x5 @28x28, 8 images, 33 us with two, 26 with one).
+    constexpr int SETS = G::GITER > 1 ? 1 : 2;
     float4 xv[SETS][G::XITER][4], gv[SETS][G::GITER][4];
     float hv[SETS][G::HITER][4];
+    double sgt[G::GITER];   // sums of the gy units' values
     auto place = [&](const int i, int &n0, int &h0, int &w0) {
         int t = tile0 + i;
         const int tw = t % tilesW; t /= tilesW;
@@ -237,7 +294,14 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     // the largest magnitudes of the channels of tile i, which is in set b
     auto note = [&](const int i, auto set) __attribute__((always_inline)) {
         constexpr int b = decltype(set)::value;
-        unsigned *const mxs = mx + (i & 3) * G::CH, *const flag = flags + (i & 3);
+        unsigned *const mxs = mx + (i & 3) * G::CH;
+        if (blockIdx.z == 0) {
+#pragma unroll
+            for (int it = 0; it < G::GITER; ++it)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    sgt[it] += ((double)gv[b][it][k].x + (double)gv[b][it][k].y) + ((double)gv[b][it][k].z + (double)gv[b][it][k].w);
+        }
 #pragma unroll
         for (int it = 0; it < G::GITER; ++it) {
             const bool ok = G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB;
@@ -262,27 +326,35 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
         }
     };
     // set b into the cells of tile i
-    auto commit = [&](const int i, auto set) __attribute__((always_inline)) {
+    auto commit = [&](const int i, auto set, auto with_values) __attribute__((always_inline)) {
         constexpr int b = decltype(set)::value;
+        constexpr bool RAW = decltype(with_values)::value;
         int *const tile = cells + (i & 1) * G::TILE_WORDS;
         const unsigned *const mxs = mx + (i & 3) * G::CH;
-        const bool raw = __builtin_amdgcn_readfirstlane((int)flags[i & 3]) != 0;
+        int *const sms = sm + (i & 3) * G::CH;
 #pragma unroll
         for (int it = 0; it < G::GITER; ++it)
-            if (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB)
-                i8_put4(gv[b][it], i8_scale(i8_exponent(mxs[gch[it]])), raw,
-                        tile + G::G0 + gch[it] * G::GPLANE + grow[it] * G::TW + gcol[it], G::GDIG);
+            if (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB) {
+                const int rounded = i8_put4<RAW>(gv[b][it], i8_scale(i8_exponent(mxs[gch[it]])),
+                                                 tile + G::G0 + gch[it] * G::GPLANE + grow[it] * G::TW + gcol[it], G::GDIG);
+                if constexpr (!RAW) i8_note_sum(rounded, sms + gch[it]);
+            }
 #pragma unroll
         for (int it = 0; it < G::XITER; ++it)
-            if (G::XUNITS % G::LTHREADS == 0 || xch[it] < G::CIB)
-                i8_put4(xv[b][it], i8_scale(i8_exponent(mxs[G::COB + xch[it]])), raw,
-                        tile + xch[it] * G::XPLANE + xrow[it] * G::TW + xcol[it], G::XDIG);
+            if (G::XUNITS % G::LTHREADS == 0 || xch[it] < G::CIB) {
+                const int rounded = i8_put4<RAW>(xv[b][it], i8_scale(i8_exponent(mxs[G::COB + xch[it]])),
+                                                 tile + xch[it] * G::XPLANE + xrow[it] * G::TW + xcol[it], G::XDIG);
+                if constexpr (!RAW) i8_note_sum(rounded, sms + G::COB + xch[it]);
+            }
 #pragma unroll
         for (int it = 0; it < G::HITER; ++it)
             if (G::HUNITS % G::LTHREADS == 0 || hch[it] < G::CIB) {
                 int cell[4];
-                if (!raw) {
-                    i8_digits(hv[b][it][0], hv[b][it][1], hv[b][it][2], hv[b][it][3], i8_scale(i8_exponent(mxs[G::COB + hch[it]])), cell);
+                if constexpr (!RAW) {
+                    const float (&v)[4] = hv[b][it], scale = i8_scale(i8_exponent(mxs[G::COB + hch[it]]));
+                    float off = 0.f;
+                    i8_digits(v[0], v[1], v[2], v[3], scale, cell, off);
+                    i8_note_sum(i8_count(v[0], v[1], v[2], v[3], scale), sms + G::COB + hch[it]);
                 } else {
 #pragma unroll
                     for (int k = 0; k < 4; ++k) cell[k] = __float_as_int(hv[b][it][k]);
@@ -294,12 +366,7 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     };
 
     // ---- the multiplying waves ----
-    const bool sg_wave = ti == 0 && nb == 0 && blockIdx.z == 0;   // also adds gy up
-    double tot[KS][4], sgt = 0.0;   // tot[j][e]: row 4 * lk + e (output channel), column l16 (input channel), tap (ti, j)
-#pragma unroll
-    for (int j = 0; j < KS; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) tot[j][e] = 0.0;
+    // tot[j][e]: row 4 * lk + e (output channel), column l16 (input channel), tap (ti, j)
     // The wave's operands: lane group lk takes strip lk of a step's four.  The cells before and after a strip are its neighbours' or,
     // at the ends of a row, the halo's.  (Steps are whole rows apart, 4 / STRIPS of them.)
     constexpr int ROWS = 4 / G::STRIPS;
@@ -309,14 +376,16 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
     const bool first = strip == 0, last = strip == G::STRIPS - 1;
     const int loff = first ? xhalo : xoff - PAD, roff = last ? xhalo + PAD : xoff + 8;
     const int lstep = ROWS * (first ? G::HC : G::TW), rstep = ROWS * (last ? G::HC : G::TW);
-    auto multiply = [&](const int i) {
-        const int *const tile = cells + (i & 1) * G::TILE_WORDS;
+    double2 *const errs = reinterpret_cast<double2 *>(cells + G::ERR0) + wave * 128 + lane;   // of rows e = 0, 1 and 64 further on of 2, 3
+    // tile i at row h0: into tot, and the squares of the errors into errs
+    auto multiply = [&](const int i, const int h0, double4v (&tot)[KS]) __attribute__((always_inline)) {
+        const int *const tile = cells + (i & 1) * G::TILE_WORDS, *const sms = sm + (i & 3) * G::CH;
         const unsigned *const mxs = mx + (i & 3) * G::CH;
         int4v acc[KS][5];
 #pragma unroll
         for (int j = 0; j < KS; ++j)
 #pragma unroll
-            for (int s = 0; s < 5; ++s) acc[j][s] = s != 3 ? int4v{0, 0, 0, 0} : int4v{128, 128, 128, 128};
+            for (int s = 0; s < 5; ++s) acc[j][s] = int4v{0, 0, 0, 0};
         // The x cells of one digit and step are a phase: KS matrix instructions per digit of gy that goes with it.  The next phase's cells
         // are asked for before a phase's instructions, a step's last gy digits (which the last phase does not need) with them.
         int4v a[SQ][4], mid[2][SQ];
@@ -365,122 +434,197 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_kernel(con
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        const double sx = i8_unit(i8_exponent(mxs[G::COB + nb * 16 + l16])) * 4294967296.0;   // (i8_product counts in 2^32)
+        const unsigned xm = mxs[G::COB + nb * 16 + l16];
+        const int xs = kRounded * sms[G::COB + nb * 16 + l16] + kLeftOut;
+        const uint4v gm = *reinterpret_cast<const uint4v *>(mxs + mb * 16 + 4 * lk);
+        const int4v gs = *reinterpret_cast<const int4v *>(sms + mb * 16 + 4 * lk);
+        const double sx = xm ? i8_unit(i8_exponent(xm)) * 4294967296.0 : 0.0;   // (i8_product counts in 2^32)
+        double err[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const double sc = sx * i8_unit(i8_exponent(mxs[mb * 16 + 4 * lk + e]));
+            const double sc = gm[e] ? sx * i8_unit(i8_exponent(gm[e])) : 0.0;
+            err[e] = (sc * sc) * (double)(kRounded * gs[e] + xs);
 #pragma unroll
             for (int j = 0; j < KS; ++j)
                 tot[j][e] = fma(i8_product(acc[j][0][e], acc[j][1][e], acc[j][2][e], acc[j][3][e], acc[j][4][e]), sc, tot[j][e]);
         }
-        if (sg_wave) {   // (read again: the digits that the matrix instructions had are gone)
-            int sd[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int rs = 0; rs < G::STEPS; ++rs)
-#pragma unroll
-                for (int q = 0; q < SQ; ++q)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const int4v g = *reinterpret_cast<const int4v *>(tile + goff + rs * ROWS * G::TW + d * G::GDIG + 4 * q);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) sd[d] = __builtin_amdgcn_sdot4(g[e], 0x01010101, sd[d], false);
-                    }
-            sgt = fma(i8_sum(sd[0], sd[1], sd[2], sd[3]), i8_unit(i8_exponent(mxs[mb * 16 + l16])), sgt);
+        // (a tap row that lies outside the image throughout the tile has no products)
+        if (max(h0, PAD - ti) < min(h0 + G::TH, min(H, H + PAD - ti))) {
+            const double2 a = errs[0], b = errs[64];
+            errs[0] = make_double2(a.x + err[0], a.y + err[1]);
+            errs[64] = make_double2(b.x + err[2], b.y + err[3]);
         }
     };
-    // a tile with an infinity or a NaN: fp64 from the values; positions outside the tensor do not count (zero times infinity)
-    auto multiply_raw = [&](const int i) {
+    // a tile's values instead of digits: fp64, four images at a time; positions outside the tensor do not count (zero times infinity)
+    auto multiply_raw = [&](const int i, double4v (&tot)[KS]) __attribute__((always_inline)) {
         int n0, h0, w0;
         place(i, n0, h0, w0);
         const int *const tile = cells + (i & 1) * G::TILE_WORDS;
-        constexpr int SHARE = 4 * G::TH * G::TW / G::PW;
-        for (int pos = pw * SHARE; pos < (pw + 1) * SHARE; ++pos) {
-            const int k = pos % 4, c = pos / 4 % G::TW, r = pos / 4 / G::TW;
-            if (n0 + k >= N || h0 + r >= H || w0 + c >= W) continue;
-            const int *gp = tile + G::G0 + mb * 16 * G::GPLANE + k * G::GDIG + r * G::TW + c;
-            float xr[KS];
+        constexpr int RROWS = G::TH / G::PW;
+        const int gch0 = G::G0 + (mb * 16 + i8_fp64_row(l16)) * G::GPLANE + lk * G::GDIG;
+#pragma unroll 1
+        for (int r = pw * RROWS; r < min((pw + 1) * RROWS, H - h0); ++r) {
+            const int xr = xch0 + lk * G::XDIG + (r + ti) * G::TW, hr = xch0 + lk * G::XDIG + G::XH + (r + ti) * G::HC;   // the row's cells and its halo's
+#pragma unroll 1
+            for (int c = 0; c < min(G::TW, W - w0); c += 4) {
+                const float4 g = *reinterpret_cast<const float4 *>(tile + gch0 + r * G::TW + c);
+                const float4 x = *reinterpret_cast<const float4 *>(tile + xr + c);
+                float win[4 + 2 * PAD];
 #pragma unroll
-            for (int j = 0; j < KS; ++j) {
-                const int cc = c + j - PAD, hc = cc < 0 ? cc + PAD : cc - G::TW + PAD;
-                xr[j] = __int_as_float(tile[xch0 + k * G::XDIG + (cc >= 0 && cc < G::TW ? (r + ti) * G::TW + cc : G::XH + (r + ti) * G::HC + hc)]);
+                for (int e = 0; e < PAD; ++e) {
+                    win[e] = __int_as_float(tile[(c ? xr + c - PAD : hr) + e]);
+                    win[PAD + 4 + e] = __int_as_float(tile[(c + 4 < G::TW ? xr + c + 4 : hr + PAD) + e]);
+                }
+                win[PAD] = x.x; win[PAD + 1] = x.y; win[PAD + 2] = x.z; win[PAD + 3] = x.w;
+                const float gs[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (w0 + c + u < W) {
+#pragma unroll
+                        for (int j = 0; j < KS; ++j) tot[j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)gs[u], (double)win[u + j], tot[j], 0, 0, 0);
+                    }
             }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const double gval = (double)__int_as_float(gp[(4 * lk + e) * G::GPLANE]);
-#pragma unroll
-                for (int j = 0; j < KS; ++j) tot[j][e] = fma((double)xr[j], gval, tot[j][e]);
-            }
-            if (sg_wave && lk == 0) sgt += (double)__int_as_float(gp[l16 * G::GPLANE]);
         }
     };
 
     // While the multiplying waves work on tile i, the loading ones write the cells of tile i + 1, ask for tile i + 3 and note the
     // largest values of tile i + 2, which has arrived meanwhile: one barrier a tile.  (Each kind of wave runs a loop of its own,
-    // with the same barriers, so that neither kind's registers are kept for the other's.)
+    // with the same barriers, so that neither kind's registers are kept for the other's.)  Should the digits not do, both go through the tiles once more.
+    double *const out = reinterpret_cast<double *>(cells), *const sgs = out + G::OUT;
+    auto again = [&]() __attribute__((always_inline)) {
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(*flag) == 0) return false;
+        __syncthreads();
+        for (int e = tid; e < G::FLAG0 - G::MX0; e += G::NTHREADS) mx[e] = 0;
+        __syncthreads();
+        return true;
+    };
     if (loader) {
         constexpr std::integral_constant<int, 0> even{};
         constexpr std::integral_constant<int, SETS - 1> odd{};
-        fetch(0, even);
-        if (SETS == 2) fetch(1, odd);
-        note(0, even);
-        __syncthreads();
-        commit(0, even);
-        fetch(SETS, even);
-        note(1, odd);
-        __syncthreads();
-        auto turn = [&](const int i, auto next, auto after) __attribute__((always_inline)) {   // the sets that hold tiles i + 1 and i + 2
-            if (i + 1 < mine) commit(i + 1, next);
-            for (int e = lt; e < G::CH; e += G::LTHREADS) mx[((i + 3) & 3) * G::CH + e] = 0;
-            if (lt == 0) flags[(i + 3) & 3] = 0;
-            fetch(i + 1 + SETS, next);
-            if (i + 2 < mine) note(i + 2, after);
+        auto pass = [&](auto with_values) __attribute__((always_inline)) {
+            asm volatile("" : "+s"(tile0));   // (no offset of the first pass is kept in a register for the second)
+#pragma unroll
+            for (int it = 0; it < G::GITER; ++it) sgt[it] = 0.0;
+            fetch(0, even);
+            if (SETS == 2) fetch(1, odd);
+            note(0, even);
             __syncthreads();
+            commit(0, even, with_values);
+            fetch(SETS, even);
+            note(1, odd);
+            __syncthreads();
+            auto turn = [&](const int i, auto next, auto after) __attribute__((always_inline)) {   // the sets that hold tiles i + 1 and i + 2
+                // (addresses in LDS are made from these in every turn: kept, they would not all stay in registers, and a wait for one from memory
+                // is a wait for the loads under way)
+#pragma unroll
+                for (int it = 0; it < G::GITER; ++it) asm volatile("" : "+v"(gch[it]));
+#pragma unroll
+                for (int it = 0; it < G::XITER; ++it) asm volatile("" : "+v"(xch[it]));
+#pragma unroll
+                for (int it = 0; it < G::HITER; ++it) asm volatile("" : "+v"(hch[it]));
+                if (i + 1 < mine) commit(i + 1, next, with_values);
+                for (int e = lt; e < G::CH; e += G::LTHREADS) mx[((i + 3) & 3) * G::CH + e] = sm[((i + 3) & 3) * G::CH + e] = 0;
+                fetch(i + 1 + SETS, next);
+                if (i + 2 < mine) note(i + 2, after);
+                __syncthreads();
+            };
+            for (int i = 0; i < mine; i += 2) {   // (always both: a wait for one set must not have to allow for the turn left out)
+                turn(i, odd, even);
+                turn(i + 1, even, odd);
+            }
         };
-        for (int i = 0; i < mine; i += 2) {   // (always both: a wait for one set must not have to allow for the turn left out)
-            turn(i, odd, even);
-            turn(i + 1, even, odd);
+        pass(std::false_type{});
+        if (again()) {
+            pass(std::true_type{});
+            __syncthreads();
         }
+        if (blockIdx.z == 0) {
+#pragma unroll
+            for (int it = 0; it < G::GITER; ++it)
+                if (G::GUNITS % G::LTHREADS == 0 || gch[it] < G::COB) sgs[lt + it * G::LTHREADS] = sgt[it];
+        }
+        for (int p = 0; p < G::PW; ++p) __syncthreads();
     } else {
+        double4v tot[KS];
+#pragma unroll
+        for (int j = 0; j < KS; ++j) tot[j] = double4v{0.0, 0.0, 0.0, 0.0};
+        errs[0] = errs[64] = make_double2(0.0, 0.0);
         __syncthreads();
         __syncthreads();
+        int n0, h0, w0;
+        place(0, n0, h0, w0);
         for (int i = 0; i < mine; ++i) {
-            if (__builtin_amdgcn_readfirstlane((int)flags[i & 3]) == 0) multiply(i);
-            else multiply_raw(i);
+            multiply(i, h0, tot);
+            if ((w0 += G::TW) >= tilesW * G::TW) {
+                w0 = 0;
+                if ((h0 += G::TH) >= tilesH * G::TH) h0 = 0;
+            }
             __syncthreads();
         }
         if (mine & 1) __syncthreads();
-    }
-
-    // ---- fold the waves that shared a tile's steps and put the block in the order of the slab, through LDS ----
-    double *const out = reinterpret_cast<double *>(cells), *const sgs = out + G::OUT;
-    sgt += __shfl_xor(sgt, 16, 64);   // the four lanes that held the channel's strips
-    sgt += __shfl_xor(sgt, 32, 64);
-    for (int p = 0; p < G::PW; ++p) {
-        if (!loader && pw == p) {
+        // a wave's rows and columns of KS taps
+        const double err[4] = {errs[0].x, errs[0].y, errs[64].x, errs[64].y};
+        double col_err = 0.0, col_res = 0.0;
+        bool fine = true;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                double *o = out + ((mb * 16 + 4 * lk + e) * G::CIB + nb * 16 + l16) * G::KK + ti * KS;
+        for (int e = 0; e < 4; ++e) {
+            const double row_err = KS * err[e];
+            double row_res = 0.0;
 #pragma unroll
-                for (int j = 0; j < KS; ++j) o[j] = p == 0 ? tot[j][e] : o[j] + tot[j][e];
-            }
-            if (ti == 0 && nb == 0 && lane < 16) sgs[mb * 16 + lane] = p == 0 ? sgt : sgs[mb * 16 + lane] + sgt;
+            for (int j = 0; j < KS; ++j) row_res = fma(tot[j][e], tot[j][e], row_res);
+            col_err += row_err;
+            col_res += row_res;
+            fine = fine && i8_fine(i8_row_sum(row_err), i8_row_sum(row_res));
         }
-        __syncthreads();
+#pragma unroll
+        for (int d = 16; d < 64; d <<= 1) {
+            col_err += __shfl_xor(col_err, d, 64);
+            col_res += __shfl_xor(col_res, d, 64);
+        }
+        if (!fine || !i8_fine(col_err, col_res)) *flag = 1;
+        if (again()) {
+#pragma unroll
+            for (int j = 0; j < KS; ++j) tot[j] = double4v{0.0, 0.0, 0.0, 0.0};
+            __syncthreads();
+            __syncthreads();
+            for (int i = 0; i < mine; ++i) {
+                multiply_raw(i, tot);
+                __syncthreads();
+            }
+            if (mine & 1) __syncthreads();
+            __syncthreads();
+        }
+        // ---- fold the waves that shared a tile's steps and put the block in the order of the slab, through LDS ----
+        for (int p = 0; p < G::PW; ++p) {
+            if (pw == p) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    double *o = out + ((mb * 16 + 4 * lk + e) * G::CIB + nb * 16 + l16) * G::KK + ti * KS;
+#pragma unroll
+                    for (int j = 0; j < KS; ++j) o[j] = p == 0 ? tot[j][e] : o[j] + tot[j][e];
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (blockIdx.z == 0 && tid < min(G::COB, Co - co_blk)) {   // a channel's sums of gy are those of TH * QW units in a row
+        double sum = 0.0;
+        for (int u = 0; u < G::TH * QW; ++u) sum += sgs[tid * (G::TH * QW) + u];
+        sgpart[(size_t)blockIdx.x * Co + co_blk + tid] = sum;
     }
     const int K = Ci * G::KK, kcols = min(G::CIB, Ci - ci_blk) * G::KK;
     double *dst = part + ((size_t)blockIdx.x * Co + co_blk) * K + (size_t)ci_blk * G::KK;
     for (int c = 0; c < min(G::COB, Co - co_blk); ++c)
         for (int k = tid; k < kcols; k += G::NTHREADS) dst[(size_t)c * K + k] = out[c * (G::CIB * G::KK) + k];
-    if (blockIdx.z == 0 && tid < min(G::COB, Co - co_blk)) sgpart[(size_t)blockIdx.x * Co + co_blk + tid] = sgs[tid];
 }
 
 // ---------------------------------------------------------------------------
 // Single taps: gw[co,ci] = sum_pos x[ci,pos] gy[co,pos] over the positions of all planes in a row (so planes of any size fill the
-// tiles), and the column matrices' gW, whose rows are such planes.  The same fixed point and digits.  A tile is 128 positions; the four
-// digits that share a cell are 32 positions apart, so that a thread's four loads are each part of a 128-byte line that eight threads
-// read, and those eight threads hold a channel's tile: its largest value needs no exchange with other waves, and a thread converts a unit
-// as soon as it has arrived and asks for the same unit of the next tile.  Each multiplying wave owns 16 MT x 16 NT results.  A tile
-// with a value that is not finite is worked out in fp64 from memory.
+// tiles).  The same fixed point and digits.  A tile is 128 positions; the four digits that share a cell are 32 positions apart, so that
+// a thread's four loads are each part of a line that eight threads read, and those eight threads hold a channel's tile: its largest
+// value needs no exchange with other waves, and a thread converts a unit as soon as it has arrived and asks for the same unit of
+// the next tile.  Each multiplying wave owns 16 MT x 16 NT results.
 // ---------------------------------------------------------------------------
 template <int MT_, int NT_, int MB_, int NB_, int LWAVES_, int MINWAVES_>
 struct GwI8RowCfg {
@@ -489,7 +633,9 @@ struct GwI8RowCfg {
     static constexpr int MWAVES = MB * NB, NTHREADS = 64 * (MWAVES + LWAVES), LTHREADS = 64 * LWAVES;
     static constexpr int CELLS = TP / 4, PLANE = 4 * CELLS + 4;      // cells per digit, per channel (channels start four banks apart)
     static constexpr int UNITS = ROWS * 8, ITER = ceil_div(UNITS, LTHREADS), STEPS = TP / 64;
-    static constexpr int TILE_WORDS = ROWS * PLANE, EX0 = 2 * TILE_WORDS, COEF0 = round_up(EX0 + 2 * ROWS + 4, 4), LDS_BYTES = COEF0 * 4;
+    static constexpr int TILE_WORDS = ROWS * PLANE, EX0 = 2 * TILE_WORDS;
+    static constexpr int SM0 = EX0 + 2 * ROWS, FLAG0 = SM0 + 2 * ROWS;
+    static constexpr int ERR0 = round_up(FLAG0 + 1, 4), LDS_BYTES = (ERR0 + 64 * MWAVES * NT * 8) * 4;   // (a wave's first row of tiles has its error sums in LDS)
     static_assert(LDS_BYTES <= 160 * 1024 && NTHREADS <= 1024 && LTHREADS % 8 == 0, "workgroup limits");
 };
 
@@ -501,12 +647,14 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
     constexpr int MT = G::MT, NT = G::NT;
     constexpr unsigned E = sizeof(bf16_t);
     extern __shared__ __align__(16) int cells[];
-    int *const ex = cells + G::EX0, *const flags = ex + 2 * G::ROWS;   // the channels' exponents of two tiles; a flag for each of four
+    // the channels' exponents in two tiles (0: nothing but zeros), how many of their values were rounded; whether the digits will not do
+    int *const ex = cells + G::EX0, *const sm = cells + G::SM0, *const flag = cells + G::FLAG0;
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
     const int co_blk = blockIdx.y * G::COB, ci_blk = blockIdx.z * G::CIB;
     const long P = (long)N * L;
-    const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, tile0 = blockIdx.x * each, mine = min(each, ntiles - tile0);
+    const int each = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x, mine = min(each, ntiles - (int)blockIdx.x * each);
+    int tile0 = blockIdx.x * each;
     const double rL = 1.0 / L;
     // image and place in its plane of position p
     auto place = [&](const long p, int &n, int &l) __attribute__((always_inline)) {
@@ -515,25 +663,22 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
         if (l < 0) { l += L; --n; }
         if (l >= L) { l -= L; ++n; }
     };
-    if (tid < 4) flags[tid] = 0;
+    if (tid == 0) *flag = 0;
     __syncthreads();
 
-    double tot[MT][NT][4], sgt[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        sgt[m] = 0.0;
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) tot[m][n][e] = 0.0;
-    }
     const int mb = wave % G::MB, nb = wave / G::MB % G::NB;
-    const bool sg_wave = nb == 0 && blockIdx.z == 0;
-
+    auto again = [&]() __attribute__((always_inline)) {
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(*flag) == 0) return false;
+        __syncthreads();
+        return true;
+    };
     if (wave >= G::MWAVES) {
         // ---- the loading waves: unit u = thread's channel row0 + it * (LTHREADS / 8), columns 4 * (u % 8) .. + 3 of each 32 ----
         const int lt = tid - 64 * G::MWAVES, col = 4 * (lt & 7), row0 = lt >> 3;
         float4 v[G::ITER][4];
+        constexpr int GITER = ceil_div(G::COB, G::LTHREADS / 8);   // its units from here on are of x
+        double sgt[GITER];   // sums of the gy rows' values
         // Offsets (bytes) of the thread's four groups from the first image of the tile that is being asked for, and of its channels; those
         // that do not exist push the sum beyond every buffer, which ends below 2^31.
         constexpr unsigned NO_GROUP = 0x80000000u, NO_ROW = 0x7fffffffu;
@@ -584,10 +729,9 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
             one(is_x ? x : gy, v[it]);
         };
         static_assert(G::COB % 8 == 0, "eight rows of a wave are of one tensor");
-        auto turn = [&](const int i) __attribute__((always_inline)) {   // writes tile i, asks for tile i + 1
+        auto turn = [&](const int i, auto with_values) __attribute__((always_inline)) {   // writes tile i, asks for tile i + 1
             int *const tile = cells + (i & 1) * G::TILE_WORDS;
             aim(i + 1);
-            if (tid == 64 * G::MWAVES) flags[(i + 2) & 3] = 0;
 #pragma unroll
             for (int it = 0; it < G::ITER; ++it) {
                 const int row = row0 + it * (G::LTHREADS / 8);
@@ -600,37 +744,69 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
                 u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
                 u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x141, 0xF, 0xF, true));   // row_half_mirror
                 const int e = i8_exponent(u);
+                if (it < GITER && blockIdx.z == 0 && wrow0 + it * (G::LTHREADS / 8) < G::COB) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) sgt[it] += ((double)v[it][k].x + (double)v[it][k].y) + ((double)v[it][k].z + (double)v[it][k].w);
+                }
                 if (ok) {
-                    if ((lt & 7) == 0) {
-                        ex[(i & 1) * G::ROWS + row] = e;
-                        if (e >= 255) flags[i & 3] = 1;
+                    int rounded = i8_put4<decltype(with_values)::value>(v[it], i8_scale(min(e, 254)), tile + row * G::PLANE + col, G::CELLS);
+                    if (__builtin_amdgcn_ballot_w64(rounded)) {   // over the eight lanes of the channel
+                        rounded += __builtin_amdgcn_update_dpp(0, rounded, 0xB1, 0xF, 0xF, true);
+                        rounded += __builtin_amdgcn_update_dpp(0, rounded, 0x4E, 0xF, 0xF, true);
+                        rounded += __builtin_amdgcn_update_dpp(0, rounded, 0x141, 0xF, 0xF, true);
                     }
-                    i8_put4(v[it], i8_scale(min(e, 254)), false, tile + row * G::PLANE + col, G::CELLS);
+                    if ((lt & 7) == 0) {
+                        ex[(i & 1) * G::ROWS + row] = u ? e : 0;
+                        sm[(i & 1) * G::ROWS + row] = rounded;
+                        if (e >= 255) *flag = 1;
+                    }
                 }
                 ask(it);
             }
         };
-        aim(0);
+        auto pass = [&](auto with_values) __attribute__((always_inline)) {
+            asm volatile("" : "+s"(tile0));   // (no offset of the first pass is kept in a register for the second)
 #pragma unroll
-        for (int it = 0; it < G::ITER; ++it) ask(it);
-        turn(0);
-        __syncthreads();
-        for (int i = 0; i < mine; ++i) {
-            if (i + 1 < mine) turn(i + 1);
+            for (int it = 0; it < GITER; ++it) sgt[it] = 0.0;
+            aim(0);
+#pragma unroll
+            for (int it = 0; it < G::ITER; ++it) ask(it);
+            turn(0, with_values);
             __syncthreads();
+            for (int i = 0; i < mine; ++i) {
+                if (i + 1 < mine) turn(i + 1, with_values);
+                __syncthreads();
+            }
+        };
+        pass(std::false_type{});
+        if (again()) {
+            pass(std::true_type{});
+            __syncthreads();
+        }
+        if (blockIdx.z == 0) {
+#pragma unroll
+            for (int it = 0; it < GITER; ++it) {
+                const int row = row0 + it * (G::LTHREADS / 8);
+                double sum = sgt[it];   // over the eight lanes of the channel
+#pragma unroll
+                for (int d = 1; d < 8; d <<= 1) sum += __shfl_xor(sum, d, 64);
+                if ((lt & 7) == 0 && row < G::COB && co_blk + row < Co) sgpart[(size_t)blockIdx.x * Co + co_blk + row] = sum;
+            }
         }
     } else {
         // ---- the multiplying waves ----
         const int goff = (mb * MT * 16 + l16) * G::PLANE + 4 * lk, xoff = (G::COB + nb * NT * 16 + l16) * G::PLANE + 4 * lk;
+        double4v tot[MT][NT], err[MT][NT];   // results and the squares of their errors (as in the kernel above; those of m = 0 in LDS)
+        double2 *const errs = reinterpret_cast<double2 *>(cells + G::ERR0) + wave * (128 * NT) + lane;
         auto multiply = [&](const int i) __attribute__((always_inline)) {
-            const int *const tile = cells + (i & 1) * G::TILE_WORDS, *const exs = ex + (i & 1) * G::ROWS;
+            const int *const tile = cells + (i & 1) * G::TILE_WORDS, *const exs = ex + (i & 1) * G::ROWS, *const sms = sm + (i & 1) * G::ROWS;
             int4v acc[MT][NT][5], a[MT][4], b[2][NT];
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
-                    for (int s = 0; s < 5; ++s) acc[m][n][s] = s != 3 ? int4v{0, 0, 0, 0} : int4v{128, 128, 128, 128};
+                    for (int s = 0; s < 5; ++s) acc[m][n][s] = int4v{0, 0, 0, 0};
             auto ask_a = [&](const int st, const int d) {
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
@@ -661,71 +837,111 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
                 __builtin_amdgcn_sched_barrier(0);
             }
             double sx[NT];
+            int xs[NT];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) sx[n] = i8_unit(exs[G::COB + (nb * NT + n) * 16 + l16]) * 4294967296.0;
+            for (int n = 0; n < NT; ++n) {
+                const int xe = exs[G::COB + (nb * NT + n) * 16 + l16];
+                sx[n] = xe ? i8_unit(xe) * 4294967296.0 : 0.0;
+                xs[n] = kRounded * sms[G::COB + (nb * NT + n) * 16 + l16] + kLeftOut;
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const int4v ge = *reinterpret_cast<const int4v *>(exs + (mb * MT + m) * 16 + 4 * lk),
+                            gs = *reinterpret_cast<const int4v *>(sms + (mb * MT + m) * 16 + 4 * lk);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double sg = ge[e] ? i8_unit(ge[e]) : 0.0;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        const double sc = sx[n] * sg;
+                        tot[m][n][e] = fma(i8_product(acc[m][n][0][e], acc[m][n][1][e], acc[m][n][2][e], acc[m][n][3][e], acc[m][n][4][e]),
+                                           sc, tot[m][n][e]);
+                        const double more = (sc * sc) * (double)(kRounded * gs[e] + xs[n]);
+                        if (m == 0) {
+                            double *const at = reinterpret_cast<double *>(errs + 64 * (2 * n + e / 2)) + e % 2;
+                            *at += more;
+                        } else {
+                            err[m][n][e] += more;
+                        }
+                    }
+                }
+            }
+        };
+        auto multiply_raw = [&](const int i) __attribute__((always_inline)) {   // a tile's values instead of digits: fp64, positions 32 apart four at a time
+            const int *const tile = cells + (i & 1) * G::TILE_WORDS + lk * G::CELLS;
+            const int goff = (mb * MT * 16 + i8_fp64_row(l16)) * G::PLANE, xoff = (G::COB + nb * NT * 16 + l16) * G::PLANE;
+#pragma unroll 1
+            for (int c = 0; c < G::CELLS; c += 4) {
+                float4 g[MT];
+#pragma unroll
+                for (int m = 0; m < MT; ++m) g[m] = *reinterpret_cast<const float4 *>(tile + goff + m * 16 * G::PLANE + c);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    const float4 x = *reinterpret_cast<const float4 *>(tile + xoff + n * 16 * G::PLANE + c);
+                    const float xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        const float gs[4] = {g[m].x, g[m].y, g[m].z, g[m].w};
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) tot[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)gs[u], (double)xs[u], tot[m][n], 0, 0, 0);
+                    }
+                }
+            }
+        };
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                tot[m][n] = err[m][n] = double4v{0.0, 0.0, 0.0, 0.0};
+                if (m == 0) errs[128 * n] = errs[128 * n + 64] = make_double2(0.0, 0.0);
+            }
+        __syncthreads();
+        for (int i = 0; i < mine; ++i) {
+            multiply(i);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const double2 a = errs[128 * n], b = errs[128 * n + 64];
+            err[0][n] = double4v{a.x, a.y, b.x, b.y};
+        }
+        bool fine = true;
+        double col_err[NT] = {}, col_res[NT] = {};
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                double row_err = 0.0, row_res = 0.0;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    const double r2 = tot[m][n][e] * tot[m][n][e];
+                    row_err += err[m][n][e];
+                    row_res += r2;
+                    col_err[n] += err[m][n][e];
+                    col_res[n] += r2;
+                }
+                fine = fine && i8_fine(i8_row_sum(row_err), i8_row_sum(row_res));
+            }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+#pragma unroll
+            for (int d = 16; d < 64; d <<= 1) {
+                col_err[n] += __shfl_xor(col_err[n], d, 64);
+                col_res[n] += __shfl_xor(col_res[n], d, 64);
+            }
+            fine = fine && i8_fine(col_err[n], col_res[n]);
+        }
+        if (!fine) *flag = 1;
+        if (again()) {
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const double sg = i8_unit(exs[(mb * MT + m) * 16 + 4 * lk + e]);
-#pragma unroll
-                    for (int n = 0; n < NT; ++n)
-                        tot[m][n][e] = fma(i8_product(acc[m][n][0][e], acc[m][n][1][e], acc[m][n][2][e], acc[m][n][3][e], acc[m][n][4][e]),
-                                           sx[n] * sg, tot[m][n][e]);
-                }
-            if (sg_wave) {
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    int sd[4] = {0, 0, 0, 0};
-#pragma unroll
-                    for (int st = 0; st < G::STEPS; ++st)
-#pragma unroll
-                        for (int d = 0; d < 4; ++d) {
-                            const int4v g = *reinterpret_cast<const int4v *>(tile + goff + m * 16 * G::PLANE + d * G::CELLS + 16 * st);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) sd[d] = __builtin_amdgcn_sdot4(g[e], 0x01010101, sd[d], false);
-                        }
-                    sgt[m] = fma(i8_sum(sd[0], sd[1], sd[2], sd[3]), i8_unit(exs[(mb * MT + m) * 16 + l16]), sgt[m]);
-                }
+                for (int n = 0; n < NT; ++n) tot[m][n] = double4v{0.0, 0.0, 0.0, 0.0};
+            __syncthreads();
+            for (int i = 0; i < mine; ++i) {
+                multiply_raw(i);
+                __syncthreads();
             }
-        };
-        auto multiply_from_memory = [&](const int i) {
-            for (int q = 0; q < G::TP; ++q) {
-                const long p = (long)(tile0 + i) * G::TP + q;
-                if (p >= P) break;
-                int n, l;
-                place(p, n, l);
-                auto value = [&](const bf16_t *t, const int C, const int ch) { return ch < C ? (double)ldf(t + ((size_t)n * C + ch) * L + l) : 0.0; };
-                auto grad = [&](const int r) {
-                    const double g = value(gy, Co, co_blk + r);
-                    return g;
-                };
-#pragma unroll 1
-                for (int m = 0; m < MT; ++m) {
-#pragma unroll 1
-                    for (int e = 0; e < 4; ++e) {
-                        const double g = grad((mb * MT + m) * 16 + 4 * lk + e);
-#pragma unroll
-                        for (int mm = 0; mm < MT; ++mm)
-#pragma unroll
-                            for (int ee = 0; ee < 4; ++ee)
-#pragma unroll
-                                for (int c = 0; c < NT; ++c)
-                                    if (mm == m && ee == e) tot[mm][c][ee] = fma(value(x, Ci, ci_blk + (nb * NT + c) * 16 + l16), g, tot[mm][c][ee]);
-                    }
-                    if (sg_wave && lk == 0) {
-                        const double g = grad((mb * MT + m) * 16 + l16);
-#pragma unroll
-                        for (int mm = 0; mm < MT; ++mm)
-                            if (mm == m) sgt[mm] += g;
-                    }
-                }
-            }
-        };
-        __syncthreads();
-        for (int i = 0; i < mine; ++i) {
-            if (__builtin_amdgcn_readfirstlane(flags[i & 3]) == 0) multiply(i);
-            else multiply_from_memory(i);
             __syncthreads();
         }
         // ---- straight to the slab: sixteen lanes hold sixteen columns in a row ----
@@ -741,10 +957,6 @@ __global__ __launch_bounds__(G::NTHREADS, G::MINWAVES) void grad_w_i8_row_kernel
                     if (co < Co && ci < Ci) dst[(size_t)co * Ci + ci] = tot[m][n][e];
                 }
             }
-            sgt[m] += __shfl_xor(sgt[m], 16, 64);   // the four lanes that held the channel's cells
-            sgt[m] += __shfl_xor(sgt[m], 32, 64);
-            const int co = co_blk + (mb * MT + m) * 16 + lane;
-            if (sg_wave && lane < 16 && co < Co) sgpart[(size_t)blockIdx.x * Co + co] = sgt[m];
         }
     }
 }
@@ -762,10 +974,9 @@ using Gi5w16 = GwI8Cfg<5, 4, 16, 1, 1, 1, 3, 2>;
 using Gi5w8  = GwI8Cfg<5, 8, 8, 1, 1, 1, 3, 2>;
 
 // Single taps: 64 x 64 and, for few output channels, 32 x 96, each of 16 (14) waves on a CU of its own.  Whole calls with their
-// finalizing and scaling kernels, fp64 matrix cores -> this: 1024 -> 256 @14x14, 64 images 146 -> 82 us (bfloat16 storage 168 -> 88),
-// 128 -> 512 @28x28, 32 images 90 -> 48, 256 -> 64 @56x56, 64 images 148 -> 82, 512 -> 2048 @7x7, 64 images 177 -> 148; against the
-// plain kernel's fp32 runs 100 -> 48 @32x32 37 -> 23, 48 -> 200 72 -> 33.  Bound by the issue of both kinds of waves together: of the
-// first layer's 82 us the multiplying waves alone take 59, the loading waves alone 60, and without their loads both 80.
+// finalizing and scaling kernels, fp64 matrix cores -> this: 128 -> 512 @28x28, 32 images 98 -> 55 us, 128 -> 128 @28x28, 16 images 33 -> 18.
+// Bound by the issue of both kinds of waves together (1024 -> 256 @14x14, 64 images, of 82 us the multiplying waves alone took 59, the loading
+// waves alone 60, and without their loads both 80).
 //                           MT NT MB NB loading waves, waves per SIMD
 using GiRow  = GwI8RowCfg<2, 1, 2, 4, 8, 4>;
 using GiRowN = GwI8RowCfg<2, 1, 1, 6, 8, 4>;
@@ -825,17 +1036,14 @@ static bool plan_i8_rows(const ConvDims &d, GradWMfmaPlan &p) {
 }
 
 // Whether it takes a layer.  Against the fp64 matrix kernel it has some more to set up (half a workgroup's waves load, digits, four
-// images at a time), 1-2 us, and a fifth to a half of the matrix time; us, fp64 -> this, layers of 4..64 images:
-//   3x3, multiply-adds with the channels filled up to 16: 1.5e8 14.5 -> 16.1, 2.3e8 19.9 -> 19.6 and 18.6 -> 16.7, 3e8 29.1 -> 18.8,
-//   6e8 30.4 -> 21.6, 1.9e9 92.7 -> 42.4, 1.9e10 (128 -> 128 @32x32, 128 images) 690 -> 272;
-//   5x5: maps wider than 8, 7e6 24.1 -> 17.7 to 2.6e9 147 -> 59 (the fp64 kernel's 25-tap blocks start late); 8x8, 1e8 19.1 -> 19.2,
-//   2e8 22.4 -> 20.8, 4e8 30.8 -> 24.3.
-//   1x1, from 64 channels on both sides: 64 -> 64 @8x8, 16 images 13.4 -> 11.6, 128 -> 128 @28x28, 16 images 31 -> 15, 256 -> 512 90 -> 44;
-//   fewer channels, planes of whole groups of four: 160 -> 48 @28x28, 16 images (9.6e7) 12.5 -> 14.0, 64 images (3.9e8) 48 -> 23,
-//   512 -> 32, 16 images (2.1e8) 23.3 -> 16.8, 1024 -> 16 (bfloat16) 48 -> 58; other planes (15x15): 48 -> 12, 2 images 11.6 -> 12.2,
-//   16 images 21.0 -> 13.2.
-// Three channels on wide maps have a block of 32 columns there (stem, 256 images @32x32: 17 against 28).  Fewer than four images
-// would leave digits empty.
+// images at a time), 2-3 us, and a fifth to a half of the matrix time; us, other kernel -> this, bfloat16:
+//   3x3, multiply-adds with the channels filled up to 16: 2.26e8 (6 images) 20.1 -> 20.8, 2.39e8 (5 images) 31.1 -> 23.4 and 25.4 -> 21.5, 2.6e8 (9 images)
+//   25.6 -> 22.3, 2.65e8 (7, 8 images) 20.7 -> 20.8 and 21.7 -> 22.5, 2.7e8 38.1 -> 28.5, 3e8 21.8 -> 20.3, 5.8e8 (5 images) 36.6 -> 31.2;
+//   5x5: maps wider than 8, 4e6 24.9 -> 21.0 to 2.6e9 147 -> 59 (the fp64 kernel's 25-tap blocks start late); 8x8, 1.5e8 and up;
+//   1x1, from 64 channels on both sides: 64 -> 64 @2x2, 64 images 14.5 -> 11.1, @8x8, 16 images 14.4 -> 11.4, 2048 -> 512 @14x14, 1 image 34.9 -> 25.4;
+//   fewer channels, planes of whole groups of four: 160 -> 48 @28x28, 64 images (3.9e8) 32.5 -> 26.5; other planes, which the plain kernel reads element by
+//   element: 8 -> 8 @15x15, 64 images 27.8 -> 15.1, 16 -> 64 25.7 -> 15.1, 24 -> 512 @25x25, 16 images 34.9 -> 25.3, 1024 -> 16 @15x15, 64 images 86 -> 33.
+// Three channels on wide maps have a block of 32 columns there (stem).  Fewer than four images would leave digits empty.
 bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
     if (d.stride != 1 || d.kh != d.kw || d.pad != d.kh / 2) return false;
     if (d.kh == 1) {
@@ -850,7 +1058,7 @@ bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
     if ((long)d.Ci * d.H * d.W > kBufferImage || (long)d.Co * d.H * d.W > kBufferImage) return false;
     if (d.kh == 3 && d.Ci * 9 <= 32 && d.W > 16) return false;
     const double macs = (double)round_up(d.Ci, 16) * round_up(d.Co, 16) * d.kh * d.kw * d.N * d.H * d.W;
-    if (macs < (d.kh == 3 ? 2.2e8 : d.W > 8 ? 0.0 : 1.5e8)) return false;
+    if (macs < (d.kh == 3 ? 2.3e8 : d.W > 8 ? 0.0 : 1.5e8)) return false;
     // the tile that needs fewest; rows in one piece load whole lines and no halo columns, which is worth a seventh
     const int n32 = ceil_div(d.H, 2) * ceil_div(d.W, 32), n16 = ceil_div(d.H, 4) * ceil_div(d.W, 16), n8 = ceil_div(d.H, 8) * ceil_div(d.W, 8);
     const int shape = 7 * n32 <= 7 * n16 && 7 * n32 <= 8 * n8 ? 0 : 7 * n16 <= 8 * n8 ? 1 : 2;
@@ -865,14 +1073,11 @@ bool plan_grad_w_i8(const ConvDims &d, GradWMfmaPlan &p) {
         }
         return true;
     }
-    if (d.kh == 5) {
-        p.variant = 28 + shape;
-        if (shape == 0) plan_i8<Gi5w32>(d, p);
-        else if (shape == 1) plan_i8<Gi5w16>(d, p);
-        else plan_i8<Gi5w8>(d, p);
-        return true;
-    }
-    return false;
+    p.variant = 28 + shape;
+    if (shape == 0) plan_i8<Gi5w32>(d, p);
+    else if (shape == 1) plan_i8<Gi5w16>(d, p);
+    else plan_i8<Gi5w8>(d, p);
+    return true;
 }
 
 int launch_grad_w_i8(const bf16_t *gy, const bf16_t *x, double *part, double *sgpart, const ConvDims &d, const GradWMfmaPlan &p, hipStream_t s) {

@@ -160,7 +160,10 @@ ADDER_API int adder_conv2d_bwd_add_f32(const float *gy, const float *x, const fl
 /* Optional reduced-storage mode: the activations and their gradients (x, y, gy, gx) are stored as bfloat16 (the
  * upper half of an fp32, rounded to nearest even on the way out) and take half the HBM traffic and half the
  * activation memory; weights and weight gradients stay fp32, and so do the sums of y and gx; those of gw are carried in
- * fp64 (fp32 runs of at most 64 terms in the kernels for narrow 1x1 layers and for the shapes without a tiled kernel).  The reference computes in fp32 only (adder.cu:310-318 hard-codes
+ * fp64 (fp32 runs of at most 64 terms in the kernels for narrow 1x1 layers and for the shapes without a tiled kernel).  Large stride-1
+ * layers multiply x and gy as 32-bit fixed point relative to the largest of a channel's neighbouring values, in which eight significant bits are exact
+ * down to 2^-22 of it; where smaller values matter -- their error's estimate above 2^-24 of a row's or column's root mean square --
+ * and where a value is infinite or not a number, they multiply in fp64 instead.  The reference computes in fp32 only (adder.cu:310-318 hard-codes
  * data<float>()), so these have no counterpart there and are never the default.  Same dimensions, semantics, eta
  * and workspace (adder_conv2d_bwd_workspace_bytes) as adder_conv2d_fwd_f32 / adder_conv2d_bwd_f32, and the same
  * kernels and tile shapes. */
@@ -179,8 +182,8 @@ ADDER_API int adder_conv2d_bwd_bf16(const adder_bf16 *gy, const adder_bf16 *x, c
  * the reference, whose backward takes every buffer from torch's allocator (adder.py:66-67).  The partial slabs
  * and norm partials live in a buffer of ADDER_NOALLOC_SCRATCH_BYTES that is part of the library's device image
  * (every GPU the library runs on holds one copy until the process ends); the call allocates and frees nothing.
- * Same arguments and results as adder_conv2d_bwd_f32 without ws / ws_bytes.  Layers whose
- * adder_conv2d_bwd_workspace_bytes exceeds ADDER_NOALLOC_SCRATCH_BYTES are refused with ADDER_ERR_WORKSPACE
+ * Same arguments and results as adder_conv2d_bwd_f32 without ws / ws_bytes.  Layers that need more than ADDER_NOALLOC_SCRATCH_BYTES of it
+ * (adder_conv2d_bwd_workspace_bytes, where the bfloat16 kernels do not need still more) are refused with ADDER_ERR_WORKSPACE
  * before anything is launched (every ResNet-20 layer at batch 256 fits) -- except 5x5 layers, which then take the general
  * kernel, whose sums have another order.  All calls on one GPU share that
  * GPU's buffer: calls that overlap in time on one GPU (different streams, or threads) race; serialise them.

@@ -168,10 +168,15 @@ def test_column_matrices(gpu, case):
     assert bool(((gw.cpu().double() - 2.0 - want).abs() <= bound).all())
 
 
-def _check_each(got, want, x, gy, smallest=0.0):
-    """Products that are exact and sums in fp64, element by element: the rounding of the result and 2^-45 of the sum of magnitudes.
-    ``smallest``: the rounding of results below the normal floats."""
-    k = want.shape[2]
+def _check_each(run, x, w, gy, storage, smallest=0.0):
+    """Exact products and sums in fp64, element by element: the rounding of the result and 2^-45 of the sum of magnitudes.  bfloat16 storage, whose
+    kernels hold the deviation of the digits' error to 2^-24 of the root mean square of a block's rows and columns: six times that of
+    the largest of a row and of a column.  ``smallest``: the rounding of results below the normal floats."""
+    x, gy = x.to(storage).float(), gy.to(storage).float()
+    k = w.shape[2]
+    got, want = run(x.to(storage), w, gy.to(storage)), c_oracle.conv2d_grad_w(gy, x, w, 1, k // 2)
+    if storage == torch.bfloat16:
+        smallest = smallest + 6 * 2.0 ** -24 * torch.minimum(want.abs().amax((1, 2, 3), keepdim=True), want.abs().amax((0, 2, 3), keepdim=True))
     sums = c_oracle.conv2d_grad_w(gy.abs(), x.abs(), torch.zeros(want.shape), 1, k // 2)
     bound = 2.0 ** -24 * want.abs() + 2.0 ** -45 * sums + smallest
     err = (got.double() - want).abs()
@@ -204,47 +209,50 @@ def _large_opposite_zeros(case, which, size):
     return x, torch.zeros_like(w), gy   # (no w: the sum of a gy that is large is large itself)
 
 
-WIDE = [CASES[3], CASES[8], CASES[13], CASES[16], CASES[20]]   # fp64 products in float32 storage
+def _run(gpu):
+    return lambda x, w, gy: _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu))
+
+
+# tiles of 16 x 4, 8 x 8 and 32 x 2, 5x5, both blocks of single taps; float32 storage: wide enough for fp64 products (the others' are float32)
+WIDE = [CASES[3], CASES[8], CASES[13], CASES[16], CASES[20]]
+STORED = [(c, torch.float32) for c in WIDE] + [(c, torch.bfloat16) for c in (*WIDE, CASES[2], CASES[25])]
+stored = pytest.mark.parametrize("case,storage", STORED, ids=str)
 
 
 @pytest.mark.parametrize("size", [1e5, 1e30])
 @pytest.mark.parametrize("which", ["x", "gy", "both"])
-@pytest.mark.parametrize("case", WIDE, ids=str)
-def test_large_values_opposite_zeros(gpu, case, which, size):
-    x, w, gy = _large_opposite_zeros(case, which, size)
-    _check_each(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), c_oracle.conv2d_grad_w(gy, x, w, 1, case[5] // 2), x, gy)
+@stored
+def test_large_values_opposite_zeros(gpu, case, storage, which, size):
+    _check_each(_run(gpu), *_large_opposite_zeros(case, which, size), storage)
 
 
 @pytest.mark.parametrize("share", [0.1, 0.001])
-@pytest.mark.parametrize("case", WIDE, ids=str)
-def test_sparse_gradients(gpu, case, share):
+@stored
+def test_sparse_gradients(gpu, case, storage, share):
     x, w, gy = _data(case, 11)
-    gy, w = gy * (torch.rand(gy.shape, generator=torch.Generator().manual_seed(12)) < share), torch.zeros_like(w)
-    _check_each(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), c_oracle.conv2d_grad_w(gy, x, w, 1, case[5] // 2), x, gy)
+    gy = gy * (torch.rand(gy.shape, generator=torch.Generator().manual_seed(12)) < share)
+    _check_each(_run(gpu), x, torch.zeros_like(w), gy, storage)
 
 
 # products that are ordinary numbers of factors that are not: gradients near the smallest float and below the normal ones
 @pytest.mark.parametrize("up,down", [(1.0, 1e-34), (1e10, 1e-39), (1e38, 1e-38)])
-@pytest.mark.parametrize("case", WIDE, ids=str)
-def test_tiny_and_huge_factors(gpu, case, up, down):
+@stored
+def test_tiny_and_huge_factors(gpu, case, storage, up, down):
     x, w, gy = _data(case, 13)
-    x, gy, w = x.clamp(max=3.0) * up, gy * down, torch.zeros_like(w)
-    _check_each(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), c_oracle.conv2d_grad_w(gy, x, w, 1, case[5] // 2), x, gy, 2.0 ** -149)
+    _check_each(_run(gpu), x.clamp(max=3.0) * up, torch.zeros_like(w), gy * down, storage, 2.0 ** -149)
 
 
 # both factors log-normal of a wide spread, and the sum of gy, which w multiplies, small against its terms
-@pytest.mark.parametrize("case", WIDE, ids=str)
-def test_long_tails(gpu, case):
+@stored
+def test_long_tails(gpu, case, storage):
     x, w, gy = _data(case, 14)
     g = torch.Generator().manual_seed(15)
     x, gy = x * torch.exp(4.0 * torch.randn(x.shape, generator=g)), gy * torch.exp(4.0 * torch.randn(gy.shape, generator=g))
-    k = case[5]
-    none = torch.zeros_like(w)
-    _check_each(_grad_w(gpu, x.to(gpu), none.to(gpu), gy.to(gpu)), c_oracle.conv2d_grad_w(gy, x, none, 1, k // 2), x, gy)
-    x = torch.zeros_like(x)
-    want = c_oracle.conv2d_grad_w(gy, x, w, 1, k // 2)
+    _check_each(_run(gpu), x, torch.zeros_like(w), gy, storage)
+    x, gy = torch.zeros_like(x), gy.to(storage).float()
+    want = c_oracle.conv2d_grad_w(gy, x, w, 1, case[5] // 2)
     sums = gy.double().abs().sum((0, 2, 3))[:, None, None, None] * w.double().abs()
-    got = _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)).double()
+    got = _grad_w(gpu, x.to(gpu, storage), w.to(gpu), gy.to(gpu, storage)).double()
     assert bool(((got - want).abs() <= 2.0 ** -24 * want.abs() + 2.0 ** -45 * sums).all())
 
 
@@ -253,7 +261,10 @@ def test_column_matrix_with_large_values_opposite_zeros(gpu):
     Co, K, NL = 64, 576, 12100
     x, w, gy = _large_opposite_zeros((1, K, 1, NL, Co, 1), "x", 1e9)
     x[:, :, :, ::16], gy[:, :, :, ::16] = 1e9, 0.0
-    gw = torch.zeros(Co, K, device=gpu)
-    adder_cuda.ADDER_CONV_WEIGHT(gy.view(Co, NL).to(gpu), x.view(K, NL).to(gpu), w.view(Co, K).to(gpu), gw)
-    torch.cuda.synchronize()
-    _check_each(gw.cpu().view(Co, K, 1, 1), c_oracle.conv2d_grad_w(gy, x, w, 1, 0), x, gy)
+
+    def run(x, w, gy):
+        gw = torch.zeros(Co, K, device=gpu)
+        adder_cuda.ADDER_CONV_WEIGHT(gy.view(Co, NL).to(gpu), x.view(K, NL).to(gpu), w.view(Co, K).to(gpu), gw)
+        torch.cuda.synchronize()
+        return gw.cpu().view(Co, K, 1, 1)
+    _check_each(run, x, w, gy, torch.float32)
