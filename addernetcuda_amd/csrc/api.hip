@@ -251,6 +251,14 @@ int adder_conv2d_bwd_workspace_bytes(int N, int Ci, int H, int W, int Co, int kh
     return ADDER_OK;
 }
 
+int adder_conv2d_grad_w_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int bf16, int *kernel) {
+    if (!kernel) return ADDER_ERR_NULL_POINTER;
+    ConvDims d;
+    if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
+    *kernel = grad_w_kernel(d, bf16 != 0);
+    return ADDER_OK;
+}
+
 static int conv2d_bwd(const float *gy, const float *x, const float *w, const float *gx_add, float *gx, float *gw,
                       float eta, void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
                       int stride, int pad, void *stream, bool general = false);

@@ -269,6 +269,7 @@ int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, 
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
 size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false);   // of the storage type's kernels
+int grad_w_kernel(const ConvDims &d, bool bf16);                       // which of them, as in adder_conv2d_grad_w_kernel
 // The sums of the backward of the BatchNorm behind a layer, as the consumer's input-gradient kernel left them
 // ((C, slots, 2) floats -- a wave's fp32 totals: sum dz, sum dz * xhat), with what turns them into the four coefficients per channel.
 // A weight-gradient kernel that is given these instead of ready coefficients adds the slots itself (every

@@ -378,6 +378,10 @@ static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
     return (bytes + 255) & ~(size_t)255;
 }
 size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16) { return workspace_bytes_of(plan_grad_w(d, bf16), d); }
+int grad_w_kernel(const ConvDims &d, bool bf16) {
+    const GradWPlan p = plan_grad_w(d, bf16);
+    return p.variant == 2 ? p.mfma.variant : p.variant == 1 ? 100 : 0;
+}
 
 // bn_y with either bn_coef or sums.part: gy is the gradient dz of the output of the BatchNorm behind the layer and
 // the kernel forms the layer's own output gradient from it, leaving it in gy_out (nullable) on the way (matrix-core

@@ -20,6 +20,8 @@
 // over its share of the positions of every staged tile; PW waves split the positions, MW x NW waves
 // the (co, k) block of the workgroup; the waves are folded in fp64 through LDS at the end.
 // sum_pos gy is collected on the A fragments.  Partials: one fp64 (Co, K) slab per grid.x slot.
+// Positions of a tile beside the map are zeros of gy times x, so an x that is infinite or not a number within their reach makes its taps not a number.
+// (A flag per tile and a masked loop for such tiles cost every 3x3 layer 5-9 %: 128 -> 128 @32x32, 128 images 684 -> 746 us.)
 #include "common.hpp"
 #include "tile3x3.hpp"
 

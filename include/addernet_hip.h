@@ -132,6 +132,11 @@ ADDER_API int adder_plain_conv2d_fwd_f32(const float *x, const float *w, float *
 ADDER_API int adder_conv2d_bwd_workspace_bytes(int N, int Ci, int H, int W, int Co, int kh, int kw,
                                      int stride, int pad, size_t *bytes);
 
+/* Which kernel the weight gradient of the backward calls takes for the dimensions and aligned tensors in float (bf16 = 0) or bfloat16
+ * storage, in the dispatch's own numbers: 0 the general one, 100 the plain 1x1 one, 1..19 the fp64 ones, from 20 on those of fixed-point digits.
+ * Host code only; for tests that have to reach a certain kernel, and no promise that the numbers stay. */
+ADDER_API int adder_conv2d_grad_w_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int bf16, int *kernel);
+
 /* Backward of the layer.  Replaces adder.backward (adder.py:62-80), ADDER_BACKWARD
  * (adder_cuda.cpp:74-86, adder.cu:194-272, 404-465), the fold that autograd runs
  * after it and the Python-side scaling of adder.py:78.

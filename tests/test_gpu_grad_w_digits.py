@@ -1,10 +1,11 @@
 """The weight gradient of layers large enough for the 8-bit matrix cores (csrc/grad_w_i8.hip), which take them in bfloat16 storage, at the edges
-of its tiles; and what those kernels could lose and the fp64 products of float32 storage do not: small values beside large ones.
+of its tiles; and what fixed-point digits can lose: values far below the largest beside them, in both storage types.
 
-Bound: with e the unit of a channel's fixed point in a tile (2^-30 of its largest magnitude, within a factor of two) and 256 positions,
-the rounding of x costs at most 2^-31 max|x| * 16 ||gy||, i.e. 2^-27 ||x|| ||gy|| over the tile, that of gy the same, the digit products left
-out 2^-29 and the two roundings of digit sums 2^-28 each: below 2^-25 ||x_ci|| ||gy_co|| together, and over the tiles of a channel pair
-(Cauchy-Schwarz) against the norms of whole channels.  Plus the float32 rounding of the result."""
+Bound of ``_check``: 2^-25 ||x_ci|| ||gy_co|| beside the float32 rounding of the result.  fp64 products and the digits of values that they hold
+exactly stay far within; the plain 1x1 kernel's float32 runs have at most 64 terms, each rounded by 2^-24 of a sum that grows like the root of
+its terms' squares, so that a run is off by about 2^-24 of that, and the runs' errors add like their squares."""
+import ctypes
+
 import pytest
 import torch
 
@@ -15,21 +16,25 @@ pytestmark = pytest.mark.gpu
 
 # (N, Ci, H, W, Co, k): every tile shape and block, images not a multiple of four, channels around multiples of 16 and 32, maps that end
 # inside a tile, rows that are whole groups of four and rows that are not
-CASES = [(4, 16, 128, 64, 33, 3), (5, 17, 100, 33, 47, 3), (11, 30, 160, 31, 15, 3), (6, 64, 65, 29, 40, 3), (15, 33, 67, 17, 40, 3), (17, 48, 15, 16, 144, 3),
-         (50, 80, 14, 14, 32, 3), (70, 130, 16, 12, 16, 3), (45, 79, 8, 8, 110, 3), (170, 90, 7, 7, 31, 3), (200, 60, 6, 5, 68, 3), (5, 16, 500, 40, 8, 3),
+CASES = [(4, 16, 136, 64, 33, 3), (5, 17, 104, 33, 47, 3), (11, 30, 160, 31, 15, 3), (6, 64, 65, 29, 40, 3), (15, 33, 67, 17, 40, 3), (17, 48, 15, 16, 144, 3),
+         (54, 80, 14, 14, 32, 3), (70, 130, 16, 12, 16, 3), (45, 79, 8, 8, 110, 3), (170, 90, 7, 7, 31, 3), (200, 60, 6, 5, 68, 3), (5, 16, 500, 40, 8, 3),
          (4, 3, 9, 17, 5, 5), (5, 18, 12, 33, 20, 5), (6, 16, 21, 13, 40, 5), (9, 5, 10, 16, 16, 5), (46, 40, 8, 8, 40, 5), (101, 33, 7, 6, 31, 5),
          # single taps: tiles that end inside a plane and inside a group of four, planes smaller than a group of rows, both blocks
          (1, 64, 2, 3, 64, 1), (3, 130, 7, 7, 70, 1), (2, 65, 14, 14, 129, 1), (14, 5, 15, 15, 7, 1), (11, 100, 17, 19, 33, 1), (30000, 33, 2, 2, 40, 1),
          (120, 97, 15, 15, 31, 1), (90, 40, 40, 32, 47, 1), (130, 200, 32, 20, 32, 1), (5, 70, 1, 4, 300, 1)]
 
 
-def _on_the_digit_kernels(case):
-    """Its rule, so that a change of it does not leave this file testing another kernel."""
+# the kernel of each case in bfloat16 storage, in the dispatch's numbers: 3x3 with up to 16 output channels 20 (tiles 32 wide), 21, 22, with more 24, 25 (both
+# 16 wide) and 26; 5x5 28, 29, 30; single taps 32, up to 32 output channels 33
+KERNELS = [24, 26, 20, 24, 26, 25, 25, 21, 26, 26, 26, 22, 28, 29, 29, 29, 30, 30, 32, 32, 32, 33, 32, 32, 33, 32, 33, 32]
+
+
+def _kernel(case, bf16):
+    from addernetcuda_amd._lib import lib, check
     N, Ci, H, W, Co, k = case
-    if k == 1:
-        return min(Ci, Co) >= 64 or (H * W % 4 and N * H * W >= 3000) or (min(Ci, Co) >= 32 and -(-Ci // 16) * -(-Co // 16) * 256 * N * H * W >= 2.2e8)
-    macs = -(-Ci // 16) * -(-Co // 16) * 256 * k * k * N * H * W
-    return N >= 4 and macs >= (2.2e8 if k == 3 else 0 if W > 8 else 1.5e8)
+    out = ctypes.c_int()
+    check(lib.adder_conv2d_grad_w_kernel(N, Ci, H, W, Co, k, k, 1, k // 2, bf16, ctypes.byref(out)), "adder_conv2d_grad_w_kernel")
+    return out.value
 
 
 def _grad_w(gpu, x, w, gy, eta=0.0):
@@ -62,15 +67,16 @@ def _check(got, x, w, gy):
 
 @pytest.mark.parametrize("case", CASES, ids=str)
 def test_parity(gpu, case):
-    assert _on_the_digit_kernels(case)
+    assert not 20 <= _kernel(case, 0) < 100   # no digits in float storage
     x, w, gy = _data(case, 1)
     got = _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu))
     _check(got, x, w, gy)
     assert torch.equal(got, _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)))
 
 
-@pytest.mark.parametrize("case", CASES, ids=str)
-def test_bfloat16_storage(gpu, case):
+@pytest.mark.parametrize("case,kernel", list(zip(CASES, KERNELS)), ids=str)
+def test_bfloat16_storage(gpu, case, kernel):
+    assert _kernel(case, 1) == kernel
     x, w, gy = _data(case, 2)
     x, gy = x.bfloat16(), gy.bfloat16()
     _check(_grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)), x.float(), w, gy.float())
@@ -120,11 +126,10 @@ def test_infinities_and_nan(gpu, case, storage):
     assert bool(fine.isfinite().all()) and bool(torch.isclose(fine, clean[keep], rtol=1e-6, atol=1e-5).all())
 
 
-# layers whose backward takes the BatchNorm links, large enough; the last: one tile for a workgroup, beside others'
+# large layers whose backward takes the BatchNorm links (float storage; the last has single taps)
 @pytest.mark.parametrize("case", [(26, 20, 32, 32, 30, 1), (64, 32, 16, 16, 48, 1), (104, 64, 8, 8, 64, 1), (30, 70, 14, 14, 136, 1, 1)],
                          ids=str)
 def test_linked_batchnorm(gpu, case):
-    assert _on_the_digit_kernels((*case[:5], 1 if len(case) > 6 else 3))
     test_gpu_bn_links.test_fused_backward_matches_the_unfused_chain_in_float64(case, True, False, gpu)
 
 
@@ -132,7 +137,7 @@ def test_linked_batchnorm(gpu, case):
 @pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5), (200, 63, 16, 16, 4096, 1)], ids=str)
 def test_without_a_workspace(gpu, case):
     from addernetcuda_amd._lib import lib, check, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace
-    assert _on_the_digit_kernels(case)
+    assert _kernel(case, 1) >= 20
     x, w, gy = _data(case, 7)
     dims, _, _ = conv_dims(x.shape, w.shape, 1, case[5] // 2)
     assert conv2d_bwd_workspace(dims, gpu)[1] > 8 << 20
