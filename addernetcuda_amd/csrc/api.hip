@@ -261,7 +261,7 @@ int adder_conv2d_grad_w_kernel(int N, int Ci, int H, int W, int Co, int kh, int 
 
 static int conv2d_bwd(const float *gy, const float *x, const float *w, const float *gx_add, float *gx, float *gw,
                       float eta, void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
-                      int stride, int pad, void *stream, bool general = false);
+                      int stride, int pad, void *stream, size_t limit = SIZE_MAX);
 
 int adder_conv2d_bwd_f32(const float *gy, const float *x, const float *w, float *gx, float *gw, float eta,
                          void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
@@ -278,7 +278,7 @@ int adder_conv2d_bwd_add_f32(const float *gy, const float *x, const float *w, co
 
 static int conv2d_bwd(const float *gy, const float *x, const float *w, const float *gx_add, float *gx, float *gw,
                       float eta, void *ws, size_t ws_bytes, int N, int Ci, int H, int W, int Co, int kh, int kw,
-                      int stride, int pad, void *stream, bool general) {
+                      int stride, int pad, void *stream, size_t limit) {
     if (!gy || !x || !w) return ADDER_ERR_NULL_POINTER;
     if (!gx && !gw) return ADDER_ERR_NULL_POINTER;
     if (!(eta >= 0.f)) return ADDER_ERR_BAD_SHAPE;
@@ -291,8 +291,12 @@ static int conv2d_bwd(const float *gy, const float *x, const float *w, const flo
         overlaps(gw, nw, gx, nx) || overlaps(gx, nx, gx_add, nx) || overlaps(gw, nw, gx_add, nx))
         return ADDER_ERR_ALIAS;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    bool general = false;
+    size_t need = 0;
     if (gw) {
-        const size_t need = general ? kGradWGeneralWs : grad_w_workspace_bytes(d);
+        need = grad_w_workspace_bytes(d, false, limit);
+        general = need > limit && kh == 5 && kw == 5;   // (their slabs do not fit: the kernel that needs none)
+        if (general) need = kGradWGeneralWs;
         if (!ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255)) return ADDER_ERR_WORKSPACE;
         if (overlaps(ws, need, x, nx) || overlaps(ws, need, w, nw) || overlaps(ws, need, gy, ny) ||
             overlaps(ws, need, gx, nx) || overlaps(ws, need, gw, nw) || overlaps(ws, need, gx_add, nx))
@@ -302,7 +306,7 @@ static int conv2d_bwd(const float *gy, const float *x, const float *w, const flo
         if (int rc = launch_grad_x(gy, x, w, gx, d, s, gx_add)) return rc;
     if (gw)
         if (int rc = general ? launch_grad_w_general(gy, x, w, gw, eta, ws, d, s)
-                             : launch_grad_w(gy, x, w, gw, eta, ws, ws_bytes, d, s))
+                             : launch_grad_w(gy, x, w, gw, eta, ws, need, d, s, nullptr, nullptr, nullptr, kNoBnSums, limit))
             return rc;
     return ADDER_OK;
 }
@@ -354,17 +358,15 @@ int adder_conv2d_bwd_noalloc_f32(const float *gy, const float *x, const float *w
     ConvDims d;
     if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
     void *ws = nullptr;
-    size_t need = 0;
-    bool general = false;
     if (gw) {   // only the weight gradient uses scratch
-        need = grad_w_workspace_bytes(d);
+        const size_t need = grad_w_workspace_bytes(d, false, ADDER_NOALLOC_SCRATCH_BYTES);
         // 5x5 layers whose slabs do not fit have the general kernel, which needs none; other layers are refused
-        general = need > ADDER_NOALLOC_SCRATCH_BYTES && kh == 5 && kw == 5;
-        if (need > ADDER_NOALLOC_SCRATCH_BYTES && !general) return ADDER_ERR_WORKSPACE;   // before any HIP call
+        if (need > ADDER_NOALLOC_SCRATCH_BYTES && !(kh == 5 && kw == 5)) return ADDER_ERR_WORKSPACE;   // before any HIP call
         if (int rc = scratch_of_current_device(&ws)) return rc;
     }
     // every kernel writes the part of the scratch it later reads (slabs, norm partials): nothing to clear
-    return conv2d_bwd(gy, x, w, nullptr, gx, gw, eta, ws, need, N, Ci, H, W, Co, kh, kw, stride, pad, stream, general);
+    return conv2d_bwd(gy, x, w, nullptr, gx, gw, eta, ws, ADDER_NOALLOC_SCRATCH_BYTES, N, Ci, H, W, Co, kh, kw, stride, pad, stream,
+                      ADDER_NOALLOC_SCRATCH_BYTES);
 }
 
 static int check_col(int K, long NL, int Co) {

@@ -268,8 +268,8 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);   // 0: no statistics epilogue for these dimensions
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
-size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false);   // of the storage type's kernels
-int grad_w_kernel(const ConvDims &d, bool bf16);                       // which of them, as in adder_conv2d_grad_w_kernel
+size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false, size_t limit = SIZE_MAX);   // of the storage type's kernels
+int grad_w_kernel(const ConvDims &d, bool bf16);                                                // which of them, as in adder_conv2d_grad_w_kernel
 // The sums of the backward of the BatchNorm behind a layer, as the consumer's input-gradient kernel left them
 // ((C, slots, 2) floats -- a wave's fp32 totals: sum dz, sum dz * xhat), with what turns them into the four coefficients per channel.
 // A weight-gradient kernel that is given these instead of ready coefficients adds the slots itself (every
@@ -285,7 +285,8 @@ static constexpr BnSums kNoBnSums{nullptr, 0, 0.0, nullptr, nullptr, nullptr, nu
 template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
                   void *ws, size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y = nullptr,
-                  const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums);
+                  const float *bn_coef = nullptr, float *gy_out = nullptr, const BnSums &sums = kNoBnSums,
+                  size_t limit = SIZE_MAX);   // limit, as given to grad_w_workspace_bytes: fewer slabs where they are too many for it
 // launch_grad_w without slabs (any layer): `ws` holds the norm partials only, kGradWGeneralWs bytes
 static constexpr size_t kGradWGeneralWs = 128 * 1024;
 template <class T>

@@ -343,11 +343,23 @@ struct GradWPlan {
     int slots;
 };
 
-// `bf16`: large layers in bfloat16 storage have kernels of their own (grad_w_i8.hip)
-static GradWPlan plan_grad_w(const ConvDims &d, bool bf16 = false) {
+static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
+    size_t bytes = sizeof(double) * kNormBlocksMax;
+    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
+    if (p.variant)
+        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
+    return (bytes + 255) & ~(size_t)255;
+}
+
+// `bf16`: large layers in bfloat16 storage have kernels of their own (grad_w_i8.hip).  `limit`: the scratch of the entry point without a workspace.
+// A wide 1x1 layer whose slabs do not fit it runs with as many as do, if the slabs of the bfloat16 kernels' blocks, often the fewer, would fit
+// (256 -> 256 @14x14, 64 images: 64 slabs, 34 MB, become 15; the other kernel's blocks take 14).
+static GradWPlan plan_grad_w(const ConvDims &d, bool bf16 = false, size_t limit = SIZE_MAX) {
     GradWPlan p{};
     const long partial_cap = 1L << 28;  // partial slab elements
-    if (!(bf16 && plan_grad_w_i8(d, p.mfma))) p.mfma = plan_grad_w_mfma(d);
+    GradWMfmaPlan digits{};
+    const bool has_digits = (bf16 || (limit != SIZE_MAX && d.kh == 1)) && plan_grad_w_i8(d, digits);
+    p.mfma = bf16 && has_digits ? digits : plan_grad_w_mfma(d);
     if (p.mfma.variant) {
         p.variant = 2;
         p.slots = p.mfma.slots;
@@ -356,6 +368,13 @@ static GradWPlan plan_grad_w(const ConvDims &d, bool bf16 = false) {
         p.slots = grad_w_1x1_slots(d);
     }
     if (p.variant && (long)p.slots * d.Co * d.K() > partial_cap) p.variant = 0;
+    if (p.variant == 2 && has_digits && workspace_bytes_of(p, d) > limit) {
+        const size_t slab = sizeof(double) * ((size_t)d.Co * d.K() + d.Co), room = limit - kGradWGeneralWs;
+        if (digits.slots * slab <= room) {
+            const int fit = (int)(room / slab);
+            p.slots = p.mfma.slots = ceil_div(p.mfma.ntiles, ceil_div(p.mfma.ntiles, fit));
+        }
+    }
     return p;
 }
 
@@ -370,14 +389,7 @@ bool grad_w_bn_supported(const ConvDims &d, const void *gy, const void *x, const
     return p.variant == 2 && (k3 || k1) && (align & 15) == 0;
 }
 
-static size_t workspace_bytes_of(const GradWPlan &p, const ConvDims &d) {
-    size_t bytes = sizeof(double) * kNormBlocksMax;
-    // (plain 1x1 layers: fp32 slabs for float storage, fp64 for bfloat16, which needs none where there is one slab)
-    if (p.variant)
-        bytes += (p.variant == 2 || p.slots > 1 ? sizeof(double) : sizeof(float)) * (size_t)p.slots * ((size_t)d.Co * d.K() + d.Co);
-    return (bytes + 255) & ~(size_t)255;
-}
-size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16) { return workspace_bytes_of(plan_grad_w(d, bf16), d); }
+size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16, size_t limit) { return workspace_bytes_of(plan_grad_w(d, bf16, limit), d); }
 int grad_w_kernel(const ConvDims &d, bool bf16) {
     const GradWPlan p = plan_grad_w(d, bf16);
     return p.variant == 2 ? p.mfma.variant : p.variant == 1 ? 100 : 0;
@@ -390,8 +402,8 @@ int grad_w_kernel(const ConvDims &d, bool bf16) {
 template <class T>
 int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta, void *ws,
                   size_t ws_bytes, const ConvDims &d, hipStream_t s, const float *bn_y, const float *bn_coef,
-                  float *gy_out, const BnSums &sums) {
-    GradWPlan p = plan_grad_w(d, sizeof(T) != 4);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
+                  float *gy_out, const BnSums &sums, size_t limit) {
+    GradWPlan p = plan_grad_w(d, sizeof(T) != 4, limit);   // made once: 0.15 to 0.25 us of a launch-bound layer's call
     if (ws_bytes < workspace_bytes_of(p, d)) return ADDER_ERR_WORKSPACE;
     if (bn_y && (sizeof(T) != 4 ||
                  !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part)))
@@ -471,9 +483,9 @@ template int launch_grad_w_general<float>(const float *, const float *, const fl
 template int launch_grad_w_general<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *,
                                            const ConvDims &, hipStream_t);
 template int launch_grad_w<float>(const float *, const float *, const float *, float *, float, void *, size_t, const ConvDims &,
-                                  hipStream_t, const float *, const float *, float *, const BnSums &);
+                                  hipStream_t, const float *, const float *, float *, const BnSums &, size_t);
 template int launch_grad_w<bf16_t>(const bf16_t *, const bf16_t *, const float *, float *, float, void *, size_t,
-                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &);
+                                   const ConvDims &, hipStream_t, const float *, const float *, float *, const BnSums &, size_t);
 
 // ---- staged weight gradient: partial slabs now, finalize + scaling for many layers later --------------
 int launch_grad_w_staged(const float *gy, const float *x, const float *w, float *gw, float eta, void *ws,

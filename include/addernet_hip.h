@@ -187,9 +187,9 @@ ADDER_API int adder_conv2d_bwd_bf16(const adder_bf16 *gy, const adder_bf16 *x, c
  * the reference, whose backward takes every buffer from torch's allocator (adder.py:66-67).  The partial slabs
  * and norm partials live in a buffer of ADDER_NOALLOC_SCRATCH_BYTES that is part of the library's device image
  * (every GPU the library runs on holds one copy until the process ends); the call allocates and frees nothing.
- * Same arguments and results as adder_conv2d_bwd_f32 without ws / ws_bytes.  Layers that need more than ADDER_NOALLOC_SCRATCH_BYTES of it
- * (adder_conv2d_bwd_workspace_bytes, where the bfloat16 kernels do not need still more) are refused with ADDER_ERR_WORKSPACE
- * before anything is launched (every ResNet-20 layer at batch 256 fits) -- except 5x5 layers, which then take the general
+ * Same arguments and results as adder_conv2d_bwd_f32 without ws / ws_bytes.  Layers whose partial slabs do not fit are refused with
+ * ADDER_ERR_WORKSPACE before anything is launched (every ResNet-20 layer at batch 256 fits) -- except stride-1 1x1 layers from 64
+ * channels that a smaller number of slabs serves, whose fp64 sums are then added in another order, and 5x5 layers, which take the general
  * kernel, whose sums have another order.  All calls on one GPU share that
  * GPU's buffer: calls that overlap in time on one GPU (different streams, or threads) race; serialise them.
  * The first call on a device looks the buffer's address up (hipGetSymbolAddress); make that call outside

@@ -133,8 +133,9 @@ def test_linked_batchnorm(gpu, case):
     test_gpu_bn_links.test_fused_backward_matches_the_unfused_chain_in_float64(case, True, False, gpu)
 
 
-# the entry point without a workspace, where the slabs of the bfloat16 kernels would not fit its scratch
-@pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5), (200, 63, 16, 16, 4096, 1)], ids=str)
+# the entry point without a workspace, where the slabs of the bfloat16 kernels or, the last two, of the fp64 ones would not fit its scratch
+@pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5), (200, 63, 16, 16, 4096, 1),
+                                  (64, 256, 14, 14, 256, 1), (40, 130, 9, 9, 1000, 1)], ids=str)
 def test_without_a_workspace(gpu, case):
     from addernetcuda_amd._lib import lib, check, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace
     assert _kernel(case, 1) >= 20
