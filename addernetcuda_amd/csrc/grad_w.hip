@@ -411,10 +411,8 @@ int launch_grad_w(const T *gy, const T *x, const float *w, float *gw, float eta,
     // loads of four elements need bases aligned to a group; tensors whose rows are read element by element do not
     // (1x1 layers on the matrix cores walk whole planes as rows: their row length is H*W)
     const bool rows_1x1 = p.variant == 2 && d.kh == 1;
-    const bool any_base = p.variant == 2 && p.mfma.variant >= 32;   // (these read element by element by themselves)
-    const bool need_x16 = p.variant == 2 && !any_base && !(rows_1x1 && d.stride > 1) &&   // (a strided 1x1 layer samples x element-wise)
-                          (rows_1x1 ? d.H * d.W : d.W) % 4 == 0;
-    const bool need_g16 = p.variant == 2 && !any_base && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
+    const bool need_x16 = p.variant == 2 && !rows_1x1 && d.W % 4 == 0;   // (stride-1 1x1 layers read element by element then, strided ones sample x so)
+    const bool need_g16 = p.variant == 2 && !(rows_1x1 && d.stride == 1) && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
     if (p.variant && ((need_x16 && !aligned_groups(x)) || (need_g16 && !aligned_groups(gy)))) p.variant = 0;
     double *ss = reinterpret_cast<double *>(ws);
     const int K = d.K();
@@ -496,8 +494,8 @@ int launch_grad_w_staged(const float *gy, const float *x, const float *w, float 
     if (bn_y && !grad_w_bn_supported(d, gy, x, bn_y, bn_coef ? (const void *)bn_coef : (const void *)sums.part))
         return ADDER_ERR_UNSUPPORTED;
     const bool rows_1x1 = p.variant == 2 && d.kh == 1;
-    const bool need_x16 = p.variant == 2 && !(rows_1x1 && d.stride > 1) && (rows_1x1 ? d.H * d.W : d.W) % 4 == 0;
-    const bool need_g16 = p.variant == 2 && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
+    const bool need_x16 = p.variant == 2 && !rows_1x1 && d.W % 4 == 0;
+    const bool need_g16 = p.variant == 2 && !(rows_1x1 && d.stride == 1) && (rows_1x1 ? d.Ho * d.Wo : d.Wo) % 4 == 0;
     if (!p.variant || (need_x16 && (reinterpret_cast<uintptr_t>(x) & 15)) ||
         (need_g16 && (reinterpret_cast<uintptr_t>(gy) & 15)))
         return ADDER_ERR_UNSUPPORTED;   // no slab-based kernel for this layer: nothing to stage

@@ -506,8 +506,8 @@ static int launch_one_v(const T *gy, const T *x, double *part, double *sgpart, c
 template <class G, class T = float>
 static int launch_one(const T *gy, const T *x, double *part, double *sgpart, const ConvDims &d,
                       const GradWMfmaPlan &p, hipStream_t s) {
-    // element-wise tile loads unless the rows of both x and gy are whole groups of four
-    if (d.W % 4 == 0 && d.Wo % 4 == 0) return launch_one_v<G, true, false, T>(gy, x, part, sgpart, d, p, s);
+    // element-wise tile loads unless the rows of both x and gy are whole groups of four, and aligned (single taps; other layers come here so)
+    if (d.W % 4 == 0 && d.Wo % 4 == 0 && aligned_groups(x) && aligned_groups(gy)) return launch_one_v<G, true, false, T>(gy, x, part, sgpart, d, p, s);
     return launch_one_v<G, false, false, T>(gy, x, part, sgpart, d, p, s);
 }
 

@@ -148,13 +148,22 @@ def test_without_a_workspace(gpu, case):
     _check(gw.cpu(), x, w, gy)
 
 
-@pytest.mark.parametrize("case", [CASES[20], CASES[25]], ids=str)
-def test_bases_between_the_groups(gpu, case):
-    """Tensors that begin one element into an allocation: the same results, element by element."""
+@pytest.mark.parametrize("storage", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("case", [CASES[20], CASES[25], (9, 130, 12, 12, 140, 1), (3, 64, 4, 4, 65, 1)], ids=str)
+def test_bases_between_the_groups(gpu, case, storage):
+    """Tensors that begin one element into an allocation: the same results, element by element; the staged call, too."""
+    from addernetcuda_amd._lib import lib, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace, GradWStage
     x, w, gy = _data(case, 8)
-    x, gy = x.bfloat16(), gy.bfloat16()
+    x, gy = x.to(storage), gy.to(storage)
     off = lambda t: torch.cat([t.new_zeros(1), t.flatten()]).to(gpu)[1:].view(t.shape)
-    assert torch.equal(_grad_w(gpu, off(x), w.to(gpu), off(gy)), _grad_w(gpu, x.to(gpu), w.to(gpu), gy.to(gpu)))
+    xo, wg, gyo = off(x), w.to(gpu), off(gy)
+    assert torch.equal(_grad_w(gpu, xo, wg, gyo), _grad_w(gpu, x.to(gpu), wg, gy.to(gpu)))
+    if storage == torch.float32 and min(case[1], case[4]) >= 64:
+        dims, _, _ = conv_dims(x.shape, w.shape, 1, 0)
+        ws, nbytes = conv2d_bwd_workspace(dims, gpu)
+        gw, stage = torch.empty_like(wg), GradWStage()
+        assert lib.adder_conv2d_grad_w_staged_f32(ptr(gyo), ptr(xo), ptr(wg), ptr(gw), 0.0, ptr(ws), nbytes, *dims, ctypes.byref(stage), stream_ptr(gpu)) == 0
+        torch.cuda.synchronize()
 
 
 # column matrices with long sums (Co, K, NL)
