@@ -20,10 +20,13 @@
 // over its share of the positions of every staged tile; PW waves split the positions, MW x NW waves
 // the (co, k) block of the workgroup; the waves are folded in fp64 through LDS at the end.
 // sum_pos gy is collected on the A fragments.  Partials: one fp64 (Co, K) slab per grid.x slot.
-// Positions of a tile beside the map are zeros of gy times x, so an x that is infinite or not a number within their reach makes its taps not a number.
-// (A flag per tile and a masked loop for such tiles cost every 3x3 layer 5-9 %: 128 -> 128 @32x32, 128 images 684 -> 746 us.)
+// Positions of a tile beside the map are zeros of gy times x, which an x that is infinite or not a number would make not a number: a workgroup on
+// such a map whose sums are not finite walks over its tiles again with zeros in place of that x (stride 1; the look at the sums costs 0.3-0.8 us of
+// a call.  Masks in the one loop cost 5-9 %, and so did this in the stride-2 kernel of 8-wide maps, 256 -> 256 @14x14, 64 images 131 -> 138 us).
 #include "common.hpp"
 #include "tile3x3.hpp"
+
+#include <type_traits>
 
 namespace adder {
 
@@ -53,7 +56,7 @@ struct GwMfmaCfg {
     static constexpr int REGS = MT * NT * 4;          // accumulator values (fp64) per lane
     static constexpr int RED = 2 * (NWAVES / 2) * (REGS + MT) * 64;  // fp64 fold area, in floats
     static constexpr int LDS_FLOATS = (2 * BUF > RED) ? 2 * BUF : RED;
-    static constexpr int LDS_BYTES = LDS_FLOATS * 4;
+    static constexpr int LDS_BYTES = LDS_FLOATS * 4 + 16;   // + one flag
     static_assert(TW % 4 == 0 && STEPS % PW == 0, "positions must split evenly over the position waves");
     static_assert((PW & (PW - 1)) == 0, "the fold is a binary tree over the position waves");
     static_assert(NTHREADS <= 1024 && LDS_BYTES <= 160 * 1024, "workgroup limits");
@@ -260,8 +263,38 @@ __global__ __launch_bounds__(G::NTHREADS) void grad_w_mfma_kernel(const T *__res
         if constexpr (FUSE) gy_commit_m_bn<G>(gs, ys, smem + XP::BUF, coef, gy_dst, co_blk, Co, n0, N, h0, w0, Ho, Wo);
         else gy_commit_m<G>(gs, smem + XP::BUF);
     }
+    constexpr bool LOOK = G::KS > 1 && S == 1;
+    const bool ragged = Ho % G::TH != 0 || Wo % G::TW != 0;
+    int *const again = reinterpret_cast<int *>(smem + G::LDS_FLOATS) + (FUSE ? 4 * G::COB : 0);   // behind the coefficients
+    if (LOOK && threadIdx.x == 0) *again = 0;
     __syncthreads();
 
+    // one step; masked: x counts as zero at positions beside the map
+    auto step = [&](const float *base, const int ws, auto masked) {
+        const int st = pw + ws * G::PW;                 // wave-uniform step: (img, row, column group)
+        const int c4 = st % (G::TW / 4);
+        const int r = (st / (G::TW / 4)) % G::TH;
+        const int img = st / (G::TW / 4) / G::TH;
+        const int a_off = img * G::COB * G::GPLANE + r * G::TW + 4 * c4;
+        const int b_off = img * G::CIB * XP::PLANE + r * S * XP::PITCH + 4 * c4 * S;
+        double a[MT], b[NT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) a[mt] = (double)base[a_base[mt] + a_off];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) b[nt] = (double)base[b_base[nt] + b_off];
+        if constexpr (decltype(masked)::value) {
+            const bool in = h0 + r < Ho && w0 + 4 * c4 + lk < Wo;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) b[nt] = in ? b[nt] : 0.0;
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            sgt[mt] += a[mt];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
+        }
+    };
     int cur = 0;
     for (; tile < ntiles; tile += gridDim.x) {
         const int next = tile + gridDim.x;
@@ -274,26 +307,7 @@ __global__ __launch_bounds__(G::NTHREADS) void grad_w_mfma_kernel(const T *__res
         const float *base = smem + cur * G::BUF;
         auto steps = [&](const int first, const int last) {
 #pragma unroll 8
-            for (int ws = first; ws < last; ++ws) {
-                const int st = pw + ws * G::PW;                 // wave-uniform step: (img, row, column group)
-                const int c4 = st % (G::TW / 4);
-                const int r = (st / (G::TW / 4)) % G::TH;
-                const int img = st / (G::TW / 4) / G::TH;
-                const int a_off = img * G::COB * G::GPLANE + r * G::TW + 4 * c4;
-                const int b_off = img * G::CIB * XP::PLANE + r * S * XP::PITCH + 4 * c4 * S;
-                double a[MT], b[NT];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) a[mt] = (double)base[a_base[mt] + a_off];
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) b[nt] = (double)base[b_base[nt] + b_off];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    sgt[mt] += a[mt];
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
-                }
-            }
+            for (int ws = first; ws < last; ++ws) step(base, ws, std::false_type{});
         };
         // the next tile is written to the other LDS buffer half-way through, so that the ds_writes
         // issue while this tile's queued MFMAs keep the matrix pipe busy
@@ -309,6 +323,38 @@ __global__ __launch_bounds__(G::NTHREADS) void grad_w_mfma_kernel(const T *__res
         steps(G::WSTEPS / 2, G::WSTEPS);
         __syncthreads();
         cur ^= 1;
+    }
+
+    if (LOOK && ragged) {
+        double odd = 0.0;   // not a number where a sum is not finite
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) odd = fma(acc[mt][nt][e], 0.0, odd);
+        if (odd != 0.0) *again = 1;
+        __syncthreads();
+        if (*again) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                sgt[mt] = 0.0;
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = double4v{0.0, 0.0, 0.0, 0.0};
+            }
+            for (tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+                decode(tile);
+                tile_fetch<XP, VEC && !SUB, SUB, T>(xs, x, ci_blk, Ci, n0, N, h0 * S - G::PAD, w0 * S, H, W, sub);
+                gy_fetch_m<G, VEC, T>(gs, gy, co_blk, Co, n0, N, h0, w0, Ho, Wo);
+                if constexpr (FUSE) gy_fetch_m<G, true, float>(ys, bn_y, co_blk, Co, n0, N, h0, w0, Ho, Wo);
+                tile_commit<XP>(xs, smem);
+                if constexpr (FUSE) gy_commit_m_bn<G>(gs, ys, smem + XP::BUF, coef, nullptr, co_blk, Co, n0, N, h0, w0, Ho, Wo);
+                else gy_commit_m<G>(gs, smem + XP::BUF);
+                __syncthreads();
+                for (int ws = 0; ws < G::WSTEPS; ++ws) step(smem, ws, std::true_type{});
+                __syncthreads();
+            }
+        }
     }
 
     // ---- fold the PW position waves of each (mw, nw) block into its pw = 0 wave: binary tree, fp64, via LDS ----
