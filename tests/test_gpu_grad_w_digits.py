@@ -133,6 +133,31 @@ def test_linked_batchnorm(gpu, case):
     test_gpu_bn_links.test_fused_backward_matches_the_unfused_chain_in_float64(case, True, False, gpu)
 
 
+@pytest.mark.parametrize("case", [(3, 18, 13, 20, 24), (2, 16, 28, 28, 17), (5, 16, 7, 4, 16)], ids=str)
+def test_infinities_behind_a_linked_batchnorm(gpu, case):
+    from addernetcuda_amd._lib import lib, check, ptr, stream_ptr, conv_dims, conv2d_bwd_workspace, BnLinks
+    x, w, dz = _data((*case, 3), 16)
+    N, Ci, H, W, Co = case
+    x[N - 1, Ci - 1, H // 2, W - 1] = float("inf")
+    x[N - 1, Ci - 2, H - 1, W // 2] = float("-inf")
+    g = torch.Generator().manual_seed(17)
+    y, coef = torch.randn(dz.shape, generator=g).to(gpu), (torch.rand(Co, 4, generator=g) * 0.1).to(gpu)
+    xg, wg, dzg = x.to(gpu), w.to(gpu), dz.to(gpu)
+    gx, gw, gy = torch.empty_like(xg), torch.empty_like(wg), torch.full_like(dzg, float("nan"))
+    dims, _, _ = conv_dims(x.shape, w.shape, 1, 1)
+    ws, nbytes = conv2d_bwd_workspace(dims, gpu)
+    links = BnLinks(out_x=ptr(y), out_coef=ptr(coef), out_gy=ptr(gy))
+    check(lib.adder_conv2d_bwd_bn_f32(ptr(dzg), ptr(xg), ptr(wg), None, ptr(gx), ptr(gw), 0.0, ptr(ws), nbytes, *dims, ctypes.byref(links),
+                                      stream_ptr(gpu)), "adder_conv2d_bwd_bn_f32")
+    torch.cuda.synchronize()
+    gy, got = gy.cpu(), gw.cpu().double()
+    assert bool(gy.isfinite().all())
+    want = c_oracle.conv2d_grad_w(gy, x, w, 1, 1).double()
+    assert bool(got.isinf().any()) and torch.equal(got.isnan(), want.isnan()) and torch.equal(got[got.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    assert bool(torch.isclose(got[fine], want[fine], rtol=1e-6, atol=1e-5).all())
+
+
 # the entry point without a workspace, where the slabs of the bfloat16 kernels or, the last two, of the fp64 ones would not fit its scratch
 @pytest.mark.parametrize("case", [(256, 32, 16, 16, 32, 3), (32, 128, 14, 14, 120, 3), (8, 48, 28, 28, 48, 5), (200, 63, 16, 16, 4096, 1),
                                   (64, 256, 14, 14, 256, 1), (40, 130, 9, 9, 1000, 1)], ids=str)
