@@ -67,6 +67,65 @@ __device__ __forceinline__ void stf2(bf16_t *p, float2 v) {
     *reinterpret_cast<uint32_t *>(p) = (uint32_t)f32_to_bf16(v.x) | ((uint32_t)f32_to_bf16(v.y) << 16);
 }
 
+// CNT consecutive elements at an address aligned to one element only (global memory takes loads and stores of any alignment).
+typedef float f32x2_any __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t u16x2_any __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint16_t u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
+template <int CNT>
+__device__ __forceinline__ void ld_strip(const float *p, float (&v)[CNT]) {
+    static_assert(CNT == 1 || CNT == 2 || CNT == 4, "one, two or four elements");
+    if constexpr (CNT == 4) {
+        const f32x4_any u = *reinterpret_cast<const f32x4_any *>(p);
+        v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
+    } else if constexpr (CNT == 2) {
+        const f32x2_any u = *reinterpret_cast<const f32x2_any *>(p);
+        v[0] = u.x; v[1] = u.y;
+    } else {
+        v[0] = *p;
+    }
+}
+template <int CNT>
+__device__ __forceinline__ void ld_strip(const bf16_t *p, float (&v)[CNT]) {
+    static_assert(CNT == 1 || CNT == 2 || CNT == 4, "one, two or four elements");
+    if constexpr (CNT == 4) {
+        const u16x4_any u = *reinterpret_cast<const u16x4_any *>(p);
+        v[0] = bf16_to_f32(u.x); v[1] = bf16_to_f32(u.y); v[2] = bf16_to_f32(u.z); v[3] = bf16_to_f32(u.w);
+    } else if constexpr (CNT == 2) {
+        const u16x2_any u = *reinterpret_cast<const u16x2_any *>(p);
+        v[0] = bf16_to_f32(u.x); v[1] = bf16_to_f32(u.y);
+    } else {
+        v[0] = ldf(p);
+    }
+}
+template <int CNT>
+__device__ __forceinline__ void st_strip(float *p, const float (&v)[CNT]) {
+    static_assert(CNT == 4, "four elements");
+    *reinterpret_cast<f32x4_any *>(p) = f32x4_any{v[0], v[1], v[2], v[3]};
+}
+template <int CNT>
+__device__ __forceinline__ void st_strip(bf16_t *p, const float (&v)[CNT]) {
+    static_assert(CNT == 4, "four elements");
+    *reinterpret_cast<u16x4_any *>(p) = u16x4_any{f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]), f32_to_bf16(v[3])};
+}
+
+static constexpr int kTapChunk = 16;   // channels per first-level sum of the 1x1 kernels without tiles (fwd_tap.hip, grad_x_tap.hip)
+
+// Workgroup number -> (tile, block) of a launch whose blocks read the same tile of x.  Workgroups go to the eight dies in turn, each
+// with its own L2: the blocks of one tile follow each other on one die, so that x crosses to it once.
+__device__ __forceinline__ void xcd_tile(unsigned id, int tiles, int blocks, int &tile, int &blk) {
+    const unsigned whole = (unsigned)(tiles & ~7);
+    if (id < whole * blocks) {
+        const unsigned j = id >> 3;
+        tile = (int)(j / blocks * 8 + (id & 7));
+        blk = (int)(j % blocks);
+    } else {
+        const unsigned r = id - whole * blocks, rem = (unsigned)tiles - whole;
+        tile = (int)(whole + r % rem);
+        blk = (int)(r / rem);
+    }
+}
+
 // Most workgroups along a grid's y (hipDeviceProp_t::maxGridSize: 65536).  Kernels with few channels per workgroup leave layers
 // with more channels than that to those with many.
 static constexpr int kMaxGridY = 65535;
@@ -260,6 +319,10 @@ int check_launch();                  // hipGetLastError -> status
 // T: storage type of the activations and their gradients, float or bf16_t (the optional reduced-storage mode).
 template <class T>
 int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
+template <class T>
+int launch_fwd_tap(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn);
+bool fwd_tap_supported(const ConvDims &d);      // 1x1 / stride 1 (fwd_tap.hip)
+int fwd_tap_stats_slots(const ConvDims &d);
 int fwd_kernel(const ConvDims &d);
 int fwd_stats_slots(const ConvDims &d);
 bool fwd_pair_supported(const ConvDims &d);

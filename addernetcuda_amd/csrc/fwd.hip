@@ -577,19 +577,14 @@ using FwdW8S2  = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 16, 1, 2>;    // stride 2, outputs
 // ... with chunks of 8 input channels: two workgroups fit a CU's LDS instead of one, which pays from 128
 // input channels on (512 -> 512 @14x14, batch 64: 740 -> 530 us; at 32 channels the extra barriers cost 2 %)
 using FwdW8S2L = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 8, 1, 2>;
-// 1x1, stride 1: every (H, W) plane is one row of H*W positions; a unit is one output channel x 8 input
-// channels (8 weights, 64 vector instructions), eight output-channel waves share the staged x tile.
-using Fwd1x1   = Tile3x3Cfg<4, 64, 1, 1, 4, 8, 16, 8, 1, 1>;   // 256 positions of one image x 32 channels
-using Fwd1x1s  = Tile3x3Cfg<4, 16, 1, 4, 4, 8, 16, 8, 1, 1>;   // planes of <= 64 positions: four images
 // 1x1 with a stride: the tile loader gathers the sampled x element by element, which costs several times what the
 // aligned float4 loads of a stride-1 plane cost, so a workgroup takes 64 output channels per staged tile instead of
 // 32 (eight per lane, chunks of eight input channels to stay within 128 registers); ResNet-50's three downsample
-// layers at batch 64: 538 -> 319, 621 -> 376, 591 -> 374 us.  (On stride-1 planes this shape is slower.)
+// layers at batch 64: 538 -> 319, 621 -> 376, 591 -> 374 us.  (Stride 1: fwd_tap.hip.)
 using Fwd1x1sub = Tile3x3Cfg<4, 16, 1, 4, 8, 8, 8, 8, 1, 1>;   // 64 sampled positions of four images x 64 channels
-// the same two with units of four input channels, for channel counts that are multiples of 4 but not of 8
-// (DenseNet's multiples of 12)
-using Fwd1x1q  = Tile3x3Cfg<4, 64, 1, 1, 4, 8, 16, 4, 1, 1>;
-using Fwd1x1sq = Tile3x3Cfg<4, 16, 1, 4, 4, 8, 16, 4, 1, 1>;
+// ... with units of four input channels, for channel counts that are multiples of 4 but not of 8
+using Fwd1x1q  = Tile3x3Cfg<4, 64, 1, 1, 4, 8, 16, 4, 1, 1>;   // 256 positions of one image x 32 channels
+using Fwd1x1sq = Tile3x3Cfg<4, 16, 1, 4, 4, 8, 16, 4, 1, 1>;   // planes of <= 64 positions: four images
 
 // ... the same register tile in workgroups of four waves that cover fewer rows, for maps whose height is not a
 // multiple of 16: 56 rows are 7 x 8, 28 rows 7 x 4 (ResNet-50 at batch 64: 64 -> 64 @56x56 340 -> 294 us,
@@ -612,16 +607,16 @@ static int rows_per_tile_w32(int H) {
 }
 
 // which tiled kernel serves these dimensions (0 = none): 1..3 3x3 stride 1 by output width, 4..5 3x3 stride 2,
-// 6..7 1x1 stride 1 by plane size, 8..9 1x1 with a stride (the sampled positions walked like a stride-1 plane),
-// 10..13 = 6..9 with units of four input channels, 14..18 5x5 (stride 1 by output width, then stride 2)
+// 6..7 1x1 stride 1 by plane size (both fwd_tap.hip), 8..9 1x1 with a stride (the sampled positions walked like a stride-1 plane),
+// 10..13 = 6..9 for channels that are no multiple of 8, 14..18 5x5 (stride 1 by output width, then stride 2)
 static int fwd_tiled_variant(const ConvDims &d) {
     // (below 64 input channels the plain 1x1 kernel of conv1x1.hip is as fast or faster)
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci % Fwd1x1q::CQ == 0 && d.Ci >= 64) {
-        const int quad = d.Ci % Fwd1x1::CQ ? 4 : 0;
+        const int quad = d.Ci % Fwd1x1sub::CQ ? 4 : 0;
         // 256 positions of one image per workgroup, or 64 positions of four: whichever pads the plane less
         // (28x28 = 784 positions fill 64-wide tiles to 94 %, 256-wide ones to 77 %: 216 -> 169 us for 128 -> 512)
         const int plane = d.Ho * d.Wo;
-        const bool wide = ceil_div(plane, Fwd1x1::TW) * Fwd1x1::TW <= ceil_div(plane, Fwd1x1s::TW) * Fwd1x1s::TW;
+        const bool wide = ceil_div(plane, Fwd1x1q::TW) * Fwd1x1q::TW <= ceil_div(plane, Fwd1x1sq::TW) * Fwd1x1sq::TW;
         if (d.stride == 1) return (wide ? 6 : 7) + quad;
         return (wide ? 8 : 9) + quad;
     }
@@ -645,11 +640,11 @@ static int fwd_chunk(const ConvDims &d, int variant) {
         case 4: return FwdW16S2::CC;
         case 5: return d.Ci >= 128 ? FwdW8S2L::CC : FwdW8S2::CC;
         case 8: case 9: return Fwd1x1sub::CC;
-        default: return Fwd1x1::CC;
+        default: return Fwd1x1q::CC;
     }
 }
-static_assert(FwdW32::CC == FwdW32H8::CC && FwdW32::CC == FwdW32H4::CC && Fwd1x1::CC == Fwd1x1s::CC &&
-              Fwd1x1::CC == Fwd1x1q::CC && Fwd1x1::CC == Fwd1x1sq::CC, "one chunk length per variant");
+static_assert(FwdW32::CC == FwdW32H8::CC && FwdW32::CC == FwdW32H4::CC && Fwd1x1q::CC == Fwd1x1sq::CC,
+              "one chunk length per variant");
 
 // Whether the kernel for few positions takes a 3x3 or 1x1 layer.  The tiled kernels last as long as one wave's chain of
 // channels x taps x results per lane, 6 ns a term, until the chip is full; this one has a chain of its share of the
@@ -710,7 +705,8 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 }
 
 // Which kernel launch_fwd runs without statistics and for bases aligned to groups of four: 0 general, 1 plain 1x1, 2 few
-// positions, else 10 * variant + which of its tiles (rows 16 / 8 / 4: 0 / 1 / 2; channels from 128 on: 1).
+// positions, else 10 * variant + which of its tiles (rows 16 / 8 / 4: 0 / 1 / 2; channels from 128 on: 1).  1x1 layers of stride 1
+// are told apart by the same rules, but one kernel runs them all, with the same bits (fwd_tap.hip).
 int fwd_kernel(const ConvDims &d) {
     const int variant = fwd_tiled_variant(d);
     if (few_positions(d, variant)) return 2;
@@ -720,6 +716,7 @@ int fwd_kernel(const ConvDims &d) {
 }
 
 int fwd_stats_slots(const ConvDims &d) {
+    if (fwd_tap_supported(d)) return fwd_tap_stats_slots(d);
     if (d.kh == 1 && few_positions(d, fwd_tiled_variant(d))) return ceil_div(d.N * d.Ho * d.Wo, 64);
     switch (fwd_tiled_variant(d)) {
         case 1: switch (rows_per_tile_w32(d.Ho)) {
@@ -731,11 +728,7 @@ int fwd_stats_slots(const ConvDims &d) {
         case 3: return stats_slots_3x3<FwdW8>(d);
         case 4: return stats_slots_3x3<FwdW16S2>(d);
         case 5: return stats_slots_3x3<FwdW8S2>(d);
-        case 6: return stats_slots_3x3<Fwd1x1>(as_one_row(d));
-        case 7: return stats_slots_3x3<Fwd1x1s>(as_one_row(d));
         case 8: case 9: return stats_slots_3x3<Fwd1x1sub>(as_one_row(d));
-        case 10: return stats_slots_3x3<Fwd1x1q>(as_one_row(d));
-        case 11: return stats_slots_3x3<Fwd1x1sq>(as_one_row(d));
         case 12: return stats_slots_3x3<Fwd1x1q>(as_one_row(d));
         case 13: return stats_slots_3x3<Fwd1x1sq>(as_one_row(d));
         default: return conv1x1_supported(d, nullptr, nullptr) ? fwd_1x1_stats_slots(d) : 0;
@@ -750,7 +743,13 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
     // rows that are whole groups of four are moved as such and need bases aligned to a group
     const bool rows_ok = (d.W % 4 != 0 || aligned_groups(x)) && (d.Wo % 4 != 0 || aligned_groups(y));
     const int variant = fwd_tiled_variant(d);
-    if ((!stats || d.kh == 1) && few_positions(d, variant)) {   // (its statistics are offered for 1x1 layers: fwd_stats_slots)
+    const bool few = few_positions(d, variant);
+    if (fwd_tap_supported(d)) {
+        // (it takes bases of any alignment; statistics for planes of whole groups are offered for aligned ones only)
+        if (stats && !few && d.H * d.W % 4 == 0 && !(aligned_groups(x) && aligned_groups(y))) return ADDER_ERR_UNSUPPORTED;
+        return launch_fwd_tap(x, w, y, stats, d, s, bn);
+    }
+    if ((!stats || d.kh == 1) && few) {   // (its statistics are offered for 1x1 layers: fwd_stats_slots)
         const int chunk = fwd_chunk(d, variant);
         return d.kh == 3 ? launch_fwd_few<3>(x, w, y, stats, d, chunk, s, bn) : launch_fwd_few<1>(x, w, y, stats, d, chunk, s, bn);
     }
@@ -761,14 +760,6 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
             case 8: case 9: return launch_fwd_3x3_v<Fwd1x1sub, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d), bn);
             case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d), bn);
             default: return launch_fwd_3x3_v<Fwd1x1sq, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d), bn);
-        }
-    } else if (variant >= 6 && variant <= 11) {
-        const ConvDims f = as_one_row(d);
-        if (f.W % 4 != 0 || (aligned_groups(x) && aligned_groups(y))) switch (variant) {
-            case 6: return launch_fwd_3x3<Fwd1x1>(x, w, y, stats, f, s, bn);
-            case 7: return launch_fwd_3x3<Fwd1x1s>(x, w, y, stats, f, s, bn);
-            case 10: return launch_fwd_3x3<Fwd1x1q>(x, w, y, stats, f, s, bn);
-            default: return launch_fwd_3x3<Fwd1x1sq>(x, w, y, stats, f, s, bn);
         }
     }
     if (rows_ok && !(stats && variant >= 14)) {   // 3x3 and 5x5 taps; statistics are offered for 3x3 and 1x1 layers

@@ -1,0 +1,254 @@
+// Forward of 1x1 / stride-1 layers from 64 input channels on, NCHW in -> NCHW out:
+//   y[n,co,p] = - sum_ci | w[co,ci] - x[n,ci,p] |        (adder_cuda/adder.cu:19-70 behind the unfold of adder.py:32)
+//
+// Two vector instructions per term bound it, as in fwd.hip: 73 T lane-instructions/s is what a bare stream of the pair reaches with
+// two waves on each of a SIMD's two issue ports (62 T with one, 31 T with one wave per SIMD), 90 us for the 3.3e9 terms of
+// 1024 -> 256 @14x14, 64 images.  A single tap shares no x between neighbouring positions, so there is nothing to stage: a wave
+// reads its strips of x straight into registers, four channels ahead, and runs without a barrier.  What that leaves to choose
+// is how many waves there are, and the channels are what can be shared out without more reads per term: the KSP waves of a
+// workgroup have the same 8 x 64 * TN outputs and take 16-channel chunks in turn; their sums meet in LDS at the end.
+// us, 256 positions x 32 channels staged in LDS per workgroup (one wave for all channels) -> this:
+//   32 images: 256 -> 64 @56x56 89 -> 72, 256 -> 128 151 -> 130, 512 -> 256 @28x28 171 -> 133, 256 -> 1024 @14x14 86 -> 71,
+//   1024 -> 256 109 -> 82, 512 -> 2048 @7x7 104 -> 84, 2048 -> 512 273 -> 97; 1024 -> 256 @14x14, 64 images 178 -> 140, 8 images 106 -> 31,
+//   one image (there the kernel for few positions) 34 -> 18; 300 -> 48 @8x8, 64 images 36 -> 8.
+// Tried on the way: sums of sums in LDS instead of registers (116 -> 84 registers) 131 -> 141 us; 16 channels x 2 positions per lane
+// 146 -> 187; the next chunk's weight lines asked for a chunk early 131 -> 140; x of eight waves staged in LDS 1024 -> 256 176.
+#include "common.hpp"
+
+#include <type_traits>
+
+namespace adder {
+
+// TM output channels x TN adjacent positions per lane; wave v of the KSP of a workgroup takes the chunks v, v + KSP, ... of input
+// channels.  Two-level sums in registers (a chunk, a wave's chunks), the waves' sums are added in the order of the waves.
+template <int TM_, int TN_, int KSP_>
+struct TapCfg {
+    static constexpr int TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = kTapChunk, FM = TM / KSP;
+    static constexpr int LDS_BYTES = KSP * TM * TN * 64 * 4;
+};
+
+static constexpr int kTapTM = 8;
+static int tap_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((long)d.N * ceil_div(d.H * d.W, tn), 64); }
+
+struct TapDims {
+    int N, Ci, Co, L;       // L = H * W positions per image
+    int strips;             // of TN positions per image; the last one of an image is moved back to end at L
+    int tiles, blocks;      // of 64 strips, of TM output channels
+};
+
+template <class C, class T, bool EVAL>
+__global__ __launch_bounds__(C::NT) void fwd_tap_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
+                                                        double *__restrict__ stats, const TapDims d, const BnEval bn) {
+    constexpr int TM = C::TM, TN = C::TN, KSP = C::KSP, CQ = 4, UM = TM * TN >= 32 ? 2 : (TM < 4 ? TM : 4), NU = TM / UM, FM = C::FM;
+    static_assert(NU == 1 || NU % 2 == 0, "the weight buffers alternate from unit to unit");
+    extern __shared__ __align__(16) float smem[];
+    int tile, blk;
+    xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, s = sc - n * d.strips;
+    const int p0 = min(s * TN, d.L - TN), co_base = blk * TM;
+    uniform_f32_ptr wc = as_uniform(w);
+    int wrow[TM];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) wrow[m] = min(co_base + m, d.Co - 1) * d.Ci;
+
+    float acc[TM][TN], tot[TM][TN];
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) acc[m][t] = tot[m][t] = 0.f;
+    float xr[2][CQ][TN], wv[2][UM][CQ];
+    // a uniform base per channel and the lane's distance from it in bytes (64 strips: far below 2^32): no address registers
+    const int n_first = __builtin_amdgcn_readfirstlane(n);
+    const unsigned xoff = (unsigned)((n - n_first) * d.Ci * d.L + p0) * (unsigned)sizeof(T);
+    const T *x_first = x + (size_t)n_first * d.Ci * d.L;
+    auto load_x = [&](const int b, const int ci) {
+#pragma unroll
+        for (int e = 0; e < CQ; ++e) ld_strip<TN>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(x_first + (size_t)(ci + e) * d.L) + xoff), xr[b][e]);
+    };
+    auto load_w = [&](const int b, const int h, const int ci) {
+#pragma unroll
+        for (int u = 0; u < UM; ++u)
+#pragma unroll
+            for (int e = 0; e < CQ; ++e) wv[b][u][e] = wc[wrow[h * UM + u] + ci + e];
+    };
+    int ci = wave * C::CC;
+    if (ci < d.Ci) {
+        load_x(0, ci);
+        load_w(0, 0, ci);
+        auto half = [&](const int cur) -> bool {
+            int next = ci + CQ;
+            const bool chunk_end = (next & (C::CC - 1)) == 0;
+            if (chunk_end) next += (KSP - 1) * C::CC;
+            const bool more = next < d.Ci;
+            const int cn = more ? next : ci;
+#pragma unroll
+            for (int h = 0; h < NU; ++h) {
+                const int wb = (cur * (NU & 1) + h) & 1;
+#pragma unroll
+                for (int idx = 0; idx < UM * CQ * TN; ++idx) {
+                    const int t = idx % TN, u = (idx / TN) % UM, e = idx / TN / UM, m = h * UM + u;
+                    acc[m][t] -= fabsf(wv[wb][u][e] - xr[cur][e][t]);
+                    if (idx == 0) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_w(wb ^ 1, h + 1 < NU ? h + 1 : 0, h + 1 < NU ? ci : cn);
+                        if (h == 0) load_x(cur ^ 1, cn);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            ci = next;
+            if (chunk_end || !more) {
+#pragma unroll
+                for (int m = 0; m < TM; ++m)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) { tot[m][t] += acc[m][t]; acc[m][t] = 0.f; }
+            }
+            return more;
+        };
+#pragma unroll 1
+        while (half(0) && half(1)) {}
+    }
+
+    // every wave finishes FM of the channels: the waves' sums are added in the order of the waves
+    float r[FM][TN];
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) smem[((wave * TM + m) * TN + t) * 64 + lane] = tot[m][t];
+    __syncthreads();
+    const int m0 = wave * FM;
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            float v = smem[((m0 + f) * TN + t) * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < KSP; ++k) v += smem[((k * TM + m0 + f) * TN + t) * 64 + lane];
+            r[f][t] = v;
+        }
+
+    const int co0 = co_base + m0;
+    unsigned own = 0;   // bit t: position p0 + t is this lane's
+#pragma unroll
+    for (int t = 0; t < TN; ++t) own |= (sidx == sc && p0 + t >= s * TN ? 1u : 0u) << t;
+    if (stats) {
+        // as in fwd.hip: sums of deviations from a pivot in fp32, moved back to the origin in fp64; one slot per tile
+        const double count = (double)wave_sum_dpp((float)__popc(own));
+#pragma unroll
+        for (int f = 0; f < FM; ++f) {
+            const float pivot = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r[f][0])));
+            float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+                if (own >> t & 1) {
+                    const float dv = r[f][t] - pivot;
+                    s1 += dv;
+                    s2 = fmaf(dv, dv, s2);
+                }
+            const double d1 = (double)wave_sum_dpp(s1), d2 = (double)wave_sum_dpp(s2), c = (double)pivot;
+            if (lane == 0 && co0 + f < d.Co) {
+                double *dst = stats + ((size_t)(co0 + f) * d.tiles + tile) * 2;
+                dst[0] = d1 + count * c;
+                dst[1] = d2 + 2.0 * c * d1 + count * c * c;
+            }
+        }
+    }
+    const int yoff = n * d.Co * d.L + p0;
+    const bool whole = TN == 4 && (d.L & 3) == 0;
+    if constexpr (EVAL) {
+        float a[FM][TN];
+#pragma unroll
+        for (int f = 0; f < FM; ++f) {   // (all loads before the first store: one counter serves both)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) a[f][t] = 0.f;
+            if (bn.res) ld_strip<TN>(bn.res + (size_t)min(co0 + f, d.Co - 1) * d.L + yoff, a[f]);
+        }
+#pragma unroll
+        for (int f = 0; f < FM; ++f) {
+            const BnEvalChannel ch(bn, min(co0 + f, d.Co - 1));
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                r[f][t] = ch(r[f][t]) + a[f][t];
+                if (bn.relu) r[f][t] = relu_keep_nan(r[f][t]);
+            }
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < FM; ++f) {
+        if (co0 + f >= d.Co) break;
+        T *dst = y + (size_t)(co0 + f) * d.L + yoff;
+        if (whole && own) {
+            if constexpr (TN == 4) st_strip<TN>(dst, r[f]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+                if (own >> t & 1) stf(dst + t, r[f][t]);
+        }
+    }
+}
+
+template <class C, class T>
+static int launch_tap(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn) {
+    const TapDims t{d.N, d.Ci, d.Co, d.H * d.W, ceil_div(d.H * d.W, C::TN), tap_tiles(d, C::TN), ceil_div(d.Co, C::TM)};
+    const long grid = (long)t.tiles * t.blocks;
+    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
+    auto launch = [&](auto eval) {
+        constexpr bool EVAL = decltype(eval)::value;
+        if (int rc = allow_dynamic_lds<&fwd_tap_kernel<C, T, EVAL>>(C::LDS_BYTES)) return rc;
+        hipLaunchKernelGGL((fwd_tap_kernel<C, T, EVAL>), dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, s, x, w, y, stats, t, bn);
+        return check_launch();
+    };
+    if constexpr (sizeof(T) == 4) {
+        if (bn.gamma) return launch(std::true_type{});
+    }
+    return launch(std::false_type{});
+}
+
+// Waves that share the channels: as many as have two chunks each, by the channels alone, so that a layer's results have the same
+// bits whatever the batch.  us with 2 / 4 / 8 of them, 32 images: 64 -> 256 @56x56 76 / 82 / 114, 128 -> 512 @28x28 71 / 74 / 80,
+// 256 -> 128 @56x56 132 / 130 / 137, 512 -> 256 @28x28 147 / 133 / 133, 1024 -> 256 @14x14 105 / 87 / 82, 2048 -> 512 @7x7 247 / 145 / 97.
+static int tap_waves(int Ci) { return Ci <= 128 ? 2 : Ci <= 256 ? 4 : 8; }
+
+// Positions per lane.  Four, unless the launch is then about one workgroup per CU or less: two (us, four -> two: 1024 -> 256 @14x14, 8
+// images, 224 workgroups, 34 -> 31, 4 images 27 -> 23; 512 -> 128 @28x28, 8 images, 400 workgroups, 25 -> 28), and one where that
+// leaves half the chip idle or costs no more tiles (64 strips of two on a plane of 49): 512 -> 128 @28x28, one image, 11.4 -> 10.0,
+// 512 -> 2048 @7x7 11.5 -> 10.0; 256 -> 64 @56x56, 200 workgroups, 7.0 -> 8.5.
+static int tap_positions(const ConvDims &d) {
+    const int L = d.H * d.W, blocks = ceil_div(d.Co, kTapTM);
+    int tn = L >= 4 ? 4 : L >= 2 ? 2 : 1;
+    if (tn == 4 && (long)tap_tiles(d, 4) * blocks < 256 + 256 / tap_waves(d.Ci)) tn = 2;
+    if (tn == 2 && ((long)tap_tiles(d, 2) * blocks < 128 || tap_tiles(d, 1) == tap_tiles(d, 2))) tn = 1;
+    return tn;
+}
+
+// Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.
+bool fwd_tap_supported(const ConvDims &d) {
+    if (d.kh != 1 || d.kw != 1 || d.pad != 0 || d.stride != 1 || d.Ci < 64 || d.Ci % 4) return false;
+    const long L = (long)d.H * d.W, images = 63 / ceil_div_l(L, 4) + 1;
+    return (images * d.Ci + 1) * L <= 0x3fffffffL;
+}
+int fwd_tap_stats_slots(const ConvDims &d) { return tap_tiles(d, tap_positions(d)); }
+
+template <class T>
+int launch_fwd_tap(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn) {
+    auto run = [&](auto tn, auto ksp) {
+        return launch_tap<TapCfg<kTapTM, decltype(tn)::value, decltype(ksp)::value>, T>(x, w, y, stats, d, s, bn);
+    };
+    auto waves = [&](auto tn) {
+        switch (tap_waves(d.Ci)) {
+            case 2: return run(tn, std::integral_constant<int, 2>{});
+            case 4: return run(tn, std::integral_constant<int, 4>{});
+            default: return run(tn, std::integral_constant<int, 8>{});
+        }
+    };
+    switch (tap_positions(d)) {
+        case 4: return waves(std::integral_constant<int, 4>{});
+        case 2: return waves(std::integral_constant<int, 2>{});
+        default: return waves(std::integral_constant<int, 1>{});
+    }
+}
+template int launch_fwd_tap<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t, const BnEval &);
+template int launch_fwd_tap<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t, const BnEval &);
+
+}  // namespace adder
