@@ -100,13 +100,17 @@ __device__ __forceinline__ void ld_strip(const bf16_t *p, float (&v)[CNT]) {
 }
 template <int CNT>
 __device__ __forceinline__ void st_strip(float *p, const float (&v)[CNT]) {
-    static_assert(CNT == 4, "four elements");
-    *reinterpret_cast<f32x4_any *>(p) = f32x4_any{v[0], v[1], v[2], v[3]};
+    static_assert(CNT == 2 || CNT == 4, "two or four elements");
+    if constexpr (CNT == 4) *reinterpret_cast<f32x4_any *>(p) = f32x4_any{v[0], v[1], v[2], v[3]};
+    else *reinterpret_cast<f32x2_any *>(p) = f32x2_any{v[0], v[1]};
 }
 template <int CNT>
 __device__ __forceinline__ void st_strip(bf16_t *p, const float (&v)[CNT]) {
-    static_assert(CNT == 4, "four elements");
-    *reinterpret_cast<u16x4_any *>(p) = u16x4_any{f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]), f32_to_bf16(v[3])};
+    static_assert(CNT == 2 || CNT == 4, "two or four elements");
+    if constexpr (CNT == 4)
+        *reinterpret_cast<u16x4_any *>(p) = u16x4_any{f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]), f32_to_bf16(v[3])};
+    else
+        *reinterpret_cast<u16x2_any *>(p) = u16x2_any{f32_to_bf16(v[0]), f32_to_bf16(v[1])};
 }
 
 static constexpr int kTapChunk = 16;   // channels per first-level sum of the 1x1 kernels without tiles (fwd_tap.hip, grad_x_tap.hip)
@@ -331,6 +335,13 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);   // 0: no statistics epilogue for these dimensions
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
+// 1x1 / stride 1 (grad_x_tap.hip); bn (nullable): the in_* half of adder_bn_links, slots of sums per channel
+template <class T>
+int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
+                      const adder_bn_links *bn);
+bool grad_x_tap_supported(const ConvDims &d);
+int grad_x_tap_bn_slots(const ConvDims &d);
+static constexpr int kSatMaxTerms1x1 = 1024;   // output channels up to which a single tap's input gradient takes two instructions a term (grad_x.hip)
 size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false, size_t limit = SIZE_MAX);   // of the storage type's kernels
 int grad_w_kernel(const ConvDims &d, bool bf16);                                                // which of them, as in adder_conv2d_grad_w_kernel
 // The sums of the backward of the BatchNorm behind a layer, as the consumer's input-gradient kernel left them

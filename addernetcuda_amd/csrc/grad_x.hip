@@ -555,7 +555,7 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
 // Below ten output channels the doubled and the subtracted sum are what rounds, not the length of the sums: 5x5 layers of 1 / 4 / 8
 // channels 1.8e-7 / 2.4e-7 / 2.5e-7 with two instructions, 0.9e-7 / 1.25e-7 / 1.3e-7 with three (kernel without tiles 0.9e-7 / 1.7e-7 / 2.4e-7);
 // 64 -> 8 @32x32, 64 images, 52 -> 63 us.
-static constexpr int kSatMaxTerms = 1152, kSatMaxTerms1x1 = 1024, kSatMaxTerms5x5 = 2500, kSatMinChannels5x5 = 10;
+static constexpr int kSatMaxTerms = 1152, kSatMaxTerms5x5 = 2500, kSatMinChannels5x5 = 10;
 template <class C>
 static bool two_instructions(int Co) {
     if (C::KS == 5 && Co < kSatMinChannels5x5) return false;
@@ -1053,7 +1053,8 @@ using GxW8  = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 16, 1>;    // inputs 8 wide: two imag
 using Gx5W32 = Tile3x3Cfg<2, 16, 8, 1, 2, 4, 8, 1, 1, 5>;   // 8 rows of one image x 8 channels
 using Gx5W16 = Tile3x3Cfg<2, 8, 16, 1, 2, 4, 8, 1, 1, 5>;   // inputs 9..16 wide: one image x 8 channels
 using Gx5W8  = Tile3x3Cfg<2, 4, 8, 4, 2, 4, 8, 1, 1, 5>;    // inputs up to 8 wide: four images x 8 channels
-// 1x1, stride 1: (H, W) planes walked as one row; a unit is one output channel x the lane's 8 input channels
+// 1x1 with a stride (stride 1: grad_x_tap.hip): the sampled positions walked as one row; a unit is one output channel x the lane's 8
+// input channels
 using Gx1x1  = Tile3x3Cfg<2, 64, 1, 1, 8, 8, 16, 2, 1, 1>;    // 128 positions of one image x 64 channels
 using Gx1x1s = Tile3x3Cfg<4, 16, 1, 4, 8, 8, 16, 1, 1, 1>;    // planes of <= 64 positions: four images
 using Gx1x1t = Tile3x3Cfg<2, 32, 1, 2, 4, 8, 16, 8, 1, 1>;    // ... two images x 32 channels, where Gx1x1s would leave CUs idle
@@ -1079,15 +1080,15 @@ static_assert(GxW32::TM == GxW16::TM && GxW16::TM == GxW8::TM && GxS2W32::TM == 
 // ---------------------------------------------------------------------------
 // Few positions: one input position x TM input channels per lane, the waves of a workgroup share the output channels
 // (the forward's counterpart of this kernel is fwd_few_kernel).  Wave v takes the chunks v, v + waves, ... of `chunk` output
-// channels, with gy (read from global memory: a map this small sits in L1 / L2) and the weights G output channels ahead
+// channels, with gy (read from global memory: a map this small sits in L1 / L2) and the weights one output channel ahead
 // of the arithmetic; the chunk sums go through LDS and are added in channel order.
 // ---------------------------------------------------------------------------
-static constexpr int kFewTM = 4;
-template <int KS, int TM, int G, class T>
+static constexpr int kFewTM = 4, kFewChunk = 8;   // input channels per lane; output channels per first-level sum (72 terms)
+template <int TM, class T>
 __global__ __launch_bounds__(512) void grad_x_few_kernel(const T *__restrict__ gy, const T *__restrict__ x,
                                                          const float *__restrict__ w, T *__restrict__ gx,
-                                                         const T *__restrict__ gadd, ConvDims d, int chunk) {
-    constexpr int KK = KS * KS;
+                                                         const T *__restrict__ gadd, ConvDims d) {
+    constexpr int KS = 3, KK = 9, chunk = kFewChunk;
     __shared__ float part[8][TM][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int plane = d.H * d.W, total = d.N * plane, K = d.Ci * KK;   // (stride 1, pad KS / 2: gy has the planes of x)
@@ -1116,42 +1117,35 @@ __global__ __launch_bounds__(512) void grad_x_few_kernel(const T *__restrict__ g
         const int c = c0 + wave;
         if (c < nchunks) {
             const int first = c * chunk, end = min(first + chunk, d.Co);
-            float acc[TM], gv[2][G * KK], wv[2][G * TM * KK];
+            float acc[TM], gv[2][KK], wv[2][TM * KK];
 #pragma unroll
             for (int m = 0; m < TM; ++m) acc[m] = 0.f;
             auto load = [&](const int b, const int co) {
+                const int cc = min(co, end - 1);
 #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const int cc = min(co + g, end - 1);
+                for (int e = 0; e < TM * KK; ++e) wv[b][e] = wc[cc * K + e];
+                const T *gc = gy + (size_t)cc * plane;
 #pragma unroll
-                    for (int e = 0; e < TM * KK; ++e) wv[b][g * TM * KK + e] = wc[cc * K + e];
-                    const T *gc = gy + (size_t)cc * plane;
-#pragma unroll
-                    for (int e = 0; e < KK; ++e) gv[b][g * KK + e] = ldf(gc + off[e]);
-                }
+                for (int e = 0; e < KK; ++e) gv[b][e] = ldf(gc + off[e]);
             };
             auto add = [&](const int b, const int co) {
+                if (co >= end) return;
 #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    if (co + g >= end) break;
+                for (int e = 0; e < KK; ++e) {
+                    const float v = ok[e] ? gv[b][e] : 0.f;
 #pragma unroll
-                    for (int e = 0; e < KK; ++e) {
-                        const float v = ok[e] ? gv[b][g * KK + e] : 0.f;
-#pragma unroll
-                        for (int m = 0; m < TM; ++m)
-                            acc[m] = fmaf(hardtanh(wv[b][(g * TM + m) * KK + e] - xv[m]), v, acc[m]);
-                    }
+                    for (int m = 0; m < TM; ++m) acc[m] = fmaf(hardtanh(wv[b][m * KK + e] - xv[m]), v, acc[m]);
                 }
             };
             load(0, first);
 #pragma unroll 1
-            for (int co = first; co < end; co += 2 * G) {
-                load(1, co + G);
+            for (int co = first; co < end; co += 2) {
+                load(1, co + 1);
                 __builtin_amdgcn_sched_barrier(0);
                 add(0, co);
-                load(0, co + 2 * G);
+                load(0, co + 2);
                 __builtin_amdgcn_sched_barrier(0);
-                add(1, co + G);
+                add(1, co + 1);
             }
 #pragma unroll
             for (int m = 0; m < TM; ++m) part[wave][m][lane] = acc[m];
@@ -1176,40 +1170,30 @@ __global__ __launch_bounds__(512) void grad_x_few_kernel(const T *__restrict__ g
     }
 }
 
-// output channels per first-level sum: 72 terms with nine taps, 16 to 64 with one
-static int few_chunk(const ConvDims &d) {
-    const int eighth = round_up(ceil_div(d.Co, 8), 8);
-    return d.kh == 3 ? 8 : eighth < 16 ? 16 : eighth > 64 ? 64 : eighth;
-}
-
-// Whether it takes a 3x3 / pad 1 or 1x1 layer of stride 1.  The tiled kernels last as long as one wave's chain of output
-// channels x taps x results per lane, 5.5 ns a term with nine taps and 9.5 with one, until the chip is full; this one has a
-// chain of its share of the output channels (0.45 / 0.15 us each) and then works at 9 / 6.5 terms per ps.  Fitted to 60
-// layers; us, tiled -> this: 37 -> 51 3x3 @27x19, 7 images, 43 -> 13; 64 -> 64 @8x8, 1 / 64 images, 29 -> 6, 30 -> 19; 512 -> 512
-// @7x7, 1 / 7 images, 267 -> 38, 323 -> 111; 128 -> 128 @16x16, 1 / 7, 90 -> 11, 92 -> 36; 64 -> 512 1x1 @8x8, 16, 44 -> 10; 512 -> 2048
-// 1x1 @7x7, 4, 202 -> 76.  Beyond the line: 16 -> 16 @32x32, 64 images, 17 against 19; 1024 -> 256 1x1 @14x14, 7, 43 against 59.
+// Whether it takes a 3x3 / pad 1 layer of stride 1.  The tiled kernels last as long as one wave's chain of output channels x
+// taps x results per lane, 5.5 ns a term, until the chip is full; this one has a chain of its share of the output channels (0.45 us
+// each) and then works at 9 terms per ps.  Fitted to 60 layers; us, tiled -> this: 37 -> 51 3x3 @27x19, 7 images, 43 -> 13; 64 -> 64
+// @8x8, 1 / 64 images, 29 -> 6, 30 -> 19; 512 -> 512 @7x7, 1 / 7 images, 267 -> 38, 323 -> 111; 128 -> 128 @16x16, 1 / 7, 90 -> 11, 92 -> 36.
+// Beyond the line: 16 -> 16 @32x32, 64 images, 17 against 19.
 // Not for float32 layers that have a BatchNorm-linked kernel (whole groups of four): linked and plain backward of a layer
 // give the same bits, and the linked kernels sum in the tiled order.
 static int grad_x_bn_variant(const ConvDims &d);
 template <class T>
 static bool few_positions(const ConvDims &d, int per_lane) {
     if ((sizeof(T) == 4 && grad_x_bn_variant(d)) || ceil_div(d.Ci, kFewTM) > kMaxGridY) return false;
-    const bool nine = d.kh == 3;
-    const int chunk = few_chunk(d);
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
-    const float tiled = nine ? 2.f + 0.0055f * 9 * per_lane * d.Co : 3.f + 0.0095f * per_lane * d.Co;
-    const float share = (float)(ceil_div(ceil_div(d.Co, chunk), 8) * chunk);
-    const float few = nine ? 2.f + 0.45f * share + terms / 9e6f : 3.f + 0.15f * share + terms / 6.5e6f;
+    const float tiled = 2.f + 0.0055f * 9 * per_lane * d.Co;
+    const float share = (float)(ceil_div(ceil_div(d.Co, kFewChunk), 8) * kFewChunk);
+    const float few = 2.f + 0.45f * share + terms / 9e6f;
     return few < 0.9f * tiled;
 }
 
-template <int KS, class T>
+template <class T>
 static int launch_grad_x_few(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
-    constexpr int TM = kFewTM, G = KS == 1 ? 8 : 1;
-    const int chunk = few_chunk(d);
-    const int chunks = ceil_div(d.Co, chunk), waves = chunks < 8 ? chunks : 8;
-    hipLaunchKernelGGL((grad_x_few_kernel<KS, TM, G, T>), dim3(ceil_div(d.N * d.H * d.W, 64), ceil_div(d.Ci, TM)),
-                       dim3(64 * waves), 0, s, gy, x, w, gx, gadd, d, chunk);
+    constexpr int TM = kFewTM;
+    const int chunks = ceil_div(d.Co, kFewChunk), waves = chunks < 8 ? chunks : 8;
+    hipLaunchKernelGGL((grad_x_few_kernel<TM, T>), dim3(ceil_div(d.N * d.H * d.W, 64), ceil_div(d.Ci, TM)),
+                       dim3(64 * waves), 0, s, gy, x, w, gx, gadd, d);
     return check_launch();
 }
 
@@ -1223,7 +1207,7 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
     const bool aligned = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
     if (k3s1p1 && d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned)) {
         if (few_positions<T>(d, d.W > 16 ? GxW32::TM * GxW32::TN : d.W > 8 ? GxW16::TM * GxW16::TN : GxW8::TM * GxW8::TN))
-            return launch_grad_x_few<3>(gy, x, w, gx, d, s, gadd);
+            return launch_grad_x_few(gy, x, w, gx, d, s, gadd);
         if (d.W > 16) switch (rows_per_tile_w32(d.H)) {
             case 16: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
             case 8: return launch_grad_x_3x3s1<GxW32H8, false, T>(gy, x, w, gx, d, s, gadd);
@@ -1243,18 +1227,10 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         if (d.W > 16) return launch_grad_x_3x3s2<GxS2W32, T>(gy, x, w, gx, d, s, gadd);
         return launch_grad_x_3x3s2<GxS2W16, T>(gy, x, w, gx, d, s, gadd);
     }
-    // (from 48 output channels on the tiled kernel is ahead of the plain one: DenseNet's 48-channel bottlenecks)
-    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride == 1 && d.Ci >= 64 && d.Co >= 48) {
-        ConvDims f = d;   // every (H, W) plane as one row of H*W positions
-        f.H = f.Ho = 1;
-        f.W = f.Wo = d.H * d.W;
-        if (f.W % 4 != 0 || aligned) {
-            if ((f.W > 64 || small_plane_tile(f)) && few_positions<T>(d, f.W > 64 ? Gx1x1::TM * Gx1x1::TN : Gx1x1t::TM * Gx1x1t::TN))
-                return launch_grad_x_few<1>(gy, x, w, gx, d, s, gadd);
-            if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, false, T>(gy, x, w, gx, f, s, gadd);
-            return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, false, T>(gy, x, w, gx, f, s, gadd)
-                                       : launch_grad_x_3x3s1<Gx1x1s, false, T>(gy, x, w, gx, f, s, gadd);
-        }
+    if (grad_x_tap_supported(d)) {
+        // (it takes bases of any alignment; a second gradient is added on planes of whole groups for aligned ones only)
+        if (gadd && d.H * d.W % 4 == 0 && !aligned) return ADDER_ERR_UNSUPPORTED;
+        return launch_grad_x_tap<T>(gy, x, w, gx, d, s, gadd, nullptr);
     }
     if (gadd) return ADDER_ERR_UNSUPPORTED;
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride > 1 && d.Ci >= 64 && d.Co >= 64) {
@@ -1283,22 +1259,11 @@ template int launch_grad_x<float>(const float *, const float *, const float *, f
 template int launch_grad_x<bf16_t>(const bf16_t *, const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t,
                                    const bf16_t *);
 
-// a 1x1 stride-1 layer seen as images of one row of H * W positions
-static ConvDims one_row(const ConvDims &d) {
-    ConvDims f = d;
-    f.H = f.Ho = 1;
-    f.W = f.Wo = d.H * d.W;
-    return f;
-}
-
 // Which tiled kernel carries the BatchNorm link for this layer: 1 GxW32, 2 GxW16, 3 GxW8 (3x3 stride 1), 4 GxS2W32,
-// 5 GxS2W16 (3x3 stride 2), 6 Gx1x1, 7 Gx1x1t, 8 Gx1x1s (1x1 stride 1 from 64 input / 48 output channels); 0: none
+// 5 GxS2W16 (3x3 stride 2), 6 the kernel of grad_x_tap.hip (1x1 stride 1 from 64 input / 48 output channels); 0: none
 // (other kernel sizes, rows or planes that are not whole float4 groups, too few channels).
 static int grad_x_bn_variant(const ConvDims &d) {
-    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride == 1 && d.Ci >= 64 && d.Co >= 48 && (d.H * d.W) % 4 == 0) {
-        const ConvDims f = one_row(d);
-        return f.W > 64 ? 6 : (small_plane_tile(f) ? 7 : 8);
-    }
+    if (grad_x_tap_supported(d)) return (d.H * d.W) % 4 == 0 ? 6 : 0;
     if (d.kh != 3 || d.kw != 3 || d.pad != 1 || d.Ci < GxW32::TM) return 0;
     if (d.stride == 1 && d.W % 4 == 0) return d.W > 16 ? 1 : (d.W > 8 ? 2 : 3);
     if (d.stride == 2 && d.W % 4 == 0 && d.Wo % 4 == 0) return d.W > 16 ? 4 : 5;
@@ -1322,9 +1287,7 @@ int grad_x_bn_slots(const ConvDims &d) {
         case 3: return bn_slots_of<GxW8>(d);
         case 4: return bn_slots_of<GxS2W32>(d);
         case 5: return bn_slots_of<GxS2W16>(d);
-        case 6: return bn_slots_of<Gx1x1>(one_row(d));
-        case 7: return bn_slots_of<Gx1x1t>(one_row(d));
-        case 8: return bn_slots_of<Gx1x1s>(one_row(d));
+        case 6: return grad_x_tap_bn_slots(d);
         default: return 0;
     }
 }
@@ -1348,9 +1311,7 @@ int launch_grad_x_bn(const float *gy, const float *x, const float *w, float *gx,
         case 3: return launch_grad_x_3x3s1_bn<GxW8>(gy, x, w, gx, d, s, gadd, bn);
         case 4: return launch_grad_x_3x3s2_bn<GxS2W32>(gy, x, w, gx, d, s, gadd, bn);
         case 5: return launch_grad_x_3x3s2_bn<GxS2W16>(gy, x, w, gx, d, s, gadd, bn);
-        case 6: return launch_grad_x_3x3s1_bn<Gx1x1>(gy, x, w, gx, one_row(d), s, gadd, bn);
-        case 7: return launch_grad_x_3x3s1_bn<Gx1x1t>(gy, x, w, gx, one_row(d), s, gadd, bn);
-        case 8: return launch_grad_x_3x3s1_bn<Gx1x1s>(gy, x, w, gx, one_row(d), s, gadd, bn);
+        case 6: return launch_grad_x_tap<float>(gy, x, w, gx, d, s, gadd, &bn);
         default: return ADDER_ERR_UNSUPPORTED;
     }
 }
