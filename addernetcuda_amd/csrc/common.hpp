@@ -114,6 +114,7 @@ __device__ __forceinline__ void st_strip(bf16_t *p, const float (&v)[CNT]) {
 }
 
 static constexpr int kTapChunk = 16;   // channels per first-level sum of the 1x1 kernels without tiles (fwd_tap.hip, grad_x_tap.hip)
+static constexpr int kNineChunk = 8;   // ... of the 3x3 forward without tiles (fwd_nine.hip): 72 terms
 
 // Workgroup number -> (tile, block) of a launch whose blocks read the same tile of x.  Workgroups go to the eight dies in turn, each
 // with its own L2: the blocks of one tile follow each other on one die, so that x crosses to it once.
@@ -327,6 +328,13 @@ template <class T>
 int launch_fwd_tap(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn);
 bool fwd_tap_supported(const ConvDims &d);      // 1x1 / stride 1 (fwd_tap.hip)
 int fwd_tap_stats_slots(const ConvDims &d);
+// 3x3 / pad 1 / stride 1 or 2 (fwd_nine.hip); mul (stride 1, float): an ordinary convolution; w_side, y_side, stats_side (nullable; stride
+// 2, float): the strided 1x1 layer beside it
+template <class T>
+int launch_fwd_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn,
+                    bool mul = false, const float *w_side = nullptr, T *y_side = nullptr, double *stats_side = nullptr);
+bool fwd_nine_supported(const ConvDims &d);
+int fwd_nine_stats_slots(const ConvDims &d);
 int fwd_kernel(const ConvDims &d);
 int fwd_stats_slots(const ConvDims &d);
 bool fwd_pair_supported(const ConvDims &d);

@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void fwd_generic_kernel(const T *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Tiled kernel for 3x3 / pad 1 and 5x5 / pad 2, stride S = 1 or 2 (the figures are the 3x3 ones).
+// Tiled kernel for 5x5 / pad 2, stride S = 1 or 2, and single taps with a stride.
 //
 // A workgroup owns NIMG images x a TH x TW patch of output positions and
 // TM*COW output channels.  TW = TN*SPR: each lane owns a strip of TN adjacent
@@ -94,26 +94,16 @@ __global__ __launch_bounds__(256) void fwd_generic_kernel(const T *__restrict__ 
 // input channels.  Column 0 of a row is input column w0*S-1, so a lane's strip
 // starts at column strip*TN*S, which is 16-byte aligned when TN*S is a multiple of 4.
 // ---------------------------------------------------------------------------
-// MUL: the same kernel as an ordinary convolution, y = sum w * x (one v_fmac per term), for the regular
-// stem layer that precedes the adder layers of a network.
 // T: storage type of x and y (float, or bf16_t for the reduced-storage mode); the arithmetic is fp32 either way.
-// PAIR (3x3 taps at stride 2 only): the strided 1x1 layer that reads the same x beside this layer (the downsample
-// branch of a residual block, resnet20.py:66-70) is computed along with it -- its one tap is the centre tap of the
-// 3x3 window, so the x values are in registers already: weights w_side (Co, Ci), output y_side and statistics
-// stats_side shaped like y and stats.
 // EVAL: bn is applied to the results (float storage; an instance of its own, so that the others keep their registers).
-template <class C, bool VEC = true, bool SUB = false, bool MUL = false, class T = float, bool PAIR = false, bool EVAL = false>
+template <class C, bool VEC, bool SUB, class T, bool EVAL>
 __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restrict__ x,
                                                                 const float *__restrict__ w,
                                                                 T *__restrict__ y,
                                                                 double *__restrict__ stats, int N, int Ci,
                                                                 int H, int W, int Co, int Ho, int Wo,
                                                                 int tilesH, int tilesW, const Subsample sub,
-                                                                const BnEval bn,
-                                                                const float *__restrict__ w_side = nullptr,
-                                                                T *__restrict__ y_side = nullptr,
-                                                                double *__restrict__ stats_side = nullptr) {
-    static_assert(!PAIR || (C::S == 2 && C::KS == 3 && !MUL && !SUB), "the side layer is a strided 1x1 beside a strided 3x3");
+                                                                const BnEval bn) {
     constexpr int TN = C::TN, TM = C::TM, CQ = C::CQ, S = C::S, STRIP = C::STRIP, KS = C::KS, KK = C::KK;
     extern __shared__ __align__(16) float smem[];
 
@@ -140,18 +130,6 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
 #pragma unroll
     for (int m = 0; m < TM; ++m)
         wrow[m] = __builtin_amdgcn_readfirstlane(min(co_base + m, Co - 1) * K);
-    uniform_f32_ptr wsc = as_uniform(w_side);
-    int wsrow[PAIR ? TM : 1];
-    float tots[PAIR ? TM : 1][TN];   // PAIR: the side layer's sums (Ci terms each: one level)
-    if constexpr (PAIR) {
-#pragma unroll
-        for (int m = 0; m < TM; ++m) {
-            wsrow[m] = __builtin_amdgcn_readfirstlane(min(co_base + m, Co - 1) * Ci);
-#pragma unroll
-            for (int t = 0; t < TN; ++t) tots[m][t] = 0.f;
-        }
-    }
-
     // two-level sum: `acc` collects one channel chunk (<= 9*CC terms), `tot` the chunks, so the
     // rounding error grows with the square roots of the two lengths instead of with K
     float acc[TM][TN], tot[TM][TN];
@@ -184,7 +162,6 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
         // operands and with the rest of the arithmetic still ahead to hide the latency.
         float xr[2][CQ][KS][STRIP];
         float wv[2][CQ * KK];
-        float wsv[2][CQ];   // PAIR: the side layer's weights, buffered like wv
 #pragma unroll
         for (int q = 0; q < CQ; ++q)
 #pragma unroll
@@ -192,10 +169,6 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
                 lds_read_strip<STRIP, C::STRIP_ALIGN>(lbase + q * C::PLANE + i * C::PITCH, xr[0][q][i]);
 #pragma unroll
         for (int e = 0; e < CQ * KK; ++e) wv[0][e] = wc[wrow[0] + ci0 * KK + e];
-        if constexpr (PAIR) {
-#pragma unroll
-            for (int q = 0; q < CQ; ++q) wsv[0][q] = wsc[wsrow[0] + ci0 + q];
-        }
 
         auto half = [&](const int cc, const int cur) {
             // cur = 0/1: which xr buffer holds channel group cc
@@ -207,27 +180,15 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
 #pragma unroll
                 for (int idx = 0; idx < CQ * KK * TN; ++idx) {
                     const int t = idx % TN, j = (idx / TN) % KS, i = (idx / TN / KS) % KS, q = idx / TN / KK;
-                    if constexpr (MUL)
-                        acc[m][t] = fmaf(wv[m & 1][q * KK + i * KS + j], xr[cur][q][i][t * S + j], acc[m][t]);
-                    else
-                        acc[m][t] -= fabsf(wv[m & 1][q * KK + i * KS + j] - xr[cur][q][i][t * S + j]);
+                    acc[m][t] -= fabsf(wv[m & 1][q * KK + i * KS + j] - xr[cur][q][i][t * S + j]);
                     if (idx == 0) {
                         __builtin_amdgcn_sched_barrier(0);
                         if (m + 1 < TM) {
 #pragma unroll
                             for (int e = 0; e < CQ * KK; ++e) wv[(m + 1) & 1][e] = wc[wrow[m + 1] + kofs + e];
-                            if constexpr (PAIR) {
-#pragma unroll
-                                for (int q2 = 0; q2 < CQ; ++q2) wsv[(m + 1) & 1][q2] = wsc[wsrow[m + 1] + ci0 + cc + q2];
-                            }
                         } else {
 #pragma unroll
                             for (int e = 0; e < CQ * KK; ++e) wv[(m + 1) & 1][e] = wc[wrow[0] + knext + e];
-                            if constexpr (PAIR) {
-#pragma unroll
-                                for (int q2 = 0; q2 < CQ; ++q2)
-                                    wsv[(m + 1) & 1][q2] = wsc[wsrow[0] + ci0 + (more ? cc + CQ : cc) + q2];
-                            }
                         }
                         if (m == 0 && more) {
 #pragma unroll
@@ -239,12 +200,6 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                }
-                if constexpr (PAIR) {   // the centre tap (1, 1) is the strided 1x1 layer's only tap
-#pragma unroll
-                    for (int q = 0; q < CQ; ++q)
-#pragma unroll
-                        for (int t = 0; t < TN; ++t) tots[m][t] -= fabsf(wsv[m & 1][q] - xr[cur][q][1][t * S + 1]);
                 }
             }
         };
@@ -269,7 +224,6 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
     }
 
     const int n = n0 + img, ho = h0 + row, wo = w0 + strip * TN;
-    auto finish = [&](float (&tot)[TM][TN], T *__restrict__ y, double *__restrict__ stats) {
     if (stats) {
         // BatchNorm statistics of the layer's output on the way out: per wave and output channel the sums of
         // y and y*y over the wave's valid positions, in the partial-sum layout of the BatchNorm kernels
@@ -339,7 +293,7 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
     if (lane_ok && n < N && ho < Ho) {
         const bool vec = TN % 4 == 0 && (Wo & 3) == 0 && wo + TN <= Wo;
         if constexpr (EVAL) {
-            static_assert(sizeof(T) == 4 && !MUL && !PAIR, "inference epilogue: float adder layers");
+            static_assert(sizeof(T) == 4, "inference epilogue: float storage");
             // Inference: the BatchNorm behind the layer, the shortcut and the ReLU on the way out instead of three more passes
             // over the map (two launches and a fill for the BatchNorm, one each for add and ReLU): ResNet-50, 32 images,
             // 9.53 -> 8.31 ms, of which 1.65 ms were those passes; ResNet-20, one image, 90 -> 25 launches, 870 -> 470 us.
@@ -386,43 +340,32 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
             }
         }
     }
-    };
-    finish(tot, y, stats);
-    if constexpr (PAIR) finish(tots, y_side, stats_side);
 }
 
 // ---------------------------------------------------------------------------
-// Few positions: one output position x TM output channels per lane, the waves of a workgroup share the reduction.
+// Few positions of a 1x1 layer with a stride: one output position x TM output channels per lane, the waves of a workgroup share the
+// reduction.
 //
-// The tiled kernels give a lane 8-16 results and walk all input channels in one wave; one image leaves them with a handful
-// of workgroups, and the launch lasts as long as that serial chain (64 -> 64 3x3 @8x8, one image: 4 workgroups, 25 us).
-// Here wave v of a workgroup takes the channel chunks v, v + waves, ...; after each round the chunk sums go through LDS and
-// are added in channel order, so every result has the bits of the tiled kernel whose chunk length is given (`chunk`
-// channels per first-level sum).  x is read from global memory (a map this small sits in L1 / L2) one channel ahead
-// of the arithmetic, as are the weights.  Whole networks: ResNet-50, one image, 4.6 -> 1.7 ms; VGG-small, two, 720 -> 184 us.
+// The tiled kernels give a lane 8-32 results and walk all input channels in one wave; one image leaves them with a handful
+// of workgroups, and the launch lasts as long as that serial chain.  Here wave v of a workgroup takes the channel chunks v, v +
+// waves, ...; after each round the chunk sums go through LDS and are added in channel order, so every result has the bits of the
+// tiled kernel whose chunk length is given (`chunk` channels per first-level sum).  x is read from global memory (a map this small
+// sits in L1 / L2) one group of channels ahead of the arithmetic, as are the weights.
 // ---------------------------------------------------------------------------
 static constexpr int kFewTM = 4;
-template <int KS, int TM, int G, class T>
+template <int TM, int G, class T>
 __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
                                                       double *__restrict__ stats, ConvDims d, int chunk, const BnEval bn) {
-    constexpr int KK = KS * KS;
     __shared__ float part[8][TM][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    const int plane = d.H * d.W, L = d.Ho * d.Wo, total = d.N * L, K = d.Ci * KK, co0 = blockIdx.y * TM;
+    const int plane = d.H * d.W, L = d.Ho * d.Wo, total = d.N * L, co0 = blockIdx.y * TM;
     const int pos = min((int)blockIdx.x * 64 + lane, total - 1);
     const int n = pos / L, ho = pos % L / d.Wo, wo = pos % L % d.Wo;
-    int off[KK];
-    bool ok[KK];
-#pragma unroll
-    for (int e = 0; e < KK; ++e) {
-        const int hi = ho * d.stride + e / KS - d.pad, wi = wo * d.stride + e % KS - d.pad;
-        ok[e] = hi >= 0 && hi < d.H && wi >= 0 && wi < d.W;
-        off[e] = n * d.Ci * plane + (ok[e] ? hi * d.W + wi : 0);
-    }
+    const int off = n * d.Ci * plane + ho * d.stride * d.W + wo * d.stride;
     uniform_f32_ptr wc = as_uniform(w);
     int wrow[TM];
 #pragma unroll
-    for (int m = 0; m < TM; ++m) wrow[m] = min(co0 + m, d.Co - 1) * K;
+    for (int m = 0; m < TM; ++m) wrow[m] = min(co0 + m, d.Co - 1) * d.Ci;
     const int nchunks = ceil_div(d.Ci, chunk);
     float tot[TM];   // of result threadIdx.x + k * blockDim.x of the workgroup's TM x 64
 #pragma unroll
@@ -432,7 +375,7 @@ __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, c
         const int c = c0 + wave;
         if (c < nchunks) {
             const int first = c * chunk, end = min(first + chunk, d.Ci);
-            float acc[TM], xv[2][G * KK], wv[2][TM * G * KK];
+            float acc[TM], xv[2][G], wv[2][TM * G];
 #pragma unroll
             for (int m = 0; m < TM; ++m) acc[m] = 0.f;
             auto load = [&](const int b, const int ci) {
@@ -440,12 +383,8 @@ __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, c
                 for (int g = 0; g < G; ++g) {
                     const int cc = min(ci + g, end - 1);
 #pragma unroll
-                    for (int m = 0; m < TM; ++m)
-#pragma unroll
-                        for (int e = 0; e < KK; ++e) wv[b][(m * G + g) * KK + e] = wc[wrow[m] + cc * KK + e];
-                    const T *xc = x + (size_t)cc * plane;
-#pragma unroll
-                    for (int e = 0; e < KK; ++e) xv[b][g * KK + e] = ldf(xc + off[e]);
+                    for (int m = 0; m < TM; ++m) wv[b][m * G + g] = wc[wrow[m] + cc];
+                    xv[b][g] = ldf(x + (size_t)cc * plane + off);
                 }
             };
             auto add = [&](const int b, const int ci) {
@@ -453,11 +392,7 @@ __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, c
                 for (int g = 0; g < G; ++g) {
                     if (ci + g >= end) break;
 #pragma unroll
-                    for (int e = 0; e < KK; ++e) {
-                        const float v = ok[e] ? xv[b][g * KK + e] : 0.f;
-#pragma unroll
-                        for (int m = 0; m < TM; ++m) acc[m] -= fabsf(wv[b][(m * G + g) * KK + e] - v);
-                    }
+                    for (int m = 0; m < TM; ++m) acc[m] -= fabsf(wv[b][m * G + g] - xv[b][g]);
                 }
             };
             load(0, first);
@@ -507,17 +442,17 @@ __global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, c
     }
 }
 
-template <int KS, class T>
+template <class T>
 static int launch_fwd_few(const T *x, const float *w, T *y, double *stats, const ConvDims &d, int chunk, hipStream_t s,
                           const BnEval &bn) {
-    constexpr int TM = kFewTM, G = KS == 1 ? 8 : 1;
+    constexpr int TM = kFewTM, G = 8;
     const int waves = ceil_div(d.Ci, chunk) < 8 ? ceil_div(d.Ci, chunk) : 8;
-    hipLaunchKernelGGL((fwd_few_kernel<KS, TM, G, T>), dim3(ceil_div(d.N * d.Ho * d.Wo, 64), ceil_div(d.Co, TM)),
+    hipLaunchKernelGGL((fwd_few_kernel<TM, G, T>), dim3(ceil_div(d.N * d.Ho * d.Wo, 64), ceil_div(d.Co, TM)),
                        dim3(64 * waves), 0, s, x, w, y, stats, d, chunk, bn);
     return check_launch();
 }
 
-template <class C, bool VEC, bool SUB = false, bool MUL = false, class T = float>
+template <class C, bool VEC, bool SUB, class T>
 static int launch_fwd_3x3_v(const T *x, const float *w, T *y, double *stats, const ConvDims &d,
                             hipStream_t s, const Subsample sub = Subsample{1, 0, 0, 0}, const BnEval &bn = kNoBnEval) {
     const int tilesH = ceil_div(d.Ho, C::TH), tilesW = ceil_div(d.Wo, C::TW);
@@ -526,13 +461,12 @@ static int launch_fwd_3x3_v(const T *x, const float *w, T *y, double *stats, con
     if (gx > 0x7fffffffL) return ADDER_ERR_TOO_LARGE;
     auto launch = [&](auto eval) {
         constexpr bool EVAL = decltype(eval)::value;
-        if (int rc = allow_dynamic_lds<&fwd_3x3_kernel<C, VEC, SUB, MUL, T, false, EVAL>>(C::LDS_BYTES)) return rc;
-        hipLaunchKernelGGL((fwd_3x3_kernel<C, VEC, SUB, MUL, T, false, EVAL>), dim3((unsigned)gx, gy), dim3(C::NTHREADS),
-                           C::LDS_BYTES, s, x, w, y, stats, d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, tilesH, tilesW, sub, bn,
-                           nullptr, nullptr, nullptr);
+        if (int rc = allow_dynamic_lds<&fwd_3x3_kernel<C, VEC, SUB, T, EVAL>>(C::LDS_BYTES)) return rc;
+        hipLaunchKernelGGL((fwd_3x3_kernel<C, VEC, SUB, T, EVAL>), dim3((unsigned)gx, gy), dim3(C::NTHREADS),
+                           C::LDS_BYTES, s, x, w, y, stats, d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, tilesH, tilesW, sub, bn);
         return check_launch();
     };
-    if constexpr (sizeof(T) == 4 && !MUL) {
+    if constexpr (sizeof(T) == 4) {
         if (bn.gamma) return launch(std::true_type{});
     }
     return launch(std::false_type{});
@@ -543,16 +477,8 @@ static int launch_fwd_3x3(const T *x, const float *w, T *y, double *stats, const
                           hipStream_t s, const BnEval &bn) {
     const Subsample all{1, 0, 0, 0};
     // element-wise tile loads when the rows of the staged tensor are not whole groups of four
-    if (d.W % 4 == 0) return launch_fwd_3x3_v<C, true, false, false, T>(x, w, y, stats, d, s, all, bn);
-    return launch_fwd_3x3_v<C, false, false, false, T>(x, w, y, stats, d, s, all, bn);
-}
-
-// the same tile shapes as an ordinary convolution (3x3 / stride 1 / pad 1 only)
-template <class C>
-static int launch_mulconv_3x3(const float *x, const float *w, float *y, double *stats, const ConvDims &d,
-                              hipStream_t s) {
-    if (d.W % 4 == 0) return launch_fwd_3x3_v<C, true, false, true>(x, w, y, stats, d, s);
-    return launch_fwd_3x3_v<C, false, false, true>(x, w, y, stats, d, s);
+    if (d.W % 4 == 0) return launch_fwd_3x3_v<C, true, false, T>(x, w, y, stats, d, s, all, bn);
+    return launch_fwd_3x3_v<C, false, false, T>(x, w, y, stats, d, s, all, bn);
 }
 
 // partial-sum slots per channel the statistics epilogue of this tile shape writes
@@ -562,21 +488,6 @@ static int stats_slots_3x3(const ConvDims &d) {
     return (int)(gx * C::POSW);
 }
 
-// Tile shapes per output width, picked by timing sweeps on MI355X.  What they have in common: a ResNet-20
-// layer at batch 256 launches 2048-4096 waves in 256-512 workgroups of eight waves; a lane keeps only
-// 2-4 output channels x 4 positions (few registers, short dependent chains); one pipeline unit is one
-// output channel x one input channel (CQ = 1: 9 weights, 18*TN vector instructions), which keeps the two
-// weight buffers far from the 102-SGPR limit (spilled SGPRs come back as v_readlane inside the hot loop)
-// and works for odd channel counts too.
-//                           TN SPR TH NIMG TM COW CC CQ S
-using FwdW32   = Tile3x3Cfg<4, 8, 16, 1, 4, 4, 8, 1, 1>;    // outputs 32 wide: half an image x 16 channels
-using FwdW16   = Tile3x3Cfg<4, 4, 16, 1, 4, 8, 16, 1, 1>;   // outputs 16 wide: one image x 32 channels
-using FwdW8    = Tile3x3Cfg<4, 2, 8, 4, 2, 8, 16, 1, 1>;    // outputs 8 wide: four images x 16 channels
-using FwdW16S2 = Tile3x3Cfg<2, 8, 16, 1, 4, 8, 8, 1, 2>;    // stride 2, outputs 16 wide: one image x 32 channels
-using FwdW8S2  = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 16, 1, 2>;    // stride 2, outputs 8 wide: two images x 32 channels
-// ... with chunks of 8 input channels: two workgroups fit a CU's LDS instead of one, which pays from 128
-// input channels on (512 -> 512 @14x14, batch 64: 740 -> 530 us; at 32 channels the extra barriers cost 2 %)
-using FwdW8S2L = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 8, 1, 2>;
 // 1x1 with a stride: the tile loader gathers the sampled x element by element, which costs several times what the
 // aligned float4 loads of a stride-1 plane cost, so a workgroup takes 64 output channels per staged tile instead of
 // 32 (eight per lane, chunks of eight input channels to stay within 128 registers); ResNet-50's three downsample
@@ -586,11 +497,6 @@ using Fwd1x1sub = Tile3x3Cfg<4, 16, 1, 4, 8, 8, 8, 8, 1, 1>;   // 64 sampled pos
 using Fwd1x1q  = Tile3x3Cfg<4, 64, 1, 1, 4, 8, 16, 4, 1, 1>;   // 256 positions of one image x 32 channels
 using Fwd1x1sq = Tile3x3Cfg<4, 16, 1, 4, 4, 8, 16, 4, 1, 1>;   // planes of <= 64 positions: four images
 
-// ... the same register tile in workgroups of four waves that cover fewer rows, for maps whose height is not a
-// multiple of 16: 56 rows are 7 x 8, 28 rows 7 x 4 (ResNet-50 at batch 64: 64 -> 64 @56x56 340 -> 294 us,
-// 128 -> 128 @28x28 330 -> 298 us); on 32 rows they are no faster than FwdW32
-using FwdW32H8 = Tile3x3Cfg<4, 8, 8, 1, 4, 4, 8, 1, 1>;    // 8 rows of one image x 16 channels
-using FwdW32H4 = Tile3x3Cfg<4, 8, 4, 2, 4, 4, 8, 1, 1>;    // 4 rows of two images x 16 channels
 // 5x5 taps: a unit is one output channel x one input channel as well (25 weights, 50*TN vector instructions); five
 // strips of eight values per buffer leave room for two output channels per lane.  Two vector instructions per term
 // bound it: 32 -> 64 @16x16, 64 images (0.84e9 terms, 27 us at the issue ceiling): generic kernel 247 us, this 40 us.
@@ -600,13 +506,7 @@ using Fwd5W8    = Tile3x3Cfg<4, 2, 8, 4, 2, 8, 8, 1, 1, 5>;     // outputs up to
 using Fwd5W16S2 = Tile3x3Cfg<2, 8, 8, 1, 2, 8, 8, 1, 2, 5>;     // stride 2: 8 rows x 16 outputs of one image
 using Fwd5W8S2  = Tile3x3Cfg<2, 4, 8, 2, 2, 8, 8, 1, 2, 5>;     // stride 2, outputs up to 8 wide: two images
 
-// rows per tile (16, 8 or 4) that pad a map of H rows least; the larger tile on a tie
-static int rows_per_tile_w32(int H) {
-    const int p16 = round_up(H, 16), p8 = round_up(H, 8), p4 = round_up(H, 4);
-    return p16 <= p8 && p16 <= p4 ? 16 : (p8 <= p4 ? 8 : 4);
-}
-
-// which tiled kernel serves these dimensions (0 = none): 1..3 3x3 stride 1 by output width, 4..5 3x3 stride 2,
+// which tiled kernel serves these dimensions (0 = none): 1..3 3x3 stride 1 by output width, 4..5 3x3 stride 2 (all fwd_nine.hip),
 // 6..7 1x1 stride 1 by plane size (both fwd_tap.hip), 8..9 1x1 with a stride (the sampled positions walked like a stride-1 plane),
 // 10..13 = 6..9 for channels that are no multiple of 8, 14..18 5x5 (stride 1 by output width, then stride 2)
 static int fwd_tiled_variant(const ConvDims &d) {
@@ -631,34 +531,15 @@ static int fwd_tiled_variant(const ConvDims &d) {
     return 0;
 }
 
-// input channels per first-level sum of the kernel that serves these dimensions
-static int fwd_chunk(const ConvDims &d, int variant) {
-    switch (variant) {
-        case 1: return FwdW32::CC;
-        case 2: return FwdW16::CC;
-        case 3: return FwdW8::CC;
-        case 4: return FwdW16S2::CC;
-        case 5: return d.Ci >= 128 ? FwdW8S2L::CC : FwdW8S2::CC;
-        case 8: case 9: return Fwd1x1sub::CC;
-        default: return Fwd1x1q::CC;
-    }
-}
-static_assert(FwdW32::CC == FwdW32H8::CC && FwdW32::CC == FwdW32H4::CC && Fwd1x1q::CC == Fwd1x1sq::CC,
-              "one chunk length per variant");
-
-// Whether the kernel for few positions takes a 3x3 or 1x1 layer.  The tiled kernels last as long as one wave's chain of
-// channels x taps x results per lane, 6 ns a term, until the chip is full; this one has a chain of its share of the
-// channels (0.4 us each with nine taps, 0.25 with one) and then works at 10.9 (nine taps) or 3.2 (one tap) terms per ps.
-// Fitted to 48 layers; us, tiled -> this: 64 -> 64 3x3 @8x8, 1 / 16 / 64 images, 27 -> 8, 28 -> 8, 28 -> 17; 512 -> 512 3x3
-// @7x7, 1 / 4 images, 205 -> 30, 213 -> 69; 1024 -> 256 1x1 @14x14, 1 / 4 images, 105 -> 34, 105 -> 94.  Beyond the line
-// the tiled kernels win: 16 -> 16 3x3 @32x32, 64 images, 15 against 18; 1024 -> 256 1x1 @14x14, 16 images, 106 against 281.
-// (The plain 1x1 kernel has short chains; 5x5 layers are not built here.)
+// Whether a 3x3 or 1x1 layer has few positions.  1x1 layers with a stride run the kernel above then: the tiled kernel lasts as long as
+// one wave's chain of channels x results per lane, 6 ns a term, until the chip is full; this one has a chain of its share of the
+// channels (0.25 us each) and then works at 3.2 terms per ps.  For the other layers it is a class of sizes that fwd_kernel tells
+// apart: fwd_nine.hip and fwd_tap.hip choose their shapes by rules of their own.
 static bool few_positions(const ConvDims &d, int variant) {
     if (variant == 0 || variant >= 14 || ceil_div(d.Co, kFewTM) > kMaxGridY) return false;
-    const int per_lane = variant == 3 ? FwdW8::TM * FwdW8::TN : variant == 4 || variant == 5 ? FwdW16S2::TM * FwdW16S2::TN
-                       : variant == 8 || variant == 9 ? Fwd1x1sub::TM * Fwd1x1sub::TN : FwdW32::TM * FwdW32::TN;
+    const int per_lane = variant >= 3 && variant <= 5 ? 8 : variant == 8 || variant == 9 ? 32 : 16;
+    const int chunk = variant == 1 || variant == 4 || variant == 8 || variant == 9 || (variant == 5 && d.Ci >= 128) ? 8 : 16;
     const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;
-    const int chunk = fwd_chunk(d, variant);
     const float tiled = 0.006f * d.K() * per_lane;
     const float share = (float)(ceil_div(ceil_div(d.Ci, chunk), 8) * chunk);
     const float few = 2.f + (d.kh == 3 ? 0.4f * share + terms / 10.9e6f : 0.25f * share + terms / 3.2e6f);
@@ -678,35 +559,26 @@ static Subsample sampling_of(const ConvDims &d) { return Subsample{d.stride, d.W
 // A strided 3x3 / pad 1 layer and the strided 1x1 / pad 0 layer beside it (same x, same Co, Ho, Wo) in one launch;
 // d describes the 3x3 layer.  Both outputs with their statistics (fwd_stats_slots(d) slots each).  Rows of whole
 // float4 groups only; ADDER_ERR_UNSUPPORTED otherwise.
-template <class C>
-static int launch_fwd_pair_3x3(const float *x, const float *w, const float *w_side, float *y, float *y_side,
-                               double *stats, double *stats_side, const ConvDims &d, hipStream_t s) {
-    const int tilesH = ceil_div(d.Ho, C::TH), tilesW = ceil_div(d.Wo, C::TW);
-    const long gx = (long)ceil_div(d.N, C::NIMG) * tilesH * tilesW;
-    const int gy = ceil_div(d.Co, C::TM * C::COW);
-    if (gx > 0x7fffffffL) return ADDER_ERR_TOO_LARGE;
-    if (int rc = allow_dynamic_lds<&fwd_3x3_kernel<C, true, false, false, float, true>>(C::LDS_BYTES)) return rc;
-    hipLaunchKernelGGL((fwd_3x3_kernel<C, true, false, false, float, true>), dim3((unsigned)gx, gy), dim3(C::NTHREADS),
-                       C::LDS_BYTES, s, x, w, y, stats, d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, tilesH, tilesW,
-                       Subsample{1, 0, 0, 0}, kNoBnEval, w_side, y_side, stats_side);
-    return check_launch();
-}
-
 bool fwd_pair_supported(const ConvDims &d) {
-    return d.kh == 3 && d.kw == 3 && d.pad == 1 && d.stride == 2 && d.W % 4 == 0 && d.H % 2 == 0 && d.W % 2 == 0;
+    return fwd_nine_supported(d) && d.stride == 2 && d.W % 4 == 0 && d.H % 2 == 0;
 }
 
 int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats,
                     double *stats_side, const ConvDims &d, hipStream_t s) {
     if (!fwd_pair_supported(d)) return ADDER_ERR_UNSUPPORTED;
-    if (d.Wo > 8) return launch_fwd_pair_3x3<FwdW16S2>(x, w, w_side, y, y_side, stats, stats_side, d, s);
-    return d.Ci >= 128 ? launch_fwd_pair_3x3<FwdW8S2L>(x, w, w_side, y, y_side, stats, stats_side, d, s)
-                       : launch_fwd_pair_3x3<FwdW8S2>(x, w, w_side, y, y_side, stats, stats_side, d, s);
+    return launch_fwd_nine<float>(x, w, y, stats, d, s, kNoBnEval, false, w_side, y_side, stats_side);
+}
+
+// rows per tile (16, 8 or 4) that pad a map of H rows least; the larger tile on a tie
+static int rows_per_tile_w32(int H) {
+    const int p16 = round_up(H, 16), p8 = round_up(H, 8), p4 = round_up(H, 4);
+    return p16 <= p8 && p16 <= p4 ? 16 : (p8 <= p4 ? 8 : 4);
 }
 
 // Which kernel launch_fwd runs without statistics and for bases aligned to groups of four: 0 general, 1 plain 1x1, 2 few
-// positions, else 10 * variant + which of its tiles (rows 16 / 8 / 4: 0 / 1 / 2; channels from 128 on: 1).  1x1 layers of stride 1
-// are told apart by the same rules, but one kernel runs them all, with the same bits (fwd_tap.hip).
+// positions, else 10 * variant + a class of sizes (3x3 on wide maps: whole groups of 16 / 8 / 4 rows 0 / 1 / 2; 5: channels from 128 on 1).
+// One kernel, with shapes of its own, runs all the classes of the 3x3 layers (fwd_nine.hip), and one those of the 1x1 layers of
+// stride 1 (fwd_tap.hip), number 2 included.
 int fwd_kernel(const ConvDims &d) {
     const int variant = fwd_tiled_variant(d);
     if (few_positions(d, variant)) return 2;
@@ -717,17 +589,9 @@ int fwd_kernel(const ConvDims &d) {
 
 int fwd_stats_slots(const ConvDims &d) {
     if (fwd_tap_supported(d)) return fwd_tap_stats_slots(d);
+    if (fwd_nine_supported(d)) return fwd_nine_stats_slots(d);
     if (d.kh == 1 && few_positions(d, fwd_tiled_variant(d))) return ceil_div(d.N * d.Ho * d.Wo, 64);
     switch (fwd_tiled_variant(d)) {
-        case 1: switch (rows_per_tile_w32(d.Ho)) {
-            case 16: return stats_slots_3x3<FwdW32>(d);
-            case 8: return stats_slots_3x3<FwdW32H8>(d);
-            default: return stats_slots_3x3<FwdW32H4>(d);
-        }
-        case 2: return stats_slots_3x3<FwdW16>(d);
-        case 3: return stats_slots_3x3<FwdW8>(d);
-        case 4: return stats_slots_3x3<FwdW16S2>(d);
-        case 5: return stats_slots_3x3<FwdW8S2>(d);
         case 8: case 9: return stats_slots_3x3<Fwd1x1sub>(as_one_row(d));
         case 12: return stats_slots_3x3<Fwd1x1q>(as_one_row(d));
         case 13: return stats_slots_3x3<Fwd1x1sq>(as_one_row(d));
@@ -749,31 +613,23 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
         if (stats && !few && d.H * d.W % 4 == 0 && !(aligned_groups(x) && aligned_groups(y))) return ADDER_ERR_UNSUPPORTED;
         return launch_fwd_tap(x, w, y, stats, d, s, bn);
     }
-    if ((!stats || d.kh == 1) && few) {   // (its statistics are offered for 1x1 layers: fwd_stats_slots)
-        const int chunk = fwd_chunk(d, variant);
-        return d.kh == 3 ? launch_fwd_few<3>(x, w, y, stats, d, chunk, s, bn) : launch_fwd_few<1>(x, w, y, stats, d, chunk, s, bn);
+    if (d.kh == 1 && few)
+        return launch_fwd_few(x, w, y, stats, d, variant <= 9 ? Fwd1x1sub::CC : Fwd1x1q::CC, s, bn);
+    if (fwd_nine_supported(d)) {
+        if (stats && !rows_ok) return ADDER_ERR_UNSUPPORTED;   // (it takes bases of any alignment; statistics are offered for aligned ones)
+        return launch_fwd_nine(x, w, y, stats, d, s, bn);
     }
     const bool strided = variant == 8 || variant == 9 || variant == 12 || variant == 13;
     if (strided) {   // x is read element by element; y is a dense row per plane
         const ConvDims f = as_one_row(d);
         if (f.Wo % 4 != 0 || aligned_groups(y)) switch (variant) {
-            case 8: case 9: return launch_fwd_3x3_v<Fwd1x1sub, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d), bn);
-            case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d), bn);
-            default: return launch_fwd_3x3_v<Fwd1x1sq, false, true, false, T>(x, w, y, stats, f, s, sampling_of(d), bn);
+            case 8: case 9: return launch_fwd_3x3_v<Fwd1x1sub, false, true, T>(x, w, y, stats, f, s, sampling_of(d), bn);
+            case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true, T>(x, w, y, stats, f, s, sampling_of(d), bn);
+            default: return launch_fwd_3x3_v<Fwd1x1sq, false, true, T>(x, w, y, stats, f, s, sampling_of(d), bn);
         }
     }
-    if (rows_ok && !(stats && variant >= 14)) {   // 3x3 and 5x5 taps; statistics are offered for 3x3 and 1x1 layers
+    if (rows_ok && !stats) {   // 5x5 taps; statistics are offered for 3x3 and 1x1 layers
         switch (variant) {
-            case 1: switch (rows_per_tile_w32(d.Ho)) {
-                case 16: return launch_fwd_3x3<FwdW32>(x, w, y, stats, d, s, bn);
-                case 8: return launch_fwd_3x3<FwdW32H8>(x, w, y, stats, d, s, bn);
-                default: return launch_fwd_3x3<FwdW32H4>(x, w, y, stats, d, s, bn);
-            }
-            case 2: return launch_fwd_3x3<FwdW16>(x, w, y, stats, d, s, bn);
-            case 3: return launch_fwd_3x3<FwdW8>(x, w, y, stats, d, s, bn);
-            case 4: return launch_fwd_3x3<FwdW16S2>(x, w, y, stats, d, s, bn);
-            case 5: return d.Ci >= 128 ? launch_fwd_3x3<FwdW8S2L>(x, w, y, stats, d, s, bn)
-                                       : launch_fwd_3x3<FwdW8S2>(x, w, y, stats, d, s, bn);
             case 14: return launch_fwd_3x3<Fwd5W32>(x, w, y, stats, d, s, bn);
             case 15: return launch_fwd_3x3<Fwd5W16>(x, w, y, stats, d, s, bn);
             case 16: return launch_fwd_3x3<Fwd5W8>(x, w, y, stats, d, s, bn);
@@ -798,22 +654,14 @@ template int launch_fwd<float>(const float *, const float *, float *, double *, 
 template int launch_fwd<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t,
                                 const BnEval &);
 
-// An ordinary convolution y = sum w * x through the tiled forward kernels: 3x3 / stride 1 / pad 1 only
+// An ordinary convolution y = sum w * x through the 3x3 forward kernel: 3x3 / stride 1 / pad 1 only
 // (ADDER_ERR_UNSUPPORTED elsewhere).  stats as in launch_fwd; the slot count is fwd_stats_slots(d).
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s) {
     const bool ok = d.kh == 3 && d.kw == 3 && d.pad == 1 && d.stride == 1 &&
                     (d.W % 4 != 0 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0);
     if (!ok) return ADDER_ERR_UNSUPPORTED;
-    switch (fwd_tiled_variant(d)) {
-        case 1: switch (rows_per_tile_w32(d.Ho)) {   // (the statistics slots are counted per tile shape)
-            case 16: return launch_mulconv_3x3<FwdW32>(x, w, y, stats, d, s);
-            case 8: return launch_mulconv_3x3<FwdW32H8>(x, w, y, stats, d, s);
-            default: return launch_mulconv_3x3<FwdW32H4>(x, w, y, stats, d, s);
-        }
-        case 2: return launch_mulconv_3x3<FwdW16>(x, w, y, stats, d, s);
-        case 3: return launch_mulconv_3x3<FwdW8>(x, w, y, stats, d, s);
-        default: return ADDER_ERR_UNSUPPORTED;
-    }
+    if (!fwd_nine_supported(d)) return ADDER_ERR_UNSUPPORTED;
+    return launch_fwd_nine<float>(x, w, y, stats, d, s, kNoBnEval, true);
 }
 
 }  // namespace adder

@@ -1,0 +1,307 @@
+// Forward of 3x3 / pad 1 layers, stride 1 or 2, NCHW in -> NCHW out:
+//   y[n,co,ho,wo] = - sum_{ci,i,j} | w[co,ci,i,j] - xpad[n,ci,ho*s+i-1,wo*s+j-1] |
+// Replaces adder_cuda/adder.cu:19-70 (CONV) together with the unfold + permute copies of adder.py:32-33,38-39 that feed it.
+//
+// Two vector instructions per term bound it: v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- 73 T lane-instructions/s is what a bare
+// stream of the pair reaches with two waves on each of a SIMD's two issue ports (62 T with one each).  Weights are wave-uniform and come
+// through the scalar cache as scalar operands.  A lane reads the window of its strip straight into registers, one channel ahead: nine
+// reads of at most 16 bytes serve 576 instructions, a quarter of what L1 delivers, so a tile in LDS, its barriers and its halo
+// columns had nothing to give.  Without a tile the strips of all images line up (14 columns are 4 strips, 56 are 14: 88 and 100 % of
+// the lanes have work where 16 x 16 and 8 x 32 tiles left 77 and 88 %), and the waves of a workgroup can share the input channels
+// instead of the positions, which is what small maps with many channels need.
+// us, tiles in LDS -> this: 32 images 64 -> 64 @56x56 158 -> 136, 128 -> 128 @28x28 180 -> 142, 256 -> 256 @14x14 186 -> 163, 512 -> 512 @7x7
+// 284 -> 190, 100 -> 100 @20x20 112 -> 53; 128 images 128 -> 128 @32x32 648 -> 625, 512 -> 512 @8x8 716 -> 688; 256 images 16 -> 16 @32x32 27.0 -> 26.2,
+// 64 -> 64 @8x8 28.6 -> 25.7; stride 2, 32 images 128 -> 128 @56x56 222 -> 152, 512 -> 512 @14x14 375 -> 203; one image (the kernel for few
+// positions there was) 64 -> 64 @8x8 7.9 -> 5.9, 256 -> 256 @14x14 19 -> 16, 512 -> 512 @7x7 30 -> 29.
+// Tried on the way: 4 channels x 4 positions per lane 132 -> 179 us (64 -> 64 @56x56: reads), 8 x 2 143.
+#include "wave_split.hpp"
+
+#include <type_traits>
+
+namespace adder {
+
+// S: stride; TM output channels x TN adjacent positions per lane; KSP waves that share the input channels in chunks of CC
+// EVEN (stride 2): rows of an even length, whose strips' columns and the one behind them are one read
+template <int S_, int TM_, int TN_, int KSP_, bool EVEN_ = false>
+struct NineCfg {
+    static constexpr int S = S_, TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = kNineChunk, FM = kFinished<TM, KSP>;
+    static constexpr bool EVEN = EVEN_;
+    static constexpr int AHEAD = TN == 1 ? 3 : 1;   // input channels that x is asked for ahead of the arithmetic
+    // Output channels whose weights are asked for together, a step ahead: a step of one channel x four positions is 72 instructions,
+    // enough to hide the request behind; with fewer positions two channels (stride 2: 512 -> 512 @14x14 284 -> 203 us, 256 -> 256 @28x28
+    // 181 -> 158; 512 -> 512 @7x7, one image, 32 -> 29).  Two x four positions run out of scalar registers (132 -> 180 us).
+    static constexpr int UM = TN == 4 ? 1 : 2, NU = TM / UM;
+    static constexpr int MID = (TN - 1) * S + 1, STRIP = MID + 2;   // columns under the strip, and with one more on either side
+    static constexpr int LDS_BYTES = KSP == 1 ? 0 : KSP * TM * TN * 64 * 4;
+    static_assert((TM % KSP == 0 || KSP % TM == 0) && (NU == 1 || NU % 2 == 0), "a wave finishes FM channels or none; two weight buffers");
+};
+
+struct NineDims {
+    int N, Ci, H, W, Co, Ho, Wo;
+    int per_row, strips;    // strips of TN positions per row (the last one is moved back to end at Wo) and per image
+    int tiles, blocks;      // of 64 strips, of TM output channels
+};
+
+// Columns c .. c + MID - 1 of a row, where c + k < W holds for every k that has a position
+template <int S, int MID, class T>
+__device__ __forceinline__ void load_mid(const T *p, float *v) {
+    if constexpr (S == 1) {
+        float u[MID];
+        ld_strip<MID>(p, u);
+#pragma unroll
+        for (int k = 0; k < MID; ++k) v[k] = u[k];
+    } else if constexpr (MID == 3) {
+        float u[2];
+        ld_strip<2>(p, u);
+        v[0] = u[0];
+        v[1] = u[1];
+        v[2] = ldf(p + 2);
+    } else {
+        v[0] = ldf(p);
+    }
+}
+
+// MUL: an ordinary convolution, y = sum w * x (one v_fmac per term), for the regular stem layer that precedes the adder layers of a
+// network.  EVAL: the inference epilogue.  PAIR (stride 2): the strided 1x1 layer that reads the same x beside this layer (the downsample branch
+// of a residual block, resnet20.py:66-70) along with it -- its one tap is the centre tap of the 3x3 window: weights w_side (Co, Ci),
+// output y_side and statistics stats_side shaped like y and stats.
+template <class C, class T, bool MUL, bool EVAL, bool PAIR>
+__global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
+                                                         double *__restrict__ stats, const NineDims d, const BnEval bn,
+                                                         const float *__restrict__ w_side, T *__restrict__ y_side,
+                                                         double *__restrict__ stats_side) {
+    constexpr int S = C::S, TM = C::TM, TN = C::TN, KSP = C::KSP, FM = C::FM, MID = C::MID, STRIP = C::STRIP, NB = C::AHEAD + 1, UM = C::UM, NU = C::NU;
+    extern __shared__ __align__(16) float smem[];
+    int tile, blk;
+    xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
+    const int ho = rest / d.per_row, s = rest - ho * d.per_row, wo = min(s * TN, d.Wo - TN), co_base = blk * TM;
+    const int plane = d.H * d.W, K = d.Ci * 9;
+    uniform_f32_ptr wc = as_uniform(w), wsc = as_uniform(w_side);
+    int wrow[TM], wsrow[PAIR ? TM : 1];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+        wrow[m] = min(co_base + m, d.Co - 1) * K;
+        if constexpr (PAIR) wsrow[m] = min(co_base + m, d.Co - 1) * d.Ci;
+    }
+    // A uniform base per channel and the lane's distances from it in bytes (64 strips: far below 2^32), per row of the window: the
+    // strip's own columns and the ones beside them.  What lies outside the map reads an element inside and is zeroed.
+    const int n_first = __builtin_amdgcn_readfirstlane(n);
+    const T *x_first = x + (size_t)n_first * d.Ci * plane;
+    const int c0 = wo * S;
+    const bool ok_l = c0 > 0, ok_r = c0 + MID < d.W;
+    bool ok[3];
+    unsigned off[3], off_l[3], off_r[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int h = ho * S + i - 1;
+        ok[i] = h >= 0 && h < d.H;
+        const int o = (n - n_first) * d.Ci * plane + min(max(h, 0), d.H - 1) * d.W + c0;
+        off[i] = (unsigned)o * (unsigned)sizeof(T);
+        off_l[i] = (unsigned)(ok_l ? o - 1 : o) * (unsigned)sizeof(T);
+        off_r[i] = (unsigned)(ok_r ? o + MID : o) * (unsigned)sizeof(T);
+    }
+
+    float acc[TM][TN], tot[TM][TN], side[PAIR ? TM : 1][TN];   // side: Ci / KSP terms each, one level
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            acc[m][t] = tot[m][t] = 0.f;
+            if constexpr (PAIR) side[m][t] = 0.f;
+        }
+    float xr[NB][3][STRIP], wv[2][UM][9], wsv[2][UM];
+    auto load_x = [&](const int b, const int ci) {
+        const char *p = reinterpret_cast<const char *>(x_first + (size_t)ci * plane);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            if constexpr (C::EVEN) {
+                float u[MID + 1];
+                ld_strip<MID + 1>(reinterpret_cast<const T *>(p + off[i]), u);
+#pragma unroll
+                for (int k = 0; k <= MID; ++k) xr[b][i][k + 1] = u[k];
+            } else {
+                load_mid<S, MID>(reinterpret_cast<const T *>(p + off[i]), &xr[b][i][1]);
+                xr[b][i][MID + 1] = ldf(reinterpret_cast<const T *>(p + off_r[i]));
+            }
+            xr[b][i][0] = ldf(reinterpret_cast<const T *>(p + off_l[i]));
+        }
+    };
+    auto load_w = [&](const int b, const int h, const int ci) {
+#pragma unroll
+        for (int u = 0; u < UM; ++u) {
+#pragma unroll
+            for (int e = 0; e < 9; ++e) wv[b][u][e] = wc[wrow[h * UM + u] + ci * 9 + e];
+            if constexpr (PAIR) wsv[b][u] = wsc[wsrow[h * UM + u] + ci];
+        }
+    };
+    auto after = [&](const int c) { return ((c + 1) & (C::CC - 1)) == 0 ? c + 1 + (KSP - 1) * C::CC : c + 1; };
+    int ci = wave * C::CC;
+    if (ci < d.Ci) {
+        int cl = ci;   // the channel that x is read of next (the last one again behind the end)
+#pragma unroll
+        for (int b = 0; b < C::AHEAD; ++b) {
+            load_x(b, cl);
+            const int c = after(cl);
+            cl = c < d.Ci ? c : cl;
+        }
+        load_w(0, 0, ci);
+        // one input channel; weights one output channel ahead of the arithmetic
+        auto channel = [&](const int cur) -> bool {
+            const int next = after(ci);
+            const bool chunk_end = ((ci + 1) & (C::CC - 1)) == 0, more = next < d.Ci;
+            const int cn = more ? next : ci;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                if (i != 1) {   // (the middle row is inside the map)
+#pragma unroll
+                    for (int k = 1; k <= MID; ++k) xr[cur][i][k] = ok[i] ? xr[cur][i][k] : 0.f;
+                }
+                xr[cur][i][0] = ok[i] && ok_l ? xr[cur][i][0] : 0.f;
+                xr[cur][i][MID + 1] = ok[i] && (C::EVEN || ok_r) ? xr[cur][i][MID + 1] : 0.f;
+            }
+#pragma unroll
+            for (int h = 0; h < NU; ++h) {
+                const int wb = (NU == 1 ? cur : h) & 1;
+#pragma unroll
+                for (int idx = 0; idx < UM * 9 * TN; ++idx) {
+                    const int t = idx % TN, j = idx / TN % 3, i = idx / TN / 3 % 3, u = idx / TN / 9, m = h * UM + u;
+                    const float a = wv[wb][u][i * 3 + j], b = xr[cur][i][t * S + j];
+                    if constexpr (MUL) acc[m][t] = fmaf(a, b, acc[m][t]);
+                    else acc[m][t] -= fabsf(a - b);
+                    if (idx == 0) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_w(wb ^ 1, h + 1 < NU ? h + 1 : 0, h + 1 < NU ? ci : cn);
+                        if (h == 0) load_x((cur + C::AHEAD) % NB, cl);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                if constexpr (PAIR) {
+#pragma unroll
+                    for (int u = 0; u < UM; ++u)
+#pragma unroll
+                        for (int t = 0; t < TN; ++t) side[h * UM + u][t] -= fabsf(wsv[wb][u] - xr[cur][1][t * S + 1]);
+                }
+            }
+            ci = next;
+            {
+                const int c = after(cl);
+                cl = c < d.Ci ? c : cl;
+            }
+            if (chunk_end || !more) {
+#pragma unroll
+                for (int m = 0; m < TM; ++m)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) { tot[m][t] += acc[m][t]; acc[m][t] = 0.f; }
+            }
+            return more;
+        };
+#pragma unroll 1
+        while (channel(0) && channel(1) && (NB == 2 || (channel(2) && channel(NB - 1)))) {}
+        static_assert(NB == 2 || NB == 4, "the buffers take turns");
+    }
+
+    unsigned own = 0;   // bit t: position wo + t is this lane's
+#pragma unroll
+    for (int t = 0; t < TN; ++t) own |= (sidx == sc && wo + t >= s * TN ? 1u : 0u) << t;
+    const int L = d.Ho * d.Wo, yoff = n * d.Co * L + ho * d.Wo + wo;
+    const bool whole = TN > 1 && d.Wo % TN == 0;
+    float r[FM][TN];
+    add_waves<TM, TN, KSP>(smem, wave, lane, tot, r);
+    const bool finishes = wave * FM < TM;
+    if (finishes)
+        finish_outputs<FM, TN, EVAL>(r, own, co_base + wave * FM, d.Co, L, yoff, whole, y, stats, d.tiles, tile, lane, bn);
+    if constexpr (PAIR) {
+        __syncthreads();
+        add_waves<TM, TN, KSP>(smem, wave, lane, side, r);
+        if (finishes)
+            finish_outputs<FM, TN, false>(r, own, co_base + wave * FM, d.Co, L, yoff, whole, y_side, stats_side, d.tiles, tile, lane, bn);
+    }
+}
+
+static int nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((long)d.N * d.Ho * ceil_div(d.Wo, tn), 64); }
+
+// Waves that share the channels: one chunk each, as many as eight, by the channels alone, so that a layer's results have the same bits
+// whatever the batch.  us with 2 / 4 / 8: 32 -> 32 @16x16, 256 images, 26 / 26 / 29, 64 -> 64 @8x8 47 / 26 / 25, 64 -> 64 @56x56, 32 images, 145 / 132 / 136,
+// 128 -> 128 @28x28 171 / 145 / 141, 512 -> 512 @7x7 471 / 255 / 189, 128 -> 128 @32x32, 128 images, 648 / 609 / 621.
+static int nine_waves(int Ci) { return Ci <= 8 ? 1 : Ci <= 16 ? 2 : Ci <= 32 ? 4 : 8; }
+
+// Output channels and positions per lane: 8 x 4 (stride 2: 8 x 2), 8 x 2 or 4 x 1, the less the fewer waves there are.  A launch lasts as
+// long as one wave's chain of channels -- 1.43, 0.93 and 0.46 us each -- or as the chip takes for the terms: 30, 26 and 12 per ps, 4 x 1 only
+// 7 on rows that are shorter than 8 and 4.5 at stride 2, where its reads are what fills.  From about 1300 waves of 8 x 4 on the chains
+// overlap.  us, 8 x 4 / 8 x 2 / 4 x 1: 128 -> 128 @28x28, 4 images, 26 / 28 / 35, one image 26 / 17 / 13; 256 -> 256 @14x14, 4, 48 / 32 / 40, one
+// 48 / 32 / 17; 512 -> 512 @7x7, 4 / 2 / 1, 92 / 60 / 68, 92 / 60 / 33, 92 / 60 / 32; 64 -> 64 @56x56, one, 15 / 10 / 13; 16 -> 16 @32x32, 32, 13 / 10 / 8;
+// stride 2: 128 -> 128 @56x56, one image, - / 17 / 29, 512 -> 512 @14x14, one, - / 59 / 34.
+struct NineShape { int tm, tn; };
+static NineShape nine_shape(const ConvDims &d) {
+    const int most = d.stride == 1 ? 4 : 2, waves = nine_waves(d.Ci);
+    int tn = d.Wo >= most ? most : d.Wo >= 2 ? 2 : 1;
+    if (tn == 4 && (long)nine_tiles(d, 4) * ceil_div(d.Co, 8) * waves < 1300) tn = 2;
+    const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;
+    const int chunks = ceil_div(ceil_div(d.Ci, kNineChunk), waves), chain = min(chunks * kNineChunk, d.Ci);
+    const float wide = fmaxf((tn == 4 ? 1.43f : 0.93f) * chain, terms / (tn == 4 ? 30e6f : 26e6f));
+    const float narrow = fmaxf(0.46f * chain, terms / (d.stride == 2 ? 4.5e6f : d.Wo < 8 ? 7e6f : 12e6f));
+    if (narrow < wide) tn = 1;
+    return {tn == 1 ? 4 : 8, tn};
+}
+
+bool fwd_nine_supported(const ConvDims &d) {
+    if (d.kh != 3 || d.kw != 3 || d.pad != 1 || d.stride < 1 || d.stride > 2) return false;
+    const long images = 63 / ((long)d.Ho * ceil_div(d.Wo, 4)) + 1;
+    return (images * d.Ci + 1) * d.H * d.W <= 0x3fffffffL;
+}
+int fwd_nine_stats_slots(const ConvDims &d) { return nine_tiles(d, nine_shape(d).tn); }
+
+template <class C, class T, bool MUL, bool EVAL, bool PAIR>
+static int launch_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn,
+                       const float *w_side, T *y_side, double *stats_side) {
+    const int per_row = ceil_div(d.Wo, C::TN);
+    const NineDims t{d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, per_row, per_row * d.Ho, nine_tiles(d, C::TN), ceil_div(d.Co, C::TM)};
+    const long grid = (long)t.tiles * t.blocks;
+    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
+    if (int rc = allow_dynamic_lds<&fwd_nine_kernel<C, T, MUL, EVAL, PAIR>>(C::LDS_BYTES)) return rc;
+    hipLaunchKernelGGL((fwd_nine_kernel<C, T, MUL, EVAL, PAIR>), dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, s, x, w, y, stats, t, bn,
+                       w_side, y_side, stats_side);
+    return check_launch();
+}
+
+// w_side != null (stride 2, float storage): the pair.  mul (stride 1, float storage): the ordinary convolution.
+template <class T>
+int launch_fwd_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn, bool mul,
+                    const float *w_side, T *y_side, double *stats_side) {
+    auto run = [&](auto cfg) {
+        using C = decltype(cfg);
+        if constexpr (sizeof(T) == 4) {
+            if (bn.gamma) return launch_nine<C, T, false, true, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
+            if constexpr (C::S == 1) {
+                if (mul) return launch_nine<C, T, true, false, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
+            } else {
+                if (w_side) return launch_nine<C, T, false, false, true>(x, w, y, stats, d, s, bn, w_side, y_side, stats_side);
+            }
+        }
+        return launch_nine<C, T, false, false, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
+    };
+    const NineShape shape = nine_shape(d);
+    auto waves = [&](auto ksp) {
+        constexpr int KSP = decltype(ksp)::value;
+        if (d.stride == 1) {
+            if (shape.tn == 4) return run(NineCfg<1, 8, 4, KSP>{});
+            return shape.tn == 2 ? run(NineCfg<1, 8, 2, KSP>{}) : run(NineCfg<1, 4, 1, KSP>{});
+        }
+        if (shape.tn == 2) return d.W % 2 ? run(NineCfg<2, 8, 2, KSP>{}) : run(NineCfg<2, 8, 2, KSP, true>{});
+        return run(NineCfg<2, 4, 1, KSP>{});
+    };
+    switch (nine_waves(d.Ci)) {
+        case 1: return waves(std::integral_constant<int, 1>{});
+        case 2: return waves(std::integral_constant<int, 2>{});
+        case 4: return waves(std::integral_constant<int, 4>{});
+        default: return waves(std::integral_constant<int, 8>{});
+    }
+}
+template int launch_fwd_nine<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t, const BnEval &,
+                                    bool, const float *, float *, double *);
+template int launch_fwd_nine<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t, const BnEval &,
+                                     bool, const float *, bf16_t *, double *);
+
+}  // namespace adder

@@ -13,7 +13,7 @@
 //   one image (there the kernel for few positions) 34 -> 18; 300 -> 48 @8x8, 64 images 36 -> 8.
 // Tried on the way: sums of sums in LDS instead of registers (116 -> 84 registers) 131 -> 141 us; 16 channels x 2 positions per lane
 // 146 -> 187; the next chunk's weight lines asked for a chunk early 131 -> 140; x of eight waves staged in LDS 1024 -> 256 176.
-#include "common.hpp"
+#include "wave_split.hpp"
 
 #include <type_traits>
 
@@ -110,82 +110,13 @@ __global__ __launch_bounds__(C::NT) void fwd_tap_kernel(const T *__restrict__ x,
         while (half(0) && half(1)) {}
     }
 
-    // every wave finishes FM of the channels: the waves' sums are added in the order of the waves
     float r[FM][TN];
-#pragma unroll
-    for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int t = 0; t < TN; ++t) smem[((wave * TM + m) * TN + t) * 64 + lane] = tot[m][t];
-    __syncthreads();
-    const int m0 = wave * FM;
-#pragma unroll
-    for (int f = 0; f < FM; ++f)
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            float v = smem[((m0 + f) * TN + t) * 64 + lane];
-#pragma unroll
-            for (int k = 1; k < KSP; ++k) v += smem[((k * TM + m0 + f) * TN + t) * 64 + lane];
-            r[f][t] = v;
-        }
-
-    const int co0 = co_base + m0;
+    add_waves<TM, TN, KSP>(smem, wave, lane, tot, r);
     unsigned own = 0;   // bit t: position p0 + t is this lane's
 #pragma unroll
     for (int t = 0; t < TN; ++t) own |= (sidx == sc && p0 + t >= s * TN ? 1u : 0u) << t;
-    if (stats) {
-        // as in fwd.hip: sums of deviations from a pivot in fp32, moved back to the origin in fp64; one slot per tile
-        const double count = (double)wave_sum_dpp((float)__popc(own));
-#pragma unroll
-        for (int f = 0; f < FM; ++f) {
-            const float pivot = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r[f][0])));
-            float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-            for (int t = 0; t < TN; ++t)
-                if (own >> t & 1) {
-                    const float dv = r[f][t] - pivot;
-                    s1 += dv;
-                    s2 = fmaf(dv, dv, s2);
-                }
-            const double d1 = (double)wave_sum_dpp(s1), d2 = (double)wave_sum_dpp(s2), c = (double)pivot;
-            if (lane == 0 && co0 + f < d.Co) {
-                double *dst = stats + ((size_t)(co0 + f) * d.tiles + tile) * 2;
-                dst[0] = d1 + count * c;
-                dst[1] = d2 + 2.0 * c * d1 + count * c * c;
-            }
-        }
-    }
-    const int yoff = n * d.Co * d.L + p0;
-    const bool whole = TN == 4 && (d.L & 3) == 0;
-    if constexpr (EVAL) {
-        float a[FM][TN];
-#pragma unroll
-        for (int f = 0; f < FM; ++f) {   // (all loads before the first store: one counter serves both)
-#pragma unroll
-            for (int t = 0; t < TN; ++t) a[f][t] = 0.f;
-            if (bn.res) ld_strip<TN>(bn.res + (size_t)min(co0 + f, d.Co - 1) * d.L + yoff, a[f]);
-        }
-#pragma unroll
-        for (int f = 0; f < FM; ++f) {
-            const BnEvalChannel ch(bn, min(co0 + f, d.Co - 1));
-#pragma unroll
-            for (int t = 0; t < TN; ++t) {
-                r[f][t] = ch(r[f][t]) + a[f][t];
-                if (bn.relu) r[f][t] = relu_keep_nan(r[f][t]);
-            }
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < FM; ++f) {
-        if (co0 + f >= d.Co) break;
-        T *dst = y + (size_t)(co0 + f) * d.L + yoff;
-        if (whole && own) {
-            if constexpr (TN == 4) st_strip<TN>(dst, r[f]);
-        } else {
-#pragma unroll
-            for (int t = 0; t < TN; ++t)
-                if (own >> t & 1) stf(dst + t, r[f][t]);
-        }
-    }
+    finish_outputs<FM, TN, EVAL>(r, own, co_base + wave * FM, d.Co, d.L, n * d.Co * d.L + p0, TN > 1 && d.L % TN == 0, y, stats, d.tiles,
+                                 tile, lane, bn);
 }
 
 template <class C, class T>

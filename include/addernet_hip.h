@@ -83,7 +83,8 @@ ADDER_API int adder_conv2d_fwd_f32(const float *x, const float *w, float *y,
                          int stride, int pad, void *stream);
 
 /* Which kernel the forward calls above and below (without statistics) take for the dimensions and aligned tensors, in the
- * dispatch's own numbers: 0 the general one, 1 the plain 1x1 one, 2 the one for few positions, from 10 on the tiled ones.
+ * dispatch's own numbers: 0 the general one, 1 the plain 1x1 one, 2 few positions, from 10 on by taps, stride and map.  (The
+ * 3x3 layers of 2 and 10 to 51 share one kernel, the 1x1 layers of stride 1 of 2, 60, 70, 100 and 110 another.)
  * Host code only; for tests that have to reach a certain kernel, and no promise that the numbers stay. */
 ADDER_API int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel);
 
