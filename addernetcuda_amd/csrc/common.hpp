@@ -113,6 +113,10 @@ __device__ __forceinline__ void st_strip(bf16_t *p, const float (&v)[CNT]) {
         *reinterpret_cast<u16x2_any *>(p) = u16x2_any{f32_to_bf16(v[0]), f32_to_bf16(v[1])};
 }
 
+// A lane's 32-bit byte offset from a uniform base, used in a loop: without this the compiler widens it to 64 bits in front of the loop and
+// adds base and offset in vector registers at every load; with it the load takes both as they are.
+__device__ __forceinline__ void keep_offset(unsigned &off) { asm volatile("" : "+v"(off)); }
+
 static constexpr int kTapChunk = 16;   // channels per first-level sum of the 1x1 kernels without tiles (fwd_tap.hip, grad_x_tap.hip)
 static constexpr int kNineChunk = 8;   // ... of the 3x3 forward without tiles (fwd_nine.hip): 72 terms
 
@@ -349,6 +353,13 @@ int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const Conv
                       const adder_bn_links *bn);
 bool grad_x_tap_supported(const ConvDims &d);
 int grad_x_tap_bn_slots(const ConvDims &d);
+// 3x3 / pad 1 / stride 1 (grad_x_nine.hip), likewise
+template <class T>
+int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
+                       const adder_bn_links *bn);
+bool grad_x_nine_supported(const ConvDims &d);
+int grad_x_nine_bn_slots(const ConvDims &d);
+static constexpr int kSatMaxTerms = 1152;      // terms up to which a 3x3 layer's input gradient takes two instructions a term (grad_x.hip)
 static constexpr int kSatMaxTerms1x1 = 1024;   // output channels up to which a single tap's input gradient takes two instructions a term (grad_x.hip)
 size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false, size_t limit = SIZE_MAX);   // of the storage type's kernels
 int grad_w_kernel(const ConvDims &d, bool bf16);                                                // which of them, as in adder_conv2d_grad_w_kernel

@@ -116,6 +116,8 @@ __global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x
         const char *p = reinterpret_cast<const char *>(x_first + (size_t)ci * plane);
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
+            keep_offset(off[i]); keep_offset(off_l[i]);
+            if constexpr (!C::EVEN) keep_offset(off_r[i]);
             if constexpr (C::EVEN) {
                 float u[MID + 1];
                 ld_strip<MID + 1>(reinterpret_cast<const T *>(p + off[i]), u);

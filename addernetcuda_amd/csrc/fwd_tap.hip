@@ -60,9 +60,10 @@ __global__ __launch_bounds__(C::NT) void fwd_tap_kernel(const T *__restrict__ x,
     float xr[2][CQ][TN], wv[2][UM][CQ];
     // a uniform base per channel and the lane's distance from it in bytes (64 strips: far below 2^32): no address registers
     const int n_first = __builtin_amdgcn_readfirstlane(n);
-    const unsigned xoff = (unsigned)((n - n_first) * d.Ci * d.L + p0) * (unsigned)sizeof(T);
+    unsigned xoff = (unsigned)((n - n_first) * d.Ci * d.L + p0) * (unsigned)sizeof(T);
     const T *x_first = x + (size_t)n_first * d.Ci * d.L;
     auto load_x = [&](const int b, const int ci) {
+        keep_offset(xoff);
 #pragma unroll
         for (int e = 0; e < CQ; ++e) ld_strip<TN>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(x_first + (size_t)(ci + e) * d.L) + xoff), xr[b][e]);
     };

@@ -555,7 +555,7 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
 // Below ten output channels the doubled and the subtracted sum are what rounds, not the length of the sums: 5x5 layers of 1 / 4 / 8
 // channels 1.8e-7 / 2.4e-7 / 2.5e-7 with two instructions, 0.9e-7 / 1.25e-7 / 1.3e-7 with three (kernel without tiles 0.9e-7 / 1.7e-7 / 2.4e-7);
 // 64 -> 8 @32x32, 64 images, 52 -> 63 us.
-static constexpr int kSatMaxTerms = 1152, kSatMaxTerms5x5 = 2500, kSatMinChannels5x5 = 10;
+static constexpr int kSatMaxTerms5x5 = 2500, kSatMinChannels5x5 = 10;
 template <class C>
 static bool two_instructions(int Co) {
     if (C::KS == 5 && Co < kSatMinChannels5x5) return false;
@@ -1046,7 +1046,6 @@ using GxS2W16 = GradX3x3S2Cfg<2, 8, 16, 1, 4, 8, 16>;    // inputs 16 wide: one 
 //                        TN SPR TH NIMG TM COW CC CQ
 using GxW32 = Tile3x3Cfg<4, 8, 16, 1, 4, 4, 8, 1>;    // inputs 32 wide: half an image x 16 channels
 using GxW16 = Tile3x3Cfg<4, 4, 16, 1, 4, 8, 16, 1>;   // inputs 16 wide: one image x 32 channels
-using GxW8  = Tile3x3Cfg<2, 4, 8, 2, 4, 8, 16, 1>;    // inputs 8 wide: two images x 32 channels
 // 5x5 taps, two input channels x two positions per lane, so that a layer of a few dozen channels still has two waves per
 // SIMD: 32 -> 64 @16x16, 64 images (0.84e9 terms) generic kernel 529 us, this 49 us (62 when the shape was picked, four positions per lane 94; but
 // 128 -> 64 167 against 184 us: a chip with enough waves would rather have fewer LDS reads per term)
@@ -1065,137 +1064,20 @@ using Gx1x1t = Tile3x3Cfg<2, 32, 1, 2, 4, 8, 16, 8, 1, 1>;    // ... two images 
 static bool small_plane_tile(const ConvDims &f) {
     return (long)ceil_div(f.N, Gx1x1s::NIMG) * ceil_div(f.Ci, Gx1x1s::TM * Gx1x1s::COW) <= 256;
 }
-// ... in workgroups of four waves that cover fewer rows, for maps whose height is not a multiple of 16 (56 = 7 x 8,
-// 28 = 7 x 4: ResNet-50 at batch 64, 64 -> 64 @56x56 366 -> 321 us, 128 -> 128 @28x28 345 -> 332 us)
-using GxW32H8 = Tile3x3Cfg<4, 8, 8, 1, 4, 4, 8, 1>;    // 8 rows of one image x 16 channels
-using GxW32H4 = Tile3x3Cfg<4, 8, 4, 2, 4, 4, 8, 1>;    // 4 rows of two images x 16 channels
-// rows per tile (16, 8 or 4) that pad a map of H rows least; the larger tile on a tie
-static int rows_per_tile_w32(int H) {
-    const int p16 = round_up(H, 16), p8 = round_up(H, 8), p4 = round_up(H, 4);
-    return p16 <= p8 && p16 <= p4 ? 16 : (p8 <= p4 ? 8 : 4);
+
+// Columns of the tiles that serve a 3x3 / stride 1 layer, 0: none, grad_x_nine.hip does.  Tiles stay where they are filled to 97 % and the
+// launch has two workgroups per CU (us, tiles -> grad_x_nine: 128 -> 128 @32x32, 128 images, 698 -> 734, 256 -> 256 @16x16 902 -> 921, 16 -> 16 @32x32, 256
+// images, 28.9 -> 29.5; 64 -> 64 @56x56, 32 images, 87 % filled, 169 -> 156; 32 -> 32 @16x16, 256 images, 256 workgroups, 28.5 -> 28.2).
+static int grad_x_tiles(const ConvDims &d) {
+    if (d.W <= 8 || d.Ci < GxW32::TM) return 0;
+    const int cols = d.W > 16 ? 32 : 16, across = ceil_div(d.W, cols), down = ceil_div(d.H, 16);
+    if (!grad_x_nine_supported(d)) return cols;
+    if (d.W % 4 || 100L * d.H * d.W < 97L * across * cols * down * 16) return 0;
+    const long wgs = (long)d.N * across * down * ceil_div(d.Ci, cols == 32 ? GxW32::TM * GxW32::COW : GxW16::TM * GxW16::COW);
+    return wgs >= 512 ? cols : 0;
 }
-static_assert(GxW32::TM == GxW16::TM && GxW16::TM == GxW8::TM && GxS2W32::TM == GxS2W16::TM,
+static_assert(GxW32::TM == GxW16::TM && GxS2W32::TM == GxS2W16::TM,
               "the launcher checks Ci against one TM per stride");
-
-// ---------------------------------------------------------------------------
-// Few positions: one input position x TM input channels per lane, the waves of a workgroup share the output channels
-// (the forward's counterpart of this kernel is fwd_few_kernel).  Wave v takes the chunks v, v + waves, ... of `chunk` output
-// channels, with gy (read from global memory: a map this small sits in L1 / L2) and the weights one output channel ahead
-// of the arithmetic; the chunk sums go through LDS and are added in channel order.
-// ---------------------------------------------------------------------------
-static constexpr int kFewTM = 4, kFewChunk = 8;   // input channels per lane; output channels per first-level sum (72 terms)
-template <int TM, class T>
-__global__ __launch_bounds__(512) void grad_x_few_kernel(const T *__restrict__ gy, const T *__restrict__ x,
-                                                         const float *__restrict__ w, T *__restrict__ gx,
-                                                         const T *__restrict__ gadd, ConvDims d) {
-    constexpr int KS = 3, KK = 9, chunk = kFewChunk;
-    __shared__ float part[8][TM][64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    const int plane = d.H * d.W, total = d.N * plane, K = d.Ci * KK;   // (stride 1, pad KS / 2: gy has the planes of x)
-    // the last group of channels is shifted down to end at Ci; channels below ci_first are not stored by it
-    const int ci_first = blockIdx.y * TM, ci0 = min(ci_first, d.Ci - TM);
-    const int pos = min((int)blockIdx.x * 64 + lane, total - 1);
-    const int n = pos / plane, hi = pos % plane / d.W, wi = pos % plane % d.W;
-    int off[KK];
-    bool ok[KK];
-#pragma unroll
-    for (int e = 0; e < KK; ++e) {
-        const int ho = hi + KS / 2 - e / KS, wo = wi + KS / 2 - e % KS;
-        ok[e] = ho >= 0 && ho < d.H && wo >= 0 && wo < d.W;
-        off[e] = n * d.Co * plane + (ok[e] ? ho * d.W + wo : 0);
-    }
-    uniform_f32_ptr wc = as_uniform(w) + ci0 * KK;
-    float xv[TM];
-#pragma unroll
-    for (int m = 0; m < TM; ++m) xv[m] = ldf(x + ((size_t)n * d.Ci + ci0 + m) * plane + pos % plane);
-    const int nchunks = ceil_div(d.Co, chunk);
-    float tot[TM];   // of result threadIdx.x + k * blockDim.x of the workgroup's TM x 64
-#pragma unroll
-    for (int k = 0; k < TM; ++k) tot[k] = 0.f;
-
-    for (int c0 = 0; c0 < nchunks; c0 += waves) {
-        const int c = c0 + wave;
-        if (c < nchunks) {
-            const int first = c * chunk, end = min(first + chunk, d.Co);
-            float acc[TM], gv[2][KK], wv[2][TM * KK];
-#pragma unroll
-            for (int m = 0; m < TM; ++m) acc[m] = 0.f;
-            auto load = [&](const int b, const int co) {
-                const int cc = min(co, end - 1);
-#pragma unroll
-                for (int e = 0; e < TM * KK; ++e) wv[b][e] = wc[cc * K + e];
-                const T *gc = gy + (size_t)cc * plane;
-#pragma unroll
-                for (int e = 0; e < KK; ++e) gv[b][e] = ldf(gc + off[e]);
-            };
-            auto add = [&](const int b, const int co) {
-                if (co >= end) return;
-#pragma unroll
-                for (int e = 0; e < KK; ++e) {
-                    const float v = ok[e] ? gv[b][e] : 0.f;
-#pragma unroll
-                    for (int m = 0; m < TM; ++m) acc[m] = fmaf(hardtanh(wv[b][m * KK + e] - xv[m]), v, acc[m]);
-                }
-            };
-            load(0, first);
-#pragma unroll 1
-            for (int co = first; co < end; co += 2) {
-                load(1, co + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                add(0, co);
-                load(0, co + 2);
-                __builtin_amdgcn_sched_barrier(0);
-                add(1, co + 1);
-            }
-#pragma unroll
-            for (int m = 0; m < TM; ++m) part[wave][m][lane] = acc[m];
-        }
-        __syncthreads();
-        const int here = min(waves, nchunks - c0);
-#pragma unroll
-        for (int k = 0; k < TM; ++k) {
-            const int e = threadIdx.x + k * blockDim.x;
-            if (e < TM * 64)
-                for (int v = 0; v < here; ++v) tot[k] += part[v][e >> 6][e & 63];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < TM; ++k) {
-        const int e = threadIdx.x + k * blockDim.x, p = blockIdx.x * 64 + (e & 63), ci = ci0 + (e >> 6);
-        if (e < TM * 64 && p < total && ci >= ci_first) {
-            const size_t o = ((size_t)(p / plane) * d.Ci + ci) * plane + p % plane;
-            stf(gx + o, gadd ? tot[k] + ldf(gadd + o) : tot[k]);
-        }
-    }
-}
-
-// Whether it takes a 3x3 / pad 1 layer of stride 1.  The tiled kernels last as long as one wave's chain of output channels x
-// taps x results per lane, 5.5 ns a term, until the chip is full; this one has a chain of its share of the output channels (0.45 us
-// each) and then works at 9 terms per ps.  Fitted to 60 layers; us, tiled -> this: 37 -> 51 3x3 @27x19, 7 images, 43 -> 13; 64 -> 64
-// @8x8, 1 / 64 images, 29 -> 6, 30 -> 19; 512 -> 512 @7x7, 1 / 7 images, 267 -> 38, 323 -> 111; 128 -> 128 @16x16, 1 / 7, 90 -> 11, 92 -> 36.
-// Beyond the line: 16 -> 16 @32x32, 64 images, 17 against 19.
-// Not for float32 layers that have a BatchNorm-linked kernel (whole groups of four): linked and plain backward of a layer
-// give the same bits, and the linked kernels sum in the tiled order.
-static int grad_x_bn_variant(const ConvDims &d);
-template <class T>
-static bool few_positions(const ConvDims &d, int per_lane) {
-    if ((sizeof(T) == 4 && grad_x_bn_variant(d)) || ceil_div(d.Ci, kFewTM) > kMaxGridY) return false;
-    const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
-    const float tiled = 2.f + 0.0055f * 9 * per_lane * d.Co;
-    const float share = (float)(ceil_div(ceil_div(d.Co, kFewChunk), 8) * kFewChunk);
-    const float few = 2.f + 0.45f * share + terms / 9e6f;
-    return few < 0.9f * tiled;
-}
-
-template <class T>
-static int launch_grad_x_few(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
-    constexpr int TM = kFewTM;
-    const int chunks = ceil_div(d.Co, kFewChunk), waves = chunks < 8 ? chunks : 8;
-    hipLaunchKernelGGL((grad_x_few_kernel<TM, T>), dim3(ceil_div(d.N * d.H * d.W, 64), ceil_div(d.Ci, TM)),
-                       dim3(64 * waves), 0, s, gy, x, w, gx, gadd, d);
-    return check_launch();
-}
 
 // gadd (nullable): a tensor shaped like gx that is added to the result (tiled 3x3 / pad 1, 5x5 / pad 2 / stride 1 and tiled
 // 1x1 stride-1 kernels only; ADDER_ERR_UNSUPPORTED elsewhere)
@@ -1205,16 +1087,15 @@ template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
     const bool k3s1p1 = d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1;
     const bool aligned = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
-    if (k3s1p1 && d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned)) {
-        if (few_positions<T>(d, d.W > 16 ? GxW32::TM * GxW32::TN : d.W > 8 ? GxW16::TM * GxW16::TN : GxW8::TM * GxW8::TN))
-            return launch_grad_x_few(gy, x, w, gx, d, s, gadd);
-        if (d.W > 16) switch (rows_per_tile_w32(d.H)) {
-            case 16: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
-            case 8: return launch_grad_x_3x3s1<GxW32H8, false, T>(gy, x, w, gx, d, s, gadd);
-            default: return launch_grad_x_3x3s1<GxW32H4, false, T>(gy, x, w, gx, d, s, gadd);
-        }
-        if (d.W > 8) return launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
-        return launch_grad_x_3x3s1<GxW8, false, T>(gy, x, w, gx, d, s, gadd);
+    if (k3s1p1 && (d.W % 4 != 0 || aligned)) switch (grad_x_tiles(d)) {
+        case 32: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
+        case 16: return launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
+        default: break;
+    }
+    if (grad_x_nine_supported(d)) {
+        // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
+        if (gadd && !(d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned))) return ADDER_ERR_UNSUPPORTED;
+        return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr);
     }
     if (d.kh == 5 && d.kw == 5 && d.stride == 1 && d.pad == 2 && d.Ci >= Gx5W32::TM && (d.W % 4 != 0 || aligned)) {
         if (d.W > 16) return launch_grad_x_3x3s1<Gx5W32, false, T>(gy, x, w, gx, d, s, gadd);
@@ -1259,13 +1140,16 @@ template int launch_grad_x<float>(const float *, const float *, const float *, f
 template int launch_grad_x<bf16_t>(const bf16_t *, const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t,
                                    const bf16_t *);
 
-// Which tiled kernel carries the BatchNorm link for this layer: 1 GxW32, 2 GxW16, 3 GxW8 (3x3 stride 1), 4 GxS2W32,
+// Which kernel carries the BatchNorm link for this layer: 1 GxW32, 2 GxW16, 3 the kernel of grad_x_nine.hip (3x3 stride 1), 4 GxS2W32,
 // 5 GxS2W16 (3x3 stride 2), 6 the kernel of grad_x_tap.hip (1x1 stride 1 from 64 input / 48 output channels); 0: none
 // (other kernel sizes, rows or planes that are not whole float4 groups, too few channels).
 static int grad_x_bn_variant(const ConvDims &d) {
     if (grad_x_tap_supported(d)) return (d.H * d.W) % 4 == 0 ? 6 : 0;
     if (d.kh != 3 || d.kw != 3 || d.pad != 1 || d.Ci < GxW32::TM) return 0;
-    if (d.stride == 1 && d.W % 4 == 0) return d.W > 16 ? 1 : (d.W > 8 ? 2 : 3);
+    if (d.stride == 1 && d.W % 4 == 0) {
+        const int cols = grad_x_tiles(d);
+        return cols == 32 ? 1 : cols == 16 ? 2 : grad_x_nine_supported(d) ? 3 : 0;
+    }
     if (d.stride == 2 && d.W % 4 == 0 && d.Wo % 4 == 0) return d.W > 16 ? 4 : 5;
     return 0;
 }
@@ -1278,13 +1162,9 @@ static int bn_slots_of(const ConvDims &d) {
 // partial-sum slots per input channel that launch_grad_x_bn writes into bn.in_part; 0: no such kernel for the layer
 int grad_x_bn_slots(const ConvDims &d) {
     switch (grad_x_bn_variant(d)) {
-        case 1: switch (rows_per_tile_w32(d.H)) {
-            case 16: return bn_slots_of<GxW32>(d);
-            case 8: return bn_slots_of<GxW32H8>(d);
-            default: return bn_slots_of<GxW32H4>(d);
-        }
+        case 1: return bn_slots_of<GxW32>(d);
         case 2: return bn_slots_of<GxW16>(d);
-        case 3: return bn_slots_of<GxW8>(d);
+        case 3: return grad_x_nine_bn_slots(d);
         case 4: return bn_slots_of<GxS2W32>(d);
         case 5: return bn_slots_of<GxS2W16>(d);
         case 6: return grad_x_tap_bn_slots(d);
@@ -1302,13 +1182,9 @@ int launch_grad_x_bn(const float *gy, const float *x, const float *w, float *gx,
     if (align & 15) return ADDER_ERR_UNSUPPORTED;
     if (!bn.in_part) return launch_grad_x(gy, x, w, gx, d, s, gadd);   // nothing to leave for a BatchNorm in front
     switch (grad_x_bn_variant(d)) {
-        case 1: switch (rows_per_tile_w32(d.H)) {
-            case 16: return launch_grad_x_3x3s1_bn<GxW32>(gy, x, w, gx, d, s, gadd, bn);
-            case 8: return launch_grad_x_3x3s1_bn<GxW32H8>(gy, x, w, gx, d, s, gadd, bn);
-            default: return launch_grad_x_3x3s1_bn<GxW32H4>(gy, x, w, gx, d, s, gadd, bn);
-        }
+        case 1: return launch_grad_x_3x3s1_bn<GxW32>(gy, x, w, gx, d, s, gadd, bn);
         case 2: return launch_grad_x_3x3s1_bn<GxW16>(gy, x, w, gx, d, s, gadd, bn);
-        case 3: return launch_grad_x_3x3s1_bn<GxW8>(gy, x, w, gx, d, s, gadd, bn);
+        case 3: return launch_grad_x_nine<float>(gy, x, w, gx, d, s, gadd, &bn);
         case 4: return launch_grad_x_3x3s2_bn<GxS2W32>(gy, x, w, gx, d, s, gadd, bn);
         case 5: return launch_grad_x_3x3s2_bn<GxS2W16>(gy, x, w, gx, d, s, gadd, bn);
         case 6: return launch_grad_x_tap<float>(gy, x, w, gx, d, s, gadd, &bn);

@@ -1,0 +1,302 @@
+// Input gradient of 3x3 / pad 1 / stride 1 layers, NCHW:
+//   gx[n,ci,h,w] = sum_{co,i,j} hardtanh(w[co,ci,i,j] - x[n,ci,h,w]) * gy[n,co,h+1-i,w+1-j]
+// Replaces the grad_i half of adder_cuda/adder.cu:194-272, adder.cu:133-192 and the fold of adder.py:32-33.
+//
+// The terms are those of grad_x.hip (two vector instructions, three above kSatMaxTerms terms) and bound it.  As in fwd_nine.hip a lane
+// reads the window of gy of its strip straight into registers, strips of all images line up and the waves of a workgroup share
+// the output channels; sums of sums live in LDS (once per 72 terms), 10 KB a wave, so that four waves per SIMD stay.  Large maps that
+// fill tiles of 16 x 16 or 8 x 32 positions are left to the tiles of grad_x.hip (see grad_x_tiles), which ask for gy once instead of nine
+// times: 128 -> 128 @32x32, 128 images, 698 us there, 734 here, 256 -> 256 @16x16 902 against 921.
+// us, tiles or the kernel for few positions there was -> this: 32 images 64 -> 64 @56x56 169 -> 156, 128 -> 128 @28x28 194 -> 164, 512 -> 512 @7x7
+// 322 -> 251, 100 -> 100 @20x20 119 -> 60; 64 -> 64 @8x8, 256 images 30.6 -> 28.3, one image 29 -> 6; 128 -> 128 @28x28, 4 / 1 images 97 -> 29, 94 -> 14;
+// 48 -> 12 @4x4, 64 images 8.4 -> 5.4; 256 -> 256 @14x14, one image 20 -> 18.
+#include "wave_split.hpp"
+
+#include <type_traits>
+
+namespace adder {
+
+// TM input channels x TN adjacent positions per lane; KSP waves that share the output channels in chunks of CC
+template <int TM_, int TN_, int KSP_>
+struct GxNineCfg {
+    static constexpr int TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = kNineChunk, FM = kFinished<TM, KSP>, STRIP = TN + 2;
+    static constexpr int AHEAD = TN == 1 ? 3 : 1;                      // output channels that gy is asked for ahead of the arithmetic
+    static constexpr int UM = TN == 4 ? 1 : 2, NU = TM / UM;           // input channels whose weights are asked for together, a step ahead
+    static constexpr int PART = KSP * TM * TN * 64, LDS_BYTES = PART * 4 + KSP * TN * 64 * 8;
+    static_assert((TM % KSP == 0 || KSP % TM == 0) && (NU == 1 || NU % 2 == 0), "a wave finishes FM channels or none; two weight buffers");
+};
+
+struct GxNineDims {
+    int N, Ci, H, W, Co;
+    int per_row, strips;    // strips of TN positions per row (the last one is moved back to end at W) and per image
+    int tiles, blocks;      // of 64 strips, of TM input channels
+};
+
+// SAT, FUSE, gadd, bn: as in grad_x_3x3s1_kernel (one slot of sums per tile).
+template <class C, bool SAT, class T, bool FUSE>
+__global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restrict__ gy, const T *__restrict__ x, const float *__restrict__ w,
+                                                               T *__restrict__ gx, const GxNineDims d, const T *__restrict__ gadd,
+                                                               const adder_bn_links bn) {
+    constexpr int TM = C::TM, TN = C::TN, KSP = C::KSP, FM = C::FM, STRIP = C::STRIP, NB = C::AHEAD + 1, UM = C::UM, NU = C::NU;
+    extern __shared__ __align__(16) float smem[];
+    int tile, blk;
+    xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
+    const int h = rest / d.per_row, s = rest - h * d.per_row, w0 = min(s * TN, d.W - TN), ci_base = blk * TM;
+    const int plane = d.H * d.W, K = d.Ci * 9;
+    uniform_f32_ptr wc = as_uniform(w);
+    int wofs[TM];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) wofs[m] = min(ci_base + m, d.Ci - 1) * 9;
+
+    float cr[TM][TN], acc[TM][TN];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+        float xv[TN];
+        ld_strip<TN>(x + ((size_t)n * d.Ci + min(ci_base + m, d.Ci - 1)) * plane + h * d.W + w0, xv);
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            cr[m][t] = SAT ? fmaf(-0.5f, xv[t], 0.5f) : xv[t];
+            acc[m][t] = 0.f;
+        }
+    }
+    // sums of sums in LDS: this wave's part, [channel][position][lane]; and of the gy values the positions met, [position][lane]
+    float *tot = smem + wave * (TM * TN * 64) + lane;
+    double *gtot = reinterpret_cast<double *>(smem + C::PART) + wave * (TN * 64) + lane;
+    bool first = true;
+
+    // a uniform base per channel and the lane's distances from it in bytes, as in fwd_nine.hip
+    const int n_first = __builtin_amdgcn_readfirstlane(n);
+    const T *g_first = gy + (size_t)n_first * d.Co * plane;
+    const bool ok_l = w0 > 0, ok_r = w0 + TN < d.W;
+    bool ok[3];
+    unsigned off[3], off_l[3], off_r[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int r = h + i - 1;
+        ok[i] = r >= 0 && r < d.H;
+        const int o = (n - n_first) * d.Co * plane + min(max(r, 0), d.H - 1) * d.W + w0;
+        off[i] = (unsigned)o * (unsigned)sizeof(T);
+        off_l[i] = (unsigned)(ok_l ? o - 1 : o) * (unsigned)sizeof(T);
+        off_r[i] = (unsigned)(ok_r ? o + TN : o) * (unsigned)sizeof(T);
+    }
+    float gr[NB][3][STRIP], wv[2][UM][9], gs[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) gs[t] = 0.f;
+    auto load_g = [&](const int b, const int co) {
+        const char *p = reinterpret_cast<const char *>(g_first + (size_t)co * plane);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            keep_offset(off[i]); keep_offset(off_l[i]); keep_offset(off_r[i]);
+            float u[TN];
+            ld_strip<TN>(reinterpret_cast<const T *>(p + off[i]), u);
+#pragma unroll
+            for (int t = 0; t < TN; ++t) gr[b][i][t + 1] = u[t];
+            gr[b][i][0] = ldf(reinterpret_cast<const T *>(p + off_l[i]));
+            gr[b][i][TN + 1] = ldf(reinterpret_cast<const T *>(p + off_r[i]));
+        }
+    };
+    auto load_w = [&](const int b, const int hh, const int co) {
+#pragma unroll
+        for (int u = 0; u < UM; ++u)
+#pragma unroll
+            for (int e = 0; e < 9; ++e) wv[b][u][e] = wc[co * K + wofs[hh * UM + u] + e];
+    };
+    auto after = [&](const int c) { return ((c + 1) & (C::CC - 1)) == 0 ? c + 1 + (KSP - 1) * C::CC : c + 1; };
+    int co = wave * C::CC;
+    if (co < d.Co) {
+        int cl = co;   // the channel that gy is read of next (the last one again behind the end)
+#pragma unroll
+        for (int b = 0; b < C::AHEAD; ++b) {
+            load_g(b, cl);
+            const int c = after(cl);
+            cl = c < d.Co ? c : cl;
+        }
+        load_w(0, 0, co);
+        auto channel = [&](const int cur) -> bool {
+            const int next = after(co);
+            const bool chunk_end = ((co + 1) & (C::CC - 1)) == 0, more = next < d.Co;
+            const int cn = more ? next : co;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {   // positions outside gy contribute nothing
+                if (i != 1) {
+#pragma unroll
+                    for (int k = 1; k <= TN; ++k) gr[cur][i][k] = ok[i] ? gr[cur][i][k] : 0.f;
+                }
+                gr[cur][i][0] = ok[i] && ok_l ? gr[cur][i][0] : 0.f;
+                gr[cur][i][TN + 1] = ok[i] && ok_r ? gr[cur][i][TN + 1] : 0.f;
+            }
+            if constexpr (SAT) {
+#pragma unroll
+                for (int t = 0; t < TN; ++t) {
+                    float c[3];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) c[k] = (gr[cur][0][t + k] + gr[cur][1][t + k]) + gr[cur][2][t + k];
+                    gs[t] += (c[0] + c[1]) + c[2];
+                }
+            }
+#pragma unroll
+            for (int hh = 0; hh < NU; ++hh) {
+                const int wb = (NU == 1 ? cur : hh) & 1;
+#pragma unroll
+                for (int idx = 0; idx < UM * 9 * TN; ++idx) {
+                    const int t = idx % TN, j = idx / TN % 3, i = idx / TN / 3 % 3, u = idx / TN / 9, m = hh * UM + u;
+                    const float wgt = wv[wb][u][i * 3 + j];
+                    const float dd = SAT ? sat01(fmaf(wgt, 0.5f, cr[m][t])) : hardtanh(wgt - cr[m][t]);
+                    acc[m][t] = fmaf(dd, gr[cur][2 - i][t + 2 - j], acc[m][t]);
+                    if (idx == 0) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_w(wb ^ 1, hh + 1 < NU ? hh + 1 : 0, hh + 1 < NU ? co : cn);
+                        if (hh == 0) load_g((cur + C::AHEAD) % NB, cl);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            co = next;
+            {
+                const int c = after(cl);
+                cl = c < d.Co ? c : cl;
+            }
+            if (chunk_end || !more) {   // 72-term first levels
+#pragma unroll
+                for (int m = 0; m < TM; ++m)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) {
+                        float *p = tot + (m * TN + t) * 64;
+                        *p = first ? acc[m][t] : *p + acc[m][t];
+                        acc[m][t] = 0.f;
+                    }
+                if constexpr (SAT) {
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) {
+                        double *p = gtot + t * 64;
+                        *p = first ? (double)gs[t] : *p + (double)gs[t];
+                        gs[t] = 0.f;
+                    }
+                }
+                first = false;
+            }
+            return more;
+        };
+#pragma unroll 1
+        while (channel(0) && channel(1) && (NB == 2 || (channel(2) && channel(NB - 1)))) {}
+        static_assert(NB == 2 || NB == 4, "the buffers take turns");
+    }
+    if (first) {   // no channels for this wave
+#pragma unroll
+        for (int e = 0; e < TM * TN; ++e) tot[e * 64] = 0.f;
+#pragma unroll
+        for (int t = 0; t < TN; ++t) gtot[t * 64] = 0.0;
+    }
+    __syncthreads();
+    if (wave * FM >= TM) return;
+    const int m0 = wave * FM, ci0 = ci_base + m0;
+    float r[FM][TN], sg[TN];
+    if constexpr (SAT) {   // sum over (co, taps) of the gy values a position met
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            const double *p = reinterpret_cast<const double *>(smem + C::PART) + t * 64 + lane;
+            double v = p[0];
+#pragma unroll
+            for (int k = 1; k < KSP; ++k) v += p[k * (TN * 64)];
+            sg[t] = (float)v;
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            float v = smem[((m0 + f) * TN + t) * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < KSP; ++k) v += smem[((k * TM + m0 + f) * TN + t) * 64 + lane];
+            r[f][t] = SAT ? fmaf(2.f, v, -sg[t]) : v;
+        }
+    if (ci0 >= d.Ci) return;
+    unsigned own = 0;   // bit t: position w0 + t is this lane's
+#pragma unroll
+    for (int t = 0; t < TN; ++t) own |= (sidx == sc && w0 + t >= s * TN ? 1u : 0u) << t;
+    finish_grad_x<FM, TN, FUSE>(r, own, ci0, ci0, d.Ci, plane, (n * d.Ci + ci0) * plane + h * d.W + w0, TN > 1 && d.W % TN == 0, x, gx, gadd, bn,
+                                d.tiles, tile, lane);
+}
+
+static int gx_nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((long)d.N * d.H * ceil_div(d.W, tn), 64); }
+
+// Waves that share the output channels, and input channels x positions per lane: by the rules of fwd_nine.hip, with a wave's chain of
+// 1.7, 1.15 and 0.55 us a channel and 24, 22 and 12 terms per ps (4 x 1: 7 on rows that are shorter than 8).  us, 8 x 4 / 8 x 2 / 4 x 1:
+// 128 -> 128 @28x28, 4 images, 29 / 31 / 36, one 29 / 20 / 14; 64 -> 64 @56x56, one, 17 / 12 / 14; 256 -> 256 @14x14, 4, 66 / 44 / 43, one 66 / 44 / 18;
+// 512 -> 512 @7x7, 4, 128 / 92 / 63, one 128 / 83 / 32.
+static int gx_nine_waves(int Co) { return Co <= 8 ? 1 : Co <= 16 ? 2 : Co <= 32 ? 4 : 8; }
+struct GxNineShape { int tm, tn; };
+static GxNineShape gx_nine_shape(const ConvDims &d) {
+    const int waves = gx_nine_waves(d.Co);
+    int tn = d.W >= 4 ? 4 : d.W >= 2 ? 2 : 1;
+    if (tn == 4 && (long)gx_nine_tiles(d, 4) * ceil_div(d.Ci, 8) * waves < 1300) tn = 2;
+    const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
+    const int chunks = ceil_div(ceil_div(d.Co, kNineChunk), waves), chain = min(chunks * kNineChunk, d.Co);
+    const float wide = fmaxf((tn == 4 ? 1.7f : 1.15f) * chain, terms / (tn == 4 ? 24e6f : 22e6f));
+    const float narrow = fmaxf(0.55f * chain, terms / (d.W < 8 ? 7e6f : 12e6f));
+    if (narrow < wide) tn = 1;
+    return {tn == 1 ? 4 : 8, tn};
+}
+
+// Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.
+bool grad_x_nine_supported(const ConvDims &d) {
+    if (d.kh != 3 || d.kw != 3 || d.pad != 1 || d.stride != 1) return false;
+    const long images = 63 / ((long)d.H * ceil_div(d.W, 4)) + 1;
+    return (images * d.Co + 1) * d.H * d.W <= 0x3fffffffL;
+}
+int grad_x_nine_bn_slots(const ConvDims &d) { return gx_nine_tiles(d, gx_nine_shape(d).tn); }
+
+template <class C, bool SAT, class T, bool FUSE>
+static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
+                          const adder_bn_links &bn) {
+    const int per_row = ceil_div(d.W, C::TN);
+    const GxNineDims t{d.N, d.Ci, d.H, d.W, d.Co, per_row, per_row * d.H, gx_nine_tiles(d, C::TN), ceil_div(d.Ci, C::TM)};
+    const long grid = (long)t.tiles * t.blocks;
+    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
+    if (FUSE && (!bn.in_part || bn.in_slots != t.tiles)) return ADDER_ERR_BAD_SHAPE;
+    if (int rc = allow_dynamic_lds<&grad_x_nine_kernel<C, SAT, T, FUSE>>(C::LDS_BYTES)) return rc;
+    hipLaunchKernelGGL((grad_x_nine_kernel<C, SAT, T, FUSE>), dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
+                       gadd, bn);
+    return check_launch();
+}
+
+// bn (nullable): the in_* half of adder_bn_links
+template <class T>
+int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
+                       const adder_bn_links *bn) {
+    auto run = [&](auto cfg) {
+        using C = decltype(cfg);
+        auto form = [&](auto sat) {
+            constexpr bool SAT = decltype(sat)::value;
+            if constexpr (sizeof(T) == 4) {
+                if (bn) return launch_gx_nine<C, SAT, T, true>(gy, x, w, gx, d, s, gadd, *bn);
+            }
+            return launch_gx_nine<C, SAT, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{});
+        };
+        // The two-instruction form only where the launch fills the chip: below that it gains nothing (32 -> 32 @16x16, 32 images, 9.1 us,
+        // three instructions 8.8; 64 -> 64 @56x56, one, 11.9, 13.2) and rounds w and x once more (1.6e-7 of the result against 2.3e-7).
+        if constexpr (C::TN == 4) {
+            if (d.Co * 9 <= kSatMaxTerms && d.Ci >= 4) return form(std::true_type{});
+        }
+        return form(std::false_type{});
+    };
+    const GxNineShape shape = gx_nine_shape(d);
+    auto waves = [&](auto ksp) {
+        constexpr int KSP = decltype(ksp)::value;
+        return shape.tn == 4 ? run(GxNineCfg<8, 4, KSP>{}) : shape.tn == 2 ? run(GxNineCfg<8, 2, KSP>{}) : run(GxNineCfg<4, 1, KSP>{});
+    };
+    switch (gx_nine_waves(d.Co)) {
+        case 1: return waves(std::integral_constant<int, 1>{});
+        case 2: return waves(std::integral_constant<int, 2>{});
+        case 4: return waves(std::integral_constant<int, 4>{});
+        default: return waves(std::integral_constant<int, 8>{});
+    }
+}
+template int launch_grad_x_nine<float>(const float *, const float *, const float *, float *, const ConvDims &, hipStream_t,
+                                       const float *, const adder_bn_links *);
+template int launch_grad_x_nine<bf16_t>(const bf16_t *, const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t,
+                                        const bf16_t *, const adder_bn_links *);
+
+}  // namespace adder

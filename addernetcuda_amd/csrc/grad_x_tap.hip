@@ -10,7 +10,7 @@
 // us, 128 positions x 64 channels with gy staged in LDS -> this: 32 images 64 -> 256 @56x56 98 -> 74, 256 -> 64 90 -> 84, 256 -> 128
 // 153 -> 144, 128 -> 512 @28x28 107 -> 77, 512 -> 256 164 -> 141, 256 -> 1024 @14x14 171 -> 85, 1024 -> 256 103 -> 75, 512 -> 2048 @7x7
 // 245 -> 113, 2048 -> 512 123 -> 79; one image: 256 -> 1024 @14x14 154 -> 16, 64 -> 256 @56x56 42 -> 8.
-#include "common.hpp"
+#include "wave_split.hpp"
 
 #include <type_traits>
 
@@ -32,7 +32,7 @@ struct GxTapDims {
 
 // SAT, FUSE, gadd, bn: as in grad_x_3x3s1_kernel (one slot of sums per tile; FUSE: float storage).
 template <class C, bool SAT, class T, bool FUSE>
-__global__ __launch_bounds__(C::NT) void grad_x_tap_kernel(const T *__restrict__ gy, const T *__restrict__ x, const float *__restrict__ w,
+__global__ __launch_bounds__(C::NT, 4) void grad_x_tap_kernel(const T *__restrict__ gy, const T *__restrict__ x, const float *__restrict__ w,
                                                            T *__restrict__ gx, const GxTapDims d, const T *__restrict__ gadd,
                                                            const adder_bn_links bn) {
     constexpr int TM = C::TM, TN = C::TN, KSP = C::KSP, CQ = 4, CU = 2, NU = CQ / CU, FM = C::FM;
@@ -178,65 +178,12 @@ __global__ __launch_bounds__(C::NT) void grad_x_tap_kernel(const T *__restrict__
             for (int k = 1; k < KSP; ++k) v += smem[((k * TM + m0 + f) * TN + t) * 64 + lane];
             r[f][t] = SAT ? fmaf(2.f, v, -sg[t]) : v;
         }
-    unsigned own = 0;
+    unsigned own = 0;   // bit t: position p0 + t is this lane's
 #pragma unroll
     for (int t = 0; t < TN; ++t) own |= (sidx == sc && p0 + t >= s * TN ? 1u : 0u) << t;
-    const int off = (n * d.Ci + ci0) * d.L + p0;
-    // (all loads before the first store: one counter serves both)
-    float a[FM][TN];
-    if (gadd) {
-#pragma unroll
-        for (int f = 0; f < FM; ++f) ld_strip<TN>(gadd + off + (size_t)f * d.L, a[f]);
-    }
-    if constexpr (FUSE) {
-        // x = relu(bn(in_x) [+ residual]): dz = (gx + gadd) * [x > 0] and per channel the sums of dz and dz * xhat.  xhat comes from x
-        // where nothing but the ReLU followed the BatchNorm and |gamma| is large enough for the division, else from in_x.
-        float xv[FM][TN], bx[FM][TN];
-#pragma unroll
-        for (int f = 0; f < FM; ++f) ld_strip<TN>(reinterpret_cast<const float *>(x) + off + (size_t)f * d.L, xv[f]);
-#pragma unroll
-        for (int f = 0; f < FM; ++f) {
-            const float g = bn.in_gamma ? as_uniform(bn.in_gamma)[ci0 + f] : 0.f, be = bn.in_gamma ? as_uniform(bn.in_beta)[ci0 + f] : 0.f;
-            const bool from_x = bn.in_gamma && fabsf(g) >= 0x1p-6f * fmaxf(1.f, fabsf(be));
-            if (!from_x) ld_strip<TN>(bn.in_x + off + (size_t)f * d.L, bx[f]);
-            const float centre = from_x ? be : as_uniform(bn.in_mean)[ci0 + f];
-            const float scale = from_x ? __builtin_amdgcn_rcpf(g) : as_uniform(bn.in_rstd)[ci0 + f];
-            float a1 = 0.f, a2 = 0.f;
-#pragma unroll
-            for (int t = 0; t < TN; ++t) {
-                if (gadd) r[f][t] += a[f][t];
-                const bool keep = (own >> t & 1) && !(bn.in_relu && !(xv[f][t] > 0.f));
-                const float v = keep ? r[f][t] : 0.f;
-                r[f][t] = v;
-                a1 += v;
-                a2 = fmaf(v, (from_x ? xv[f][t] : bx[f][t]) - centre, a2);
-            }
-            const float s1 = wave_sum_dpp(a1), s2 = wave_sum_dpp(a2) * scale;
-            if (lane == 0 && ci0 + f >= ci_first) {
-                float *dst = bn.in_part + ((size_t)(ci0 + f) * d.tiles + tile) * 2;
-                dst[0] = s1;
-                dst[1] = s2;
-            }
-        }
-    } else if (gadd) {
-#pragma unroll
-        for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int t = 0; t < TN; ++t) r[f][t] += a[f][t];
-    }
-    const bool whole = TN == 2 && (d.L & 1) == 0;
-#pragma unroll
-    for (int f = 0; f < FM; ++f) {
-        if (ci0 + f < ci_first) continue;
-        T *dst = gx + off + (size_t)f * d.L;
-        if (whole && own) {
-            if constexpr (TN == 2) st_strip<TN>(dst, r[f]);
-        } else {
-#pragma unroll
-            for (int t = 0; t < TN; ++t)
-                if (own >> t & 1) stf(dst + t, r[f][t]);
-        }
-    }
+    // the last group of channels is shifted down to end at Ci; channels below ci_first are not stored by it
+    finish_grad_x<FM, TN, FUSE>(r, own, ci0, max(ci_first, ci0), d.Ci, d.L, (n * d.Ci + ci0) * d.L + p0, TN > 1 && d.L % TN == 0, x, gx, gadd, bn,
+                                d.tiles, tile, lane);
 }
 
 static int gx_tap_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((long)d.N * ceil_div(d.H * d.W, tn), 64); }

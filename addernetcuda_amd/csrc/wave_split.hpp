@@ -60,7 +60,7 @@ __device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], unsigned own,
             sums[2 * f] = s1;
             sums[2 * f + 1] = s2;
         }
-        if constexpr (FM >= 2) {   // all sums in one reduce-scatter: lane l < 2 FM ends with number j(l), moment j % 2 of channel j / 2
+        if constexpr (FM >= 2 && FM <= 8) {   // all sums in one reduce-scatter: lane l < 2 FM ends with number j(l), moment j % 2 of channel j / 2
             const float mine = wave_sum_scatter<2 * FM>(sums, lane), other = __shfl_xor(mine, FM, 64);
             const int j = wave_sum_scatter_index<2 * FM>(lane), f = j >> 1;
             float piv = pivot[0];
@@ -103,6 +103,73 @@ __device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], unsigned own,
         T *dst = y + (size_t)(co0 + f) * L + off;
         if (whole && own) {
             if constexpr (TN == 4 || TN == 2) st_strip<TN>(dst, r[f]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+                if (own >> t & 1) stf(dst + t, r[f][t]);
+        }
+    }
+}
+
+// The same for input gradients: a second gradient (gadd, nullable) is added, the first pass of the BatchNorm in front of the layer is
+// made where FUSE (the in_* fields of adder_bn_links: one slot of sums per tile; float storage), channels first <= c < Ci of the
+// FM from ci0 on are stored.  off: the lane's first position in channel ci0.
+template <int FM, int TN, bool FUSE, class T>
+__device__ __forceinline__ void finish_grad_x(float (&r)[FM][TN], unsigned own, int ci0, int first, int Ci, int L, int off, bool whole,
+                                              const T *__restrict__ x, T *__restrict__ gx, const T *__restrict__ gadd,
+                                              const adder_bn_links &bn, int tiles, int tile, int lane) {
+    // (all loads before the first store: one counter serves both; channels past Ci read the last one)
+    float a[FM][TN];
+    if (gadd) {
+#pragma unroll
+        for (int f = 0; f < FM; ++f) ld_strip<TN>(gadd + off + (size_t)min(f, Ci - 1 - ci0) * L, a[f]);
+    }
+    if constexpr (FUSE) {
+        // x = relu(bn(in_x) [+ residual]): dz = (gx + gadd) * [x > 0] and per channel the sums of dz and dz * xhat.  xhat comes from x
+        // where nothing but the ReLU followed the BatchNorm and |gamma| is large enough for the division, else from in_x.
+        float xv[FM][TN];
+#pragma unroll
+        for (int f = 0; f < FM; ++f) ld_strip<TN>(x + off + (size_t)min(f, Ci - 1 - ci0) * L, xv[f]);
+#pragma unroll
+        for (int f = 0; f < FM; ++f) {
+            const int c = min(ci0 + f, Ci - 1);
+            const float g = bn.in_gamma ? as_uniform(bn.in_gamma)[c] : 0.f, be = bn.in_gamma ? as_uniform(bn.in_beta)[c] : 0.f;
+            const bool from_x = bn.in_gamma && fabsf(g) >= 0x1p-6f * fmaxf(1.f, fabsf(be));
+            float bx[TN];
+#pragma unroll
+            for (int t = 0; t < TN; ++t) bx[t] = xv[f][t];
+            if (!from_x) ld_strip<TN>(bn.in_x + off + (size_t)(c - ci0) * L, bx);
+            const float centre = from_x ? be : as_uniform(bn.in_mean)[c];
+            const float scale = from_x ? __builtin_amdgcn_rcpf(g) : as_uniform(bn.in_rstd)[c];
+            float a1 = 0.f, a2 = 0.f;
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                if (gadd) r[f][t] += a[f][t];
+                const bool keep = (own >> t & 1) && !(bn.in_relu && !(xv[f][t] > 0.f));
+                const float v = keep ? r[f][t] : 0.f;
+                r[f][t] = v;
+                a1 += v;
+                a2 = fmaf(v, bx[t] - centre, a2);
+            }
+            const float s1 = wave_sum_dpp(a1), s2 = wave_sum_dpp(a2) * scale;
+            if (lane == 0 && ci0 + f >= first && ci0 + f < Ci) {
+                float *dst = bn.in_part + ((size_t)(ci0 + f) * tiles + tile) * 2;
+                dst[0] = s1;
+                dst[1] = s2;
+            }
+        }
+    } else if (gadd) {
+#pragma unroll
+        for (int f = 0; f < FM; ++f)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) r[f][t] += a[f][t];
+    }
+#pragma unroll
+    for (int f = 0; f < FM; ++f) {
+        if (ci0 + f < first || ci0 + f >= Ci) continue;
+        T *dst = gx + off + (size_t)f * L;
+        if (whole && own) {
+            if constexpr (TN == 2 || TN == 4) st_strip<TN>(dst, r[f]);
         } else {
 #pragma unroll
             for (int t = 0; t < TN; ++t)
