@@ -226,10 +226,9 @@ static int gx_nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((lo
 // 1.7, 1.15 and 0.55 us a channel and 24, 22 and 12 terms per ps (4 x 1: 7 on rows that are shorter than 8).  us, 8 x 4 / 8 x 2 / 4 x 1:
 // 128 -> 128 @28x28, 4 images, 29 / 31 / 36, one 29 / 20 / 14; 64 -> 64 @56x56, one, 17 / 12 / 14; 256 -> 256 @14x14, 4, 66 / 44 / 43, one 66 / 44 / 18;
 // 512 -> 512 @7x7, 4, 128 / 92 / 63, one 128 / 83 / 32.
-static int gx_nine_waves(int Co) { return Co <= 8 ? 1 : Co <= 16 ? 2 : Co <= 32 ? 4 : 8; }
-struct GxNineShape { int tm, tn; };
+struct GxNineShape { int tn, waves; };
 static GxNineShape gx_nine_shape(const ConvDims &d) {
-    const int waves = gx_nine_waves(d.Co);
+    const int waves = d.Co <= 8 ? 1 : d.Co <= 16 ? 2 : d.Co <= 32 ? 4 : 8;
     int tn = d.W >= 4 ? 4 : d.W >= 2 ? 2 : 1;
     if (tn == 4 && (long)gx_nine_tiles(d, 4) * ceil_div(d.Ci, 8) * waves < 1300) tn = 2;
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
@@ -237,7 +236,8 @@ static GxNineShape gx_nine_shape(const ConvDims &d) {
     const float wide = fmaxf((tn == 4 ? 1.7f : 1.15f) * chain, terms / (tn == 4 ? 24e6f : 22e6f));
     const float narrow = fmaxf(0.55f * chain, terms / (d.W < 8 ? 7e6f : 12e6f));
     if (narrow < wide) tn = 1;
-    return {tn == 1 ? 4 : 8, tn};
+    // (two waves would share nine to twelve channels two to one: 48 -> 12 @32x32, 64 images, 25.0 us, one wave 23.5)
+    return {tn, tn == 4 && d.Co <= 12 ? 1 : waves};
 }
 
 // Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.
@@ -287,7 +287,7 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
         constexpr int KSP = decltype(ksp)::value;
         return shape.tn == 4 ? run(GxNineCfg<8, 4, KSP>{}) : shape.tn == 2 ? run(GxNineCfg<8, 2, KSP>{}) : run(GxNineCfg<4, 1, KSP>{});
     };
-    switch (gx_nine_waves(d.Co)) {
+    switch (shape.waves) {
         case 1: return waves(std::integral_constant<int, 1>{});
         case 2: return waves(std::integral_constant<int, 2>{});
         case 4: return waves(std::integral_constant<int, 4>{});
