@@ -359,6 +359,10 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
                        const adder_bn_links *bn);
 bool grad_x_nine_supported(const ConvDims &d);
 int grad_x_nine_bn_slots(const ConvDims &d);
+// 3x3 / pad 1 and 5x5 / pad 2 / stride 2 (grad_x_s2.hip); sat: two instructions a term
+template <class T>
+int launch_grad_x_s2(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd, bool sat);
+bool grad_x_s2_supported(const ConvDims &d);
 static constexpr int kSatMaxTerms = 1152;      // terms up to which a 3x3 layer's input gradient takes two instructions a term (grad_x.hip)
 static constexpr int kSatMaxTerms1x1 = 1024;   // output channels up to which a single tap's input gradient takes two instructions a term (grad_x.hip)
 size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false, size_t limit = SIZE_MAX);   // of the storage type's kernels

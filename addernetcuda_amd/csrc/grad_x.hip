@@ -1076,6 +1076,12 @@ static int grad_x_tiles(const ConvDims &d) {
     const long wgs = (long)d.N * across * down * ceil_div(d.Ci, cols == 32 ? GxW32::TM * GxW32::COW : GxW16::TM * GxW16::COW);
     return wgs >= 512 ? cols : 0;
 }
+// us, tiles / grad_x_s2.hip, bfloat16: 16 -> 32 @32x32, 256 images, 21 / 26, 1024 -> 64 @16x16, 16 images, 35 / 48; 87 % filled, 128 -> 128 @56x56, 32
+// images, 260 / 243; half the channels of a workgroup, 8 -> 64 @64x64, 64 images, 34 / 26; 64 workgroups, 128 -> 128 @56x56, one image, 42 / 15.
+static bool fills_s2_tiles(const ConvDims &d) {
+    const int cols = d.W > 16 ? 32 : 16, channels = d.W > 16 ? GxS2W32::TM * GxS2W32::CIW : GxS2W16::TM * GxS2W16::CIW;
+    return d.W % cols == 0 && d.H % 16 == 0 && d.Ci % channels == 0 && (long)d.N * (d.H / 16) * (d.W / cols) * (d.Ci / channels) >= 256;
+}
 static_assert(GxW32::TM == GxW16::TM && GxS2W32::TM == GxS2W16::TM,
               "the launcher checks Ci against one TM per stride");
 
@@ -1102,11 +1108,19 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         if (d.W > 8) return launch_grad_x_3x3s1<Gx5W16, false, T>(gy, x, w, gx, d, s, gadd);
         return launch_grad_x_3x3s1<Gx5W8, false, T>(gy, x, w, gx, d, s, gadd);
     }
-    if (d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM &&
-        (d.Wo % 4 != 0 || aligned_groups(gy)) &&
-        ((reinterpret_cast<uintptr_t>(gx) | reinterpret_cast<uintptr_t>(gadd)) & (2 * sizeof(T) - 1)) == 0) {
+    // 3x3 with a stride of two: layers the BatchNorm link may ask for (grad_x_bn_variant) keep the tiles, so that the plain call has the linked
+    // one's bits; bfloat16, which has no links, only where they are filled and give every CU a workgroup
+    const bool adds_s2 = d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM &&
+                         (d.Wo % 4 != 0 || aligned_groups(gy)) &&
+                         ((reinterpret_cast<uintptr_t>(gx) | reinterpret_cast<uintptr_t>(gadd)) & (2 * sizeof(T) - 1)) == 0;
+    if (adds_s2 && (!grad_x_s2_supported(d) || (d.Wo % 4 == 0 && (sizeof(T) == 4 || fills_s2_tiles(d))))) {
         if (d.W > 16) return launch_grad_x_3x3s2<GxS2W32, T>(gy, x, w, gx, d, s, gadd);
         return launch_grad_x_3x3s2<GxS2W16, T>(gy, x, w, gx, d, s, gadd);
+    }
+    if (grad_x_s2_supported(d)) {
+        // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
+        if (gadd && !adds_s2) return ADDER_ERR_UNSUPPORTED;
+        return launch_grad_x_s2<T>(gy, x, w, gx, d, s, gadd, adds_s2 && d.Co * 4 <= kSatMaxTerms);
     }
     if (grad_x_tap_supported(d)) {
         // (it takes bases of any alignment; a second gradient is added on planes of whole groups for aligned ones only)
