@@ -330,7 +330,7 @@ template <class T>
 int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
 template <class T>
 int launch_fwd_tap(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn);
-bool fwd_tap_supported(const ConvDims &d);      // 1x1 / stride 1 (fwd_tap.hip)
+bool fwd_tap_supported(const ConvDims &d);      // 1x1 / pad 0, any stride (fwd_tap.hip)
 int fwd_tap_stats_slots(const ConvDims &d);
 // 3x3 / pad 1 / stride 1 or 2 (fwd_nine.hip); mul (stride 1, float): an ordinary convolution; w_side, y_side, stats_side (nullable; stride
 // 2, float): the strided 1x1 layer beside it

@@ -96,13 +96,13 @@ __global__ __launch_bounds__(256) void fwd_generic_kernel(const T *__restrict__ 
 // ---------------------------------------------------------------------------
 // T: storage type of x and y (float, or bf16_t for the reduced-storage mode); the arithmetic is fp32 either way.
 // EVAL: bn is applied to the results (float storage; an instance of its own, so that the others keep their registers).
-template <class C, bool VEC, bool SUB, class T, bool EVAL>
+template <class C, bool VEC, class T, bool EVAL>
 __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restrict__ x,
                                                                 const float *__restrict__ w,
                                                                 T *__restrict__ y,
                                                                 double *__restrict__ stats, int N, int Ci,
                                                                 int H, int W, int Co, int Ho, int Wo,
-                                                                int tilesH, int tilesW, const Subsample sub,
+                                                                int tilesH, int tilesW,
                                                                 const BnEval bn) {
     constexpr int TN = C::TN, TM = C::TM, CQ = C::CQ, S = C::S, STRIP = C::STRIP, KS = C::KS, KK = C::KK;
     extern __shared__ __align__(16) float smem[];
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
     const int nchunks = ceil_div(Ci, C::CC);
 
     TileStage<typename C::Patch> st;
-    tile_fetch<typename C::Patch, VEC, SUB, T>(st, x, 0, Ci, n0, N, h0 * S - C::PAD, w0 * S, H, W, sub);
+    tile_fetch<typename C::Patch, VEC, false, T>(st, x, 0, Ci, n0, N, h0 * S - C::PAD, w0 * S, H, W);
     {   // this workgroup's output channels: one contiguous run of weights
         const int co_blk = blockIdx.y * C::COW * TM;
         l2_warm(w + (size_t)co_blk * K, 1, 0, min(C::COW * TM, Co - co_blk) * K);
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
 
     for (int c = 0; c < nchunks; ++c) {
         const int ci0 = c * C::CC;
-        if (c + 1 < nchunks) tile_fetch<typename C::Patch, VEC, SUB, T>(st, x, ci0 + C::CC, Ci, n0, N, h0 * S - C::PAD, w0 * S, H, W, sub);
+        if (c + 1 < nchunks) tile_fetch<typename C::Patch, VEC, false, T>(st, x, ci0 + C::CC, Ci, n0, N, h0 * S - C::PAD, w0 * S, H, W);
 
         const float *lbase = smem + (c & 1) * C::BUF + lane_off;
         const int ccnt = min(C::CC, Ci - ci0);
@@ -342,128 +342,18 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_3x3_kernel(const T *__restric
     }
 }
 
-// ---------------------------------------------------------------------------
-// Few positions of a 1x1 layer with a stride: one output position x TM output channels per lane, the waves of a workgroup share the
-// reduction.
-//
-// The tiled kernels give a lane 8-32 results and walk all input channels in one wave; one image leaves them with a handful
-// of workgroups, and the launch lasts as long as that serial chain.  Here wave v of a workgroup takes the channel chunks v, v +
-// waves, ...; after each round the chunk sums go through LDS and are added in channel order, so every result has the bits of the
-// tiled kernel whose chunk length is given (`chunk` channels per first-level sum).  x is read from global memory (a map this small
-// sits in L1 / L2) one group of channels ahead of the arithmetic, as are the weights.
-// ---------------------------------------------------------------------------
-static constexpr int kFewTM = 4;
-template <int TM, int G, class T>
-__global__ __launch_bounds__(512) void fwd_few_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
-                                                      double *__restrict__ stats, ConvDims d, int chunk, const BnEval bn) {
-    __shared__ float part[8][TM][64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    const int plane = d.H * d.W, L = d.Ho * d.Wo, total = d.N * L, co0 = blockIdx.y * TM;
-    const int pos = min((int)blockIdx.x * 64 + lane, total - 1);
-    const int n = pos / L, ho = pos % L / d.Wo, wo = pos % L % d.Wo;
-    const int off = n * d.Ci * plane + ho * d.stride * d.W + wo * d.stride;
-    uniform_f32_ptr wc = as_uniform(w);
-    int wrow[TM];
-#pragma unroll
-    for (int m = 0; m < TM; ++m) wrow[m] = min(co0 + m, d.Co - 1) * d.Ci;
-    const int nchunks = ceil_div(d.Ci, chunk);
-    float tot[TM];   // of result threadIdx.x + k * blockDim.x of the workgroup's TM x 64
-#pragma unroll
-    for (int k = 0; k < TM; ++k) tot[k] = 0.f;
-
-    for (int c0 = 0; c0 < nchunks; c0 += waves) {
-        const int c = c0 + wave;
-        if (c < nchunks) {
-            const int first = c * chunk, end = min(first + chunk, d.Ci);
-            float acc[TM], xv[2][G], wv[2][TM * G];
-#pragma unroll
-            for (int m = 0; m < TM; ++m) acc[m] = 0.f;
-            auto load = [&](const int b, const int ci) {
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const int cc = min(ci + g, end - 1);
-#pragma unroll
-                    for (int m = 0; m < TM; ++m) wv[b][m * G + g] = wc[wrow[m] + cc];
-                    xv[b][g] = ldf(x + (size_t)cc * plane + off);
-                }
-            };
-            auto add = [&](const int b, const int ci) {
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    if (ci + g >= end) break;
-#pragma unroll
-                    for (int m = 0; m < TM; ++m) acc[m] -= fabsf(wv[b][m * G + g] - xv[b][g]);
-                }
-            };
-            load(0, first);
-#pragma unroll 1
-            for (int ci = first; ci < end; ci += 2 * G) {
-                load(1, ci + G);
-                __builtin_amdgcn_sched_barrier(0);
-                add(0, ci);
-                load(0, ci + 2 * G);
-                __builtin_amdgcn_sched_barrier(0);
-                add(1, ci + G);
-            }
-#pragma unroll
-            for (int m = 0; m < TM; ++m) part[wave][m][lane] = acc[m];
-        }
-        __syncthreads();
-        const int here = min(waves, nchunks - c0);
-#pragma unroll
-        for (int k = 0; k < TM; ++k) {
-            const int e = threadIdx.x + k * blockDim.x;
-            if (e < TM * 64)
-                for (int v = 0; v < here; ++v) tot[k] += part[v][e >> 6][e & 63];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < TM; ++k) {
-        const int e = threadIdx.x + k * blockDim.x, p = blockIdx.x * 64 + (e & 63), co = co0 + (e >> 6);
-        if (stats && e < TM * 64 && co < d.Co) {   // (wave-uniform: a wave holds 64 positions of one channel)
-            const double v = p < total ? (double)tot[k] : 0.0, s1 = wave_sum(v), s2 = wave_sum(v * v);
-            if (lane == 0) {
-                double *dst = stats + ((size_t)co * gridDim.x + blockIdx.x) * 2;
-                dst[0] = s1;
-                dst[1] = s2;
-            }
-        }
-        if (e < TM * 64 && p < total && co < d.Co) {
-            const size_t o = ((size_t)(p / L) * d.Co + co) * L + p % L;
-            float v = tot[k];
-            if (sizeof(T) == 4 && bn.gamma) {
-                v = BnEvalChannel(bn, co)(v);
-                if (bn.res) v += bn.res[o];
-                if (bn.relu) v = relu_keep_nan(v);
-            }
-            stf(y + o, v);
-        }
-    }
-}
-
-template <class T>
-static int launch_fwd_few(const T *x, const float *w, T *y, double *stats, const ConvDims &d, int chunk, hipStream_t s,
-                          const BnEval &bn) {
-    constexpr int TM = kFewTM, G = 8;
-    const int waves = ceil_div(d.Ci, chunk) < 8 ? ceil_div(d.Ci, chunk) : 8;
-    hipLaunchKernelGGL((fwd_few_kernel<TM, G, T>), dim3(ceil_div(d.N * d.Ho * d.Wo, 64), ceil_div(d.Co, TM)),
-                       dim3(64 * waves), 0, s, x, w, y, stats, d, chunk, bn);
-    return check_launch();
-}
-
-template <class C, bool VEC, bool SUB, class T>
+template <class C, bool VEC, class T>
 static int launch_fwd_3x3_v(const T *x, const float *w, T *y, double *stats, const ConvDims &d,
-                            hipStream_t s, const Subsample sub = Subsample{1, 0, 0, 0}, const BnEval &bn = kNoBnEval) {
+                            hipStream_t s, const BnEval &bn) {
     const int tilesH = ceil_div(d.Ho, C::TH), tilesW = ceil_div(d.Wo, C::TW);
     const long gx = (long)ceil_div(d.N, C::NIMG) * tilesH * tilesW;
     const int gy = ceil_div(d.Co, C::TM * C::COW);
     if (gx > 0x7fffffffL) return ADDER_ERR_TOO_LARGE;
     auto launch = [&](auto eval) {
         constexpr bool EVAL = decltype(eval)::value;
-        if (int rc = allow_dynamic_lds<&fwd_3x3_kernel<C, VEC, SUB, T, EVAL>>(C::LDS_BYTES)) return rc;
-        hipLaunchKernelGGL((fwd_3x3_kernel<C, VEC, SUB, T, EVAL>), dim3((unsigned)gx, gy), dim3(C::NTHREADS),
-                           C::LDS_BYTES, s, x, w, y, stats, d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, tilesH, tilesW, sub, bn);
+        if (int rc = allow_dynamic_lds<&fwd_3x3_kernel<C, VEC, T, EVAL>>(C::LDS_BYTES)) return rc;
+        hipLaunchKernelGGL((fwd_3x3_kernel<C, VEC, T, EVAL>), dim3((unsigned)gx, gy), dim3(C::NTHREADS),
+                           C::LDS_BYTES, s, x, w, y, stats, d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, tilesH, tilesW, bn);
         return check_launch();
     };
     if constexpr (sizeof(T) == 4) {
@@ -475,27 +365,10 @@ static int launch_fwd_3x3_v(const T *x, const float *w, T *y, double *stats, con
 template <class C, class T = float>
 static int launch_fwd_3x3(const T *x, const float *w, T *y, double *stats, const ConvDims &d,
                           hipStream_t s, const BnEval &bn) {
-    const Subsample all{1, 0, 0, 0};
     // element-wise tile loads when the rows of the staged tensor are not whole groups of four
-    if (d.W % 4 == 0) return launch_fwd_3x3_v<C, true, false, T>(x, w, y, stats, d, s, all, bn);
-    return launch_fwd_3x3_v<C, false, false, T>(x, w, y, stats, d, s, all, bn);
+    if (d.W % 4 == 0) return launch_fwd_3x3_v<C, true, T>(x, w, y, stats, d, s, bn);
+    return launch_fwd_3x3_v<C, false, T>(x, w, y, stats, d, s, bn);
 }
-
-// partial-sum slots per channel the statistics epilogue of this tile shape writes
-template <class C>
-static int stats_slots_3x3(const ConvDims &d) {
-    const long gx = (long)ceil_div(d.N, C::NIMG) * ceil_div(d.Ho, C::TH) * ceil_div(d.Wo, C::TW);
-    return (int)(gx * C::POSW);
-}
-
-// 1x1 with a stride: the tile loader gathers the sampled x element by element, which costs several times what the
-// aligned float4 loads of a stride-1 plane cost, so a workgroup takes 64 output channels per staged tile instead of
-// 32 (eight per lane, chunks of eight input channels to stay within 128 registers); ResNet-50's three downsample
-// layers at batch 64: 538 -> 319, 621 -> 376, 591 -> 374 us.  (Stride 1: fwd_tap.hip.)
-using Fwd1x1sub = Tile3x3Cfg<4, 16, 1, 4, 8, 8, 8, 8, 1, 1>;   // 64 sampled positions of four images x 64 channels
-// ... with units of four input channels, for channel counts that are multiples of 4 but not of 8
-using Fwd1x1q  = Tile3x3Cfg<4, 64, 1, 1, 4, 8, 16, 4, 1, 1>;   // 256 positions of one image x 32 channels
-using Fwd1x1sq = Tile3x3Cfg<4, 16, 1, 4, 4, 8, 16, 4, 1, 1>;   // planes of <= 64 positions: four images
 
 // 5x5 taps: a unit is one output channel x one input channel as well (25 weights, 50*TN vector instructions); five
 // strips of eight values per buffer leave room for two output channels per lane.  Two vector instructions per term
@@ -507,16 +380,12 @@ using Fwd5W16S2 = Tile3x3Cfg<2, 8, 8, 1, 2, 8, 8, 1, 2, 5>;     // stride 2: 8 r
 using Fwd5W8S2  = Tile3x3Cfg<2, 4, 8, 2, 2, 8, 8, 1, 2, 5>;     // stride 2, outputs up to 8 wide: two images
 
 // which tiled kernel serves these dimensions (0 = none): 1..3 3x3 stride 1 by output width, 4..5 3x3 stride 2 (all fwd_nine.hip),
-// 6..7 1x1 stride 1 by plane size (both fwd_tap.hip), 8..9 1x1 with a stride (the sampled positions walked like a stride-1 plane),
-// 10..13 = 6..9 for channels that are no multiple of 8, 14..18 5x5 (stride 1 by output width, then stride 2)
+// 6..7 1x1 stride 1 from 64 channels on by plane size, 8..9 1x1 with a stride, 10..13 = 6..9 for channels that are no multiple of 8 (all
+// fwd_tap.hip), 14..18 5x5 (stride 1 by output width, then stride 2)
 static int fwd_tiled_variant(const ConvDims &d) {
-    // (below 64 input channels the plain 1x1 kernel of conv1x1.hip is as fast or faster)
-    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci % Fwd1x1q::CQ == 0 && d.Ci >= 64) {
-        const int quad = d.Ci % Fwd1x1sub::CQ ? 4 : 0;
-        // 256 positions of one image per workgroup, or 64 positions of four: whichever pads the plane less
-        // (28x28 = 784 positions fill 64-wide tiles to 94 %, 256-wide ones to 77 %: 216 -> 169 us for 128 -> 512)
-        const int plane = d.Ho * d.Wo;
-        const bool wide = ceil_div(plane, Fwd1x1q::TW) * Fwd1x1q::TW <= ceil_div(plane, Fwd1x1sq::TW) * Fwd1x1sq::TW;
+    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci % 4 == 0 && d.Ci >= 64) {
+        const int quad = d.Ci % 8 ? 4 : 0, plane = d.Ho * d.Wo;
+        const bool wide = ceil_div(plane, 256) * 256 <= ceil_div(plane, 64) * 64;
         if (d.stride == 1) return (wide ? 6 : 7) + quad;
         return (wide ? 8 : 9) + quad;
     }
@@ -531,12 +400,10 @@ static int fwd_tiled_variant(const ConvDims &d) {
     return 0;
 }
 
-// Whether a 3x3 or 1x1 layer has few positions.  1x1 layers with a stride run the kernel above then: the tiled kernel lasts as long as
-// one wave's chain of channels x results per lane, 6 ns a term, until the chip is full; this one has a chain of its share of the
-// channels (0.25 us each) and then works at 3.2 terms per ps.  For the other layers it is a class of sizes that fwd_kernel tells
-// apart: fwd_nine.hip and fwd_tap.hip choose their shapes by rules of their own.
+// Whether a 3x3 or 1x1 layer has few positions: a class of sizes that fwd_kernel tells apart, and whose statistics are offered for bases of
+// any alignment.  fwd_nine.hip and fwd_tap.hip choose their shapes by rules of their own.
 static bool few_positions(const ConvDims &d, int variant) {
-    if (variant == 0 || variant >= 14 || ceil_div(d.Co, kFewTM) > kMaxGridY) return false;
+    if (variant == 0 || variant >= 14 || ceil_div(d.Co, 4) > kMaxGridY) return false;
     const int per_lane = variant >= 3 && variant <= 5 ? 8 : variant == 8 || variant == 9 ? 32 : 16;
     const int chunk = variant == 1 || variant == 4 || variant == 8 || variant == 9 || (variant == 5 && d.Ci >= 128) ? 8 : 16;
     const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;
@@ -545,16 +412,6 @@ static bool few_positions(const ConvDims &d, int variant) {
     const float few = 2.f + (d.kh == 3 ? 0.4f * share + terms / 10.9e6f : 0.25f * share + terms / 3.2e6f);
     return few < 0.9f * tiled;
 }
-
-// a 1x1 layer seen as N x Ci "images" of one row of Ho*Wo positions (the whole plane when the stride is 1)
-static ConvDims as_one_row(const ConvDims &d) {
-    ConvDims f = d;
-    f.H = f.Ho = 1;
-    f.W = f.Wo = d.Ho * d.Wo;
-    f.stride = 1;
-    return f;
-}
-static Subsample sampling_of(const ConvDims &d) { return Subsample{d.stride, d.Wo, d.W, d.H * d.W}; }
 
 // A strided 3x3 / pad 1 layer and the strided 1x1 / pad 0 layer beside it (same x, same Co, Ho, Wo) in one launch;
 // d describes the 3x3 layer.  Both outputs with their statistics (fwd_stats_slots(d) slots each).  Rows of whole
@@ -577,8 +434,8 @@ static int rows_per_tile_w32(int H) {
 
 // Which kernel launch_fwd runs without statistics and for bases aligned to groups of four: 0 general, 1 plain 1x1, 2 few
 // positions, else 10 * variant + a class of sizes (3x3 on wide maps: whole groups of 16 / 8 / 4 rows 0 / 1 / 2; 5: channels from 128 on 1).
-// One kernel, with shapes of its own, runs all the classes of the 3x3 layers (fwd_nine.hip), and one those of the 1x1 layers of
-// stride 1 (fwd_tap.hip), number 2 included.
+// One kernel, with shapes of its own, runs all the classes of the 3x3 layers (fwd_nine.hip), and one those of the 1x1 layers
+// (fwd_tap.hip; plain ones, 1, too unless they are wide maps of few channels), number 2 included.
 int fwd_kernel(const ConvDims &d) {
     const int variant = fwd_tiled_variant(d);
     if (few_positions(d, variant)) return 2;
@@ -588,15 +445,9 @@ int fwd_kernel(const ConvDims &d) {
 }
 
 int fwd_stats_slots(const ConvDims &d) {
-    if (fwd_tap_supported(d)) return fwd_tap_stats_slots(d);
+    if (fwd_tap_supported(d)) return d.stride <= 2 || fwd_tiled_variant(d) ? fwd_tap_stats_slots(d) : 0;
     if (fwd_nine_supported(d)) return fwd_nine_stats_slots(d);
-    if (d.kh == 1 && few_positions(d, fwd_tiled_variant(d))) return ceil_div(d.N * d.Ho * d.Wo, 64);
-    switch (fwd_tiled_variant(d)) {
-        case 8: case 9: return stats_slots_3x3<Fwd1x1sub>(as_one_row(d));
-        case 12: return stats_slots_3x3<Fwd1x1q>(as_one_row(d));
-        case 13: return stats_slots_3x3<Fwd1x1sq>(as_one_row(d));
-        default: return conv1x1_supported(d, nullptr, nullptr) ? fwd_1x1_stats_slots(d) : 0;
-    }
+    return conv1x1_supported(d, nullptr, nullptr) ? fwd_1x1_stats_slots(d) : 0;
 }
 
 // stats (nullable): per-channel partial sums of y and y*y, fwd_stats_slots(d) > 0 slots per channel.
@@ -609,24 +460,15 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
     const int variant = fwd_tiled_variant(d);
     const bool few = few_positions(d, variant);
     if (fwd_tap_supported(d)) {
-        // (it takes bases of any alignment; statistics for planes of whole groups are offered for aligned ones only)
-        if (stats && !few && d.H * d.W % 4 == 0 && !(aligned_groups(x) && aligned_groups(y))) return ADDER_ERR_UNSUPPORTED;
+        // (it takes bases of any alignment; from 64 channels on statistics for planes of whole groups are offered for aligned ones only, below
+        // for strides up to two)
+        const bool aligned = (d.stride > 1 || aligned_groups(x)) && aligned_groups(y);
+        if (stats && (variant ? !few && d.Ho * d.Wo % 4 == 0 && !aligned : d.stride > 2)) return ADDER_ERR_UNSUPPORTED;
         return launch_fwd_tap(x, w, y, stats, d, s, bn);
     }
-    if (d.kh == 1 && few)
-        return launch_fwd_few(x, w, y, stats, d, variant <= 9 ? Fwd1x1sub::CC : Fwd1x1q::CC, s, bn);
     if (fwd_nine_supported(d)) {
         if (stats && !rows_ok) return ADDER_ERR_UNSUPPORTED;   // (it takes bases of any alignment; statistics are offered for aligned ones)
         return launch_fwd_nine(x, w, y, stats, d, s, bn);
-    }
-    const bool strided = variant == 8 || variant == 9 || variant == 12 || variant == 13;
-    if (strided) {   // x is read element by element; y is a dense row per plane
-        const ConvDims f = as_one_row(d);
-        if (f.Wo % 4 != 0 || aligned_groups(y)) switch (variant) {
-            case 8: case 9: return launch_fwd_3x3_v<Fwd1x1sub, false, true, T>(x, w, y, stats, f, s, sampling_of(d), bn);
-            case 12: return launch_fwd_3x3_v<Fwd1x1q, false, true, T>(x, w, y, stats, f, s, sampling_of(d), bn);
-            default: return launch_fwd_3x3_v<Fwd1x1sq, false, true, T>(x, w, y, stats, f, s, sampling_of(d), bn);
-        }
     }
     if (rows_ok && !stats) {   // 5x5 taps; statistics are offered for 3x3 and 1x1 layers
         switch (variant) {
@@ -638,11 +480,7 @@ int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &
             default: break;
         }
     }
-    if (conv1x1_supported(d, x, y)) {
-        // (a tiled variant that was turned down for its alignment counted its statistics slots differently)
-        if (stats && variant != 0) return ADDER_ERR_UNSUPPORTED;
-        return launch_fwd_1x1(x, w, y, stats, d, s, bn);
-    }
+    if (conv1x1_supported(d, x, y)) return launch_fwd_1x1(x, w, y, stats, d, s, bn);
     if (stats) return ADDER_ERR_UNSUPPORTED;   // the generic kernel has no statistics epilogue
     constexpr int TM = 8;
     const long total = (long)d.N * d.Ho * d.Wo;

@@ -6,12 +6,13 @@
 
 namespace adder {
 
-// The sums of the KSP waves, added in the order of the waves; smem holds KSP * TM * TN * 64 floats (one wave: not used).
+// The sums of the KSP waves, added in the order of the waves; smem holds KSP * TM * TN * 64 floats (one wave: not used, unless TURN).
+// TURN: a lane's sums are those of positions lane, 64 + lane, ... of the tile; what it gets is those of TN adjacent ones.
 template <int TM, int KSP>
 static constexpr int kFinished = TM >= KSP ? TM / KSP : 1;
-template <int TM, int TN, int KSP>
+template <int TM, int TN, int KSP, bool TURN = false>
 __device__ __forceinline__ void add_waves(float *smem, int wave, int lane, const float (&tot)[TM][TN], float (&r)[kFinished<TM, KSP>][TN]) {
-    if constexpr (KSP == 1) {
+    if constexpr (KSP == 1 && !TURN) {
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
@@ -29,9 +30,10 @@ __device__ __forceinline__ void add_waves(float *smem, int wave, int lane, const
     for (int f = 0; f < FM; ++f)
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
-            float v = smem[((m0 + f) * TN + t) * 64 + lane];
+            const int e = TURN ? lane * TN + t : t * 64 + lane;
+            float v = smem[(m0 + f) * TN * 64 + e];
 #pragma unroll
-            for (int k = 1; k < KSP; ++k) v += smem[((k * TM + m0 + f) * TN + t) * 64 + lane];
+            for (int k = 1; k < KSP; ++k) v += smem[(k * TM + m0 + f) * TN * 64 + e];
             r[f][t] = v;
         }
 }

@@ -1,4 +1,4 @@
-"""The 1x1 / stride-1 forward kernel (csrc/fwd_tap.hip) against the float64 oracle where its strips, tiles and waves end: planes of 1
+"""The 1x1 forward kernel (csrc/fwd_tap.hip) against the float64 oracle where its strips, tiles and waves end: planes of 1
 to 4 positions and of no whole strips, channels that give a wave no chunk or part of one, output channels that fill no block, one,
 two and four positions per lane -- with its statistics, its inference epilogue, bases of any alignment and both storage types."""
 import pytest
@@ -62,3 +62,44 @@ def test_infinities_and_nan_pass(gpu):
     y = adder.adder2d_function(x.to(gpu), w.to(gpu), 1, 0).cpu()
     want = -(w.view(1, 12, 64, 1, 1) - x.unsqueeze(1)).abs().sum(2)
     assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isinf(), want.isinf())
+
+
+# (N, Ci, H, W, Co, stride): channels below, at and beside whole groups and chunks, with and without a stride; planes whose sampled positions are
+# no whole strips, whose last row or column is not read, and tiles that span several images
+ANY = [(1, 1, 1, 1, 1, 1), (3, 3, 5, 7, 9, 1), (5, 17, 9, 9, 10, 1), (68, 33, 7, 7, 19, 1), (4, 373, 13, 16, 9, 1), (2, 131, 9, 10, 33, 1), (40, 30, 32, 32, 24, 1),
+       (30, 24, 30, 30, 9, 1), (1, 16, 32, 32, 32, 2), (20, 6, 29, 29, 18, 2), (1, 5, 1, 1, 3, 2), (9, 68, 3, 3, 40, 2), (2, 130, 7, 9, 17, 3), (70, 40, 13, 13, 64, 2),
+       (33, 68, 27, 28, 40, 2), (20, 263, 14, 14, 130, 2), (40, 64, 20, 21, 60, 3), (30, 20, 61, 62, 9, 2), (64, 12, 60, 61, 24, 3)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", ANY, ids=str)
+def test_any_channels_and_strides(shape, dtype, gpu):
+    from addernetcuda_amd import adder
+    from addernetcuda_amd._lib import lib, ptr, stream_ptr
+    from oracle import c_oracle
+    N, Ci, H, W, Co, s = shape
+    x, w, gy = make_case(N, Ci, H, W, Co, 1, s, 0)
+    x = x.to(dtype)
+    want = c_oracle.conv2d_fwd(x.float(), w, s, 0)
+    xg, wg = x.to(gpu), w.to(gpu)
+    y = adder.adder2d_function(xg, wg, s, 0)
+    (assert_close if dtype == torch.float32 else _close_bf16)(y, want, f"forward {shape}")
+    off = torch.empty(xg.numel() + 1, dtype=dtype, device=gpu)[1:].view_as(xg).copy_(xg)   # aligned to one element only
+    assert torch.equal(adder.adder2d_function(off, wg, s, 0), y)
+    if dtype != torch.float32:
+        return
+    y2, stats = adder.adder2d_function_with_stats(xg, wg, s, 0)
+    assert torch.equal(y2, y)
+    assert (stats is None) == (s > 2 and (Ci < 64 or Ci % 4 != 0))   # (never offered for those)
+    if stats is not None:
+        tot = stats.sum(dim=1).cpu()
+        assert torch.allclose(tot[:, 0], want.sum(dim=(0, 2, 3)), rtol=1e-5, atol=1e-3)
+        assert torch.allclose(tot[:, 1], (want * want).sum(dim=(0, 2, 3)), rtol=1e-5, atol=1e-2)
+    out, res = torch.empty_like(y), torch.randn_like(y)
+    gamma, beta, mean, var = (torch.rand(Co, device=gpu) + 0.5 for _ in range(4))
+    assert lib.adder_conv2d_fwd_bn_eval_f32(ptr(xg), ptr(wg), ptr(out), ptr(gamma), ptr(beta), ptr(mean), ptr(var), 1e-5, ptr(res), 1,
+                                            N, Ci, H, W, Co, 1, 1, s, 0, stream_ptr(xg.device)) == 0
+    col = lambda t: t.view(1, -1, 1, 1)
+    want = torch.relu((y - col(mean)) * torch.rsqrt(col(var) + 1e-5) * col(gamma) + col(beta) + res)
+    # a few roundings of values of y's size: 4 ulp
+    assert torch.allclose(out, want, rtol=0, atol=4 * 2 ** -23 * (float(y.abs().max()) * 2 + 4))
