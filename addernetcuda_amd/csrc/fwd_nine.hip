@@ -1,5 +1,5 @@
-// Forward of 3x3 / pad 1 layers, stride 1 or 2, NCHW in -> NCHW out:
-//   y[n,co,ho,wo] = - sum_{ci,i,j} | w[co,ci,i,j] - xpad[n,ci,ho*s+i-1,wo*s+j-1] |
+// Forward of 3x3 / pad 1 and 5x5 / pad 2 layers, stride 1 or 2, NCHW in -> NCHW out:
+//   y[n,co,ho,wo] = - sum_{ci,i,j} | w[co,ci,i,j] - xpad[n,ci,ho*s+i-p,wo*s+j-p] |
 // Replaces adder_cuda/adder.cu:19-70 (CONV) together with the unfold + permute copies of adder.py:32-33,38-39 that feed it.
 //
 // Two vector instructions per term bound it: v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- 73 T lane-instructions/s is what a bare
@@ -14,6 +14,13 @@
 // 64 -> 64 @8x8 28.6 -> 25.7; stride 2, 32 images 128 -> 128 @56x56 222 -> 152, 512 -> 512 @14x14 375 -> 203; one image (the kernel for few
 // positions there was) 64 -> 64 @8x8 7.9 -> 5.9, 256 -> 256 @14x14 19 -> 16, 512 -> 512 @7x7 30 -> 29.
 // Tried on the way: 4 channels x 4 positions per lane 132 -> 179 us (64 -> 64 @56x56: reads), 8 x 2 143.
+//
+// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 128 registers.  us, tiles in LDS
+// -> this: 64 -> 64 @56x56, 16 images, 253 -> 190 (floor 166), 128 -> 64 @16x16, 64 images, 135 -> 123, 32 -> 64 @16x16 39.7 -> 38.7, 64 -> 64 @8x8 63 -> 20, one
+// image 62 -> 9.6, 47 -> 19 @14x14, 193 images, 102 -> 58, 9 -> 20 @53x53, 32 images, 47 -> 37, 813 -> 551 @9x9, two images, 872 -> 243 (1.2e-7 -> 5.8e-8 of the
+// result from float64); stride 2: 64 -> 64 @56x56, 32 images, 170 -> 138, 7 -> 144 @23x26, 202 images, 84 -> 51, 36 -> 34 @38x41, 6 images, 30 -> 11, 32 -> 64
+// @32x32, 64 images, 47.5 -> 49.3.  On the way, 64 -> 64 @56x56: comparisons instead of bit masks for what lies outside 387 (the masks of 20 elements fill the scalar
+// registers), the columns beside a strip read one by one 315, three waves per SIMD instead of four with a few spilled registers 218.
 #include "wave_split.hpp"
 
 #include <type_traits>
@@ -22,18 +29,24 @@ namespace adder {
 
 // S: stride; TM output channels x TN adjacent positions per lane; KSP waves that share the input channels in chunks of CC
 // EVEN (stride 2): rows of an even length, whose strips' columns and the one behind them are one read
-template <int S_, int TM_, int TN_, int KSP_, bool EVEN_ = false>
+// KS: taps per side, 3 or 5
+template <int S_, int TM_, int TN_, int KSP_, bool EVEN_ = false, int KS_ = 3>
 struct NineCfg {
     static constexpr int S = S_, TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = kNineChunk, FM = kFinished<TM, KSP>;
+    static constexpr int KS = KS_, KK = KS * KS, PAD = KS / 2;
     static constexpr bool EVEN = EVEN_;
-    static constexpr int AHEAD = TN == 1 ? 3 : 1;   // input channels that x is asked for ahead of the arithmetic
+    static constexpr int AHEAD = TN == 1 && KS == 3 ? 3 : 1;   // input channels that x is asked for ahead of the arithmetic
     // Output channels whose weights are asked for together, a step ahead: a step of one channel x four positions is 72 instructions,
     // enough to hide the request behind; with fewer positions two channels (stride 2: 512 -> 512 @14x14 284 -> 203 us, 256 -> 256 @28x28
     // 181 -> 158; 512 -> 512 @7x7, one image, 32 -> 29).  Two x four positions run out of scalar registers (132 -> 180 us).
-    static constexpr int UM = TN == 4 ? 1 : 2, NU = TM / UM;
-    static constexpr int MID = (TN - 1) * S + 1, STRIP = MID + 2;   // columns under the strip, and with one more on either side
+    static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;
+    static constexpr int MID = (TN - 1) * S + 1, STRIP = MID + 2 * PAD;   // columns under the strip, and with those beside it
     static constexpr int LDS_BYTES = KSP == 1 ? 0 : KSP * TM * TN * 64 * 4;
     static_assert((TM % KSP == 0 || KSP % TM == 0) && (NU == 1 || NU % 2 == 0), "a wave finishes FM channels or none; two weight buffers");
+    // 25 taps, more than one position: the two columns on a side are both inside the map or both outside -- at stride 1 unless a row is four strips and one
+    // column long, at stride 2 on the left, and on the right of rows of an odd length
+    static constexpr bool PAIRS = KS == 5 && TN > 1;
+    static_assert(KS == 3 || KS == 5, "nine or 25 taps");
 };
 
 struct NineDims {
@@ -66,18 +79,19 @@ __device__ __forceinline__ void load_mid(const T *p, float *v) {
 // of a residual block, resnet20.py:66-70) along with it -- its one tap is the centre tap of the 3x3 window: weights w_side (Co, Ci),
 // output y_side and statistics stats_side shaped like y and stats.
 template <class C, class T, bool MUL, bool EVAL, bool PAIR>
-__global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
+__global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
                                                          double *__restrict__ stats, const NineDims d, const BnEval bn,
                                                          const float *__restrict__ w_side, T *__restrict__ y_side,
                                                          double *__restrict__ stats_side) {
     constexpr int S = C::S, TM = C::TM, TN = C::TN, KSP = C::KSP, FM = C::FM, MID = C::MID, STRIP = C::STRIP, NB = C::AHEAD + 1, UM = C::UM, NU = C::NU;
+    constexpr int KS = C::KS, KK = C::KK, PAD = C::PAD;
     extern __shared__ __align__(16) float smem[];
     int tile, blk;
     xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
     const int ho = rest / d.per_row, s = rest - ho * d.per_row, wo = min(s * TN, d.Wo - TN), co_base = blk * TM;
-    const int plane = d.H * d.W, K = d.Ci * 9;
+    const int plane = d.H * d.W, K = d.Ci * KK;
     uniform_f32_ptr wc = as_uniform(w), wsc = as_uniform(w_side);
     int wrow[TM], wsrow[PAIR ? TM : 1];
 #pragma unroll
@@ -90,17 +104,31 @@ __global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x
     const int n_first = __builtin_amdgcn_readfirstlane(n);
     const T *x_first = x + (size_t)n_first * d.Ci * plane;
     const int c0 = wo * S;
+    // (nine taps: a distance per row and side; 25: one per row, and the side columns' distances from the strip, a further add per read)
+    constexpr int NSIDE = KS == 3 ? 3 : 1;
     const bool ok_l = c0 > 0, ok_r = c0 + MID < d.W;
-    bool ok[3];
-    unsigned off[3], off_l[3], off_r[3];
+    bool ok[KS];
+    unsigned in_row[KS], in_col[2 * PAD];   // 25 taps: all ones, or zero for what lies outside (lane masks of 20 elements are 40 scalar registers)
+    unsigned off[KS], off_l[NSIDE], off_r[NSIDE];
+    int beside[2 * PAD];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const int h = ho * S + i - 1;
+    for (int k = 0; k < 2 * PAD; ++k) {
+        const int c = k < PAD ? k - PAD : MID + k - PAD;   // from the strip's first column
+        const bool in = c0 + c >= 0 && c0 + c < d.W;
+        in_col[k] = in ? ~0u : 0u;
+        beside[k] = (in ? c : 0) * (int)sizeof(T);
+    }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+        const int h = ho * S + i - PAD;
         ok[i] = h >= 0 && h < d.H;
+        in_row[i] = ok[i] ? ~0u : 0u;
         const int o = (n - n_first) * d.Ci * plane + min(max(h, 0), d.H - 1) * d.W + c0;
         off[i] = (unsigned)o * (unsigned)sizeof(T);
-        off_l[i] = (unsigned)(ok_l ? o - 1 : o) * (unsigned)sizeof(T);
-        off_r[i] = (unsigned)(ok_r ? o + MID : o) * (unsigned)sizeof(T);
+        if constexpr (KS == 3) {
+            off_l[i] = (unsigned)(ok_l ? o - 1 : o) * (unsigned)sizeof(T);
+            off_r[i] = (unsigned)(ok_r ? o + MID : o) * (unsigned)sizeof(T);
+        }
     }
 
     float acc[TM][TN], tot[TM][TN], side[PAIR ? TM : 1][TN];   // side: Ci / KSP terms each, one level
@@ -111,13 +139,38 @@ __global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x
             acc[m][t] = tot[m][t] = 0.f;
             if constexpr (PAIR) side[m][t] = 0.f;
         }
-    float xr[NB][3][STRIP], wv[2][UM][9], wsv[2][UM];
+    float xr[NB][KS][STRIP], wv[2][UM][KK], wsv[2][UM];
     auto load_x = [&](const int b, const int ci) {
         const char *p = reinterpret_cast<const char *>(x_first + (size_t)ci * plane);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            keep_offset(off[i]); keep_offset(off_l[i]);
-            if constexpr (!C::EVEN) keep_offset(off_r[i]);
+        for (int i = 0; i < KS; ++i) {
+            keep_offset(off[i]);
+            if constexpr (KS == 5) {
+                auto side = [&](const int k) { return reinterpret_cast<const T *>(p + (off[i] + (unsigned)beside[k])); };
+                float *v = xr[b][i], u[4], q[2];
+                if constexpr (C::PAIRS) {
+                    ld_strip<2>(side(0), q);
+                    v[0] = q[0]; v[1] = q[1];
+                } else {
+                    v[0] = ldf(side(0)); v[1] = ldf(side(1));
+                }
+                if constexpr (S == 2 && TN == 2 && C::EVEN) {
+                    ld_strip<4>(reinterpret_cast<const T *>(p + off[i]), u);
+                    v[2] = u[0]; v[3] = u[1]; v[4] = u[2]; v[5] = u[3];
+                    v[6] = ldf(side(3));
+                } else {
+                    load_mid<S, MID>(reinterpret_cast<const T *>(p + off[i]), v + 2);
+                    if constexpr (C::PAIRS) {
+                        ld_strip<2>(side(2), q);
+                        v[MID + 2] = q[0]; v[MID + 3] = q[1];
+                    } else {
+                        v[MID + 2] = ldf(side(2)); v[MID + 3] = ldf(side(3));
+                    }
+                }
+                continue;
+            }
+            keep_offset(off_l[i % NSIDE]);
+            if constexpr (!C::EVEN) keep_offset(off_r[i % NSIDE]);
             if constexpr (C::EVEN) {
                 float u[MID + 1];
                 ld_strip<MID + 1>(reinterpret_cast<const T *>(p + off[i]), u);
@@ -125,16 +178,16 @@ __global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x
                 for (int k = 0; k <= MID; ++k) xr[b][i][k + 1] = u[k];
             } else {
                 load_mid<S, MID>(reinterpret_cast<const T *>(p + off[i]), &xr[b][i][1]);
-                xr[b][i][MID + 1] = ldf(reinterpret_cast<const T *>(p + off_r[i]));
+                xr[b][i][MID + 1] = ldf(reinterpret_cast<const T *>(p + off_r[i % NSIDE]));
             }
-            xr[b][i][0] = ldf(reinterpret_cast<const T *>(p + off_l[i]));
+            xr[b][i][0] = ldf(reinterpret_cast<const T *>(p + off_l[i % NSIDE]));
         }
     };
     auto load_w = [&](const int b, const int h, const int ci) {
 #pragma unroll
         for (int u = 0; u < UM; ++u) {
 #pragma unroll
-            for (int e = 0; e < 9; ++e) wv[b][u][e] = wc[wrow[h * UM + u] + ci * 9 + e];
+            for (int e = 0; e < KK; ++e) wv[b][u][e] = wc[wrow[h * UM + u] + ci * KK + e];
             if constexpr (PAIR) wsv[b][u] = wsc[wsrow[h * UM + u] + ci];
         }
     };
@@ -155,21 +208,40 @@ __global__ __launch_bounds__(C::NT) void fwd_nine_kernel(const T *__restrict__ x
             const bool chunk_end = ((ci + 1) & (C::CC - 1)) == 0, more = next < d.Ci;
             const int cn = more ? next : ci;
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                if (i != 1) {   // (the middle row is inside the map)
+            for (int i = 0; i < KS; ++i) {
+                if (KS == 3 && i != PAD) {   // (the middle row is inside the map)
 #pragma unroll
-                    for (int k = 1; k <= MID; ++k) xr[cur][i][k] = ok[i] ? xr[cur][i][k] : 0.f;
+                    for (int k = PAD; k < PAD + MID; ++k) xr[cur][i][k] = ok[i] ? xr[cur][i][k] : 0.f;
                 }
-                xr[cur][i][0] = ok[i] && ok_l ? xr[cur][i][0] : 0.f;
-                xr[cur][i][MID + 1] = ok[i] && (C::EVEN || ok_r) ? xr[cur][i][MID + 1] : 0.f;
+                if constexpr (KS == 5) {
+                    auto keep = [&](float &v, const unsigned m) { v = __uint_as_float(__float_as_uint(v) & m); };
+                    keep_offset(in_row[i]);
+                    if (i != PAD) {
+#pragma unroll
+                        for (int k = PAD; k < PAD + MID; ++k) keep(xr[cur][i][k], in_row[i]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 2 * PAD; ++k) {
+                        const int e = C::PAIRS && !(C::EVEN && k >= PAD) ? k & ~1 : k;   // (the element of in_col that says so)
+                        if (C::EVEN && k == PAD) {
+                            keep(xr[cur][i][MID + k], in_row[i]);
+                            continue;
+                        }
+                        keep_offset(in_col[e]);
+                        keep(xr[cur][i][k < PAD ? k : MID + k], in_row[i] & in_col[e]);
+                    }
+                } else {
+                    xr[cur][i][0] = ok[i] && ok_l ? xr[cur][i][0] : 0.f;
+                    xr[cur][i][MID + 1] = ok[i] && (C::EVEN || ok_r) ? xr[cur][i][MID + 1] : 0.f;
+                }
             }
 #pragma unroll
             for (int h = 0; h < NU; ++h) {
                 const int wb = (NU == 1 ? cur : h) & 1;
 #pragma unroll
-                for (int idx = 0; idx < UM * 9 * TN; ++idx) {
-                    const int t = idx % TN, j = idx / TN % 3, i = idx / TN / 3 % 3, u = idx / TN / 9, m = h * UM + u;
-                    const float a = wv[wb][u][i * 3 + j], b = xr[cur][i][t * S + j];
+                for (int idx = 0; idx < UM * KK * TN; ++idx) {
+                    const int t = idx % TN, j = idx / TN % KS, i = idx / TN / KS % KS, u = idx / TN / KK, m = h * UM + u;
+                    const float a = wv[wb][u][i * KS + j], b = xr[cur][i][t * S + j];
                     if constexpr (MUL) acc[m][t] = fmaf(a, b, acc[m][t]);
                     else acc[m][t] -= fabsf(a - b);
                     if (idx == 0) {
@@ -237,6 +309,13 @@ static int nine_waves(int Ci) { return Ci <= 8 ? 1 : Ci <= 16 ? 2 : Ci <= 32 ? 4
 // stride 2: 128 -> 128 @56x56, one image, - / 17 / 29, 512 -> 512 @14x14, one, - / 59 / 34.
 struct NineShape { int tm, tn; };
 static NineShape nine_shape(const ConvDims &d) {
+    if (d.kh == 5) {   // 4 x 4, or 4 x 1 for few waves (one image of 64 -> 64 @32x32, 512 waves of 4 x 4, 18.6 / 10.2 us; 64 of @8x8, 2048 waves, 19.8 / 26) and
+                       // where pairs of columns would be cut (PAIRS); stride 2: 4 x 2 (64 -> 64 @16x16, one image, 12.7; 4 x 1 24.6)
+        const int most = d.stride == 1 ? 4 : 2;
+        int tn = d.Wo >= most && (d.stride == 2 || d.W % 4 != 1) ? most : 1;
+        if (tn == 4 && (long)nine_tiles(d, 4) * ceil_div(d.Co, 4) * nine_waves(d.Ci) < 1000) tn = 1;
+        return {4, tn};
+    }
     const int most = d.stride == 1 ? 4 : 2, waves = nine_waves(d.Ci);
     int tn = d.Wo >= most ? most : d.Wo >= 2 ? 2 : 1;
     if (tn == 4 && (long)nine_tiles(d, 4) * ceil_div(d.Co, 8) * waves < 1300) tn = 2;
@@ -249,11 +328,11 @@ static NineShape nine_shape(const ConvDims &d) {
 }
 
 bool fwd_nine_supported(const ConvDims &d) {
-    if (d.kh != 3 || d.kw != 3 || d.pad != 1 || d.stride < 1 || d.stride > 2) return false;
+    if (d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride < 1 || d.stride > 2) return false;
     const long images = 63 / ((long)d.Ho * ceil_div(d.Wo, 4)) + 1;
     return (images * d.Ci + 1) * d.H * d.W <= 0x3fffffffL;
 }
-int fwd_nine_stats_slots(const ConvDims &d) { return nine_tiles(d, nine_shape(d).tn); }
+int fwd_nine_stats_slots(const ConvDims &d) { return d.kh == 3 ? nine_tiles(d, nine_shape(d).tn) : 0; }   // (25 taps: none)
 
 template <class C, class T, bool MUL, bool EVAL, bool PAIR>
 static int launch_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn,
@@ -276,7 +355,9 @@ int launch_fwd_nine(const T *x, const float *w, T *y, double *stats, const ConvD
         using C = decltype(cfg);
         if constexpr (sizeof(T) == 4) {
             if (bn.gamma) return launch_nine<C, T, false, true, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
-            if constexpr (C::S == 1) {
+            if constexpr (C::KS == 5) {
+                if (mul || w_side) return static_cast<int>(ADDER_ERR_UNSUPPORTED);
+            } else if constexpr (C::S == 1) {
                 if (mul) return launch_nine<C, T, true, false, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
             } else {
                 if (w_side) return launch_nine<C, T, false, false, true>(x, w, y, stats, d, s, bn, w_side, y_side, stats_side);
@@ -287,6 +368,11 @@ int launch_fwd_nine(const T *x, const float *w, T *y, double *stats, const ConvD
     const NineShape shape = nine_shape(d);
     auto waves = [&](auto ksp) {
         constexpr int KSP = decltype(ksp)::value;
+        if (d.kh == 5) {
+            if (d.stride == 1) return shape.tn == 4 ? run(NineCfg<1, 4, 4, KSP, false, 5>{}) : run(NineCfg<1, 4, 1, KSP, false, 5>{});
+            if (shape.tn == 2) return d.W % 2 ? run(NineCfg<2, 4, 2, KSP, false, 5>{}) : run(NineCfg<2, 4, 2, KSP, true, 5>{});
+            return run(NineCfg<2, 4, 1, KSP, false, 5>{});
+        }
         if (d.stride == 1) {
             if (shape.tn == 4) return run(NineCfg<1, 8, 4, KSP>{});
             return shape.tn == 2 ? run(NineCfg<1, 8, 2, KSP>{}) : run(NineCfg<1, 4, 1, KSP>{});

@@ -39,7 +39,8 @@ __device__ __forceinline__ void add_waves(float *smem, int wave, int lane, const
 }
 
 // own: bit t of the positions that are this lane's; off: its first one in channel 0 of its image; L: positions per plane.
-// stats (nullable): one slot per tile, sums of deviations from a pivot in fp32, moved back to the origin in fp64 (fwd.hip).
+// stats (nullable): one slot per tile, sums of deviations from a pivot in fp32, moved back to the origin in fp64, so that the
+// cancellation in E[y*y] - E[y]^2 happens in double precision.
 // EVAL: bn is applied (float storage).  whole: four positions are always this lane's own.
 template <int FM, int TN, bool EVAL, class T>
 __device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], unsigned own, int co0, int Co, int L, int off, bool whole,
