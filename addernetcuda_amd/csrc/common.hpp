@@ -364,6 +364,7 @@ template <class T>
 int launch_grad_x_s2(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd, bool sat);
 bool grad_x_s2_supported(const ConvDims &d);
 static constexpr int kSatMaxTerms = 1152;      // terms up to which a 3x3 layer's input gradient takes two instructions a term (grad_x.hip)
+static constexpr bool two_instructions_5x5(int Co) { return Co >= 10 && Co * 25 <= 2500; }   // ... and those of 5x5 layers (grad_x.hip)
 static constexpr int kSatMaxTerms1x1 = 1024;   // output channels up to which a single tap's input gradient takes two instructions a term (grad_x.hip)
 size_t grad_w_workspace_bytes(const ConvDims &d, bool bf16 = false, size_t limit = SIZE_MAX);   // of the storage type's kernels
 int grad_w_kernel(const ConvDims &d, bool bf16);                                                // which of them, as in adder_conv2d_grad_w_kernel

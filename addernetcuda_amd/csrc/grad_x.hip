@@ -555,11 +555,10 @@ __global__ __launch_bounds__(C::NTHREADS, 4) void grad_x_3x3s1_kernel(const T *_
 // Below ten output channels the doubled and the subtracted sum are what rounds, not the length of the sums: 5x5 layers of 1 / 4 / 8
 // channels 1.8e-7 / 2.4e-7 / 2.5e-7 with two instructions, 0.9e-7 / 1.25e-7 / 1.3e-7 with three (kernel without tiles 0.9e-7 / 1.7e-7 / 2.4e-7);
 // 64 -> 8 @32x32, 64 images, 52 -> 63 us.
-static constexpr int kSatMaxTerms5x5 = 2500, kSatMinChannels5x5 = 10;
 template <class C>
 static bool two_instructions(int Co) {
-    if (C::KS == 5 && Co < kSatMinChannels5x5) return false;
-    return Co * C::KK <= (C::KS == 1 ? kSatMaxTerms1x1 : (C::KS == 5 ? kSatMaxTerms5x5 : kSatMaxTerms));
+    if (C::KS == 5) return two_instructions_5x5(Co);
+    return Co * C::KK <= (C::KS == 1 ? kSatMaxTerms1x1 : kSatMaxTerms);
 }
 
 static const adder_bn_links kNoLinks{};
@@ -1082,6 +1081,19 @@ static bool fills_s2_tiles(const ConvDims &d) {
     const int cols = d.W > 16 ? 32 : 16, channels = d.W > 16 ? GxS2W32::TM * GxS2W32::CIW : GxS2W16::TM * GxS2W16::CIW;
     return d.W % cols == 0 && d.H % 16 == 0 && d.Ci % channels == 0 && (long)d.N * (d.H / 16) * (d.W / cols) * (d.Ci / channels) >= 256;
 }
+
+// 5x5 layers of stride 1 that stay in tiles: up to 100 output channels, tiles filled to 85 % and channel groups altogether, a workgroup per CU (us, tiles ->
+// grad_x_nine.hip: 32 -> 64 @16x16, 64 images, 51 -> 53, 64 -> 64 @56x56, 16 images, 268 -> 284, 64 -> 8 @32x32, 64 images, 64.5 -> 65.8; 76 % filled, 16 -> 16 @28x28, 256
+// images, 89 -> 78; three of eight channels, 3 -> 32 @32x32, 128 images, 43 -> 29; 128 workgroups, 64 -> 64 @8x8, 64 images, 50 -> 29; three instructions a
+// term on either side, 128 -> 64 @16x16, 64 images, 212 -> 193).
+static bool fills_5x5_tiles(const ConvDims &d) {
+    if (d.Co > 100 || d.Ci % (Gx5W32::TM * Gx5W32::COW)) return false;
+    const int rows = d.W > 16 ? Gx5W32::TH : d.W > 8 ? Gx5W16::TH : Gx5W8::TH, cols = d.W > 16 ? Gx5W32::TW : d.W > 8 ? Gx5W16::TW : Gx5W8::TW;
+    const long tiles = (long)ceil_div(d.H, rows) * ceil_div(d.W, cols);
+    if (100L * d.H * d.W < 85L * tiles * rows * cols) return false;
+    return ceil_div(d.N, d.W > 8 ? 1 : Gx5W8::NIMG) * tiles * (d.Ci / (Gx5W32::TM * Gx5W32::COW)) >= 256;
+}
+static_assert(Gx5W32::TM * Gx5W32::COW == Gx5W16::TM * Gx5W16::COW && Gx5W32::TM * Gx5W32::COW == Gx5W8::TM * Gx5W8::COW, "one group of channels");
 static_assert(GxW32::TM == GxW16::TM && GxS2W32::TM == GxS2W16::TM,
               "the launcher checks Ci against one TM per stride");
 
@@ -1098,15 +1110,17 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         case 16: return launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
         default: break;
     }
-    if (grad_x_nine_supported(d)) {
-        // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
-        if (gadd && !(d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned))) return ADDER_ERR_UNSUPPORTED;
-        return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr);
-    }
-    if (d.kh == 5 && d.kw == 5 && d.stride == 1 && d.pad == 2 && d.Ci >= Gx5W32::TM && (d.W % 4 != 0 || aligned)) {
+    // (25 taps: the tiles add a second gradient from two input channels on)
+    const bool tiles5 = d.kh == 5 && d.kw == 5 && d.stride == 1 && d.pad == 2 && d.Ci >= Gx5W32::TM && (d.W % 4 != 0 || aligned);
+    if (tiles5 && (fills_5x5_tiles(d) || !grad_x_nine_supported(d))) {
         if (d.W > 16) return launch_grad_x_3x3s1<Gx5W32, false, T>(gy, x, w, gx, d, s, gadd);
         if (d.W > 8) return launch_grad_x_3x3s1<Gx5W16, false, T>(gy, x, w, gx, d, s, gadd);
         return launch_grad_x_3x3s1<Gx5W8, false, T>(gy, x, w, gx, d, s, gadd);
+    }
+    if (grad_x_nine_supported(d)) {
+        // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
+        if (gadd && !(d.kh == 5 ? tiles5 : d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned))) return ADDER_ERR_UNSUPPORTED;
+        return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr);
     }
     // 3x3 with a stride of two: layers the BatchNorm link may ask for (grad_x_bn_variant) keep the tiles, so that the plain call has the linked
     // one's bits; bfloat16, which has no links, only where they are filled and give every CU a workgroup

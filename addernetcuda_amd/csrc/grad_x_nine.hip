@@ -1,5 +1,5 @@
-// Input gradient of 3x3 / pad 1 / stride 1 layers, NCHW:
-//   gx[n,ci,h,w] = sum_{co,i,j} hardtanh(w[co,ci,i,j] - x[n,ci,h,w]) * gy[n,co,h+1-i,w+1-j]
+// Input gradient of 3x3 / pad 1 and 5x5 / pad 2 layers of stride 1, NCHW:
+//   gx[n,ci,h,w] = sum_{co,i,j} hardtanh(w[co,ci,i,j] - x[n,ci,h,w]) * gy[n,co,h+p-i,w+p-j]
 // Replaces the grad_i half of adder_cuda/adder.cu:194-272, adder.cu:133-192 and the fold of adder.py:32-33.
 //
 // The terms are those of grad_x.hip (two vector instructions, three above kSatMaxTerms terms) and bound it.  As in fwd_nine.hip a lane
@@ -10,20 +10,34 @@
 // us, tiles or the kernel for few positions there was -> this: 32 images 64 -> 64 @56x56 169 -> 156, 128 -> 128 @28x28 194 -> 164, 512 -> 512 @7x7
 // 322 -> 251, 100 -> 100 @20x20 119 -> 60; 64 -> 64 @8x8, 256 images 30.6 -> 28.3, one image 29 -> 6; 128 -> 128 @28x28, 4 / 1 images 97 -> 29, 94 -> 14;
 // 48 -> 12 @4x4, 64 images 8.4 -> 5.4; 256 -> 256 @14x14, one image 20 -> 18.
+//
+// 25 taps: 4 channels x 2 positions per lane, three reads per row of the window a channel ahead; rows of an odd length and small launches 4 x 1 with three
+// instructions a term.  us, tiles in LDS -> this: 342 channels of gy -> 48 of gx @10x10, 8 images, 279 -> 57, 261 -> 10 @27x27, 5 images, bfloat16, 206 -> 43,
+// 813 -> 551 @9x9, two images, 730 -> 255, 64 -> 64 @8x8, 64 images, 50 -> 29, one image 44 -> 12, 19 -> 47 @14x14, 193 images, 73 -> 58, 100 -> 100 @28x28, 32 images,
+// bfloat16, 379 -> 311; what fills tiles stays there (fills_5x5_tiles).  Error against float64 1.2e-7 to 2.0e-7 of the result (tiles 2.1e-7 to 3.7e-7).
+// Tried on the way: 4 x 4 per lane 64 -> 64 @56x56, 16 images, 471 (66 registers spilled), 4 x 2 in three instructions 295, with five waves per SIMD 327.
 #include "wave_split.hpp"
 
 #include <type_traits>
 
 namespace adder {
 
+// Output channels per first-level sum: 72 terms (25 taps: 50)
+static constexpr int gx_nine_chunk(int ks) { return ks == 3 ? kNineChunk : 2; }
+
 // TM input channels x TN adjacent positions per lane; KSP waves that share the output channels in chunks of CC
-template <int TM_, int TN_, int KSP_>
+// KS: taps per side, 3 or 5
+template <int TM_, int TN_, int KSP_, int KS_ = 3>
 struct GxNineCfg {
-    static constexpr int TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = kNineChunk, FM = kFinished<TM, KSP>, STRIP = TN + 2;
-    static constexpr int AHEAD = TN == 1 ? 3 : 1;                      // output channels that gy is asked for ahead of the arithmetic
-    static constexpr int UM = TN == 4 ? 1 : 2, NU = TM / UM;           // input channels whose weights are asked for together, a step ahead
+    static constexpr int KS = KS_, KK = KS * KS, PAD = KS / 2;
+    static constexpr int TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = gx_nine_chunk(KS), FM = kFinished<TM, KSP>, STRIP = TN + 2 * PAD;
+    static constexpr int AHEAD = TN == 1 && KS == 3 ? 3 : 1;           // output channels that gy is asked for ahead of the arithmetic
+    static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;   // input channels whose weights are asked for together, a step ahead
     static constexpr int PART = KSP * TM * TN * 64, LDS_BYTES = PART * 4 + KSP * TN * 64 * 8;
     static_assert((TM % KSP == 0 || KSP % TM == 0) && (NU == 1 || NU % 2 == 0), "a wave finishes FM channels or none; two weight buffers");
+    // 25 taps, two positions of rows of an even length: the two columns on a side are both inside the map or both outside, and one read
+    static constexpr bool PAIRS = KS == 5 && TN == 2;
+    static_assert(KS == 3 || (KS == 5 && TN <= 2), "nine taps, or 25 of one or two positions");
 };
 
 struct GxNineDims {
@@ -38,17 +52,18 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
                                                                T *__restrict__ gx, const GxNineDims d, const T *__restrict__ gadd,
                                                                const adder_bn_links bn) {
     constexpr int TM = C::TM, TN = C::TN, KSP = C::KSP, FM = C::FM, STRIP = C::STRIP, NB = C::AHEAD + 1, UM = C::UM, NU = C::NU;
+    constexpr int KS = C::KS, KK = C::KK, PAD = C::PAD;
     extern __shared__ __align__(16) float smem[];
     int tile, blk;
     xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
     const int h = rest / d.per_row, s = rest - h * d.per_row, w0 = min(s * TN, d.W - TN), ci_base = blk * TM;
-    const int plane = d.H * d.W, K = d.Ci * 9;
+    const int plane = d.H * d.W, K = d.Ci * KK;
     uniform_f32_ptr wc = as_uniform(w);
     int wofs[TM];
 #pragma unroll
-    for (int m = 0; m < TM; ++m) wofs[m] = min(ci_base + m, d.Ci - 1) * 9;
+    for (int m = 0; m < TM; ++m) wofs[m] = min(ci_base + m, d.Ci - 1) * KK;
 
     float cr[TM][TN], acc[TM][TN];
 #pragma unroll
@@ -69,39 +84,68 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
     // a uniform base per channel and the lane's distances from it in bytes, as in fwd_nine.hip
     const int n_first = __builtin_amdgcn_readfirstlane(n);
     const T *g_first = gy + (size_t)n_first * d.Co * plane;
+    constexpr int NSIDE = KS == 3 ? 3 : 1;
     const bool ok_l = w0 > 0, ok_r = w0 + TN < d.W;
-    bool ok[3];
-    unsigned off[3], off_l[3], off_r[3];
+    bool ok[KS];
+    unsigned off[KS], off_l[NSIDE], off_r[NSIDE];
+    unsigned in_row[KS], in_col[2 * PAD];   // 25 taps: bit masks and one distance per row, as in fwd_nine.hip
+    int beside[2 * PAD];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const int r = h + i - 1;
+    for (int k = 0; k < 2 * PAD; ++k) {
+        const int c = k < PAD ? k - PAD : TN + k - PAD;   // from the strip's first column
+        const bool in = w0 + c >= 0 && w0 + c < d.W;
+        in_col[k] = in ? ~0u : 0u;
+        beside[k] = (in ? c : 0) * (int)sizeof(T);
+    }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+        const int r = h + i - PAD;
         ok[i] = r >= 0 && r < d.H;
+        in_row[i] = ok[i] ? ~0u : 0u;
         const int o = (n - n_first) * d.Co * plane + min(max(r, 0), d.H - 1) * d.W + w0;
         off[i] = (unsigned)o * (unsigned)sizeof(T);
-        off_l[i] = (unsigned)(ok_l ? o - 1 : o) * (unsigned)sizeof(T);
-        off_r[i] = (unsigned)(ok_r ? o + TN : o) * (unsigned)sizeof(T);
+        if constexpr (KS == 3) {
+            off_l[i] = (unsigned)(ok_l ? o - 1 : o) * (unsigned)sizeof(T);
+            off_r[i] = (unsigned)(ok_r ? o + TN : o) * (unsigned)sizeof(T);
+        }
     }
-    float gr[NB][3][STRIP], wv[2][UM][9], gs[TN];
+    float gr[NB][KS][STRIP], wv[2][UM][KK], gs[TN];
 #pragma unroll
     for (int t = 0; t < TN; ++t) gs[t] = 0.f;
     auto load_g = [&](const int b, const int co) {
         const char *p = reinterpret_cast<const char *>(g_first + (size_t)co * plane);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            keep_offset(off[i]); keep_offset(off_l[i]); keep_offset(off_r[i]);
+        for (int i = 0; i < KS; ++i) {
+            keep_offset(off[i]);
             float u[TN];
             ld_strip<TN>(reinterpret_cast<const T *>(p + off[i]), u);
 #pragma unroll
-            for (int t = 0; t < TN; ++t) gr[b][i][t + 1] = u[t];
-            gr[b][i][0] = ldf(reinterpret_cast<const T *>(p + off_l[i]));
-            gr[b][i][TN + 1] = ldf(reinterpret_cast<const T *>(p + off_r[i]));
+            for (int t = 0; t < TN; ++t) gr[b][i][t + PAD] = u[t];
+            if constexpr (KS == 3) {
+                keep_offset(off_l[i]); keep_offset(off_r[i]);
+                gr[b][i][0] = ldf(reinterpret_cast<const T *>(p + off_l[i]));
+                gr[b][i][TN + 1] = ldf(reinterpret_cast<const T *>(p + off_r[i]));
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k += 2) {
+                    float q[2];
+                    if constexpr (C::PAIRS) {
+                        ld_strip<2>(reinterpret_cast<const T *>(p + (off[i] + (unsigned)beside[k])), q);
+                    } else {
+                        q[0] = ldf(reinterpret_cast<const T *>(p + (off[i] + (unsigned)beside[k])));
+                        q[1] = ldf(reinterpret_cast<const T *>(p + (off[i] + (unsigned)beside[k + 1])));
+                    }
+                    gr[b][i][k < PAD ? k : TN + k] = q[0];
+                    gr[b][i][(k < PAD ? k : TN + k) + 1] = q[1];
+                }
+            }
         }
     };
     auto load_w = [&](const int b, const int hh, const int co) {
 #pragma unroll
         for (int u = 0; u < UM; ++u)
 #pragma unroll
-            for (int e = 0; e < 9; ++e) wv[b][u][e] = wc[co * K + wofs[hh * UM + u] + e];
+            for (int e = 0; e < KK; ++e) wv[b][u][e] = wc[co * K + wofs[hh * UM + u] + e];
     };
     auto after = [&](const int c) { return ((c + 1) & (C::CC - 1)) == 0 ? c + 1 + (KSP - 1) * C::CC : c + 1; };
     int co = wave * C::CC;
@@ -119,32 +163,52 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
             const bool chunk_end = ((co + 1) & (C::CC - 1)) == 0, more = next < d.Co;
             const int cn = more ? next : co;
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {   // positions outside gy contribute nothing
-                if (i != 1) {
+            for (int i = 0; i < KS; ++i) {   // positions outside gy contribute nothing
+                if constexpr (KS == 3) {
+                    if (i != PAD) {
 #pragma unroll
-                    for (int k = 1; k <= TN; ++k) gr[cur][i][k] = ok[i] ? gr[cur][i][k] : 0.f;
+                        for (int k = 1; k <= TN; ++k) gr[cur][i][k] = ok[i] ? gr[cur][i][k] : 0.f;
+                    }
+                    gr[cur][i][0] = ok[i] && ok_l ? gr[cur][i][0] : 0.f;
+                    gr[cur][i][TN + 1] = ok[i] && ok_r ? gr[cur][i][TN + 1] : 0.f;
+                } else {
+                    auto keep = [&](float &v, const unsigned m) { v = __uint_as_float(__float_as_uint(v) & m); };
+                    keep_offset(in_row[i]);
+                    if (i != PAD) {
+#pragma unroll
+                        for (int k = PAD; k < PAD + TN; ++k) keep(gr[cur][i][k], in_row[i]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 2 * PAD; ++k) {
+                        const int e = C::PAIRS ? k & ~1 : k;
+                        keep_offset(in_col[e]);
+                        keep(gr[cur][i][k < PAD ? k : TN + k], in_row[i] & in_col[e]);
+                    }
                 }
-                gr[cur][i][0] = ok[i] && ok_l ? gr[cur][i][0] : 0.f;
-                gr[cur][i][TN + 1] = ok[i] && ok_r ? gr[cur][i][TN + 1] : 0.f;
             }
             if constexpr (SAT) {
+                float c[STRIP];   // sums over the window's rows
+#pragma unroll
+                for (int k = 0; k < STRIP; ++k) {
+                    c[k] = (gr[cur][0][k] + gr[cur][1][k]) + gr[cur][2][k];
+                    if constexpr (KS == 5) c[k] += gr[cur][KS - 2][k] + gr[cur][KS - 1][k];
+                }
 #pragma unroll
                 for (int t = 0; t < TN; ++t) {
-                    float c[3];
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) c[k] = (gr[cur][0][t + k] + gr[cur][1][t + k]) + gr[cur][2][t + k];
-                    gs[t] += (c[0] + c[1]) + c[2];
+                    float v = (c[t] + c[t + 1]) + c[t + 2];
+                    if constexpr (KS == 5) v += c[t + KS - 2] + c[t + KS - 1];
+                    gs[t] += v;
                 }
             }
 #pragma unroll
             for (int hh = 0; hh < NU; ++hh) {
                 const int wb = (NU == 1 ? cur : hh) & 1;
 #pragma unroll
-                for (int idx = 0; idx < UM * 9 * TN; ++idx) {
-                    const int t = idx % TN, j = idx / TN % 3, i = idx / TN / 3 % 3, u = idx / TN / 9, m = hh * UM + u;
-                    const float wgt = wv[wb][u][i * 3 + j];
+                for (int idx = 0; idx < UM * KK * TN; ++idx) {
+                    const int t = idx % TN, j = idx / TN % KS, i = idx / TN / KS % KS, u = idx / TN / KK, m = hh * UM + u;
+                    const float wgt = wv[wb][u][i * KS + j];
                     const float dd = SAT ? sat01(fmaf(wgt, 0.5f, cr[m][t])) : hardtanh(wgt - cr[m][t]);
-                    acc[m][t] = fmaf(dd, gr[cur][2 - i][t + 2 - j], acc[m][t]);
+                    acc[m][t] = fmaf(dd, gr[cur][2 * PAD - i][t + 2 * PAD - j], acc[m][t]);
                     if (idx == 0) {
                         __builtin_amdgcn_sched_barrier(0);
                         load_w(wb ^ 1, hh + 1 < NU ? hh + 1 : 0, hh + 1 < NU ? co : cn);
@@ -158,7 +222,7 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
                 const int c = after(cl);
                 cl = c < d.Co ? c : cl;
             }
-            if (chunk_end || !more) {   // 72-term first levels
+            if (chunk_end || !more) {   // first levels of 72 terms (25 taps: 50)
 #pragma unroll
                 for (int m = 0; m < TM; ++m)
 #pragma unroll
@@ -229,6 +293,9 @@ static int gx_nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((lo
 struct GxNineShape { int tn, waves; };
 static GxNineShape gx_nine_shape(const ConvDims &d) {
     const int waves = d.Co <= 8 ? 1 : d.Co <= 16 ? 2 : d.Co <= 32 ? 4 : 8;
+    if (d.kh == 5)   // us, 4 x 2 / 4 x 1 (W even): 64 -> 64 @8x8, 64 images, 4096 waves of 4 x 2, 32 / 37, 48 -> 342 @10x10, 8 images, 672, 70 / 56, 64 -> 64 @32x32, one, 1024, 17.5 / 13.4;
+                     // W odd, the columns beside a strip one by one: 27 -> 267 @15x15, 40 images, 167 / 160, 551 -> 813 @9x9, two, 347 / 249
+        return {d.W % 2 == 0 && (long)gx_nine_tiles(d, 2) * ceil_div(d.Ci, 4) * waves >= 2048 ? 2 : 1, waves};
     int tn = d.W >= 4 ? 4 : d.W >= 2 ? 2 : 1;
     if (tn == 4 && (long)gx_nine_tiles(d, 4) * ceil_div(d.Ci, 8) * waves < 1300) tn = 2;
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
@@ -242,7 +309,7 @@ static GxNineShape gx_nine_shape(const ConvDims &d) {
 
 // Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.
 bool grad_x_nine_supported(const ConvDims &d) {
-    if (d.kh != 3 || d.kw != 3 || d.pad != 1 || d.stride != 1) return false;
+    if (d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride != 1) return false;
     const long images = 63 / ((long)d.H * ceil_div(d.W, 4)) + 1;
     return (images * d.Co + 1) * d.H * d.W <= 0x3fffffffL;
 }
@@ -270,7 +337,7 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
         using C = decltype(cfg);
         auto form = [&](auto sat) {
             constexpr bool SAT = decltype(sat)::value;
-            if constexpr (sizeof(T) == 4) {
+            if constexpr (sizeof(T) == 4 && C::KS == 3) {
                 if (bn) return launch_gx_nine<C, SAT, T, true>(gy, x, w, gx, d, s, gadd, *bn);
             }
             return launch_gx_nine<C, SAT, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{});
@@ -280,11 +347,15 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
         if constexpr (C::TN == 4) {
             if (d.Co * 9 <= kSatMaxTerms && d.Ci >= 4) return form(std::true_type{});
         }
+        if constexpr (C::PAIRS) {
+            if (two_instructions_5x5(d.Co)) return form(std::true_type{});
+        }
         return form(std::false_type{});
     };
     const GxNineShape shape = gx_nine_shape(d);
     auto waves = [&](auto ksp) {
         constexpr int KSP = decltype(ksp)::value;
+        if (d.kh == 5) return shape.tn == 2 ? run(GxNineCfg<4, 2, KSP, 5>{}) : run(GxNineCfg<4, 1, KSP, 5>{});
         return shape.tn == 4 ? run(GxNineCfg<8, 4, KSP>{}) : shape.tn == 2 ? run(GxNineCfg<8, 2, KSP>{}) : run(GxNineCfg<4, 1, KSP>{});
     };
     switch (shape.waves) {

@@ -50,3 +50,37 @@ def test_infinities_and_nan_pass(gpu):
     u = torch.nn.functional.unfold(x, 5, padding=2)
     want = -(w.view(1, 12, -1, 1) - u.unsqueeze(1)).abs().sum(2).view_as(y)
     assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isinf(), want.isinf())
+
+
+# 4 x 2 and 4 x 1 results per lane with one to eight waves, rows of an odd length, more than 100 output channels; the last two stay in tiles
+GRAD_X = SHAPES + [(40, 33, 16, 18, 12), (64, 40, 10, 10, 40), (9, 30, 22, 26, 131), (33, 40, 16, 16, 30), (70, 64, 16, 16, 24), (40, 64, 8, 32, 12)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", GRAD_X, ids=str)
+def test_input_gradient(shape, dtype, gpu):
+    from addernetcuda_amd import adder
+    from oracle import c_oracle
+    x, w, gy = make_case(*shape, 5, 1, 2)
+    x, gy = x.to(dtype), gy.to(dtype)
+    want = c_oracle.conv2d_grad_x(gy.float(), x.float(), w, 1, 2)
+    for base in (0, 1):   # aligned, and aligned to one element only
+        g = torch.empty(gy.numel() + 1, dtype=dtype, device=gpu)[base:base + gy.numel()].view(gy.shape).copy_(gy)
+        xg = x.to(gpu).requires_grad_(True)
+        adder.adder2d_function(xg, w.to(gpu), 1, 2).backward(g)
+        (assert_close if dtype == torch.float32 else _close_bf16)(xg.grad, want, f"grad_x {shape}, base {base}")
+
+
+@pytest.mark.parametrize("shape", [(2, 7, 5, 6, 9), (64, 40, 10, 10, 40), (70, 64, 16, 16, 24), (2, 1, 9, 9, 4)], ids=str)
+def test_second_gradient(shape, gpu):
+    from addernetcuda_amd._lib import lib, ptr, stream_ptr, conv_dims
+    x, w, gy = (t.to(gpu) for t in make_case(*shape, 5, 1, 2))
+    gadd, gx, out = torch.randn_like(x), torch.empty_like(x), torch.empty_like(x)
+    dims, _, _ = conv_dims(x.shape, w.shape, 1, 2)
+    st = stream_ptr(x.device)
+    assert lib.adder_conv2d_bwd_f32(ptr(gy), ptr(x), ptr(w), ptr(gx), None, 0.0, None, 0, *dims, st) == 0
+    rc = lib.adder_conv2d_bwd_add_f32(ptr(gy), ptr(x), ptr(w), ptr(gadd), ptr(out), None, 0.0, None, 0, *dims, st)
+    if shape[1] >= 2:
+        assert rc == 0 and torch.equal(out, gx + gadd)
+    else:
+        assert rc == -7   # one channel never had one
