@@ -352,6 +352,7 @@ template <class T>
 int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
                       const adder_bn_links *bn);
 bool grad_x_tap_supported(const ConvDims &d);
+bool grad_x_tap_narrow(const ConvDims &d);      // layers it takes beside those, without links and second gradients
 int grad_x_tap_bn_slots(const ConvDims &d);
 // 3x3 / pad 1 / stride 1 (grad_x_nine.hip), likewise
 template <class T>

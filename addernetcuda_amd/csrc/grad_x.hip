@@ -1142,6 +1142,7 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
         return launch_grad_x_tap<T>(gy, x, w, gx, d, s, gadd, nullptr);
     }
     if (gadd) return ADDER_ERR_UNSUPPORTED;
+    if (grad_x_tap_narrow(d)) return launch_grad_x_tap<T>(gy, x, w, gx, d, s, nullptr, nullptr);
     if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride > 1 && d.Ci >= 64 && d.Co >= 64) {
         ConvDims f = d;   // the sampled positions of every plane as one row; x and gx are read / written in place
         f.H = f.Ho = 1;

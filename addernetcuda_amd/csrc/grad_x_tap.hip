@@ -1,4 +1,4 @@
-// Input gradient of 1x1 / stride-1 layers from 64 input and 48 output channels on, NCHW:
+// Input gradient of 1x1 / stride-1 layers from four input and 16 output channels on, NCHW:
 //   gx[n,ci,p] = sum_co hardtanh(w[co,ci] - x[n,ci,p]) * gy[n,co,p]      (adder_cuda/adder.cu:133-272)
 //
 // The terms are those of grad_x.hip (two vector instructions, three above kSatMaxTerms1x1 output channels) and bound it: 90 us for
@@ -210,6 +210,16 @@ bool grad_x_tap_supported(const ConvDims &d) {
     const long L = (long)d.H * d.W, images = 63 / ceil_div_l(L, 2) + 1;
     return (images * d.Co + 1) * L <= 0x3fffffffL;
 }
+// Layers of fewer channels that no BatchNorm is linked to and nothing is added to: three instructions a term, error 7e-8 to 1.4e-7 of the result where
+// conv1x1.hip, which walks all output channels in one wave, has 1.4e-7 to 2.9e-7.  us, conv1x1.hip -> this: 7 -> 482 @10x10, 12 images, 91 -> 14.5, 24 -> 300 @8x8, 64
+// images, 59 -> 7.4, 7 -> 227 @41x40, 26 images, bfloat16, 93 -> 13, 32 -> 200 @56x56, 64 images, 185 -> 86, 40 -> 16 @64x64, 200 images, 111 -> 61, 24 -> 48 @32x32, 64 images,
+// 15.1 -> 12.6, 10 -> 23 @9x9, five, 9.5 -> 7.0, 4 -> 16 @64x64, 64 images, 7.0 -> 7.3; left there: 51 -> 15 @64x64, 23 images, bfloat16, 12.5 -> 13.4, 200 -> 24 @16x16, 64
+// images, 13.9 -> 15.3.
+bool grad_x_tap_narrow(const ConvDims &d) {
+    if (d.kh != 1 || d.kw != 1 || d.pad != 0 || d.stride != 1 || d.Ci < 4 || d.Co < (d.Ci < 64 ? 16 : 32)) return false;
+    const long L = (long)d.H * d.W, images = 63 / ceil_div_l(L, 2) + 1;
+    return (images * d.Co + 1) * L <= 0x3fffffffL;
+}
 int grad_x_tap_bn_slots(const ConvDims &d) { return gx_tap_tiles(d, gx_tap_shape(d).tn); }
 
 template <class C, bool SAT, class T, bool FUSE>
@@ -233,7 +243,12 @@ int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const Conv
     // (8 x 1: 128 -> 512 @28x28 9.5 -> 9.2 us, 64 -> 256 @56x56 8.3 -> 8.5); planes that no BatchNorm can be linked to have it with eight
     // waves too (1024 -> 256 @14x14, 8 images, which can: 26.5 -> 31.9).
     const GxTapShape shape = gx_tap_shape(d);
-    const bool exact = shape.tm == 8 || (shape.waves == 8 && (d.H * d.W) % 4 != 0);
+    if (d.Ci < 16) {   // (no link and no second gradient: grad_x_tap_narrow)
+        auto narrow = [&](auto cfg) { return launch_gx_tap<decltype(cfg), false, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{}); };
+        if (d.Ci < 8) return d.H * d.W >= 2 ? narrow(GxTapCfg<4, 2, 4>{}) : narrow(GxTapCfg<4, 1, 4>{});
+        return shape.tn == 1 ? narrow(GxTapCfg<8, 1, 8>{}) : narrow(GxTapCfg<8, 2, 4>{});
+    }
+    const bool exact = shape.tm == 8 || d.Ci < 64 || (shape.waves == 8 && (d.H * d.W) % 4 != 0);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         auto form = [&](auto sat) {
