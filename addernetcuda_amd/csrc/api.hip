@@ -144,7 +144,7 @@ int adder_conv2d_fwd_bn_eval_f32(const float *x, const float *w, float *y, const
     const Span ins[] = {{x, sizeof(float) * (size_t)N * Ci * H * W}, {w, sizeof(float) * (size_t)Co * d.K()}, {gamma, nco},
                         {beta, nco}, {mean, nco}, {var, nco}, {residual, ny}};
     if (any_alias(outs, ins)) return ADDER_ERR_ALIAS;
-    const BnEval bn{gamma, beta, mean, var, residual, eps, relu, aligned_groups(residual)};
+    const BnEval bn{gamma, beta, mean, var, residual, eps, relu};
     return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream), bn);
 }
 
@@ -157,7 +157,7 @@ int adder_bn_eval_f32(const float *x, float *y, const float *gamma, const float 
     const Span outs[] = {{y, nx}};
     const Span ins[] = {{x, nx}, {gamma, nc}, {beta, nc}, {mean, nc}, {var, nc}, {residual, nx}};
     if (any_alias(outs, ins)) return ADDER_ERR_ALIAS;
-    return launch_bn_eval(x, y, BnEval{gamma, beta, mean, var, residual, eps, relu, 0}, N, C, HW, static_cast<hipStream_t>(stream));
+    return launch_bn_eval(x, y, BnEval{gamma, beta, mean, var, residual, eps, relu}, N, C, HW, static_cast<hipStream_t>(stream));
 }
 
 int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel) {

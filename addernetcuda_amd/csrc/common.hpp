@@ -304,9 +304,9 @@ __device__ __forceinline__ float wave_sum_scatter(float (&v)[K], int lane) {
 struct BnEval {
     const float *gamma, *beta, *mean, *var, *res;   // res (nullable): shaped like the output
     float eps;
-    int relu, res_vec;                              // res_vec: res is aligned to groups of four
+    int relu;
 };
-static constexpr BnEval kNoBnEval{nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0, 0};
+static constexpr BnEval kNoBnEval{nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0};
 struct BnEvalChannel {
     float mean, rstd, gamma, beta;
     __device__ __forceinline__ BnEvalChannel(const BnEval &b, int c)
