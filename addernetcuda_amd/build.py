@@ -11,7 +11,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libaddernet_hip.so")
-SOURCES = ["api.hip", "fwd.hip", "fwd_nine.hip", "fwd_tap.hip", "grad_x.hip", "grad_x_nine.hip", "grad_x_s2.hip", "grad_x_tap.hip", "grad_w.hip", "grad_w_mfma.hip", "grad_w_i8.hip", "conv1x1.hip", "col.hip", "bn_act.hip", "head.hip", "sgd.hip"]
+SOURCES = ["api.hip", "fwd.hip", "fwd_nine.hip", "fwd_tap.hip", "fwd_tile.hip", "grad_x.hip", "grad_x_nine.hip", "grad_x_s2.hip", "grad_x_tap.hip", "grad_w.hip", "grad_w_mfma.hip", "grad_w_i8.hip", "conv1x1.hip", "col.hip", "bn_act.hip", "head.hip", "sgd.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",

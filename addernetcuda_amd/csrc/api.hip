@@ -130,7 +130,7 @@ int adder_conv2d_fwd_f32(const float *x, const float *w, float *y, int N, int Ci
     const size_t nx = sizeof(float) * (size_t)N * Ci * H * W, nw = sizeof(float) * (size_t)Co * d.K(),
                  ny = sizeof(float) * (size_t)N * Co * d.Ho * d.Wo;
     if (overlaps(y, ny, x, nx) || overlaps(y, ny, w, nw)) return ADDER_ERR_ALIAS;
-    return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream));
+    return launch_fwd(x, w, y, d, static_cast<hipStream_t>(stream));
 }
 
 int adder_conv2d_fwd_bn_eval_f32(const float *x, const float *w, float *y, const float *gamma, const float *beta,
@@ -145,7 +145,7 @@ int adder_conv2d_fwd_bn_eval_f32(const float *x, const float *w, float *y, const
                         {beta, nco}, {mean, nco}, {var, nco}, {residual, ny}};
     if (any_alias(outs, ins)) return ADDER_ERR_ALIAS;
     const BnEval bn{gamma, beta, mean, var, residual, eps, relu};
-    return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream), bn);
+    return launch_fwd(x, w, y, d, static_cast<hipStream_t>(stream), bn);
 }
 
 int adder_bn_eval_f32(const float *x, float *y, const float *gamma, const float *beta, const float *mean, const float *var,
@@ -190,7 +190,7 @@ int adder_conv2d_fwd_stats_f32(const float *x, const float *w, float *y, double 
     if (overlaps(y, ny, x, nx) || overlaps(y, ny, w, nw) || overlaps(stats, ns, x, nx) || overlaps(stats, ns, w, nw) ||
         overlaps(stats, ns, y, ny))
         return ADDER_ERR_ALIAS;
-    return launch_fwd(x, w, y, stats, d, static_cast<hipStream_t>(stream));
+    return launch_fwd_stats(x, w, y, stats, d, static_cast<hipStream_t>(stream));
 }
 
 int adder_conv2d_fwd_pair_stats_f32(const float *x, const float *w, const float *w_side, float *y, float *y_side,
@@ -319,7 +319,7 @@ int adder_conv2d_fwd_bf16(const adder_bf16 *x, const float *w, adder_bf16 *y, in
     const size_t nx = sizeof(adder_bf16) * (size_t)N * Ci * H * W, nw = sizeof(float) * (size_t)Co * d.K(),
                  ny = sizeof(adder_bf16) * (size_t)N * Co * d.Ho * d.Wo;
     if (overlaps(y, ny, x, nx) || overlaps(y, ny, w, nw)) return ADDER_ERR_ALIAS;
-    return launch_fwd(x, w, y, nullptr, d, static_cast<hipStream_t>(stream));
+    return launch_fwd(x, w, y, d, static_cast<hipStream_t>(stream));
 }
 
 int adder_conv2d_bwd_bf16(const adder_bf16 *gy, const adder_bf16 *x, const float *w, adder_bf16 *gx, float *gw,

@@ -117,8 +117,8 @@ __device__ __forceinline__ void st_strip(bf16_t *p, const float (&v)[CNT]) {
 // adds base and offset in vector registers at every load; with it the load takes both as they are.
 __device__ __forceinline__ void keep_offset(unsigned &off) { asm volatile("" : "+v"(off)); }
 
-static constexpr int kTapChunk = 16;   // channels per first-level sum of the 1x1 kernels without tiles (fwd_tap.hip, grad_x_tap.hip)
-static constexpr int kNineChunk = 8;   // ... of the 3x3 forward without tiles (fwd_nine.hip): 72 terms
+static constexpr int kTapChunk = 16;   // output channels that a wave of grad_x_tap.hip takes at a time
+static constexpr int kNineChunk = 8;   // ... of grad_x_nine.hip and grad_x_s2.hip: at most 72 terms
 
 // Workgroup number -> (tile, block) of a launch whose blocks read the same tile of x.  Workgroups go to the eight dies in turn, each
 // with its own L2: the blocks of one tile follow each other on one die, so that x crosses to it once.
@@ -326,25 +326,28 @@ int check_launch();                  // hipGetLastError -> status
 
 // Launchers implemented in the kernel translation units.
 // T: storage type of the activations and their gradients, float or bf16_t (the optional reduced-storage mode).
+// Forward without statistics (fwd.hip): which kernel, then those for 1x1 / pad 0 of any stride (fwd_tap.hip) and for 3x3 / pad 1 and
+// 5x5 / pad 2 of stride 1 or 2 (fwd_nine.hip)
 template <class T>
-int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
-template <class T>
-int launch_fwd_tap(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn);
-bool fwd_tap_supported(const ConvDims &d);      // 1x1 / pad 0, any stride (fwd_tap.hip)
-int fwd_tap_stats_slots(const ConvDims &d);
-// 3x3 / pad 1 / stride 1 or 2 (fwd_nine.hip); mul (stride 1, float): an ordinary convolution; w_side, y_side, stats_side (nullable; stride
-// 2, float): the strided 1x1 layer beside it
-template <class T>
-int launch_fwd_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn,
-                    bool mul = false, const float *w_side = nullptr, T *y_side = nullptr, double *stats_side = nullptr);
-bool fwd_nine_supported(const ConvDims &d);
-int fwd_nine_stats_slots(const ConvDims &d);
+int launch_fwd(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
 int fwd_kernel(const ConvDims &d);
-int fwd_stats_slots(const ConvDims &d);
+template <class T>
+int launch_fwd_tap(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn);
+bool fwd_tap_supported(const ConvDims &d);
+template <class T>
+int launch_fwd_nine(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn);
+bool fwd_nine_supported(const ConvDims &d);
+// ... large strided 1x1 layers in tiles (y aligned to groups where planes are whole groups); with statistics, and the ordinary convolution (fwd_tile.hip)
+template <class T>
+int launch_fwd_strided_tile(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn);
+bool fwd_strided_tile_supported(const ConvDims &d);
+int launch_fwd_stats(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
+int fwd_stats_slots(const ConvDims &d);        // 0: no statistics epilogue for these dimensions
+int fwd_chunk(const ConvDims &d);              // input channels per first-level sum of every forward of these dimensions: 8, 16 or 64
 bool fwd_pair_supported(const ConvDims &d);
-int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats,
-                    double *stats_side, const ConvDims &d, hipStream_t s);
-int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);   // 0: no statistics epilogue for these dimensions
+int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats, double *stats_side,
+                    const ConvDims &d, hipStream_t s);
+int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
 // 1x1 / stride 1 (grad_x_tap.hip); bn (nullable): the in_* half of adder_bn_links, slots of sums per channel

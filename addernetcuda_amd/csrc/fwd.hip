@@ -4,8 +4,8 @@
 // copies of adder.py:32-33,38-39 that feed it.
 //
 // Which kernel a layer takes, and the one for any layer.  The inner operation is two fp32 VALU instructions per (co,k,position) term
-// -- v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- and cannot use FMA or MFMA, so the kernels of fwd_nine.hip (3x3, 5x5) and
-// fwd_tap.hip (1x1) keep everything else off the vector ALU: lanes own output positions, weights are wave-uniform and arrive
+// -- v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- and cannot use FMA or MFMA, so the kernels of fwd_nine.hip (3x3, 5x5),
+// fwd_tap.hip (1x1) and fwd_tile.hip (with statistics) keep everything else off the vector ALU: lanes own output positions, weights are wave-uniform and arrive
 // through the scalar cache as SGPR operands.
 #include "common.hpp"
 
@@ -109,19 +109,6 @@ static bool few_positions(const ConvDims &d, int variant) {
     return few < 0.9f * tiled;
 }
 
-// A strided 3x3 / pad 1 layer and the strided 1x1 / pad 0 layer beside it (same x, same Co, Ho, Wo) in one launch;
-// d describes the 3x3 layer.  Both outputs with their statistics (fwd_stats_slots(d) slots each).  Rows of whole
-// float4 groups only; ADDER_ERR_UNSUPPORTED otherwise.
-bool fwd_pair_supported(const ConvDims &d) {
-    return fwd_nine_supported(d) && d.kh == 3 && d.stride == 2 && d.W % 4 == 0 && d.H % 2 == 0;
-}
-
-int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats,
-                    double *stats_side, const ConvDims &d, hipStream_t s) {
-    if (!fwd_pair_supported(d)) return ADDER_ERR_UNSUPPORTED;
-    return launch_fwd_nine<float>(x, w, y, stats, d, s, kNoBnEval, false, w_side, y_side, stats_side);
-}
-
 // rows per tile (16, 8 or 4) that pad a map of H rows least; the larger tile on a tie
 static int rows_per_tile_w32(int H) {
     const int p16 = round_up(H, 16), p8 = round_up(H, 8), p4 = round_up(H, 4);
@@ -140,52 +127,21 @@ int fwd_kernel(const ConvDims &d) {
     return 10 * variant + (variant == 1 ? (rows == 16 ? 0 : rows == 8 ? 1 : 2) : variant == 5 && d.Ci >= 128 ? 1 : 0);
 }
 
-int fwd_stats_slots(const ConvDims &d) {
-    if (fwd_tap_supported(d)) return d.stride <= 2 || fwd_tiled_variant(d) ? fwd_tap_stats_slots(d) : 0;
-    if (fwd_nine_supported(d)) return fwd_nine_stats_slots(d);
-    return conv1x1_supported(d, nullptr, nullptr) ? fwd_1x1_stats_slots(d) : 0;
-}
-
-// stats (nullable): per-channel partial sums of y and y*y, fwd_stats_slots(d) > 0 slots per channel.
-// Both storage types take the same kernels and tile shapes: the arithmetic, which bounds them, is the same fp32.
+// Both storage types take the same kernels and shapes: the arithmetic, which bounds them, is the same fp32.
 // (bfloat16 layers other than 3x3 once went to the generic kernel: 128 -> 512 1x1 @28x28, 32 images, 561 us.)
 template <class T>
-int launch_fwd(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn) {
-    // rows that are whole groups of four are moved as such and need bases aligned to a group
-    const bool rows_ok = (d.W % 4 != 0 || aligned_groups(x)) && (d.Wo % 4 != 0 || aligned_groups(y));
-    const int variant = fwd_tiled_variant(d);
-    const bool few = few_positions(d, variant);
-    if (fwd_tap_supported(d)) {
-        // (it takes bases of any alignment; from 64 channels on statistics for planes of whole groups are offered for aligned ones only, below
-        // for strides up to two)
-        const bool aligned = (d.stride > 1 || aligned_groups(x)) && aligned_groups(y);
-        if (stats && (variant ? !few && d.Ho * d.Wo % 4 == 0 && !aligned : d.stride > 2)) return ADDER_ERR_UNSUPPORTED;
-        return launch_fwd_tap(x, w, y, stats, d, s, bn);
-    }
-    if (fwd_nine_supported(d)) {
-        if (stats && (!rows_ok || d.kh != 3)) return ADDER_ERR_UNSUPPORTED;   // (it takes bases of any alignment; statistics are offered for aligned ones)
-        return launch_fwd_nine(x, w, y, stats, d, s, bn);
-    }
-    if (conv1x1_supported(d, x, y)) return launch_fwd_1x1(x, w, y, stats, d, s, bn);
-    if (stats) return ADDER_ERR_UNSUPPORTED;   // the generic kernel has no statistics epilogue
+int launch_fwd(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn) {
+    if (fwd_strided_tile_supported(d) && (d.Ho * d.Wo % 4 != 0 || aligned_groups(y))) return launch_fwd_strided_tile(x, w, y, d, s, bn);
+    if (fwd_tap_supported(d)) return launch_fwd_tap(x, w, y, d, s, bn);
+    if (fwd_nine_supported(d)) return launch_fwd_nine(x, w, y, d, s, bn);
+    if (conv1x1_supported(d, x, y)) return launch_fwd_1x1(x, w, y, nullptr, d, s, bn);
     constexpr int TM = 8;
     const long total = (long)d.N * d.Ho * d.Wo;
     hipLaunchKernelGGL((fwd_generic_kernel<TM, T>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Co, TM)),
                        dim3(256), 0, s, x, w, y, d, bn);
     return check_launch();
 }
-template int launch_fwd<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t, const BnEval &);
-template int launch_fwd<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t,
-                                const BnEval &);
-
-// An ordinary convolution y = sum w * x through the 3x3 forward kernel: 3x3 / stride 1 / pad 1 only
-// (ADDER_ERR_UNSUPPORTED elsewhere).  stats as in launch_fwd; the slot count is fwd_stats_slots(d).
-int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s) {
-    const bool ok = d.kh == 3 && d.kw == 3 && d.pad == 1 && d.stride == 1 &&
-                    (d.W % 4 != 0 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0);
-    if (!ok) return ADDER_ERR_UNSUPPORTED;
-    if (!fwd_nine_supported(d)) return ADDER_ERR_UNSUPPORTED;
-    return launch_fwd_nine<float>(x, w, y, stats, d, s, kNoBnEval, true);
-}
+template int launch_fwd<float>(const float *, const float *, float *, const ConvDims &, hipStream_t, const BnEval &);
+template int launch_fwd<bf16_t>(const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t, const BnEval &);
 
 }  // namespace adder

@@ -8,18 +8,20 @@
 // reads of at most 16 bytes serve 576 instructions, a quarter of what L1 delivers, so a tile in LDS, its barriers and its halo
 // columns had nothing to give.  Without a tile the strips of all images line up (14 columns are 4 strips, 56 are 14: 88 and 100 % of
 // the lanes have work where 16 x 16 and 8 x 32 tiles left 77 and 88 %), and the waves of a workgroup can share the input channels
-// instead of the positions, which is what small maps with many channels need.
-// us, tiles in LDS -> this: 32 images 64 -> 64 @56x56 158 -> 136, 128 -> 128 @28x28 180 -> 142, 256 -> 256 @14x14 186 -> 163, 512 -> 512 @7x7
-// 284 -> 190, 100 -> 100 @20x20 112 -> 53; 128 images 128 -> 128 @32x32 648 -> 625, 512 -> 512 @8x8 716 -> 688; 256 images 16 -> 16 @32x32 27.0 -> 26.2,
-// 64 -> 64 @8x8 28.6 -> 25.7; stride 2, 32 images 128 -> 128 @56x56 222 -> 152, 512 -> 512 @14x14 375 -> 203; one image (the kernel for few
-// positions there was) 64 -> 64 @8x8 7.9 -> 5.9, 256 -> 256 @14x14 19 -> 16, 512 -> 512 @7x7 30 -> 29.
+// instead of the positions, which is what small maps with many channels need.  Each chunk's sums meet in LDS in channel order (ChunkSums):
+// any other order changes the last bits of a layer, which a deep network amplifies (ResNet-50's logits by up to 0.07 of their root
+// mean square), and costs the launches below 3 to 10 % against sums that meet once at the end, small ones of 16-channel chunks up to 30 %.
+// us, tiles in LDS -> this: 32 images 64 -> 64 @56x56 184 -> 158, 128 -> 128 @28x28 200 -> 169, 256 -> 256 @14x14 208 -> 191, 512 -> 512 @7x7
+// 290 -> 191, 100 -> 100 @20x20 119 -> 66; 128 images 128 -> 128 @32x32 659 -> 627, 512 -> 512 @8x8 716 -> 689; 256 images 16 -> 16 @32x32 30.5 -> 31.2,
+// 64 -> 64 @8x8 31.8 -> 29.5; stride 2, 32 images 128 -> 128 @56x56 225 -> 158, 512 -> 512 @14x14 376 -> 233; one image (the kernel for few
+// positions there was) 64 -> 64 @8x8 7.6 -> 6.6, 256 -> 256 @14x14 19.9 -> 17.0, 512 -> 512 @7x7 30 -> 29.
 // Tried on the way: 4 channels x 4 positions per lane 132 -> 179 us (64 -> 64 @56x56: reads), 8 x 2 143.
 //
-// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 128 registers.  us, tiles in LDS
-// -> this: 64 -> 64 @56x56, 16 images, 253 -> 190 (floor 166), 128 -> 64 @16x16, 64 images, 135 -> 123, 32 -> 64 @16x16 39.7 -> 38.7, 64 -> 64 @8x8 63 -> 20, one
-// image 62 -> 9.6, 47 -> 19 @14x14, 193 images, 102 -> 58, 9 -> 20 @53x53, 32 images, 47 -> 37, 813 -> 551 @9x9, two images, 872 -> 243 (1.2e-7 -> 5.8e-8 of the
-// result from float64); stride 2: 64 -> 64 @56x56, 32 images, 170 -> 138, 7 -> 144 @23x26, 202 images, 84 -> 51, 36 -> 34 @38x41, 6 images, 30 -> 11, 32 -> 64
-// @32x32, 64 images, 47.5 -> 49.3.  On the way, 64 -> 64 @56x56: comparisons instead of bit masks for what lies outside 387 (the masks of 20 elements fill the scalar
+// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 117 to 128 registers (shared
+// bfloat16 layers spill 15 of them).  us, tiles in LDS -> this: 64 -> 64 @56x56, 16 images, 271 -> 202, 128 -> 64 @16x16, 64 images, 137 -> 132, 32 -> 64 @16x16 40.9 -> 39.8,
+// 64 -> 64 @8x8 65 -> 22, one image 61 -> 9.7, 47 -> 19 @14x14, 193 images, 111 -> 71, 9 -> 20 @53x53, 32 images, 51 -> 31, 813 -> 551 @9x9, two images, 865 -> 258;
+// stride 2: 64 -> 64 @56x56, 32 images, 176 -> 145, 7 -> 144 @23x26, 202 images, 86 -> 60, 36 -> 34 @38x41, 6 images, 30 -> 12, 32 -> 64 @32x32, 64 images, 52 -> 55.
+// On the way, 64 -> 64 @56x56: comparisons instead of bit masks for what lies outside 387 (the masks of 20 elements fill the scalar
 // registers), the columns beside a strip read one by one 315, three waves per SIMD instead of four with a few spilled registers 218.
 #include "wave_split.hpp"
 
@@ -27,22 +29,23 @@
 
 namespace adder {
 
-// S: stride; TM output channels x TN adjacent positions per lane; KSP waves that share the input channels in chunks of CC
+// S: stride; TM output channels x TN adjacent positions per lane; SHARED: two to eight waves share the input channels
 // EVEN (stride 2): rows of an even length, whose strips' columns and the one behind them are one read
 // KS: taps per side, 3 or 5
-template <int S_, int TM_, int TN_, int KSP_, bool EVEN_ = false, int KS_ = 3>
+template <int S_, int TM_, int TN_, bool SHARED_, bool EVEN_ = false, int KS_ = 3>
 struct NineCfg {
-    static constexpr int S = S_, TM = TM_, TN = TN_, KSP = KSP_, NT = 64 * KSP, CC = kNineChunk, FM = kFinished<TM, KSP>;
+    static constexpr int S = S_, TM = TM_, TN = TN_, NT = SHARED_ ? 512 : 64;
+    static constexpr bool SHARED = SHARED_;
+    using Sums = ChunkSums<TM, TN, SHARED>;
     static constexpr int KS = KS_, KK = KS * KS, PAD = KS / 2;
     static constexpr bool EVEN = EVEN_;
     static constexpr int AHEAD = TN == 1 && KS == 3 ? 3 : 1;   // input channels that x is asked for ahead of the arithmetic
     // Output channels whose weights are asked for together, a step ahead: a step of one channel x four positions is 72 instructions,
     // enough to hide the request behind; with fewer positions two channels (stride 2: 512 -> 512 @14x14 284 -> 203 us, 256 -> 256 @28x28
     // 181 -> 158; 512 -> 512 @7x7, one image, 32 -> 29).  Two x four positions run out of scalar registers (132 -> 180 us).
-    static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;
+        static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;
     static constexpr int MID = (TN - 1) * S + 1, STRIP = MID + 2 * PAD;   // columns under the strip, and with those beside it
-    static constexpr int LDS_BYTES = KSP == 1 ? 0 : KSP * TM * TN * 64 * 4;
-    static_assert((TM % KSP == 0 || KSP % TM == 0) && (NU == 1 || NU % 2 == 0), "a wave finishes FM channels or none; two weight buffers");
+    static_assert(NU == 1 || NU % 2 == 0, "two weight buffers");
     // 25 taps, more than one position: the two columns on a side are both inside the map or both outside -- at stride 1 unless a row is four strips and one
     // column long, at stride 2 on the left, and on the right of rows of an odd length
     static constexpr bool PAIRS = KS == 5 && TN > 1;
@@ -53,6 +56,7 @@ struct NineDims {
     int N, Ci, H, W, Co, Ho, Wo;
     int per_row, strips;    // strips of TN positions per row (the last one is moved back to end at Wo) and per image
     int tiles, blocks;      // of 64 strips, of TM output channels
+    int chunk, chunks;      // input channels per first-level sum (a power of two), and how many sums there are
 };
 
 // Columns c .. c + MID - 1 of a row, where c + k < W holds for every k that has a position
@@ -74,31 +78,23 @@ __device__ __forceinline__ void load_mid(const T *p, float *v) {
     }
 }
 
-// MUL: an ordinary convolution, y = sum w * x (one v_fmac per term), for the regular stem layer that precedes the adder layers of a
-// network.  EVAL: the inference epilogue.  PAIR (stride 2): the strided 1x1 layer that reads the same x beside this layer (the downsample branch
-// of a residual block, resnet20.py:66-70) along with it -- its one tap is the centre tap of the 3x3 window: weights w_side (Co, Ci),
-// output y_side and statistics stats_side shaped like y and stats.
-template <class C, class T, bool MUL, bool EVAL, bool PAIR>
-__global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
-                                                         double *__restrict__ stats, const NineDims d, const BnEval bn,
-                                                         const float *__restrict__ w_side, T *__restrict__ y_side,
-                                                         double *__restrict__ stats_side) {
-    constexpr int S = C::S, TM = C::TM, TN = C::TN, KSP = C::KSP, FM = C::FM, MID = C::MID, STRIP = C::STRIP, NB = C::AHEAD + 1, UM = C::UM, NU = C::NU;
+// EVAL: the inference epilogue.
+template <class C, class T, bool EVAL>
+__global__ __launch_bounds__(C::NT, 4) void fwd_nine_kernel(const T *__restrict__ x, const float *__restrict__ w, T *__restrict__ y,
+                                                            const NineDims d, const BnEval bn) {
+    constexpr int S = C::S, TM = C::TM, TN = C::TN, MID = C::MID, STRIP = C::STRIP, NB = C::AHEAD + 1, UM = C::UM, NU = C::NU;
     constexpr int KS = C::KS, KK = C::KK, PAD = C::PAD;
     extern __shared__ __align__(16) float smem[];
     int tile, blk;
     xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wave = C::SHARED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, waves = C::SHARED ? blockDim.x >> 6 : 1, lane = threadIdx.x & 63;
     const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
     const int ho = rest / d.per_row, s = rest - ho * d.per_row, wo = min(s * TN, d.Wo - TN), co_base = blk * TM;
     const int plane = d.H * d.W, K = d.Ci * KK;
-    uniform_f32_ptr wc = as_uniform(w), wsc = as_uniform(w_side);
-    int wrow[TM], wsrow[PAIR ? TM : 1];
+    uniform_f32_ptr wc = as_uniform(w);
+    int wrow[TM];
 #pragma unroll
-    for (int m = 0; m < TM; ++m) {
-        wrow[m] = min(co_base + m, d.Co - 1) * K;
-        if constexpr (PAIR) wsrow[m] = min(co_base + m, d.Co - 1) * d.Ci;
-    }
+    for (int m = 0; m < TM; ++m) wrow[m] = min(co_base + m, d.Co - 1) * K;
     // A uniform base per channel and the lane's distances from it in bytes (64 strips: far below 2^32), per row of the window: the
     // strip's own columns and the ones beside them.  What lies outside the map reads an element inside and is zeroed.
     const int n_first = __builtin_amdgcn_readfirstlane(n);
@@ -131,15 +127,13 @@ __global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(con
         }
     }
 
-    float acc[TM][TN], tot[TM][TN], side[PAIR ? TM : 1][TN];   // side: Ci / KSP terms each, one level
+    typename C::Sums sums(smem, wave, lane, waves, d.chunks);
+    float acc[TM][TN];
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            acc[m][t] = tot[m][t] = 0.f;
-            if constexpr (PAIR) side[m][t] = 0.f;
-        }
-    float xr[NB][KS][STRIP], wv[2][UM][KK], wsv[2][UM];
+        for (int t = 0; t < TN; ++t) acc[m][t] = 0.f;
+    float xr[NB][KS][STRIP], wv[2][UM][KK];
     auto load_x = [&](const int b, const int ci) {
         const char *p = reinterpret_cast<const char *>(x_first + (size_t)ci * plane);
 #pragma unroll
@@ -185,15 +179,13 @@ __global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(con
     };
     auto load_w = [&](const int b, const int h, const int ci) {
 #pragma unroll
-        for (int u = 0; u < UM; ++u) {
+        for (int u = 0; u < UM; ++u)
 #pragma unroll
             for (int e = 0; e < KK; ++e) wv[b][u][e] = wc[wrow[h * UM + u] + ci * KK + e];
-            if constexpr (PAIR) wsv[b][u] = wsc[wsrow[h * UM + u] + ci];
-        }
     };
-    auto after = [&](const int c) { return ((c + 1) & (C::CC - 1)) == 0 ? c + 1 + (KSP - 1) * C::CC : c + 1; };
-    int ci = wave * C::CC;
-    if (ci < d.Ci) {
+    auto after = [&](const int c) { return ((c + 1) & (d.chunk - 1)) == 0 ? c + 1 + (waves - 1) * d.chunk : c + 1; };
+    int ci = wave * d.chunk;   // (no more waves than chunks)
+    {
         int cl = ci;   // the channel that x is read of next (the last one again behind the end)
 #pragma unroll
         for (int b = 0; b < C::AHEAD; ++b) {
@@ -205,7 +197,7 @@ __global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(con
         // one input channel; weights one output channel ahead of the arithmetic
         auto channel = [&](const int cur) -> bool {
             const int next = after(ci);
-            const bool chunk_end = ((ci + 1) & (C::CC - 1)) == 0, more = next < d.Ci;
+            const bool chunk_end = ((ci + 1) & (d.chunk - 1)) == 0, more = next < d.Ci;
             const int cn = more ? next : ci;
 #pragma unroll
             for (int i = 0; i < KS; ++i) {
@@ -242,8 +234,7 @@ __global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(con
                 for (int idx = 0; idx < UM * KK * TN; ++idx) {
                     const int t = idx % TN, j = idx / TN % KS, i = idx / TN / KS % KS, u = idx / TN / KK, m = h * UM + u;
                     const float a = wv[wb][u][i * KS + j], b = xr[cur][i][t * S + j];
-                    if constexpr (MUL) acc[m][t] = fmaf(a, b, acc[m][t]);
-                    else acc[m][t] -= fabsf(a - b);
+                    acc[m][t] -= fabsf(a - b);
                     if (idx == 0) {
                         __builtin_amdgcn_sched_barrier(0);
                         load_w(wb ^ 1, h + 1 < NU ? h + 1 : 0, h + 1 < NU ? ci : cn);
@@ -251,24 +242,13 @@ __global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(con
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                if constexpr (PAIR) {
-#pragma unroll
-                    for (int u = 0; u < UM; ++u)
-#pragma unroll
-                        for (int t = 0; t < TN; ++t) side[h * UM + u][t] -= fabsf(wsv[wb][u] - xr[cur][1][t * S + 1]);
-                }
             }
             ci = next;
             {
                 const int c = after(cl);
                 cl = c < d.Ci ? c : cl;
             }
-            if (chunk_end || !more) {
-#pragma unroll
-                for (int m = 0; m < TM; ++m)
-#pragma unroll
-                    for (int t = 0; t < TN; ++t) { tot[m][t] += acc[m][t]; acc[m][t] = 0.f; }
-            }
+            if (chunk_end || !more) sums.add(acc);
             return more;
         };
 #pragma unroll 1
@@ -276,55 +256,60 @@ __global__ __launch_bounds__(C::NT, C::KS == 5 ? 4 : 1) void fwd_nine_kernel(con
         static_assert(NB == 2 || NB == 4, "the buffers take turns");
     }
 
+    sums.finish(acc);
+
     unsigned own = 0;   // bit t: position wo + t is this lane's
 #pragma unroll
     for (int t = 0; t < TN; ++t) own |= (sidx == sc && wo + t >= s * TN ? 1u : 0u) << t;
-    const int L = d.Ho * d.Wo, yoff = n * d.Co * L + ho * d.Wo + wo;
-    const bool whole = TN > 1 && d.Wo % TN == 0;
-    float r[FM][TN];
-    add_waves<TM, TN, KSP>(smem, wave, lane, tot, r);
-    const bool finishes = wave * FM < TM;
-    if (finishes)
-        finish_outputs<FM, TN, EVAL>(r, own, co_base + wave * FM, d.Co, L, yoff, whole, y, stats, d.tiles, tile, lane, bn);
-    if constexpr (PAIR) {
-        __syncthreads();
-        add_waves<TM, TN, KSP>(smem, wave, lane, side, r);
-        if (finishes)
-            finish_outputs<FM, TN, false>(r, own, co_base + wave * FM, d.Co, L, yoff, whole, y_side, stats_side, d.tiles, tile, lane, bn);
-    }
+    const int L = d.Ho * d.Wo, first = sums.first_channel();
+    if (first < TM)
+        finish_outputs<C::Sums::FM, TN, EVAL>(sums.tot, min(sums.per_wave, TM - first), own, co_base + first, d.Co, L, n * d.Co * L + ho * d.Wo + wo,
+                                              TN > 1 && d.Wo % TN == 0, y, bn);
 }
 
 static int nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((long)d.N * d.Ho * ceil_div(d.Wo, tn), 64); }
 
-// Waves that share the channels: one chunk each, as many as eight, by the channels alone, so that a layer's results have the same bits
-// whatever the batch.  us with 2 / 4 / 8: 32 -> 32 @16x16, 256 images, 26 / 26 / 29, 64 -> 64 @8x8 47 / 26 / 25, 64 -> 64 @56x56, 32 images, 145 / 132 / 136,
-// 128 -> 128 @28x28 171 / 145 / 141, 512 -> 512 @7x7 471 / 255 / 189, 128 -> 128 @32x32, 128 images, 648 / 609 / 621.
-static int nine_waves(int Ci) { return Ci <= 8 ? 1 : Ci <= 16 ? 2 : Ci <= 32 ? 4 : 8; }
+// Waves that share the chunks of a launch of wgs workgroups: at most four where that makes 2800 waves, else as many as eight, or five
+// where they need no more rounds: a CU holds 16 waves, three workgroups of five but two of six to eight (144 -> 144, 16 images, us: @28x28, 18 chunks, four waves 117, six 154,
+// eight 116; @14x14, nine chunks, 32 images, four 74, five 66, eight 80).
+static int nine_waves(const ConvDims &d, int chunk, long wgs) {
+    const int chunks = ceil_div(d.Ci, chunk), full = full_chunks(d.Ci, chunk), four = full < 4 ? full : 4;
+    if (wgs * four >= 2800) return four;
+    return chunks >= 5 && ceil_div(chunks, 5) == ceil_div(chunks, 8) ? 5 : chunks < 8 ? chunks : 8;
+}
 
-// Output channels and positions per lane: 8 x 4 (stride 2: 8 x 2), 8 x 2 or 4 x 1, the less the fewer waves there are.  A launch lasts as
+// Output channels and positions per lane: 8 x 4 (stride 2: 8 x 2), 8 x 2, 4 x 1 or 2 x 1, the less the fewer waves there are.  A launch lasts as
 // long as one wave's chain of channels -- 1.43, 0.93 and 0.46 us each -- or as the chip takes for the terms: 30, 26 and 12 per ps, 4 x 1 only
-// 7 on rows that are shorter than 8 and 4.5 at stride 2, where its reads are what fills.  From about 1300 waves of 8 x 4 on the chains
-// overlap.  us, 8 x 4 / 8 x 2 / 4 x 1: 128 -> 128 @28x28, 4 images, 26 / 28 / 35, one image 26 / 17 / 13; 256 -> 256 @14x14, 4, 48 / 32 / 40, one
-// 48 / 32 / 17; 512 -> 512 @7x7, 4 / 2 / 1, 92 / 60 / 68, 92 / 60 / 33, 92 / 60 / 32; 64 -> 64 @56x56, one, 15 / 10 / 13; 16 -> 16 @32x32, 32, 13 / 10 / 8;
-// stride 2: 128 -> 128 @56x56, one image, - / 17 / 29, 512 -> 512 @14x14, one, - / 59 / 34.
-struct NineShape { int tm, tn; };
+// 7 on rows that are shorter than 8 and 4 to 4.5 at stride 2, where its reads are what fills.  Between 8 x 4 and 8 x 2 the busiest CU's workgroups
+// decide.  us, 8 x 4 / 8 x 2 / 4 x 1 / 2 x 1: 128 -> 128 @28x28, 4 images, 31 / 33 / 38 / 48, 256 -> 256 @14x14, 4, 54 / 37 / 41 / 50, 144 -> 144 @14x14, 128, 217 / 203;
+// 86 -> 34 @29x29, 15, 42 / 28 / 33; 64 -> 64 @8x8, one, 23 / 17 / 8.4 / 6.7, 48 -> 12 @4x4, 64, 23 / 16 / 7.8 / 6.4, 64 -> 64 @8x8, 64, 23 / 17 / 14 / 17;
+// stride 2: 40 -> 40 @16x16, 64 images, - / 17 / 20 / 31, 64 -> 64 @8x8, 64, - / 16 / 11.5 / 21.
+struct NineShape { int tm, tn, waves; };
 static NineShape nine_shape(const ConvDims &d) {
+    const int chunk = fwd_chunk(d), chunks = ceil_div(d.Ci, fwd_chunk(d));
     if (d.kh == 5) {   // 4 x 4, or 4 x 1 for few waves (one image of 64 -> 64 @32x32, 512 waves of 4 x 4, 18.6 / 10.2 us; 64 of @8x8, 2048 waves, 19.8 / 26) and
                        // where pairs of columns would be cut (PAIRS); stride 2: 4 x 2 (64 -> 64 @16x16, one image, 12.7; 4 x 1 24.6)
         const int most = d.stride == 1 ? 4 : 2;
         int tn = d.Wo >= most && (d.stride == 2 || d.W % 4 != 1) ? most : 1;
-        if (tn == 4 && (long)nine_tiles(d, 4) * ceil_div(d.Co, 4) * nine_waves(d.Ci) < 1000) tn = 1;
-        return {4, tn};
+        const long wgs = (long)nine_tiles(d, tn) * ceil_div(d.Co, 4);
+        const int waves = nine_waves(d, chunk, wgs);
+        if (tn == 4 && wgs * waves < 1000) return {4, 1, nine_waves(d, chunk, (long)nine_tiles(d, 1) * ceil_div(d.Co, 4))};
+        return {4, tn, waves};
     }
-    const int most = d.stride == 1 ? 4 : 2, waves = nine_waves(d.Ci);
+    const int most = d.stride == 1 ? 4 : 2;
     int tn = d.Wo >= most ? most : d.Wo >= 2 ? 2 : 1;
-    if (tn == 4 && (long)nine_tiles(d, 4) * ceil_div(d.Co, 8) * waves < 1300) tn = 2;
+    auto wgs = [&](int n) { return (long)nine_tiles(d, n) * ceil_div(d.Co, n == 1 ? 4 : 8); };
+    if (tn == 4) {   // the busiest CU's workgroups, by what one of 8 x 4 and of 8 x 2 takes; and waves enough to overlap their chains
+        const int waves = nine_waves(d, chunk, wgs(4));
+        if (wgs(4) * waves < (waves == 1 ? 3300 : waves <= 4 ? 1800 : 1300) || 26 * 2 * ceil_div_l(wgs(4), 256) > 30 * ceil_div_l(wgs(2), 256)) tn = 2;
+    }
+    const int waves = nine_waves(d, chunk, wgs(tn)), share = chunks < 8 ? chunks : 8;
     const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;
-    const int chunks = ceil_div(ceil_div(d.Ci, kNineChunk), waves), chain = min(chunks * kNineChunk, d.Ci);
-    const float wide = fmaxf((tn == 4 ? 1.43f : 0.93f) * chain, terms / (tn == 4 ? 30e6f : 26e6f));
-    const float narrow = fmaxf(0.46f * chain, terms / (d.stride == 2 ? 4.5e6f : d.Wo < 8 ? 7e6f : 12e6f));
-    if (narrow < wide) tn = 1;
-    return {tn == 1 ? 4 : 8, tn};
+    const float wide = fmaxf((tn == 4 ? 1.43f : 0.93f) * min(ceil_div(chunks, waves) * chunk, d.Ci), terms / (tn == 4 ? 30e6f : 26e6f));
+    const float narrow = fmaxf(0.46f * min(ceil_div(chunks, share) * chunk, d.Ci),
+                               d.stride == 2 ? 3.f + terms / (d.Wo < 8 ? 4e6f : 4.5e6f) : terms / (d.Wo < 8 ? 7e6f : 12e6f));
+    if (tn > 1 && narrow >= wide) return {8, tn, waves};
+    return {wgs(1) * share <= (d.stride == 2 ? 200 : chunks <= 8 ? 1024 : 600) ? 2 : 4, 1, share};
 }
 
 bool fwd_nine_supported(const ConvDims &d) {
@@ -332,64 +317,47 @@ bool fwd_nine_supported(const ConvDims &d) {
     const long images = 63 / ((long)d.Ho * ceil_div(d.Wo, 4)) + 1;
     return (images * d.Ci + 1) * d.H * d.W <= 0x3fffffffL;
 }
-int fwd_nine_stats_slots(const ConvDims &d) { return d.kh == 3 ? nine_tiles(d, nine_shape(d).tn) : 0; }   // (25 taps: none)
 
-template <class C, class T, bool MUL, bool EVAL, bool PAIR>
-static int launch_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn,
-                       const float *w_side, T *y_side, double *stats_side) {
+template <class C, class T, bool EVAL>
+static int launch_nine(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn, int waves) {
     const int per_row = ceil_div(d.Wo, C::TN);
-    const NineDims t{d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, per_row, per_row * d.Ho, nine_tiles(d, C::TN), ceil_div(d.Co, C::TM)};
+    const NineDims t{d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, per_row, per_row * d.Ho, nine_tiles(d, C::TN), ceil_div(d.Co, C::TM), fwd_chunk(d), ceil_div(d.Ci, fwd_chunk(d))};
     const long grid = (long)t.tiles * t.blocks;
     if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
-    if (int rc = allow_dynamic_lds<&fwd_nine_kernel<C, T, MUL, EVAL, PAIR>>(C::LDS_BYTES)) return rc;
-    hipLaunchKernelGGL((fwd_nine_kernel<C, T, MUL, EVAL, PAIR>), dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, s, x, w, y, stats, t, bn,
-                       w_side, y_side, stats_side);
+    const int lds = waves * C::Sums::WAVE_FLOATS * 4;
+    if (int rc = allow_dynamic_lds<&fwd_nine_kernel<C, T, EVAL>>(8 * C::Sums::WAVE_FLOATS * 4)) return rc;
+    hipLaunchKernelGGL((fwd_nine_kernel<C, T, EVAL>), dim3((unsigned)grid), dim3(64 * waves), lds, s, x, w, y, t, bn);
     return check_launch();
 }
 
-// w_side != null (stride 2, float storage): the pair.  mul (stride 1, float storage): the ordinary convolution.
 template <class T>
-int launch_fwd_nine(const T *x, const float *w, T *y, double *stats, const ConvDims &d, hipStream_t s, const BnEval &bn, bool mul,
-                    const float *w_side, T *y_side, double *stats_side) {
+int launch_fwd_nine(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn) {
+    const NineShape shape = nine_shape(d);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         if constexpr (sizeof(T) == 4) {
-            if (bn.gamma) return launch_nine<C, T, false, true, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
-            if constexpr (C::KS == 5) {
-                if (mul || w_side) return static_cast<int>(ADDER_ERR_UNSUPPORTED);
-            } else if constexpr (C::S == 1) {
-                if (mul) return launch_nine<C, T, true, false, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
-            } else {
-                if (w_side) return launch_nine<C, T, false, false, true>(x, w, y, stats, d, s, bn, w_side, y_side, stats_side);
-            }
+            if (bn.gamma) return launch_nine<C, T, true>(x, w, y, d, s, bn, shape.waves);
         }
-        return launch_nine<C, T, false, false, false>(x, w, y, stats, d, s, bn, nullptr, nullptr, nullptr);
+        return launch_nine<C, T, false>(x, w, y, d, s, bn, shape.waves);
     };
-    const NineShape shape = nine_shape(d);
-    auto waves = [&](auto ksp) {
-        constexpr int KSP = decltype(ksp)::value;
+    auto waves = [&](auto shared) {
+        constexpr bool SHARED = decltype(shared)::value;
         if (d.kh == 5) {
-            if (d.stride == 1) return shape.tn == 4 ? run(NineCfg<1, 4, 4, KSP, false, 5>{}) : run(NineCfg<1, 4, 1, KSP, false, 5>{});
-            if (shape.tn == 2) return d.W % 2 ? run(NineCfg<2, 4, 2, KSP, false, 5>{}) : run(NineCfg<2, 4, 2, KSP, true, 5>{});
-            return run(NineCfg<2, 4, 1, KSP, false, 5>{});
+            if (d.stride == 1) return shape.tn == 4 ? run(NineCfg<1, 4, 4, SHARED, false, 5>{}) : run(NineCfg<1, 4, 1, SHARED, false, 5>{});
+            if (shape.tn == 2) return d.W % 2 ? run(NineCfg<2, 4, 2, SHARED, false, 5>{}) : run(NineCfg<2, 4, 2, SHARED, true, 5>{});
+            return run(NineCfg<2, 4, 1, SHARED, false, 5>{});
         }
         if (d.stride == 1) {
-            if (shape.tn == 4) return run(NineCfg<1, 8, 4, KSP>{});
-            return shape.tn == 2 ? run(NineCfg<1, 8, 2, KSP>{}) : run(NineCfg<1, 4, 1, KSP>{});
+            if (shape.tn == 4) return run(NineCfg<1, 8, 4, SHARED>{});
+            if (shape.tn == 2) return run(NineCfg<1, 8, 2, SHARED>{});
+            return shape.tm == 4 ? run(NineCfg<1, 4, 1, SHARED>{}) : run(NineCfg<1, 2, 1, SHARED>{});
         }
-        if (shape.tn == 2) return d.W % 2 ? run(NineCfg<2, 8, 2, KSP>{}) : run(NineCfg<2, 8, 2, KSP, true>{});
-        return run(NineCfg<2, 4, 1, KSP>{});
+        if (shape.tn == 2) return d.W % 2 ? run(NineCfg<2, 8, 2, SHARED>{}) : run(NineCfg<2, 8, 2, SHARED, true>{});
+        return shape.tm == 4 ? run(NineCfg<2, 4, 1, SHARED>{}) : run(NineCfg<2, 2, 1, SHARED>{});
     };
-    switch (nine_waves(d.Ci)) {
-        case 1: return waves(std::integral_constant<int, 1>{});
-        case 2: return waves(std::integral_constant<int, 2>{});
-        case 4: return waves(std::integral_constant<int, 4>{});
-        default: return waves(std::integral_constant<int, 8>{});
-    }
+    return shape.waves == 1 ? waves(std::false_type{}) : waves(std::true_type{});
 }
-template int launch_fwd_nine<float>(const float *, const float *, float *, double *, const ConvDims &, hipStream_t, const BnEval &,
-                                    bool, const float *, float *, double *);
-template int launch_fwd_nine<bf16_t>(const bf16_t *, const float *, bf16_t *, double *, const ConvDims &, hipStream_t, const BnEval &,
-                                     bool, const float *, bf16_t *, double *);
+template int launch_fwd_nine<float>(const float *, const float *, float *, const ConvDims &, hipStream_t, const BnEval &);
+template int launch_fwd_nine<bf16_t>(const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t, const BnEval &);
 
 }  // namespace adder

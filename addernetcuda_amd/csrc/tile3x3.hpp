@@ -1,10 +1,10 @@
 // Tile geometry and global->LDS staging shared by the tiled 3x3 / pad-1 and 5x5 / pad-2
 // kernels (stride 1 or 2; the figures below are the 3x3 ones).  A workgroup covers NIMG images x TH x TW positions of the
-// "lane space" (output positions for the weight-gradient kernels,
+// "lane space" (output positions for the forward and weight-gradient kernels,
 // input positions for the stride-1 input gradient) and stages, per channel, the
 // haloed patch of the source tensor those positions touch:
 //   rows  h0*S-1 .. h0*S-1 + (TH-1)*S+2,   columns  w0*S-1 .. w0*S-1 + (TW-1)*S+2,
-// zero-filled outside the tensor.  (For the weight gradient the zeros are the padding
+// zero-filled outside the tensor.  (For those two the zeros are the padding
 // taps, x = 0; for the input gradient they are output positions that do not
 // exist and must contribute nothing.)
 #pragma once
@@ -143,7 +143,7 @@ __device__ __forceinline__ void tile_commit(const TileStage<P> &st, float *buf) 
 }
 
 // Geometry of the tiled kernels (see the header comment).  KS = 3: 3x3 taps, pad 1.  KS = 5: 5x5 taps, pad 2.  KS = 1: a single tap,
-// pad 0 -- no halo; the input gradient of strided 1x1 layers walks the sampled positions of a plane as one long row.
+// pad 0 -- no halo; the positions of a plane (with a stride the sampled ones) are walked as one long row.
 template <int TN_, int SPR_, int TH_, int NIMG_, int TM_, int COW_, int CC_, int CQ_, int S_ = 1, int KS_ = 3>
 struct Tile3x3Cfg {
     static constexpr int TN = TN_, SPR = SPR_, TH = TH_, NIMG = NIMG_, TM = TM_, COW = COW_,

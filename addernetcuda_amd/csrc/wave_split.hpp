@@ -1,87 +1,164 @@
-// What the kernels whose waves share the input channels of one set of results do at their end: add the waves' sums, take the
-// statistics, apply the inference epilogue, store.  A lane holds TM channels x TN adjacent positions; wave v finishes the
-// FM channels from v * FM on: TM / KSP, or one (then the waves from TM on finish none).
+// What the kernels whose waves share the channels of one set of results have in common: sums that meet in LDS, the inference
+// epilogue, the stores.  A lane holds TM channels x TN adjacent positions.
 #pragma once
 #include "common.hpp"
 
 namespace adder {
 
-// The sums of the KSP waves, added in the order of the waves; smem holds KSP * TM * TN * 64 floats (one wave: not used, unless TURN).
-// TURN: a lane's sums are those of positions lane, 64 + lane, ... of the tile; what it gets is those of TN adjacent ones.
-template <int TM, int KSP>
-static constexpr int kFinished = TM >= KSP ? TM / KSP : 1;
-template <int TM, int TN, int KSP, bool TURN = false>
-__device__ __forceinline__ void add_waves(float *smem, int wave, int lane, const float (&tot)[TM][TN], float (&r)[kFinished<TM, KSP>][TN]) {
-    if constexpr (KSP == 1 && !TURN) {
+// TN adjacent floats of LDS, aligned to as many
+template <int TN>
+__device__ __forceinline__ void lds_ld(const float *p, float (&v)[TN]) {
+    static_assert(TN == 1 || TN == 2 || TN == 4, "one, two or four positions");
+    if constexpr (TN == 4) {
+        const float4 u = *reinterpret_cast<const float4 *>(p);
+        v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
+    } else if constexpr (TN == 2) {
+        const float2 u = *reinterpret_cast<const float2 *>(p);
+        v[0] = u.x; v[1] = u.y;
+    } else {
+        v[0] = *p;
+    }
+}
+template <int TN>
+__device__ __forceinline__ void lds_st(float *p, const float (&v)[TN]) {
+    if constexpr (TN == 4) *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    else if constexpr (TN == 2) *reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
+    else *p = v[0];
+}
+
+// Forward sums: chunks of input channels, added in channel order (fwd_chunk), so that a layer's results have the same bits in
+// every kernel and however many waves share its chunks -- wave v takes the chunks v, v + waves, ...
+// SHARED: after each round the waves' chunk sums meet in LDS and a wave adds those of its FM channels, from v * per_wave on, to what
+// it holds.  Otherwise one wave has all chunks and keeps the sums of sums in LDS, a place of its own per lane, which frees TM * TN
+// registers.
+// TURN: a lane's sums are those of positions lane, 64 + lane, ... of the tile; what it has at the end is those of TN adjacent ones.
+template <int TM_, int TN_, bool SHARED_, bool TURN_ = false>
+struct ChunkSums {
+    static constexpr int TM = TM_, TN = TN_;
+    static constexpr bool SHARED = SHARED_, TURN = TURN_;
+    static constexpr int FM = SHARED ? TM / 2 : TM;      // most channels a wave finishes
+    static constexpr int WAVE_FLOATS = TM * TN * 64;     // of LDS
+    static_assert(TM % 2 == 0, "two waves finish half of the channels each");
+    float *smem;
+    int wave, lane, waves, chunks, per_wave, round = 0;
+    float tot[FM][TN];
+
+    __device__ __forceinline__ ChunkSums(float *smem_, int wave_, int lane_, int waves_, int chunks_)
+        : smem(smem_), wave(wave_), lane(lane_), waves(waves_), chunks(chunks_), per_wave(SHARED ? (TM + waves_ - 1) / waves_ : TM) {
+        if constexpr (SHARED) {
+#pragma unroll
+            for (int f = 0; f < FM; ++f)
+#pragma unroll
+                for (int t = 0; t < TN; ++t) tot[f][t] = 0.f;
+        }
+    }
+    __device__ __forceinline__ int chunk() const { return SHARED ? round * waves + wave : round; }   // that this wave is at
+    __device__ __forceinline__ bool pending() const { return chunk() < chunks; }
+    __device__ __forceinline__ int first_channel() const { return SHARED ? wave * per_wave : 0; }
+
+    // A chunk of this wave ends (mine), or it has none in this round: acc -> the sums of sums, and zero.
+    __device__ __forceinline__ void add(float (&acc)[TM][TN], const bool mine = true) {
+        if constexpr (SHARED) {
+            if (round > 0) __syncthreads();   // the sums of the round before have been read
+            if (mine) {
+#pragma unroll
+                for (int m = 0; m < TM; ++m) lds_st<TN>(smem + wave * WAVE_FLOATS + (m * 64 + lane) * TN, acc[m]);
+            }
+            __syncthreads();
+            if (first_channel() < TM) {
+                const int here = min(waves, chunks - round * waves);
+                if (per_wave == 1) gather<1>(here);
+                else if (per_wave == 2) gather<(FM < 2 ? FM : 2)>(here);
+                else if (FM <= 4 || per_wave <= 4) gather<(FM < 4 ? FM : 4)>(here);
+                else gather<FM>(here);
+            }
+        } else if (round == 0) {
+#pragma unroll
+            for (int m = 0; m < TM; ++m) lds_st<TN>(smem + (m * 64 + lane) * TN, acc[m]);
+        } else {
+            constexpr int R = TM < 4 ? TM : 4;   // rows at a time
+#pragma unroll
+            for (int m0 = 0; m0 < TM; m0 += R) {
+                float u[R][TN];
+#pragma unroll
+                for (int m = 0; m < R; ++m) lds_ld<TN>(smem + ((m0 + m) * 64 + lane) * TN, u[m]);
+#pragma unroll
+                for (int m = 0; m < R; ++m) {
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) u[m][t] += acc[m0 + m][t];
+                    lds_st<TN>(smem + ((m0 + m) * 64 + lane) * TN, u[m]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        ++round;
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
-            for (int t = 0; t < TN; ++t) r[m][t] = tot[m][t];
-        return;
+            for (int t = 0; t < TN; ++t) acc[m][t] = 0.f;
     }
+    // this round's sums of the first F of this wave's channels (and of others, which nobody asks for, where it has fewer)
+    template <int F>
+    __device__ __forceinline__ void gather(const int here) {
+        const float *p = smem + (first_channel() * 64 + lane) * TN;
+        const int last = TM - 1 - first_channel();
+        constexpr int B = 8 / F;   // waves whose sums are asked for together
+        for (int v0 = 0; v0 < here; v0 += B) {
+            float u[B][F][TN];
 #pragma unroll
-    for (int m = 0; m < TM; ++m)
+            for (int b = 0; b < B; ++b)
 #pragma unroll
-        for (int t = 0; t < TN; ++t) smem[((wave * TM + m) * TN + t) * 64 + lane] = tot[m][t];
-    __syncthreads();
-    constexpr int FM = kFinished<TM, KSP>;
-    const int m0 = FM * KSP > TM ? min(wave, TM - 1) : wave * FM;   // (a wave that finishes none repeats the last channel)
+                for (int f = 0; f < F; ++f) lds_ld<TN>(p + min(v0 + b, here - 1) * WAVE_FLOATS + min(f, last) * (64 * TN), u[b][f]);
 #pragma unroll
-    for (int f = 0; f < FM; ++f)
+            for (int b = 0; b < B; ++b) {
+                if (v0 + b >= here) break;
 #pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            const int e = TURN ? lane * TN + t : t * 64 + lane;
-            float v = smem[(m0 + f) * TN * 64 + e];
+                for (int f = 0; f < F; ++f)
 #pragma unroll
-            for (int k = 1; k < KSP; ++k) v += smem[(k * TM + m0 + f) * TN * 64 + e];
-            r[f][t] = v;
-        }
-}
-
-// own: bit t of the positions that are this lane's; off: its first one in channel 0 of its image; L: positions per plane.
-// stats (nullable): one slot per tile, sums of deviations from a pivot in fp32, moved back to the origin in fp64, so that the
-// cancellation in E[y*y] - E[y]^2 happens in double precision.
-// EVAL: bn is applied (float storage).  whole: four positions are always this lane's own.
-template <int FM, int TN, bool EVAL, class T>
-__device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], unsigned own, int co0, int Co, int L, int off, bool whole,
-                                               T *__restrict__ y, double *__restrict__ stats, int tiles, int tile, int lane,
-                                               const BnEval &bn) {
-    if (stats) {
-        const double count = (double)wave_sum_dpp((float)__popc(own));
-        float sums[2 * FM], pivot[FM];
-#pragma unroll
-        for (int f = 0; f < FM; ++f) {
-            pivot[f] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r[f][0])));
-            float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-            for (int t = 0; t < TN; ++t)
-                if (own >> t & 1) {
-                    const float dv = r[f][t] - pivot[f];
-                    s1 += dv;
-                    s2 = fmaf(dv, dv, s2);
-                }
-            sums[2 * f] = s1;
-            sums[2 * f + 1] = s2;
-        }
-        if constexpr (FM >= 2 && FM <= 8) {   // all sums in one reduce-scatter: lane l < 2 FM ends with number j(l), moment j % 2 of channel j / 2
-            const float mine = wave_sum_scatter<2 * FM>(sums, lane), other = __shfl_xor(mine, FM, 64);
-            const int j = wave_sum_scatter_index<2 * FM>(lane), f = j >> 1;
-            float piv = pivot[0];
-#pragma unroll
-            for (int k = 1; k < FM; ++k) piv = f == k ? pivot[k] : piv;
-            const double c = (double)piv;
-            if (lane < 2 * FM && co0 + f < Co)
-                stats[((size_t)(co0 + f) * tiles + tile) * 2 + (j & 1)] =
-                    (j & 1) ? (double)mine + 2.0 * c * (double)other + count * c * c : (double)mine + count * c;
-        } else {
-            const double d1 = (double)wave_sum_dpp(sums[0]), d2 = (double)wave_sum_dpp(sums[1]), c = (double)pivot[0];
-            if (lane == 0 && co0 < Co) {
-                double *dst = stats + ((size_t)co0 * tiles + tile) * 2;
-                dst[0] = d1 + count * c;
-                dst[1] = d2 + 2.0 * c * d1 + count * c * c;
+                    for (int t = 0; t < TN; ++t) tot[f][t] += u[b][f][t];
             }
         }
     }
+    // Behind the last chunk: a wave that had none in the last round meets the others there; tot holds this wave's results
+    __device__ __forceinline__ void finish(float (&acc)[TM][TN]) {
+        if constexpr (SHARED) {
+            if (round * waves < chunks) add(acc, false);
+        } else {
+#pragma unroll
+            for (int m = 0; m < TM; ++m) lds_ld<TN>(smem + (m * 64 + lane) * TN, tot[m]);
+        }
+        if constexpr (TURN) {
+            __syncthreads();   // the last sums have been read
+            float *p = smem + first_channel() * (64 * TN);
+#pragma unroll
+            for (int f = 0; f < FM; ++f)
+                if (first_channel() + f < TM && f < per_wave) {
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) p[(f * TN + t) * 64 + lane] = tot[f][t];
+                }
+            __syncthreads();
+#pragma unroll
+            for (int f = 0; f < FM; ++f)
+                if (first_channel() + f < TM && f < per_wave) lds_ld<TN>(p + (f * 64 + lane) * TN, tot[f]);
+        }
+    }
+};
+
+// Waves that share `chunks` chunks, at most `most`: as few as finish them in the same number of rounds
+static inline int waves_for(int chunks, int most) { return ceil_div(chunks, ceil_div(chunks, most)); }
+
+// Chunks of `channels` input channels, one less where less than half of the last one is filled: what counts where waves share them
+static inline int full_chunks(int channels, int chunk) {
+    const int chunks = ceil_div(channels, chunk);
+    return chunks > 1 && 2 * (channels - (chunks - 1) * chunk) < chunk ? chunks - 1 : chunks;
+}
+
+// The waves' results on their way out, count of the FM channels from co0 on.  own: bit t of the positions that are this lane's; off: its
+// first one in channel 0 of its image; L: positions per plane.  EVAL: bn is applied (float storage).  whole: TN positions are always
+// this lane's own.
+template <int FM, int TN, bool EVAL, class T>
+__device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], int count, unsigned own, int co0, int Co, int L, int off, bool whole,
+                                               T *__restrict__ y, const BnEval &bn) {
     if constexpr (EVAL) {
         float a[FM][TN];
 #pragma unroll
@@ -102,7 +179,7 @@ __device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], unsigned own,
     }
 #pragma unroll
     for (int f = 0; f < FM; ++f) {
-        if (co0 + f >= Co) break;
+        if (f >= count || co0 + f >= Co) break;
         T *dst = y + (size_t)(co0 + f) * L + off;
         if (whole && own) {
             if constexpr (TN == 4 || TN == 2) st_strip<TN>(dst, r[f]);
@@ -114,7 +191,11 @@ __device__ __forceinline__ void finish_outputs(float (&r)[FM][TN], unsigned own,
     }
 }
 
-// The same for input gradients: a second gradient (gadd, nullable) is added, the first pass of the BatchNorm in front of the layer is
+// Of the rows of results of an input gradient, those that one of KSP waves finishes: all share them, or one each
+template <int TM, int KSP>
+static constexpr int kFinished = TM >= KSP ? TM / KSP : 1;
+
+// Input gradients likewise: a second gradient (gadd, nullable) is added, the first pass of the BatchNorm in front of the layer is
 // made where FUSE (the in_* fields of adder_bn_links: one slot of sums per tile; float storage), channels first <= c < Ci of the
 // FM from ci0 on are stored.  off: the lane's first position in channel ci0.
 template <int FM, int TN, bool FUSE, class T>
