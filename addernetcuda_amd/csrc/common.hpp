@@ -350,6 +350,12 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
+// Whether the input gradient of a stride-1 layer is small and has no kernel that a BatchNorm is linked to: bfloat16, or rows (1x1: planes) that are no
+// whole groups of four.  Those take three instructions a term: the doubled sum minus the sum of gy that two need rounds once more (3x3 of 60 to
+// 100 output channels: 2.4e-7 of the result against 1.7e-7, the largest element 1.5 times as far) and makes an infinite gy NaN.
+static constexpr bool small_unlinked(const ConvDims &d, bool bf16, int row, long elements) {
+    return (bf16 || row % 4 != 0) && (long)d.N * d.Ci * d.H * d.W < elements;
+}
 // 1x1 / stride 1 (grad_x_tap.hip); bn (nullable): the in_* half of adder_bn_links, slots of sums per channel
 template <class T>
 int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
@@ -357,10 +363,11 @@ int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const Conv
 bool grad_x_tap_supported(const ConvDims &d);
 bool grad_x_tap_narrow(const ConvDims &d);      // layers it takes beside those, without links and second gradients
 int grad_x_tap_bn_slots(const ConvDims &d);
-// 3x3 / pad 1 / stride 1 (grad_x_nine.hip), likewise
+// 3x3 / pad 1 and 5x5 / pad 2 / stride 1 (grad_x_nine.hip), likewise; groups: rows are no whole groups of four, or the bases are aligned to
+// groups (elsewhere three instructions a term)
 template <class T>
 int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
-                       const adder_bn_links *bn);
+                       const adder_bn_links *bn, bool groups = true);
 bool grad_x_nine_supported(const ConvDims &d);
 int grad_x_nine_bn_slots(const ConvDims &d);
 // 3x3 / pad 1 and 5x5 / pad 2 / stride 2 (grad_x_s2.hip); sat: two instructions a term

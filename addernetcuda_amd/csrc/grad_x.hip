@@ -1120,7 +1120,7 @@ int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims
     if (grad_x_nine_supported(d)) {
         // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
         if (gadd && !(d.kh == 5 ? tiles5 : d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned))) return ADDER_ERR_UNSUPPORTED;
-        return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr);
+        return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr, d.W % 4 != 0 || aligned);
     }
     // 3x3 with a stride of two: layers the BatchNorm link may ask for (grad_x_bn_variant) keep the tiles, so that the plain call has the linked
     // one's bits; bfloat16, which has no links, only where they are filled and give every CU a workgroup

@@ -332,7 +332,7 @@ static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const 
 // bn (nullable): the in_* half of adder_bn_links
 template <class T>
 int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
-                       const adder_bn_links *bn) {
+                       const adder_bn_links *bn, bool groups) {
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         auto form = [&](auto sat) {
@@ -345,10 +345,10 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
         // The two-instruction form only where the launch fills the chip: below that it gains nothing (32 -> 32 @16x16, 32 images, 9.1 us,
         // three instructions 8.8; 64 -> 64 @56x56, one, 11.9, 13.2) and rounds w and x once more (1.6e-7 of the result against 2.3e-7).
         if constexpr (C::TN == 4) {
-            if (d.Co * 9 <= kSatMaxTerms && d.Ci >= 4) return form(std::true_type{});
+            if (groups && d.Co * 9 <= kSatMaxTerms && d.Ci >= 4 && !small_unlinked(d, sizeof(T) == 2, d.W, 660000)) return form(std::true_type{});
         }
         if constexpr (C::PAIRS) {
-            if (two_instructions_5x5(d.Co)) return form(std::true_type{});
+            if (groups && d.Ci >= 2 && two_instructions_5x5(d.Co)) return form(std::true_type{});
         }
         return form(std::false_type{});
     };
@@ -366,8 +366,8 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
     }
 }
 template int launch_grad_x_nine<float>(const float *, const float *, const float *, float *, const ConvDims &, hipStream_t,
-                                       const float *, const adder_bn_links *);
+                                       const float *, const adder_bn_links *, bool);
 template int launch_grad_x_nine<bf16_t>(const bf16_t *, const bf16_t *, const float *, bf16_t *, const ConvDims &, hipStream_t,
-                                        const bf16_t *, const adder_bn_links *);
+                                        const bf16_t *, const adder_bn_links *, bool);
 
 }  // namespace adder

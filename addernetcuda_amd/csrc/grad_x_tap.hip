@@ -241,14 +241,15 @@ int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const Conv
                       const adder_bn_links *bn) {
     // The three-instruction form rounds once less (error 8.7e-8 of the result, two instructions 1.58e-7) and costs a small launch nothing
     // (8 x 1: 128 -> 512 @28x28 9.5 -> 9.2 us, 64 -> 256 @56x56 8.3 -> 8.5); planes that no BatchNorm can be linked to have it with eight
-    // waves too (1024 -> 256 @14x14, 8 images, which can: 26.5 -> 31.9).
+    // waves too (1024 -> 256 @14x14, 8 images, which can: 26.5 -> 31.9), and so have narrow layers and small ones without a link (small_unlinked).
     const GxTapShape shape = gx_tap_shape(d);
     if (d.Ci < 16) {   // (no link and no second gradient: grad_x_tap_narrow)
         auto narrow = [&](auto cfg) { return launch_gx_tap<decltype(cfg), false, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{}); };
         if (d.Ci < 8) return d.H * d.W >= 2 ? narrow(GxTapCfg<4, 2, 4>{}) : narrow(GxTapCfg<4, 1, 4>{});
         return shape.tn == 1 ? narrow(GxTapCfg<8, 1, 8>{}) : narrow(GxTapCfg<8, 2, 4>{});
     }
-    const bool exact = shape.tm == 8 || d.Ci < 64 || (shape.waves == 8 && (d.H * d.W) % 4 != 0);
+    const bool exact = shape.tm == 8 || !grad_x_tap_supported(d) || (shape.waves == 8 && (d.H * d.W) % 4 != 0) ||
+                       small_unlinked(d, sizeof(T) == 2, d.H * d.W, 770000);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         auto form = [&](auto sat) {
