@@ -320,6 +320,13 @@ struct ConvDims {
     __host__ __device__ int K() const { return Ci * kh * kw; }
 };
 
+// A wave's strips of `strips` per image lie in the image of the first and so many behind it
+static inline long images_ahead(const ConvDims &d, long strips) {
+    const long most = 63 / strips + 1;
+    return most < d.N - 1 ? most : d.N - 1;
+}
+static constexpr long kMaxThreads = 0xffffffffL;   // of a launch
+
 // ---- host-side launch plumbing -------------------------------------------------
 int record_hip_error(hipError_t e);  // stores the message, returns ADDER_ERR_HIP
 int check_launch();                  // hipGetLastError -> status

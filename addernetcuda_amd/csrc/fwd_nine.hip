@@ -312,21 +312,21 @@ static NineShape nine_shape(const ConvDims &d) {
     return {wgs(1) * share <= (d.stride == 2 ? 200 : chunks <= 8 ? 1024 : 600) ? 2 : 4, 1, share};
 }
 
+// Layers it takes: the distance of a wave's strips from the first one's image has to fit 32 bits, and so have the launch's threads.
 bool fwd_nine_supported(const ConvDims &d) {
     if (d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride < 1 || d.stride > 2) return false;
-    const long images = 63 / ((long)d.Ho * ceil_div(d.Wo, 4)) + 1;
-    return (images * d.Ci + 1) * d.H * d.W <= 0x3fffffffL;
+    if ((images_ahead(d, (long)d.Ho * ceil_div(d.Wo, 4)) * d.Ci + 1) * d.H * d.W > 0x3fffffffL) return false;
+    const NineShape shape = nine_shape(d);
+    return (long)nine_tiles(d, shape.tn) * ceil_div(d.Co, shape.tm) * 64 * shape.waves <= kMaxThreads;
 }
 
 template <class C, class T, bool EVAL>
 static int launch_nine(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn, int waves) {
     const int per_row = ceil_div(d.Wo, C::TN);
     const NineDims t{d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, per_row, per_row * d.Ho, nine_tiles(d, C::TN), ceil_div(d.Co, C::TM), fwd_chunk(d), ceil_div(d.Ci, fwd_chunk(d))};
-    const long grid = (long)t.tiles * t.blocks;
-    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
     const int lds = waves * C::Sums::WAVE_FLOATS * 4;
     if (int rc = allow_dynamic_lds<&fwd_nine_kernel<C, T, EVAL>>(8 * C::Sums::WAVE_FLOATS * 4)) return rc;
-    hipLaunchKernelGGL((fwd_nine_kernel<C, T, EVAL>), dim3((unsigned)grid), dim3(64 * waves), lds, s, x, w, y, t, bn);
+    hipLaunchKernelGGL((fwd_nine_kernel<C, T, EVAL>), dim3((unsigned)t.tiles * t.blocks), dim3(64 * waves), lds, s, x, w, y, t, bn);
     return check_launch();
 }
 

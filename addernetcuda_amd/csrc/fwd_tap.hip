@@ -205,23 +205,22 @@ static TapShape tap_shape(const ConvDims &d) {
 
 // Layers it takes: all but large strided ones of 8-channel chunks (fwd_strided_tile_supported) and wide maps of few channels, which memory bounds and conv1x1.hip reads in rows (24 -> 48 @32x32, 64 images, 9.6 us there, 10.1
 // here; 8 -> 64 @64x64 of stride 2 10.1, 10.5; 7 -> 227 @41x40, 26 images, bfloat16, 11.1, 11.5; 32 -> 200 @56x56 106, 70).  The distance of a wave's
-// strips from the first one's image has to fit 32 bits.
+// strips from the first one's image has to fit 32 bits, and so have the launch's threads.
 bool fwd_tap_supported(const ConvDims &d) {
     if (d.kh != 1 || d.kw != 1 || d.pad != 0) return false;
     if (d.Ci <= 24 && d.stride <= 2 && (long)d.N * d.Ho * d.Wo >= 16384) return false;
-    const long images = 63 / ceil_div_l((long)d.Ho * d.Wo, 4) + 1;
-    return (images * d.Ci + 1) * d.H * d.W <= 0x3fffffffL;
+    if ((images_ahead(d, ceil_div_l((long)d.Ho * d.Wo, 4)) * d.Ci + 1) * d.H * d.W > 0x3fffffffL) return false;
+    const TapShape shape = tap_shape(d);
+    return (long)tap_tiles(d, shape.tn) * ceil_div(d.Co, shape.tm) * 64 * shape.waves <= kMaxThreads;
 }
 
 template <class C, class T, bool EVAL>
 static int launch_tap(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn, int waves) {
     const TapDims t{d.N, d.Ci, d.Co, d.Ho * d.Wo, d.H * d.W, d.W, d.Wo, d.stride, ceil_div(d.Ho * d.Wo, C::TN), tap_tiles(d, C::TN), ceil_div(d.Co, C::TM),
                     fwd_chunk(d), tap_chunks(d)};
-    const long grid = (long)t.tiles * t.blocks;
-    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
     const int lds = waves * C::Sums::WAVE_FLOATS * 4;
     if (int rc = allow_dynamic_lds<&fwd_tap_kernel<C, T, EVAL>>(8 * C::Sums::WAVE_FLOATS * 4)) return rc;
-    hipLaunchKernelGGL((fwd_tap_kernel<C, T, EVAL>), dim3((unsigned)grid), dim3(64 * waves), lds, s, x, w, y, t, bn);
+    hipLaunchKernelGGL((fwd_tap_kernel<C, T, EVAL>), dim3((unsigned)t.tiles * t.blocks), dim3(64 * waves), lds, s, x, w, y, t, bn);
     return check_launch();
 }
 

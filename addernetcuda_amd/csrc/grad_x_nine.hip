@@ -307,11 +307,12 @@ static GxNineShape gx_nine_shape(const ConvDims &d) {
     return {tn, tn == 4 && d.Co <= 12 ? 1 : waves};
 }
 
-// Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.
+// Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits, and so have the launch's threads.
 bool grad_x_nine_supported(const ConvDims &d) {
     if (d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride != 1) return false;
-    const long images = 63 / ((long)d.H * ceil_div(d.W, 4)) + 1;
-    return (images * d.Co + 1) * d.H * d.W <= 0x3fffffffL;
+    if ((images_ahead(d, (long)d.H * ceil_div(d.W, 4)) * d.Co + 1) * d.H * d.W > 0x3fffffffL) return false;
+    const GxNineShape shape = gx_nine_shape(d);
+    return (long)gx_nine_tiles(d, shape.tn) * ceil_div(d.Ci, d.kh == 5 || shape.tn == 1 ? 4 : 8) * 64 * shape.waves <= kMaxThreads;
 }
 int grad_x_nine_bn_slots(const ConvDims &d) { return gx_nine_tiles(d, gx_nine_shape(d).tn); }
 
@@ -320,11 +321,9 @@ static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const 
                           const adder_bn_links &bn) {
     const int per_row = ceil_div(d.W, C::TN);
     const GxNineDims t{d.N, d.Ci, d.H, d.W, d.Co, per_row, per_row * d.H, gx_nine_tiles(d, C::TN), ceil_div(d.Ci, C::TM)};
-    const long grid = (long)t.tiles * t.blocks;
-    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
     if (FUSE && (!bn.in_part || bn.in_slots != t.tiles)) return ADDER_ERR_BAD_SHAPE;
     if (int rc = allow_dynamic_lds<&grad_x_nine_kernel<C, SAT, T, FUSE>>(C::LDS_BYTES)) return rc;
-    hipLaunchKernelGGL((grad_x_nine_kernel<C, SAT, T, FUSE>), dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
+    hipLaunchKernelGGL((grad_x_nine_kernel<C, SAT, T, FUSE>), dim3((unsigned)t.tiles * t.blocks), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
                        gadd, bn);
     return check_launch();
 }

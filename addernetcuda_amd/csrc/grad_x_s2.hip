@@ -266,8 +266,7 @@ static bool gx_s2_wide(const ConvDims &d) {
 // Layers it takes: from two input channels on; the distance of a wave's strips from the first one's image has to fit 32 bits, and the grid 2^32 threads.
 bool grad_x_s2_supported(const ConvDims &d) {
     if (d.Ci < 2 || d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride != 2) return false;
-    const long images = 63 / ((long)d.Ho * d.Wo) + 1;
-    if ((images * d.Co + 1) * d.Ho * d.Wo > 0x3fffffffL || (long)d.Ci * d.H * d.W > 0x7fffffffL) return false;
+    if ((images_ahead(d, (long)d.Ho * d.Wo) * d.Co + 1) * d.Ho * d.Wo > 0x3fffffffL || (long)d.Ci * d.H * d.W > 0x7fffffffL) return false;
     return (long)gx_s2_tiles(d) * ceil_div(d.Ci, 2) <= 0x7fffffL;
 }
 

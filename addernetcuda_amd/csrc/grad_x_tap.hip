@@ -204,11 +204,15 @@ static GxTapShape gx_tap_shape(const ConvDims &d) {
     return {16, 2, d.Co <= 128 && wgs >= 2048 ? 1 : 4};
 }
 
-// Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.
+// Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits.  (The launch's threads do for tensors below 2^31
+// elements: eight waves share 512 output channels or a few hundred workgroups only, and four of them have 4 x 2 results a lane at least.)
+static bool gx_tap_fits(const ConvDims &d) {
+    const long L = (long)d.H * d.W;
+    return (images_ahead(d, ceil_div_l(L, 2)) * d.Co + 1) * L <= 0x3fffffffL;
+}
 bool grad_x_tap_supported(const ConvDims &d) {
     if (d.kh != 1 || d.kw != 1 || d.pad != 0 || d.stride != 1 || d.Ci < 64 || d.Co < 48) return false;
-    const long L = (long)d.H * d.W, images = 63 / ceil_div_l(L, 2) + 1;
-    return (images * d.Co + 1) * L <= 0x3fffffffL;
+    return gx_tap_fits(d);
 }
 // Layers of fewer channels that no BatchNorm is linked to and nothing is added to: three instructions a term, error 7e-8 to 1.4e-7 of the result where
 // conv1x1.hip, which walks all output channels in one wave, has 1.4e-7 to 2.9e-7.  us, conv1x1.hip -> this: 7 -> 482 @10x10, 12 images, 91 -> 14.5, 24 -> 300 @8x8, 64
@@ -217,8 +221,7 @@ bool grad_x_tap_supported(const ConvDims &d) {
 // images, 13.9 -> 15.3.
 bool grad_x_tap_narrow(const ConvDims &d) {
     if (d.kh != 1 || d.kw != 1 || d.pad != 0 || d.stride != 1 || d.Ci < 4 || d.Co < (d.Ci < 64 ? 16 : 32)) return false;
-    const long L = (long)d.H * d.W, images = 63 / ceil_div_l(L, 2) + 1;
-    return (images * d.Co + 1) * L <= 0x3fffffffL;
+    return gx_tap_fits(d);
 }
 int grad_x_tap_bn_slots(const ConvDims &d) { return gx_tap_tiles(d, gx_tap_shape(d).tn); }
 
@@ -226,11 +229,9 @@ template <class C, bool SAT, class T, bool FUSE>
 static int launch_gx_tap(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
                          const adder_bn_links &bn) {
     const GxTapDims t{d.N, d.Ci, d.Co, d.H * d.W, ceil_div(d.H * d.W, C::TN), gx_tap_tiles(d, C::TN), ceil_div(d.Ci, C::TM)};
-    const long grid = (long)t.tiles * t.blocks;
-    if (grid > 0x7fffffL) return ADDER_ERR_TOO_LARGE;   // (2^32 threads; tensors below 2^31 elements stay far from it)
     if (FUSE && (!bn.in_part || bn.in_slots != t.tiles)) return ADDER_ERR_BAD_SHAPE;
     if (int rc = allow_dynamic_lds<&grad_x_tap_kernel<C, SAT, T, FUSE>>(C::LDS_BYTES)) return rc;
-    hipLaunchKernelGGL((grad_x_tap_kernel<C, SAT, T, FUSE>), dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
+    hipLaunchKernelGGL((grad_x_tap_kernel<C, SAT, T, FUSE>), dim3((unsigned)t.tiles * t.blocks), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
                        gadd, bn);
     return check_launch();
 }
