@@ -33,6 +33,8 @@ _SIGNATURES = {
     "adder_out_dim": (_i, [_i, _i, _i, _i]),
     "adder_conv2d_fwd_f32": (_i, [_p, _p, _p] + [_i] * 9 + [_p]),
     "adder_conv2d_fwd_kernel": (_i, [_i] * 9 + [ctypes.POINTER(ctypes.c_int)]),
+    "adder_conv2d_fwd_stats_kernel": (_i, [_i] * 9 + [ctypes.POINTER(ctypes.c_int)]),
+    "adder_conv2d_grad_x_kernel": (_i, [_i] * 10 + [ctypes.POINTER(ctypes.c_int)]),
     "adder_conv2d_grad_w_kernel": (_i, [_i] * 10 + [ctypes.POINTER(ctypes.c_int)]),
     "adder_conv2d_fwd_bn_eval_f32": (_i, [_p] * 7 + [_f, _p] + [_i] * 10 + [_p]),
     "adder_bn_eval_f32": (_i, [_p] * 6 + [_f, _p] + [_i] * 4 + [_p]),

@@ -168,6 +168,22 @@ int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw,
     return ADDER_OK;
 }
 
+int adder_conv2d_fwd_stats_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel) {
+    if (!kernel) return ADDER_ERR_NULL_POINTER;
+    ConvDims d;
+    if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
+    *kernel = fwd_stats_kernel(d);
+    return ADDER_OK;
+}
+
+int adder_conv2d_grad_x_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int bf16, int *kernel) {
+    if (!kernel) return ADDER_ERR_NULL_POINTER;
+    ConvDims d;
+    if (int rc = make_dims(N, Ci, H, W, Co, kh, kw, stride, pad, d)) return rc;
+    *kernel = grad_x_kernel(d, bf16 != 0);
+    return ADDER_OK;
+}
+
 int adder_conv2d_fwd_stats_slots(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad,
                                  int *slots) {
     if (!slots) return ADDER_ERR_NULL_POINTER;

@@ -335,9 +335,13 @@ int check_launch();                  // hipGetLastError -> status
 // T: storage type of the activations and their gradients, float or bf16_t (the optional reduced-storage mode).
 // Forward without statistics (fwd.hip): which kernel, then those for 1x1 / pad 0 of any stride (fwd_tap.hip) and for 3x3 / pad 1 and
 // 5x5 / pad 2 of stride 1 or 2 (fwd_nine.hip)
+enum class FwdKernel { general = 0, plain_1x1 = 1, strided_tile = 2, tap = 3, nine = 4 };
+struct LaneShape { int tm, tn, waves; };        // channels and positions per lane, waves that share the channels that are summed over
 template <class T>
 int launch_fwd(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn = kNoBnEval);
-int fwd_kernel(const ConvDims &d);
+int fwd_kernel(const ConvDims &d);              // as in adder_conv2d_fwd_kernel
+LaneShape fwd_tap_shape(const ConvDims &d);
+LaneShape fwd_nine_shape(const ConvDims &d);
 template <class T>
 int launch_fwd_tap(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn);
 bool fwd_tap_supported(const ConvDims &d);
@@ -350,6 +354,7 @@ int launch_fwd_strided_tile(const T *x, const float *w, T *y, const ConvDims &d,
 bool fwd_strided_tile_supported(const ConvDims &d);
 int launch_fwd_stats(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
 int fwd_stats_slots(const ConvDims &d);        // 0: no statistics epilogue for these dimensions
+int fwd_stats_kernel(const ConvDims &d);       // as in adder_conv2d_fwd_stats_kernel
 int fwd_chunk(const ConvDims &d);              // input channels per first-level sum of every forward of these dimensions: 8, 16 or 64
 bool fwd_pair_supported(const ConvDims &d);
 int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *y, float *y_side, double *stats, double *stats_side,
@@ -357,6 +362,11 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
 int launch_mulconv_fwd(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s);
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd = nullptr);
+int grad_x_kernel(const ConvDims &d, bool bf16);   // as in adder_conv2d_grad_x_kernel
+struct GradXShape { int tm, tn, waves; bool two; };   // of the kernels without tiles; two: two instructions a term, not three
+GradXShape grad_x_tap_shape(const ConvDims &d, bool bf16);
+GradXShape grad_x_nine_shape(const ConvDims &d, bool bf16, bool groups);
+GradXShape grad_x_s2_shape(const ConvDims &d, bool sat);
 // Whether the input gradient of a stride-1 layer is small and has no kernel that a BatchNorm is linked to: bfloat16, or rows (1x1: planes) that are no
 // whole groups of four.  Those take three instructions a term: the doubled sum minus the sum of gy that two need rounds once more (3x3 of 60 to
 // 100 output channels: 2.4e-7 of the result against 1.7e-7, the largest element 1.5 times as far) and makes an infinite gy NaN.

@@ -75,66 +75,31 @@ __global__ __launch_bounds__(256) void fwd_generic_kernel(const T *__restrict__ 
     }
 }
 
-// A class of sizes (0 = none): 1..3 3x3 stride 1 by output width, 4..5 3x3 stride 2 (all fwd_nine.hip),
-// 6..7 1x1 stride 1 from 64 channels on by plane size, 8..9 1x1 with a stride, 10..13 = 6..9 for channels that are no multiple of 8 (all
-// fwd_tap.hip), 14..18 5x5 (stride 1 by output width, then stride 2; fwd_nine.hip)
-static int fwd_tiled_variant(const ConvDims &d) {
-    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.Ci % 4 == 0 && d.Ci >= 64) {
-        const int quad = d.Ci % 8 ? 4 : 0, plane = d.Ho * d.Wo;
-        const bool wide = ceil_div(plane, 256) * 256 <= ceil_div(plane, 64) * 64;
-        if (d.stride == 1) return (wide ? 6 : 7) + quad;
-        return (wide ? 8 : 9) + quad;
-    }
-    if (d.kh == 5 && d.kw == 5 && d.pad == 2) {
-        if (d.stride == 1) return d.Wo > 16 ? 14 : (d.Wo > 8 ? 15 : 16);
-        if (d.stride == 2) return d.Wo > 8 ? 17 : 18;
-        return 0;
-    }
-    if (d.kh != 3 || d.kw != 3 || d.pad != 1) return 0;
-    if (d.stride == 1) return d.Wo > 16 ? 1 : (d.Wo > 8 ? 2 : 3);
-    if (d.stride == 2) return d.Wo > 8 ? 4 : 5;
-    return 0;
+// Which kernel a forward without statistics takes; y aligned to groups of four.  (The others take bases of any alignment.)
+static FwdKernel choose_fwd(const ConvDims &d, bool y_aligned) {
+    if (fwd_strided_tile_supported(d) && (d.Ho * d.Wo % 4 != 0 || y_aligned)) return FwdKernel::strided_tile;
+    if (fwd_tap_supported(d)) return FwdKernel::tap;
+    if (fwd_nine_supported(d)) return FwdKernel::nine;
+    return conv1x1_supported(d, nullptr, nullptr) ? FwdKernel::plain_1x1 : FwdKernel::general;
 }
 
-// Whether a 3x3 or 1x1 layer has few positions: a class of sizes that fwd_kernel tells apart, and whose statistics are offered for bases of
-// any alignment.  fwd_nine.hip and fwd_tap.hip choose their shapes by rules of their own.
-static bool few_positions(const ConvDims &d, int variant) {
-    if (variant == 0 || variant >= 14 || ceil_div(d.Co, 4) > kMaxGridY) return false;
-    const int per_lane = variant >= 3 && variant <= 5 ? 8 : variant == 8 || variant == 9 ? 32 : 16;
-    const int chunk = variant == 1 || variant == 4 || variant == 8 || variant == 9 || (variant == 5 && d.Ci >= 128) ? 8 : 16;
-    const float terms = (float)d.K() * d.Co * d.N * d.Ho * d.Wo;
-    const float tiled = 0.006f * d.K() * per_lane;
-    const float share = (float)(ceil_div(ceil_div(d.Ci, chunk), 8) * chunk);
-    const float few = 2.f + (d.kh == 3 ? 0.4f * share + terms / 10.9e6f : 0.25f * share + terms / 3.2e6f);
-    return few < 0.9f * tiled;
-}
-
-// rows per tile (16, 8 or 4) that pad a map of H rows least; the larger tile on a tie
-static int rows_per_tile_w32(int H) {
-    const int p16 = round_up(H, 16), p8 = round_up(H, 8), p4 = round_up(H, 4);
-    return p16 <= p8 && p16 <= p4 ? 16 : (p8 <= p4 ? 8 : 4);
-}
-
-// Which kernel launch_fwd runs without statistics and for bases aligned to groups of four: 0 general, 1 plain 1x1, 2 few
-// positions, else 10 * variant + a class of sizes (3x3 on wide maps: whole groups of 16 / 8 / 4 rows 0 / 1 / 2; 5: channels from 128 on 1).
-// One kernel, with shapes of its own, runs all the classes of the 3x3 layers (fwd_nine.hip), and one those of the 1x1 layers
-// (fwd_tap.hip; plain ones, 1, too unless they are wide maps of few channels), number 2 included.
 int fwd_kernel(const ConvDims &d) {
-    const int variant = fwd_tiled_variant(d);
-    if (few_positions(d, variant)) return 2;
-    if (variant == 0) return conv1x1_supported(d, nullptr, nullptr) ? 1 : 0;
-    const int rows = rows_per_tile_w32(d.Ho);
-    return 10 * variant + (variant == 1 ? (rows == 16 ? 0 : rows == 8 ? 1 : 2) : variant == 5 && d.Ci >= 128 ? 1 : 0);
+    const FwdKernel kernel = choose_fwd(d, true);
+    const LaneShape shape = kernel == FwdKernel::tap ? fwd_tap_shape(d) : kernel == FwdKernel::nine ? fwd_nine_shape(d) : LaneShape{0, 0, 0};
+    return static_cast<int>(kernel) * 100000 + shape.tm * 1000 + shape.tn * 100 + shape.waves;
 }
 
 // Both storage types take the same kernels and shapes: the arithmetic, which bounds them, is the same fp32.
 // (bfloat16 layers other than 3x3 once went to the generic kernel: 128 -> 512 1x1 @28x28, 32 images, 561 us.)
 template <class T>
 int launch_fwd(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn) {
-    if (fwd_strided_tile_supported(d) && (d.Ho * d.Wo % 4 != 0 || aligned_groups(y))) return launch_fwd_strided_tile(x, w, y, d, s, bn);
-    if (fwd_tap_supported(d)) return launch_fwd_tap(x, w, y, d, s, bn);
-    if (fwd_nine_supported(d)) return launch_fwd_nine(x, w, y, d, s, bn);
-    if (conv1x1_supported(d, x, y)) return launch_fwd_1x1(x, w, y, nullptr, d, s, bn);
+    switch (choose_fwd(d, aligned_groups(y))) {
+        case FwdKernel::strided_tile: return launch_fwd_strided_tile(x, w, y, d, s, bn);
+        case FwdKernel::tap: return launch_fwd_tap(x, w, y, d, s, bn);
+        case FwdKernel::nine: return launch_fwd_nine(x, w, y, d, s, bn);
+        case FwdKernel::plain_1x1: return launch_fwd_1x1(x, w, y, nullptr, d, s, bn);
+        case FwdKernel::general: break;
+    }
     constexpr int TM = 8;
     const long total = (long)d.N * d.Ho * d.Wo;
     hipLaunchKernelGGL((fwd_generic_kernel<TM, T>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Co, TM)),

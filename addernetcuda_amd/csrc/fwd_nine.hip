@@ -284,8 +284,7 @@ static int nine_waves(const ConvDims &d, int chunk, long wgs) {
 // decide.  us, 8 x 4 / 8 x 2 / 4 x 1 / 2 x 1: 128 -> 128 @28x28, 4 images, 31 / 33 / 38 / 48, 256 -> 256 @14x14, 4, 54 / 37 / 41 / 50, 144 -> 144 @14x14, 128, 217 / 203;
 // 86 -> 34 @29x29, 15, 42 / 28 / 33; 64 -> 64 @8x8, one, 23 / 17 / 8.4 / 6.7, 48 -> 12 @4x4, 64, 23 / 16 / 7.8 / 6.4, 64 -> 64 @8x8, 64, 23 / 17 / 14 / 17;
 // stride 2: 40 -> 40 @16x16, 64 images, - / 17 / 20 / 31, 64 -> 64 @8x8, 64, - / 16 / 11.5 / 21.
-struct NineShape { int tm, tn, waves; };
-static NineShape nine_shape(const ConvDims &d) {
+LaneShape fwd_nine_shape(const ConvDims &d) {
     const int chunk = fwd_chunk(d), chunks = ceil_div(d.Ci, fwd_chunk(d));
     if (d.kh == 5) {   // 4 x 4, or 4 x 1 for few waves (one image of 64 -> 64 @32x32, 512 waves of 4 x 4, 18.6 / 10.2 us; 64 of @8x8, 2048 waves, 19.8 / 26) and
                        // where pairs of columns would be cut (PAIRS); stride 2: 4 x 2 (64 -> 64 @16x16, one image, 12.7; 4 x 1 24.6)
@@ -316,7 +315,7 @@ static NineShape nine_shape(const ConvDims &d) {
 bool fwd_nine_supported(const ConvDims &d) {
     if (d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride < 1 || d.stride > 2) return false;
     if ((images_ahead(d, (long)d.Ho * ceil_div(d.Wo, 4)) * d.Ci + 1) * d.H * d.W > 0x3fffffffL) return false;
-    const NineShape shape = nine_shape(d);
+    const LaneShape shape = fwd_nine_shape(d);
     return (long)nine_tiles(d, shape.tn) * ceil_div(d.Co, shape.tm) * 64 * shape.waves <= kMaxThreads;
 }
 
@@ -332,7 +331,7 @@ static int launch_nine(const T *x, const float *w, T *y, const ConvDims &d, hipS
 
 template <class T>
 int launch_fwd_nine(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn) {
-    const NineShape shape = nine_shape(d);
+    const LaneShape shape = fwd_nine_shape(d);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         if constexpr (sizeof(T) == 4) {

@@ -184,8 +184,7 @@ static int tap_chunks(const ConvDims &d) {
 // 1024 -> 256 @14x14, 4 images 42 / 34; 512 -> 128 @28x28, 4 images, 22.7 / 24.3), and one position where that leaves half the chip idle or costs no
 // more tiles (64 strips of two on a plane of 49; 2048 -> 512 @7x7, 4 images, 78 / 55 / 45); 4 x 1 up to 1400 waves of 8 x 1, whose weights are what
 // a wave waits for (8 x 1 / 4 x 1: 300 -> 48 @8x8, one image, 9.4 / 6.9, 64 images, 1920 waves, 13.9 / 13.2, 11.9 with 8 x 2).
-struct TapShape { int tm, tn, waves; };
-static TapShape tap_shape(const ConvDims &d) {
+LaneShape fwd_tap_shape(const ConvDims &d) {
     const int L = d.Ho * d.Wo, blocks = ceil_div(d.Co, kTapTM), chunks = tap_chunks(d), waves = waves_for(chunks, 8);
     int tn = L >= 4 ? 4 : L >= 2 ? 2 : 1;
     if (tn == 4 && (long)tap_tiles(d, 4) * blocks < 256 + 256 / waves) tn = 2;
@@ -210,7 +209,7 @@ bool fwd_tap_supported(const ConvDims &d) {
     if (d.kh != 1 || d.kw != 1 || d.pad != 0) return false;
     if (d.Ci <= 24 && d.stride <= 2 && (long)d.N * d.Ho * d.Wo >= 16384) return false;
     if ((images_ahead(d, ceil_div_l((long)d.Ho * d.Wo, 4)) * d.Ci + 1) * d.H * d.W > 0x3fffffffL) return false;
-    const TapShape shape = tap_shape(d);
+    const LaneShape shape = fwd_tap_shape(d);
     return (long)tap_tiles(d, shape.tn) * ceil_div(d.Co, shape.tm) * 64 * shape.waves <= kMaxThreads;
 }
 
@@ -226,7 +225,7 @@ static int launch_tap(const T *x, const float *w, T *y, const ConvDims &d, hipSt
 
 template <class T>
 int launch_fwd_tap(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn) {
-    const TapShape shape = tap_shape(d);
+    const LaneShape shape = fwd_tap_shape(d);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         if constexpr (sizeof(T) == 4) {

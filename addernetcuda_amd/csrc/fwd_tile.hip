@@ -575,6 +575,13 @@ int fwd_stats_slots(const ConvDims &d) {
     }
 }
 
+int fwd_stats_kernel(const ConvDims &d) {
+    const int variant = tile_variant(d), rows = rows_per_tile_w32(d.Ho);
+    if (few_positions(d, variant)) return 2;
+    if (variant == 0) return conv1x1_supported(d, nullptr, nullptr) ? 1 : 0;
+    return 10 * variant + (variant == 1 ? (rows == 16 ? 0 : rows == 8 ? 1 : 2) : variant == 5 && d.Ci >= 128 ? 1 : 0);
+}
+
 // stats: per-channel partial sums of y and y*y, fwd_stats_slots(d) > 0 slots per channel.
 int launch_fwd_stats(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s) {
     // rows that are whole groups of four are moved as such and need bases aligned to a group

@@ -1097,72 +1097,87 @@ static_assert(Gx5W32::TM * Gx5W32::COW == Gx5W16::TM * Gx5W16::COW && Gx5W32::TM
 static_assert(GxW32::TM == GxW16::TM && GxS2W32::TM == GxS2W16::TM,
               "the launcher checks Ci against one TM per stride");
 
-// gadd (nullable): a tensor shaped like gx that is added to the result (tiled 3x3 / pad 1, 5x5 / pad 2 / stride 1 and tiled
-// 1x1 stride-1 kernels only; ADDER_ERR_UNSUPPORTED elsewhere)
+// Which kernel a call takes.  groups: gy, gx and the second gradient are aligned to groups of four; gy_groups: gy is; pairs: gx and the second
+// gradient are aligned to pairs.  adds: the kernel adds a second gradient where it always was added.
+enum class GradXKernel { general = 0, plain_1x1 = 1, tiles = 2, tap = 3, nine = 4, s2 = 5 };
+struct GradXRoute { GradXKernel kernel; bool adds; };
+static GradXRoute grad_x_route(const ConvDims &d, bool bf16, bool groups, bool gy_groups, bool pairs) {
+    const bool rows_ok = d.W % 4 != 0 || groups;
+    const bool k3s1p1 = d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1;
+    if (k3s1p1 && rows_ok && grad_x_tiles(d)) return {GradXKernel::tiles, true};
+    // (25 taps: the tiles add a second gradient from two input channels on)
+    const bool tiles5 = d.kh == 5 && d.kw == 5 && d.stride == 1 && d.pad == 2 && d.Ci >= Gx5W32::TM && rows_ok;
+    if (tiles5 && (fills_5x5_tiles(d) || !grad_x_nine_supported(d))) return {GradXKernel::tiles, true};
+    // (from here on: bases of any alignment and any number of channels)
+    if (grad_x_nine_supported(d)) return {GradXKernel::nine, d.kh == 5 ? tiles5 : d.Ci >= GxW32::TM && rows_ok};
+    // 3x3 with a stride of two: layers the BatchNorm link may ask for (grad_x_bn_variant) keep the tiles, so that the plain call has the linked
+    // one's bits; bfloat16, which has no links, only where they are filled and give every CU a workgroup
+    const bool adds_s2 = d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM && (d.Wo % 4 != 0 || gy_groups) && pairs;
+    if (adds_s2 && (!grad_x_s2_supported(d) || (d.Wo % 4 == 0 && (!bf16 || fills_s2_tiles(d))))) return {GradXKernel::tiles, true};
+    if (grad_x_s2_supported(d)) return {GradXKernel::s2, adds_s2};
+    // (on planes of whole groups for aligned bases only)
+    if (grad_x_tap_supported(d)) return {GradXKernel::tap, d.H * d.W % 4 != 0 || groups};
+    if (grad_x_tap_narrow(d)) return {GradXKernel::tap, false};
+    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride > 1 && d.Ci >= 64 && d.Co >= 64 && (d.Ho * d.Wo % 4 != 0 || gy_groups))
+        return {GradXKernel::tiles, false};
+    const bool plain = conv1x1_supported(d, nullptr, nullptr) && ceil_div(d.Ci, kGx1x1TM) <= kMaxGridY;
+    return {plain ? GradXKernel::plain_1x1 : GradXKernel::general, false};
+}
+
+// the strided 3x3 layers' two-instruction form, where their tiles had it: of rows in pairs, at most kSatMaxTerms terms
+static bool s2_two(const ConvDims &d, const GradXRoute &route) { return route.adds && d.Co * 4 <= kSatMaxTerms; }
+
+int grad_x_kernel(const ConvDims &d, bool bf16) {
+    const GradXRoute route = grad_x_route(d, bf16, true, true, true);
+    GradXShape shape{0, 0, 0, false};
+    if (route.kernel == GradXKernel::tap) shape = grad_x_tap_shape(d, bf16);
+    if (route.kernel == GradXKernel::nine) shape = grad_x_nine_shape(d, bf16, true);
+    if (route.kernel == GradXKernel::s2) shape = grad_x_s2_shape(d, s2_two(d, route));
+    return static_cast<int>(route.kernel) * 1000000 + shape.tm * 10000 + shape.tn * 1000 + shape.waves * 10 + (shape.tm ? (shape.two ? 2 : 3) : 0);
+}
+
+// gadd (nullable): a tensor shaped like gx that is added to the result (where the route says so; ADDER_ERR_UNSUPPORTED elsewhere)
 // Both storage types take the same kernels and tile shapes.  (bfloat16 layers other than 3x3 once went to the generic
 // kernel: 128 -> 512 1x1 @28x28, 32 images, 845 us.)
 template <class T>
 int launch_grad_x(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd) {
-    const bool k3s1p1 = d.kh == 3 && d.kw == 3 && d.stride == 1 && d.pad == 1;
-    const bool aligned = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
-    if (k3s1p1 && (d.W % 4 != 0 || aligned)) switch (grad_x_tiles(d)) {
-        case 32: return launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd);
-        case 16: return launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
-        default: break;
+    const bool groups = aligned_groups(gy) && aligned_groups(gx) && aligned_groups(gadd);
+    const bool pairs = ((reinterpret_cast<uintptr_t>(gx) | reinterpret_cast<uintptr_t>(gadd)) & (2 * sizeof(T) - 1)) == 0;
+    const GradXRoute route = grad_x_route(d, sizeof(T) == 2, groups, aligned_groups(gy), pairs);
+    if (gadd && !route.adds) return ADDER_ERR_UNSUPPORTED;
+    switch (route.kernel) {
+        case GradXKernel::tiles: break;
+        case GradXKernel::nine: return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr, d.W % 4 != 0 || groups);
+        case GradXKernel::s2: return launch_grad_x_s2<T>(gy, x, w, gx, d, s, gadd, s2_two(d, route));
+        case GradXKernel::tap: return launch_grad_x_tap<T>(gy, x, w, gx, d, s, gadd, nullptr);
+        case GradXKernel::plain_1x1: return launch_grad_x_1x1(gy, x, w, gx, d, s);
+        case GradXKernel::general: {
+            constexpr int TM = 8;
+            const long total = (long)d.N * d.H * d.W;
+            hipLaunchKernelGGL((grad_x_generic_kernel<TM, T>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Ci, TM)),
+                               dim3(256), 0, s, gy, x, w, gx, d);
+            return check_launch();
+        }
     }
-    // (25 taps: the tiles add a second gradient from two input channels on)
-    const bool tiles5 = d.kh == 5 && d.kw == 5 && d.stride == 1 && d.pad == 2 && d.Ci >= Gx5W32::TM && (d.W % 4 != 0 || aligned);
-    if (tiles5 && (fills_5x5_tiles(d) || !grad_x_nine_supported(d))) {
-        if (d.W > 16) return launch_grad_x_3x3s1<Gx5W32, false, T>(gy, x, w, gx, d, s, gadd);
-        if (d.W > 8) return launch_grad_x_3x3s1<Gx5W16, false, T>(gy, x, w, gx, d, s, gadd);
-        return launch_grad_x_3x3s1<Gx5W8, false, T>(gy, x, w, gx, d, s, gadd);
-    }
-    if (grad_x_nine_supported(d)) {
-        // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
-        if (gadd && !(d.kh == 5 ? tiles5 : d.Ci >= GxW32::TM && (d.W % 4 != 0 || aligned))) return ADDER_ERR_UNSUPPORTED;
-        return launch_grad_x_nine<T>(gy, x, w, gx, d, s, gadd, nullptr, d.W % 4 != 0 || aligned);
-    }
-    // 3x3 with a stride of two: layers the BatchNorm link may ask for (grad_x_bn_variant) keep the tiles, so that the plain call has the linked
-    // one's bits; bfloat16, which has no links, only where they are filled and give every CU a workgroup
-    const bool adds_s2 = d.kh == 3 && d.kw == 3 && d.stride == 2 && d.pad == 1 && d.W % 2 == 0 && d.Ci >= GxS2W32::TM &&
-                         (d.Wo % 4 != 0 || aligned_groups(gy)) &&
-                         ((reinterpret_cast<uintptr_t>(gx) | reinterpret_cast<uintptr_t>(gadd)) & (2 * sizeof(T) - 1)) == 0;
-    if (adds_s2 && (!grad_x_s2_supported(d) || (d.Wo % 4 == 0 && (sizeof(T) == 4 || fills_s2_tiles(d))))) {
-        if (d.W > 16) return launch_grad_x_3x3s2<GxS2W32, T>(gy, x, w, gx, d, s, gadd);
-        return launch_grad_x_3x3s2<GxS2W16, T>(gy, x, w, gx, d, s, gadd);
-    }
-    if (grad_x_s2_supported(d)) {
-        // (it takes bases of any alignment and any number of channels; a second gradient is added where it always was)
-        if (gadd && !adds_s2) return ADDER_ERR_UNSUPPORTED;
-        return launch_grad_x_s2<T>(gy, x, w, gx, d, s, gadd, adds_s2 && d.Co * 4 <= kSatMaxTerms);
-    }
-    if (grad_x_tap_supported(d)) {
-        // (it takes bases of any alignment; a second gradient is added on planes of whole groups for aligned ones only)
-        if (gadd && d.H * d.W % 4 == 0 && !aligned) return ADDER_ERR_UNSUPPORTED;
-        return launch_grad_x_tap<T>(gy, x, w, gx, d, s, gadd, nullptr);
-    }
-    if (gadd) return ADDER_ERR_UNSUPPORTED;
-    if (grad_x_tap_narrow(d)) return launch_grad_x_tap<T>(gy, x, w, gx, d, s, nullptr, nullptr);
-    if (d.kh == 1 && d.kw == 1 && d.pad == 0 && d.stride > 1 && d.Ci >= 64 && d.Co >= 64) {
+    if (d.kh == 1) {
         ConvDims f = d;   // the sampled positions of every plane as one row; x and gx are read / written in place
         f.H = f.Ho = 1;
         f.W = f.Wo = d.Ho * d.Wo;
         f.stride = 1;
         const Subsample sub{d.stride, d.Wo, d.W, d.H * d.W};
         const T *none = nullptr;
-        if (f.W % 4 != 0 || aligned_groups(gy)) {
-            if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, true, T>(gy, x, w, gx, f, s, none, sub);
-            return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, true, T>(gy, x, w, gx, f, s, none, sub)
-                                       : launch_grad_x_3x3s1<Gx1x1s, true, T>(gy, x, w, gx, f, s, none, sub);
-        }
+        if (f.W > 64) return launch_grad_x_3x3s1<Gx1x1, true, T>(gy, x, w, gx, f, s, none, sub);
+        return small_plane_tile(f) ? launch_grad_x_3x3s1<Gx1x1t, true, T>(gy, x, w, gx, f, s, none, sub)
+                                   : launch_grad_x_3x3s1<Gx1x1s, true, T>(gy, x, w, gx, f, s, none, sub);
     }
-    if (conv1x1_supported(d, gy, gx) && ceil_div(d.Ci, kGx1x1TM) <= kMaxGridY)
-        return launch_grad_x_1x1(gy, x, w, gx, d, s);
-    constexpr int TM = 8;
-    const long total = (long)d.N * d.H * d.W;
-    hipLaunchKernelGGL((grad_x_generic_kernel<TM, T>), dim3((unsigned)ceil_div_l(total, 256), ceil_div(d.Ci, TM)),
-                       dim3(256), 0, s, gy, x, w, gx, d);
-    return check_launch();
+    if (d.kh == 5) {
+        if (d.W > 16) return launch_grad_x_3x3s1<Gx5W32, false, T>(gy, x, w, gx, d, s, gadd);
+        if (d.W > 8) return launch_grad_x_3x3s1<Gx5W16, false, T>(gy, x, w, gx, d, s, gadd);
+        return launch_grad_x_3x3s1<Gx5W8, false, T>(gy, x, w, gx, d, s, gadd);
+    }
+    if (d.stride == 2) return d.W > 16 ? launch_grad_x_3x3s2<GxS2W32, T>(gy, x, w, gx, d, s, gadd) : launch_grad_x_3x3s2<GxS2W16, T>(gy, x, w, gx, d, s, gadd);
+    return grad_x_tiles(d) == 32 ? launch_grad_x_3x3s1<GxW32, false, T>(gy, x, w, gx, d, s, gadd)
+                                 : launch_grad_x_3x3s1<GxW16, false, T>(gy, x, w, gx, d, s, gadd);
 }
 template int launch_grad_x<float>(const float *, const float *, const float *, float *, const ConvDims &, hipStream_t,
                                   const float *);

@@ -328,10 +328,20 @@ static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const 
     return check_launch();
 }
 
+// The two-instruction form only where the launch fills the chip: below that it gains nothing (32 -> 32 @16x16, 32 images, 9.1 us,
+// three instructions 8.8; 64 -> 64 @56x56, one, 11.9, 13.2) and rounds w and x once more (1.6e-7 of the result against 2.3e-7).
+GradXShape grad_x_nine_shape(const ConvDims &d, bool bf16, bool groups) {
+    const GxNineShape shape = gx_nine_shape(d);
+    if (d.kh == 5) return {4, shape.tn, shape.waves, shape.tn == 2 && groups && d.Ci >= 2 && two_instructions_5x5(d.Co)};
+    const bool two = shape.tn == 4 && groups && d.Co * 9 <= kSatMaxTerms && d.Ci >= 4 && !small_unlinked(d, bf16, d.W, 660000);
+    return {shape.tn == 1 ? 4 : 8, shape.tn, shape.waves, two};
+}
+
 // bn (nullable): the in_* half of adder_bn_links
 template <class T>
 int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
                        const adder_bn_links *bn, bool groups) {
+    const GradXShape shape = grad_x_nine_shape(d, sizeof(T) == 2, groups);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         auto form = [&](auto sat) {
@@ -341,17 +351,11 @@ int launch_grad_x_nine(const T *gy, const T *x, const float *w, T *gx, const Con
             }
             return launch_gx_nine<C, SAT, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{});
         };
-        // The two-instruction form only where the launch fills the chip: below that it gains nothing (32 -> 32 @16x16, 32 images, 9.1 us,
-        // three instructions 8.8; 64 -> 64 @56x56, one, 11.9, 13.2) and rounds w and x once more (1.6e-7 of the result against 2.3e-7).
-        if constexpr (C::TN == 4) {
-            if (groups && d.Co * 9 <= kSatMaxTerms && d.Ci >= 4 && !small_unlinked(d, sizeof(T) == 2, d.W, 660000)) return form(std::true_type{});
-        }
-        if constexpr (C::PAIRS) {
-            if (groups && d.Ci >= 2 && two_instructions_5x5(d.Co)) return form(std::true_type{});
+        if constexpr (C::TN == 4 || C::PAIRS) {
+            if (shape.two) return form(std::true_type{});
         }
         return form(std::false_type{});
     };
-    const GxNineShape shape = gx_nine_shape(d);
     auto waves = [&](auto ksp) {
         constexpr int KSP = decltype(ksp)::value;
         if (d.kh == 5) return shape.tn == 2 ? run(GxNineCfg<4, 2, KSP, 5>{}) : run(GxNineCfg<4, 1, KSP, 5>{});

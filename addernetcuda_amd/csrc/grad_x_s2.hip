@@ -279,19 +279,25 @@ static int launch_gx_s2(const T *gy, const T *x, const float *w, T *gx, const Co
     return check_launch();
 }
 
+GradXShape grad_x_s2_shape(const ConvDims &d, bool sat) {
+    const bool wide = gx_s2_wide(d);
+    return {wide ? 4 : 2, 1, gx_s2_waves(d.Co), wide && sat && d.kh == 3};
+}
+
 // sat: the two-instruction form (grad_x.hip), where the launch fills the chip
 template <class T>
 int launch_grad_x_s2(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd, bool sat) {
+    const GradXShape shape = grad_x_s2_shape(d, sat);
     auto run = [&](auto ks, auto ksp) {
         constexpr int KS = decltype(ks)::value, KSP = decltype(ksp)::value;
-        if (!gx_s2_wide(d)) return launch_gx_s2<GxS2Cfg<KS, 2, KSP>, false, T>(gy, x, w, gx, d, s, gadd);
+        if (shape.tm == 2) return launch_gx_s2<GxS2Cfg<KS, 2, KSP>, false, T>(gy, x, w, gx, d, s, gadd);
         if constexpr (KS == 3) {
-            if (sat) return launch_gx_s2<GxS2Cfg<KS, 4, KSP>, true, T>(gy, x, w, gx, d, s, gadd);
+            if (shape.two) return launch_gx_s2<GxS2Cfg<KS, 4, KSP>, true, T>(gy, x, w, gx, d, s, gadd);
         }
         return launch_gx_s2<GxS2Cfg<KS, 4, KSP>, false, T>(gy, x, w, gx, d, s, gadd);
     };
     auto waves = [&](auto ks) {
-        switch (gx_s2_waves(d.Co)) {
+        switch (shape.waves) {
             case 1: return run(ks, std::integral_constant<int, 1>{});
             case 2: return run(ks, std::integral_constant<int, 2>{});
             case 4: return run(ks, std::integral_constant<int, 4>{});

@@ -236,21 +236,28 @@ static int launch_gx_tap(const T *gy, const T *x, const float *w, T *gx, const C
     return check_launch();
 }
 
+// The three-instruction form rounds once less (error 8.7e-8 of the result, two instructions 1.58e-7) and costs a small launch nothing
+// (8 x 1: 128 -> 512 @28x28 9.5 -> 9.2 us, 64 -> 256 @56x56 8.3 -> 8.5); planes that no BatchNorm can be linked to have it with eight
+// waves too (1024 -> 256 @14x14, 8 images, which can: 26.5 -> 31.9), and so have narrow layers and small ones without a link (small_unlinked).
+GradXShape grad_x_tap_shape(const ConvDims &d, bool bf16) {
+    const GxTapShape shape = gx_tap_shape(d);
+    if (d.Ci < 8) return {4, d.H * d.W >= 2 ? 2 : 1, 4, false};   // (no link and no second gradient: grad_x_tap_narrow)
+    if (d.Ci < 16) return {8, shape.tn, shape.tn == 1 ? 8 : 4, false};
+    const bool exact = shape.tm == 8 || !grad_x_tap_supported(d) || (shape.waves == 8 && (d.H * d.W) % 4 != 0) ||
+                       small_unlinked(d, bf16, d.H * d.W, 770000);
+    return {shape.tm, shape.tn, shape.waves, !exact && d.Co <= kSatMaxTerms1x1};
+}
+
 // bn (nullable): the in_* half of adder_bn_links
 template <class T>
 int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
                       const adder_bn_links *bn) {
-    // The three-instruction form rounds once less (error 8.7e-8 of the result, two instructions 1.58e-7) and costs a small launch nothing
-    // (8 x 1: 128 -> 512 @28x28 9.5 -> 9.2 us, 64 -> 256 @56x56 8.3 -> 8.5); planes that no BatchNorm can be linked to have it with eight
-    // waves too (1024 -> 256 @14x14, 8 images, which can: 26.5 -> 31.9), and so have narrow layers and small ones without a link (small_unlinked).
-    const GxTapShape shape = gx_tap_shape(d);
-    if (d.Ci < 16) {   // (no link and no second gradient: grad_x_tap_narrow)
+    const GradXShape shape = grad_x_tap_shape(d, sizeof(T) == 2);
+    if (d.Ci < 16) {
         auto narrow = [&](auto cfg) { return launch_gx_tap<decltype(cfg), false, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{}); };
-        if (d.Ci < 8) return d.H * d.W >= 2 ? narrow(GxTapCfg<4, 2, 4>{}) : narrow(GxTapCfg<4, 1, 4>{});
+        if (shape.tm == 4) return shape.tn == 2 ? narrow(GxTapCfg<4, 2, 4>{}) : narrow(GxTapCfg<4, 1, 4>{});
         return shape.tn == 1 ? narrow(GxTapCfg<8, 1, 8>{}) : narrow(GxTapCfg<8, 2, 4>{});
     }
-    const bool exact = shape.tm == 8 || !grad_x_tap_supported(d) || (shape.waves == 8 && (d.H * d.W) % 4 != 0) ||
-                       small_unlinked(d, sizeof(T) == 2, d.H * d.W, 770000);
     auto run = [&](auto cfg) {
         using C = decltype(cfg);
         auto form = [&](auto sat) {
@@ -260,7 +267,7 @@ int launch_grad_x_tap(const T *gy, const T *x, const float *w, T *gx, const Conv
             }
             return launch_gx_tap<C, SAT, T, false>(gy, x, w, gx, d, s, gadd, adder_bn_links{});
         };
-        return d.Co <= kSatMaxTerms1x1 && !exact ? form(std::true_type{}) : form(std::false_type{});
+        return shape.two ? form(std::true_type{}) : form(std::false_type{});
     };
     if (shape.tm == 8) return run(GxTapCfg<8, 1, 8>{});
     return shape.waves == 1 ? run(GxTapCfg<16, 2, 1>{}) : shape.waves == 4 ? run(GxTapCfg<16, 2, 4>{}) : run(GxTapCfg<16, 2, 8>{});

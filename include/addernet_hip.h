@@ -82,11 +82,20 @@ ADDER_API int adder_conv2d_fwd_f32(const float *x, const float *w, float *y,
                          int N, int Ci, int H, int W, int Co, int kh, int kw,
                          int stride, int pad, void *stream);
 
-/* Which kernel the forward calls above and below (without statistics) take for the dimensions and aligned tensors, in the
- * dispatch's own numbers: 0 the general one, 1 the plain 1x1 one, 2 few positions, from 10 on by taps, stride and map.  (The
- * 3x3 layers of 2 and 10 to 51 share one kernel, the 1x1 layers of stride 1 of 2, 60, 70, 100 and 110 another.)
- * Host code only; for tests that have to reach a certain kernel, and no promise that the numbers stay. */
+/* Which kernel the forward calls above and below (without statistics) take for the dimensions and aligned tensors: 0 the general one,
+ * 100000 the plain 1x1 one, 200000 the strided 1x1 one in tiles, and of the kernels without tiles 300000 (1x1) and 400000 (3x3, 5x5) plus 1000 x output
+ * channels per lane, 100 x positions per lane and the waves that share the input channels.
+ * This and the next two: host code only, for tests that have to reach a certain kernel, and no promise that the numbers stay. */
 ADDER_API int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel);
+
+/* ... the forward calls with statistics: 0 none, 1 the plain 1x1 one, 2 the 1x1 one for few positions, from 10 on those in tiles: 10 x (1..3 3x3 by
+ * output width, 4..5 with stride 2, 6..7 1x1 by plane size, 8..9 with a stride, 10..13 the same for channels that are no multiple of eight) plus a shape. */
+ADDER_API int adder_conv2d_fwd_stats_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel);
+
+/* ... the input gradient of the backward calls in float (bf16 = 0) or bfloat16 storage: 0 the general one, 1000000 the plain 1x1 one, 2000000 those in
+ * tiles, and without tiles 3000000 (1x1), 4000000 (3x3, 5x5) and 5000000 (strided 3x3, 5x5) plus 10000 x input channels per lane, 1000 x positions per lane (strided:
+ * blocks of 2 x 2), 10 x the waves that share the output channels and the instructions a term takes. */
+ADDER_API int adder_conv2d_grad_x_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int bf16, int *kernel);
 
 /* The same forward with the BatchNorm that follows it (fixed statistics: inference), the shortcut and the ReLU applied on
  * the way out: y = act((conv - mean) / sqrt(var + eps) * gamma + beta [+ residual]), act = ReLU when relu is set;

@@ -6,12 +6,11 @@ import copy
 import pytest
 import torch
 
-from tests.util import make_case, assert_close, fwd_kernel, TILED_FORWARD, ATOL, RTOL
+from tests.util import make_case, assert_close, stats_kernel, TILED_FORWARD, ATOL, RTOL
 
 pytestmark = pytest.mark.gpu
 
-# (N, Ci, H, W, Co, k, stride, pad): 3x3 by width, strided 3x3, tiled / sampled / plain 1x1, 5x5, generic; about half of them run the
-# few-positions kernel (the tiled ones: below)
+# (N, Ci, H, W, Co, k, stride, pad): 3x3 by width, strided 3x3, strided and plain 1x1, 5x5, generic
 SHAPES = [(2, 16, 32, 32, 18, 3, 1, 1), (3, 5, 24, 27, 7, 3, 1, 1), (3, 8, 20, 28, 9, 3, 1, 1), (2, 33, 14, 14, 35, 3, 1, 1),
           (5, 16, 7, 7, 17, 3, 1, 1), (2, 16, 32, 32, 33, 3, 2, 1), (3, 12, 15, 15, 20, 3, 2, 1), (2, 64, 20, 20, 40, 1, 1, 0),
           (5, 72, 7, 7, 33, 1, 1, 0), (3, 68, 8, 8, 36, 1, 1, 0), (2, 64, 18, 18, 70, 1, 2, 0), (2, 68, 18, 18, 36, 1, 2, 0),
@@ -66,13 +65,19 @@ def test_fused_inference_matches_the_oracle(case, relu, with_res, offset, gpu):
 
 
 @pytest.mark.parametrize("kernel,case", [(k, c) for k, cases in TILED_FORWARD.items() for c in cases], ids=str)
-def test_every_tiled_kernel_plain_and_with_the_epilogue(kernel, case, gpu):
+def test_layers_of_every_tiled_kernel_plain_with_statistics_and_with_the_epilogue(kernel, case, gpu):
+    from addernetcuda_amd import adder
     from addernetcuda_amd.unit import _eval_unit
     from oracle import c_oracle
-    assert fwd_kernel(case) == kernel
+    assert stats_kernel(case) == kernel
     x, layer, bn, res, want, bound = _modules(case, gpu, True)
     with torch.no_grad():
-        assert_close(layer(x), c_oracle.conv2d_fwd(x.cpu(), layer.adder.cpu(), case[6], case[7]), f"forward {case}")
+        conv = c_oracle.conv2d_fwd(x.cpu(), layer.adder.cpu(), case[6], case[7])
+        assert_close(layer(x), conv, f"forward {case}")
+        y, stats = adder.adder2d_function_with_stats(x, layer.adder, case[6], case[7])
+        assert torch.equal(y, layer(x))
+        sums = torch.stack([conv.sum((0, 2, 3)), (conv * conv).sum((0, 2, 3))], 1)
+        assert_close(stats.sum(1) / sums.abs().max(), sums / sums.abs().max(), f"statistics {case}")
         for offset in (None, 0, 1):
             got = _eval_unit(layer, bn, x, None if offset is None else _at(res, gpu, offset))
             err = (got.double().cpu() - (want if offset is None else want + res.double()).clamp(min=0)).abs()

@@ -1,4 +1,4 @@
-"""Seeded synthetic tensors shared by the tests (CPU float32), and layers that reach each forward kernel."""
+"""Seeded synthetic tensors shared by the tests (CPU float32), and which kernels layers take."""
 import ctypes
 import math
 
@@ -39,17 +39,37 @@ def assert_close(actual, expected, what, rtol=RTOL, atol=ATOL):
             f"{a[tuple(idx)].item()} vs {e[tuple(idx)].item()}")
 
 
-def fwd_kernel(case):
-    """The number of the forward kernel that the library takes for (N, Ci, H, W, Co, k, stride, pad)."""
+def _kernel(query, case, *more):
     from addernetcuda_amd._lib import lib, check
     N, Ci, H, W, Co, k, stride, pad = case
     kernel = ctypes.c_int(-1)
-    check(lib.adder_conv2d_fwd_kernel(N, Ci, H, W, Co, k, k, stride, pad, ctypes.byref(kernel)), "adder_conv2d_fwd_kernel")
+    check(getattr(lib, query)(N, Ci, H, W, Co, k, k, stride, pad, *more, ctypes.byref(kernel)), query)
     return kernel.value
 
 
+GENERAL, PLAIN_1X1, TILES, TAP, NINE, S2 = range(6)
+
+
+def fwd_kernel(case):
+    """(kernel, output channels per lane, positions per lane, waves) of the forward the library takes for (N, Ci, H, W, Co, k, stride, pad);
+    TILES: strided 1x1 layers."""
+    v = _kernel("adder_conv2d_fwd_kernel", case)
+    return v // 100000, v // 1000 % 100, v // 100 % 10, v % 100
+
+
+def stats_kernel(case):
+    """The number of the kernel that the forward with statistics takes."""
+    return _kernel("adder_conv2d_fwd_stats_kernel", case)
+
+
+def grad_x_kernel(case, bf16=False):
+    """(kernel, input channels per lane, positions per lane, waves, instructions a term) of the input gradient."""
+    v = _kernel("adder_conv2d_grad_x_kernel", case, int(bf16))
+    return v // 1000000, v // 10000 % 100, v // 1000 % 10, v // 10 % 100, v % 10
+
+
 FEW_POSITIONS = 2
-# every tiled forward kernel, by its number, on a layer whose rows (1x1: planes) are whole groups of four and on one whose are not
+# every tiled kernel of the forward with statistics, by its number, on a layer whose rows (1x1: planes) are whole groups of four and on one whose are not
 TILED_FORWARD = {
     10: [(2, 3, 32, 32, 18, 3, 1, 1), (1, 5, 32, 30, 18, 3, 1, 1)],
     11: [(2, 3, 24, 24, 18, 3, 1, 1), (3, 5, 24, 27, 7, 3, 1, 1)],
@@ -67,13 +87,9 @@ TILED_FORWARD = {
     110: [(1, 68, 8, 8, 18, 1, 1, 0), (1, 68, 7, 7, 18, 1, 1, 0)],
     120: [(1, 68, 28, 28, 18, 1, 2, 0), (1, 68, 32, 30, 18, 1, 2, 0)],
     130: [(1, 68, 8, 8, 18, 1, 2, 0), (1, 68, 7, 7, 18, 1, 3, 0)],
-    140: [(1, 3, 20, 20, 18, 5, 1, 2), (2, 9, 17, 30, 18, 5, 1, 2)],
-    150: [(1, 3, 12, 12, 18, 5, 1, 2), (2, 9, 14, 14, 18, 5, 1, 2)],
-    160: [(5, 3, 8, 8, 18, 5, 1, 2), (1, 9, 7, 7, 18, 5, 1, 2)],
-    170: [(1, 9, 20, 24, 18, 5, 2, 2), (2, 3, 18, 18, 18, 5, 2, 2)],
-    180: [(3, 3, 16, 16, 18, 5, 2, 2), (1, 9, 13, 7, 18, 5, 2, 2)],
 }
-# layers of one image for the few-positions kernel, with a batch that is large enough for the tiled kernel of that number
+# layers of one image, with a batch that is large enough for another kernel or shape of the plain forward, by the kernel in tiles that the batch takes with
+# statistics (from 60 on, 1x1 layers, one image takes the one for few positions there)
 FEW_AND_TILED = {
     10: ((1, 16, 32, 32, 40, 3, 1, 1), 16), 11: ((1, 16, 24, 24, 16, 3, 1, 1), 64), 12: ((1, 16, 17, 32, 16, 3, 1, 1), 64),
     20: ((1, 33, 14, 14, 37, 3, 1, 1), 128), 30: ((1, 200, 7, 7, 31, 3, 1, 1), 2048), 40: ((1, 32, 17, 32, 33, 3, 2, 1), 256),
