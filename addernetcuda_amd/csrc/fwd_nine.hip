@@ -17,9 +17,10 @@
 // positions there was) 64 -> 64 @8x8 7.6 -> 6.6, 256 -> 256 @14x14 19.9 -> 17.0, 512 -> 512 @7x7 30 -> 29.
 // Tried on the way: 4 channels x 4 positions per lane 132 -> 179 us (64 -> 64 @56x56: reads), 8 x 2 143.
 //
-// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 117 to 128 registers (shared
-// bfloat16 layers spill 15 of them).  us, tiles in LDS -> this: 64 -> 64 @56x56, 16 images, 271 -> 202, 128 -> 64 @16x16, 64 images, 137 -> 132, 32 -> 64 @16x16 40.9 -> 39.8,
-// 64 -> 64 @8x8 65 -> 22, one image 61 -> 9.7, 47 -> 19 @14x14, 193 images, 111 -> 71, 9 -> 20 @53x53, 32 images, 51 -> 31, 813 -> 551 @9x9, two images, 865 -> 258;
+// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 117 to 128
+// registers.  us, tiles in LDS -> this: 64 -> 64 @56x56, 16 images, 271 -> 202, 128 -> 64 @16x16, 64 images, 137 -> 132, 32 -> 64 @16x16 40.9 -> 39.8,
+// 64 -> 64 @8x8 65 -> 22, one image 61 -> 9.7, 47 -> 19 @14x14, 193 images, 111 -> 71, 9 -> 20 @53x53, 32 images, 51 -> 31, 813 -> 551 @9x9, two images, 865 -> 258,
+// 32 -> 64, 32 images, @13x13 37 -> 22, @21x21 77 -> 44, @29x29 81 -> 75 (4 x 1 on such rows of whole strips and one column: 98);
 // stride 2: 64 -> 64 @56x56, 32 images, 176 -> 145, 7 -> 144 @23x26, 202 images, 86 -> 60, 36 -> 34 @38x41, 6 images, 30 -> 12, 32 -> 64 @32x32, 64 images, 52 -> 55.
 // On the way, 64 -> 64 @56x56: comparisons instead of bit masks for what lies outside 387 (the masks of 20 elements fill the scalar
 // registers), the columns beside a strip read one by one 315, three waves per SIMD instead of four with a few spilled registers 218.
@@ -46,15 +47,16 @@ struct NineCfg {
         static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;
     static constexpr int MID = (TN - 1) * S + 1, STRIP = MID + 2 * PAD;   // columns under the strip, and with those beside it
     static_assert(NU == 1 || NU % 2 == 0, "two weight buffers");
-    // 25 taps, more than one position: the two columns on a side are both inside the map or both outside -- at stride 1 unless a row is four strips and one
-    // column long, at stride 2 on the left, and on the right of rows of an odd length
+    // 25 taps, more than one position: the two columns on a side are both inside the map or both outside -- at stride 1 (rows of whole strips and one
+    // column: see Strips), at stride 2 on the left, and on the right of rows of an odd length
     static constexpr bool PAIRS = KS == 5 && TN > 1;
     static_assert(KS == 3 || KS == 5, "nine or 25 taps");
 };
 
 struct NineDims {
     int N, Ci, H, W, Co, Ho, Wo;
-    int per_row, strips;    // strips of TN positions per row (the last one is moved back to end at Wo) and per image
+    Strips row;
+    int strips;             // of TN positions per image
     int tiles, blocks;      // of 64 strips, of TM output channels
     int chunk, chunks;      // input channels per first-level sum (a power of two), and how many sums there are
 };
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(C::NT, 4) void fwd_nine_kernel(const T *__restrict_
     xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
     const int wave = C::SHARED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, waves = C::SHARED ? blockDim.x >> 6 : 1, lane = threadIdx.x & 63;
     const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
-    const int ho = rest / d.per_row, s = rest - ho * d.per_row, wo = min(s * TN, d.Wo - TN), co_base = blk * TM;
+    const int ho = rest / d.row.per_row, s = rest - ho * d.row.per_row, wo = d.row.start(s, TN, d.Wo), co_base = blk * TM;
     const int plane = d.H * d.W, K = d.Ci * KK;
     uniform_f32_ptr wc = as_uniform(w);
     int wrow[TM];
@@ -260,7 +262,7 @@ __global__ __launch_bounds__(C::NT, 4) void fwd_nine_kernel(const T *__restrict_
 
     unsigned own = 0;   // bit t: position wo + t is this lane's
 #pragma unroll
-    for (int t = 0; t < TN; ++t) own |= (sidx == sc && wo + t >= s * TN ? 1u : 0u) << t;
+    for (int t = 0; t < TN; ++t) own |= (sidx == sc && wo + t >= d.row.first(s, TN) ? 1u : 0u) << t;
     const int L = d.Ho * d.Wo, first = sums.first_channel();
     if (first < TM)
         finish_outputs<C::Sums::FM, TN, EVAL>(sums.tot, min(sums.per_wave, TM - first), own, co_base + first, d.Co, L, n * d.Co * L + ho * d.Wo + wo,
@@ -287,9 +289,9 @@ static int nine_waves(const ConvDims &d, int chunk, long wgs) {
 LaneShape fwd_nine_shape(const ConvDims &d) {
     const int chunk = fwd_chunk(d), chunks = ceil_div(d.Ci, fwd_chunk(d));
     if (d.kh == 5) {   // 4 x 4, or 4 x 1 for few waves (one image of 64 -> 64 @32x32, 512 waves of 4 x 4, 18.6 / 10.2 us; 64 of @8x8, 2048 waves, 19.8 / 26) and
-                       // where pairs of columns would be cut (PAIRS); stride 2: 4 x 2 (64 -> 64 @16x16, one image, 12.7; 4 x 1 24.6)
+                       // rows of five, which have no strips without a cut pair; stride 2: 4 x 2 (64 -> 64 @16x16, one image, 12.7; 4 x 1 24.6)
         const int most = d.stride == 1 ? 4 : 2;
-        int tn = d.Wo >= most && (d.stride == 2 || d.W % 4 != 1) ? most : 1;
+        const int tn = d.Wo >= most && (d.stride == 2 || d.W != 5) ? most : 1;
         const long wgs = (long)nine_tiles(d, tn) * ceil_div(d.Co, 4);
         const int waves = nine_waves(d, chunk, wgs);
         if (tn == 4 && wgs * waves < 1000) return {4, 1, nine_waves(d, chunk, (long)nine_tiles(d, 1) * ceil_div(d.Co, 4))};
@@ -322,7 +324,7 @@ bool fwd_nine_supported(const ConvDims &d) {
 template <class C, class T, bool EVAL>
 static int launch_nine(const T *x, const float *w, T *y, const ConvDims &d, hipStream_t s, const BnEval &bn, int waves) {
     const int per_row = ceil_div(d.Wo, C::TN);
-    const NineDims t{d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, per_row, per_row * d.Ho, nine_tiles(d, C::TN), ceil_div(d.Co, C::TM), fwd_chunk(d), ceil_div(d.Ci, fwd_chunk(d))};
+    const NineDims t{d.N, d.Ci, d.H, d.W, d.Co, d.Ho, d.Wo, Strips{per_row, C::PAIRS && C::S == 1 && d.Wo % C::TN == 1 ? 1 : kNoShift}, per_row * d.Ho, nine_tiles(d, C::TN), ceil_div(d.Co, C::TM), fwd_chunk(d), ceil_div(d.Ci, fwd_chunk(d))};
     const int lds = waves * C::Sums::WAVE_FLOATS * 4;
     if (int rc = allow_dynamic_lds<&fwd_nine_kernel<C, T, EVAL>>(8 * C::Sums::WAVE_FLOATS * 4)) return rc;
     hipLaunchKernelGGL((fwd_nine_kernel<C, T, EVAL>), dim3((unsigned)t.tiles * t.blocks), dim3(64 * waves), lds, s, x, w, y, t, bn);

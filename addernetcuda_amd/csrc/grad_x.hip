@@ -1082,10 +1082,11 @@ static bool fills_s2_tiles(const ConvDims &d) {
     return d.W % cols == 0 && d.H % 16 == 0 && d.Ci % channels == 0 && (long)d.N * (d.H / 16) * (d.W / cols) * (d.Ci / channels) >= 256;
 }
 
-// 5x5 layers of stride 1 that stay in tiles: up to 100 output channels, tiles filled to 85 % and channel groups altogether, a workgroup per CU (us, tiles ->
+// 5x5 layers of stride 1 that stay in tiles: up to 100 output channels, tiles filled to 85 %, whole groups of input channels, a workgroup per CU (us, tiles ->
 // grad_x_nine.hip: 32 -> 64 @16x16, 64 images, 51 -> 53, 64 -> 64 @56x56, 16 images, 268 -> 284, 64 -> 8 @32x32, 64 images, 64.5 -> 65.8; 76 % filled, 16 -> 16 @28x28, 256
 // images, 89 -> 78; three of eight channels, 3 -> 32 @32x32, 128 images, 43 -> 29; 128 workgroups, 64 -> 64 @8x8, 64 images, 50 -> 29; three instructions a
-// term on either side, 128 -> 64 @16x16, 64 images, 212 -> 193).
+// term on either side, 128 -> 64 @16x16, 64 images, 212 -> 193).  Groups that are nearly whole go either way -- 32 images, 39 -> 37 @32x32 68 -> 72, 15 -> 32 @32x32 24 -> 27, 35 -> 64
+// @32x32 106 -> 99, 44 -> 64 @28x28 107 -> 99 -- and are nearer to float64 there (2.0e-7 of the result, tiles 2.4e-7).
 static bool fills_5x5_tiles(const ConvDims &d) {
     if (d.Co > 100 || d.Ci % (Gx5W32::TM * Gx5W32::COW)) return false;
     const int rows = d.W > 16 ? Gx5W32::TH : d.W > 8 ? Gx5W16::TH : Gx5W8::TH, cols = d.W > 16 ? Gx5W32::TW : d.W > 8 ? Gx5W16::TW : Gx5W8::TW;

@@ -11,10 +11,11 @@
 // 322 -> 251, 100 -> 100 @20x20 119 -> 60; 64 -> 64 @8x8, 256 images 30.6 -> 28.3, one image 29 -> 6; 128 -> 128 @28x28, 4 / 1 images 97 -> 29, 94 -> 14;
 // 48 -> 12 @4x4, 64 images 8.4 -> 5.4; 256 -> 256 @14x14, one image 20 -> 18.
 //
-// 25 taps: 4 channels x 2 positions per lane, three reads per row of the window a channel ahead; rows of an odd length and small launches 4 x 1 with three
-// instructions a term.  us, tiles in LDS -> this: 342 channels of gy -> 48 of gx @10x10, 8 images, 279 -> 57, 261 -> 10 @27x27, 5 images, bfloat16, 206 -> 43,
-// 813 -> 551 @9x9, two images, 730 -> 255, 64 -> 64 @8x8, 64 images, 50 -> 29, one image 44 -> 12, 19 -> 47 @14x14, 193 images, 73 -> 58, 100 -> 100 @28x28, 32 images,
-// bfloat16, 379 -> 311; what fills tiles stays there (fills_5x5_tiles).  Error against float64 1.2e-7 to 2.0e-7 of the result (tiles 2.1e-7 to 3.7e-7).
+// 25 taps: 4 channels x 2 positions per lane, three reads per row of the window a channel ahead; small launches 4 x 1.  Rows of an odd length and 4 x 1 take three
+// instructions a term (error against float64 1.3e-7 to 1.5e-7 of the result; two instructions 2.0e-7 to 2.1e-7, tiles 2.1e-7 to 3.7e-7).  us, tiles in LDS ->
+// this: 342 channels of gy -> 48 of gx @10x10, 8 images, 279 -> 57, 261 -> 10 @27x27, 5 images, bfloat16, 206 -> 43, 813 -> 551 @9x9, two images, 730 -> 255, 64 -> 64 @8x8,
+// 64 images, 50 -> 29, one image 44 -> 12, 19 -> 47 @14x14, 193 images, 73 -> 58, 100 -> 100 @28x28, 32 images, bfloat16, 379 -> 311; odd rows, where tiles ran two instructions:
+// 32 images, 64 -> 32 @17x17 78 -> 45, @21x21 82 -> 62, @25x25 83 -> 83, @29x29 82 -> 97, @53x53 258 -> 285; what fills tiles stays there (fills_5x5_tiles).
 // Tried on the way: 4 x 4 per lane 64 -> 64 @56x56, 16 images, 471 (66 registers spilled), 4 x 2 in three instructions 295, with five waves per SIMD 327.
 #include "wave_split.hpp"
 
@@ -35,14 +36,15 @@ struct GxNineCfg {
     static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;   // input channels whose weights are asked for together, a step ahead
     static constexpr int PART = KSP * TM * TN * 64, LDS_BYTES = PART * 4 + KSP * TN * 64 * 8;
     static_assert((TM % KSP == 0 || KSP % TM == 0) && (NU == 1 || NU % 2 == 0), "a wave finishes FM channels or none; two weight buffers");
-    // 25 taps, two positions of rows of an even length: the two columns on a side are both inside the map or both outside, and one read
+    // 25 taps, two positions: the two columns on a side are both inside the map or both outside (rows of an odd length: see Strips), and one read
     static constexpr bool PAIRS = KS == 5 && TN == 2;
     static_assert(KS == 3 || (KS == 5 && TN <= 2), "nine taps, or 25 of one or two positions");
 };
 
 struct GxNineDims {
     int N, Ci, H, W, Co;
-    int per_row, strips;    // strips of TN positions per row (the last one is moved back to end at W) and per image
+    Strips row;
+    int strips;             // of TN positions per image
     int tiles, blocks;      // of 64 strips, of TM input channels
 };
 
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
     xcd_tile(blockIdx.x, d.tiles, d.blocks, tile, blk);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int sidx = tile * 64 + lane, sc = min(sidx, d.N * d.strips - 1), n = sc / d.strips, rest = sc - n * d.strips;
-    const int h = rest / d.per_row, s = rest - h * d.per_row, w0 = min(s * TN, d.W - TN), ci_base = blk * TM;
+    const int h = rest / d.row.per_row, s = rest - h * d.row.per_row, w0 = d.row.start(s, TN, d.W), ci_base = blk * TM;
     const int plane = d.H * d.W, K = d.Ci * KK;
     uniform_f32_ptr wc = as_uniform(w);
     int wofs[TM];
@@ -279,7 +281,7 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
     if (ci0 >= d.Ci) return;
     unsigned own = 0;   // bit t: position w0 + t is this lane's
 #pragma unroll
-    for (int t = 0; t < TN; ++t) own |= (sidx == sc && w0 + t >= s * TN ? 1u : 0u) << t;
+    for (int t = 0; t < TN; ++t) own |= (sidx == sc && w0 + t >= d.row.first(s, TN) ? 1u : 0u) << t;
     finish_grad_x<FM, TN, FUSE>(r, own, ci0, ci0, d.Ci, plane, (n * d.Ci + ci0) * plane + h * d.W + w0, TN > 1 && d.W % TN == 0, x, gx, gadd, bn,
                                 d.tiles, tile, lane);
 }
@@ -293,9 +295,13 @@ static int gx_nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((lo
 struct GxNineShape { int tn, waves; };
 static GxNineShape gx_nine_shape(const ConvDims &d) {
     const int waves = d.Co <= 8 ? 1 : d.Co <= 16 ? 2 : d.Co <= 32 ? 4 : 8;
-    if (d.kh == 5)   // us, 4 x 2 / 4 x 1 (W even): 64 -> 64 @8x8, 64 images, 4096 waves of 4 x 2, 32 / 37, 48 -> 342 @10x10, 8 images, 672, 70 / 56, 64 -> 64 @32x32, one, 1024, 17.5 / 13.4;
-                     // W odd, the columns beside a strip one by one: 27 -> 267 @15x15, 40 images, 167 / 160, 551 -> 813 @9x9, two, 347 / 249
-        return {d.W % 2 == 0 && (long)gx_nine_tiles(d, 2) * ceil_div(d.Ci, 4) * waves >= 2048 ? 2 : 1, waves};
+    if (d.kh == 5) {
+        // us, 4 x 2 / 4 x 1: W even, two instructions a term, 64 -> 64 @8x8, 64 images, 4096 waves of 4 x 2, 32 / 37, 48 -> 342 @10x10, 8 images, 672, 70 / 56, 64 -> 64
+        // @32x32, one, 1024, 17.5 / 13.4; W odd, three, 64 -> 32 @29x29, 32 images, 97 / 119, 16 -> 16 @17x17, 64 images, 1224 waves, 16.0 / 16.9, 32 -> 64 @21x21, 4 images,
+        // 960, 15.6 / 14.4.  (Rows of three and five columns have no strips without a cut pair.)
+        const bool pairs = d.W % 2 == 0 || d.W >= 7;
+        return {pairs && (long)gx_nine_tiles(d, 2) * ceil_div(d.Ci, 4) * waves >= (d.W % 2 ? 1200 : 2048) ? 2 : 1, waves};
+    }
     int tn = d.W >= 4 ? 4 : d.W >= 2 ? 2 : 1;
     if (tn == 4 && (long)gx_nine_tiles(d, 4) * ceil_div(d.Ci, 8) * waves < 1300) tn = 2;
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
@@ -320,7 +326,7 @@ template <class C, bool SAT, class T, bool FUSE>
 static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
                           const adder_bn_links &bn) {
     const int per_row = ceil_div(d.W, C::TN);
-    const GxNineDims t{d.N, d.Ci, d.H, d.W, d.Co, per_row, per_row * d.H, gx_nine_tiles(d, C::TN), ceil_div(d.Ci, C::TM)};
+    const GxNineDims t{d.N, d.Ci, d.H, d.W, d.Co, Strips{per_row, C::PAIRS && d.W % 2 ? 2 : kNoShift}, per_row * d.H, gx_nine_tiles(d, C::TN), ceil_div(d.Ci, C::TM)};
     if (FUSE && (!bn.in_part || bn.in_slots != t.tiles)) return ADDER_ERR_BAD_SHAPE;
     if (int rc = allow_dynamic_lds<&grad_x_nine_kernel<C, SAT, T, FUSE>>(C::LDS_BYTES)) return rc;
     hipLaunchKernelGGL((grad_x_nine_kernel<C, SAT, T, FUSE>), dim3((unsigned)t.tiles * t.blocks), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
@@ -332,7 +338,7 @@ static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const 
 // three instructions 8.8; 64 -> 64 @56x56, one, 11.9, 13.2) and rounds w and x once more (1.6e-7 of the result against 2.3e-7).
 GradXShape grad_x_nine_shape(const ConvDims &d, bool bf16, bool groups) {
     const GxNineShape shape = gx_nine_shape(d);
-    if (d.kh == 5) return {4, shape.tn, shape.waves, shape.tn == 2 && groups && d.Ci >= 2 && two_instructions_5x5(d.Co)};
+    if (d.kh == 5) return {4, shape.tn, shape.waves, shape.tn == 2 && d.W % 2 == 0 && groups && d.Ci >= 2 && two_instructions_5x5(d.Co)};
     const bool two = shape.tn == 4 && groups && d.Co * 9 <= kSatMaxTerms && d.Ci >= 4 && !small_unlinked(d, bf16, d.W, 660000);
     return {shape.tn == 1 ? 4 : 8, shape.tn, shape.waves, two};
 }

@@ -144,6 +144,16 @@ struct ChunkSums {
     }
 };
 
+// Strips of TN columns per row: strip s starts at column s * TN, the last one is moved back to end with the row.  Where the columns beside a strip are read in
+// pairs (25 taps) no pair may be half inside the row, so rows that would cut one take the strips from number `from` on a column earlier.
+// start, first: a strip's first column, and the first that is its own and not the strip's before it.
+struct Strips {
+    int per_row, from;
+    __device__ __forceinline__ int start(int s, int tn, int row) const { return min(s * tn - (s >= from ? 1 : 0), row - tn); }
+    __device__ __forceinline__ int first(int s, int tn) const { return s * tn - (s > from ? 1 : 0); }
+};
+static constexpr int kNoShift = 0x7fffffff;
+
 // Waves that share `chunks` chunks, at most `most`: as few as finish them in the same number of rounds
 static inline int waves_for(int chunks, int most) { return ceil_div(chunks, ceil_div(chunks, most)); }
 

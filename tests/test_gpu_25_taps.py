@@ -1,10 +1,10 @@
 """5x5 layers (csrc/fwd_nine.hip with 25 taps) against the float64 oracle where strips, tiles, pairs of columns and waves end: maps of one row or
-column, rows one longer than whole strips (4 x 1 results per lane), rows whose last strip is moved back, even and odd rows at stride 2, channels that
+column, rows one longer than whole strips, rows whose last strip is moved back, even and odd rows at stride 2, channels that
 give a wave none -- with the inference epilogue, bases of any alignment and both storage types."""
 import pytest
 import torch
 
-from tests.util import make_case, assert_close
+from tests.util import make_case, assert_close, fwd_kernel, grad_x_kernel, NINE
 from tests.test_gpu_bf16 import _close_bf16
 
 pytestmark = pytest.mark.gpu
@@ -84,3 +84,22 @@ def test_second_gradient(shape, gpu):
         assert rc == 0 and torch.equal(out, gx + gadd)
     else:
         assert rc == -7   # one channel never had one
+
+
+# Rows whose strips start a column earlier, so that no pair of columns beside one is half inside the row: four positions per lane on rows of whole strips and
+# one column, two on rows of an odd length (from seven columns on)
+ODD_ROWS = [(60, 12, 20, 9, 41), (100, 13, 11, 13, 41), (40, 20, 17, 17, 30), (60, 9, 14, 21, 41), (9, 41, 20, 37, 41), (20, 75, 17, 29, 21)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", ODD_ROWS, ids=str)
+def test_rows_of_whole_strips_and_one_column(shape, dtype, gpu):
+    assert fwd_kernel(shape + (5, 1, 2))[:3] == (NINE, 4, 4)
+    test_forward(shape, 1, dtype, gpu)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", ODD_ROWS + [(60, 30, 13, 7, 41), (33, 21, 9, 11, 60), (20, 20, 14, 23, 131)], ids=str)
+def test_input_gradient_of_odd_rows(shape, dtype, gpu):
+    assert grad_x_kernel(shape + (5, 1, 2), dtype == torch.bfloat16)[:3] == (NINE, 4, 2)
+    test_input_gradient(shape, dtype, gpu)
