@@ -367,11 +367,20 @@ struct GradXShape { int tm, tn, waves; bool two; };   // of the kernels without 
 GradXShape grad_x_tap_shape(const ConvDims &d, bool bf16);
 GradXShape grad_x_nine_shape(const ConvDims &d, bool bf16, bool groups);
 GradXShape grad_x_s2_shape(const ConvDims &d, bool sat);
-// Whether the input gradient of a stride-1 layer is small and has no kernel that a BatchNorm is linked to: bfloat16, or rows (1x1: planes) that are no
-// whole groups of four.  Those take three instructions a term: the doubled sum minus the sum of gy that two need rounds once more (3x3 of 60 to
-// 100 output channels: 2.4e-7 of the result against 1.7e-7, the largest element 1.5 times as far) and makes an infinite gy NaN.
-static constexpr bool small_unlinked(const ConvDims &d, bool bf16, int row, long elements) {
-    return (bf16 || row % 4 != 0) && (long)d.N * d.Ci * d.H * d.W < elements;
+// Whether the input gradient of a 3x3 or 1x1 layer of stride 1 is small and has no kernel that a BatchNorm is linked to: bfloat16, or rows (1x1: planes)
+// that are no whole groups of four.  Those take three instructions a term: the doubled sum minus the sum of gy that two need rounds once more (3x3 of 60
+// to 100 output channels: 2.4e-7 of the result against 1.7e-7, the largest element 1.5 times as far) and makes an infinite gy NaN.  Small: a launch that a
+// kernel of one position per lane finishes (0.45 us of nine taps or 0.15 of one a channel of a wave's share, then 9 or 6.5 terms per ps) before one of 16
+// results per lane (small maps: eight) has walked all output channels (5.5 or 9.5 ns a term and result).
+static inline bool small_unlinked(const ConvDims &d, bool bf16) {
+    const bool nine = d.kh == 3;
+    const int row = nine ? d.W : d.H * d.W;
+    if (!bf16 && row % 4 == 0) return false;
+    if (!nine && row <= 64 && (long)ceil_div(d.N, 4) * ceil_div(d.Ci, 64) > 256) return false;
+    const int results = row > (nine ? 8 : 64) ? 16 : 8, eighth = round_up(ceil_div(d.Co, 8), 8), chunk = nine ? 8 : eighth < 16 ? 16 : eighth > 64 ? 64 : eighth;
+    const float terms = (float)d.K() * d.Co * d.N * d.H * d.W, share = (float)(ceil_div(ceil_div(d.Co, chunk), 8) * chunk);
+    const float all = nine ? 2.f + 0.0055f * 9 * results * d.Co : 3.f + 0.0095f * results * d.Co;
+    return (nine ? 2.f + 0.45f * share + terms / 9e6f : 3.f + 0.15f * share + terms / 6.5e6f) < 0.9f * all;
 }
 // 1x1 / stride 1 (grad_x_tap.hip); bn (nullable): the in_* half of adder_bn_links, slots of sums per channel
 template <class T>

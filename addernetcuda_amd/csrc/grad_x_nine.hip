@@ -288,39 +288,60 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_nine_kernel(const T *__restri
 
 static int gx_nine_tiles(const ConvDims &d, int tn) { return (int)ceil_div_l((long)d.N * d.H * ceil_div(d.W, tn), 64); }
 
-// Waves that share the output channels, and input channels x positions per lane: by the rules of fwd_nine.hip, with a wave's chain of
-// 1.7, 1.15 and 0.55 us a channel and 24, 22 and 12 terms per ps (4 x 1: 7 on rows that are shorter than 8).  us, 8 x 4 / 8 x 2 / 4 x 1:
-// 128 -> 128 @28x28, 4 images, 29 / 31 / 36, one 29 / 20 / 14; 64 -> 64 @56x56, one, 17 / 12 / 14; 256 -> 256 @14x14, 4, 66 / 44 / 43, one 66 / 44 / 18;
-// 512 -> 512 @7x7, 4, 128 / 92 / 63, one 128 / 83 / 32.
-struct GxNineShape { int tn, waves; };
-static GxNineShape gx_nine_shape(const ConvDims &d) {
+// Positions per lane (input channels: 8 x 4, 8 x 2 or 4 x 1, 25 taps 4), waves that share the output channels, and whether a term takes two instructions.
+//
+// Two instructions, 8 x 4 only and only where the launch fills the chip: below that they gain nothing (32 -> 32 @16x16, 32 images, 9.1 us, three 8.8; 64 -> 64
+// @56x56, one, 11.9, 13.2) and round w and x once more (2.3e-7 of the result against 1.6e-7).  The line to the smaller shapes is that of fwd_nine.hip, with a
+// wave's chain of 1.7, 1.15 and 0.55 us a channel and 24, 22 and 12 terms per ps (4 x 1: 7 on rows that are shorter than 8).  us, 8 x 4 / 8 x 2 / 4 x 1: 128 -> 128
+// @28x28, 4 images, 29 / 31 / 36, one 29 / 20 / 14; 64 -> 64 @56x56, one, 17 / 12 / 14.
+//
+// Three instructions: a workgroup of 8 x 4 is long and few fill the chip, and two of them on a CU wait for each other's weights, so that the smaller shapes are
+// ahead until some ten of 8 x 4 lie on each CU.  By what the busiest CU takes for a wave's channels, us per channel and workgroup of eight waves there.
+// us, 8 x 4 / 8 x 2 / 4 x 1 with eight waves: 921 -> 174 (channels of gy -> of gx) @42x42, one image, 321 / 278 / 219, 713 -> 149 @42x50, one, 258 / 214 / 172, 517 -> 535
+// @15x18, three, 294 / 172 / 177, 242 -> 15 @53x53, 13, 139 / 114 / 100, 144 -> 144 @28x28, eight, 82 / 88 / 89, 32, 245 / 266 / 309, 200 -> 200 @14x14, 128, 498 / 490 / 560,
+// 512 -> 512 @8x8, 128, 978 / 1058 / 1293, 512 -> 512 @7x7, one, 128 / 83 / 32.
+GradXShape grad_x_nine_shape(const ConvDims &d, bool bf16, bool groups) {
     const int waves = d.Co <= 8 ? 1 : d.Co <= 16 ? 2 : d.Co <= 32 ? 4 : 8;
     if (d.kh == 5) {
         // us, 4 x 2 / 4 x 1: W even, two instructions a term, 64 -> 64 @8x8, 64 images, 4096 waves of 4 x 2, 32 / 37, 48 -> 342 @10x10, 8 images, 672, 70 / 56, 64 -> 64
-        // @32x32, one, 1024, 17.5 / 13.4; W odd, three, 64 -> 32 @29x29, 32 images, 97 / 119, 16 -> 16 @17x17, 64 images, 1224 waves, 16.0 / 16.9, 32 -> 64 @21x21, 4 images,
-        // 960, 15.6 / 14.4.  (Rows of three and five columns have no strips without a cut pair.)
-        const bool pairs = d.W % 2 == 0 || d.W >= 7;
-        return {pairs && (long)gx_nine_tiles(d, 2) * ceil_div(d.Ci, 4) * waves >= (d.W % 2 ? 1200 : 2048) ? 2 : 1, waves};
+        // @32x32, one, 1024, 17.5 / 13.4; W odd, three, by the busiest CU's workgroups, where one of 4 x 2 takes 1.63 times as long as one of 4 x 1: 64 -> 32 @29x29, 32
+        // images, 97 / 119, 16 -> 16 @17x17, 64 images, 1224 waves, 16.0 / 16.9, 32 -> 64 @21x21, 4 images, 960, 15.6 / 14.4, 821 -> 665 @9x9, two, 334 and 501 workgroups,
+        // 316 / 256.  (Rows of three and five columns have no strips without a cut pair.)
+        const long wide = (long)gx_nine_tiles(d, 2) * ceil_div(d.Ci, 4), narrow = (long)gx_nine_tiles(d, 1) * ceil_div(d.Ci, 4);
+        const bool odd = d.W % 2 != 0, pairs = !odd || d.W >= 7;
+        const int tn = pairs && wide * waves >= (odd ? 1200 : 2048) && (!odd || 163 * ceil_div_l(wide, 256) <= 100 * ceil_div_l(narrow, 256)) ? 2 : 1;
+        return {4, tn, waves, tn == 2 && d.W % 2 == 0 && groups && d.Ci >= 2 && two_instructions_5x5(d.Co)};
     }
-    int tn = d.W >= 4 ? 4 : d.W >= 2 ? 2 : 1;
-    if (tn == 4 && (long)gx_nine_tiles(d, 4) * ceil_div(d.Ci, 8) * waves < 1300) tn = 2;
+    auto wgs = [&](int n) { return (long)gx_nine_tiles(d, n) * ceil_div(d.Ci, n == 1 ? 4 : 8); };
+    const int most = d.W >= 4 ? 4 : d.W >= 2 ? 2 : 1;
     const float terms = (float)d.K() * d.Co * d.N * d.H * d.W;
     const int chunks = ceil_div(ceil_div(d.Co, kNineChunk), waves), chain = min(chunks * kNineChunk, d.Co);
-    const float wide = fmaxf((tn == 4 ? 1.7f : 1.15f) * chain, terms / (tn == 4 ? 24e6f : 22e6f));
-    const float narrow = fmaxf(0.55f * chain, terms / (d.W < 8 ? 7e6f : 12e6f));
-    if (narrow < wide) tn = 1;
-    // (two waves would share nine to twelve channels two to one: 48 -> 12 @32x32, 64 images, 25.0 us, one wave 23.5)
-    return {tn, tn == 4 && d.Co <= 12 ? 1 : waves};
+    if (most == 4 && groups && d.Co * 9 <= kSatMaxTerms && d.Ci >= 4 && !small_unlinked(d, bf16) && wgs(4) * waves >= 1300) {
+        const float wide = fmaxf(1.7f * chain, terms / 24e6f), narrow = fmaxf(0.55f * chain, terms / (d.W < 8 ? 7e6f : 12e6f));
+        // (waves that would have less than half a chunk are left out: 17 channels @28x28, 32 images, four waves 34.6 us, two 30.1, 33 channels, eight 53.6, four 48.5)
+        const int full = full_chunks(d.Co, kNineChunk);
+        if (narrow >= wide) return {8, 4, full <= 2 ? full : full <= 4 ? 4 : 8, true};
+    }
+    int tn = 1;
+    float least = 0.f;
+    for (int n = 1; n <= most; n *= 2) {
+        const float load = (float)ceil_div_l(wgs(n), 256) * waves / 8, share = (float)d.Co / waves;
+        const float per = n == 1 ? fmaxf(0.55f, (d.W < 8 ? 0.48f : 0.37f) * load) : n == 2 ? fmaxf(1.2f + 0.2f * load, 0.3f + 1.1f * load)
+                                                                                         : fmaxf(2.f + 0.8f * load, 2.f * load);
+        const float cost = per * (load <= 2.f ? 0.5f * (chain + share) : share);
+        if (n == 1 || cost < least) { tn = n; least = cost; }
+    }
+    return {tn == 1 ? 4 : 8, tn, waves, false};
 }
 
 // Layers it takes; the distance of a wave's strips from the first one's image has to fit 32 bits, and so have the launch's threads.
 bool grad_x_nine_supported(const ConvDims &d) {
     if (d.kh != d.kw || (d.kh != 3 && d.kh != 5) || d.pad != d.kh / 2 || d.stride != 1) return false;
     if ((images_ahead(d, (long)d.H * ceil_div(d.W, 4)) * d.Co + 1) * d.H * d.W > 0x3fffffffL) return false;
-    const GxNineShape shape = gx_nine_shape(d);
-    return (long)gx_nine_tiles(d, shape.tn) * ceil_div(d.Ci, d.kh == 5 || shape.tn == 1 ? 4 : 8) * 64 * shape.waves <= kMaxThreads;
+    const GradXShape shape = grad_x_nine_shape(d, false, true);
+    return (long)gx_nine_tiles(d, shape.tn) * ceil_div(d.Ci, shape.tm) * 64 * shape.waves <= kMaxThreads;
 }
-int grad_x_nine_bn_slots(const ConvDims &d) { return gx_nine_tiles(d, gx_nine_shape(d).tn); }
+int grad_x_nine_bn_slots(const ConvDims &d) { return gx_nine_tiles(d, grad_x_nine_shape(d, false, true).tn); }
 
 template <class C, bool SAT, class T, bool FUSE>
 static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const ConvDims &d, hipStream_t s, const T *gadd,
@@ -332,15 +353,6 @@ static int launch_gx_nine(const T *gy, const T *x, const float *w, T *gx, const 
     hipLaunchKernelGGL((grad_x_nine_kernel<C, SAT, T, FUSE>), dim3((unsigned)t.tiles * t.blocks), dim3(C::NT), C::LDS_BYTES, s, gy, x, w, gx, t,
                        gadd, bn);
     return check_launch();
-}
-
-// The two-instruction form only where the launch fills the chip: below that it gains nothing (32 -> 32 @16x16, 32 images, 9.1 us,
-// three instructions 8.8; 64 -> 64 @56x56, one, 11.9, 13.2) and rounds w and x once more (1.6e-7 of the result against 2.3e-7).
-GradXShape grad_x_nine_shape(const ConvDims &d, bool bf16, bool groups) {
-    const GxNineShape shape = gx_nine_shape(d);
-    if (d.kh == 5) return {4, shape.tn, shape.waves, shape.tn == 2 && d.W % 2 == 0 && groups && d.Ci >= 2 && two_instructions_5x5(d.Co)};
-    const bool two = shape.tn == 4 && groups && d.Co * 9 <= kSatMaxTerms && d.Ci >= 4 && !small_unlinked(d, bf16, d.W, 660000);
-    return {shape.tn == 1 ? 4 : 8, shape.tn, shape.waves, two};
 }
 
 // bn (nullable): the in_* half of adder_bn_links

@@ -244,7 +244,7 @@ GradXShape grad_x_tap_shape(const ConvDims &d, bool bf16) {
     if (d.Ci < 8) return {4, d.H * d.W >= 2 ? 2 : 1, 4, false};   // (no link and no second gradient: grad_x_tap_narrow)
     if (d.Ci < 16) return {8, shape.tn, shape.tn == 1 ? 8 : 4, false};
     const bool exact = shape.tm == 8 || !grad_x_tap_supported(d) || (shape.waves == 8 && (d.H * d.W) % 4 != 0) ||
-                       small_unlinked(d, bf16, d.H * d.W, 770000);
+                       small_unlinked(d, bf16);
     return {shape.tm, shape.tn, shape.waves, !exact && d.Co <= kSatMaxTerms1x1};
 }
 

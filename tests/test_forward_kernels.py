@@ -34,9 +34,12 @@ def test_kernels_of_some_layers():
     assert fwd_kernel((32, 256, 56, 56, 512, 1, 2, 0))[0] == TILES and fwd_kernel((1, 256, 56, 56, 512, 1, 2, 0))[0] == TAP
     assert grad_x_kernel((128, 128, 32, 32, 128, 3, 1, 1))[0] == TILES
     assert grad_x_kernel((32, 64, 56, 56, 64, 3, 1, 1)) == (NINE, 8, 4, 8, 2)
-    assert grad_x_kernel((7, 63, 28, 31, 96, 3, 1, 1)) == (NINE, 8, 4, 8, 3)
+    assert grad_x_kernel((7, 63, 28, 31, 96, 3, 1, 1)) == (NINE, 4, 1, 8, 3)
     assert grad_x_kernel((32, 256, 14, 14, 1024, 1, 1, 0)) == (TAP, 16, 2, 8, 2)
     assert grad_x_kernel((5, 107, 23, 23, 278, 3, 2, 1))[0] == S2
+    # three instructions a term: small shapes until the chip is full, whole groups of waves
+    assert grad_x_kernel((1, 174, 42, 42, 921, 3, 1, 1)) == (NINE, 4, 1, 8, 3) and grad_x_kernel((128, 512, 8, 8, 512, 3, 1, 1)) == (NINE, 8, 4, 8, 3)
+    assert grad_x_kernel((32, 96, 28, 28, 17, 3, 1, 1)) == (NINE, 8, 4, 2, 2) and grad_x_kernel((32, 96, 28, 28, 33, 3, 1, 1)) == (NINE, 8, 4, 4, 2)
     assert grad_x_kernel((1, 3, 8, 8, 3, 1, 1, 0))[0] == PLAIN_1X1 and grad_x_kernel((1, 3, 8, 8, 3, 1, 3, 0))[0] == GENERAL
 
 
