@@ -29,9 +29,9 @@ def emulate(x, w, stride, pad):
     xp = torch.nn.functional.pad(x, (pad, pad, pad, pad))
     chunk, joins = chunk_of(Ci, Wo, k, stride)
     starts = list(range(0, max(1, Ci & ~3) if joins else Ci, chunk))
-    tot = torch.zeros(N, Co, Ho, Wo)
+    tot = torch.zeros(N, Co, Ho, Wo, device=x.device)
     for c0, c1 in zip(starts, starts[1:] + [Ci]):
-        acc = torch.zeros(N, Co, Ho, Wo)
+        acc = torch.zeros(N, Co, Ho, Wo, device=x.device)
         for ci in range(c0, c1):
             for i in range(k):
                 for j in range(k):

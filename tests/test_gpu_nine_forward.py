@@ -1,7 +1,8 @@
 """The 3x3 forward kernel (csrc/fwd_nine.hip) against the float64 oracle where its strips, rows, tiles and waves end: rows of one, two
 and three columns, maps of one row, odd and even rows at stride 2, channels that give a wave no chunk or part of one, output channels
-that fill no block, each number of waves and of positions per lane -- with its statistics, its inference epilogue, bases of any
-alignment and both storage types.  (As an ordinary convolution and with the strided 1x1 layer beside it: test_gpu_resnet20, test_gpu_pair.)"""
+that fill no block -- with its statistics, its inference epilogue, bases of any
+alignment and both storage types.  (Each number of waves and of positions per lane:
+test_gpu_kernel_shapes; as an ordinary convolution and with the strided 1x1 layer beside it: test_gpu_resnet20, test_gpu_pair.)"""
 import pytest
 import torch
 
@@ -12,8 +13,8 @@ pytestmark = pytest.mark.gpu
 
 # (N, Ci, H, W, Co, stride)
 SHAPES = [(1, 1, 1, 1, 1, 1), (2, 9, 5, 1, 9, 1), (3, 33, 1, 2, 7, 1), (2, 8, 3, 3, 12, 1), (70, 17, 2, 5, 5, 1), (1, 264, 7, 7, 31, 1),
-          (3, 130, 14, 14, 33, 1), (9, 24, 9, 33, 40, 1), (2, 70, 56, 55, 9, 1),                      # small launches: 1 and 2 positions per lane
-          (200, 7, 32, 29, 12, 1), (64, 16, 33, 35, 20, 1), (60, 30, 17, 17, 70, 1), (12, 64, 30, 32, 40, 1),   # 4 positions; 1, 2, 4, 8 waves
+          (3, 130, 14, 14, 33, 1), (9, 24, 9, 33, 40, 1), (2, 70, 56, 55, 9, 1),                      # one position per lane
+          (200, 7, 32, 29, 12, 1), (64, 16, 33, 35, 20, 1), (60, 30, 17, 17, 70, 1), (12, 64, 30, 32, 40, 1),   # two and four
           (1, 3, 1, 1, 2, 2), (2, 9, 5, 1, 9, 2), (2, 12, 1, 7, 5, 2), (5, 35, 2, 2, 3, 2), (4, 20, 18, 18, 18, 2), (4, 20, 17, 19, 18, 2),
           (64, 16, 32, 32, 32, 2), (130, 40, 9, 9, 40, 2), (40, 5, 21, 24, 70, 2)]
 

@@ -1,7 +1,8 @@
 """The input-gradient kernel of 3x3 / stride-1 layers (csrc/grad_x_nine.hip) against the float64 oracle where its strips, tiles, groups
 of channels and waves end: rows that are shorter than a strip or whose last strip is moved back, input channels that do not fill a
-group, output channels that end inside a chunk or give a wave none, each of its shapes with one to eight waves and both forms -- with
-bases of any alignment and both storage types; and with the BatchNorm link, which gives the plain kernel's bits."""
+group, output channels that end inside a chunk or give a wave none, one to eight waves -- with bases
+of any alignment and both storage types; and with the BatchNorm link, which gives the plain kernel's bits.  (Each of its shapes in both forms:
+test_gpu_kernel_shapes.)"""
 import ctypes
 
 import pytest
@@ -12,7 +13,7 @@ from tests.test_gpu_bf16 import _close_bf16
 
 pytestmark = pytest.mark.gpu
 
-# (N, Ci, H, W, Co): 4 x 1 with one to eight waves, then 8 x 2, then 8 x 4; more than 128 output channels are the second form
+# (N, Ci, H, W, Co): 4 channels x 1 position with one to eight waves; 8 x 4 in two instructions a term
 SHAPES = [(1, 4, 1, 1, 1), (3, 5, 1, 2, 7), (70, 9, 1, 3, 8), (2, 7, 5, 4, 9), (1, 3, 9, 9, 17), (9, 65, 7, 7, 129), (64, 17, 8, 8, 12),
           (60, 70, 17, 13, 16), (16, 67, 21, 19, 32), (9, 67, 21, 20, 40), (9, 67, 21, 20, 136),
           (40, 61, 33, 30, 5), (40, 70, 31, 29, 16), (30, 57, 21, 22, 30), (20, 67, 21, 18, 37), (20, 66, 21, 18, 131)]
@@ -39,9 +40,10 @@ def test_matches_the_oracle(shape, dtype, gpu):
     assert torch.equal(_grad_x(xg, wg, off), got)
 
 
-# (links are offered for whole groups of four positions per row; the shapes above, and the tiles that are left to grad_x.hip)
+# (links are offered for whole groups of four positions per row: 4 x 1, 8 x 2 and 8 x 4, one to eight waves, two instructions a term and three)
 LINKED = [(2, 9, 3, 4, 7), (16, 19, 8, 8, 130), (60, 70, 17, 12, 16), (9, 68, 21, 20, 40), (40, 60, 33, 32, 5), (30, 57, 21, 20, 30),
-          (20, 67, 21, 20, 131), (260, 9, 16, 16, 9), (130, 9, 32, 32, 9)]
+          (20, 67, 21, 20, 131), (260, 9, 16, 16, 9), (130, 9, 32, 32, 9),
+          (300, 30, 13, 16, 5), (300, 263, 3, 4, 11), (300, 130, 3, 4, 19), (60, 263, 3, 4, 41), (200, 263, 3, 4, 19), (200, 130, 3, 4, 41), (130, 5, 28, 28, 150)]
 
 
 @pytest.mark.parametrize("shape", LINKED, ids=str)

@@ -1,7 +1,7 @@
 """The input-gradient kernel of strided 3x3 and 5x5 layers (csrc/grad_x_s2.hip) against the float64 oracle where its blocks, tiles, groups of
 channels and waves end: odd maps, whose last blocks are cut, maps of one row or column, input channels that do not fill a group,
-output channels that end inside a chunk or give a wave none, both of its shapes with one to eight waves and both forms -- with bases
-of any alignment and both storage types; and a second gradient where the entry point adds one."""
+output channels that end inside a chunk or give a wave none, one to eight waves -- with bases of any alignment and both storage
+types; and a second gradient where the entry point adds one.  (All with two channels per lane: test_gpu_kernel_shapes has the layers of four, in both forms.)"""
 import pytest
 import torch
 
@@ -10,7 +10,7 @@ from tests.test_gpu_bf16 import _close_bf16
 
 pytestmark = pytest.mark.gpu
 
-# (N, Ci, H, W, Co): two channels per lane with one to eight waves, then four; rows of an even length are the form of two instructions
+# (N, Ci, H, W, Co)
 SHAPES = [(1, 2, 1, 1, 1), (3, 5, 1, 2, 7), (70, 9, 2, 3, 8), (2, 7, 5, 4, 9), (1, 3, 9, 9, 17), (9, 65, 7, 7, 129), (2, 6, 13, 18, 40),
           (150, 41, 17, 21, 5), (70, 70, 17, 13, 16), (20, 67, 21, 19, 32), (20, 67, 21, 22, 32), (9, 67, 21, 20, 40), (9, 64, 22, 22, 136),
           (9, 64, 21, 22, 300)]

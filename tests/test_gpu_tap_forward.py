@@ -1,6 +1,6 @@
 """The 1x1 forward kernel (csrc/fwd_tap.hip) against the float64 oracle where its strips, tiles and waves end: planes of 1
 to 4 positions and of no whole strips, channels that give a wave no chunk or part of one, output channels that fill no block, one,
-two and four positions per lane -- with its statistics, its inference epilogue, bases of any alignment and both storage types."""
+two and four positions per lane (with each number of waves: test_gpu_kernel_shapes) -- with its statistics, its inference epilogue, bases of any alignment and both storage types."""
 import pytest
 import torch
 
@@ -9,7 +9,7 @@ from tests.test_gpu_bf16 import _close_bf16
 
 pytestmark = pytest.mark.gpu
 
-# (N, Ci, H, W, Co): one position per lane, two, four (with two, four and eight waves, planes of whole strips and not)
+# (N, Ci, H, W, Co): one position per lane, two, four; planes of whole strips and not
 SHAPES = [(1, 64, 1, 1, 8), (3, 64, 1, 2, 9), (70, 68, 1, 3, 5), (65, 64, 2, 2, 1), (5, 128, 7, 7, 18), (2, 132, 13, 1, 1), (1, 1028, 5, 5, 7),
           (16, 128, 20, 20, 64), (9, 516, 9, 9, 130), (300, 64, 7, 7, 64), (40, 256, 15, 15, 72), (64, 260, 14, 14, 64), (33, 76, 32, 32, 24)]
 

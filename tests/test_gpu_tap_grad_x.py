@@ -1,7 +1,8 @@
 """The input-gradient kernel of 1x1 / stride-1 layers (csrc/grad_x_tap.hip) against the float64 oracle where its strips, tiles, groups
 of channels and waves end: planes of one to three positions and of an odd number, input channels that shift the last group, output
-channels that end inside a group of four or give a wave no chunk, each of its shapes and both forms -- with a second gradient, bases
-of any alignment and both storage types; and with the BatchNorm link, which gives the plain kernel's bits."""
+channels that end inside a group of four or give a wave no chunk -- with a second gradient, bases
+of any alignment and both storage types; and with the BatchNorm link, which gives the plain kernel's bits.
+(Each of its shapes in both forms: test_gpu_kernel_shapes.)"""
 import ctypes
 
 import pytest
@@ -12,7 +13,7 @@ from tests.test_gpu_bf16 import _close_bf16
 
 pytestmark = pytest.mark.gpu
 
-# (N, Ci, H, W, Co): 8 x 1 positions, then 16 x 2 with eight, four and one wave
+# (N, Ci, H, W, Co): 8 channels x 1 position, then 16 x 2 with one to eight waves
 SHAPES = [(1, 64, 1, 1, 48), (3, 65, 1, 2, 49), (70, 66, 1, 3, 51), (1, 64, 7, 7, 1030), (2, 127, 13, 1, 130), (5, 79, 9, 9, 64),
           (37, 67, 9, 9, 1027), (64, 72, 14, 14, 48), (40, 270, 7, 7, 129), (30, 100, 21, 21, 50), (160, 65, 21, 21, 50), (40, 80, 33, 32, 65)]
 

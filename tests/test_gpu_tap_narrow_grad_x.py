@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 # (N, Ci, H, W, Co)
 SHAPES = [(1, 4, 1, 1, 16), (3, 5, 1, 2, 17), (70, 7, 1, 3, 40), (9, 8, 5, 5, 19), (200, 9, 7, 7, 131), (40, 15, 20, 21, 33), (2, 16, 9, 9, 64), (130, 23, 14, 14, 65),
-          (65, 63, 9, 10, 47), (12, 63, 31, 33, 130), (9, 70, 9, 9, 33), (4, 6, 30, 31, 300)]
+          (65, 63, 9, 10, 47), (12, 63, 31, 33, 130), (9, 70, 9, 9, 33), (4, 6, 30, 31, 300),
+          (40, 70, 21, 21, 40), (160, 66, 21, 21, 35)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)

@@ -1,0 +1,40 @@
+"""The lists of tests/kernel_shapes.py against the library's answers (no GPU): each layer takes the shape it stands for, and no layer takes one that no
+list has.  A line of a dispatch that moves fails here, with the layer that has to be found again."""
+import random
+
+import pytest
+
+from tests.kernel_shapes import FORWARD, GRAD_X, forward_shape, grad_x_shape
+from tests.util import TAP, NINE, S2, fwd_kernel, grad_x_kernel
+
+
+@pytest.mark.parametrize("shape", FORWARD, ids=str)
+def test_forward_layers_take_their_shape(shape):
+    for waves, case in FORWARD[shape].items():
+        assert forward_shape(case) == (shape, waves), case
+    assert set(FORWARD[shape]) == ({1} if shape == (TAP, 1, True, None, 8, 4) else {1, 2, 4, 8})
+
+
+@pytest.mark.parametrize("shape", GRAD_X, ids=str)
+def test_input_gradients_take_their_shape(shape):
+    for waves, case in GRAD_X[shape].items():
+        assert grad_x_shape(case) == grad_x_shape(case, bf16=True) == (shape, waves), case
+
+
+def _layers(n):
+    r = random.Random(5)
+    for _ in range(n):
+        k = r.choice([1, 3, 5])
+        size = lambda most: int(2 ** r.uniform(0, most))
+        yield size(9), size(10), size(6), size(6), size(10), k, r.choice([1, 2, 3] if k == 1 else [1, 2]), k // 2
+
+
+def test_no_layer_takes_another_shape():
+    for case in _layers(20000):
+        if fwd_kernel(case)[0] in (TAP, NINE):
+            shape, waves = forward_shape(case)
+            assert waves in FORWARD[shape], case
+        for bf16 in (False, True):
+            if grad_x_kernel(case, bf16)[0] in (TAP, NINE, S2):
+                shape, waves = grad_x_shape(case, bf16)
+                assert waves in GRAD_X[shape], case
