@@ -253,14 +253,21 @@ __global__ __launch_bounds__(C::NT, 4) void grad_x_s2_kernel(const T *__restrict
 
 static int gx_s2_tiles(const ConvDims &d) { return (int)ceil_div_l((long)d.N * d.Ho * d.Wo, 64); }
 
-// Waves that share the output channels: one chunk each, as many as eight.
-static int gx_s2_waves(int Co) { return Co <= 8 ? 1 : Co <= 16 ? 2 : Co <= 32 ? 4 : 8; }
-
 // Input channels per lane: four where the launch fills the chip and they waste few, else two (us, four / two: 256 -> 256 @28x28, 32 images, 233 / 304,
 // one image, 2048 waves of four, 19.5 / 20.5, 107 -> 278 @23x23, 5 images, 2592 waves, 31 / 28, 128 -> 128 @56x56, one image, 3328 waves, 16.5 / 19.2;
 // 5x5: 36 -> 34 @38x41, 6 images, 2736 waves, 13.9 / 12.4; six channels, 6 -> 897 @41x49, 27 images, 173 / 137).
-static bool gx_s2_wide(const ConvDims &d) {
-    return d.Ci >= 4 && (long)gx_s2_tiles(d) * ceil_div(d.Ci, 4) * gx_s2_waves(d.Co) >= 3000 && 5 * ceil_div(d.Ci, 4) <= 3 * ceil_div(d.Ci, 2);
+// Waves that share the output channels: one chunk each, as many as eight.  Up to 64 channels at most four, and none for less than half a chunk, where
+// that still makes 2800 waves (us, 3x3 / 5x5: 64 -> 33 @29x29, 64 images, eight waves 38 / 83, four 30 / 64; -> 64 52 / 116, 46 / 105; 60 -> 33 @21x21, 32 images, 12.9 /
+// 24.6, 11.2 / 21.0; 47 -> 17 @58x58, 62 images, bfloat16, four waves 55 / 108, two 43 / 86, -> 9 two 34 / 63, one 27 / 51; but 40 -> 19 @29x29, eight images, 580
+// workgroups, four 5.7 / 7.8, two 6.1 / 8.4, and 60 -> 130 @21x21, 32 images, eight 27 / 65, four 29 / 67).
+static GradXShape gx_s2_shape(const ConvDims &d) {
+    const int most = d.Co <= 8 ? 1 : d.Co <= 16 ? 2 : d.Co <= 32 ? 4 : 8, full = full_chunks(d.Co, kNineChunk), few = full <= 2 ? full : 4;
+    auto shape = [&](int waves) {
+        const bool wide = d.Ci >= 4 && (long)gx_s2_tiles(d) * ceil_div(d.Ci, 4) * waves >= 3000 && 5 * ceil_div(d.Ci, 4) <= 3 * ceil_div(d.Ci, 2);
+        return GradXShape{wide ? 4 : 2, 1, waves, false};
+    };
+    const GradXShape shared = shape(few);
+    return d.Co <= 64 && (long)gx_s2_tiles(d) * ceil_div(d.Ci, shared.tm) * few >= 2800 ? shared : shape(most);
 }
 
 // Layers it takes: from two input channels on; the distance of a wave's strips from the first one's image has to fit 32 bits, and the grid 2^32 threads.
@@ -280,8 +287,9 @@ static int launch_gx_s2(const T *gy, const T *x, const float *w, T *gx, const Co
 }
 
 GradXShape grad_x_s2_shape(const ConvDims &d, bool sat) {
-    const bool wide = gx_s2_wide(d);
-    return {wide ? 4 : 2, 1, gx_s2_waves(d.Co), wide && sat && d.kh == 3};
+    GradXShape shape = gx_s2_shape(d);
+    shape.two = shape.tm == 4 && sat && d.kh == 3;
+    return shape;
 }
 
 // sat: the two-instruction form (grad_x.hip), where the launch fills the chip

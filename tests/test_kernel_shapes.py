@@ -38,3 +38,10 @@ def test_no_layer_takes_another_shape():
             if grad_x_kernel(case, bf16)[0] in (TAP, NINE, S2):
                 shape, waves = grad_x_shape(case, bf16)
                 assert waves in GRAD_X[shape], case
+
+
+@pytest.mark.parametrize("Co,waves", [(8, 1), (9, 1), (12, 2), (17, 2), (20, 4), (33, 4), (64, 4), (65, 8)])
+@pytest.mark.parametrize("k", [3, 5])
+def test_no_wave_of_a_full_strided_launch_is_mostly_idle(Co, waves, k):
+    assert grad_x_shape((62, 47, 58, 57, Co, k, 2, k // 2))[1] == waves
+    assert grad_x_shape((1, 47, 14, 13, Co, k, 2, k // 2))[1] == (1 if Co <= 8 else 2 if Co <= 16 else 4 if Co <= 32 else 8)   # (a small one needs all)
