@@ -5,8 +5,8 @@
 // Two vector instructions per term bound it: v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- 73 T lane-instructions/s is what a bare
 // stream of the pair reaches with two waves on each of a SIMD's two issue ports (62 T with one each).  Weights are wave-uniform and come
 // through the scalar cache as scalar operands.  A lane reads the window of its strip straight into registers, one channel ahead: nine
-// reads of at most 16 bytes serve 576 instructions, a quarter of what L1 delivers, so a tile in LDS, its barriers and its halo
-// columns had nothing to give.  Without a tile the strips of all images line up (14 columns are 4 strips, 56 are 14: 88 and 100 % of
+// reads of at most 16 bytes serve 576 instructions, 4.6 KB in the 288 cycles that a CU takes for them or a quarter of the 64 bytes a cycle
+// that L1 delivers, so a tile in LDS, its barriers and its halo columns had nothing to give.  Without a tile the strips of all images line up (14 columns are 4 strips, 56 are 14: 88 and 100 % of
 // the lanes have work where 16 x 16 and 8 x 32 tiles left 77 and 88 %), and the waves of a workgroup can share the input channels
 // instead of the positions, which is what small maps with many channels need.  Each chunk's sums meet in LDS in channel order (ChunkSums):
 // any other order changes the last bits of a layer, which a deep network amplifies (ResNet-50's logits by up to 0.07 of their root
@@ -17,8 +17,8 @@
 // positions there was) 64 -> 64 @8x8 7.6 -> 6.6, 256 -> 256 @14x14 19.9 -> 17.0, 512 -> 512 @7x7 30 -> 29.
 // Tried on the way: 4 channels x 4 positions per lane 132 -> 179 us (64 -> 64 @56x56: reads), 8 x 2 143.
 //
-// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 117 to 128
-// registers.  us, tiles in LDS -> this: 64 -> 64 @56x56, 16 images, 271 -> 202, 128 -> 64 @16x16, 64 images, 137 -> 132, 32 -> 64 @16x16 40.9 -> 39.8,
+// 25 taps: 4 channels x 4 positions (stride 2: x 2) per lane, three or four reads per row of the window a channel ahead, 92 to 128
+// registers.  (No instance of this file spills vector registers; with the inference epilogue up to 43 scalar ones live in vector lanes.)  us, tiles in LDS -> this: 64 -> 64 @56x56, 16 images, 271 -> 202, 128 -> 64 @16x16, 64 images, 137 -> 132, 32 -> 64 @16x16 40.9 -> 39.8,
 // 64 -> 64 @8x8 65 -> 22, one image 61 -> 9.7, 47 -> 19 @14x14, 193 images, 111 -> 71, 9 -> 20 @53x53, 32 images, 51 -> 31, 813 -> 551 @9x9, two images, 865 -> 258,
 // 32 -> 64, 32 images, @13x13 37 -> 22, @21x21 77 -> 44, @29x29 81 -> 75 (4 x 1 on such rows of whole strips and one column: 98);
 // stride 2: 64 -> 64 @56x56, 32 images, 176 -> 145, 7 -> 144 @23x26, 202 images, 86 -> 60, 36 -> 34 @38x41, 6 images, 30 -> 12, 32 -> 64 @32x32, 64 images, 52 -> 55.
@@ -44,7 +44,7 @@ struct NineCfg {
     // Output channels whose weights are asked for together, a step ahead: a step of one channel x four positions is 72 instructions,
     // enough to hide the request behind; with fewer positions two channels (stride 2: 512 -> 512 @14x14 284 -> 203 us, 256 -> 256 @28x28
     // 181 -> 158; 512 -> 512 @7x7, one image, 32 -> 29).  Two x four positions run out of scalar registers (132 -> 180 us).
-        static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;
+    static constexpr int UM = TN == 4 || KS == 5 ? 1 : 2, NU = TM / UM;
     static constexpr int MID = (TN - 1) * S + 1, STRIP = MID + 2 * PAD;   // columns under the strip, and with those beside it
     static_assert(NU == 1 || NU % 2 == 0, "two weight buffers");
     // 25 taps, more than one position: the two columns on a side are both inside the map or both outside -- at stride 1 (rows of whole strips and one

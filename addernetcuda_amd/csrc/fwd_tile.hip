@@ -5,8 +5,9 @@
 // Why not those kernels here as well: a slot of statistics sums the results of one wave, and their strips of all images in a row
 // group the results otherwise than a tile does.  The sums then differ in their last bits, the normalised maps behind them with them,
 // and a deep network amplifies that: the logits of an untrained ResNet-50 whose BatchNorm statistics came from either grouping lie up to
-// 0.07 of their root mean square apart.  The training steps that call these forwards are within 1 % of what strips gave them (ResNet-20,
-// batch 256, 2041 us here, 2021 with strips; VGG-small and DenseNet alike).
+// 0.07 of their root mean square apart.  The price is small on ResNet-20 (step at batch 256 2041 us here, 2021 with strips), VGG-small and
+// DenseNet, and larger on ResNet-50 at batch 64 (us, tiles with statistics / strips without: 64 -> 64 @56x56 296 / 251, 128 -> 128 @28x28 300 / 261,
+// stride 2 128 -> 128 @56x56 464 / 282, 64 -> 256 1x1 @56x56 167 / 140).
 //
 // The inner operation is two fp32 VALU instructions per (co,k,position) term
 // -- v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- and cannot use FMA or

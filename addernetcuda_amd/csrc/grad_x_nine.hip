@@ -7,15 +7,16 @@
 // the output channels; sums of sums live in LDS (once per 72 terms), 10 KB a wave, so that four waves per SIMD stay.  Large maps that
 // fill tiles of 16 x 16 or 8 x 32 positions are left to the tiles of grad_x.hip (see grad_x_tiles), which ask for gy once instead of nine
 // times: 128 -> 128 @32x32, 128 images, 698 us there, 734 here, 256 -> 256 @16x16 902 against 921.
-// us, tiles or the kernel for few positions there was -> this: 32 images 64 -> 64 @56x56 169 -> 156, 128 -> 128 @28x28 194 -> 164, 512 -> 512 @7x7
-// 322 -> 251, 100 -> 100 @20x20 119 -> 60; 64 -> 64 @8x8, 256 images 30.6 -> 28.3, one image 29 -> 6; 128 -> 128 @28x28, 4 / 1 images 97 -> 29, 94 -> 14;
-// 48 -> 12 @4x4, 64 images 8.4 -> 5.4; 256 -> 256 @14x14, one image 20 -> 18.
+// us, tiles or the kernel for few positions there was -> this: 32 images 64 -> 64 @56x56 168 -> 161, 128 -> 128 @28x28 193 -> 167, 256 -> 256 @14x14 244 -> 228,
+// 512 -> 512 @7x7 321 -> 281, 100 -> 100 @20x20 118 -> 64; 64 -> 64 @8x8, 256 images 29.8 -> 30.3, one image 29 -> 6.3; 128 -> 128 @28x28, 4 / 1 images 97 -> 34,
+// 94 -> 16; 12 -> 48 @4x4, 64 images 8.5 -> 5.6; 256 -> 256 @14x14, one image 19.9 -> 17.6.  8 x 4 results in two instructions a term are 128 registers and five to
+// seven spilled ones (24 to 32 bytes of scratch per lane).
 //
 // 25 taps: 4 channels x 2 positions per lane, three reads per row of the window a channel ahead; small launches 4 x 1.  Rows of an odd length and 4 x 1 take three
 // instructions a term (error against float64 1.3e-7 to 1.5e-7 of the result; two instructions 2.0e-7 to 2.1e-7, tiles 2.1e-7 to 3.7e-7).  us, tiles in LDS ->
-// this: 342 channels of gy -> 48 of gx @10x10, 8 images, 279 -> 57, 261 -> 10 @27x27, 5 images, bfloat16, 206 -> 43, 813 -> 551 @9x9, two images, 730 -> 255, 64 -> 64 @8x8,
-// 64 images, 50 -> 29, one image 44 -> 12, 19 -> 47 @14x14, 193 images, 73 -> 58, 100 -> 100 @28x28, 32 images, bfloat16, 379 -> 311; odd rows, where tiles ran two instructions:
-// 32 images, 64 -> 32 @17x17 78 -> 45, @21x21 82 -> 62, @25x25 83 -> 83, @29x29 82 -> 97, @53x53 258 -> 285; what fills tiles stays there (fills_5x5_tiles).
+// this: 342 channels of gy -> 48 of gx @10x10, 8 images, 277 -> 56, 261 -> 10 @27x27, 5 images, bfloat16, 204 -> 42, 813 -> 551 @9x9, two images, 727 -> 252, 64 -> 64 @8x8,
+// 64 images, 46 -> 27, one image 44 -> 11, 19 -> 47 @14x14, 193 images, 64 -> 51, 100 -> 100 @28x28, 32 images, bfloat16, 349 -> 285; odd rows, where tiles ran two instructions:
+// 32 images, 64 -> 32 @17x17 71 -> 40, @21x21 71 -> 51, @25x25 72 -> 73, @29x29 72 -> 86, @53x53 242 -> 273; what fills tiles stays there (fills_5x5_tiles).
 // Tried on the way: 4 x 4 per lane 64 -> 64 @56x56, 16 images, 471 (66 registers spilled), 4 x 2 in three instructions 295, with five waves per SIMD 327.
 #include "wave_split.hpp"
 

@@ -10,10 +10,10 @@
 //
 // Three vector instructions per term (two for the layers that had them in tiles: rows of an even length, at most kSatMaxTerms terms) bound
 // it, and a weight meets one position only, so that scalar loads and the reads of gy are what competes with them.  us, one position per lane from
-// memory (the kernel for any layer), or tiles for rows of an even length -> this: 533 -> 113 @19x19, 28 images, 1480 -> 130; 498 -> 124 @10x9, 225 images,
-// bfloat16, 2783 -> 259; 107 -> 278 @23x23, 5 images, 894 -> 26; 5x5: 6 -> 897 @41x49, 27 images, bfloat16, 8330 -> 149, 7 -> 144 @23x26, 202 images,
-// 1425 -> 70, 23 -> 182 @31x39, 5 images, 1478 -> 25; even rows: 512 -> 512 @14x14, 32 images, 334 -> 271, 256 -> 256 @28x28 243 -> 239, one image
-// 74 -> 19, 27 -> 968 @52x52, 16 images, 397 -> 195.  Error against float64 1.1e-7 to 1.7e-7 of the result (tiles 1.6e-7 to 2.2e-7).
+// memory (the kernel for any layer), or tiles for rows of an even length -> this: 533 -> 113 @19x19, 28 images, 1452 -> 124; 498 -> 124 @10x9, 225 images,
+// bfloat16, 2801 -> 257; 107 -> 278 @23x23, 5 images, 897 -> 25; 5x5: 6 -> 897 @41x49, 27 images, bfloat16, 8345 -> 150, 7 -> 144 @23x26, 202 images,
+// 1415 -> 66, 23 -> 182 @31x39, 5 images, 1482 -> 25; even rows: 512 -> 512 @14x14, 32 images, 320 -> 247, 256 -> 256 @28x28 218 -> 212, one image
+// 73 -> 18, 27 -> 968 @52x52, 16 images, 389 -> 173.  Error against float64 1.1e-7 to 1.7e-7 of the result (tiles 1.6e-7 to 2.2e-7).
 // Tried on the way: 4 channels x 2 blocks per lane 256 -> 256 @28x28 239 -> 313 (four waves per SIMD instead of eight); 8 channels x one block 224
 // with two instructions a term, but 512 -> 512 @14x14 271 -> 333; the weights of a block's channels asked for one channel at a time 257.
 #include "wave_split.hpp"

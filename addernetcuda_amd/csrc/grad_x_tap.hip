@@ -7,9 +7,9 @@
 // the KSP waves of a workgroup share the output channels, so that planes of 14x14 and 7x7 and few images still fill the chip.
 // Sums of sums live in LDS (once per 64 terms): 96 registers, two waves on each issue port; in registers 16 x 1 or 8 x 2 positions
 // fit, 168 and 165 us where this takes 141 (512 -> 256 @28x28, 32 images).
-// us, 128 positions x 64 channels with gy staged in LDS -> this: 32 images 64 -> 256 @56x56 98 -> 74, 256 -> 64 90 -> 84, 256 -> 128
-// 153 -> 144, 128 -> 512 @28x28 107 -> 77, 512 -> 256 164 -> 141, 256 -> 1024 @14x14 171 -> 85, 1024 -> 256 103 -> 75, 512 -> 2048 @7x7
-// 245 -> 113, 2048 -> 512 123 -> 79; one image: 256 -> 1024 @14x14 154 -> 16, 64 -> 256 @56x56 42 -> 8.
+// us, 128 positions x 64 channels with gy staged in LDS -> this: 32 images 64 -> 256 @56x56 104 -> 80, 256 -> 64 92 -> 81, 256 -> 128
+// 157 -> 145, 128 -> 512 @28x28 107 -> 80, 512 -> 256 167 -> 140, 256 -> 1024 @14x14 169 -> 89, 1024 -> 256 105 -> 77, 512 -> 2048 @7x7
+// 242 -> 118, 2048 -> 512 127 -> 84; one image: 256 -> 1024 @14x14 153 -> 17, 64 -> 256 @56x56 42 -> 9.
 #include "wave_split.hpp"
 
 #include <type_traits>
