@@ -2,12 +2,13 @@
 // or 2 and 1x1 / pad 0, float storage, tiles of x in LDS.  The forwards without statistics are those of fwd_nine.hip and fwd_tap.hip,
 // which have the same bits: every result adds its channels' terms in chunks (fwd_chunk) and the chunks in channel order.
 //
-// Why not those kernels here as well: a slot of statistics sums the results of one wave, and their strips of all images in a row
+// Why the tiles: a slot of statistics sums the results of one wave, and the strips of those kernels, which line up over all images,
 // group the results otherwise than a tile does.  The sums then differ in their last bits, the normalised maps behind them with them,
 // and a deep network amplifies that: the logits of an untrained ResNet-50 whose BatchNorm statistics came from either grouping lie up to
-// 0.07 of their root mean square apart.  The price is small on ResNet-20 (step at batch 256 2041 us here, 2021 with strips), VGG-small and
-// DenseNet, and larger on ResNet-50 at batch 64 (us, tiles with statistics / strips without: 64 -> 64 @56x56 296 / 251, 128 -> 128 @28x28 300 / 261,
-// stride 2 128 -> 128 @56x56 464 / 282, 64 -> 256 1x1 @56x56 167 / 140).
+// 0.07 of their root mean square apart.  So the grouping stays the tiles' whichever kernel makes the results: launches that leave the
+// tiles half empty run the kernel without tiles, and tile_stats_kernel sums its y as the tiles would have (statistics_apart).  us for a training step,
+// all forwards in tiles -> this: ResNet-20, 8 images 1427 -> 957, 47 images 1466 -> 1173, 128 images 1626 -> 1569, VGG-small, 8 images 2357 -> 1224, 30
+// 3324 -> 2839 (input gradients without tiles among them; with the statistics in the kernels without tiles and their grouping 849, 1127, 1508, 1195, 2848).
 //
 // The inner operation is two fp32 VALU instructions per (co,k,position) term
 // -- v_sub_f32 d, s_w, v_x ; v_sub_f32 acc, acc, |d| -- and cannot use FMA or
@@ -24,6 +25,53 @@
 #include <type_traits>
 
 namespace adder {
+
+// BatchNorm statistics of a layer's output: per wave and output channel the sums of y and y*y over the wave's positions, in the partial-sum
+// layout of the BatchNorm kernels (slot = position wave of the launch, stats[(co * slots + slot) * 2 + {0, 1}]).
+// The lanes sum deviations from a pivot (lane 0's first value) in fp32 and lane 0 moves the sums back
+// to the origin in fp64, so the cancellation in E[y*y] - E[y]^2 happens in double precision.
+// row_ok: the lane's row is inside the map; wo: its first column; co_base: the first of the wave's TM channels.
+template <int TM, int TN>
+__device__ __forceinline__ void tile_stats(const float (&tot)[TM][TN], const bool row_ok, const int wo, const int Wo, const int co_base, const int Co,
+                                           const int slots, const int slot, const int lane, double *__restrict__ stats) {
+    float cnt = 0.f;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) cnt += (row_ok && wo + t < Wo) ? 1.f : 0.f;
+    const double count = (double)wave_sum_dpp(cnt);
+    static_assert(TM == 2 || TM == 4 || TM == 8, "channels per lane of the tile shapes");
+    // all 2 TM sums of the wave in one reduce-scatter: lane l < 2 TM ends with sum number j(l) (channel j / 2,
+    // first or second moment j % 2), fetches the other moment of its channel from the lane that holds it,
+    // and moves its own one back to the origin
+    float sums[2 * TM], pivot[TM];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+        pivot[m] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(tot[m][0])));
+        float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+            if (row_ok && wo + t < Wo) {
+                const float dv = tot[m][t] - pivot[m];
+                s1 += dv;
+                s2 = fmaf(dv, dv, s2);
+            }
+        sums[2 * m] = s1;
+        sums[2 * m + 1] = s2;
+    }
+    const float mine = wave_sum_scatter<2 * TM>(sums, lane);
+    constexpr int TOP = TM;   // lane bit that j % 2 comes from: j is the bit reversal of the lane
+    const float other = __shfl_xor(mine, TOP, 64);
+    const int j = wave_sum_scatter_index<2 * TM>(lane), m = j >> 1;
+    float piv = pivot[0];
+#pragma unroll
+    for (int k = 1; k < TM; ++k) piv = m == k ? pivot[k] : piv;
+    const double c = (double)piv;
+    const int co = co_base + m;
+    if (lane < 2 * TM && co < Co) {
+        // j % 2 == 0: sum of y = d1 + n c;  else: sum of y*y = d2 + 2 c d1 + n c*c
+        const double v = (j & 1) ? (double)mine + 2.0 * c * (double)other + count * c * c : (double)mine + count * c;
+        stats[((size_t)co * slots + slot) * 2 + (j & 1)] = v;
+    }
+}
 
 // ---------------------------------------------------------------------------
 // Tiled kernel for 3x3 / pad 1, stride S = 1 or 2, and 1x1 / pad 0 (the figures are the 3x3 ones).
@@ -209,72 +257,8 @@ __global__ __launch_bounds__(C::NTHREADS) void fwd_tile_kernel(const T *__restri
 
     const int n = n0 + img, ho = h0 + row, wo = w0 + strip * TN;
     auto finish = [&](float (&tot)[TM][TN], T *__restrict__ y, double *__restrict__ stats) {
-    if (stats) {
-        // BatchNorm statistics of the layer's output on the way out: per wave and output channel the sums of
-        // y and y*y over the wave's valid positions, in the partial-sum layout of the BatchNorm kernels
-        // (slot = position wave of this launch, stats[(co * slots + slot) * 2 + {0, 1}]).
-        // The lanes sum deviations from a pivot (lane 0's first value) in fp32 and lane 0 moves the sums back
-        // to the origin in fp64, so the cancellation in E[y*y] - E[y]^2 happens in double precision.
-        const bool row_ok = lane_ok && n < N && ho < Ho;
-        const int slots = gridDim.x * C::POSW, slot = blockIdx.x * C::POSW + pw;
-        float cnt = 0.f;
-#pragma unroll
-        for (int t = 0; t < TN; ++t) cnt += (row_ok && wo + t < Wo) ? 1.f : 0.f;
-        const double count = (double)wave_sum_dpp(cnt);
-        if constexpr (TM == 2 || TM == 4 || TM == 8) {
-            // all 2 TM sums of the wave in one reduce-scatter: lane l < 2 TM ends with sum number j(l) (channel j / 2,
-            // first or second moment j % 2), fetches the other moment of its channel from the lane that holds it,
-            // and moves its own one back to the origin
-            float sums[2 * TM], pivot[TM];
-#pragma unroll
-            for (int m = 0; m < TM; ++m) {
-                pivot[m] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(tot[m][0])));
-                float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-                    if (row_ok && wo + t < Wo) {
-                        const float dv = tot[m][t] - pivot[m];
-                        s1 += dv;
-                        s2 = fmaf(dv, dv, s2);
-                    }
-                sums[2 * m] = s1;
-                sums[2 * m + 1] = s2;
-            }
-            const float mine = wave_sum_scatter<2 * TM>(sums, lane);
-            constexpr int TOP = TM;   // lane bit that j % 2 comes from: j is the bit reversal of the lane
-            const float other = __shfl_xor(mine, TOP, 64);
-            const int j = wave_sum_scatter_index<2 * TM>(lane), m = j >> 1;
-            float piv = pivot[0];
-#pragma unroll
-            for (int k = 1; k < TM; ++k) piv = m == k ? pivot[k] : piv;
-            const double c = (double)piv;
-            const int co = co_base + m;
-            if (lane < 2 * TM && co < Co) {
-                // j % 2 == 0: sum of y = d1 + n c;  else: sum of y*y = d2 + 2 c d1 + n c*c
-                const double v = (j & 1) ? (double)mine + 2.0 * c * (double)other + count * c * c : (double)mine + count * c;
-                stats[((size_t)co * slots + slot) * 2 + (j & 1)] = v;
-            }
-        } else {
-#pragma unroll
-            for (int m = 0; m < TM; ++m) {
-                const float pivot = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(tot[m][0])));
-                float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-                    if (row_ok && wo + t < Wo) {
-                        const float dv = tot[m][t] - pivot;
-                        s1 += dv;
-                        s2 = fmaf(dv, dv, s2);
-                    }
-                const double d1 = (double)wave_sum_dpp(s1), d2 = (double)wave_sum_dpp(s2), c = (double)pivot;
-                const int co = co_base + m;
-                if (lane == 0 && co < Co) {
-                    stats[((size_t)co * slots + slot) * 2] = d1 + count * c;
-                    stats[((size_t)co * slots + slot) * 2 + 1] = d2 + 2.0 * c * d1 + count * c * c;
-                }
-            }
-        }
-    }
+    if (stats)
+        tile_stats<TM, TN>(tot, lane_ok && n < N && ho < Ho, wo, Wo, co_base, Co, (int)gridDim.x * C::POSW, (int)blockIdx.x * C::POSW + pw, lane, stats);
     if (lane_ok && n < N && ho < Ho) {
         const bool vec = TN % 4 == 0 && (Wo & 3) == 0 && wo + TN <= Wo;
         if constexpr (EVAL) {
@@ -404,6 +388,51 @@ __global__ __launch_bounds__(512) void fwd_few_kernel(const float *__restrict__ 
             if (p < total) y[((size_t)(p / L) * d.Co + co) * L + p % L] = tot[k];
         }
     }
+}
+
+// The statistics of a y that another kernel left, a wave per slot and TM channels: each wave has the results that a wave of
+// fwd_tile_kernel<C> has, in the same lanes, so that the statistics are the same bits.  One read of y and about 3 us.
+template <class C>
+__global__ __launch_bounds__(256) void tile_stats_kernel(const float *__restrict__ y, double *__restrict__ stats, int N, int Co, int Ho, int Wo, int tilesH, int tilesW,
+                                                         int slots) {
+    constexpr int TM = C::TM, TN = C::TN;
+    static_assert(C::LANES % 64 == 0, "whole waves of positions");
+    const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6))), lane = threadIdx.x & 63;
+    const int co_base = wave / slots * TM, slot = wave % slots;
+    if (co_base >= Co) return;
+    int b = slot / C::POSW;
+    const int tw = b % tilesW; b /= tilesW;
+    const int th = b % tilesH; b /= tilesH;
+    const int p = slot % C::POSW * 64 + lane;
+    const int n = b * C::NIMG + p / (C::SPR * C::TH), ho = th * C::TH + p / C::SPR % C::TH, wo = tw * C::TW + p % C::SPR * TN;
+    const bool row_ok = n < N && ho < Ho;
+    const float *src = y + ((size_t)min(n, N - 1) * Co * Ho + min(ho, Ho - 1)) * Wo;
+    float tot[TM][TN];
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+        const float *row = src + (size_t)min(co_base + m, Co - 1) * Ho * Wo;
+        if (Wo % TN == 0) {   // (a strip lies inside the row or beside it)
+            ld_strip<TN>(row + min(wo, Wo - TN), tot[m]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < TN; ++t) tot[m][t] = row[min(wo + t, Wo - 1)];
+        }
+    }
+    if (!row_ok) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) tot[m][t] = 0.f;
+    }
+    tile_stats<TM, TN>(tot, row_ok, wo, Wo, co_base, Co, slots, slot, lane, stats);
+}
+
+template <class C>
+static int launch_tile_stats(const float *y, double *stats, const ConvDims &d, hipStream_t s) {
+    const int tilesH = ceil_div(d.Ho, C::TH), tilesW = ceil_div(d.Wo, C::TW), slots = ceil_div(d.N, C::NIMG) * tilesH * tilesW * C::POSW;
+    hipLaunchKernelGGL((tile_stats_kernel<C>), dim3((unsigned)ceil_div_l((long)slots * ceil_div(d.Co, C::TM), 4)), dim3(256), 0, s, y, stats, d.N, d.Co, d.Ho, d.Wo, tilesH,
+                       tilesW, slots);
+    return check_launch();
 }
 
 template <class C, bool VEC, bool SUB = false, bool MUL = false, bool PAIR = false, bool EVAL = false, class T = float>
@@ -554,39 +583,62 @@ int launch_fwd_pair(const float *x, const float *w, const float *w_side, float *
     return d.Ci >= 128 ? run(FwdW8S2L{}) : run(FwdW8S2{});
 }
 
+// f(tile shape, dimensions): of a layer's variant, 1x1 layers as one row
+template <class F>
+static auto with_tile(const ConvDims &d, int variant, F f) {
+    switch (variant) {
+        case 1: switch (rows_per_tile_w32(d.Ho)) {
+            case 16: return f(FwdW32{}, d);
+            case 8: return f(FwdW32H8{}, d);
+            default: return f(FwdW32H4{}, d);
+        }
+        case 2: return f(FwdW16{}, d);
+        case 3: return f(FwdW8{}, d);
+        case 4: return f(FwdW16S2{}, d);
+        case 5: return d.Ci >= 128 ? f(FwdW8S2L{}, d) : f(FwdW8S2{}, d);
+        case 6: return f(Fwd1x1{}, as_one_row(d));
+        case 7: return f(Fwd1x1s{}, as_one_row(d));
+        case 8: case 9: return f(Fwd1x1sub{}, as_one_row(d));
+        case 10: case 12: return f(Fwd1x1q{}, as_one_row(d));
+        default: return f(Fwd1x1sq{}, as_one_row(d));
+    }
+}
+
 int fwd_stats_slots(const ConvDims &d) {
     const int variant = tile_variant(d);
     if (few_positions(d, variant)) return ceil_div(d.N * d.Ho * d.Wo, 64);
-    switch (variant) {
-        case 1: switch (rows_per_tile_w32(d.Ho)) {
-            case 16: return tile_slots<FwdW32>(d);
-            case 8: return tile_slots<FwdW32H8>(d);
-            default: return tile_slots<FwdW32H4>(d);
-        }
-        case 2: return tile_slots<FwdW16>(d);
-        case 3: return tile_slots<FwdW8>(d);
-        case 4: return tile_slots<FwdW16S2>(d);
-        case 5: return tile_slots<FwdW8S2>(d);
-        case 6: return tile_slots<Fwd1x1>(as_one_row(d));
-        case 7: return tile_slots<Fwd1x1s>(as_one_row(d));
-        case 8: case 9: return tile_slots<Fwd1x1sub>(as_one_row(d));
-        case 10: case 12: return tile_slots<Fwd1x1q>(as_one_row(d));
-        case 11: case 13: return tile_slots<Fwd1x1sq>(as_one_row(d));
-        default: return conv1x1_supported(d, nullptr, nullptr) ? fwd_1x1_stats_slots(d) : 0;
-    }
+    if (variant == 0) return conv1x1_supported(d, nullptr, nullptr) ? fwd_1x1_stats_slots(d) : 0;
+    return with_tile(d, variant, [](auto cfg, const ConvDims &f) { return tile_slots<decltype(cfg)>(f); });
+}
+
+// Whether a forward with statistics is the kernel without tiles and, behind it, tile_stats_kernel: where the tiles leave half of the CUs without a workgroup, or
+// a good share of their lanes without a position and the layer is long enough for that to outweigh the read of y.  us, tiles / plain forward, to which
+// the statistics add 3 to 4 and a read of y: 16 -> 16 @32x32, 64 images, 128 workgroups, 15.7 / 11.1, 128 images 16.6 / 16.0; 64 -> 64 @8x8, 8 images 28 / 7.3, 128 28.6 / 18.2,
+// 256 29.1 / 26.1, stride 2 32 -> 64 @16x16, 32 images, 18.6 / 11.2, 64 18.7 / 16.5; 64 -> 64 @56x56 (88 % of the lanes), 32 images, 160 / 136, 512 -> 512 @7x7 (77 %) 285 / 180, stride 2 128 -> 128 @56x56 (77 %) 221 / 153;
+// 512 -> 512 @8x8, 32 images, 256 workgroups, 276 / 182; whole tiles, 128 -> 128 @32x32, 128 images, 654 / 622 with 67 MB of y; 1x1, 1024 -> 256 @14x14 (77 %), 128 images, 336 / 297,
+// 512 -> 128 @28x28 (94 %), 32 images, 93 / 86.
+static bool statistics_apart(const ConvDims &d, int variant) {
+    if (variant == 0 || few_positions(d, variant) || d.K() < 100) return false;
+    if (variant < 6 ? !fwd_nine_supported(d) : !fwd_tap_supported(d) || fwd_strided_tile_supported(d)) return false;
+    return with_tile(d, variant, [&](auto cfg, const ConvDims &f) {
+        using C = decltype(cfg);
+        const long tiles = (long)ceil_div(f.N, C::NIMG) * ceil_div(f.Ho, C::TH) * ceil_div(f.Wo, C::TW), wgs = tiles * ceil_div(f.Co, C::TM * C::COW);
+        if (tiles * C::POSW * ceil_div(f.Co, C::TM) * 64 > kMaxThreads - 256) return false;
+        constexpr int waves = C::NTHREADS / 64 < 8 ? C::NTHREADS / 64 : 8;
+        if (wgs * waves <= (d.K() >= 2000 ? 2048 : variant == 5 ? 384 : 1024)) return true;
+        return d.K() >= 500 && 100L * f.N * f.Ho * f.Wo < (d.kh == 3 ? 90 : 80) * tiles * (C::NIMG * C::TH * C::TW);
+    });
 }
 
 int fwd_stats_kernel(const ConvDims &d) {
     const int variant = tile_variant(d), rows = rows_per_tile_w32(d.Ho);
     if (few_positions(d, variant)) return 2;
     if (variant == 0) return conv1x1_supported(d, nullptr, nullptr) ? 1 : 0;
-    return 10 * variant + (variant == 1 ? (rows == 16 ? 0 : rows == 8 ? 1 : 2) : variant == 5 && d.Ci >= 128 ? 1 : 0);
+    return (statistics_apart(d, variant) ? 1000 : 0) + 10 * variant + (variant == 1 ? (rows == 16 ? 0 : rows == 8 ? 1 : 2) : variant == 5 && d.Ci >= 128 ? 1 : 0);
 }
 
 // stats: per-channel partial sums of y and y*y, fwd_stats_slots(d) > 0 slots per channel.
 int launch_fwd_stats(const float *x, const float *w, float *y, double *stats, const ConvDims &d, hipStream_t s) {
-    // rows that are whole groups of four are moved as such and need bases aligned to a group
-    const bool rows_ok = (d.W % 4 != 0 || aligned_groups(x)) && (d.Wo % 4 != 0 || aligned_groups(y));
     const int variant = tile_variant(d);
     if (few_positions(d, variant)) {
         const int chunk = fwd_chunk(d), chunks = ceil_div(d.Ci, chunk);
@@ -594,24 +646,16 @@ int launch_fwd_stats(const float *x, const float *w, float *y, double *stats, co
                            0, s, x, w, y, stats, d, chunk);
         return check_launch();
     }
-    const bool strided = variant == 8 || variant == 9 || variant == 12 || variant == 13;
-    if (strided) {   // x is read element by element; y is a dense row per plane
-        const ConvDims f = as_one_row(d);
-        if (f.Wo % 4 != 0 || aligned_groups(y)) switch (variant) {
-            case 8: case 9: return launch_tile_v<Fwd1x1sub, false, true>(x, w, y, stats, f, s, sampling_of(d));
-            case 12: return launch_tile_v<Fwd1x1q, false, true>(x, w, y, stats, f, s, sampling_of(d));
-            default: return launch_tile_v<Fwd1x1sq, false, true>(x, w, y, stats, f, s, sampling_of(d));
-        }
-    } else if (variant >= 6) {
-        const ConvDims f = as_one_row(d);
-        if (f.W % 4 != 0 || (aligned_groups(x) && aligned_groups(y))) switch (variant) {
-            case 6: return launch_tile<Fwd1x1>(x, w, y, stats, f, s);
-            case 7: return launch_tile<Fwd1x1s>(x, w, y, stats, f, s);
-            case 10: return launch_tile<Fwd1x1q>(x, w, y, stats, f, s);
-            default: return launch_tile<Fwd1x1sq>(x, w, y, stats, f, s);
-        }
+    if (variant == 0) return conv1x1_supported(d, x, y) ? launch_fwd_1x1(x, w, y, stats, d, s, kNoBnEval) : static_cast<int>(ADDER_ERR_UNSUPPORTED);
+    // rows (1x1: planes) that are whole groups of four are moved as such and need bases aligned to a group; x of a strided 1x1 layer is read element by element
+    const ConvDims f = variant >= 6 ? as_one_row(d) : d;
+    const bool strided = variant >= 6 && d.stride > 1;
+    if ((!strided && f.W % 4 == 0 && !aligned_groups(x)) || (f.Wo % 4 == 0 && !aligned_groups(y))) return ADDER_ERR_UNSUPPORTED;
+    if (statistics_apart(d, variant)) {
+        if (int rc = variant < 6 ? launch_fwd_nine(x, w, y, d, s, kNoBnEval) : launch_fwd_tap(x, w, y, d, s, kNoBnEval)) return rc;
+        return with_tile(d, variant, [&](auto cfg, const ConvDims &g) { return launch_tile_stats<decltype(cfg)>(y, stats, g, s); });
     }
-    if (rows_ok) switch (variant) {
+    switch (variant) {
         case 1: switch (rows_per_tile_w32(d.Ho)) {
             case 16: return launch_tile<FwdW32>(x, w, y, stats, d, s);
             case 8: return launch_tile<FwdW32H8>(x, w, y, stats, d, s);
@@ -621,11 +665,14 @@ int launch_fwd_stats(const float *x, const float *w, float *y, double *stats, co
         case 3: return launch_tile<FwdW8>(x, w, y, stats, d, s);
         case 4: return launch_tile<FwdW16S2>(x, w, y, stats, d, s);
         case 5: return d.Ci >= 128 ? launch_tile<FwdW8S2L>(x, w, y, stats, d, s) : launch_tile<FwdW8S2>(x, w, y, stats, d, s);
-        default: break;
+        case 6: return launch_tile<Fwd1x1>(x, w, y, stats, f, s);
+        case 7: return launch_tile<Fwd1x1s>(x, w, y, stats, f, s);
+        case 8: case 9: return launch_tile_v<Fwd1x1sub, false, true>(x, w, y, stats, f, s, sampling_of(d));
+        case 10: return launch_tile<Fwd1x1q>(x, w, y, stats, f, s);
+        case 11: return launch_tile<Fwd1x1sq>(x, w, y, stats, f, s);
+        case 12: return launch_tile_v<Fwd1x1q, false, true>(x, w, y, stats, f, s, sampling_of(d));
+        default: return launch_tile_v<Fwd1x1sq, false, true>(x, w, y, stats, f, s, sampling_of(d));
     }
-    // (a tiled variant that was turned down for its alignment counts its statistics slots differently)
-    if (variant == 0 && conv1x1_supported(d, x, y)) return launch_fwd_1x1(x, w, y, stats, d, s, kNoBnEval);
-    return ADDER_ERR_UNSUPPORTED;
 }
 
 // Strided 1x1 layers without statistics that stay in tiles: chunks of eight channels, whose sums the waves of fwd_tap.hip would have to bring together after 16

@@ -89,7 +89,8 @@ ADDER_API int adder_conv2d_fwd_f32(const float *x, const float *w, float *y,
 ADDER_API int adder_conv2d_fwd_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel);
 
 /* ... the forward calls with statistics: 0 none, 1 the plain 1x1 one, 2 the 1x1 one for few positions, from 10 on those in tiles: 10 x (1..3 3x3 by
- * output width, 4..5 with stride 2, 6..7 1x1 by plane size, 8..9 with a stride, 10..13 the same for channels that are no multiple of eight) plus a shape. */
+ * output width, 4..5 with stride 2, 6..7 1x1 by plane size, 8..9 with a stride, 10..13 the same for channels that are no multiple of eight) plus a shape;
+ * plus 1000 where the forward is the one without tiles and the statistics are summed behind it, as those tiles group them. */
 ADDER_API int adder_conv2d_fwd_stats_kernel(int N, int Ci, int H, int W, int Co, int kh, int kw, int stride, int pad, int *kernel);
 
 /* ... the input gradient of the backward calls in float (bf16 = 0) or bfloat16 storage: 0 the general one, 1000000 the plain 1x1 one, 2000000 those in

@@ -4,8 +4,8 @@ import random
 
 import pytest
 
-from tests.kernel_shapes import FORWARD, GRAD_X, forward_shape, grad_x_shape
-from tests.util import TAP, NINE, S2, fwd_kernel, grad_x_kernel
+from tests.kernel_shapes import FORWARD, GRAD_X, STATS_APART, forward_shape, grad_x_shape
+from tests.util import TAP, NINE, S2, TILED_FORWARD, fwd_kernel, grad_x_kernel, stats_apart, stats_kernel
 
 
 @pytest.mark.parametrize("shape", FORWARD, ids=str)
@@ -45,3 +45,11 @@ def test_no_layer_takes_another_shape():
 def test_no_wave_of_a_full_strided_launch_is_mostly_idle(Co, waves, k):
     assert grad_x_shape((62, 47, 58, 57, Co, k, 2, k // 2))[1] == waves
     assert grad_x_shape((1, 47, 14, 13, Co, k, 2, k // 2))[1] == (1 if Co <= 8 else 2 if Co <= 16 else 4 if Co <= 32 else 8)   # (a small one needs all)
+
+
+def test_statistics_of_few_images_are_summed_behind_the_forward():
+    assert set(STATS_APART) == set(TILED_FORWARD) | {51}
+    for kernel, cases in STATS_APART.items():
+        for case, batch in cases:
+            many = (batch,) + case[1:]
+            assert stats_kernel(case) == stats_kernel(many) == kernel and stats_apart(case) and not stats_apart(many), case

@@ -58,8 +58,13 @@ def fwd_kernel(case):
 
 
 def stats_kernel(case):
-    """The number of the kernel that the forward with statistics takes."""
-    return _kernel("adder_conv2d_fwd_stats_kernel", case)
+    """The number of the kernel that the forward with statistics takes, or whose tiles group them (stats_apart)."""
+    return _kernel("adder_conv2d_fwd_stats_kernel", case) % 1000
+
+
+def stats_apart(case):
+    """Whether the forward with statistics is the one without tiles, and sums them behind it."""
+    return _kernel("adder_conv2d_fwd_stats_kernel", case) >= 1000
 
 
 def grad_x_kernel(case, bf16=False):
